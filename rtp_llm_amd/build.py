@@ -27,12 +27,12 @@ HEADERS = [os.path.join(INCLUDE, "mi355_hybrid.h"), os.path.join(CSRC, "common.h
 # the hybrid decoder family (attention / linear-recurrence mixers over dense [out, in] weights) lives in a library of its own
 HYBRID_SOURCES = ["gemm_dense.hip", "hybrid_ops.hip", "error.cpp"]
 HYBRID_LIB = os.path.join(LIBDIR, "libmi355_hybrid.so")
-# hipcc forms packed fp32 instructions by itself from scalar code; the new sources are compiled without them
-HYBRID_CFLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
-CFLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off", "-fno-slp-vectorize", "-Wno-unused-result", "-x", "hip"]
+CFLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off", "-fno-slp-vectorize", "-Wno-unused-result", "-x", "hip",
+          # hipcc forms packed fp32 instructions by itself from scalar code; every source is compiled without them
+          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
 def _stale(src, obj):
@@ -81,7 +81,7 @@ def build_hybrid(force=False, verbose=True):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=len(HYBRID_SOURCES)) as ex:
-        res = list(ex.map(lambda s: _compile(s, force, flags=HYBRID_CFLAGS, tag="_hy"), HYBRID_SOURCES))
+        res = list(ex.map(lambda s: _compile(s, force, tag="_hy"), HYBRID_SOURCES))
     if any(ch for _, ch in res) or not os.path.exists(HYBRID_LIB):
         tmp = HYBRID_LIB + f".{os.getpid()}.tmp"
         r = subprocess.run([HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + [o for o, _ in res] + ["-ldl"],
