@@ -27,7 +27,7 @@ extern "C" int mi355_gemm_smallm(const void* gp, int wbits, int group_size, int 
                                  mi355_stream_t stream);
 extern "C" int mi355_gemm_wide(const void* gp, int wbits, int group_size, int want_partial, int max_splits,
                                mi355_stream_t stream);
-extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, mi355_stream_t stream);
+extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, double t_limit, mi355_stream_t stream);
 extern "C" int mi355_gemm_fullk(const void* gp, int wbits, int group_size, const void* norm, mi355_stream_t stream);
 extern "C" int mi355_gemm_fullk_residual(const void* gp, int wbits, int group_size, const void* residual_in, void* residual_out,
                                          float* ssq_out, int ssq_ld, mi355_stream_t stream);
@@ -752,22 +752,15 @@ extern "C" int mi355_linear_forward(const void* x, int32_t M, const mi355_weight
     const int ldy  = (mode == MODE_SILU) ? w->N / 2 : w->N;
     const size_t ysz = (mode == MODE_F32) ? 4 : 2;
     hipStream_t st = (hipStream_t)stream;
-    // prefill-sized M: the compute-shaped kernel reads every weight once per 128 rows.  Its grid is (N / 256) x (M / 128)
-    // blocks without a K split: narrow outputs at moderate M (down_proj, N = 3584: 14 blocks per 128 rows) would leave
-    // most CUs idle (measured M = 128: 246 us vs 2 x 21 us as 64-row slabs), so those stay on the decode kernels
-    const bool bf = w->act_dtype == MI355_ACT_BF16;   // bf16 activations: 64-row slabs through the staged kernel at every M
-    // compute-shaped kernel or 64-row slabs of the decode kernels?  A small time model (us), calibrated on MI355X at the Qwen2-7B
-    // shapes (profiles/r03_prefill_gemm_tiles_per_wave.txt): the prefill kernel takes ~2.2 us per 128-k chunk per round of 256
-    // column x row blocks, a 64-row slab ~(weight MB / 1.6 + 6) us.  Narrow outputs at moderate M stay on the slabs (down_proj
-    // at M = 512: 56 blocks, 280 vs 218 us), wider / deeper cases move over earlier than the old ">= 128 blocks" rule allowed
-    // (o_proj at M = 1024: 112 blocks, ~68 vs 204 us).
-    const long pf_blocks = (long)cdiv(w->N_pad / 16, 16) * cdiv(M, 128);
-    const double t_pf = (double)cdiv((int)pf_blocks, 256) * (w->K_pad / 128) * 2.2;
-    const double t_slab = (double)cdiv(M, 64) * ((double)w->K_pad * w->N_pad * w->wbits / 8 / 1.6e6 + 6.0);
-    if (!bf && M >= 128 && w->wbits != 16 && t_pf < t_slab) {
+    const bool bf = w->act_dtype == MI355_ACT_BF16;
+    // more than 64 rows: the compute-shaped kernel, which reads every weight once per row tile, or 64-row slabs of the decode kernels?  A slab of fp16
+    // W4 / W8 is one launch at ~(weight MB / 1.6 + 6) us; 16-bit weights and bf16 activations have no such slab kernel (staged kernel + fold of its K splits,
+    // 24-40 us a slab at the Qwen2-0.5B shapes where the compute-shaped kernel takes 5-20 for all rows) and take it always.
+    if (M > 64) {
+        const double t_slab = (double)cdiv(M, 64) * ((double)w->K_pad * w->N_pad * w->wbits / 8 / 1.6e6 + 6.0);
         GemmParams ps; fill_params(ps, x, M, w);
         ps.mode = mode; ps.bias = (const f16*)bias; ps.y = y; ps.ldy = ldy;
-        const int rc = mi355_gemm_prefill(&ps, w->wbits, w->group_size, stream);
+        const int rc = mi355_gemm_prefill(&ps, w->wbits, w->group_size, (bf || w->wbits == 16) ? 1e30 : t_slab, stream);
         if (rc != MI355_ERR_UNSUPPORTED) return rc;
     }
     for (int m0 = 0; m0 < M; m0 += 64) {

@@ -1,40 +1,69 @@
-// Weight-only dequant GEMM for large M (prefill chunks, M >= 128 rows), gfx950.
+// GEMM on the packed weight images for large M (prefill chunks, more than 64 rows), gfx950.
 //
 // Same contract and weight image as gemm.hip (reference slot: LinearBase.forward,
 // rtp_llm/models_py/modules/factory/linear/linear_base.py:75-85; the reference notes that weight-only quantisation "may
 // cause performance degradation for long sequences during the Prefill phase", docs/backend/quantization.md:3 -- the
 // decode kernels of this library would re-read every weight once per 64 rows).  Here the problem is compute-shaped:
-//   * block = 8 waves, tile = 128 rows x 256 columns; a wave owns 2 adjacent 16-column weight tiles and all 128 rows;
-//   * per 128-k chunk a wave dequantises its 2 x 4 A-fragments ONCE (operand side, fp16) and uses each for the 8 row
-//     blocks: 64 v_mfma_f32_16x16x32_f16 per 104 dequant VALU, so the matrix pipe, not the VALU, sets the pace; the second
-//     wave of each SIMD dequantises while the first one multiplies;
-//   * the activation chunk (128 rows x 128 k fp16 = 32 KiB) is staged once per block in LDS in the fragment-major,
-//     XOR-swizzled image of gemm.hip (conflict-free ds_read_b128) and double-buffered; one B-fragment read feeds two MFMAs;
-//   * weights stream from HBM/L2 once per 128 rows (the M/128 row blocks of a column block run back to back on different
-//     CUs and meet in L2 / Infinity Cache), through a 2-deep register ring, buffer range checks instead of tail branches.
+//   * block = 8 waves; a wave owns 1, 2 or 4 adjacent 16-column weight tiles and all rows of the block's tile (32, 64 or 128);
+//   * per 128-k chunk a wave dequantises its tiles' A-fragments ONCE (operand side) and uses each for every row block: at 128 rows 64 v_mfma_f32_16x16x32 per
+//     104 dequant VALU, so the matrix pipe, not the VALU, sets the pace; the second wave of each SIMD dequantises while the first one multiplies;
+//   * the activation chunk (128 rows x 128 k = 32 KiB) is staged once per block in LDS in the fragment-major, XOR-swizzled image of gemm.hip (conflict-free
+//     ds_read_b128) and double-buffered;
+//   * weights stream from HBM/L2 once per row tile (the row tiles of a column tile run back to back on different CUs and meet in L2 / Infinity Cache),
+//     through a 2-deep register ring, buffer range checks instead of tail branches.
 #include "gemm_common.h"
 
 namespace {
 
-// TPW = weight tiles per wave: 2 (tile 128 x 256, two blocks per CU) or 4 (128 x 512, one block per CU).  One B-fragment read from
-// LDS feeds TPW MFMAs: at TPW = 2 the 8 waves of a block pull 256 KiB of fragments per 128-k chunk through the CU's LDS port for
-// 512 MFMAs -- 2048 cycles of each, neither hidden behind the other; TPW = 4 halves the LDS traffic per MFMA.
-template <int WBITS, int GS, int TPW>
-__global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(const GemmParams p) {
-    constexpr int BM = 128, MB = BM / 16, NW = 8;             // rows, row blocks, waves
+// the epilogue of gemm_store for bf16 tensors: bias, one rounding, SiLU-gate on the rounded pair
+__device__ __forceinline__ void store_bf16(const GemmParams& p, f32x4 v, int m, int n0) {
+    if (n0 >= p.N) return;
+    if (p.bias) {
+        const u32x2 b = *reinterpret_cast<const u32x2*>(p.bias + n0);
+        v[0] += act_lo<true>(b[0]); v[1] += act_hi<true>(b[0]); v[2] += act_lo<true>(b[1]); v[3] += act_hi<true>(b[1]);
+    }
+    if (p.mode == MODE_SILU) {
+        float o[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const float g = act_round<true>(v[2 * t]), u = act_round<true>(v[2 * t + 1]);
+            o[t] = (g / (1.f + __expf(-g))) * u;
+        }
+        *reinterpret_cast<uint32_t*>((f16*)p.y + (size_t)m * p.ldy + (n0 >> 1)) = act_pack<true>(o[0], o[1]);
+    } else {
+        u32x2 o;
+        o[0] = act_pack<true>(v[0], v[1]); o[1] = act_pack<true>(v[2], v[3]);
+        *reinterpret_cast<u32x2*>((f16*)p.y + (size_t)m * p.ldy + n0) = o;
+    }
+}
+
+// One block = 8 waves: NWN = 8 / KS of them side by side along N, KS of them along K (slice ks takes the chunks c with c % KS == ks; the slices' sums meet in
+// LDS at the end).  TPW = weight tiles per wave, MB = 16-row blocks of the tile, so the tile is 16 MB rows x 16 TPW NWN columns.
+//   TPW = 4, MB = 8 (128 x 512, one block per CU): one B-fragment read from LDS feeds four MFMAs.  At TPW = 2 (128 x 256, two blocks per CU) the 8 waves of a
+//   block pull 256 KiB of fragments per 128-k chunk through the CU's LDS port for 512 MFMAs -- 2048 cycles of each, neither hidden behind the other.
+//   MB = 4 and the K-sliced forms are for grids that would leave most CUs without a block (narrow outputs, short prompts): see launch_prefill_t.
+// BF: bf16 activations.  16-bit weights are the MFMA operand as they are; a 4-bit code enters it as the exact integer u - z and the group's scale multiplies the
+// group's fp32 sums (a bf16 product s (u - z) would round the weight to 8 bits); an 8-bit code as the exact u - 128, its column scale on the finished sums.
+template <int WBITS, int GS, bool BF, int MB, int TPW, int KS>
+__global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p) {
+    constexpr int BM = 16 * MB, NWN = 8 / KS;                 // rows, waves side by side
     constexpr int LPC  = WBITS / 4;
     constexpr int NSUB = (GS > 0) ? 4 / GS : 1;
     constexpr int SPG  = 4 / NSUB;
     constexpr bool GROUPED = GS > 0;
+    constexpr bool CSCALE = BF && GROUPED;                    // the group's scale on the accumulator side
     constexpr int XSLOTS = 256 * MB;                          // 16-byte pieces of an x chunk tile
-    constexpr int UPT = XSLOTS / 512;                         // pieces per thread
-    __shared__ u32x4 xs[2][XSLOTS];
+    constexpr int GT = 512 / KS;                              // threads of a K slice
+    constexpr int UPT = XSLOTS / GT;                          // pieces per thread
+    __shared__ u32x4 xs[KS][2][XSLOTS];
+    static_assert(KS == 1 || (size_t)(KS - 1) * NWN * TPW * MB * 1024 <= sizeof(u32x4) * 2 * KS * XSLOTS, "the slices' sums meet in the x buffers");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = wave / NWN, tg = tid - ks * GT;
     const int jj = lane & 15, q = lane >> 4;
     const int m0 = blockIdx.y * BM;
-    const int nt_base = (blockIdx.x * NW + wave) * TPW;
+    const int nt_base = (blockIdx.x * NWN + wave % NWN) * TPW;
     const int KC = p.KC;
 
     constexpr uint32_t FLAGS = 0x00020000u;
@@ -48,17 +77,17 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
         rw[t] = __builtin_amdgcn_make_buffer_rsrc((void*)wb, 0, tile_ok[t] ? KC * LPC * 1024 : 0, FLAGS);
         const char* mb = (const char*)p.meta + (size_t)nt * 16 * 4;
         const int mbytes = GROUPED ? ((KC * NSUB - 1) * p.N_pad + 16) * 4 : 64;
-        rm[t] = __builtin_amdgcn_make_buffer_rsrc((void*)mb, 0, tile_ok[t] ? mbytes : 0, FLAGS);
+        rm[t] = __builtin_amdgcn_make_buffer_rsrc((void*)mb, 0, tile_ok[t] && WBITS != 16 ? mbytes : 0, FLAGS);
     }
     __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, p.x_bytes, FLAGS);
 
-    // x staging: thread owns pieces pi = tid + 512 u: row j = pi >> 4 of the tile, 16-byte piece pp = pi & 15 of the chunk
+    // x staging: thread owns pieces pi = tg + GT u: row j = pi >> 4 of the tile, 16-byte piece pp = pi & 15 of the chunk
     uint32_t xoff[UPT];
     int xslot[UPT];
     bool xrow_ok[UPT];
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-        const int pi = tid + 512 * u, j = pi >> 4, pp = pi & 15;
+        const int pi = tg + GT * u, j = pi >> 4, pp = pi & 15;
         xrow_ok[u] = m0 + j < p.M;
         xoff[u]  = (uint32_t)(((size_t)(m0 + j) * p.K + pp * 8) * 2);
         xslot[u] = pp * (16 * MB) + (j ^ (pp & 3));
@@ -67,14 +96,14 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
     auto load_x = [&](u32x4 (&xr)[UPT], int c) {
 #pragma unroll
         for (int u = 0; u < UPT; ++u) {
-            const int pp = (tid + 512 * u) & 15;
+            const int pp = (tg + GT * u) & 15;
             const bool ok = xrow_ok[u] && c < KC && c * 128 + pp * 8 < p.K;   // rows past M / columns past K read as zero
             xr[u] = bload128<0>(rx, ok ? xoff[u] : OOBX, (uint32_t)c * 256u);
         }
     };
     auto store_x = [&](const u32x4 (&xr)[UPT], int buf) {
 #pragma unroll
-        for (int u = 0; u < UPT; ++u) xs[buf][xslot[u]] = xr[u];
+        for (int u = 0; u < UPT; ++u) xs[ks][buf][xslot[u]] = xr[u];
     };
 
     const uint32_t lane16 = lane * 16u, jj4 = jj * 4u;
@@ -93,7 +122,7 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
         }
     };
     uint32_t mch[TPW];
-    if (!GROUPED) {
+    if (!GROUPED && WBITS != 16) {
 #pragma unroll
         for (int t = 0; t < TPW; ++t) mch[t] = __builtin_amdgcn_raw_buffer_load_b32(rm[t], jj4, 0, 0);
     }
@@ -107,24 +136,67 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
     const f16x2 c960 = {(f16)960.f, (f16)960.f};
 
     u32x4 xr[UPT];
-    load_x(xr, 0);
-    load_w(0, 0);
+    load_x(xr, ks);
+    load_w(0, ks);
     store_x(xr, 0);
-    load_x(xr, 1);
-    load_w(1, 1);
+    load_x(xr, ks + KS);
+    load_w(1, ks + KS);
     __syncthreads();
 
-    auto dq = [&](int d, int t, int s) -> f16x8 {
+    auto dq = [&](int d, int t, int s) -> u32x4 {
+        if constexpr (WBITS == 16) return wr[d][t][s];
         const uint32_t m = GROUPED ? mr[d][t][s / SPG] : mch[t];
         const f16x2 zn = as_h2(__builtin_amdgcn_perm(m, m, 0x05040504u));
         const f16x2 sc = as_h2(__builtin_amdgcn_perm(m, m, 0x07060706u));
-        if (WBITS == 4) return dequant_w4_vc(wr[d][t][0][s], zn, zn + c960, sc, w4c);
-        const u32x4 w = wr[d][t][(s >> 1) % LPC];   // per-channel int8: exact (u - z) operand, the column scale is applied in fp32 in the epilogue
-        return dequant_w8<GROUPED>(w[(s & 1) * 2], w[(s & 1) * 2 + 1], zn, sc);
+        if constexpr (BF) {          // small integers: exact in fp16, in fp32 and in bf16 (the high half of the fp32)
+            f16x8 v;
+            if constexpr (WBITS == 4) {
+                const f16x2 one = {(f16)1.f, (f16)1.f};
+                v = dequant_w4_vc(wr[d][t][0][s], zn, zn + c960, one, w4c);
+            } else {
+                const u32x4 w = wr[d][t][(s >> 1) % LPC];
+                v = dequant_w8<false>(w[(s & 1) * 2], w[(s & 1) * 2 + 1], zn, sc);
+            }
+            u32x4 r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                r[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, (float)v[2 * i + 1]), __builtin_bit_cast(uint32_t, (float)v[2 * i]), 0x07060302u);
+            return r;
+        } else {
+            if constexpr (WBITS == 4) return __builtin_bit_cast(u32x4, dequant_w4_vc(wr[d][t][0][s], zn, zn + c960, sc, w4c));
+            const u32x4 w = wr[d][t][(s >> 1) % LPC];   // per-channel int8: exact (u - z) operand, the column scale is applied in fp32 in the epilogue
+            return __builtin_bit_cast(u32x4, dequant_w8<GROUPED>(w[(s & 1) * 2], w[(s & 1) * 2 + 1], zn, sc));
+        }
     };
+    auto frag = [&](int buf, int s, int mb) { return xs[ks][buf][(s * 4 + q) * (16 * MB) + mb * 16 + (jj ^ q)]; };
     auto compute = [&](int d, int buf) {
-        if constexpr (TPW == 2) {            // all 8 operands of the chunk first, then 64 MFMAs
-            f16x8 a[TPW][4];
+        if constexpr (CSCALE) {              // a group's sums on accumulators of their own, scaled as they join the tile's
+#pragma unroll
+            for (int gi = 0; gi < NSUB; ++gi) {
+                f32x4 ag[TPW][MB];
+#pragma unroll
+                for (int ss = 0; ss < SPG; ++ss) {
+                    u32x4 a[TPW];
+#pragma unroll
+                    for (int t = 0; t < TPW; ++t) a[t] = dq(d, t, gi * SPG + ss);
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) {
+                        const u32x4 b = frag(buf, gi * SPG + ss, mb);
+#pragma unroll
+                        for (int t = 0; t < TPW; ++t) ag[t][mb] = mfma_act<BF>(a[t], b, ss ? ag[t][mb] : (f32x4){0.f, 0.f, 0.f, 0.f});
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {   // this lane's rows of the sums are columns 4 q + r: their scales sit in lanes 4 q + r
+                        const float sc = (float)as_h2((uint32_t)__builtin_amdgcn_ds_bpermute((q * 4 + r) * 4, (int)mr[d][t][gi]))[1];
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb) acc[t][mb][r] = __builtin_fmaf(sc, ag[t][mb][r], acc[t][mb][r]);
+                    }
+            }
+        } else if constexpr (TPW <= 2 && WBITS != 16) {   // all operands of the chunk first, then the MFMAs
+            u32x4 a[TPW][4];
 #pragma unroll
             for (int t = 0; t < TPW; ++t)
 #pragma unroll
@@ -133,38 +205,57 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const f16x8 b = __builtin_bit_cast(f16x8, xs[buf][(s * 4 + q) * (16 * MB) + mb * 16 + (jj ^ q)]);
+                    const u32x4 b = frag(buf, s, mb);
 #pragma unroll
-                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma16x16x32(a[t][s], b, acc[t][mb]);
+                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma_act<BF>(a[t][s], b, acc[t][mb]);
                 }
-        } else {                             // per k-step: TPW operands (16 registers), 8 fragment reads, 8 x TPW MFMAs
+        } else {                             // per k-step: TPW operands (16 registers), MB fragment reads, MB x TPW MFMAs
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                f16x8 a[TPW];
+                u32x4 a[TPW];
 #pragma unroll
                 for (int t = 0; t < TPW; ++t) a[t] = dq(d, t, s);
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
-                    const f16x8 b = __builtin_bit_cast(f16x8, xs[buf][(s * 4 + q) * (16 * MB) + mb * 16 + (jj ^ q)]);
+                    const u32x4 b = frag(buf, s, mb);
 #pragma unroll
-                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma16x16x32(a[t], b, acc[t][mb]);
+                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma_act<BF>(a[t], b, acc[t][mb]);
                 }
             }
         }
     };
 
-    for (int c = 0; c < KC; c += 2) {
-        // chunk c (buffer 0, ring 0); x(c+1) is in registers, w(c+1) in ring 1
+    for (int c = ks; c - ks < KC; c += 2 * KS) {     // the same number of rounds for every slice; chunks past KC are zero rows of x
+        // chunk c (buffer 0, ring 0); x(c + KS) is in registers, w(c + KS) in ring 1
         compute(0, 0);
         store_x(xr, 1);
-        load_x(xr, c + 2);
-        load_w(0, c + 2);
+        load_x(xr, c + 2 * KS);
+        load_w(0, c + 2 * KS);
         __syncthreads();
-        if (c + 1 < KC) compute(1, 1);
+        if (c - ks + KS < KC) compute(1, 1);
         store_x(xr, 0);
-        load_x(xr, c + 3);
-        load_w(1, c + 3);
+        load_x(xr, c + 3 * KS);
+        load_w(1, c + 3 * KS);
         __syncthreads();
+    }
+
+    if constexpr (KS > 1) {                          // the slices' sums, in slice order
+        f32x4* red = (f32x4*)&xs[0][0][0];
+        const int wn = wave % NWN;
+        if (ks > 0) {
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) red[((((ks - 1) * NWN + wn) * TPW + t) * MB + mb) * 64 + lane] = acc[t][mb];
+        }
+        __syncthreads();
+        if (ks > 0) return;
+#pragma unroll
+        for (int k = 1; k < KS; ++k)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) acc[t][mb] += red[((((k - 1) * NWN + wn) * TPW + t) * MB + mb) * 64 + lane];
     }
 
     // ---- epilogue: lane holds, for row m0 + mb*16 + jj, the 4 consecutive columns 16 nt + 4q + r
@@ -173,7 +264,7 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
         if (!tile_ok[t]) continue;
         const int n0 = (nt_base + t) * 16 + q * 4;
         f32x4 sc = {1.f, 1.f, 1.f, 1.f};
-        if (!GROUPED) {
+        if (!GROUPED && WBITS != 16) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t m = __builtin_amdgcn_raw_buffer_load_b32(rm[t], (uint32_t)(q * 4 + r) * 4u, 0, 0);
@@ -183,22 +274,61 @@ __global__ __launch_bounds__(512, TPW == 2 ? 2 : 1) void gemm_prefill_kernel(con
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
             const int m = m0 + mb * 16 + jj;
-            if (m < p.M) gemm_store(p, acc[t][mb] * sc, m, n0, 0);
+            if (m >= p.M) continue;
+            if constexpr (BF) store_bf16(p, acc[t][mb] * sc, m, n0);
+            else              gemm_store(p, acc[t][mb] * sc, m, n0, 0);
         }
     }
 }
 
-template <int WBITS, int GS>
-int launch_prefill_t(const GemmParams& p, hipStream_t st) {
-    // four tiles per wave (one block per CU) when its grid is one well-filled round of the 256 CUs or many rounds; in between
-    // (257..~560 blocks: a second round that is mostly empty) and for small grids the two-tile shape with two blocks per CU wins
-    // (profiles/r03_prefill_gemm_tiles_per_wave.txt: gate_up M = 4096 959 -> 1055 TFLOP/s, down 932 -> 1066, o 885 -> 1015;
-    // qkv M = 4096 with 288 blocks 755 vs 667, gate_up M = 512 with 296 blocks 776 vs 701)
-    const long b4 = (long)cdiv(p.NT, 32) * cdiv(p.M, 128);
-    const bool wide = TUNE(3) == 4 || (TUNE(3) != 2 && ((b4 >= 140 && b4 <= 256) || b4 >= 560));
-    dim3 grid(cdiv(p.NT, wide ? 32 : 16), cdiv(p.M, 128));
-    if (wide) hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, 4>), grid, dim3(512), 0, st, p);
-    else      hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, 2>), grid, dim3(512), 0, st, p);
+// Block shapes: {row blocks, weight tiles per wave, K slices}.
+struct PrefillShape { int mb, tpw, ks; };
+constexpr PrefillShape kPrefillShapes[] = {{8, 4, 1}, {8, 2, 1}, {4, 2, 1}, {4, 1, 1}, {4, 1, 2}, {2, 1, 2}, {2, 1, 4}};
+constexpr int kPrefillShapeCount = sizeof(kPrefillShapes) / sizeof(kPrefillShapes[0]);
+
+// The shape of a call: a time model in us.  A round of a block (KS chunks of 128 k) takes `lat` alone on its CU -- loads, LDS, barrier -- and `sat` of a CU whose
+// share of the grid keeps it busy; the share counts half as the exact quotient and half as the whole blocks of the fullest CU.  Measured (random operands, one MI355X) per
+// operand class over M = 70..4096 at the Qwen2-0.5B and 7B projections: the pick is within 10 % of the fastest shape.  Examples, us at 128x512 / 128x256 / 64x256 /
+// 64x128 / 64x64 / 32x64 / 32x32 tiles: fp16 W4 37888 x 3584 at M = 4096 1088 / 1155 / 1183 / 1368 / 1722 / 1965 / 2945, 3584 x 18944 at M = 128 424 / 250 / 147 / 130 / 66 / 51 / 47;
+// W16 9728 x 896 at M = 512 - / 26 / 26 / 20 / 23 / 27 / 43; bf16 W4 37888 x 3584 at M = 512 - / 195 / 232 / 205 / 238 / 290 / 420.
+struct PrefillCost { double lat, sat; };
+constexpr PrefillCost kPrefillCost[3][kPrefillShapeCount] = {
+    {{3.15, 4.1}, {1.85, 2.2}, {1.1, 1.14}, {0.95, 0.66}, {1.1, 0.83}, {0.8, 0.475}, {1.55, 0.71}},     // codes on the operand side
+    {{1e9, 1e9},  {2.25, 2.4}, {1.65, 1.65}, {0.95, 0.76}, {1.25, 0.9}, {0.85, 0.56}, {1.6, 0.8}},      // bf16 under group scales: two sets of accumulators
+    {{1e9, 1e9},  {2.6, 3.8}, {1.6, 2.1}, {1.05, 1.0}, {1.55, 1.07}, {1.1, 0.64}, {2.0, 1.11}},         // 16-bit weights
+};
+int pick_shape(const GemmParams& p, int wbits, double* t_best) {
+    const PrefillCost* cost = kPrefillCost[wbits == 16 ? 2 : (p.bf16 && wbits == 4) ? 1 : 0];
+    int best = 1;
+    *t_best = 1e30;
+    for (int i = (p.bf16 || wbits == 16) ? 1 : 0; i < kPrefillShapeCount; ++i) {
+        const PrefillShape s = kPrefillShapes[i];
+        const double full = (double)cdiv(p.NT, 8 / s.ks * s.tpw) * cdiv(p.M, 16 * s.mb) / 256.0;
+        const double whole = (double)(long)(full + 0.9999), share = cost[i].sat * 0.5 * (full + whole);
+        const double t = cdiv(p.KC, s.ks) * (share > cost[i].lat ? share : cost[i].lat) + 2.5;
+        if (t < *t_best) { *t_best = t; best = i; }
+    }
+    return best;
+}
+
+template <int WBITS, int GS, bool BF, int I>
+void launch_shape_t(const GemmParams& p, hipStream_t st) {
+    constexpr PrefillShape s = kPrefillShapes[I];
+    const dim3 grid(cdiv(p.NT, 8 / s.ks * s.tpw), cdiv(p.M, 16 * s.mb));
+    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks>), grid, dim3(512), 0, st, p);
+}
+template <int WBITS, int GS, bool BF>
+int launch_shape(int i, const GemmParams& p, hipStream_t st) {
+    switch (i) {
+        case 0: if constexpr (!BF && WBITS != 16) { launch_shape_t<WBITS, GS, BF, 0>(p, st); break; } return MI355_ERR_UNSUPPORTED;
+        case 1: launch_shape_t<WBITS, GS, BF, 1>(p, st); break;
+        case 2: launch_shape_t<WBITS, GS, BF, 2>(p, st); break;
+        case 3: launch_shape_t<WBITS, GS, BF, 3>(p, st); break;
+        case 4: launch_shape_t<WBITS, GS, BF, 4>(p, st); break;
+        case 5: launch_shape_t<WBITS, GS, BF, 5>(p, st); break;
+        case 6: launch_shape_t<WBITS, GS, BF, 6>(p, st); break;
+        default: return MI355_ERR_UNSUPPORTED;
+    }
     MI355_CHECK_LAUNCH("gemm_prefill_kernel");
     return MI355_OK;
 }
@@ -206,16 +336,22 @@ int launch_prefill_t(const GemmParams& p, hipStream_t st) {
 } // namespace
 
 // Direct-mode launch (fused epilogue in p.mode).  MI355_ERR_UNSUPPORTED: shape / format not covered, caller falls back.
-extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, mi355_stream_t stream) {
+// t_limit: the caller's estimate (us) for its other path; a launch expected to take longer is not made (MI355_ERR_UNSUPPORTED).
+extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, double t_limit, mi355_stream_t stream) {
     const GemmParams& g = *reinterpret_cast<const GemmParams*>(gp);
-    if (g.M < 128 || g.mode == MODE_PARTIAL || g.mode == MODE_F32) return MI355_ERR_UNSUPPORTED;
+    if (g.M <= 64 || g.mode == MODE_PARTIAL || g.mode == MODE_F32) return MI355_ERR_UNSUPPORTED;
     if ((uint64_t)g.M * g.K * 2 >= 0x7FFFFFF0ull) return MI355_ERR_UNSUPPORTED;       // x image must stay below the OOB offset
     hipStream_t st = (hipStream_t)stream;
+    const bool bf = g.bf16 != 0;
+    double t;
+    const int s = pick_shape(g, wbits, &t);
+    if (t > t_limit) return MI355_ERR_UNSUPPORTED;
+    if (wbits == 16) return bf ? launch_shape<16, 0, true>(s, g, st) : launch_shape<16, 0, false>(s, g, st);
+    if (wbits == 8 && group_size == 0) return bf ? launch_shape<8, 0, true>(s, g, st) : launch_shape<8, 0, false>(s, g, st);
     if (wbits == 4) {
-        if (group_size == 128) return launch_prefill_t<4, 4>(g, st);
-        if (group_size == 64) return launch_prefill_t<4, 2>(g, st);
-        if (group_size == 32) return launch_prefill_t<4, 1>(g, st);
+        if (group_size == 128) return bf ? launch_shape<4, 4, true>(s, g, st) : launch_shape<4, 4, false>(s, g, st);
+        if (group_size == 64) return bf ? launch_shape<4, 2, true>(s, g, st) : launch_shape<4, 2, false>(s, g, st);
+        if (group_size == 32) return bf ? launch_shape<4, 1, true>(s, g, st) : launch_shape<4, 1, false>(s, g, st);
     }
-    if (wbits == 8 && group_size == 0) return launch_prefill_t<8, 0>(g, st);
     return MI355_ERR_UNSUPPORTED;
 }

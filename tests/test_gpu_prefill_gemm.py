@@ -1,0 +1,70 @@
+"""The GEMM of prefill chunks at the edges of its block shapes: more than 64 rows, remainders of the row, column and K tiles, every operand form, against a
+64-bit product with a bound built from the formats: half an ulp of the output, plus 2^-11 sum |x w| where fp16 rounds s (u - z) to the operand (fp16 W4), plus
+the fp32 sums (K terms of at most 2^-24 sum |x w|, far from all of one sign: 2^-18)."""
+import pytest
+import torch
+
+from rtp_llm_amd import _C, model, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _gen(seed):
+    return torch.Generator().manual_seed(seed)
+
+
+def _dense64(c):
+    if c.kind == "fp16":
+        return c.w.double()
+    if c.kind == "int8":
+        return c.q.double() * c.scales.double()
+    g = c.group_size
+    return ((c.q.double().view(-1, g, c.N) - c.z_eff.double()[:, None]) * c.scales.double()[:, None]).view(c.K, c.N)
+
+
+# the shapes of a call go from 32 x 32 tiles on four K slices (narrow, deep, few rows) to 128 x 512 (many rows, wide)
+SHAPES = [(65, 136, 24), (66, 4864, 64), (129, 1280, 200), (130, 896, 1152), (257, 640, 4096), (513, 384, 9728), (1100, 256, 8208)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,group", [("w4", 128), ("w4", 64), ("w4", 32), ("int8", 0), ("fp16", 0)])
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_prefill_gemm_shapes(kind, group, dtype, M, K, N):
+    if group and K % group:
+        K = -(-K // group) * group
+    c = model.synth_linear(K, N, kind, "cpu", _gen(K + N), group or 128)
+    if kind == "fp16":
+        c.w = c.w.to(dtype)
+    x = (torch.randn(M, K, generator=_gen(M)) * 0.5).to(dtype)
+    bias = (torch.randn(N, generator=_gen(3)) * 0.1).to(dtype)
+    w = _dense64(c)
+    ref = x.double() @ w + bias.double()
+    mag = x.double().abs() @ w.abs()
+    y = ops.linear(x.to(DEV), c.pack(dtype=dtype).to(DEV), bias.to(DEV)).cpu().double()
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10      # spacing at 1: 8 and 11 significant bits
+    bound = ulp / 2 * 1.01 * ref.abs() + (2.0 ** -11 if kind == "w4" and dtype == torch.float16 else 0.0) * mag + 2.0 ** -18 * mag + 1e-6
+    over = (y - ref).abs() / bound
+    assert float(over.max()) <= 1.0, (float(over.max()), float((y - ref).abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["w4", "int8", "fp16"])
+def test_prefill_gemm_silu_pairs(kind, dtype):
+    """The gate-up epilogue on the same launches, rows independent of how many there are."""
+    M, K, I = 195, 896, 608
+    c = model.synth_linear(K, 2 * I, kind, "cpu", _gen(5))
+    if kind == "fp16":
+        c.w = c.w.to(dtype)
+    x = (torch.randn(M, K, generator=_gen(6)) * 0.5).to(dtype)
+    w = _dense64(c)
+    exact, mag = x.double() @ w, x.double().abs() @ w.abs()
+    gu = exact.to(dtype).double()
+    g, u = gu[:, :I], gu[:, I:]
+    act = g / (1 + torch.exp(-g))
+    y = ops.linear(x.to(DEV), c.pack(gate_up=True, dtype=dtype).to(DEV), None, _C.EPI_SILU_MUL).cpu().double()
+    # what each half of the pair may be off by: the sums' bound of the test above, then one spacing where a sum sits on a rounding boundary; |silu'| <= 1.1
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    off = (2.0 ** -11 if kind == "w4" and dtype == torch.float16 else 0.0) * mag + 2.0 ** -18 * mag + ulp * exact.abs()
+    bound = 1.1 * off[:, :I] * (u.abs() + off[:, I:]) + act.abs() * off[:, I:] + ulp * (act * u).abs() + 1e-6
+    assert float(((y - act * u).abs() / bound).max()) <= 1.0
