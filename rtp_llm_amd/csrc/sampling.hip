@@ -33,13 +33,13 @@ __device__ __forceinline__ float block_sum(float v, float* s_red) {
 }
 
 // Inverse-CDF draw from the unnormalised non-negative weights f(0..V-1): the first index j with f(j) > 0 whose inclusive
-// prefix sum, taken in index order, exceeds u01 * sum (V - 1 when rounding leaves none: sampling.cu:418).  Thread tx owns
+// prefix sum, taken in index order, exceeds u01 * sum (`none` when rounding leaves none; V - 1 in the reference: sampling.cu:418).  Thread tx owns
 // the contiguous segment [lo, hi) (a multiple of 4 long: segments start on 16-byte boundaries of an aligned row), so the block-level
 // prefix over threads is the prefix over indices.  Result in *s_found (valid for every thread after the call); returns sum.
 __device__ __forceinline__ int draw_segment(int V) { return (((V + kThreads - 1) / kThreads) + 3) & ~3; }
 
 template <class F>
-__device__ __forceinline__ float block_draw(F&& f, int V, float u01, float* s_red, float* s_scan, int* s_found) {
+__device__ __forceinline__ float block_draw(F&& f, int V, float u01, float* s_red, float* s_scan, int* s_found, int none) {
     const int tx = threadIdx.x;
     const int seg = draw_segment(V);
     const int lo = min(V, tx * seg), hi = min(V, lo + seg);
@@ -50,7 +50,7 @@ __device__ __forceinline__ float block_draw(F&& f, int V, float u01, float* s_re
     const float u = u01 * total;
     // inclusive prefix over threads (Hillis-Steele in LDS; 1024 entries)
     s_scan[tx] = local;
-    if (tx == 0) *s_found = V - 1;
+    if (tx == 0) *s_found = none;
     __syncthreads();
     for (int off = 1; off < kThreads; off <<= 1) {
         const float add = (tx >= off) ? s_scan[tx - off] : 0.f;
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kThreads) void rejection_sample_kernel(const Reject
         const float pv = dp ? dp[j] : (j == dtok ? 1.0f : 0.0f);
         return fmaxf(q[j] - pv, 0.f);
     };
-    block_draw(resid, p.V, p.uniform[row * G1 + min(pos + 1, G)], s_red, s_scan, &s_found);
+    block_draw(resid, p.V, p.uniform[row * G1 + min(pos + 1, G)], s_red, s_scan, &s_found, p.V - 1);
     if (tx == 0) {
         p.out_ids[row * G1 + pos] = s_found;
         for (int n = pos + 1; n < G1; ++n) p.out_ids[row * G1 + n] = -1;
@@ -162,8 +162,7 @@ __global__ __launch_bounds__(kThreads) void rejection_sample_kernel(const Reject
 
 // probs[r, :] = softmax(logits[r, :] / temperature), fp32 (the sampler's distribution; SpeculativeSampler.cc feeds
 // rejection sampling with these rows)
-__global__ __launch_bounds__(kThreads) void softmax_rows_kernel(const float* __restrict__ logits, int V, int ld, float inv_temp,
-                                                                float* __restrict__ probs) {
+__global__ __launch_bounds__(kThreads) void softmax_rows_kernel(const float* logits, int V, int ld, float inv_temp, float* probs) {
     __shared__ float s_red[kThreads / 64];
     const float* x = logits + (size_t)blockIdx.x * ld;
     float* y = probs + (size_t)blockIdx.x * V;
@@ -179,22 +178,23 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_kernel(const float* __r
     float s = 0.f;
     row_pass(x, V, vec, [&](float v) { s += __expf((v - m) * inv_temp); });
     s = block_sum(s, s_red);
+    // probs may be logits (every read of the sum is behind the block's barriers); 16-byte stores: the scalar loop took 45 of the 67 us of 64 rows of 152064
     const float inv = 1.f / s;
-    for (int j = threadIdx.x; j < V; j += kThreads) y[j] = __expf((x[j] - m) * inv_temp) * inv;
+    int done = 0;
+    if (vec && (V & 3) == 0 && (reinterpret_cast<uintptr_t>(probs) & 15) == 0) {
+        const f32x4* x4 = reinterpret_cast<const f32x4*>(x);
+        f32x4* y4 = reinterpret_cast<f32x4*>(y);
+        done = V;
+#pragma unroll 4
+        for (int j = threadIdx.x; j < V >> 2; j += kThreads) {
+            f32x4 v = x4[j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = __expf((v[r] - m) * inv_temp) * inv;
+            y4[j] = v;
+        }
+    }
+    for (int j = done + threadIdx.x; j < V; j += kThreads) y[j] = __expf((x[j] - m) * inv_temp) * inv;
 }
-
-// ids[r] = inverse-CDF sample of probs[r, :] with uniform[r] (the top_k = 0 / top_p = 1 branch of the sampler:
-// softmax, then sampling from the probabilities, bindings/core/CudaSampleOp.cc:702-737)
-__global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float* __restrict__ probs, int V, int ld,
-                                                               const float* __restrict__ uniform, int32_t* __restrict__ ids) {
-    __shared__ float s_red[kThreads / 64];
-    __shared__ float s_scan[kThreads];
-    __shared__ int   s_found;
-    const float* q = probs + (size_t)blockIdx.x * ld;
-    block_draw([&](int j) { return fmaxf(q[j], 0.f); }, V, uniform[blockIdx.x], s_red, s_scan, &s_found);
-    if (threadIdx.x == 0) ids[blockIdx.x] = s_found;
-}
-
 
 // (a, b) summed over the block in a fixed order (wave butterfly, then 16 partials added by every thread): deterministic.
 __device__ __forceinline__ void block_sum2(float& a, float& b, float (*s_pair)[2]) {
@@ -209,11 +209,12 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float (*s_pair)[2
     a = ta; b = tb;
 }
 
-// Temperature, then repetition / presence / frequency penalties, in place on fp32 logits: one block per row.
+// Temperature, then repetition / presence / frequency penalties, in place on fp32 logits.
 //   batchApplyTemperaturePenalty (sampling_penalty_kernels.cu:26-54): logit *= 1 / (T[row] + 1e-6)
 //   batchApplyPenaltyLongSeq (:129-180): every vocabulary id seen among output_ids[0 .. step)[row] (padding positions
 //   [input_length, max_input_length) skipped, ids outside [0, V) skipped) is penalised ONCE:
 //   logit = logit < 0 ? logit * rep : logit / rep;  logit -= presence;  logit -= frequency * count.
+// Temperature runs over the row in a launch of its own, the penalties in one behind it.
 struct PenaltyParams {
     float*         logits;
     int            V, ld;
@@ -221,45 +222,79 @@ struct PenaltyParams {
     const int32_t* output_ids;     // [step][batch]
     const int32_t* input_lengths;  // [batch] or null
     int            batch, max_input_length, step;
-    int32_t*       counts;         // [batch][V], zero on entry
+    int32_t*       counts;         // [batch][V]: histories of more than kShortHistory entries
 };
 
+// Temperature alone: blockIdx.x splits the row.  64 rows of 152064: 14 us, the copy rate of their 78 MB.
+__global__ __launch_bounds__(kThreads) void temperature_kernel(const PenaltyParams p) {
+    const int row = blockIdx.y, start = blockIdx.x * kThreads + threadIdx.x, stride = gridDim.x * kThreads;
+    float* x = p.logits + (size_t)row * p.ld;
+    const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
+    int done = 0;
+    if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0) {
+        f32x4* x4 = reinterpret_cast<f32x4*>(x);
+        const int V4 = p.V >> 2;
+#pragma unroll 4
+        for (int j = start; j < V4; j += stride) {
+            f32x4 v = x4[j];
+            v[0] *= inv_t; v[1] *= inv_t; v[2] *= inv_t; v[3] *= inv_t;
+            x4[j] = v;
+        }
+        done = V4 << 2;
+    }
+    for (int j = done + start; j < p.V; j += stride) x[j] *= inv_t;
+}
+
+__device__ __forceinline__ float penalised(const PenaltyParams& p, int row, float logit, int count) {
+    if (p.repetition) logit = logit < 0.0f ? logit * p.repetition[row] : logit / p.repetition[row];
+    if (p.presence) logit -= p.presence[row];
+    if (p.frequency) logit -= p.frequency[row] * (float)count;
+    return logit;
+}
+
+// History of at most kShortHistory entries, one block per row: the entries lie in LDS, the first entry of an id counts its equals and penalises it.  No
+// [batch][V] counters to clear (39 MB at 64 rows of 152064, more than all the other work of the launch).
+constexpr int kShortHistory = 2048;
+__global__ __launch_bounds__(256) void penalties_short_kernel(const PenaltyParams p) {
+    __shared__ __attribute__((aligned(16))) int s_tok[kShortHistory];
+    const int row = blockIdx.x, tx = threadIdx.x;
+    float* x = p.logits + (size_t)row * p.ld;
+    const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
+    const int padded = (p.step + 3) & ~3;
+    for (int i = tx; i < padded; i += 256) {
+        int tok = -1;                                       // nothing to penalise: padding, or an id outside the vocabulary
+        if (i < p.step && !(i >= input_length && i < p.max_input_length)) {
+            tok = p.output_ids[(size_t)i * p.batch + row];
+            if (tok >= p.V || tok < 0) tok = -1;
+        }
+        s_tok[i] = tok;
+    }
+    __syncthreads();
+    for (int i = tx; i < p.step; i += 256) {
+        const int tok = s_tok[i];
+        if (tok < 0) continue;
+        int count = 0, before = 0;
+        for (int j = 0; j < padded; j += 4) {
+            const int4 t = *reinterpret_cast<const int4*>(&s_tok[j]);
+            const int c = (t.x == tok) + (t.y == tok) + (t.z == tok) + (t.w == tok);
+            count += c;
+            if (j + 3 < i) before += c;
+            else before += (j < i && t.x == tok) + (j + 1 < i && t.y == tok) + (j + 2 < i && t.z == tok);
+        }
+        if (before == 0) x[tok] = penalised(p, row, x[tok], count);
+    }
+}
+
+// Longer histories: counters in memory, cleared by the first of two launches.
+__global__ __launch_bounds__(kThreads) void clear_counts_kernel(int32_t* counts, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads) counts[i] = 0;
+}
 __global__ __launch_bounds__(kThreads) void penalties_kernel(const PenaltyParams p) {
     const int row = blockIdx.x, tx = threadIdx.x;
     float* x = p.logits + (size_t)row * p.ld;
-    const bool pen = p.output_ids != nullptr;
-    int32_t* cnt = pen ? p.counts + (size_t)row * p.V : nullptr;
-    // ---- temperature: the whole row, 16-byte accesses
-    if (p.temperature) {
-        const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
-        int done = 0;
-        if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0) {
-            f32x4* x4 = reinterpret_cast<f32x4*>(x);
-            const int V4 = p.V >> 2;
-#pragma unroll 4
-            for (int j = tx; j < V4; j += kThreads) {
-                f32x4 v = x4[j];
-                v[0] *= inv_t; v[1] *= inv_t; v[2] *= inv_t; v[3] *= inv_t;
-                x4[j] = v;
-            }
-            done = V4 << 2;
-        }
-        for (int j = done + tx; j < p.V; j += kThreads) x[j] *= inv_t;
-    }
-    if (!pen) return;
-    // ---- penalties: count the ids of the history; the lane whose increment found a zero owns the id and penalises it once the
-    // counts are final -- the work is proportional to the history, not to the vocabulary (histories beyond 32 entries per lane
-    // fall back to a scan of the row)
-    const float rep = p.repetition ? p.repetition[row] : 1.0f, pres = p.presence ? p.presence[row] : 0.0f,
-                freq = p.frequency ? p.frequency[row] : 0.0f;
-    auto penalise = [&](int j, int c) {
-        // written by other lanes of this block (temperature pass above): read past the CU's vector cache
-        float logit = __uint_as_float(__hip_atomic_load(reinterpret_cast<uint32_t*>(x + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        if (p.repetition) logit = logit < 0.0f ? logit * rep : logit / rep;
-        if (p.presence) logit -= pres;
-        if (p.frequency) logit -= freq * (float)c;
-        x[j] = logit;
-    };
+    int32_t* cnt = p.counts + (size_t)row * p.V;
+    // count the ids of the history; the lane whose increment found a zero owns the id and penalises it once the counts are final -- the work is
+    // proportional to the history, not to the vocabulary (histories beyond 32 entries per lane fall back to a scan of the row)
     const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
     uint32_t mine = 0;                                     // bit s: the s-th history entry of this lane was the first of its id
     int s = 0;
@@ -276,12 +311,12 @@ __global__ __launch_bounds__(kThreads) void penalties_kernel(const PenaltyParams
         for (int index = tx; index < p.step; index += kThreads, ++s) {
             if (!((mine >> s) & 1u)) continue;
             const int tok = p.output_ids[(size_t)index * p.batch + row];
-            penalise(tok, __hip_atomic_load(&cnt[tok], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            x[tok] = penalised(p, row, x[tok], __hip_atomic_load(&cnt[tok], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         }
     } else {
         for (int j = tx; j < p.V; j += kThreads) {
             const int c = __hip_atomic_load(&cnt[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (c > 0) penalise(j, c);
+            if (c > 0) x[j] = penalised(p, row, x[j], c);
         }
     }
 }
@@ -293,8 +328,13 @@ __global__ __launch_bounds__(kThreads) void penalties_kernel(const PenaltyParams
 //       its equals: with S = mass of all strictly larger entries, its j-th occurrence stays while S + j v <= p;
 //   the survivors are renormalised by max(sum, 1e-10) (probs_out, optional) and one index is drawn by inverse CDF in index order
 //   with uniform[row] (torch.multinomial in the reference: same distribution, explicit randomness).
-// No sort: both thresholds are built bit by bit from the top of the fp32 pattern (non-negative floats order like their bits), one
-// pass over the row and one fixed-order block reduction per bit.
+// No sort.  What bounds it is the number of passes over the row: bit by bit from the top of the fp32 pattern (non-negative floats order like their bits) the
+// two thresholds took 31 passes of 24 us over 152064 values on one CU.  A histogram of the pattern's top 12 bits (a sixteenth of an octave per bin) with the
+// count and the mass of every bin names the one bin each threshold lies in; the values of those two bins go to LDS and the low 19 bits are searched there.  The
+// values of a bin share their exponent, so its mass is a sum of integers, exact whatever the order of the atomics, and packs with the count into one 64-bit
+// word: one LDS atomic a value.  The draw reads the row twice more, a wave per contiguous sixteenth.  Rows whose boundary bin holds more than kSet values (flat
+// rows, long runs of one value) are searched bit by bit as before.
+// 64 rows of 152064, top-k 0..100, top-p 0.8..0.95 of a distribution with a heavy tail: 827 -> 97 us.
 struct TopKPParams {
     const float*   probs;
     int            V, ld;
@@ -306,91 +346,343 @@ struct TopKPParams {
     int            ld_out;
 };
 
-__global__ __launch_bounds__(kThreads) void top_k_top_p_sample_kernel(const TopKPParams p) {
-    __shared__ float s_red[kThreads / 64];
-    __shared__ float s_pair[kThreads / 64][2];
-    __shared__ float s_scan[kThreads];
-    __shared__ int   s_found;
-    const int row = blockIdx.x, tx = threadIdx.x, V = p.V;
-    const float* q = p.probs + (size_t)row * p.ld;
-    auto pos = [](float v) { return v > 0.f ? v : 0.f; };   // +0 for -0, negatives and NaN: the bit pattern is the order
-    int k = p.top_k ? p.top_k[row] : 0;
-    const bool use_k = k > 0 && k < V;
-    float tp = p.top_p ? p.top_p[row] : 1.0f;
-    if (fabsf(tp) < 1e-7f) tp = 1.0f;
-    bool use_p = fabsf(tp - 1.0f) >= 1e-7f;
-    uint32_t tk = 0, tq = 0;   // tk: largest t with #(bits >= t) >= k;  tq: largest t with mass(bits > t) > p
-    const bool vec = ((p.ld & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.probs) & 15) == 0);
-    if (use_p) {               // nothing to drop when even the mass above 0 fits
-        float m = 0.f, z = 0.f;
-        row_pass(q, V, vec, [&](float x) { m += pos(x); });
-        block_sum2(m, z, s_pair);
-        use_p = m > tp;
+constexpr int kSet = 4096, kBinShift = 19, kBins = 1 << (31 - kBinShift), kWaves = kThreads / 64;
+
+struct SampleShared {
+    float    red[kWaves];
+    float    pair[kWaves][2];
+    float    scan[kThreads];
+    unsigned long long hist[kBins];          // count << 40 | sum of the low 19 bits
+    uint32_t set_k[kSet], set_q[kSet];
+    int      n_k, n_q, bin_k, bin_q, found;
+    uint32_t above_k;                        // entries in the bins above bin_k
+    double   above_q;                        // mass in the bins above bin_q
+    uint32_t wave_n[kWaves];
+    unsigned long long wave_m[kWaves];
+    double   wave_d[kWaves];
+};
+
+__device__ __forceinline__ float sample_pos(float v) { return v > 0.f ? v : 0.f; }   // +0 for -0, negatives and NaN: the bit pattern is the order
+
+// four values of a row from index j on; past its end: zeros
+__device__ __forceinline__ f32x4 row4(const float* q, int j, int end, bool vec) {
+    if (vec && j + 3 < end) return *reinterpret_cast<const f32x4*>(q + j);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) if (j + r < end) v[r] = q[j + r];
+    return v;
+}
+
+// sum over the wave without the LDS crossbar (row operations, then the swaps of 16 and 32 lanes): every lane gets it
+__device__ __forceinline__ float lane_sum(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, true));
+    return xor32_sum(xor16_sum(v));
+}
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+// One index of the row by inverse CDF over w(value), one contiguous run of the row per wave: the runs' sums, their prefix, and a second walk of the run that
+// holds u.  The same rule as block_draw (a run that the rounding of the second walk leaves without a crossing gives its last index of positive weight).
+template <class W>
+__device__ __forceinline__ float row_draw(const float* q, int V, bool vec, float u01, SampleShared& sh, W&& weight) {
+    const int tx = threadIdx.x, lane = tx & 63, wave = tx >> 6;
+    const int chunk = ((V + kWaves - 1) / kWaves + 255) & ~255;                 // 256 values per step
+    const int w0 = min(V, wave * chunk), w1 = min(V, w0 + chunk);
+    float s = 0.f;
+#pragma unroll 4
+    for (int j = w0 + lane * 4; j < w1; j += 256) {
+        const f32x4 v = row4(q, j, w1, vec);
+        s += (weight(v[0]) + weight(v[1])) + (weight(v[2]) + weight(v[3]));
     }
-    if (use_k || use_p) {
-        for (int bit = 30; bit >= 0; --bit) {
-            const uint32_t ck = tk | (1u << bit), cq = tq | (1u << bit);
-            float cnt = 0.f, mass = 0.f;
-            row_pass(q, V, vec, [&](float x) {
-                const float v = pos(x);
-                const uint32_t b = __float_as_uint(v);
-                cnt += (b >= ck) ? 1.f : 0.f;
-                mass += (b > cq) ? v : 0.f;
-            });
-            block_sum2(cnt, mass, s_pair);
-            if (use_k && cnt >= (float)k) tk = ck;
-            if (use_p && mass > tp) tq = cq;
+    s = lane_sum(s);
+    if (lane == 0) sh.red[wave] = s;
+    if (tx == 0) sh.found = V - 1;
+    __syncthreads();
+    float total = 0.f, excl = 0.f;
+    for (int w = 0; w < kWaves; ++w) { if (w == wave) excl = total; total += sh.red[w]; }
+    const float u = u01 * total, incl = excl + s;
+    if (s > 0.f && excl <= u && incl > u) {                                     // the same for every lane of the wave
+        float c = excl;
+        int hit = -1, last = -1;
+        for (int j = w0 + lane * 4; j - lane * 4 < w1; j += 256) {
+            const f32x4 v = row4(q, j, w1, vec);
+            float t[4], mine = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { t[r] = weight(v[r]); mine += t[r]; }
+            const unsigned long long any = __ballot(mine > 0.f);
+            if (any == 0ull) continue;
+            float pre = mine;                                                   // inclusive over the lanes
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) { const float y = __shfl_up(pre, o); if (lane >= o) pre += y; }
+            float at = c + (pre - mine);
+            int h = -1;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { at += t[r]; if (t[r] > 0.f && h < 0 && at > u) h = j + r; }
+            const unsigned long long crossed = __ballot(h >= 0);
+            if (crossed) { hit = __shfl(h, __ffsll((unsigned long long)crossed) - 1); break; }
+            int l = -1;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) if (t[r] > 0.f) l = j + r;
+            last = __shfl(l, 63 - __clzll((long long)any));
+            c += __shfl(pre, 63);
         }
+        if (lane == 0) sh.found = hit >= 0 ? hit : last;
     }
-    // top-p boundary value vb = tq + 1 (an entry's value: the mass above a threshold only changes at entries).  Its equals are
-    // ranked in index order over the contiguous segments block_draw uses; `cut` = first index of this thread's segment from
-    // which they are dropped.
-    const uint32_t kb = use_k ? tk : 0u, vbits = use_p ? tq + 1u : 0u;
+    __syncthreads();
+    return total;
+}
+
+// The filter and the draw over the row with equals of the top-p boundary value dropped from some index on; kept(j), for j of this thread's segment
+// [lo, hi), is what stays of value j.
+template <class Out>
+__device__ __forceinline__ void filter_and_draw(const float* q, int V, uint32_t kb, uint32_t vbits, bool use_p, float tp, float u, SampleShared& sh, Out&& out) {
+    const int tx = threadIdx.x;
+    // top-p boundary value (an entry's value: the mass above a threshold only changes at entries).  Its equals are ranked in index order over the
+    // contiguous segments block_draw uses; `cut` = first index of this thread's segment from which they are dropped.
     const int seg = draw_segment(V);
     const int lo = min(V, tx * seg), hi = min(V, lo + seg);
     int cut = hi;
     if (use_p) {
         float sb = 0.f, ties = 0.f;
         for (int j = lo; j < hi; ++j) {
-            const float v = pos(q[j]);
+            const float v = sample_pos(q[j]);
             const uint32_t b = __float_as_uint(v);
             sb += (b > vbits) ? v : 0.f;
             ties += (b == vbits) ? 1.f : 0.f;
         }
         const float mine = ties;
         float z = 0.f;
-        block_sum2(sb, z, s_pair);
-        s_scan[tx] = mine;                       // inclusive scan of the tie counts over threads (exact: counts < 2^24)
+        block_sum2(sb, z, sh.pair);
+        sh.scan[tx] = mine;                       // inclusive scan of the tie counts over threads (exact: counts < 2^24)
         __syncthreads();
         for (int off = 1; off < kThreads; off <<= 1) {
-            const float add = (tx >= off) ? s_scan[tx - off] : 0.f;
+            const float add = (tx >= off) ? sh.scan[tx - off] : 0.f;
             __syncthreads();
-            s_scan[tx] += add;
+            sh.scan[tx] += add;
             __syncthreads();
         }
-        float rank = s_scan[tx] - mine;
+        float rank = sh.scan[tx] - mine;
         __syncthreads();
         const float vb = __uint_as_float(vbits);
         for (int j = lo; j < hi; ++j) {
-            if (__float_as_uint(pos(q[j])) != vbits) continue;
+            if (__float_as_uint(sample_pos(q[j])) != vbits) continue;
             if (sb + rank * vb > tp) { cut = j; break; }
             rank += 1.f;
         }
     }
     auto kept = [&](int j) {      // j inside this thread's segment
-        const float v = pos(q[j]);
+        const float v = sample_pos(q[j]);
         const uint32_t b = __float_as_uint(v);
         return (b >= kb && (b > vbits || (b == vbits && j < cut))) ? v : 0.f;
     };
-    const float total = block_draw(kept, V, p.uniform[row], s_red, s_scan, &s_found);
-    if (tx == 0) p.ids[row] = s_found;
-    if (p.probs_out) {
-        const float den = fmaxf(total, 1e-10f);
-        float* y = p.probs_out + (size_t)row * p.ld_out;
-        for (int j = lo; j < hi; ++j) y[j] = kept(j) / den;
+    const float total = block_draw(kept, V, u, sh.red, sh.scan, &sh.found, V - 1);
+    out(kept, lo, hi, total);
+}
+
+// Both thresholds from the histogram: kb = the k-th largest value's bits (0: every entry), vbits = the smallest value's bits that top-p keeps.  use_p is cleared when the
+// whole row's mass fits.  Returns 0 when the row has to be searched bit by bit, 1 when all equals of the boundary value stay, 2 when some of them go.
+__device__ __forceinline__ int search_histogram(const float* q, int V, bool vec, bool use_k, int k, bool& use_p, float tp, uint32_t& kb, uint32_t& vbits,
+                                                SampleShared& sh) {
+    const int tx = threadIdx.x, lane = tx & 63, wave = tx >> 6;
+    constexpr uint32_t LOW = (1u << kBinShift) - 1u;
+    if (V > (1 << 20) || (use_p && tp < 0.f)) return 0;                         // the packed sums hold 2^21 values
+    for (int i = tx; i < kBins; i += kThreads) sh.hist[i] = 0ull;
+    if (tx == 0) { sh.n_k = sh.n_q = 0; sh.bin_k = sh.bin_q = -1; }
+    __syncthreads();
+    row_pass(q, V, vec, [&](float x) {
+        const uint32_t b = __float_as_uint(sample_pos(x));
+        if (b != 0u) atomicAdd(&sh.hist[b >> kBinShift], (1ull << 40) + (unsigned long long)(b & LOW));
+    });
+    __syncthreads();
+    // from the largest values down: a thread takes kBins / kThreads bins, prefixes over the lanes and the waves
+    constexpr int PB = kBins / kThreads;
+    uint32_t c[PB], ci = 0;
+    double m[PB], mi = 0.0;
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+        const int bin = kBins - 1 - (tx * PB + i), e = bin >> (23 - kBinShift);
+        const unsigned long long h = sh.hist[bin];
+        c[i] = (uint32_t)(h >> 40);
+        m[i] = (double)c[i] * (double)__uint_as_float((uint32_t)bin << kBinShift) + (double)(h & ((1ull << 40) - 1ull)) * __builtin_ldexp(1.0, (e ? e : 1) - 150);
+        if (c[i] == 0u) m[i] = 0.0;
+        if (bin >= (0x7F800000 >> kBinShift) && c[i]) sh.bin_k = -2;            // an infinity
+        ci += c[i]; mi += m[i];
+    }
+    const uint32_t c_own = ci;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t yc = __shfl_up(ci, o);
+        const double ym = __shfl_up(mi, o);
+        if (lane >= o) { ci += yc; mi += ym; }
+    }
+    if (lane == 63) { sh.wave_n[wave] = ci; sh.wave_d[wave] = mi; }
+    __syncthreads();
+    if (sh.bin_k == -2) return 0;
+    uint32_t c_at = ci - c_own;
+    double m_at = 0.0, total = 0.0;
+    for (int w = 0; w < kWaves; ++w) {
+        if (w < wave) c_at += sh.wave_n[w];
+        if (w == wave) m_at = total;
+        total += sh.wave_d[w];
+    }
+    const double m_lane = __shfl_up(mi, 1);
+    if (lane > 0) m_at += m_lane;
+    if (use_p) use_p = total > (double)tp;                                      // nothing to drop when even the mass above 0 fits
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+        const int bin = kBins - 1 - (tx * PB + i);
+        if (use_k && c_at < (uint32_t)k && c_at + c[i] >= (uint32_t)k) { sh.bin_k = bin; sh.above_k = c_at; }
+        if (use_p && m_at <= (double)tp && m_at + m[i] > (double)tp) { sh.bin_q = bin; sh.above_q = m_at; }
+        c_at += c[i]; m_at += m[i];
+    }
+    __syncthreads();
+    const int bin_k = use_k ? sh.bin_k : -1, bin_q = use_p ? sh.bin_q : -1;     // bin_k -1: fewer than k entries are above zero
+    if (use_p && bin_q < 0) return 0;                                           // the sums crossed p between a thread's last bin and the next thread's first
+    kb = 0; vbits = 0;
+    if (bin_k < 0 && bin_q < 0) return 1;
+    row_pass(q, V, vec, [&](float x) {
+        const uint32_t b = __float_as_uint(sample_pos(x));
+        const int bin = (int)(b >> kBinShift);
+        if (b == 0u) return;
+        if (bin == bin_k) { const int at = atomicAdd(&sh.n_k, 1); if (at < kSet) sh.set_k[at] = b; }
+        if (bin == bin_q) { const int at = atomicAdd(&sh.n_q, 1); if (at < kSet) sh.set_q[at] = b; }
+    });
+    __syncthreads();
+    const int n_k = sh.n_k, n_q = sh.n_q;
+    if (n_k > kSet || n_q > kSet) return 0;
+    // low bits, most significant first: the largest threshold that leaves k entries (more mass than p) at or above it.  The sets lie in registers.
+    constexpr int PT = kSet / kThreads;
+    const int e_q = max(bin_q, 0) >> (23 - kBinShift);
+    const uint32_t implicit = e_q ? 0x800000u : 0u;
+    const double unit = __builtin_ldexp(1.0, (e_q ? e_q : 1) - 150);
+    uint32_t vk[PT], vq[PT];
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+        const int j = tx + i * kThreads;
+        vk[i] = j < n_k ? sh.set_k[j] : 0u;
+        vq[i] = j < n_q ? sh.set_q[j] : 0u;
+    }
+    auto mantissa = [&](uint32_t b) { return (unsigned long long)((b & 0x7FFFFFu) | implicit); };
+    if (bin_k >= 0) kb = (uint32_t)bin_k << kBinShift;
+    if (bin_q >= 0) vbits = (uint32_t)bin_q << kBinShift;
+    const uint32_t above_k = sh.above_k;
+    const double above_q = sh.above_q;
+    for (int bit = kBinShift - 1; bit >= 0; --bit) {
+        const uint32_t ck = kb | (1u << bit), cq = vbits | (1u << bit);
+        uint32_t cnt = 0;
+        unsigned long long mass = 0;
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            cnt += (uint32_t)__popcll(__ballot(vk[i] >= ck));
+            if (vq[i] >= cq) mass += mantissa(vq[i]);
+        }
+        if (bin_q >= 0) mass = wave_sum_u64(mass);
+        if (lane == 0) { sh.wave_n[wave] = cnt; sh.wave_m[wave] = mass; }
+        __syncthreads();
+        cnt = above_k; mass = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) { cnt += sh.wave_n[w]; mass += sh.wave_m[w]; }
+        __syncthreads();
+        if (bin_k >= 0 && cnt >= (uint32_t)k) kb = ck;
+        if (bin_q >= 0 && above_q + (double)mass * unit > (double)tp) vbits = cq;
+    }
+    if (bin_q < 0) return 1;
+    // equals of the boundary value: the j-th of T stays while S + j v <= p, S = the mass above it
+    uint32_t ties = 0;
+    unsigned long long mass = 0;
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+        ties += (uint32_t)__popcll(__ballot(vq[i] == vbits && vq[i] != 0u));
+        if (vq[i] > vbits) mass += mantissa(vq[i]);
+    }
+    mass = wave_sum_u64(mass);
+    if (lane == 0) { sh.wave_n[wave] = ties; sh.wave_m[wave] = mass; }
+    __syncthreads();
+    ties = 0; mass = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) { ties += sh.wave_n[w]; mass += sh.wave_m[w]; }
+    __syncthreads();
+    return ties <= 1u || above_q + (double)(mass + (unsigned long long)(ties - 1u) * mantissa(vbits)) * unit <= (double)tp ? 1 : 2;
+}
+
+__global__ __launch_bounds__(kThreads) void top_k_top_p_sample_kernel(const TopKPParams p) {
+    __shared__ SampleShared sh;
+    const int row = blockIdx.x, tx = threadIdx.x, V = p.V;
+    const float* q = p.probs + (size_t)row * p.ld;
+    const int k = p.top_k ? p.top_k[row] : 0;
+    const bool use_k = k > 0 && k < V;
+    float tp = p.top_p ? p.top_p[row] : 1.0f;
+    if (fabsf(tp) < 1e-7f) tp = 1.0f;
+    bool use_p = fabsf(tp - 1.0f) >= 1e-7f;
+    const bool vec = ((p.ld & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.probs) & 15) == 0);
+    uint32_t kb = 0, vbits = 0;
+    int how = 1;                                       // 0: bit by bit over the row, 1: kept are the values at or above kb and vbits, 2: some equals of vbits go
+    if (use_k || use_p) {
+        how = search_histogram(q, V, vec, use_k, k, use_p, tp, kb, vbits, sh);
+        if (how == 0) {
+            use_p = fabsf(tp - 1.0f) >= 1e-7f;
+            if (use_p) {                               // nothing to drop when even the mass above 0 fits
+                float m = 0.f, z = 0.f;
+                row_pass(q, V, vec, [&](float x) { m += sample_pos(x); });
+                block_sum2(m, z, sh.pair);
+                use_p = m > tp;
+            }
+            uint32_t tk = 0, tq = 0;                   // tk: largest t with #(bits >= t) >= k;  tq: largest t with mass(bits > t) > p
+            if (use_k || use_p) {
+                for (int bit = 30; bit >= 0; --bit) {
+                    const uint32_t ck = tk | (1u << bit), cq = tq | (1u << bit);
+                    float cnt = 0.f, mass = 0.f;
+                    row_pass(q, V, vec, [&](float x) {
+                        const float v = sample_pos(x);
+                        const uint32_t b = __float_as_uint(v);
+                        cnt += (b >= ck) ? 1.f : 0.f;
+                        mass += (b > cq) ? v : 0.f;
+                    });
+                    block_sum2(cnt, mass, sh.pair);
+                    if (use_k && cnt >= (float)k) tk = ck;
+                    if (use_p && mass > tp) tq = cq;
+                }
+            }
+            kb = use_k ? tk : 0u; vbits = use_p ? tq + 1u : 0u;
+            how = 2;
+        }
+    }
+    float* y = p.probs_out ? p.probs_out + (size_t)row * p.ld_out : nullptr;
+    if (how == 1) {
+        const uint32_t floor_bits = max(kb, vbits);
+        auto weight = [&](float x) { const float v = sample_pos(x); return __float_as_uint(v) >= floor_bits ? v : 0.f; };
+        const float total = row_draw(q, V, vec, p.uniform[row], sh, weight);
+        if (tx == 0) p.ids[row] = sh.found;
+        if (y) {
+            const float den = fmaxf(total, 1e-10f);
+            for (int j = tx; j < V; j += kThreads) y[j] = weight(q[j]) / den;
+        }
+    } else {
+        filter_and_draw(q, V, kb, vbits, use_p, tp, p.uniform[row], sh, [&](auto& kept, int lo, int hi, float total) {
+            if (tx == 0) p.ids[row] = sh.found;
+            if (!y) return;
+            const float den = fmaxf(total, 1e-10f);
+            for (int j = lo; j < hi; ++j) y[j] = kept(j) / den;
+        });
     }
 }
 
+
+// ids[r] = inverse-CDF sample of probs[r, :] with uniform[r] (the top_k = 0 / top_p = 1 branch of the sampler:
+// softmax, then sampling from the probabilities, bindings/core/CudaSampleOp.cc:702-737)
+__global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float* __restrict__ probs, int V, int ld,
+                                                               const float* __restrict__ uniform, int32_t* __restrict__ ids) {
+    __shared__ SampleShared sh;
+    const bool vec = ((ld & 3) == 0) && ((reinterpret_cast<uintptr_t>(probs) & 15) == 0);
+    row_draw(probs + (size_t)blockIdx.x * ld, V, vec, uniform[blockIdx.x], sh, [](float v) { return fmaxf(v, 0.f); });
+    if (threadIdx.x == 0) ids[blockIdx.x] = sh.found;
+}
 
 // no_repeat_ngram_size: ban_repeat_ngram (bindings/common/kernels/banRepeatNgram.cu:30-136, greedy case beam_width = 1; called from
 // CudaSampleOp.cc:242-283).  With N = last_index[row] + 1 tokens so far and n = ngram[row]: every position i <= N - n whose n - 1
@@ -464,17 +756,24 @@ extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t 
     MI355_CHECK_ARG(!pen || (output_ids && penalty_ws && step >= 0 && max_input_length >= 0),
                     "apply_penalties: penalties need output_ids [step][batch] and a [batch][V] int32 workspace");
     if (!pen && !temperature) return MI355_OK;
-    if (pen) {
-        if (hipMemsetAsync(penalty_ws, 0, (size_t)batch_size * V * sizeof(int32_t), (hipStream_t)stream) != hipSuccess) {
-            (void)hipGetLastError();
-            mi355_set_error("apply_penalties: hipMemsetAsync failed");
-            return MI355_ERR_HIP;
-        }
-    }
     PenaltyParams p{logits, V, ld, temperature, repetition_penalty, presence_penalty, frequency_penalty,
                     pen ? output_ids : nullptr, input_lengths, batch_size, max_input_length, step, penalty_ws};
-    hipLaunchKernelGGL(penalties_kernel, dim3(batch_size), dim3(kThreads), 0, (hipStream_t)stream, p);
-    MI355_CHECK_LAUNCH("penalties_kernel");
+    hipStream_t st = (hipStream_t)stream;
+    if (temperature) {
+        const int split = batch_size >= 256 ? 1 : batch_size >= 32 ? 8 : 16;
+        hipLaunchKernelGGL(temperature_kernel, dim3(split, batch_size), dim3(kThreads), 0, st, p);
+        MI355_CHECK_LAUNCH("temperature_kernel");
+    }
+    if (pen && step > kShortHistory) {
+        const size_t n = (size_t)batch_size * V;
+        hipLaunchKernelGGL(clear_counts_kernel, dim3((unsigned)(n / (16 * kThreads) < 1024 ? n / (16 * kThreads) + 1 : 1024)), dim3(kThreads), 0, st, penalty_ws, n);
+        MI355_CHECK_LAUNCH("clear_counts_kernel");
+        hipLaunchKernelGGL(penalties_kernel, dim3(batch_size), dim3(kThreads), 0, st, p);
+        MI355_CHECK_LAUNCH("penalties_kernel");
+    } else if (pen && step > 0) {
+        hipLaunchKernelGGL(penalties_short_kernel, dim3(batch_size), dim3(256), 0, st, p);
+        MI355_CHECK_LAUNCH("penalties_short_kernel");
+    }
     return MI355_OK;
 }
 

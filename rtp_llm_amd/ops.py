@@ -441,11 +441,16 @@ def argmax(logits: torch.Tensor) -> torch.Tensor:
     return ids
 
 
-def softmax_rows(logits: torch.Tensor, temperature: float = 1.0) -> torch.Tensor:
-    """probs = softmax(logits / temperature) per row, fp32 (input of rejection sampling)."""
+def softmax_rows(logits: torch.Tensor, temperature: float = 1.0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """probs = softmax(logits / temperature) per row, fp32 (input of rejection sampling).  out: a tensor of the same shape that receives them
+    (it may be `logits`)."""
     _chk(logits, torch.float32, "softmax_rows.logits")
     R, V = logits.shape
-    probs = torch.empty_like(logits)
+    probs = torch.empty_like(logits) if out is None else out
+    if out is not None:
+        _chk(out, torch.float32, "softmax_rows.out")
+        if out.shape != logits.shape:
+            raise _C.Mi355Error(f"softmax_rows: out {tuple(out.shape)} for logits {tuple(logits.shape)}")
     _C.check(_C.lib().mi355_softmax_rows(logits.data_ptr(), R, V, V, float(temperature), probs.data_ptr(), _stream()), "softmax_rows")
     return probs
 
@@ -488,7 +493,7 @@ def apply_penalties(logits: torch.Tensor, temperature: Optional[torch.Tensor] = 
         _chk(output_ids, torch.int32, "apply_penalties.output_ids")
         if output_ids.dim() != 2 or output_ids.shape[1] != B or output_ids.shape[0] < step:
             raise _C.Mi355Error("apply_penalties: output_ids must be [>= step, B]")
-        ws = torch.empty(B, V, dtype=torch.int32, device=dev)
+        ws = torch.empty((B, V) if step > 2048 else (1,), dtype=torch.int32, device=dev)      # counters of long histories; short ones are counted on chip
     ptr = lambda t: t.data_ptr() if t is not None else None
     _C.check(_C.lib().mi355_apply_penalties(logits.data_ptr(), B, V, V, ptr(temp), ptr(rep), ptr(pres), ptr(freq), ptr(output_ids),
                                             ptr(lens), int(max_input_length), int(step), ptr(ws), _stream()), "apply_penalties")

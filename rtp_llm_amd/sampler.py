@@ -44,6 +44,18 @@ def _host(t: torch.Tensor, dtype) -> torch.Tensor:
     return t.detach().to(device="cpu", dtype=dtype)
 
 
+def _upload(tensors, device):
+    """The named host tensors of 32-bit values on the device, contiguous: packed into one buffer and sent in one copy."""
+    if not tensors:
+        return {}
+    flat = torch.cat([t.reshape(-1).view(torch.int32) for t in tensors.values()]).to(device)
+    out, at = {}, 0
+    for name, t in tensors.items():
+        out[name] = flat[at:at + t.numel()].view(t.dtype).view(t.shape)
+        at += t.numel()
+    return out
+
+
 def sample_greedy(params: GreedyParams) -> torch.Tensor:
     """-> the new token ids [batch_size] int32 on the GPU (also written to params.token_ids[:, step])."""
     logits = params.logits
@@ -52,23 +64,46 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
     step = int(params.step)
     if params.token_ids.shape != (B, step + 1):
         raise ValueError("sample_greedy: token_ids must be [batch_size, step + 1]")
-    transposed = params.token_ids.to(device=dev, dtype=torch.int32).t().contiguous()       # [step + 1, batch_size]
-
     temperature = _host(params.temperature, torch.float32)
-    if bool((temperature != 1.0).any()):
-        ops.apply_penalties(logits, temperature=temperature)
-
+    scale = bool((temperature != 1.0).any())
+    penalise = False
     if params.repetition_penalty is not None:
         if params.presence_penalty is None or params.frequency_penalty is None:
             raise ValueError("sample_greedy: repetition_penalty comes with presence_penalty and frequency_penalty")
         rep, pres, freq = (_host(t, torch.float32) for t in (params.repetition_penalty, params.presence_penalty, params.frequency_penalty))
-        if bool((rep != 1.0).any()) or bool((pres != 0.0).any()) or bool((freq != 0.0).any()):
-            lengths = _host(params.input_lengths, torch.int32).clone()
-            nd = params.sequence_lengths.numel()
-            if nd > 0:
-                lengths[:nd] = _host(params.sequence_lengths, torch.int32)
-            ops.apply_penalties(logits, repetition_penalty=rep, presence_penalty=pres, frequency_penalty=freq, output_ids=transposed,
-                                input_lengths=lengths, max_input_length=step + 1, step=step + 1)
+        penalise = bool((rep != 1.0).any()) or bool((pres != 0.0).any()) or bool((freq != 0.0).any())
+    top_k = _host(params.top_k, torch.int32)
+    all_greedy = bool((top_k == 1).all())
+    draw = not all_greedy
+    if draw and params.uniform is None:
+        raise ValueError("sample_greedy: sampling rows need params.uniform (one value in [0, 1) per row)")
+
+    # everything the step needs on the device that is on the host: one buffer, one copy
+    up = {}
+    if scale:
+        up["temperature"] = temperature
+    if penalise:
+        lengths = _host(params.input_lengths, torch.int32).clone()
+        nd = params.sequence_lengths.numel()
+        if nd > 0:
+            lengths[:nd] = _host(params.sequence_lengths, torch.int32)
+        up.update(rep=rep, pres=pres, freq=freq, lengths=lengths)
+        if params.token_ids.device.type == "cpu":
+            up["history"] = params.token_ids.to(torch.int32).t()                          # [step + 1, batch_size]
+    if draw:
+        top_p = _host(params.top_p, torch.float32).clone()
+        top_p[top_p.abs() < 1e-7] = 1.0
+        up.update(top_k=top_k, top_p=top_p)
+        if params.uniform.device.type == "cpu":
+            up["uniform"] = params.uniform.to(torch.float32)
+    up = _upload(up, dev)
+
+    if scale:
+        ops.apply_penalties(logits, temperature=up["temperature"])
+    if penalise:
+        transposed = up["history"] if "history" in up else params.token_ids.to(device=dev, dtype=torch.int32).t().contiguous()
+        ops.apply_penalties(logits, repetition_penalty=up["rep"], presence_penalty=up["pres"], frequency_penalty=up["freq"], output_ids=transposed,
+                            input_lengths=up["lengths"], max_input_length=step + 1, step=step + 1)
 
     if params.no_repeat_ngram_size is not None and params.sequence_lengths.numel() > 0:
         ngram = _host(params.no_repeat_ngram_size, torch.int32)
@@ -78,15 +113,10 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
             tokens = params.token_ids.to(device=dev, dtype=torch.int32).contiguous()
             ops.ban_repeat_ngram(logits, tokens[:nd], _host(params.sequence_lengths, torch.int32) - 1, ngram[:nd])
 
-    top_k = _host(params.top_k, torch.int32)
-    all_greedy = bool((top_k == 1).all())
     if all_greedy and params.output_all_probs is None:
         ids = ops.argmax(logits)
     else:
-        probs = ops.softmax_rows(logits)
-        logits.copy_(probs)
-        top_p = _host(params.top_p, torch.float32).clone()
-        top_p[top_p.abs() < 1e-7] = 1.0
+        probs = ops.softmax_rows(logits, out=logits)
         want_renorm = params.output_all_probs is not None and not params.return_original_all_probs
         if all_greedy:
             ids = ops.argmax(probs)
@@ -94,12 +124,12 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
                 _, renorm = ops.top_k_top_p_sample(probs, top_k, None, torch.zeros(B, device=dev), return_probs=True)
                 params.output_all_probs.copy_(renorm)
         else:
-            if params.uniform is None:
-                raise ValueError("sample_greedy: sampling rows need params.uniform (one value in [0, 1) per row)")
-            u = params.uniform.to(device=dev, dtype=torch.float32).contiguous()
-            ids, renorm = ops.top_k_top_p_sample(probs, top_k, top_p, u, return_probs=True)
+            u = up["uniform"] if "uniform" in up else params.uniform.to(device=dev, dtype=torch.float32).contiguous()
             if want_renorm:
+                ids, renorm = ops.top_k_top_p_sample(probs, up["top_k"], up["top_p"], u, return_probs=True)
                 params.output_all_probs.copy_(renorm)
+            else:
+                ids = ops.top_k_top_p_sample(probs, up["top_k"], up["top_p"], u)
         if params.return_original_all_probs and params.output_all_probs is not None:
             params.output_all_probs.copy_(probs)
     params.token_ids[:, step] = ids.to(params.token_ids.device)
