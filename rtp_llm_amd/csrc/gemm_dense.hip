@@ -3,7 +3,8 @@
 // Both operands are contiguous along K, which is the layout v_mfma_f32_16x16x32_bf16 wants for its A and B fragments (8 consecutive k per
 // lane), so no weight image is built: a model whose layers have many small, differently shaped projections (recurrent gates, low-rank
 // decays, shared-KV attention) loads its tensors as they are.  Three kernels, all with fp32 accumulation and an fp32 epilogue:
-//   * tile kernel, bf16:  64 x 128 block tile, 4 waves of 32 x 64, K staged through LDS 64 at a time, MFMA 16x16x32;
+//   * tile kernels, bf16: block tiles of 64 x 128 up to 256 x 256, both operands through LDS by DMA, MFMA 16x16x32; one that stages 64 x 128 through registers
+//     for operands without 16-byte alignment;
 //   * tile kernel, fp32:  64 x 64 block tile, 4 x 4 register micro-tiles, true fp32 FMAs (no reduced-precision matrix mode);
 //   * skinny kernel, bf16, 2 <= M <= 16: one block per 16 outputs, its waves split K, MFMA fragments loaded straight from memory;
 //   * row kernel (M = 1; fp32 up to M = 16): a wave per output column streams its weight row once, 16-byte loads, wave reduction at the end.
@@ -29,6 +30,7 @@ struct DenseParams {
     int out_f32;
     float softcap;   // > 0: y = cap * tanh(y / cap)
     int vec;         // 16-byte loads allowed (alignment and K % 8 == 0 checked on the host)
+    int yvec;        // four consecutive outputs of a row that start at a multiple of four may be stored together (ldy % 4 == 0, y aligned)
     // groups (tile kernels, blockIdx.z): group g multiplies its rows by the weight w + g * ws (bias + g * N) and writes columns ys * g + ...
     // of y; it reads x from column xs * g on.  Its rows are all M rows, or rows offs[g] .. offs[g + 1] - 1 of a list sorted by group, whose
     // entry r reads x row gather[r] (identity without gather) and writes y row r.  tiles (with offs): {count, (group, first row) x count}, the
@@ -44,20 +46,22 @@ struct DenseParams {
 // that an XCD walks a contiguous run of tiles in an order of bands of DN_BAND row tiles, column by column: its blocks share the band's rows of x and read
 // every weight column of the run once.
 constexpr int DN_XCD = 8, DN_BAND = 16;
+template <int BAND>
 __device__ __forceinline__ void dn_block_tile(int gx, int gy, int& bx, int& by) {
     const int nb = gx * gy, id = blockIdx.y * gridDim.x + blockIdx.x;
     if (id >= nb) { bx = 0; by = gy; return; }               // a block past the list of tiles
     const int k = id % DN_XCD, j = k * (nb / DN_XCD) + min(k, nb % DN_XCD) + id / DN_XCD;
-    const int band = j / (gx * DN_BAND), rest = j - band * gx * DN_BAND, h = min(DN_BAND, gy - band * DN_BAND);
-    bx = rest / h; by = band * DN_BAND + rest % h;
+    const int band = j / (gx * BAND), rest = j - band * gx * BAND, h = min(BAND, gy - band * BAND);
+    bx = rest / h; by = band * BAND + rest % h;
 }
 
 // the block's column tile, first row and end of the rows of its tile in its group, and the group's operand bases
 struct DnGroup { int bx, m0, rend; long long xo, wo, yo; int bo; };
+template <int BAND = DN_BAND>
 __device__ __forceinline__ DnGroup dn_group(const DenseParams& p, int tile_rows) {
     int g = blockIdx.z, by;
     DnGroup r;
-    dn_block_tile(gridDim.x, p.tiles ? p.tiles[0] : gridDim.y, r.bx, by);
+    dn_block_tile<BAND>(gridDim.x, p.tiles ? p.tiles[0] : gridDim.y, r.bx, by);
     if (p.tiles) {
         if (by >= p.tiles[0]) { r.m0 = r.rend = 0; return r; }
         g = p.tiles[1 + 2 * by]; r.m0 = p.tiles[2 + 2 * by]; r.rend = p.offs[g + 1];
@@ -94,6 +98,34 @@ __device__ __forceinline__ void dn_store(const DenseParams& p, int row, int col,
     if (p.egate) v *= 1.f / (1.f + expf(-p.egate[(size_t)row * p.ldg + p.goff + col]));
     if (p.out_f32) ((float*)p.y)[(size_t)row * p.ldy + col] = v;
     else           ((T*)p.y)[(size_t)row * p.ldy + col] = (T)v;
+}
+
+// four consecutive outputs of one row (cnt of them exist)
+__device__ __forceinline__ void dn_store4(const DenseParams& p, int row, int col, f32x4 v, int cnt) {
+    if (p.softcap > 0.f) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = p.softcap * tanhf(v[e] / p.softcap);
+    }
+    if (p.egate) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) if (e < cnt) v[e] *= 1.f / (1.f + expf(-p.egate[(size_t)row * p.ldg + p.goff + col + e]));
+    }
+    const size_t at = (size_t)row * p.ldy + col;
+    if (p.out_f32) {
+        float* y = (float*)p.y + at;
+        if (cnt == 4 && p.yvec && !(col & 3)) *(f32x4*)y = v;
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) if (e < cnt) y[e] = v[e];
+        }
+    } else {
+        bf16* y = (bf16*)p.y + at;
+        if (cnt == 4 && p.yvec && !(col & 3)) { u32x2 o = {act_pack<true>(v[0], v[1]), act_pack<true>(v[2], v[3])}; *(u32x2*)y = o; }
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) if (e < cnt) y[e] = (bf16)v[e];
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ bf16 tile kernel
@@ -194,6 +226,208 @@ __global__ __launch_bounds__(256) void dense_tile_bf16_kernel(DenseParams p) {
                 }
             }
         }
+}
+
+// ------------------------------------------------------------------------------------------------ bf16 tile kernel, LDS-DMA staging
+// BM rows of x by BN rows of w per block, K in tiles of BK; waves of WM x WN outputs.  Both operands go to LDS by `global_load_lds_dwordx4` (no staging registers, no
+// ds_write) into NS stages, one barrier per tile.  An LDS row is the BK * 2 bytes of a K tile; its 16-byte pieces are permuted by the row (applied to the source
+// address, which the DMA leaves free per lane), so that the 16-row fragment reads hit every bank once.  w is the MFMA's first operand: a lane ends with four
+// consecutive outputs of one row.  The sums run over k in steps of 32 like the other tile kernel's: same bits.
+// NS = 2: tiles of 64, two blocks or more per CU hide each other's waits.  NS >= 3: tiles of 32, a wave reads the fragments of tile t + 1 between the products of tile t.
+// Time in us of 256x256 (NS 4) / 128x128 (NS 2) / 64x128 (NS 2) / 64x128 (NS 4) tiles and of the 64x128 kernel that stages through registers:
+//   M x N x K       8192x11264x2048 gated  355 / 357 / 424 / 567, 599    8192x2048x5632  148 / 175 / 214 / 297, 307    8192x2048x2048  63 / 71 / 83 / 111, 120
+//                   2048x11264x2048 gated  109 /  96 / 108 / 146, 156    2048x2048x2048   48 /  26 /  25 /  31,  41     512x2048x5632 109 / 57 / 48 / 43, 77
+//                   1537x1024x1024          28 /  12 /  10 /   9,  21      70x2048x2048   42 /  18 /  15 /  12,  32
+__device__ __forceinline__ void dn_dma16(uint32_t lds, uint32_t voff, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
+
+// waits until at most VM of the wave's vector-memory operations and none of its LDS operations are left.  (A builtin, not asm: the compiler's own counting sees it.)
+template <int VM> __device__ __forceinline__ void dn_wait() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+
+template <int BM, int BN, int WM, int WN, int BK, int NS>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_kernel(DenseParams p) {
+    constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, MI = WM / 16, NJ = WN / 16;
+    constexpr bool AHEAD = NS >= 3;                                           // fragments of tile t + 1 are read while tile t is multiplied
+    constexpr int RB = BK * 2, PPR = BK / 8, RPL = 64 / PPR;                  // bytes and 16-byte pieces of a row, rows per wave load
+    constexpr int STAGE = (BM + BN) * RB, ULD = (BM + BN) / (RPL * NW), ULA = BM / (RPL * NW);   // loads per wave and tile; the first ULA are rows of x
+    static_assert((AHEAD ? BK == 32 : BK == 64) && BM % (RPL * NW) == 0 && BN % (RPL * NW) == 0, "whole wave loads per operand");
+    constexpr int PH = MI >= 4 && NS * STAGE >= NW * 16384 ? 4 : MI >= 2 ? 2 : 1;   // 16-row blocks of results that pass through LDS together
+    static_assert(WN == 64 && NS * STAGE >= NW * PH * 4096, "a wave's output columns; room for its results");
+    __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % NWM, wn = wave / NWM;
+    const DnGroup gr = dn_group<1024 / BM>(p, BM);
+    const int m0 = gr.m0, n0 = gr.bx * BN;
+    if (m0 >= gr.rend) return;
+    const bf16* X = (const bf16*)p.x + gr.xo + (p.gather ? 0 : (size_t)m0 * p.ldx);
+    const bf16* W = (const bf16*)p.w + gr.wo + (size_t)n0 * p.K;
+    // lane l of a wave load owns row (l >> 3) of its eight, LDS piece l & 7 = source piece (l & 7) ^ (row & 7); rows past the end repeat the last one
+    auto swizzle = [](int row) { return BK == 64 ? row & 7 : (row >> 1) & 3; };
+    const int lr = lane / PPR, piece = (lane % PPR) ^ swizzle(lr);
+    uint32_t voff[ULD];
+    int xrow[ULA];
+#pragma unroll
+    for (int u = 0; u < ULD; ++u) {
+        const int r = ((u < ULA ? u : u - ULA) * NW + wave) * RPL + lr;
+        if (u < ULA) {
+            const int m = min(m0 + r, gr.rend - 1);
+            xrow[u] = p.gather ? p.gather[m] : m - m0;
+            voff[u] = (uint32_t)xrow[u] * (uint32_t)p.ldx * 2u + piece * 16u;
+        } else {
+            voff[u] = (uint32_t)min(r, p.N - 1 - n0) * (uint32_t)p.K * 2u + piece * 16u;
+        }
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem);
+    auto issue = [&](int buf, int kt) {
+#pragma unroll
+        for (int u = 0; u < ULD; ++u)
+            dn_dma16(lds0 + buf * STAGE + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024, voff[u], u < ULA ? X + kt * BK : W + kt * BK);
+    };
+    f32x4 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int fr = lane & 15, q = lane >> 4;
+    struct Frags { bf16x8 w[NJ], x[MI]; };
+    auto load = [&](Frags& f, int buf, int ks) {
+        const int foff = (((ks * 4 + q) ^ swizzle(fr)) << 4) + fr * RB;
+        const char* xs = smem + buf * STAGE + wm * WM * RB + foff;
+        const char* ws = smem + buf * STAGE + (BM + wn * WN) * RB + foff;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) f.w[j] = *(const bf16x8*)(ws + j * 16 * RB);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) f.x[i] = *(const bf16x8*)(xs + i * 16 * RB);
+    };
+    auto multiply = [&](const Frags& f) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j], f.x[i], acc[i][j], 0, 0, 0);
+    };
+    const int nk = p.K / BK;
+    Frags fa, fb;
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t) if (t < nk) issue(t, t);
+    if constexpr (!AHEAD) {
+        for (int kt = 0; kt < nk; ++kt) {
+            dn_wait<0>();                                                   // this wave's part of tile kt is in LDS, its reads of tile kt - 1 are done
+            __builtin_amdgcn_s_barrier();
+            if (kt + 1 < nk) issue((kt + 1) & 1, kt + 1);
+#pragma unroll
+            for (int ks = 0; ks < BK / 32; ++ks) { load(fa, kt & 1, ks); multiply(fa); }
+        }
+    } else {
+        if (nk > 0) {
+            if (nk >= NS - 1) dn_wait<ULD * (NS - 2)>(); else dn_wait<0>();
+            __builtin_amdgcn_s_barrier();
+            load(fa, 0, 0);
+        }
+        int next = 1, ahead = NS - 1, kt = 0;                               // stages of tile kt + 1 and of tile kt + NS - 1
+        // IN_FLIGHT: tile kt + 1 is in LDS once at most that many of the wave's loads are left; its reads of tile kt are done by then, so behind the barrier
+        // tile kt + NS - 1 may go over tile kt - 1
+        auto advance = [&](Frags& nxt, auto in_flight, bool more) {
+            dn_wait<decltype(in_flight)::value>();
+            __builtin_amdgcn_s_barrier();
+            if (more) issue(ahead, kt + NS - 1);
+            load(nxt, next, 0);
+            next = next + 1 == NS ? 0 : next + 1;
+            ahead = ahead + 1 == NS ? 0 : ahead + 1;
+        };
+        auto interleave = [&]() {      // reads between products, nothing across the tile's end (left alone, the scheduler puts the reads in front of the barrier's wait)
+#pragma unroll
+            for (int g = 0; g < MI + NJ; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, MI * NJ / (MI + NJ), 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, MI * NJ, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        constexpr std::integral_constant<int, ULD * (NS - 3)> steady{};
+        for (; kt + NS < nk; ++kt) {                                        // no conditions inside: the compiler's own waits stay as late as they can be
+            advance(fb, steady, true);
+            multiply(fa);
+            interleave();
+            ++kt;
+            advance(fa, steady, true);
+            multiply(fb);
+            interleave();
+        }
+        for (; kt < nk; ++kt) {
+            if (kt + 1 < nk) {
+                if (kt + NS - 1 < nk) advance(fb, steady, true); else advance(fb, std::integral_constant<int, 0>{}, false);
+            }
+            multiply(fa);
+            if (kt + 1 < nk) fa = fb;
+        }
+    }
+    if (p.K % BK) {                                                         // the last K % BK columns: through registers, zeros behind them
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < ULD; ++u) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            const char* src = (const char*)(u < ULA ? X : W) + voff[u] + (size_t)nk * RB;
+            if (nk * BK + piece * 8 < p.K) v = *(const u32x4*)src;
+            *(u32x4*)(smem + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024 + lane * 16) = v;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < BK / 32; ++ks) { load(fa, 0, ks); multiply(fa); }
+    }
+    // Results through LDS, up to 64 rows of a wave's 64 columns at a time: a lane holds four outputs (4 q + e of 16) of row fr, and reads back four consecutive ones of a
+    // row that its 15 neighbours continue -- whole 256-byte runs per store, and ONE copy of the epilogue's code (unrolled over the 32 fragments it did not fit the
+    // instruction cache: 46 of the 93 us of an 8192 x 2048 x 2048 product).  16-byte pieces permuted by the row.
+    const bf16* Bi = p.bias ? (const bf16*)p.bias + gr.bo : nullptr;
+    char* mine = smem + wave * (PH * 4096);
+    const int nc = n0 + wn * WN;                                            // the wave's first weight row
+    __syncthreads();
+#pragma unroll
+    for (int i0 = 0; i0 < MI; i0 += PH) {
+#pragma unroll
+        for (int i = 0; i < PH; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) *(f32x4*)(mine + (i * 16 + fr) * 256 + (((j * 4 + q) ^ fr) << 4)) = acc[i0 + i][j];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // the wave's own stores, read by its other lanes
+        const int r0 = m0 + wm * WM + i0 * 16, rows = min(PH * 16, gr.rend - r0);
+        if (p.gated) {
+            const int c4 = lane & 7;                                        // channels 4 c4 .. of the wave's 32
+            if (nc + c4 * 4 + 32 < p.N)
+#pragma unroll 1
+                for (int r = lane >> 3; r < rows; r += 8) {
+                    f32x4 g = *(const f32x4*)(mine + r * 256 + ((c4 ^ (r & 15)) << 4)), u = *(const f32x4*)(mine + r * 256 + (((c4 + 8) ^ (r & 15)) << 4)), v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (Bi) { g[e] += dn_ld(Bi + nc + c4 * 4 + e); u[e] += dn_ld(Bi + nc + 32 + c4 * 4 + e); }
+                        v[e] = dn_gated(g[e], u[e], p.act, p.act_param);
+                    }
+                    dn_store4(p, r0 + r, (int)gr.yo + (nc >> 1) + c4 * 4, v, 4);
+                }
+        } else {
+            const int c4 = lane & 15, n = nc + c4 * 4, cnt = min(4, p.N - n);
+            f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+            if (Bi) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) if (e < cnt) bias[e] = dn_ld(Bi + n + e);
+            }
+            if (cnt > 0)
+#pragma unroll 1
+                for (int r = lane >> 4; r < rows; r += 4) {
+                    f32x4 v = *(const f32x4*)(mine + r * 256 + ((c4 ^ (r & 15)) << 4));
+                    if (Bi) v += bias;
+                    if (p.act != DN_ACT_NONE) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = dn_act(v[e], p.act);
+                    }
+                    dn_store4(p, r0 + r, (int)gr.yo + n, v, cnt);
+                }
+        }
+        if (i0 + PH < MI) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next rows overwrite them
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ fp32 tile kernel
@@ -414,6 +648,31 @@ __global__ __launch_bounds__(256) void dense_rows_grouped_kernel(DenseParams p) 
     }
 }
 
+// The bf16 tile launch of p: gy64 row tiles of 64 rows (blockIdx.y) when the rows are grouped, groups in z.
+void launch_tiles_bf16(const DenseParams& p, int gy64, int gz, hipStream_t st) {
+    const bool dma = p.vec && (!p.gather || (uint64_t)p.M * p.ldx * 2 < 0xFFFFFFFFull) && (uint64_t)p.ldx * 512 < 0xFFFFFFFFull && (uint64_t)p.K * 512 < 0xFFFFFFFFull;
+    if (!dma) {                                                             // unaligned operands, K % 8 != 0, 32-bit offsets that do not reach
+        hipLaunchKernelGGL(dense_tile_bf16_kernel, dim3((p.N + TB_N - 1) / TB_N, gy64, gz), dim3(256), 0, st, p);
+        return;
+    }
+    // the shape with the least expected time, us per 32 columns of k: a constant and the blocks per CU times what one costs a busy CU (256 x 256: whole rounds
+    // count half, one block fills a CU).  Measured at M = 70..8192, N = 16..32000, K = 16..5632: within 10 % of the fastest of the four.  Grouped rows
+    // come in tiles of 64.
+    auto share = [&](int bm, int bn) { return (double)((p.N + bn - 1) / bn) * (p.offs ? gy64 : (p.M + bm - 1) / bm) * gz / 256.0; };
+    const double sa = share(256, 256), sb = share(128, 128), sc = share(64, 128), k = p.K / 32.0;
+    const double ta = k * fmax(0.65, 0.475 * (sa + ceil(sa))) + 12.0, tb = k * fmax(0.30, 0.255 * sb + 0.13) + 5.0;
+    const double tc = k * fmax(0.23, 0.15 * sc + 0.10) + 4.0, td = k * fmax(0.185, 0.19 * sc + 0.10) + 4.0;
+    const int gn = (p.N + 127) / 128;
+    if (p.offs || (tc <= tb && tc <= ta) || (td <= tb && td <= ta)) {
+        if (td < tc) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 32, 4>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
+        else         hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 2>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
+    } else if (tb < ta) {
+        hipLaunchKernelGGL((dense_dma_bf16_kernel<128, 128, 32, 64, 64, 2>), dim3(gn, (p.M + 127) / 128, gz), dim3(512), 0, st, p);
+    } else {
+        hipLaunchKernelGGL((dense_dma_bf16_kernel<256, 256, 128, 64, 32, 4>), dim3((p.N + 255) / 256, (p.M + 255) / 256, gz), dim3(512), 0, st, p);
+    }
+}
+
 template <typename T, bool GATED>
 void launch_rows(const DenseParams& p, hipStream_t st) {
     const int nout = GATED ? p.N / 2 : p.N;
@@ -512,6 +771,7 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
     p.x = x; p.w = w; p.bias = bias; p.y = y; p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = ldy;
     p.gated = gated; p.act = act; p.act_param = act_param; p.out_f32 = bf ? out_f32 : 1; p.softcap = softcap;
     p.vec = (K % 8 == 0) && (ldx % 8 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
+    p.yvec = (ldy % 4 == 0) && ((uintptr_t)y % (p.out_f32 ? 16 : 8) == 0);
     p.G = 1; p.xs = p.ws = p.ys = 0; p.offs = nullptr; p.gather = nullptr; p.tiles = nullptr; p.egate = nullptr; p.ldg = p.goff = 0;
     (void)es;
     hipStream_t st = (hipStream_t)stream;
@@ -530,9 +790,8 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
         return MI355_OK;
     }
     if (bf) {
-        const dim3 grid((N + TB_N - 1) / TB_N, (M + TB_M - 1) / TB_M);
-        hipLaunchKernelGGL(dense_tile_bf16_kernel, grid, dim3(256), 0, st, p);
-        MI355_CHECK_LAUNCH("dense_tile_bf16_kernel");
+        launch_tiles_bf16(p, (M + TB_M - 1) / TB_M, 1, st);
+        MI355_CHECK_LAUNCH("dense bf16 tile kernel");
     } else {
         const dim3 grid((N + TF_N - 1) / TF_N, (M + TF_M - 1) / TF_M);
         hipLaunchKernelGGL(dense_tile_f32_kernel, grid, dim3(256), 0, st, p);
@@ -573,6 +832,7 @@ extern "C" int mi355_dense_grouped_ex(const void* x, int32_t ldx, int32_t M, con
     p.x = x; p.w = w; p.bias = bias; p.y = y; p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = ldy;
     p.gated = gated; p.act = act; p.act_param = act_param; p.out_f32 = bf ? out_f32 : 1; p.softcap = 0.f;
     p.vec = (K % 8 == 0) && (ldx % 8 == 0) && (xs % 8 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
+    p.yvec = (ldy % 4 == 0) && ((uintptr_t)y % (p.out_f32 ? 16 : 8) == 0);
     p.G = G; p.xs = xs; p.ws = (long long)N * K; p.ys = ys; p.offs = offs; p.gather = gather; p.tiles = tiles;
     p.egate = egate; p.ldg = ldg; p.goff = goff;
     MI355_CHECK_ARG(!egate || (goff >= 0 && ldg >= goff + (offs ? 0 : ys * (G - 1)) + (gated ? N / 2 : N)), "dense_grouped: gate row stride %d", ldg);
@@ -604,9 +864,8 @@ extern "C" int mi355_dense_grouped_ex(const void* x, int32_t ldx, int32_t M, con
         return MI355_OK;
     }
     if (bf) {
-        const dim3 grid((N + TB_N - 1) / TB_N, gy, gz);
-        hipLaunchKernelGGL(dense_tile_bf16_kernel, grid, dim3(256), 0, st, p);
-        MI355_CHECK_LAUNCH("dense_tile_bf16_kernel");
+        launch_tiles_bf16(p, gy, gz, st);
+        MI355_CHECK_LAUNCH("dense bf16 tile kernel");
     } else {
         const dim3 grid((N + TF_N - 1) / TF_N, gy, gz);
         hipLaunchKernelGGL(dense_tile_f32_kernel, grid, dim3(256), 0, st, p);
