@@ -44,6 +44,11 @@ def _host(t: torch.Tensor, dtype) -> torch.Tensor:
     return t.detach().to(device="cpu", dtype=dtype)
 
 
+def _softmax_in_place(logits: torch.Tensor) -> torch.Tensor:
+    # the kernel may overwrite its input; host tensors reach this flow only with another `ops`, which need not
+    return ops.softmax_rows(logits, out=logits) if logits.is_cuda else logits.copy_(ops.softmax_rows(logits))
+
+
 def _upload(tensors, device):
     """The named host tensors of 32-bit values on the device, contiguous: packed into one buffer and sent in one copy."""
     if not tensors:
@@ -116,7 +121,7 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
     if all_greedy and params.output_all_probs is None:
         ids = ops.argmax(logits)
     else:
-        probs = ops.softmax_rows(logits, out=logits)
+        probs = _softmax_in_place(logits)
         want_renorm = params.output_all_probs is not None and not params.return_original_all_probs
         if all_greedy:
             ids = ops.argmax(probs)
