@@ -441,6 +441,21 @@ SCAN_CHUNK_BYTES = 512 << 20
 SCAN_BLOCKS_AT_ONCE = 512  # blocks of the scan kernel the chip runs side by side (two per compute unit)
 
 
+WALK_MAX_DIM = 128         # key channels of mi355_hy_walk
+
+
+def walk_chunk(T: int, nseq: int, max_rows: int, heads: int, vdim: int) -> int:
+    """Chunk size of the gated recurrence over prompt portions, 0: walked whole.  A model of both in us: the whole walk takes 0.33 a token of the longest
+    sequence for every 512 blocks of 64 columns; the chunks (of 32, 64 or 128 tokens, so that their blocks fill the chip once) two walks of a chunk behind 30 of
+    launches and prefix, or 1.85e-3 a token and head where the chip is full.  Measured, heads of 64 x 128, whole / chunks: 4 x 2048 tokens 16 heads 680 / 253,
+    1 x 2048 16 heads 665 / 103, 1 x 1537 8 heads 504 / 64, 2 x 300 8 heads 100 / 46, 16 x 512 16 heads 225 / 254, 8 x 96 16 heads 38 / 55."""
+    longest = max_rows if max_rows > 0 else T - (nseq - 1)
+    work = T * heads * ((vdim + 127) // 128)
+    C = 32 if work < 50000 else 64 if work < 100000 else 128
+    whole = 0.33 * longest * -(-nseq * heads * ((vdim + 63) // 64) // 512)
+    return C if longest > C and max(30.0 + 0.6 * C, 12.0 + 1.85e-3 * work) < whole else 0
+
+
 def scan_prefers_chunks(T: int, nseq: int, max_rows: int, heads: int, vdim: int, C: int) -> bool:
     """Whether the chunked form is expected to be faster: the token-by-token walk takes (rounds of blocks) x (rows of the longest sequence)
     token steps, the chunked form two passes of (rounds of blocks over all chunks) x (chunk size)."""
@@ -469,11 +484,11 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
          heads: int, dim: int, vdim: int, row_start, slot, first_pos, state: torch.Tensor, act: torch.dtype, *, plans: Optional[dict] = None,
          chunked: Optional[bool] = None, max_rows: int = 0) -> torch.Tensor:
     """Gated linear recurrence over the rows of every sequence, continuing (and leaving) the fp32 state of its slot -> fp32 [T, heads * vdim].
-    The modes with a constant decay per head (SCAN_FIXED, SCAN_FIXED_SILU) run long prompt portions in chunks that are walked side by side
-    (every chunk from a zero state, a prefix over each sequence's chunks, then the chunk-start states' share of the outputs): the same sums in
-    another order.  They do so when that is expected to be faster (scan_prefers_chunks: few long sequences; max_rows = the rows of the step's
-    longest sequence when the caller knows it).  plans: a dict that keeps the step's chunk plan between calls (the layers of one step share
-    it); chunked forces the choice."""
+    Long prompt portions run in chunks that are walked side by side, the same sums in another order, when that is expected to be faster (few long sequences;
+    max_rows = the rows of the step's longest sequence when the caller knows it).  The modes with a constant decay per head (SCAN_FIXED, SCAN_FIXED_SILU):
+    every chunk from a zero state, a prefix over each sequence's chunks, then the chunk-start states' share of the outputs (scan_prefers_chunks).
+    The gated modes: what every chunk leaves from a zero state and its total decays, the prefix, then the tokens again from the chunk-start states (walk_chunk).
+    plans: a dict that keeps the step's chunk plan between calls (the layers of one step share it); chunked forces the choice."""
     _dev(proj, torch.float32, "scan.proj"); _dev(state, torch.float32, "scan.state")
     T = proj.shape[0]
     out = torch.empty(T, heads * vdim, dtype=torch.float32, device=proj.device)
@@ -488,6 +503,28 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
                                           act_code(act), _stream()), "hy_scan")
 
     fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
+    if not fixed and chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim):
+        def walk(rs, sl, fp, n, st, dst, cdecay, keep):
+            _C.check_hybrid(lib.mi355_hy_walk(mode, proj.data_ptr(), ld, qo, ko, vo, _p(z), 0 if z is None else _rows(z, "scan.z"), _p(lower), _p(fbias), float(tau),
+                                              float(qscale), heads, dim, vdim, rs.data_ptr(), sl.data_ptr(), fp.data_ptr(), n, st.data_ptr(), _p(dst), _p(cdecay), keep,
+                                              act_code(act), _stream()), "hy_walk")
+
+        C = walk_chunk(T, nseq, max_rows, heads, vdim)
+        if not C and nseq * heads * ((vdim + 127) // 128) < 192:                            # few blocks: the walk with more of them takes 0.33 us a token, not 0.41
+            run(mode, row_start, slot, first_pos, nseq, state)
+            return out
+        if not C:
+            walk(row_start, slot, first_pos, nseq, state, out, None, 1)
+            return out
+        plan = _chunk_plan(row_start, T, nseq, heads * dim * vdim * 4, plans, C)
+        n = plan.max_chunks
+        cstate = torch.empty(n, heads, dim, vdim, dtype=torch.float32, device=proj.device)
+        cdecay = torch.empty(n, heads, dim, dtype=torch.float32, device=proj.device)
+        walk(plan.cs, plan.ids, plan.zeros, n, cstate, None, cdecay, 1)                     # 1: what every chunk leaves from a zero state, and its total decays
+        _C.check_hybrid(lib.mi355_hy_chunk_prefix_rows(plan.cs.data_ptr(), plan.sc.data_ptr(), slot.data_ptr(), first_pos.data_ptr(), nseq, None, cdecay.data_ptr(),
+                                                       vdim, heads, dim * vdim, cstate.data_ptr(), state.data_ptr(), _stream()), "hy_chunk_prefix")
+        walk(plan.cs, plan.ids, plan.ones, n, cstate, out, None, 0)                         # 3: the tokens again, from the states at the chunks' starts
+        return out
     if chunked is None:
         chunked = fixed and scan_prefers_chunks(T, nseq, max_rows, heads, vdim, SCAN_CHUNK)
     if not chunked:
@@ -505,9 +542,9 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
     return out
 
 
-def _chunk_plan(row_start, T: int, nseq: int, per_chunk_bytes: int, plans: Optional[dict]) -> ChunkPlan:
-    """The step's plan with chunks of SCAN_CHUNK rows, or of more when the chunk states would not fit the scratch limit."""
-    C = SCAN_CHUNK
+def _chunk_plan(row_start, T: int, nseq: int, per_chunk_bytes: int, plans: Optional[dict], C: int = 0) -> ChunkPlan:
+    """The step's plan with chunks of C (SCAN_CHUNK) rows, or of more when the chunk states would not fit the scratch limit."""
+    C = C or SCAN_CHUNK
     while (T // C + nseq + 1) * per_chunk_bytes > SCAN_CHUNK_BYTES and C < T:
         C *= 2
     key = (row_start.data_ptr(), T, nseq, C)
@@ -515,7 +552,8 @@ def _chunk_plan(row_start, T: int, nseq: int, per_chunk_bytes: int, plans: Optio
     if plan is None:
         plan = ChunkPlan(row_start, T, nseq, C)
         if plans is not None:
-            plans.clear()
+            if len(plans) >= 4:                                   # layers of one step may want chunks of different sizes
+                plans.clear()
             plans[key] = plan
     return plan
 

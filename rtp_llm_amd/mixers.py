@@ -332,7 +332,7 @@ class GatedLinearRecurrence:
         if self.mode == hops.SCAN_GLA:
             z = hops.dense_linear(hops.dense_linear(h, self.w_a1), self.w_a2, self.b_a2, out_dtype=torch.float32)
         o = hops.scan(self.mode, proj, self.qo, self.ko, self.vo, z, self.lower, self.fbias, s.tau, 1.0 / math.sqrt(s.dim), s.heads, s.dim, s.vdim,
-                      batch.row_start, batch.slot, batch.first_pos, state, self.act)
+                      batch.row_start, batch.slot, batch.first_pos, state, self.act, plans=batch.plans, max_rows=batch.max_rows)
         o = hops.head_norm(o, s.heads, s.vdim, self.norm, self.eps, proj if self.go is not None else None, self.go or 0)
         return hops.dense_linear(o, self.w_o, out_dtype=torch.float32)
 
