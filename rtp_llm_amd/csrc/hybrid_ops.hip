@@ -832,217 +832,305 @@ __global__ __launch_bounds__(256) void hy_attn_merge_kernel(const float* parts, 
 }
 
 // ------------------------------------------------------------------------------------------------ attention for prompt portions: MFMA tiles (bf16 cache)
-// One wave per (tile of up to 16 consecutive rows of one sequence, head); up to four heads of one key/value head form a block.  Keys go by 32: S = Q K^T with v_mfma_f32_16x16x32_bf16 (K fragments
-// straight from the cache: 8 consecutive channels per lane), mask and online softmax on the fp32 accumulator fragments, then O += P V with P
-// passed through LDS into the A layout and the 32 value rows transposed through LDS into the B layout.  Scores and weights stay 32-bit: the
-// fp32 queries (scaled) and the fp32 weights enter the matrix unit as an exact sum of two bf16 terms (high part + remainder), the cached
-// keys and values are bf16 as stored, every accumulation is fp32.
+// A wave per (tile of up to 16 consecutive rows of one sequence, head), four waves to a block: HW query heads of one key/value head times 4 / HW tiles, all walking the
+// same keys.  Keys go by 32.  Both products are taken transposed, S^T = K Q^T and O^T = V^T P^T (v_mfma_f32_16x16x32_bf16): a lane then owns ONE query row throughout, so
+// that the running maximum, the denominator and the rescaling are per lane, the reductions over keys are eight registers and two exchanges, and the weights are
+// the second product's operand where they are (its k index is a permutation of the keys that the value fragments share): no LDS pass for them.
+// Scores and weights stay 32-bit: the fp32 queries (scaled) and the fp32 weights enter the matrix unit as an exact sum of two bf16 terms (high part + remainder), the
+// cached keys and values are bf16 as stored, every accumulation is fp32.
+// Key and value rows come by DMA into three LDS stages, two steps ahead, pieces of 16 bytes swizzled by the key so that fragment reads meet no bank twice; values are read
+// through the transposing LDS load.  One barrier a step.  A latent cache (one row that is key and, with its leading channels, value) is staged once.
+// What bounded the kernel before was the chain of a step: one wave per SIMD (234 to 512 registers, keys and values of the next step in them), page lookups, a transpose
+// through 2-byte LDS writes, 16-lane reductions and two barriers in series: 2.8 us per 32 keys at 128 channels, 6 us at 256.  Before / now, 16 query over 4 key heads of
+// 128: 4 x 2048 rows under a block mask of 1024 319 / 176 us, 8 x 96 rows 26 / 15 us; 8 heads over a latent row of 256 (192), 1537 rows: 281 / 98 us; 8 heads of
+// 128 without sharing, 2048 rows: 294 / 100 us; 2 x 1024 rows, 28 over 4: 335 / 113 us.  What bounds it now: a wave's own chain of products, softmax and products, with
+// two or three waves on a SIMD; the matrix units alone would take 30 us of the 176.
 __device__ __forceinline__ void hy_split_bf16(float x, bf16& hi, bf16& lo) { hi = (bf16)x; lo = (bf16)(x - (float)hi); }
-// reductions over the 16 lanes of a DPP row (the lanes that hold one fragment row): quad swaps, then the half-row and row mirrors
+// reductions over the 16 lanes of a DPP row: quad swaps, then the half-row and row mirrors
 template <int CTRL> __device__ __forceinline__ float hy_dpp(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float hy_max16(float v) {
-    v = fmaxf(v, hy_dpp<0xB1>(v));      // quad_perm [1,0,3,2]
-    v = fmaxf(v, hy_dpp<0x4E>(v));      // quad_perm [2,3,0,1]
-    v = fmaxf(v, hy_dpp<0x141>(v));     // row_half_mirror
-    return fmaxf(v, hy_dpp<0x140>(v));  // row_mirror
-}
 __device__ __forceinline__ float hy_sum16(float v) {
-    v += hy_dpp<0xB1>(v);
-    v += hy_dpp<0x4E>(v);
-    v += hy_dpp<0x141>(v);
-    return v + hy_dpp<0x140>(v);
+    v += hy_dpp<0xB1>(v);      // quad_perm [1,0,3,2]
+    v += hy_dpp<0x4E>(v);      // quad_perm [2,3,0,1]
+    v += hy_dpp<0x141>(v);     // row_half_mirror
+    return v + hy_dpp<0x140>(v);  // row_mirror
+}
+// the value of lane ^ X beside the lane's own, in either order (32, 16).  Asm: from the builtin with one value for both operands the compiler takes one result twice.
+template <int X> __device__ __forceinline__ void hy_swap(float v, float& a, float& b) {
+    a = b = v;
+    if (X == 32) asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    else         asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ float hy_max_groups(float v) {
+    float a, b;
+    hy_swap<32>(v, a, b); v = fmaxf(a, b);
+    hy_swap<16>(v, a, b); return fmaxf(a, b);
+}
+__device__ __forceinline__ float hy_sum_groups(float v) {
+    float a, b;
+    hy_swap<32>(v, a, b); v = a + b;
+    hy_swap<16>(v, a, b); return a + b;
+}
+// 16 bytes per lane straight into LDS, at `lds` + 16 lane
+__device__ __forceinline__ void hy_dma16(uint32_t lds, const void* src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(src) : "memory", "m0");
+}
+// until at most VM of the wave's vector-memory operations and none of its LDS operations are left (a builtin, which the compiler's own counting sees)
+template <int VM> __device__ __forceinline__ void hy_wait() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+    asm volatile("" ::: "memory");
 }
 
-constexpr int AT_LD = 40;     // LDS row stride (elements) of the 32-key tiles: 80 bytes, 16-byte aligned
+constexpr int AT_STAGES = 3, AT_PAGES = 1024;     // block-table entries of the walked range held in LDS
 
-template <int DKM, int NCBM, int NWV>     // most 32-channel steps of a key row / 16-channel fragments of a value row the instance holds; waves per block
-__global__ __launch_bounds__(256) void hy_attn_tiles_kernel(const float* q, int ldq, float scale, AttnGeom g, int chunk, const float* sink, const float* vfreq,
-                                                           const int32_t* pos, const int32_t* seq, const int32_t* block_table,
-                                                           const int32_t* tile_row0, const int32_t* tile_n, int ntiles, const bf16* kcache, const bf16* vcache,
-                                                           bf16* out, AttnExtra ex) {
-    __shared__ __attribute__((aligned(16))) bf16 Ph_all[4][16 * AT_LD];
-    __shared__ __attribute__((aligned(16))) bf16 Pl_all[4][16 * AT_LD];
-    __shared__ __attribute__((aligned(16))) bf16 Vt[NCBM * 16 * AT_LD];
-    // the waves of a block are query heads that share one key/value head: they walk the same keys and share the transposed value tile
-    const int wave = threadIdx.x >> 6;
-    constexpr int VEM = NCBM / NWV;                           // 32 VP pieces of 16 bytes over 64 NWV threads: at most NCBM / NWV per thread
-    const int h = blockIdx.y * NWV + wave, lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
-    bf16* Ph = Ph_all[wave];
-    bf16* Pl = Pl_all[wave];
-    // a block takes tile b and then tile ntiles - 1 - b: under a causal mask an early (short) tile of a prompt and a late (long) one, so that
-    // the blocks of one prompt walk about the same number of keys
-    for (int pass = 0; pass < 2; ++pass) {
-    const int tile = pass == 0 ? (int)blockIdx.x : ntiles - 1 - (int)blockIdx.x;
-    if (pass == 1 && tile <= (int)blockIdx.x) break;
-    const int r0 = tile_row0[tile], n = tile_n[tile];
-    const int p0 = pos[r0], kvh = h / (g.H / g.G);
-    const int32_t* bt = block_table + (size_t)seq[r0] * g.max_blocks;
-    const int DK = g.dim / 32, NCB = g.vdim / 16, VP = g.vdim / 8;
+// DK: 32-channel steps of a key row.  NCBM: 16-channel fragments of a value row the instance holds; they are multiplied by fours (fragments past the row's end hold what lies
+// behind it in LDS and are never stored).
+template <int DK, int NCBM>
+__global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_tiles_kernel(const float* q, int ldq, float scale, AttnGeom g, int chunk, const float* sink, const float* vfreq,
+                                                                           const int32_t* pos, const int32_t* seq, const int32_t* block_table, const int32_t* tile_row0,
+                                                                           const int32_t* tile_n, int ntiles, const bf16* kcache, const bf16* vcache, bf16* out, AttnExtra ex,
+                                                                           int HW, int same, int vec) {
+    extern __shared__ __attribute__((aligned(16))) char at_sm[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+    const int TW = 4 / HW, h = blockIdx.y * HW + wave % HW, tw = wave / HW;
+    const int kvh = (int)blockIdx.y * HW / (g.H / g.G);
+    const int NCB = g.vdim / 16;
+    // pieces of 16 bytes in a key row, of a value row; DMA loads per wave and step; swizzle: piece c of key k lies at c ^ (k & mask)
+    constexpr int CK = DK * 4, JK = (CK + 7) / 8, JVM = (NCBM + 3) / 4;
+    const int CV = same ? CK : NCB * 2, JV = same ? 0 : (CV + 7) / 8;
+    const int mk = ((CK & -CK) - 1) & 15, mv = same ? mk : ((CV & -CV) - 1) & 15;
+    const int kbytes = JK * 4096, stage = kbytes + JV * 4096;
+    int32_t* bt_s = (int32_t*)(at_sm + AT_STAGES * stage);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)at_sm;
+    // long (late) tiles of a prompt first
+    const int first_tile = ((int)gridDim.x - 1 - (int)blockIdx.x) * TW, ntw = min(TW, ntiles - first_tile);
+    const bool has = tw < ntw;
+    const int tile = first_tile + min(tw, ntw - 1), r0 = __builtin_amdgcn_readfirstlane(tile_row0[tile]), n = __builtin_amdgcn_readfirstlane(tile_n[tile]);
+    const int p0 = __builtin_amdgcn_readfirstlane(pos[r0]), plast = p0 + n - 1;
     const int psh = (g.page & (g.page - 1)) == 0 ? __builtin_ctz(g.page) : -1;       // page size a power of two: shifts instead of divisions
-    auto cache_row = [&](int kc) {
-        const int pi = psh >= 0 ? kc >> psh : kc / g.page, po = psh >= 0 ? kc & (g.page - 1) : kc % g.page;
-        return (size_t)(bt[pi] * g.G + kvh) * g.page + po;
-    };
     // scores are kept times log2(e): the weights are then 2^(s - m), one v_exp_f32 each; the sink (score 0) and the ratios are unchanged
     // (with a cap the products come out in natural units, are capped, and only then go to the log2 scale)
     const float scale2 = ex.softcap > 0.f ? scale : scale * 1.44269504088896340736f;
     const float cap2 = ex.softcap * 1.44269504088896340736f, icap2 = ex.softcap > 0.f ? 2.f * 1.44269504088896340736f / ex.softcap : 0.f;
-    bf16x8 qh[DKM], ql[DKM];
+    bf16x8 qh[DK], ql[DK];
 #pragma unroll
-    for (int ks = 0; ks < DKM; ++ks) {
-        if (ks >= DK) continue;
+    for (int ks = 0; ks < DK; ++ks) {
         const float* qp = q + (size_t)(r0 + min(lr, n - 1)) * ldq + h * g.dim + ks * 32 + lq * 8;
+        float v[8];
+        if (vec & 1) {
+            const f32x4 a = *(const f32x4*)qp, b = *(const f32x4*)(qp + 4);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { bf16 a, b; hy_split_bf16(qp[i] * scale2, a, b); qh[ks][i] = a; ql[ks][i] = b; }
+            for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[4 + i] = b[i]; }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = qp[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { bf16 a, b; hy_split_bf16(v[i] * scale2, a, b); qh[ks][i] = a; ql[ks][i] = b; }
     }
-    float m[4], l[4];
-    f32x4 o[NCBM];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { m[e] = sink ? sink[h] * 1.44269504088896340736f : -INFINITY; l[e] = (sink && lr == 0) ? 1.f : 0.f; }   // l: per-lane share of the row's denominator
+    float m = sink ? sink[h] * 1.44269504088896340736f : -INFINITY, l = sink && lq == 0 ? 1.f : 0.f;      // l: the lane's share of the row's denominator
+    f32x4 o[NCBM];                                            // fragment element e: channel cb * 16 + 4 lq + e of row lr
 #pragma unroll
     for (int cb = 0; cb < NCBM; ++cb) o[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int plast = p0 + n - 1;
-    const int rlo_last = hy_first_visible(plast, chunk, ex.window);
-    const int kstart = hy_first_visible(p0, chunk, ex.window) & ~31;
-    // with kept first tokens: the steps that hold those in front of kstart come first (what else they hold is masked)
-    const int keep = ex.window > 0 ? ex.keep : 0, nkept = (min(keep, kstart) + 31) >> 5, nsteps = nkept + ((plast - kstart) >> 5) + 1;
-    unsigned gap4[4];                                         // hidden keys between the kept ones and the window of the lane's four rows: keep .. keep + gap - 1
+    const int rpos = lr < n ? p0 + lr : -1;
+    const int rlo_last = hy_first_visible(plast, chunk, ex.window), rlo_first = hy_first_visible(p0, chunk, ex.window);
+    const int keep = ex.window > 0 ? ex.keep : 0;
+    const unsigned gap = (unsigned)max(hy_first_visible(p0 + lr, chunk, ex.window) - keep, 0);    // hidden keys between the kept ones and the row's window
+    // where the lane's fragments lie in a stage: keys lr (+ 16), pieces 4 ks + lq; and for the transposing load keys 4 lq + lr / 4 (+ 16), 4 channels each
+    const int krow = lr * CK * 16, kx = lr & mk;
+    const int vkey = 4 * lq + (lr >> 2), vrow = vkey * CV * 16 + (lr & 1) * 8, vx = vkey & mv, vhi = (lr & 3) >> 1;
+    const int VJ = same ? 0 : kbytes;
+    int vpiece[JVM];                                          // the lane's value pieces of a step: key | channel << 5
 #pragma unroll
-    for (int e = 0; e < 4; ++e) gap4[e] = (unsigned)max(hy_first_visible(p0 + lq * 4 + e, chunk, ex.window) - keep, 0);
-    auto step_key = [&](int st) { return (st < nkept ? 0 : kstart - 32 * nkept) + 32 * st; };
-    // the key fragments and raw value rows of the next 32 keys are fetched while the current 32 are worked on
-    bf16x8 kn[2][DKM];
-    u32x4 vn[VEM];
-    auto fetch = [&](int t0) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            const int kc = min(t0 + kb * 16 + lr, plast);
-            const bf16* kp = kcache + cache_row(kc) * g.dim + lq * 8;
-#pragma unroll
-            for (int ks = 0; ks < DKM; ++ks) if (ks < DK) kn[kb][ks] = *(const bf16x8*)(kp + ks * 32);
+    for (int j = 0; j < JVM; ++j) {
+        const int slot = (j * 4 + wave) * 64 + lane, key = min(slot / CV, 31), c = slot % CV;
+        vpiece[j] = key | (c ^ (key & mv)) << 8;
+    }
+    // the tiles of the block in runs of one sequence (one run unless a block's tiles belong to several): the run's keys are staged for all its tiles
+    for (int ft = 0; ft < ntw;) {
+        const int fr = tile_row0[first_tile + ft], sq = seq[fr];
+        int lt = ft, kstart = INT_MAX, klast = 0;
+        for (; lt < ntw; ++lt) {
+            const int tr = tile_row0[first_tile + lt];
+            if (seq[tr] != sq) break;
+            const int tp = pos[tr];
+            kstart = min(kstart, hy_first_visible(tp, chunk, ex.window) & ~31);
+            klast = max(klast, tp + tile_n[first_tile + lt] - 1);
         }
-#pragma unroll
-        for (int e = 0; e < VEM; ++e) {
-            const int i = threadIdx.x + e * 64 * NWV;
-            if (i < 32 * VP) {
-                const int kc = min(t0 + (i & 31), plast);
-                vn[e] = *(const u32x4*)(vcache + cache_row(kc) * g.v_ld + (i >> 5) * 8);
+        kstart = __builtin_amdgcn_readfirstlane(kstart); klast = __builtin_amdgcn_readfirstlane(klast);
+        const bool mine = has && tw >= ft && tw < lt;
+        ft = lt;
+        const int32_t* bt = block_table + (size_t)__builtin_amdgcn_readfirstlane(sq) * g.max_blocks;
+        // with kept first tokens: the steps that hold those in front of kstart come first (what else they hold is masked)
+        const int nkept = (min(keep, kstart) + 31) >> 5, nsteps = nkept + ((klast - kstart) >> 5) + 1;
+        auto step_key = [&](int st) { return (st < nkept ? 0 : kstart - 32 * nkept) + 32 * st; };
+        auto page_of = [&](int k) { return psh >= 0 ? k >> psh : k / g.page; };
+        int bt0 = INT_MIN;                                    // first block-table entry in LDS
+        auto issue = [&](int st, int buf) {
+            const int t0 = step_key(st), plo = page_of(t0), phi = page_of(min(t0 + 31, klast));
+            if (bt0 == INT_MIN || plo < bt0 || phi >= bt0 + AT_PAGES) {        // seldom: the same for the whole block
+                __syncthreads();
+                bt0 = plo;
+                for (int i = threadIdx.x; i < AT_PAGES; i += 256) if (bt0 + i <= page_of(klast)) bt_s[i] = bt[bt0 + i];
+                __syncthreads();
             }
-        }
-    };
-    fetch(step_key(0));
-    for (int st = 0; st < nsteps; ++st) {
-        const int t0 = step_key(st);
-        f32x4 s[2];
+            auto row = [&](int key) {
+                const int kc = min(t0 + key, klast), pi = page_of(kc), po = psh >= 0 ? kc & (g.page - 1) : kc - pi * g.page;
+                return (size_t)(bt_s[pi - bt0] * g.G + kvh) * g.page + po;
+            };
+            const uint32_t base = buf * stage + wave * 1024;
+            auto piece = [&](uint32_t at, const bf16* src) {
+                if (vec & 2) { hy_dma16(lds0 + at, src); return; }
+                bf16x8 v;                                     // a cache that is not on 16 bytes
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < 8; ++i) v[i] = src[i];
+                *(bf16x8*)(at_sm + at + lane * 16) = v;
+            };
 #pragma unroll
-            for (int ks = 0; ks < DKM; ++ks)
-                if (ks < DK) {
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh[ks], kn[kb][ks], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql[ks], kn[kb][ks], acc, 0, 0, 0);
+            for (int j = 0; j < JK; ++j) {
+                const int slot = (j * 4 + wave) * 64 + lane, key = min(slot / CK, 31), c = slot % CK;
+                piece(base + j * 4096, kcache + row(key) * g.dim + ((c ^ (key & mk)) << 3));
+            }
+#pragma unroll
+            for (int j = 0; j < JVM; ++j) {
+                if (j >= JV) break;
+                piece(base + kbytes + j * 4096, vcache + row(vpiece[j] & 31) * g.v_ld + (vpiece[j] >> 5));
+            }
+        };
+        __syncthreads();                                      // the stages and bt_s are free
+        issue(0, 0);
+        if (nsteps > 1) issue(1, 1);
+        int buf = 0;
+        for (int st = 0; st < nsteps; ++st) {
+            if (st + 1 < nsteps) {                            // all but the next step's loads of this wave
+                switch (JK + JV) {
+                    case 1: hy_wait<1>(); break;
+                    case 2: hy_wait<2>(); break;
+                    case 3: hy_wait<3>(); break;
+                    case 4: hy_wait<4>(); break;
+                    case 5: hy_wait<5>(); break;
+                    case 6: hy_wait<6>(); break;
+                    case 7: hy_wait<7>(); break;
+                    default: hy_wait<8>(); break;
                 }
+            } else hy_wait<0>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int t0 = step_key(st), cur = buf * stage;
+            if (st + 2 < nsteps) issue(st + 2, buf == 0 ? 2 : buf - 1);
+            buf = buf == 2 ? 0 : buf + 1;
+            if (!mine || t0 > plast || (t0 + 31 < rlo_first && t0 >= keep)) continue;
+            f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks) {
+                        const char* kp = at_sm + cur + krow + (((ks * 4 + lq) ^ kx) << 4);
+                const bf16x8 k0 = *(const bf16x8*)kp, k1 = *(const bf16x8*)(kp + 256 * CK);
+                s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qh[ks], s[0], 0, 0, 0);
+                s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qh[ks], s[1], 0, 0, 0);
+                s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, ql[ks], s[0], 0, 0, 0);
+                s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, ql[ks], s[1], 0, 0, 0);
+            }
             if (ex.softcap > 0.f) {       // cap tanh(s / cap) = cap (t - 1) / (t + 1), t = 2^(2 s log2(e) / cap), the exponent kept inside fp32's range
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float t = __builtin_amdgcn_exp2f(fminf(fmaxf(acc[e] * icap2, -60.f), 60.f));
-                    acc[e] = cap2 * ((t - 1.f) / (t + 1.f));
+                for (int i = 0; i < 8; ++i) {
+                    const float t = __builtin_amdgcn_exp2f(fminf(fmaxf(s[i >> 2][i & 3] * icap2, -60.f), 60.f));
+                    s[i >> 2][i & 3] = cap2 * ((t - 1.f) / (t + 1.f));
                 }
             }
-            s[kb] = acc;
-        }
-        // the 32 value rows, transposed: Vt[channel][key]; neighbouring lanes write neighbouring keys of one channel row
+            // a step whose 32 keys are visible to every row of the tile (behind the first row, inside the last row's block) needs no mask
+            if (!(t0 + 31 <= p0 && (t0 >= rlo_last || t0 + 32 <= keep))) {
 #pragma unroll
-        for (int e = 0; e < VEM; ++e) {
-            const int i = threadIdx.x + e * 64 * NWV;
-            if (i < 32 * VP) {
-                const int key = i & 31, c8 = (i >> 5) * 8;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    *(uint16_t*)&Vt[(c8 + 2 * j) * AT_LD + key] = (uint16_t)(vn[e][j] & 0xFFFFu);
-                    *(uint16_t*)&Vt[(c8 + 2 * j + 1) * AT_LD + key] = (uint16_t)(vn[e][j] >> 16);
+                for (int i = 0; i < 8; ++i) {
+                    const int kpos = t0 + (i >> 2) * 16 + lq * 4 + (i & 3);
+                    if (!(kpos <= rpos && (unsigned)(kpos - keep) >= gap)) s[i >> 2][i & 3] = -INFINITY;
                 }
             }
-        }
-        if (st + 1 < nsteps) fetch(step_key(st + 1));          // in flight during the softmax and the second product
-        // a step whose 32 keys are visible to every row of the tile (behind the first row, inside the last row's block) needs no mask
-        const bool interior = t0 + 31 <= p0 && (t0 >= rlo_last || t0 + 32 <= keep);
-        // mask, running maximum, weights; fragment element e is row 4 lq + e, the lane's key columns are kb * 16 + lr
+            float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+            const float mn = fmaxf(m, hy_max_groups(mx)), ms = mn == -INFINITY ? 0.f : mn;
+            if (__builtin_amdgcn_ballot_w64(mn != m)) {
+                const float corr = __builtin_amdgcn_exp2f(m - ms);
+                l *= corr;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = lq * 4 + e, rpos = p0 + row;
-            const unsigned gap = gap4[e];
-            float sv[2];
+                for (int cb = 0; cb < NCBM; ++cb) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                const int kpos = t0 + kb * 16 + lr;
-                sv[kb] = (interior || (row < n && kpos <= rpos && (unsigned)(kpos - keep) >= gap)) ? s[kb][e] : -INFINITY;
+                    for (int e = 0; e < 4; ++e) o[cb][e] *= corr;
+                }
+                m = mn;
             }
-            const float mn = fmaxf(m[e], hy_max16(fmaxf(sv[0], sv[1])));
-            float pw[2] = {0.f, 0.f}, corr = 1.f;
-            if (mn != -INFINITY) {
-                corr = (m[e] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[e] - mn);
+            bf16x8 ph, pl;
+            float sum = 0.f;
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb) pw[kb] = (sv[kb] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(sv[kb] - mn);
-            }
-            l[e] = l[e] * corr + pw[0] + pw[1];
-            m[e] = mn;
-#pragma unroll
-            for (int cb = 0; cb < NCBM; ++cb) if (cb < NCB) o[cb][e] *= corr;
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
+            for (int i = 0; i < 8; ++i) {
+                const float pw = __builtin_amdgcn_exp2f(s[i >> 2][i & 3] - ms);
+                sum += pw;
                 bf16 a, b;
-                hy_split_bf16(pw[kb], a, b);
-                Ph[row * AT_LD + kb * 16 + lr] = a; Pl[row * AT_LD + kb * 16 + lr] = b;
+                hy_split_bf16(pw, a, b);
+                ph[i] = a; pl[i] = b;
+            }
+            l += sum;
+            typedef short s16x4 __attribute__((ext_vector_type(4)));
+            typedef short s16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+            for (int c0 = 0; c0 < NCBM; c0 += 4) {
+                if (c0 >= NCB) continue;
+                bf16x8 vf[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const char* vp = at_sm + cur + VJ + vrow + ((((c0 + i) * 2 + vhi) ^ vx) << 4);
+                    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)vp);
+                    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vp + 256 * CV));
+                    vf[i] = __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[c0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i], ph, o[c0 + i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[c0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i], pl, o[c0 + i], 0, 0, 0);
             }
         }
+    }
+    const float lt = hy_sum_groups(l);
+    float inv = lt > 0.f ? 1.f / lt : 0.f;
+    if (ex.ogate && !ex.gate_channels && lr < n) inv *= hy_sigmoid(ex.ogate[(size_t)(r0 + lr) * ex.ldg + h]);
+    bf16* od = out + ((size_t)r0 * g.H + h) * g.vdim;
+    const int ldo = g.H * g.vdim;
+    if (vfreq) {              // turn back by the row's position, pair by pair: the rows pass through LDS, whose stages are free behind the barrier
         __syncthreads();
-        const bf16x8 ph = *(const bf16x8*)&Ph[lr * AT_LD + lq * 8], pl = *(const bf16x8*)&Pl[lr * AT_LD + lq * 8];
+        if (!has) return;
+        const int ldr = g.vdim + 4, pairs = g.vdim / 2;
+        float* rows = (float*)at_sm + wave * 16 * ldr;
 #pragma unroll
         for (int cb = 0; cb < NCBM; ++cb)
-            if (cb < NCB) {
-                const bf16x8 vf = *(const bf16x8*)&Vt[(cb * 16 + lr) * AT_LD + lq * 8];
-                o[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vf, o[cb], 0, 0, 0);
-                o[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vf, o[cb], 0, 0, 0);
-            }
-        __syncthreads();
+            if (cb < NCB) *(f32x4*)(rows + lr * ldr + cb * 16 + lq * 4) = o[cb] * inv;
+        for (int i = lane; i < n * pairs; i += 64) {
+            const int r = i / pairs, mi = i - r * pairs;
+            int c0, c1;
+            hy_pair(g.v_layout, mi, g.vdim, c0, c1);
+            float sn, cs;
+            sincosf((float)(p0 + r) * vfreq[mi], &sn, &cs);
+            const float x = rows[r * ldr + c0], y = rows[r * ldr + c1];
+            od[(size_t)r * ldo + c0] = (bf16)((x * cs + y * sn) * hy_channel_gate(ex, r0 + r, h, g.vdim, c0));
+            od[(size_t)r * ldo + c1] = (bf16)((y * cs - x * sn) * hy_channel_gate(ex, r0 + r, h, g.vdim, c1));
+        }
+        return;
     }
+    if (!has || lr >= n) return;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int row = lq * 4 + e;
-        const float lt = hy_sum16(l[e]);
-        float inv = lt > 0.f ? 1.f / lt : 0.f;
-        if (ex.ogate && !ex.gate_channels && row < n) inv *= hy_sigmoid(ex.ogate[(size_t)(r0 + row) * ex.ldg + h]);
-        const float fp = (float)(p0 + row);
-        bf16* od = out + ((size_t)(r0 + row) * g.H + h) * g.vdim;
+    for (int cb = 0; cb < NCBM; ++cb) {
+        if (cb >= NCB) continue;
+        const int c = cb * 16 + lq * 4;
+        typedef bf16 bf16x4_ __attribute__((ext_vector_type(4)));
+        bf16x4_ w;
 #pragma unroll
-        for (int cb = 0; cb < NCBM; ++cb) {
-            if (cb >= NCB) continue;
-            const int c = cb * 16 + lr;
-            float v = o[cb][e] * inv;
-            if (vfreq) {          // turn back by the row's position; the partner channel sits in the next lane (interleaved) or NCB / 2 fragments away (halves)
-                float other, sn, cs;
-                bool first;
-                int mi;
-                if (g.v_layout == 0) { other = __shfl_xor(v, 1, 64); first = (c & 1) == 0; mi = c >> 1; }
-                else {
-                    const int half = NCB / 2;
-                    first = cb < half; mi = first ? c : c - g.vdim / 2;
-                    float t = 0.f;
+        for (int e = 0; e < 4; ++e) w[e] = (bf16)(o[cb][e] * inv * hy_channel_gate(ex, r0 + lr, h, g.vdim, c + e));
+        bf16* to = od + (size_t)lr * ldo + c;
+        if (vec & 4) *(bf16x4_*)to = w;
+        else {
 #pragma unroll
-                    for (int k = 0; k < NCBM; ++k) if (k == (first ? cb + half : cb - half)) t = o[k][e] * inv;
-                    other = t;
-                }
-                sincosf(fp * vfreq[mi], &sn, &cs);
-                v = first ? (v * cs + other * sn) : (v * cs - other * sn);
-            }
-            if (row < n) od[c] = (bf16)(v * hy_channel_gate(ex, r0 + row, h, g.vdim, c));
+            for (int e = 0; e < 4; ++e) to[e] = w[e];
         }
     }
-    }   // pass
 }
 
 // decay^n for a constant decay in [0, 1] and n >= 0 (n = 0: 1, also for a decay of 0)
@@ -2507,12 +2595,18 @@ extern "C" int mi355_hy_attn_tiles_ex3(const float* q, int32_t ldq, float scale,
         mi355_set_error("hy_attn_tiles: bf16, dim %% 32 == 0, vdim %% 16 == 0 only (dim=%d vdim=%d dtype=%d)", g.dim, g.vdim, act_dtype);
         return MI355_ERR_UNSUPPORTED;
     }
-    const int gq = g.H / g.G, nwv = gq % 4 == 0 ? 4 : gq % 2 == 0 ? 2 : 1;       // query heads of one key/value head per block
-#define HY_TILES(DKM_, NCBM_, NWV_)                                                                                                            \
-    hipLaunchKernelGGL((hy_attn_tiles_kernel<DKM_, NCBM_, NWV_>), dim3((tiles + 1) / 2, g.H / NWV_), dim3(64 * NWV_), 0, (hipStream_t)stream, q, ldq, scale, g, chunk, \
-                       sink, vfreq, pos, seq, block_table, tile_row0, tile_n, tiles, (const bf16*)kcache, (const bf16*)vcache, (bf16*)out, ex)
-    if (g.dim <= 128 && g.vdim <= 128) { if (nwv == 4) HY_TILES(4, 8, 4); else if (nwv == 2) HY_TILES(4, 8, 2); else HY_TILES(4, 8, 1); }
-    else                               { if (nwv == 4) HY_TILES(8, 16, 4); else if (nwv == 2) HY_TILES(8, 16, 2); else HY_TILES(8, 16, 1); }
+    const int gq = g.H / g.G, HW = gq % 4 == 0 ? 4 : gq % 2 == 0 ? 2 : 1;       // query heads of one key/value head per block, 4 / HW tiles each
+    const int same = kcache == vcache && g.v_ld == g.dim && g.vdim <= g.dim;    // the value is a part of the staged key row
+    const int vec = ((uintptr_t)q % 16 == 0 && ldq % 4 == 0 ? 1 : 0) | (((uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 ? 2 : 0) | ((uintptr_t)out % 8 == 0 ? 4 : 0);
+    const int staged = AT_STAGES * 4096 * ((g.dim / 8 + 7) / 8 + (same ? 0 : (g.vdim / 8 + 7) / 8)) + 4 * AT_PAGES, turned = vfreq ? 4 * 16 * (g.vdim + 4) * 4 : 0;
+    const int lds = staged > turned ? staged : turned;
+#define HY_TILES(DK_, NCBM_)                                                                                                                                     \
+    hipLaunchKernelGGL((hy_attn_tiles_kernel<DK_, NCBM_>), dim3((tiles + 4 / HW - 1) / (4 / HW), g.H / HW), dim3(256), lds, (hipStream_t)stream, q, ldq, scale, g, chunk, \
+                       sink, vfreq, pos, seq, block_table, tile_row0, tile_n, tiles, (const bf16*)kcache, (const bf16*)vcache, (bf16*)out, ex, HW, same, vec)
+#define HY_TILES_V(DK_) \
+    case DK_: if (g.vdim <= 64) HY_TILES(DK_, 4); else if (g.vdim <= 128) HY_TILES(DK_, 8); else if (g.vdim <= 192) HY_TILES(DK_, 12); else HY_TILES(DK_, 16); break
+    switch (g.dim / 32) { HY_TILES_V(1); HY_TILES_V(2); HY_TILES_V(3); HY_TILES_V(4); HY_TILES_V(5); HY_TILES_V(6); HY_TILES_V(7); HY_TILES_V(8); }
+#undef HY_TILES_V
 #undef HY_TILES
     MI355_CHECK_LAUNCH("hy_attn_tiles_kernel");
     return MI355_OK;
