@@ -332,6 +332,12 @@ int mi355_rope_kv_write_rows(const void* qkv_f16, const float* partials, int32_t
                              const int32_t* positions, const int32_t* block_table,
                              int32_t max_blocks_per_seq, int32_t T, int32_t q_len, int32_t nh,
                              const mi355_kv_layer_t* kv, void* q_out, int32_t* oob_count, mi355_stream_t stream);
+/* row_seq non-null (device, [T]): the sequence of every row, rows back to back without padding; q_len is 1 then. */
+int mi355_rope_kv_write_rows_ragged(const void* qkv_f16, const float* partials, int32_t nsplit, int32_t ld,
+                                    const void* qkv_bias, const float* cos_sin, int32_t rope_dim, int32_t max_pos,
+                                    const int32_t* positions, const int32_t* row_seq, const int32_t* block_table, int32_t max_blocks_per_seq,
+                                    int32_t T, int32_t q_len, int32_t nh, const mi355_kv_layer_t* kv, void* q_out,
+                                    int32_t* oob_count, mi355_stream_t stream);
 
 /*
  * Paged decode attention (flash-decoding, split over the sequence) — replaces
@@ -362,6 +368,12 @@ int mi355_paged_attn_rows(const void* q, const mi355_kv_layer_t* kv, const int32
                           int32_t max_blocks_per_seq, const int32_t* positions, int32_t B, int32_t q_len, int32_t nh,
                           float scale, int32_t max_seq_len, void* out, void* workspace, size_t workspace_bytes,
                           mi355_stream_t stream);
+
+/* The same without padding rows: q, positions and out hold `rows` rows, sequence b those from row_start[b] (device, [B + 1]) on, at most q_len. */
+int mi355_paged_attn_rows_ragged(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table,
+                                 int32_t max_blocks_per_seq, const int32_t* positions, const int32_t* row_start, int32_t B, int32_t q_len,
+                                 int32_t rows, int32_t nh, float scale, int32_t max_seq_len, void* out, void* workspace,
+                                 size_t workspace_bytes, mi355_stream_t stream);
 
 /* Greedy fast path: ids[b] = argmax(logits[b, :]) on fp32 logits, lowest index on ties
  * (bindings/core/CudaSampleOp.cc:687-700).  workspace >= B * 64 * 8 bytes. */
@@ -610,6 +622,11 @@ size_t mi355_decoder_prefill_workspace_bytes(mi355_decoder_t* d, int32_t max_tok
 int    mi355_decoder_prefill(mi355_decoder_t* d, const int32_t* token_ids, const int32_t* positions, const int32_t* block_table,
                              int32_t nseq, int32_t q_len, const int32_t* logit_rows, float* logits_out, void* workspace,
                              size_t workspace_bytes, mi355_stream_t stream);
+/* The same without padding rows: token_ids, positions and row_seq (the sequence of a row) hold `rows` rows, sequence s those from row_start[s] (device,
+ * [nseq + 1]) on, at most q_len of them; logit_rows index them.  row_seq and row_start null: rows = nseq * q_len, padded as above. */
+int    mi355_decoder_prefill_ragged(mi355_decoder_t* d, const int32_t* token_ids, const int32_t* positions, const int32_t* row_seq,
+                                    const int32_t* row_start, const int32_t* block_table, int32_t nseq, int32_t q_len, int32_t rows,
+                                    const int32_t* logit_rows, float* logits_out, void* workspace, size_t workspace_bytes, mi355_stream_t stream);
 /* Dynamic-NTK RoPE styles only: {cos, sin} rows [max_pos][rope_dim / 2][2] (fp32, device) the prefill chunks that follow rotate with, or NULL for the model's
  * table.  The reference's context_rope (bindings/common/kernels/rotary_position_embedding.h:1000-1025) gives every token of a prefill batch the base of the
  * batch's longest prompt (fused_rope_kvcache_kernel.cu:219-260), while decode uses the base of each position (the model's table). */

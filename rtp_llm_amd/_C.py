@@ -105,6 +105,8 @@ SIGNATURES = {
     "mi355_qkv_rope_kv_write": (i32, [vp, i32, C.POINTER(Weight), vp, C.POINTER(FusedNorm), vp, i32, i32, vp, vp, i32, i32, i32, C.POINTER(KVLayer), vp, vp, vp]),
     "mi355_paged_attn_workspace_bytes": (sz, [i32, i32, i32, i32]),
     "mi355_paged_decode_attn": (i32, [vp, C.POINTER(KVLayer), vp, i32, vp, i32, i32, f32, i32, vp, vp, sz, vp]),
+    "mi355_rope_kv_write_rows_ragged": (i32, [vp, vp, i32, i32, vp, vp, i32, i32, vp, vp, vp, i32, i32, i32, i32, C.POINTER(KVLayer), vp, vp, vp]),
+    "mi355_paged_attn_rows_ragged": (i32, [vp, C.POINTER(KVLayer), vp, i32, vp, vp, i32, i32, i32, i32, f32, i32, vp, vp, sz, vp]),
     "mi355_paged_attn_rows": (i32, [vp, C.POINTER(KVLayer), vp, i32, vp, i32, i32, i32, f32, i32, vp, vp, sz, vp]),
     "mi355_argmax": (i32, [vp, i32, i32, i32, vp, vp, sz, vp]),
     "mi355_softmax_rows": (i32, [vp, i32, i32, i32, f32, vp, vp]),
@@ -151,6 +153,7 @@ SIGNATURES = {
     "mi355_decoder_step": (i32, [vp, i32, vp]),
     "mi355_decoder_prefill_workspace_bytes": (sz, [vp, i32, i32]),
     "mi355_decoder_prefill": (i32, [vp, vp, vp, vp, i32, i32, vp, vp, vp, sz, vp]),
+    "mi355_decoder_prefill_ragged": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, sz, vp]),
     "mi355_decoder_set_prefill_rope_table": (i32, [vp, vp]),
     "mi355_decoder_capture": (i32, [vp, i32]),
     "mi355_decoder_replay": (i32, [vp, i32, i32, vp]),

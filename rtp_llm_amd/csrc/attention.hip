@@ -43,7 +43,9 @@ struct AttnParams {
     float*         tmp_out; // [B][nh][P][hd]
     float*         tmp_ml;  // [B][nh][P][2]
     int B, nh, nkv, G, page, max_blocks, P, PS, seq_add, max_seq, num_blocks;
-    int q_len, R, ntile;   // rows per sequence, rows per 16-column tile (16 / G), row tiles per sequence
+    int q_len, R, ntile;   // rows per sequence (of the longest, with row_start), rows per 16-column tile (16 / G), row tiles per sequence
+    const int32_t* row_start; // non-null (the two-tile instances): sequence b has rows row_start[b] .. row_start[b + 1] - 1, no padding rows between
+    int rows;              // all rows
     uint32_t page_magic;   // 2^32 / page + 1: floor(t / page) == (t * magic) >> 32 for t * page < 2^32
     float scale_log2; // softmax scale * log2(e)
     int img_mblk;     // > 0: out is an activation image of that many row blocks (common.h act_img_index) instead of [rows][nh * hd]
@@ -91,8 +93,12 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     const int part = blockIdx.x, kh = blockIdx.y;
     const int b = blockIdx.z / p.ntile, tile = blockIdx.z - b * p.ntile;
     const int RT = NT * p.R;                       // query rows of this block
-    const int row0 = b * p.q_len + tile * RT;      // first row (index into q / positions / out)
-    const int nrows = min(RT, p.q_len - tile * RT);
+    int base = b * p.q_len, len = p.q_len;
+    if constexpr (NT == 2) {
+        if (p.row_start) { base = p.row_start[b]; len = p.row_start[b + 1] - base; if (tile * RT >= len) return; }
+    }
+    const int row0 = base + tile * RT;             // first row (index into q / positions / out)
+    const int nrows = min(RT, len - tile * RT);
     // context of a row = its position + 1 (seq_add = 1: positions hold tokens already cached) or seq_lens[row] itself;
     // a negative value marks a padding row.  The block walks up to the longest context of its rows.
     const int pstart = part * p.PS;
@@ -538,7 +544,7 @@ template <int HD, bool BF = false>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(const AttnParams p) {
     const int lane = threadIdx.x & 63;
     const int gid = blockIdx.x * 4 + (threadIdx.x >> 6); // (row, h)
-    if (gid >= p.B * p.q_len * p.nh) return;
+    if (gid >= p.rows * p.nh) return;
     const int row = gid / p.nh;
     // ONE memory round trip: the row's length, the (max, sum) pairs (partition i in lane i) and the first 16 partial rows are requested
     // together; only the masks depend on the length.  (A loop bounded by the length waited for it, then walked the pairs one load at a
@@ -633,7 +639,8 @@ extern "C" size_t mi355_paged_attn_workspace_bytes(int32_t B, int32_t nh, int32_
 namespace {
 int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table, int32_t max_blocks_per_seq,
                 const int32_t* seq_lens, int32_t seq_lens_minus_one, int32_t B, int32_t q_len, int32_t nh, float scale,
-                int32_t max_seq_len, void* out, void* workspace, size_t workspace_bytes, mi355_stream_t stream, int img_mblk = 0) {
+                int32_t max_seq_len, void* out, void* workspace, size_t workspace_bytes, mi355_stream_t stream, int img_mblk = 0,
+                const int32_t* row_start = nullptr, int32_t total_rows = 0) {
     MI355_CHECK_ARG(q && kv && kv->kv_base && block_table && seq_lens && out, "paged_attn: null pointer");
     MI355_CHECK_ARG(kv->hd == 64 || kv->hd == 128, "paged_attn: hd=%d (64 or 128)", kv->hd);
     MI355_CHECK_ARG(kv->page >= 16 && kv->page % 8 == 0, "paged_attn: page=%d (>= 16, multiple of 8)", kv->page);
@@ -656,11 +663,12 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     p.stamps = g_attn_stamps;
 #endif
     p.page_magic = (uint32_t)((1ull << 32) / (unsigned)kv->page + 1);
-    const int NT = q_len > p.R ? 2 : 1;                 // column tiles per block: 2 x R rows share one pass over the KV
+    const int NT = q_len > p.R || row_start ? 2 : 1;    // column tiles per block: 2 x R rows share one pass over the KV
     p.ntile = cdiv(q_len, NT * p.R);
     p.P = plan_partitions(B * p.ntile, kv->nkv, max_seq_len, &p.PS);
     p.scale_log2 = scale * 1.4426950408889634f;
-    const size_t rows = (size_t)B * q_len;
+    const size_t rows = row_start ? (size_t)total_rows : (size_t)B * q_len;
+    p.row_start = row_start; p.rows = (int)rows;
     const size_t need = p.P > 1 ? rows * nh * p.P * (kv->hd + 2) * sizeof(float) : 0;
     if (need > workspace_bytes || (need && !workspace)) {
         mi355_set_error("paged_attn: workspace %zu < %zu", workspace_bytes, need);
@@ -726,6 +734,16 @@ extern "C" int mi355_paged_attn_rows(const void* q, const mi355_kv_layer_t* kv, 
                                      mi355_stream_t stream) {
     return launch_attn(q, kv, block_table, max_blocks_per_seq, positions, 1, B, q_len, nh, scale, max_seq_len, out, workspace,
                        workspace_bytes, stream);
+}
+
+// the same without padding rows: q, positions and out hold `rows` rows, sequence b those from row_start[b] (device, [B + 1]) on, at most q_len
+extern "C" int mi355_paged_attn_rows_ragged(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table,
+                                            int32_t max_blocks_per_seq, const int32_t* positions, const int32_t* row_start, int32_t B, int32_t q_len,
+                                            int32_t rows, int32_t nh, float scale, int32_t max_seq_len, void* out, void* workspace,
+                                            size_t workspace_bytes, mi355_stream_t stream) {
+    MI355_CHECK_ARG(row_start && rows > 0 && (long)rows <= (long)B * q_len, "paged_attn_rows_ragged: %d rows, %d sequences of at most %d", rows, B, q_len);
+    return launch_attn(q, kv, block_table, max_blocks_per_seq, positions, 1, B, q_len, nh, scale, max_seq_len, out, workspace,
+                       workspace_bytes, stream, 0, row_start, rows);
 }
 
 // the same with `out` written as an activation image (mi355_act_image_*: B * q_len <= 64 rows, K = nh * hd) for the O projection's

@@ -23,6 +23,7 @@ struct RopeParams {
     const int32_t* positions;
     const int32_t* block_table;
     int            max_blocks, T, nh, nkv, hd, page, max_pos, num_blocks, q_len;
+    const int32_t* row_seq;   // non-null: the sequence of every row (t / q_len otherwise)
     int32_t*       oob_count;
     void*          kv_base;
     float*         scale_base;
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(const RopeParams p) 
     const int pos_lim = min(p.max_pos, p.max_blocks * p.page);
     const int pos = min(max(pos_in, 0), pos_lim - 1);       // clamped: the rotation table and the block table stay in range
     const bool is_v = h >= p.nh + p.nkv;
-    const int blk = (h >= p.nh) ? p.block_table[(size_t)(t / p.q_len) * p.max_blocks + pos / p.page] : 0;
+    const int blk = (h >= p.nh) ? p.block_table[(size_t)(p.row_seq ? p.row_seq[t] : t / p.q_len) * p.max_blocks + pos / p.page] : 0;
     float2 cs = {1.f, 0.f};
     if (!is_v && act) cs = *reinterpret_cast<const float2*>(p.cos_sin + ((size_t)pos * half + lane) * 2);
     float x0 = 0.f, x1 = 0.f;
@@ -143,6 +144,16 @@ extern "C" int mi355_rope_kv_write_rows(const void* qkv_f16, const float* partia
                                         const int32_t* positions, const int32_t* block_table, int32_t max_blocks_per_seq,
                                         int32_t T, int32_t q_len, int32_t nh, const mi355_kv_layer_t* kv, void* q_out,
                                         int32_t* oob_count, mi355_stream_t stream) {
+    return mi355_rope_kv_write_rows_ragged(qkv_f16, partials, nsplit, ld, qkv_bias, cos_sin, rope_dim, max_pos, positions, nullptr, block_table,
+                                           max_blocks_per_seq, T, q_len, nh, kv, q_out, oob_count, stream);
+}
+
+// row_seq non-null (device, [T]): the sequence of every row; q_len is 1 then
+extern "C" int mi355_rope_kv_write_rows_ragged(const void* qkv_f16, const float* partials, int32_t nsplit, int32_t ld,
+                                               const void* qkv_bias, const float* cos_sin, int32_t rope_dim, int32_t max_pos,
+                                               const int32_t* positions, const int32_t* row_seq, const int32_t* block_table, int32_t max_blocks_per_seq,
+                                               int32_t T, int32_t q_len, int32_t nh, const mi355_kv_layer_t* kv, void* q_out,
+                                               int32_t* oob_count, mi355_stream_t stream) {
     MI355_CHECK_ARG(q_len >= 1 && T % q_len == 0, "rope_kv_write: T=%d must be a multiple of q_len=%d", T, q_len);
     MI355_CHECK_ARG((qkv_f16 != nullptr) != (partials != nullptr), "rope_kv_write: exactly one of qkv_f16 / partials");
     MI355_CHECK_ARG(kv && kv->kv_base && cos_sin && positions && block_table && q_out, "rope_kv_write: null pointer");
@@ -161,7 +172,7 @@ extern "C" int mi355_rope_kv_write_rows(const void* qkv_f16, const float* partia
     p.qkv = (const f16*)qkv_f16; p.partials = partials; p.nsplit = nsplit; p.ld = ld; p.bias = (const f16*)qkv_bias;
     p.cos_sin = cos_sin; p.positions = positions; p.block_table = block_table; p.max_blocks = max_blocks_per_seq;
     p.T = T; p.nh = nh; p.nkv = kv->nkv; p.hd = kv->hd; p.page = kv->page; p.kv_base = kv->kv_base;
-    p.max_pos = max_pos; p.num_blocks = kv->num_blocks; p.oob_count = oob_count; p.q_len = q_len;
+    p.max_pos = max_pos; p.num_blocks = kv->num_blocks; p.oob_count = oob_count; p.q_len = q_len; p.row_seq = row_seq;
     p.scale_base = kv->scale_base; p.kv_int8 = kv->kv_dtype == MI355_KV_INT8; p.q_out = (f16*)q_out;
     if (bf)
         hipLaunchKernelGGL(rope_kv_write_kernel<true>, dim3(T, cdiv(nheads, 4)), dim3(256), 0, (hipStream_t)stream, p);

@@ -553,7 +553,7 @@ class DecoderEngine:
 
     def prefill(self, prompts: List[List[int]], block_table, chunk: int = 512, start: Optional[List[int]] = None) -> torch.Tensor:
         """Real prefill (csrc/engine.cpp mi355_decoder_prefill): the prompts go through the large-M GEMMs and the causal
-        multi-row attention in chunks of `chunk` tokens per sequence (ragged prompts are padded with position -1 rows).
+        multi-row attention in chunks of `chunk` tokens per sequence (the rows of ragged prompts lie back to back).
         `start[b]` tokens of sequence b are already cached.  Returns the fp32 logits [nseq, vocab] of every sequence's LAST
         prompt token (its K/V is in the cache afterwards: decoding continues with the sampled token at position len)."""
         nseq = len(prompts)
@@ -583,34 +583,35 @@ class DecoderEngine:
         btd[:, : bt.shape[1]].copy_(bt)
         longest = max(len(p) for p in prompts)
         logits = torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
-        done = torch.zeros(nseq, dtype=torch.bool)
         for c0 in range(0, longest, chunk):
             q_len = min(chunk, longest - c0)
-            toks = torch.zeros(nseq, q_len, dtype=torch.int32)
-            pos = torch.full((nseq, q_len), -1, dtype=torch.int32)
+            counts = [max(0, min(q_len, len(p) - c0)) for p in prompts]
+            first = [sum(counts[:b]) for b in range(nseq + 1)]
+            T = first[nseq]
+            toks = torch.cat([torch.as_tensor(p[c0:c0 + n], dtype=torch.int32) for p, n in zip(prompts, counts)])
+            pos = torch.cat([torch.arange(start[b] + c0, start[b] + c0 + n, dtype=torch.int32) for b, n in enumerate(counts)])
+            ending = [b for b, p in enumerate(prompts) if counts[b] and c0 + counts[b] == len(p)]
             last = torch.zeros(nseq, dtype=torch.int32)
-            need_logits = torch.zeros(nseq, dtype=torch.bool)
-            for b, p in enumerate(prompts):
-                n = max(0, min(q_len, len(p) - c0))
-                if n:
-                    toks[b, :n] = torch.tensor(p[c0:c0 + n], dtype=torch.int32)
-                    pos[b, :n] = torch.arange(start[b] + c0, start[b] + c0 + n, dtype=torch.int32)
-                    if c0 + n == len(p):
-                        last[b], need_logits[b] = b * q_len + n - 1, True
-            T = nseq * q_len
+            for b in ending:
+                last[b] = first[b] + counts[b] - 1
+            # the chunk's integers in one copy: tokens, positions, logit rows and, unless every sequence has q_len rows, where each sequence's rows lie
+            parts = [toks, pos, last]
+            if T < nseq * q_len:
+                parts += [torch.repeat_interleave(torch.arange(nseq, dtype=torch.int32), torch.tensor(counts)), torch.tensor(first, dtype=torch.int32)]
+            td, pd, ld, *ragged = torch.cat(parts).to(dev).split([p.numel() for p in parts])
             ws_bytes = self.lib.mi355_decoder_prefill_workspace_bytes(self.handle, T, nseq)
             if getattr(self, "_prefill_ws", None) is None or self._prefill_ws.numel() < ws_bytes:
                 self._prefill_ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            tmp_logits = torch.empty(nseq, self.cfg.vocab, dtype=torch.float32, device=dev) if bool(need_logits.any()) else None
-            td, pd, ld = toks.reshape(-1).to(dev), pos.reshape(-1).to(dev), last.to(dev)
-            _C.check(self.lib.mi355_decoder_prefill(self.handle, td.data_ptr(), pd.data_ptr(), btd.data_ptr(), nseq, q_len,
-                                                    ld.data_ptr() if tmp_logits is not None else None,
-                                                    tmp_logits.data_ptr() if tmp_logits is not None else None,
-                                                    self._prefill_ws.data_ptr(), self._prefill_ws.numel(), st), "decoder_prefill")
-            if tmp_logits is not None:
-                sel = need_logits.to(dev)
+            tmp_logits = torch.empty(nseq, self.cfg.vocab, dtype=torch.float32, device=dev) if ending else None
+            seqd, firstd = (r.data_ptr() for r in ragged) if ragged else (None, None)
+            _C.check(self.lib.mi355_decoder_prefill_ragged(self.handle, td.data_ptr(), pd.data_ptr(), seqd, firstd, btd.data_ptr(), nseq, q_len, T,
+                                                           ld.data_ptr() if ending else None, tmp_logits.data_ptr() if ending else None,
+                                                           self._prefill_ws.data_ptr(), self._prefill_ws.numel(), st), "decoder_prefill")
+            if len(ending) == nseq:
+                logits = tmp_logits
+            elif ending:
+                sel = torch.tensor(ending, device=dev)
                 logits[sel] = tmp_logits[sel]
-            done |= need_logits
         return logits
 
     def generate(self, prompts: List[List[int]], block_table, max_new_tokens: int, prefill_chunk: int = 512) -> List[List[int]]:
