@@ -7,8 +7,10 @@
 //   * block = 8 waves; a wave owns 1, 2 or 4 adjacent 16-column weight tiles and all rows of the block's tile (32, 64 or 128);
 //   * per 128-k chunk a wave dequantises its tiles' A-fragments ONCE (operand side) and uses each for every row block: at 128 rows 64 v_mfma_f32_16x16x32 per
 //     104 dequant VALU, so the matrix pipe, not the VALU, sets the pace; the second wave of each SIMD dequantises while the first one multiplies;
-//   * the activation chunk (128 rows x 128 k = 32 KiB) is staged once per block in LDS in the fragment-major, XOR-swizzled image of gemm.hip (conflict-free
-//     ds_read_b128) and double-buffered;
+//   * the activation chunk (128 rows x 128 k = 32 KiB) goes to LDS by DMA while the chunk before it is multiplied, row by row with the 16-byte pieces of a row swizzled
+//     by the row (conflict-free ds_read_b128); two buffers, one barrier a chunk.  Through registers, as before, the chunk cost 16 of them, and with them the reach of the
+//     fragment reads: 3 fragments are now read ahead of their products.  37888 x 3584 in fp16 W4 at 4096 rows 1066 -> 1002 us, 3584 x 18944 493 -> 459 us (at the rate of
+//     a large dense product on the 224 of 256 CUs that have a block); 8 bits at 1055 rows 343 -> 315 and 159 -> 157 us; bf16 W16 9728 x 896 at 512 rows 20.3 -> 17.8 us;
 //   * weights stream from HBM/L2 once per row tile (the row tiles of a column tile run back to back on different CUs and meet in L2 / Infinity Cache),
 //     through a 2-deep register ring, buffer range checks instead of tail branches.
 #include "gemm_common.h"
@@ -53,14 +55,14 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     constexpr bool GROUPED = GS > 0;
     constexpr bool CSCALE = BF && GROUPED;                    // the group's scale on the accumulator side
     constexpr int XSLOTS = 256 * MB;                          // 16-byte pieces of an x chunk tile
-    constexpr int GT = 512 / KS;                              // threads of a K slice
-    constexpr int UPT = XSLOTS / GT;                          // pieces per thread
+    constexpr int UPT = XSLOTS / (64 * NWN);                  // staging loads per wave
+    constexpr int WLD = TPW * (LPC + (GS > 0 ? NSUB : 0));    // weight loads per wave and chunk
     __shared__ u32x4 xs[KS][2][XSLOTS];
     static_assert(KS == 1 || (size_t)(KS - 1) * NWN * TPW * MB * 1024 <= sizeof(u32x4) * 2 * KS * XSLOTS, "the slices' sums meet in the x buffers");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ks = wave / NWN, tg = tid - ks * GT;
+    const int ks = wave / NWN;
     const int jj = lane & 15, q = lane >> 4;
     const int m0 = blockIdx.y * BM;
     const int nt_base = (blockIdx.x * NWN + wave % NWN) * TPW;
@@ -81,29 +83,28 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     }
     __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, p.x_bytes, FLAGS);
 
-    // x staging: thread owns pieces pi = tg + GT u: row j = pi >> 4 of the tile, 16-byte piece pp = pi & 15 of the chunk
+    // x staging: load u of a wave covers 64 pieces of 16 bytes = 4 rows of the chunk; piece pp of row j lies at j * 16 + (pp ^ (j & 15))
     uint32_t xoff[UPT];
-    int xslot[UPT];
-    bool xrow_ok[UPT];
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-        const int pi = tg + GT * u, j = pi >> 4, pp = pi & 15;
-        xrow_ok[u] = m0 + j < p.M;
-        xoff[u]  = (uint32_t)(((size_t)(m0 + j) * p.K + pp * 8) * 2);
-        xslot[u] = pp * (16 * MB) + (j ^ (pp & 3));
+        const int pi = (u * NWN + wave % NWN) * 64 + lane, j = pi >> 4, pp = (pi & 15) ^ (j & 15);
+        xoff[u] = (uint32_t)(((size_t)min(m0 + j, p.M - 1) * p.K + pp * 8) * 2);      // rows past M repeat the last one: their sums are never stored
     }
-    const uint32_t OOBX = 0x80000000u;
-    auto load_x = [&](u32x4 (&xr)[UPT], int c) {
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&xs[ks][0][0];
+    const bool dma = (uintptr_t)p.x % 16 == 0 && p.K % 8 == 0;
+    auto load_x = [&](int c, int buf) {
+        if (dma && c * 128 + 128 <= p.K) {
 #pragma unroll
-        for (int u = 0; u < UPT; ++u) {
-            const int pp = (tg + GT * u) & 15;
-            const bool ok = xrow_ok[u] && c < KC && c * 128 + pp * 8 < p.K;   // rows past M / columns past K read as zero
-            xr[u] = bload128<0>(rx, ok ? xoff[u] : OOBX, (uint32_t)c * 256u);
+            for (int u = 0; u < UPT; ++u)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             :: "s"(lds0 + (buf * XSLOTS + (u * NWN + wave % NWN) * 64) * 16), "v"(xoff[u]), "s"((const char*)p.x + (size_t)c * 256) : "memory", "m0");
+        } else {                                              // the last chunk of a K that is no multiple of 128 (columns past K are zero), a tensor off 16 bytes
+#pragma unroll
+            for (int u = 0; u < UPT; ++u) {
+                const int pi = (u * NWN + wave % NWN) * 64 + lane, pp = (pi & 15) ^ (pi >> 4 & 15);
+                xs[ks][buf][pi] = bload128<0>(rx, c * 128 + pp * 8 < p.K ? xoff[u] : 0x80000000u, (uint32_t)c * 256u);
+            }
         }
-    };
-    auto store_x = [&](const u32x4 (&xr)[UPT], int buf) {
-#pragma unroll
-        for (int u = 0; u < UPT; ++u) xs[ks][buf][xslot[u]] = xr[u];
     };
 
     const uint32_t lane16 = lane * 16u, jj4 = jj * 4u;
@@ -135,13 +136,9 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     const W4Consts w4c = w4_consts();
     const f16x2 c960 = {(f16)960.f, (f16)960.f};
 
-    u32x4 xr[UPT];
-    load_x(xr, ks);
+    load_x(ks, 0);
     load_w(0, ks);
-    store_x(xr, 0);
-    load_x(xr, ks + KS);
     load_w(1, ks + KS);
-    __syncthreads();
 
     auto dq = [&](int d, int t, int s) -> u32x4 {
         if constexpr (WBITS == 16) return wr[d][t][s];
@@ -168,7 +165,12 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
             return __builtin_bit_cast(u32x4, dequant_w8<GROUPED>(w[(s & 1) * 2], w[(s & 1) * 2 + 1], zn, sc));
         }
     };
-    auto frag = [&](int buf, int s, int mb) { return xs[ks][buf][(s * 4 + q) * (16 * MB) + mb * 16 + (jj ^ q)]; };
+    auto frag = [&](int buf, int s, int mb) { return xs[ks][buf][mb * 256 + jj * 16 + ((s * 4 + q) ^ jj)]; };
+    u32x4 an[TPW];                                            // operands of the next k-step (a chunk starts with those the one before left)
+    auto next = [&](int d, int s) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) an[t] = dq(d, t, s);
+    };
     auto compute = [&](int d, int buf) {
         if constexpr (CSCALE) {              // a group's sums on accumulators of their own, scaled as they join the tile's
 #pragma unroll
@@ -195,49 +197,57 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
                         for (int mb = 0; mb < MB; ++mb) acc[t][mb][r] = __builtin_fmaf(sc, ag[t][mb][r], acc[t][mb][r]);
                     }
             }
-        } else if constexpr (TPW <= 2 && WBITS != 16) {   // all operands of the chunk first, then the MFMAs
-            u32x4 a[TPW][4];
+        } else {
+            // Fragment i + AHEAD is read while fragment i is multiplied, the next k-step's operands are formed between the products: left to itself the compiler
+            // reads two fragments, waits for them and multiplies (one LDS latency per 8 products and wave)
+            constexpr int AHEAD = WBITS == 8 && TPW == 4 ? 1 : 3, N = 4 * MB;
+            u32x4 b[AHEAD + 1];
 #pragma unroll
-            for (int t = 0; t < TPW; ++t)
-#pragma unroll
-                for (int s = 0; s < 4; ++s) a[t][s] = dq(d, t, s);
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const u32x4 b = frag(buf, s, mb);
-#pragma unroll
-                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma_act<BF>(a[t][s], b, acc[t][mb]);
-                }
-        } else {                             // per k-step: TPW operands (16 registers), MB fragment reads, MB x TPW MFMAs
+            for (int i = 0; i < AHEAD; ++i) b[i] = frag(buf, i / MB, i % MB);
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 u32x4 a[TPW];
 #pragma unroll
-                for (int t = 0; t < TPW; ++t) a[t] = dq(d, t, s);
+                for (int t = 0; t < TPW; ++t) a[t] = an[t];
+                next(s == 3 ? d ^ 1 : d, (s + 1) & 3);
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
-                    const u32x4 b = frag(buf, s, mb);
+                    const int i = s * MB + mb;
+                    if (i + AHEAD < N) b[(i + AHEAD) % (AHEAD + 1)] = frag(buf, (i + AHEAD) / MB, (i + AHEAD) % MB);
 #pragma unroll
-                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma_act<BF>(a[t], b, acc[t][mb]);
+                    for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma_act<BF>(a[t], b[i % (AHEAD + 1)], acc[t][mb]);
+                }
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                if (i + AHEAD < N) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+                for (int t = 0; t < TPW; ++t) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if constexpr (WBITS != 16) __builtin_amdgcn_sched_group_barrier(0x002, (14 + MB - 1) / MB, 0);
                 }
             }
         }
     };
 
-    for (int c = ks; c - ks < KC; c += 2 * KS) {     // the same number of rounds for every slice; chunks past KC are zero rows of x
-        // chunk c (buffer 0, ring 0); x(c + KS) is in registers, w(c + KS) in ring 1
-        compute(0, 0);
-        store_x(xr, 1);
-        load_x(xr, c + 2 * KS);
-        load_w(0, c + 2 * KS);
-        __syncthreads();
-        if (c - ks + KS < KC) compute(1, 1);
-        store_x(xr, 0);
-        load_x(xr, c + 3 * KS);
-        load_w(1, c + 3 * KS);
-        __syncthreads();
+    // Chunk c lies in buffer and ring d.  One barrier: behind it every wave's part of chunk c is in LDS and chunk c - KS is done with, so that the DMA of chunk c + KS may
+    // go over it.  At most the weights of chunk c + KS are younger than the DMA of chunk c.
+    auto chunk = [&](int c, int d) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt((WLD & 15) | (7 << 4) | ((WLD >> 4) << 14));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (c + KS < KC) load_x(c + KS, d ^ 1);
+        if (c < KC) compute(d, d);                   // slices past the end have nothing left
+        load_w(d, c + 2 * KS);
+    };
+    if constexpr (!CSCALE) next(0, 0);
+    for (int c = ks; c - ks < KC; c += 2 * KS) {     // the same number of rounds for every slice
+        chunk(c, 0);
+        if (c - ks + KS < KC) chunk(c + KS, 1);
     }
+    if constexpr (KS > 1) __syncthreads();
 
     if constexpr (KS > 1) {                          // the slices' sums, in slice order
         f32x4* red = (f32x4*)&xs[0][0][0];
@@ -288,14 +298,14 @@ constexpr int kPrefillShapeCount = sizeof(kPrefillShapes) / sizeof(kPrefillShape
 
 // The shape of a call: a time model in us.  A round of a block (KS chunks of 128 k) takes `lat` alone on its CU -- loads, LDS, barrier -- and `sat` of a CU whose
 // share of the grid keeps it busy; the share counts half as the exact quotient and half as the whole blocks of the fullest CU.  Measured (random operands, one MI355X) per
-// operand class over M = 70..4096 at the Qwen2-0.5B and 7B projections: the pick is within 10 % of the fastest shape.  Examples, us at 128x512 / 128x256 / 64x256 /
-// 64x128 / 64x64 / 32x64 / 32x32 tiles: fp16 W4 37888 x 3584 at M = 4096 1088 / 1155 / 1183 / 1368 / 1722 / 1965 / 2945, 3584 x 18944 at M = 128 424 / 250 / 147 / 130 / 66 / 51 / 47;
-// W16 9728 x 896 at M = 512 - / 26 / 26 / 20 / 23 / 27 / 43; bf16 W4 37888 x 3584 at M = 512 - / 195 / 232 / 205 / 238 / 290 / 420.
+// operand class over M = 70..4096 at the Qwen2-0.5B and 7B projections: the pick is within 8 % of the fastest shape.  Examples, us at 128x512 / 128x256 / 64x256 /
+// 64x128 / 64x64 / 32x64 / 32x32 tiles: fp16 W4 37888 x 3584 at M = 4096 1002 / 1057 / 1144 / 1244 / 1503 / 1806 / 2516, bf16 W4 3584 x 18944 at M = 128 - / 309 / 223 / 144 / 81 /
+// 64 / 50; W16 9728 x 896 at M = 512 - / 22 / 23 / 18 / 18 / 23 / 33; bf16 W4 37888 x 3584 at M = 512 - / 192 / 180 / 188 / 222 / 263 / 363.
 struct PrefillCost { double lat, sat; };
 constexpr PrefillCost kPrefillCost[3][kPrefillShapeCount] = {
-    {{3.15, 4.1}, {1.85, 2.2}, {1.1, 1.14}, {0.95, 0.66}, {1.1, 0.83}, {0.8, 0.475}, {1.55, 0.71}},     // codes on the operand side
-    {{1e9, 1e9},  {2.25, 2.4}, {1.65, 1.65}, {0.95, 0.76}, {1.25, 0.9}, {0.85, 0.56}, {1.6, 0.8}},      // bf16 under group scales: two sets of accumulators
-    {{1e9, 1e9},  {2.6, 3.8}, {1.6, 2.1}, {1.05, 1.0}, {1.55, 1.07}, {1.1, 0.64}, {2.0, 1.11}},         // 16-bit weights
+    {{2.82, 3.58}, {1.59, 2.02}, {1.12, 1.14}, {0.69, 0.613}, {0.75, 0.708}, {0.53, 0.439}, {0.61, 0.585}},     // codes on the operand side
+    {{1e9, 1e9},   {2.16, 2.45}, {1.52, 1.32}, {0.94, 0.708}, {0.98, 0.856}, {0.72, 0.507}, {0.69, 0.708}},      // bf16 under group scales: two sets of accumulators
+    {{1e9, 1e9},   {1.41, 2.82}, {0.92, 1.84}, {0.49, 0.856}, {0.49, 0.779}, {0.45, 0.532}, {0.37, 0.742}},     // 16-bit weights
 };
 int pick_shape(const GemmParams& p, int wbits, double* t_best) {
     const PrefillCost* cost = kPrefillCost[wbits == 16 ? 2 : (p.bf16 && wbits == 4) ? 1 : 0];
