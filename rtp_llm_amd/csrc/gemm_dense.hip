@@ -233,11 +233,13 @@ __global__ __launch_bounds__(256) void dense_tile_bf16_kernel(DenseParams p) {
 // ds_write) into NS stages, one barrier per tile.  An LDS row is the BK * 2 bytes of a K tile; its 16-byte pieces are permuted by the row (applied to the source
 // address, which the DMA leaves free per lane), so that the 16-row fragment reads hit every bank once.  w is the MFMA's first operand: a lane ends with four
 // consecutive outputs of one row.  The sums run over k in steps of 32 like the other tile kernel's: same bits.
-// NS = 2: tiles of 64, two blocks or more per CU hide each other's waits.  NS >= 3: tiles of 32, a wave reads the fragments of tile t + 1 between the products of tile t.
-// Time in us of 256x256 (NS 4) / 128x128 (NS 2) / 64x128 (NS 2) / 64x128 (NS 4) tiles and of the 64x128 kernel that stages through registers:
-//   M x N x K       8192x11264x2048 gated  355 / 357 / 424 / 567, 599    8192x2048x5632  148 / 175 / 214 / 297, 307    8192x2048x2048  63 / 71 / 83 / 111, 120
-//                   2048x11264x2048 gated  109 /  96 / 108 / 146, 156    2048x2048x2048   48 /  26 /  25 /  31,  41     512x2048x5632 109 / 57 / 48 / 43, 77
-//                   1537x1024x1024          28 /  12 /  10 /   9,  21      70x2048x2048   42 /  18 /  15 /  12,  32
+// BK = 64: NS = 2, two blocks or more per CU hide each other's waits; NS = 3 and 4 where few blocks have to keep the loads in flight alone.  BK = 32: a wave reads the
+// fragments of tile t + 1 between the products of tile t.
+// Time in us of 256x256 (BK 32, NS 4) / 128x128 (NS 2) / 64x128 (NS 2) / 64x128 (NS 3) / 64x64 (NS 4) tiles and of the 64x128 kernel that stages through registers;
+// weights not in L2, as in a model:
+//   M x N x K       8192x2048x2048 62 / 71 / 82 / 86 / 112, 118    6148x1408x1024 gated 33 / 31 / 29 / 32 / 37, 43     768x11264x2048 gated 50 / 52 / 49 / 53 / 61, 73
+//                   1537x2176x1024 30 / 15 / 14 / 13 /  17,  25    1537x1024x1024       29 / 15 / 13 / 11 / 10, 21     768x2048x5632       109 / 57 / 52 / 36 / 34, 77
+//                   1537x3072x1024 30 / 20 / 18 / 21 /  22,  30    1537x1024x2816       60 / 32 / 29 / 21 / 20, 45      70x2048x2048        42 / 23 / 20 / 16 / 12, 32
 __device__ __forceinline__ void dn_dma16(uint32_t lds, uint32_t voff, const void* base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
@@ -252,10 +254,10 @@ template <int VM> __device__ __forceinline__ void dn_wait() {
 template <int BM, int BN, int WM, int WN, int BK, int NS>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_kernel(DenseParams p) {
     constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, MI = WM / 16, NJ = WN / 16;
-    constexpr bool AHEAD = NS >= 3;                                           // fragments of tile t + 1 are read while tile t is multiplied
+    constexpr bool AHEAD = BK == 32;                                          // fragments of tile t + 1 are read while tile t is multiplied
     constexpr int RB = BK * 2, PPR = BK / 8, RPL = 64 / PPR;                  // bytes and 16-byte pieces of a row, rows per wave load
     constexpr int STAGE = (BM + BN) * RB, ULD = (BM + BN) / (RPL * NW), ULA = BM / (RPL * NW);   // loads per wave and tile; the first ULA are rows of x
-    static_assert((AHEAD ? BK == 32 : BK == 64) && BM % (RPL * NW) == 0 && BN % (RPL * NW) == 0, "whole wave loads per operand");
+    static_assert((AHEAD ? NS >= 3 : BK == 64) && BM % (RPL * NW) == 0 && BN % (RPL * NW) == 0, "whole wave loads per operand");
     constexpr int PH = MI >= 4 && NS * STAGE >= NW * 16384 ? 4 : MI >= 2 ? 2 : 1;   // 16-row blocks of results that pass through LDS together
     static_assert(WN == 64 && NS * STAGE >= NW * PH * 4096, "a wave's output columns; room for its results");
     __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
@@ -315,12 +317,15 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
 #pragma unroll
     for (int t = 0; t < NS - 1; ++t) if (t < nk) issue(t, t);
     if constexpr (!AHEAD) {
+        int at = 0;
         for (int kt = 0; kt < nk; ++kt) {
-            dn_wait<0>();                                                   // this wave's part of tile kt is in LDS, its reads of tile kt - 1 are done
+            // this wave's part of tile kt is in LDS, its reads of tile kt - 1 are done
+            if (NS == 2 || kt + NS - 2 >= nk) dn_wait<0>(); else dn_wait<ULD * (NS - 2)>();
             __builtin_amdgcn_s_barrier();
-            if (kt + 1 < nk) issue((kt + 1) & 1, kt + 1);
+            if (kt + NS - 1 < nk) issue(at == 0 ? NS - 1 : at - 1, kt + NS - 1);
 #pragma unroll
-            for (int ks = 0; ks < BK / 32; ++ks) { load(fa, kt & 1, ks); multiply(fa); }
+            for (int ks = 0; ks < BK / 32; ++ks) { load(fa, at, ks); multiply(fa); }
+            at = at + 1 == NS ? 0 : at + 1;
         }
     } else {
         if (nk > 0) {
@@ -656,21 +661,19 @@ void launch_tiles_bf16(const DenseParams& p, int gy64, int gz, hipStream_t st) {
         return;
     }
     // the shape with the least expected time, us per 32 columns of k: a constant and the blocks per CU times what one costs a busy CU (256 x 256: whole rounds
-    // count half, one block fills a CU).  Measured at M = 70..8192, N = 16..32000, K = 16..5632: within 10 % of the fastest of the four.  Grouped rows
-    // come in tiles of 64.
+    // count half, one block fills a CU; 64x128 in three stages: two blocks fill one).  Measured at M = 70..8192, N = 16..32000, K = 16..5632: within 10 % of the fastest.
+    // Grouped rows come in tiles of 64.
     auto share = [&](int bm, int bn) { return (double)((p.N + bn - 1) / bn) * (p.offs ? gy64 : (p.M + bm - 1) / bm) * gz / 256.0; };
-    const double sa = share(256, 256), sb = share(128, 128), sc = share(64, 128), k = p.K / 32.0;
-    const double ta = k * fmax(0.65, 0.475 * (sa + ceil(sa))) + 12.0, tb = k * fmax(0.30, 0.255 * sb + 0.13) + 5.0;
-    const double tc = k * fmax(0.23, 0.15 * sc + 0.10) + 4.0, td = k * fmax(0.185, 0.19 * sc + 0.10) + 4.0;
+    const double sa = share(256, 256), sb = share(128, 128), sc = share(64, 128), se = share(64, 64), k = p.K / 32.0;
+    const double ta = p.offs ? 1e30 : k * fmax(0.65, 0.475 * (sa + ceil(sa))) + 12.0, tb = p.offs ? 1e30 : k * fmax(0.34, 0.255 * sb + 0.13) + 5.0;
+    const double tc = k * fmax(0.27, 0.15 * sc + 0.09) + 4.0, td = k * (sc <= 2.0 ? 0.18 + 0.06 * sc : 0.15 * sc + 0.22) + 4.0;
+    const double te = k * fmax(0.125, 0.105 * se + 0.02) + 4.0, t = fmin(fmin(ta, tb), fmin(tc, fmin(td, te)));
     const int gn = (p.N + 127) / 128;
-    if (p.offs || (tc <= tb && tc <= ta) || (td <= tb && td <= ta)) {
-        if (td < tc) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 32, 4>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
-        else         hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 2>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
-    } else if (tb < ta) {
-        hipLaunchKernelGGL((dense_dma_bf16_kernel<128, 128, 32, 64, 64, 2>), dim3(gn, (p.M + 127) / 128, gz), dim3(512), 0, st, p);
-    } else {
-        hipLaunchKernelGGL((dense_dma_bf16_kernel<256, 256, 128, 64, 32, 4>), dim3((p.N + 255) / 256, (p.M + 255) / 256, gz), dim3(512), 0, st, p);
-    }
+    if (t == te)      hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 64, 16, 64, 64, 4>), dim3((p.N + 63) / 64, gy64, gz), dim3(256), 0, st, p);
+    else if (t == td) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 3>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
+    else if (t == tc) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 2>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
+    else if (t == tb) hipLaunchKernelGGL((dense_dma_bf16_kernel<128, 128, 32, 64, 64, 2>), dim3(gn, (p.M + 127) / 128, gz), dim3(512), 0, st, p);
+    else              hipLaunchKernelGGL((dense_dma_bf16_kernel<256, 256, 128, 64, 32, 4>), dim3((p.N + 255) / 256, (p.M + 255) / 256, gz), dim3(512), 0, st, p);
 }
 
 template <typename T, bool GATED>
