@@ -694,26 +694,29 @@ void launch_rows(const DenseParams& p, hipStream_t st) {
 // the A operand and 16 weight rows as B, both fragments loaded straight from memory (8 consecutive k per lane, no LDS staging).  The weight
 // stream is read once whatever M is; the waves' partial tiles are summed through LDS.  Under GATED a tile is 16 channels: their gate rows and
 // their up rows share the A fragments.
-template <bool GATED>
+// HALF (M <= 8, K % 64 == 0): 8 outputs per block.  Rows 0 to 7 of the first operand are x over the first half of K, rows 8 to 15 x over the second, the second
+// operand likewise: of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are the halves of the result, the rest is not used.
+template <bool GATED, bool HALF>
 __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, int mbase) {
     __shared__ f32x4 red[8][2][64];
+    constexpr int NO = HALF ? 8 : 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, NW = blockDim.x >> 6;
     const int nout = GATED ? p.N / 2 : p.N, grp = blockIdx.y;
-    const int r = lane & 15, kq = (lane >> 4) * 8;
-    const int o = min((int)blockIdx.x * 16 + r, nout - 1);
+    const int r = lane & (NO - 1), K = HALF ? p.K / 2 : p.K, kq = (lane >> 4) * 8, kh = HALF && (lane & 8) ? K : 0;
+    const int o = min((int)blockIdx.x * NO + r, nout - 1);
     const int n = GATED ? (o >> 5) * 64 + (o & 31) : o;
-    const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kq;
+    const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kh + kq;
     const bf16* wu = wg + (size_t)32 * p.K;
-    const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(mbase + r, p.M - 1) * p.ldx + kq;
+    const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(mbase + r, p.M - 1) * p.ldx + kh + kq;
     f32x4 ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
     const bf16x8 zero = {};
     const int stride = NW * 32;
-    for (int k0 = wave * 32; k0 < p.K; k0 += 4 * stride) {
+    for (int k0 = wave * 32; k0 < K; k0 += 4 * stride) {
         bf16x8 a[4], b[4], c[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int k = k0 + u * stride;
-            const bool ok = k + kq < p.K;
+            const bool ok = k + kq < K;
             a[u] = ok ? *(const bf16x8*)(xr + k) : zero;
             b[u] = ok ? *(const bf16x8*)(wg + k) : zero;
             if (GATED) c[u] = ok ? *(const bf16x8*)(wu + k) : zero;
@@ -732,8 +735,18 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
         ag += red[w][0][lane];
         if (GATED) au += red[w][1][lane];
     }
-    // C fragment: lane holds output (lane & 15), rows 4 * (lane >> 4) + e
-    const int oc = blockIdx.x * 16 + r;
+    // C fragment: lane holds output (lane & 15), rows 4 * (lane >> 4) + e; HALF: the second half's sum of (output, row) lies at (output + 8, row + 8), 40 lanes on
+    if constexpr (HALF) {
+        if ((lane & 8) || lane >= 32) return;
+        f32x4 g2 = red[0][0][lane + 40], u2 = GATED ? red[0][1][lane + 40] : g2;
+        for (int w = 1; w < NW; ++w) {
+            g2 += red[w][0][lane + 40];
+            if (GATED) u2 += red[w][1][lane + 40];
+        }
+        ag += g2;
+        if (GATED) au += u2;
+    }
+    const int oc = blockIdx.x * NO + r;
     if (oc >= nout) return;
     const int nb = GATED ? (oc >> 5) * 64 + (oc & 31) : oc;
 #pragma unroll
@@ -744,6 +757,22 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
         if (p.bias) { const bf16* Bi = (const bf16*)p.bias + (size_t)grp * p.N; g += dn_ld(Bi + nb); if (GATED) u += dn_ld(Bi + nb + 32); }
         dn_store<bf16>(p, row, (int)(p.ys * grp) + oc, GATED ? dn_gated(g, u, p.act, p.act_param) : dn_act(g, p.act));
     }
+}
+
+// M of 2 to 16, p.vec.  Few outputs (2048 make 128 blocks of 16): 8 per block where M allows it, so that all compute units pull weights; narrow outputs: more waves per
+// tile keep the memory system busy.  M = 8, weights from memory, us with 16 / 8 outputs: 2048 x 5632 12.5 / 9.5, 2048 x 2048 6.3 / 5.6, 16 x 2048 5.3 / 4.8,
+// 1024 x 1024 4.5 / 4.1 (4 waves), 4096 x 2048 7.4 / 8.2.
+void launch_skinny(const DenseParams& p, hipStream_t st) {
+    const int nout = p.gated ? p.N / 2 : p.N, tiles = (nout + 15) / 16;
+    if (p.M <= 8 && p.K % 64 == 0 && p.K >= 128 && tiles * p.G <= 192) {
+        const dim3 grid((nout + 7) / 8, p.G), block(p.K < 2048 ? 256 : 512);
+        if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, true>), grid, block, 0, st, p, 0);
+        else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, true>), grid, block, 0, st, p, 0);
+        return;
+    }
+    const dim3 grid(tiles, p.G), block((tiles * p.G >= 1024 || p.K < 1024) ? 256 : 512);
+    if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, false>), grid, block, 0, st, p, 0);
+    else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, false>), grid, block, 0, st, p, 0);
 }
 
 } // namespace
@@ -779,10 +808,7 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
     (void)es;
     hipStream_t st = (hipStream_t)stream;
     if (bf && M > 1 && M <= 16 && p.vec) {
-        const int tiles = ((gated ? N / 2 : N) + 15) / 16;
-        const int nw = (tiles >= 1024 || K < 1024) ? 4 : 8;        // narrow outputs: more waves per tile keep the memory system busy
-        if (gated) hipLaunchKernelGGL(dense_skinny_bf16_kernel<true>, dim3(tiles), dim3(64 * nw), 0, st, p, 0);
-        else       hipLaunchKernelGGL(dense_skinny_bf16_kernel<false>, dim3(tiles), dim3(64 * nw), 0, st, p, 0);
+        launch_skinny(p, st);
         MI355_CHECK_LAUNCH("dense_skinny_bf16_kernel");
         return MI355_OK;
     }
@@ -853,11 +879,8 @@ extern "C" int mi355_dense_grouped_ex(const void* x, int32_t ldx, int32_t M, con
         return MI355_OK;
     }
     if (!offs && M <= 16) {                    // a decode step's rows through every group: the kernels of the plain linear, groups in the grid
-        const int nout = gated ? N / 2 : N, nt = (nout + 15) / 16;
         if (bf && M > 1 && p.vec) {
-            const int nw = (nt * G >= 1024 || K < 1024) ? 4 : 8;
-            if (gated) hipLaunchKernelGGL(dense_skinny_bf16_kernel<true>, dim3(nt, G), dim3(64 * nw), 0, st, p, 0);
-            else       hipLaunchKernelGGL(dense_skinny_bf16_kernel<false>, dim3(nt, G), dim3(64 * nw), 0, st, p, 0);
+            launch_skinny(p, st);
             MI355_CHECK_LAUNCH("dense_skinny_bf16_kernel");
             return MI355_OK;
         }
