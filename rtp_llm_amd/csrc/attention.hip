@@ -42,6 +42,7 @@ struct AttnParams {
     f16*           out;
     float*         tmp_out; // [B][nh][P][hd]
     float*         tmp_ml;  // [B][nh][P][2]
+    int32_t*       done;    // non-null (zeros before and after): [row tile of a sequence][kv head], the partitions that have left their part; the last one merges
     int B, nh, nkv, G, page, max_blocks, P, PS, seq_add, max_seq, num_blocks;
     int q_len, R, ntile;   // rows per sequence (of the longest, with row_start), rows per 16-column tile (16 / G), row tiles per sequence
     const int32_t* row_start; // non-null (the two-tile instances): sequence b has rows row_start[b] .. row_start[b + 1] - 1, no padding rows between
@@ -64,6 +65,14 @@ __device__ __forceinline__ size_t out_index(const AttnParams& p, int row, int co
 }
 
 constexpr float NEG_BIG = -1e30f;
+
+// two floats written through to, read from where all XCDs see them
+__device__ __forceinline__ void put2(float* p, float a, float b) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, make_float2(a, b)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 get2(const float* p) {
+    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
 
 // NW waves per block split the partition between them (each wave keeps two 32-token groups of K/V in flight).  NW = 8 for
 // the one-block-per-CU grids (B * nkv * P <= 256) was measured and lost: 34.2 vs 29.8 us at b = 64 / ctx 1024 fp16 KV and
@@ -129,6 +138,19 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     }
     if (pstart >= seq_len) return;
     const int pend = min(seq_len, pstart + p.PS);
+    // partitions of this tile that write (1: the outputs themselves; without `done` attn_reduce_kernel merges whatever their number)
+    const int nparts = p.P == 1 ? 1 : p.done ? (seq_len + p.PS - 1) / p.PS : p.P;
+    auto store_out = [&](int row, int col, const f32x4& acc, float l) {
+        const float inv = l > 0.f ? 1.f / l : 0.f;                  // padding row / empty context: zeros, not NaN
+        u32x2 ov;
+        if (BF && p.img_mblk > 0) {   // an image holds fp16 (common.h): the bf16-rounded outputs x 2^-8 (img_val)
+            ov[0] = act_pack<false>(img_val<true>(act_round<true>(acc[0] * inv)), img_val<true>(act_round<true>(acc[1] * inv)));
+            ov[1] = act_pack<false>(img_val<true>(act_round<true>(acc[2] * inv)), img_val<true>(act_round<true>(acc[3] * inv)));
+        } else {
+            ov[0] = act_pack<BF>(acc[0] * inv, acc[1] * inv); ov[1] = act_pack<BF>(acc[2] * inv, acc[3] * inv);
+        }
+        *reinterpret_cast<u32x2*>(p.out + out_index(p, row, col, HD)) = ov;
+    };
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -519,24 +541,61 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
                 l += s_l[ww][jj] * f;
             }
             const int row = row0 + rl, h = kh * p.G + (jj - (jj / p.G) * p.G);
-            if (p.P == 1) {
-                const float inv = l > 0.f ? 1.f / l : 0.f;          // padding row / empty context: zeros, not NaN
-                u32x2 ov;
-                if (BF && p.img_mblk > 0) {   // an image holds fp16 (common.h): the bf16-rounded outputs x 2^-8 (img_val)
-                    ov[0] = act_pack<false>(img_val<true>(act_round<true>(acc[0] * inv)), img_val<true>(act_round<true>(acc[1] * inv)));
-                    ov[1] = act_pack<false>(img_val<true>(act_round<true>(acc[2] * inv)), img_val<true>(act_round<true>(acc[3] * inv)));
-                } else {
-                    ov[0] = act_pack<BF>(acc[0] * inv, acc[1] * inv); ov[1] = act_pack<BF>(acc[2] * inv, acc[3] * inv);
-                }
-                *reinterpret_cast<u32x2*>(p.out + out_index(p, row, h * HD + d0, HD)) = ov;
+            if (nparts == 1) {
+                store_out(row, h * HD + d0, acc, l);
             } else {
                 const size_t slot = ((size_t)row * p.nh + h) * p.P + part;
-                *reinterpret_cast<f32x4*>(p.tmp_out + slot * HD + d0) = acc;
-                if (d0 == 0) { p.tmp_ml[slot * 2] = mstar; p.tmp_ml[slot * 2 + 1] = l; }
+                if (p.done) {      // seen by the other XCDs without a write-back of the whole L2 (a release fence: 3 to 13 us here)
+                    put2(p.tmp_out + slot * HD + d0, acc[0], acc[1]);
+                    put2(p.tmp_out + slot * HD + d0 + 2, acc[2], acc[3]);
+                    if (d0 == 0) put2(p.tmp_ml + slot * 2, mstar, l);
+                } else {
+                    *reinterpret_cast<f32x4*>(p.tmp_out + slot * HD + d0) = acc;
+                    if (d0 == 0) { p.tmp_ml[slot * 2] = mstar; p.tmp_ml[slot * 2 + 1] = l; }
+                }
             }
         }
     }
     AT_STAMP(5);
+    if (!p.done || nparts == 1) return;
+    // The partition that is done last merges: its own launch (attn_reduce_kernel) costs 3 to 5 us behind an attention of 4 to 6 at one sequence.  Every thread's part is
+    // written through to where the other XCDs see it before the block counts itself; the last block sees all counts, then reads all parts from there.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's part has arrived
+    __syncthreads();
+    if (tid == 0) s_m[0][0] = __builtin_bit_cast(float, __hip_atomic_fetch_add(p.done + (size_t)blockIdx.z * p.nkv + kh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    __syncthreads();
+    if (__builtin_bit_cast(int, s_m[0][0]) != nparts - 1) return;
+    for (int idx = tid; idx < nrows * p.G * (HD / 4); idx += NTHR) {
+        const int col = idx / (HD / 4), d0 = (idx - col * (HD / 4)) * 4, rl = col / p.G, row = row0 + rl, h = kh * p.G + (col - rl * p.G);
+        const int np = (min(max(p.seq_lens[row] + p.seq_add, 0), p.max_seq) + p.PS - 1) / p.PS;      // partitions that saw this row
+        const size_t slot = ((size_t)row * p.nh + h) * p.P;
+        const float* ml = p.tmp_ml + slot * 2;
+        const float* po = p.tmp_out + slot * HD + d0;
+        float mstar = NEG_BIG, l = 0.f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int i0 = 0; i0 < np; i0 += 8) {                     // eight parts in flight, summed in partition order
+            float2 v[8], oa[8], ob[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = min(i0 + u, np - 1);
+                v[u] = get2(ml + i * 2); oa[u] = get2(po + (size_t)i * HD); ob[u] = get2(po + (size_t)i * HD + 2);
+            }
+            float mnew = mstar;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) mnew = fmaxf(mnew, v[u].x);
+            const float resc = __builtin_amdgcn_exp2f(mstar - mnew);
+            l *= resc; acc *= resc; mstar = mnew;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (i0 + u >= np) continue;
+                const float f = __builtin_amdgcn_exp2f(v[u].x - mstar);
+                l += v[u].y * f;
+                acc += f32x4{oa[u].x, oa[u].y, ob[u].x, ob[u].y} * f;
+            }
+        }
+        store_out(row, h * HD + d0, acc, l);
+    }
+    if (tid == 0) __hip_atomic_store(p.done + (size_t)blockIdx.z * p.nkv + kh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Merge partitions: one wave per (sequence, head); lane owns HD/64 channels.
@@ -640,7 +699,7 @@ namespace {
 int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table, int32_t max_blocks_per_seq,
                 const int32_t* seq_lens, int32_t seq_lens_minus_one, int32_t B, int32_t q_len, int32_t nh, float scale,
                 int32_t max_seq_len, void* out, void* workspace, size_t workspace_bytes, mi355_stream_t stream, int img_mblk = 0,
-                const int32_t* row_start = nullptr, int32_t total_rows = 0) {
+                const int32_t* row_start = nullptr, int32_t total_rows = 0, int32_t* done = nullptr) {
     MI355_CHECK_ARG(q && kv && kv->kv_base && block_table && seq_lens && out, "paged_attn: null pointer");
     MI355_CHECK_ARG(kv->hd == 64 || kv->hd == 128, "paged_attn: hd=%d (64 or 128)", kv->hd);
     MI355_CHECK_ARG(kv->page >= 16 && kv->page % 8 == 0, "paged_attn: page=%d (>= 16, multiple of 8)", kv->page);
@@ -674,6 +733,7 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
         mi355_set_error("paged_attn: workspace %zu < %zu", workspace_bytes, need);
         return MI355_ERR_WORKSPACE;
     }
+    p.done = p.P > 1 ? done : nullptr;
     p.tmp_out = (float*)workspace;
     p.tmp_ml  = p.tmp_out + rows * nh * p.P * kv->hd;
     hipStream_t st = (hipStream_t)stream;
@@ -699,7 +759,7 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
 #undef L2_
 #undef L_
     MI355_CHECK_LAUNCH("paged_attn_kernel");
-    if (p.P > 1) {
+    if (p.P > 1 && !p.done) {
         const int nblk = cdiv((int)rows * nh, 4);
         if (bf) {
             if (kv->hd == 128) hipLaunchKernelGGL((attn_reduce_kernel<128, true>), dim3(nblk), dim3(256), 0, st, p);
@@ -755,4 +815,14 @@ extern "C" int mi355_paged_attn_rows_img(const void* q, const mi355_kv_layer_t* 
     MI355_CHECK_ARG(B > 0 && q_len > 0 && B * q_len <= 64 && kv && (nh * kv->hd) % 32 == 0, "paged_attn_rows_img: %d x %d rows (<= 64)", B, q_len);
     return launch_attn(q, kv, block_table, max_blocks_per_seq, positions, 1, B, q_len, nh, scale, max_seq_len, out_img, workspace,
                        workspace_bytes, stream, cdiv(B * q_len, 16));
+}
+
+// What the step driver calls: out row-major or (img) an activation image; done: [B * row tiles][nkv] counters that are zero (B * q_len * nkv of them suffice), left at zero.
+// Calls that share them must not overlap.
+extern "C" int mi355_paged_attn_step(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table, int32_t max_blocks_per_seq, const int32_t* positions,
+                                     int32_t B, int32_t q_len, int32_t nh, float scale, int32_t max_seq_len, void* out, int32_t img, void* workspace, size_t workspace_bytes,
+                                     int32_t* done, mi355_stream_t stream) {
+    MI355_CHECK_ARG(!img || (B > 0 && q_len > 0 && B * q_len <= 64 && kv && (nh * kv->hd) % 32 == 0), "paged_attn_step: %d x %d rows (<= 64)", B, q_len);
+    return launch_attn(q, kv, block_table, max_blocks_per_seq, positions, 1, B, q_len, nh, scale, max_seq_len, out, workspace, workspace_bytes, stream,
+                       img ? cdiv(B * q_len, 16) : 0, nullptr, 0, done);
 }
