@@ -394,6 +394,12 @@ int mi355_argmax(const float* logits, int32_t B, int32_t V, int32_t ld, int32_t*
  * mi355_softmax_rows: probs[r][:] = softmax(logits[r][:] / temperature) in fp32 (the rows the sampler hands over). */
 int mi355_softmax_rows(const float* logits, int32_t rows, int32_t V, int32_t ld, float temperature, float* probs,
                        mi355_stream_t stream);
+/* The sampler's row in two launches: temperature, then penalties over at most 2048 history entries (MI355_ERR_UNSUPPORTED beyond), each as in mi355_apply_penalties
+ * with entry i of row r at output_ids[i * id_step + r * id_row], then softmax, in place on logits [rows][ld].  Any of temperature and the penalties may be null. */
+size_t mi355_sampling_probs_workspace_bytes(int32_t rows);
+int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
+                         const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
+                         int32_t step, void* workspace, mi355_stream_t stream);
 /* ids[r] = first index whose inclusive fp32 prefix sum of probs[r, :] (index order) exceeds uniform_samples[r] * sum --
  * sampling from the probabilities, the top_k = 0 / top_p = 1 branch of the sampler (bindings/core/CudaSampleOp.cc:702-737);
  * gives the target model's own sampled token per verify row (target_token_ids of mi355_rejection_sample). */

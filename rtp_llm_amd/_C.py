@@ -109,6 +109,8 @@ SIGNATURES = {
     "mi355_paged_attn_rows_ragged": (i32, [vp, C.POINTER(KVLayer), vp, i32, vp, vp, i32, i32, i32, i32, f32, i32, vp, vp, sz, vp]),
     "mi355_paged_attn_rows": (i32, [vp, C.POINTER(KVLayer), vp, i32, vp, i32, i32, i32, f32, i32, vp, vp, sz, vp]),
     "mi355_argmax": (i32, [vp, i32, i32, i32, vp, vp, sz, vp]),
+    "mi355_sampling_probs_workspace_bytes": (sz, [i32]),
+    "mi355_sampling_probs": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp]),
     "mi355_softmax_rows": (i32, [vp, i32, i32, i32, f32, vp, vp]),
     "mi355_sample_rows": (i32, [vp, i32, i32, i32, vp, vp, vp]),
     "mi355_apply_penalties": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp]),

@@ -285,6 +285,99 @@ __global__ __launch_bounds__(256) void penalties_short_kernel(const PenaltyParam
     }
 }
 
+// Temperature, penalties and softmax of the sampler in two launches, every row split over blocks.  One block per row, the softmax alone took 36 us of 64 rows of 152064 (its
+// three passes at what one CU pulls), behind 14 of temperature and 14 of penalties; the two take 29 and 11.
+// Prepare: a block scales its slice, penalises the history's ids that lie in it (as penalties_short_kernel) and leaves the slice's maximum and sum of exponentials.
+__global__ __launch_bounds__(kThreads) void sampling_prepare_kernel(const PenaltyParams p, float2* parts, int id_step, int id_row, int slice) {
+    __shared__ __attribute__((aligned(16))) int s_tok[kShortHistory];
+    __shared__ float s_red[kThreads / 64];
+    const int row = blockIdx.y, tx = threadIdx.x, lo = min(p.V, (int)blockIdx.x * slice), n = min(p.V, lo + slice) - lo;
+    float* x = p.logits + (size_t)row * p.ld + lo;
+    const bool vec = (p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;       // lo is a multiple of 4
+    const int padded = p.output_ids ? (p.step + 3) & ~3 : 0;
+    if (padded) {
+        const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
+        for (int i = tx; i < padded; i += kThreads) {
+            int tok = -1;                                   // nothing to penalise: padding, or an id outside the vocabulary
+            if (i < p.step && !(i >= input_length && i < p.max_input_length)) {
+                tok = p.output_ids[(size_t)i * id_step + (size_t)row * id_row];
+                if (tok >= p.V || tok < 0) tok = -1;
+            }
+            s_tok[i] = tok;
+        }
+    }
+    if (p.temperature) {
+        const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
+        int done = 0;
+        if (vec) {
+            f32x4* x4 = reinterpret_cast<f32x4*>(x);
+#pragma unroll 4
+            for (int j = tx; j < n >> 2; j += kThreads) {
+                f32x4 v = x4[j];
+                v[0] *= inv_t; v[1] *= inv_t; v[2] *= inv_t; v[3] *= inv_t;
+                x4[j] = v;
+            }
+            done = n & ~3;
+        }
+        for (int j = done + tx; j < n; j += kThreads) x[j] *= inv_t;
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (padded) {
+        for (int i = tx; i < p.step; i += kThreads) {
+            const int tok = s_tok[i];
+            if (tok < lo || tok >= lo + n) continue;
+            int count = 0, before = 0;
+            for (int j = 0; j < padded; j += 4) {
+                const int4 t = *reinterpret_cast<const int4*>(&s_tok[j]);
+                const int c = (t.x == tok) + (t.y == tok) + (t.z == tok) + (t.w == tok);
+                count += c;
+                if (j + 3 < i) before += c;
+                else before += (j < i && t.x == tok) + (j + 1 < i && t.y == tok) + (j + 2 < i && t.z == tok);
+            }
+            if (before == 0) x[tok - lo] = penalised(p, row, x[tok - lo], count);
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
+    float m = -3.0e38f;
+    row_pass(x, n, vec, [&](float v) { m = fmaxf(m, v); });
+    m = wave_max(m);
+    if ((tx & 63) == 0) s_red[tx >> 6] = m;
+    __syncthreads();
+    m = s_red[0];
+    for (int w = 1; w < kThreads / 64; ++w) m = fmaxf(m, s_red[w]);
+    __syncthreads();
+    float s = 0.f;
+    row_pass(x, n, vec, [&](float v) { s += __expf(v - m); });
+    s = block_sum(s, s_red);
+    if (tx == 0) parts[(size_t)row * gridDim.x + blockIdx.x] = make_float2(m, s);
+}
+
+// Probabilities in place: exp(x - m) / sum from the slices' maxima and sums.
+__global__ __launch_bounds__(kThreads) void sampling_probs_kernel(float* logits, int V, int ld, const float2* parts, int slice) {
+    const int row = blockIdx.y, tx = threadIdx.x, lo = min(V, (int)blockIdx.x * slice), n = min(V, lo + slice) - lo;
+    float* x = logits + (size_t)row * ld + lo;
+    const float2* pr = parts + (size_t)row * gridDim.x;
+    float m = pr[0].x, s = 0.f;
+    for (int i = 1; i < (int)gridDim.x; ++i) m = fmaxf(m, pr[i].x);
+    for (int i = 0; i < (int)gridDim.x; ++i) s += pr[i].y * __expf(pr[i].x - m);
+    const float inv = 1.f / s;
+    int done = 0;
+    if ((ld & 3) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0) {
+        f32x4* x4 = reinterpret_cast<f32x4*>(x);
+#pragma unroll 4
+        for (int j = tx; j < n >> 2; j += kThreads) {
+            f32x4 v = x4[j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = __expf(v[r] - m) * inv;
+            x4[j] = v;
+        }
+        done = n & ~3;
+    }
+    for (int j = done + tx; j < n; j += kThreads) x[j] = __expf(x[j] - m) * inv;
+}
+
 // Longer histories: counters in memory, cleared by the first of two launches.
 __global__ __launch_bounds__(kThreads) void clear_counts_kernel(int32_t* counts, size_t n) {
     for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads) counts[i] = 0;
@@ -774,6 +867,26 @@ extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t 
         hipLaunchKernelGGL(penalties_short_kernel, dim3(batch_size), dim3(256), 0, st, p);
         MI355_CHECK_LAUNCH("penalties_short_kernel");
     }
+    return MI355_OK;
+}
+
+// splits of a row: enough blocks for the chip, no more than kSamplingSplits
+static int sampling_splits(int rows) { return rows >= 256 ? 1 : rows >= 32 ? 8 : 16; }
+
+extern "C" size_t mi355_sampling_probs_workspace_bytes(int32_t rows) { return rows > 0 ? (size_t)rows * sampling_splits(rows) * sizeof(float2) : 0; }
+
+extern "C" int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
+                                    const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
+                                    int32_t step, void* workspace, mi355_stream_t stream) {
+    MI355_CHECK_ARG(logits && workspace && rows > 0 && V > 0 && ld >= V && step >= 0 && (uintptr_t)workspace % 8 == 0, "sampling_probs: bad args");
+    if (output_ids && step > kShortHistory) return MI355_ERR_UNSUPPORTED;      // apply_penalties counts those in memory
+    const bool pen = output_ids && step > 0 && (repetition || presence || frequency);
+    const int S = sampling_splits(rows), slice = ((V + S - 1) / S + 3) & ~3;
+    const PenaltyParams p{logits, V, ld, temperature, repetition, presence, frequency, pen ? output_ids : nullptr, input_lengths, rows, max_input_length, step, nullptr};
+    hipLaunchKernelGGL(sampling_prepare_kernel, dim3(S, rows), dim3(kThreads), 0, (hipStream_t)stream, p, (float2*)workspace, id_step, id_row, slice);
+    MI355_CHECK_LAUNCH("sampling_prepare_kernel");
+    hipLaunchKernelGGL(sampling_probs_kernel, dim3(S, rows), dim3(kThreads), 0, (hipStream_t)stream, logits, V, ld, (const float2*)workspace, slice);
+    MI355_CHECK_LAUNCH("sampling_probs_kernel");
     return MI355_OK;
 }
 

@@ -500,6 +500,32 @@ def apply_penalties(logits: torch.Tensor, temperature: Optional[torch.Tensor] = 
     return logits
 
 
+def sampling_probs(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None, repetition_penalty: Optional[torch.Tensor] = None,
+                   presence_penalty: Optional[torch.Tensor] = None, frequency_penalty: Optional[torch.Tensor] = None, token_ids: Optional[torch.Tensor] = None,
+                   input_lengths: Optional[torch.Tensor] = None, max_input_length: int = 0, step: int = 0) -> torch.Tensor:
+    """apply_penalties and softmax_rows in place on fp32 logits [B, V], in two launches.  The vectors are of their kernel's types on the device, one value per row; the
+    history is token_ids [B, >= step] int32, step <= 2048."""
+    _chk(logits, torch.float32, "sampling_probs.logits")
+    B, V = logits.shape
+    for t, dt in ((temperature, torch.float32), (repetition_penalty, torch.float32), (presence_penalty, torch.float32), (frequency_penalty, torch.float32), (input_lengths, torch.int32)):
+        if t is not None:
+            _chk(t, dt, "sampling_probs")
+            if t.numel() != B:
+                raise _C.Mi355Error("sampling_probs: one value per row")
+    if token_ids is not None:
+        _chk(token_ids, torch.int32, "sampling_probs.token_ids")
+        if token_ids.dim() != 2 or token_ids.shape[0] != B or token_ids.shape[1] < step:
+            raise _C.Mi355Error("sampling_probs: token_ids must be [B, >= step]")
+    elif repetition_penalty is not None or presence_penalty is not None or frequency_penalty is not None:
+        raise _C.Mi355Error("sampling_probs: penalties need the token history token_ids [B, step]")
+    lib = _C.lib()
+    ws = torch.empty(max(8, lib.mi355_sampling_probs_workspace_bytes(B)), dtype=torch.uint8, device=logits.device)
+    _C.check(lib.mi355_sampling_probs(logits.data_ptr(), B, V, V, _p(temperature), _p(repetition_penalty), _p(presence_penalty), _p(frequency_penalty), _p(token_ids),
+                                      1, 0 if token_ids is None else token_ids.shape[1], _p(input_lengths), int(max_input_length), int(step), ws.data_ptr(), _stream()),
+             "sampling_probs")
+    return logits
+
+
 def ban_repeat_ngram(logits: torch.Tensor, token_ids: torch.Tensor, sequence_last_index: torch.Tensor,
                      no_repeat_ngram_size: torch.Tensor) -> torch.Tensor:
     """In place on fp32 logits [B', V] (the first B rows are touched): token_ids [B, L] int32, sequence_last_index [B],

@@ -16,6 +16,7 @@ are not on this path (the reference's ROCm branch does not update them per token
 from dataclasses import dataclass
 from typing import Optional
 
+import numpy as np
 import torch
 
 from . import ops
@@ -44,6 +45,10 @@ def _host(t: torch.Tensor, dtype) -> torch.Tensor:
     return t.detach().to(device="cpu", dtype=dtype)
 
 
+def _off(t: torch.Tensor, default) -> bool:
+    return bool((t.numpy() != default).any())
+
+
 def _softmax_in_place(logits: torch.Tensor) -> torch.Tensor:
     # the kernel may overwrite its input; host tensors reach this flow only with another `ops`, which need not
     return ops.softmax_rows(logits, out=logits) if logits.is_cuda else logits.copy_(ops.softmax_rows(logits))
@@ -53,11 +58,13 @@ def _upload(tensors, device):
     """The named host tensors of 32-bit values on the device, contiguous: packed into one buffer and sent in one copy."""
     if not tensors:
         return {}
-    flat = torch.cat([t.reshape(-1).view(torch.int32) for t in tensors.values()]).to(device)
+    host = np.concatenate([t.numpy().reshape(-1).view(np.int32) for t in tensors.values()])
+    flat = torch.from_numpy(host).to(device)
     out, at = {}, 0
     for name, t in tensors.items():
-        out[name] = flat[at:at + t.numel()].view(t.dtype).view(t.shape)
-        at += t.numel()
+        n = t.numel()
+        out[name] = flat[at:at + n].view(t.dtype).view(t.shape)
+        at += n
     return out
 
 
@@ -70,18 +77,25 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
     if params.token_ids.shape != (B, step + 1):
         raise ValueError("sample_greedy: token_ids must be [batch_size, step + 1]")
     temperature = _host(params.temperature, torch.float32)
-    scale = bool((temperature != 1.0).any())
+    scale = _off(temperature, 1.0)
     penalise = False
     if params.repetition_penalty is not None:
         if params.presence_penalty is None or params.frequency_penalty is None:
             raise ValueError("sample_greedy: repetition_penalty comes with presence_penalty and frequency_penalty")
         rep, pres, freq = (_host(t, torch.float32) for t in (params.repetition_penalty, params.presence_penalty, params.frequency_penalty))
-        penalise = bool((rep != 1.0).any()) or bool((pres != 0.0).any()) or bool((freq != 0.0).any())
+        penalise = _off(rep, 1.0) or _off(pres, 0.0) or _off(freq, 0.0)
     top_k = _host(params.top_k, torch.int32)
-    all_greedy = bool((top_k == 1).all())
+    all_greedy = not _off(top_k, 1)
     draw = not all_greedy
     if draw and params.uniform is None:
         raise ValueError("sample_greedy: sampling rows need params.uniform (one value in [0, 1) per row)")
+    ngram = None
+    if params.no_repeat_ngram_size is not None and params.sequence_lengths.numel() > 0:
+        ngram = _host(params.no_repeat_ngram_size, torch.int32)
+        if not _off(ngram[:params.sequence_lengths.numel()], 0):
+            ngram = None
+    # logits -> probabilities in two launches, unless something else comes between
+    together = logits.is_cuda and ngram is None and step < 2048 and B <= 65535 and not (all_greedy and params.output_all_probs is None)
 
     # everything the step needs on the device that is on the host: one buffer, one copy
     up = {}
@@ -94,7 +108,8 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
             lengths[:nd] = _host(params.sequence_lengths, torch.int32)
         up.update(rep=rep, pres=pres, freq=freq, lengths=lengths)
         if params.token_ids.device.type == "cpu":
-            up["history"] = params.token_ids.to(torch.int32).t()                          # [step + 1, batch_size]
+            history = params.token_ids.to(torch.int32)                                    # [batch_size, step + 1]
+            up["history"] = history if together else history.t()
     if draw:
         top_p = _host(params.top_p, torch.float32).clone()
         top_p[top_p.abs() < 1e-7] = 1.0
@@ -103,25 +118,30 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
             up["uniform"] = params.uniform.to(torch.float32)
     up = _upload(up, dev)
 
-    if scale:
-        ops.apply_penalties(logits, temperature=up["temperature"])
-    if penalise:
-        transposed = up["history"] if "history" in up else params.token_ids.to(device=dev, dtype=torch.int32).t().contiguous()
-        ops.apply_penalties(logits, repetition_penalty=up["rep"], presence_penalty=up["pres"], frequency_penalty=up["freq"], output_ids=transposed,
-                            input_lengths=up["lengths"], max_input_length=step + 1, step=step + 1)
-
-    if params.no_repeat_ngram_size is not None and params.sequence_lengths.numel() > 0:
-        ngram = _host(params.no_repeat_ngram_size, torch.int32)
-        nd = params.sequence_lengths.numel()
-        if bool((ngram[:nd] != 0).any()):
+    if together:
+        vectors = {}
+        if penalise:
+            vectors = dict(repetition_penalty=up["rep"], presence_penalty=up["pres"], frequency_penalty=up["freq"], input_lengths=up["lengths"], max_input_length=step + 1,
+                           step=step + 1, token_ids=up["history"] if "history" in up else params.token_ids.to(device=dev, dtype=torch.int32).contiguous())
+        probs = ops.sampling_probs(logits, up.get("temperature"), **vectors)
+    else:
+        if scale:
+            ops.apply_penalties(logits, temperature=up["temperature"])
+        if penalise:
+            transposed = up["history"] if "history" in up else params.token_ids.to(device=dev, dtype=torch.int32).t().contiguous()
+            ops.apply_penalties(logits, repetition_penalty=up["rep"], presence_penalty=up["pres"], frequency_penalty=up["freq"], output_ids=transposed,
+                                input_lengths=up["lengths"], max_input_length=step + 1, step=step + 1)
+        if ngram is not None:
             # the kernel takes the index of the last valid token and adds one itself (CudaSampleOp.cc:262-265)
+            nd = params.sequence_lengths.numel()
             tokens = params.token_ids.to(device=dev, dtype=torch.int32).contiguous()
             ops.ban_repeat_ngram(logits, tokens[:nd], _host(params.sequence_lengths, torch.int32) - 1, ngram[:nd])
 
     if all_greedy and params.output_all_probs is None:
         ids = ops.argmax(logits)
     else:
-        probs = _softmax_in_place(logits)
+        if not together:
+            probs = _softmax_in_place(logits)
         want_renorm = params.output_all_probs is not None and not params.return_original_all_probs
         if all_greedy:
             ids = ops.argmax(probs)
