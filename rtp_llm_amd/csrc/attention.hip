@@ -598,6 +598,178 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     if (tid == 0) __hip_atomic_store(p.done + (size_t)blockIdx.z * p.nkv + kh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ------------------------------------------------------------------------------------------------ prompt rows (16-bit cache)
+// The same attention for many rows per sequence: a wave per (16 rows, head), the HW heads of one key/value head (times TW row tiles) in a block of at most eight waves that
+// walks the keys by 32 once for all of them.  paged_attn_kernel gives a block 32 / G rows and pulls the keys and values for them through registers: 4096 blocks of 4
+// rows read 537 MB out of L2 for 8 prompts of 512 tokens (28 over 4 heads of 128).  Here keys and values come by DMA into three LDS stages, two steps ahead, one barrier a
+// step.  Products transposed as there (a lane owns one row: its maximum, sum and rescaling are its own; the weights are the second product's operand where they
+// are: the keys of a step are handed to the first product in an order that leaves every lane eight consecutive ones).  16-byte pieces of a key row are swizzled by the
+// key, a value row (one channel, 32 tokens) is 64 bytes and needs none.
+// 8 x 512 rows, 28 over 4 heads of 128: 179 -> 86 us; 3 ragged of 389: 51 -> 29.
+// What bounds it: a step of one wave, about 1.4 us of product, softmax and product in series whatever the depth of the staging (3 to 6 stages measured the same).
+// 16 bytes per lane to LDS at `lds` + 16 lane, from base + voff
+__device__ __forceinline__ void pr_dma16(uint32_t lds, uint32_t voff, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
+template <int VM> __device__ __forceinline__ void pr_wait() {     // at most VM vector-memory operations of the wave left, no LDS operation
+    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+}
+__device__ __forceinline__ void pr_wait(int left) {
+    asm volatile("" ::: "memory");
+    switch (left) {
+        case 0: pr_wait<0>(); break;    case 1: pr_wait<1>(); break;    case 2: pr_wait<2>(); break;    case 3: pr_wait<3>(); break;
+        case 4: pr_wait<4>(); break;    case 5: pr_wait<5>(); break;    case 6: pr_wait<6>(); break;    case 7: pr_wait<7>(); break;
+        case 8: pr_wait<8>(); break;    case 9: pr_wait<9>(); break;    case 10: pr_wait<10>(); break;  case 11: pr_wait<11>(); break;
+        case 12: pr_wait<12>(); break;  case 13: pr_wait<13>(); break;  case 14: pr_wait<14>(); break;  case 15: pr_wait<15>(); break;
+        default: pr_wait<16>(); break;
+    }
+    asm volatile("" ::: "memory");
+}
+
+template <int HD, bool BF>
+__global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p, int HW, int TW, int NS) {
+    constexpr int NSTEP = HD / 32, NDB = HD / 16, KL = HD / 16, LOADS = 2 * KL;     // 1 KB loads of a key tile (32 rows), of a step
+    constexpr int CK = HD / 8;
+    extern __shared__ __attribute__((aligned(16))) char pr_sm[];
+    const int NW = HW * TW, JT = (LOADS + NW - 1) / NW, stage = JT * NW * 1024;
+    int* klim_s = reinterpret_cast<int*>(pr_sm + NS * stage);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lq = lane >> 4;
+    const int b = blockIdx.z, h = blockIdx.y * HW + wave % HW, kh = (int)blockIdx.y * HW / p.G;
+    int base = b * p.q_len, len = p.q_len;
+    if (p.row_start) { base = p.row_start[b]; len = p.row_start[b + 1] - base; }
+    const int t0r = ((int)gridDim.x - 1 - (int)blockIdx.x) * TW * 16;                // late (long) rows first
+    if (t0r >= len) return;
+    const int r0 = t0r + wave / HW * 16, n = min(16, len - r0);                       // n <= 0: a wave without rows
+    const int row = base + min(max(r0 + lr, 0), len - 1);
+    const int limit = lr < n ? min(max(p.seq_lens[row] + p.seq_add, 0), p.max_seq) : 0;
+    if (tid == 0) *klim_s = 0;
+    __syncthreads();
+    int wmax = limit, wmin = lr < n ? limit : 0x7fffffff;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) { wmax = max(wmax, __shfl_xor(wmax, o)); wmin = min(wmin, __shfl_xor(wmin, o)); }
+    if (lane == 0) atomicMax(klim_s, wmax);
+    __syncthreads();
+    const int klim = __builtin_amdgcn_readfirstlane(*klim_s);
+    wmax = __builtin_amdgcn_readfirstlane(wmax); wmin = __builtin_amdgcn_readfirstlane(wmin);
+    u32x4 qf[NSTEP];
+#pragma unroll
+    for (int s = 0; s < NSTEP; ++s) qf[s] = *reinterpret_cast<const u32x4*>(p.q + ((size_t)row * p.nh + h) * HD + s * 32 + lq * 8);
+    f32x4 o[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    float m = NEG_BIG, l = 0.f;
+    if (klim > 0) {
+        const int32_t* bt = p.block_table + (size_t)b * p.max_blocks;
+        const int last = klim - 1, lastw = last & ~7, nsteps = (last >> 5) + 1;
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)pr_sm;
+        auto page_of = [&](int t) { return (int)__builtin_amdgcn_readfirstlane((int)(((unsigned long long)(unsigned)t * p.page_magic) >> 32)); };
+        // The wave's loads of a step: K rows (a load lies in one window of 8 tokens), then for every window 64 channels of V (past the step's loads, where LOADS is no
+        // multiple of the waves, the last once more into the stage's end).  A window lies in one page: its address is the scalar unit's work, a lane's offset
+        // from it stays (per-lane addresses took more vector instructions than the products and the softmax together).
+        constexpr int JM = HD == 128 ? 4 : 2, KPL = 64 / CK, VPW = HD / 64;               // keys per load, V loads per window
+        uint32_t voff[JM];
+        int win[JM], koff[JM];
+        bool isv[JM];
+#pragma unroll
+        for (int j = 0; j < JM; ++j) {
+            const int load = min(j * NW + wave, LOADS - 1), k0 = load * KPL, v = load - KL;
+            isv[j] = load >= KL;
+            win[j] = isv[j] ? v / VPW : k0 >> 3; koff[j] = isv[j] ? 0 : k0 & 7;
+            const int key = k0 + lane / CK, c = lane % CK, d = v % VPW * 64 + lane;
+            voff[j] = isv[j] ? (uint32_t)(d * p.page) * 2u : (uint32_t)((lane / CK) * HD + ((c ^ (((key & 3) | (key >> 3 & 3) << 2) & (CK - 1))) << 3)) * 2u;
+        }
+        int id[JM];                                               // block ids of the next step to be issued
+        auto fetch = [&](int st) {
+#pragma unroll
+            for (int j = 0; j < JM; ++j) id[j] = bt[page_of(min(st * 32 + win[j] * 8, lastw))];
+        };
+        auto issue = [&](int st, int buf) {
+#pragma unroll
+            for (int j = 0; j < JM; ++j) {
+                if (j >= JT) continue;
+                const int wt = min(st * 32 + win[j] * 8, lastw), ti = wt - page_of(wt) * p.page, blk = min(max(id[j], 0), p.num_blocks - 1);
+                const uint32_t hk = (uint32_t)blk * (uint32_t)(2 * p.nkv) + (uint32_t)(isv[j] ? p.nkv + kh : kh);
+                const uint16_t* src = (const uint16_t*)p.kv_base + (uint64_t)hk * (uint32_t)(p.page * HD) + (uint32_t)(isv[j] ? ti : (ti + koff[j]) * HD);
+                pr_dma16(__builtin_amdgcn_readfirstlane(lds0 + buf * stage + (j * NW + wave) * 1024), voff[j], src);
+            }
+        };
+        pr_wait(0);                                               // the rows' queries are here: no wait for them (and with it for the DMA) inside the loop
+        for (int st = 0; st < min(NS - 1, nsteps); ++st) { fetch(st); issue(st, st); }
+        fetch(NS - 1);
+        int buf = 0;
+        const int kswz = lr & 3;                                  // key of the lane's row: (lr >> 2) * 8 + tau * 4 + (lr & 3)
+        for (int st = 0; st < nsteps; ++st) {
+            pr_wait(JT * min(NS - 2, nsteps - 1 - st));           // all but the later steps' loads of this wave
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int t0 = st * 32;
+            const char* cur = pr_sm + buf * stage;
+            if (st + NS - 1 < nsteps) { issue(st + NS - 1, buf == 0 ? NS - 1 : buf - 1); fetch(st + NS); }
+            buf = buf == NS - 1 ? 0 : buf + 1;
+            if (t0 >= wmax) continue;                             // nothing for this wave's rows
+            f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ks = 0; ks < NSTEP; ++ks)
+#pragma unroll
+                for (int tau = 0; tau < 2; ++tau) {
+                    const int key = (lr >> 2) * 8 + tau * 4 + kswz, g = (kswz | (lr >> 2) << 2) & (CK - 1);
+                    s[tau] = mfma_act<BF>(*reinterpret_cast<const u32x4*>(cur + key * (HD * 2) + (((ks * 4 + lq) ^ g) << 4)), qf[ks], s[tau]);
+                }
+            const bool masked = t0 + 32 > wmin;
+            const int vwin = t0 + lq * 8;                         // the lane's eight keys
+            float sv[8], mx = NEG_BIG;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float v = s[e >> 2][e & 3] * p.scale_log2;
+                if (masked) v = vwin + e < limit ? v : NEG_BIG;
+                sv[e] = v;
+                mx = fmaxf(mx, v);
+            }
+            mx = fmaxf(m, xor32_max(xor16_max(mx)));
+            if (__builtin_amdgcn_ballot_w64(mx != m)) {
+                const float alpha = __builtin_amdgcn_exp2f(m - mx);
+                l *= alpha;
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+                m = mx;
+            }
+            float psum = 0.f, pes[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pe = !masked || vwin + e < limit ? __builtin_amdgcn_exp2f(sv[e] - m) : 0.f;
+                psum += pe;
+                pes[e] = pe;
+            }
+            const u32x4 pf = act_pack8<BF>(pes);
+            l += psum;
+            auto value = [&](int db) { return *reinterpret_cast<const u32x4*>(cur + KL * 1024 + (lq * HD + db * 16 + lr) * 16); };
+            if (t0 + 32 <= klim) {
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) o[db] = mfma_act<BF>(value(db), pf, o[db]);
+            } else {                                              // values past the context may be garbage (NaN / Inf): zero them, their weights are zero
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) {
+                    u32x4 a = value(db);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (vwin + e >= klim) a[e >> 1] &= (e & 1) ? 0x0000FFFFu : 0xFFFF0000u;
+                    o[db] = mfma_act<BF>(a, pf, o[db]);
+                }
+            }
+        }
+    }
+    l = xor32_sum(xor16_sum(l));
+    if (lr >= n) return;
+    const float inv = l > 0.f ? 1.f / l : 0.f;                    // padding row / empty context: zeros
+    f16* out = p.out + ((size_t)row * p.nh + h) * HD + lq * 4;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+        u32x2 ov;
+        ov[0] = act_pack<BF>(o[db][0] * inv, o[db][1] * inv); ov[1] = act_pack<BF>(o[db][2] * inv, o[db][3] * inv);
+        *reinterpret_cast<u32x2*>(out + db * 16) = ov;
+    }
+}
+
 // Merge partitions: one wave per (sequence, head); lane owns HD/64 channels.
 template <int HD, bool BF = false>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(const AttnParams p) {
@@ -722,12 +894,33 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     p.stamps = g_attn_stamps;
 #endif
     p.page_magic = (uint32_t)((1ull << 32) / (unsigned)kv->page + 1);
+    p.row_start = row_start; p.rows = row_start ? total_rows : B * q_len;
+    p.scale_log2 = scale * 1.4426950408889634f;
+    const bool bf = kv->act_dtype == MI355_ACT_BF16;
+    MI355_CHECK_ARG(kv->act_dtype == MI355_ACT_F16 || bf, "paged_attn: act_dtype=%d", kv->act_dtype);
+    MI355_CHECK_ARG(int8 || (bf == (kv->kv_dtype == MI355_KV_BF16)), "paged_attn: a 16-bit cache has the dtype of the activations");
+    int HW = p.G < 8 ? p.G : 8;
+    while (p.G % HW) --HW;                                  // heads of a key/value head per block
+    const int TW = 8 / HW, NW = HW * TW, JT = (kv->hd / 8 + NW - 1) / NW;
+    const dim3 pgrid(cdiv(q_len, 16 * TW), nh / HW, B);
+    // Prompt rows: where the blocks fill the chip; with fewer of them the other kernel's smaller row tiles and split contexts win (28 over 4 heads of 128, us there / here:
+    // 8 x 512 rows 179 / 86, 3 x 352 72 / 52, 1 x 1500 137 / 106, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100)
+    if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)pgrid.x * pgrid.y * pgrid.z >= 256 && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
+        constexpr int NS = 3;
+        const dim3 grid = pgrid;
+        const size_t lds = (size_t)NS * JT * NW * 1024 + 16;
+        hipStream_t st = (hipStream_t)stream;
+        if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS);
+                             else          hipLaunchKernelGGL((prompt_attn_kernel<128, false>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS); }
+        else               { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<64, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS);
+                             else          hipLaunchKernelGGL((prompt_attn_kernel<64, false>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS); }
+        MI355_CHECK_LAUNCH("prompt_attn_kernel");
+        return MI355_OK;
+    }
     const int NT = q_len > p.R || row_start ? 2 : 1;    // column tiles per block: 2 x R rows share one pass over the KV
     p.ntile = cdiv(q_len, NT * p.R);
     p.P = plan_partitions(B * p.ntile, kv->nkv, max_seq_len, &p.PS);
-    p.scale_log2 = scale * 1.4426950408889634f;
-    const size_t rows = row_start ? (size_t)total_rows : (size_t)B * q_len;
-    p.row_start = row_start; p.rows = (int)rows;
+    const size_t rows = (size_t)p.rows;
     const size_t need = p.P > 1 ? rows * nh * p.P * (kv->hd + 2) * sizeof(float) : 0;
     if (need > workspace_bytes || (need && !workspace)) {
         mi355_set_error("paged_attn: workspace %zu < %zu", workspace_bytes, need);
@@ -747,9 +940,6 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
 // (NG = 3: 72.7), ctx 1024 unchanged; fp16 loses with more than two (28.4 -> 30.6 us at ctx 1024)
 #define L2_(HD_, I8_) do { if (NT == 1) L_(HD_, I8_, 1, 4, (I8_ ? 4 : 2)); else L_(HD_, I8_, 2, 4, 2); } while (0)
 #endif
-    const bool bf = kv->act_dtype == MI355_ACT_BF16;
-    MI355_CHECK_ARG(kv->act_dtype == MI355_ACT_F16 || bf, "paged_attn: act_dtype=%d", kv->act_dtype);
-    MI355_CHECK_ARG(int8 || (bf == (kv->kv_dtype == MI355_KV_BF16)), "paged_attn: a 16-bit cache has the dtype of the activations");
 #define LB_(HD_, I8_) do { if (NT == 1) hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, 1, 4, (I8_ ? 4 : 2), true>), grid, dim3(256), 0, st, p); \
                            else         hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, 2, 4, 2, true>), grid, dim3(256), 0, st, p); } while (0)
     if (bf)            { if (kv->hd == 128) { if (int8) LB_(128, true); else LB_(128, false); } else { if (int8) LB_(64, true); else LB_(64, false); } }
