@@ -406,14 +406,14 @@ int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int32_t ld, con
 int mi355_sample_rows(const float* probs, int32_t rows, int32_t V, int32_t ld, const float* uniform_samples, int32_t* ids,
                       mi355_stream_t stream);
 /* The non-greedy branch of the sampler (sampleGreedy, bindings/core/CudaSampleOp.cc:619-800), on fp32 logit rows.
- * mi355_apply_penalties: in place, one launch (+ one memset node):
+ * mi355_apply_penalties: in place, a launch for the temperature and one for the penalties (two for histories of more than 2048 entries):
  *   temperature [B] or NULL: logit *= 1 / (T + 1e-6)          (batchApplyTemperaturePenalty, sampling_penalty_kernels.cu:26-54;
  *                the caller passes NULL when every T == 1, as CudaSampleOp.cc:633-645 skips the launch)
  *   repetition / presence / frequency [B] or NULL, output_ids [step][batch_size] int32 (the transposed token history),
  *   input_lengths [B] or NULL, max_input_length, step: argument for argument invokeBatchApplyRepetitionPenalty
  *   (sampling_penalty_kernels.cu:129-213): every id seen in the history (padding [input_length, max_input_length) skipped)
  *   is penalised once: logit = logit < 0 ? logit * rep : logit / rep; logit -= presence; logit -= frequency * count.
- *   penalty_ws: [B][V] int32 scratch (zeroed here).
+ *   penalty_ws: [B][V] int32 scratch for histories of more than 2048 entries (zeroed here), else not read.
  * mi355_top_k_top_p_sample (CudaSampleOp.cc:748-786): per row of probabilities, drop what is below the top_k-th largest value
  *   (top_k <= 0 or >= V: keep all; ties with the k-th value stay), drop an entry when the mass before it in descending order
  *   (equal values in index order) exceeds top_p (|top_p| < 1e-7 reads as 1), renormalise by max(sum, 1e-10) into probs_out (optional, may alias probs) and draw

@@ -10,14 +10,14 @@
 //
 // Launches per layer (tp = 1):
 //   * 5-64 rows (bf16 and per-channel W8: 1-64), W4 group-wise or W8 per-channel weights, 16-bit cache (rounds 4-5): SIX launches, activations handed over as fragment-ordered images
-//     (common.h act_img_index): QKV + bias + RoPE + KV write (gemm_fullk64.hip) -> paged attention (+ partition reduce) ->
+//     (common.h act_img_index): QKV + bias + RoPE + KV write (gemm_fullk64.hip) -> paged attention (the partition that is done last merges) ->
 //     O + residual, leaving gamma 2^-e h' as an image and the sums of squares -> gate_up + SiLU with the RMSNorm finished on its
 //     accumulators (gemm_wide.hip) -> down as 4 K-quarters (gemm_splitk64.hip) -> fold: slabs + residual + RMSNorm -> image;
-//   * up to 4 rows every GEMM is a full-K launch with its consumer fused (gemm_fullk.hip), 6 launches:
-//     [RMSNorm on load +] QKV + bias + RoPE + KV write -> attention -> partition reduce -> O + residual (leaves the
+//   * up to 4 rows every GEMM is a full-K launch with its consumer fused (gemm_fullk.hip), 5 launches:
+//     [RMSNorm on load +] QKV + bias + RoPE + KV write -> attention -> O + residual (leaves the
 //     per-tile sums of squares) -> RMSNorm on load + gate_up + SiLU-gate -> down + residual;
-//   * other formats / TP (above 12 rows): QKV GEMM (split-K slabs) -> reduce+bias+RoPE+KV-write -> paged attention (+ partition
-//     reduce) -> O GEMM (slabs) -> reduce+residual+RMSNorm -> gate_up GEMM with fused SiLU-gate -> down GEMM (slabs) ->
+//   * other formats / TP (above 12 rows): QKV GEMM (split-K slabs) -> reduce+bias+RoPE+KV-write -> paged attention
+//     -> O GEMM (slabs) -> reduce+residual+RMSNorm -> gate_up GEMM with fused SiLU-gate -> down GEMM (slabs) ->
 //     reduce+residual+RMSNorm (already the next layer's input norm).  No standalone reduce / add / activation kernels.
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -272,7 +272,7 @@ extern "C" mi355_decoder_t* mi355_decoder_create(const mi355_model_config_t* cfg
     d->fuse_rows = 12;
    // tuning build: crossover experiments (tools/batch_sweep.py --tune 6=N)
     // W4 layers only: for small fp16 models (the 0.5B draft of speculative decoding: 36-56 blocks per launch) the fused
-    // launches measured behind the staged kernels (draft step 1.11 vs 1.05 ms), although the kernels take fp16 weights
+    // launches measured behind the staged kernels (0.5B at one sequence: 888 vs 845 us), although the kernels take fp16 weights
     auto w4ok = [](const mi355_weight_t* w) { return w->wbits == 4 && mi355_fullk_weight_ok(w); };
     for (const auto& L : d->layers) {
         d->fuse_qkv = d->fuse_qkv && w4ok(&L.qkv);
@@ -743,7 +743,7 @@ extern "C" int mi355_decoder_set_prefill_rope_table(mi355_decoder_t* d, const fl
 }
 
 // ------------------------------------------------------------------ prefill
-// One chunk of nseq x q_len prompt tokens through the same weights: large-M GEMMs (gemm_prefill.hip above 128 rows), the
+// One chunk of nseq x q_len prompt tokens through the same weights: large-M GEMMs (gemm_prefill.hip above 64 rows), the
 // rows-mode KV writer, causal multi-row attention over the paged cache (earlier chunks of the same prompt are already
 // there), fused residual + RMSNorm; logits only for the requested rows (the reference computes lm_head on the last token
 // of each sequence, PyWrappedModel.cc:1003-1047).
@@ -773,7 +773,7 @@ size_t carve_prefill(const mi355_model_config_t& c, int T, int nseq, void* base,
     b.resid = cv.take(Ts * c.hidden * 2); b.xn = cv.take(Ts * c.hidden * 2); b.qkv = cv.take(Ts * qkvdim * 2);
     b.q = cv.take(Ts * qdim * 2); b.attn = cv.take(Ts * qdim * 2); b.act = cv.take(Ts * c.inter * 2); b.tmp = cv.take(Ts * c.hidden * 2);
     b.last_h = cv.take((size_t)nseq * c.hidden * 2 * 2);
-    // 64-row slabs through the decode kernels (chunks below 128 rows) may split K into fp32 slabs: ask the planner
+    // calls of at most 64 rows go through the decode kernels, which may split K into fp32 slabs: ask the planner
     b.gemm_ws_bytes = linear_ws_bound(c);
     b.gemm_ws = cv.take(b.gemm_ws_bytes);
     b.attn_ws_bytes = mi355_paged_attn_workspace_bytes(T, c.nh, c.hd, c.max_seq_len);
