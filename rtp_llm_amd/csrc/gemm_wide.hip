@@ -319,25 +319,34 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const WideParams wp) {
             for (int mb = 0; mb < MB; ++mb)
                 if (mb != ks) red[((size_t)(wave * (T * 3) + t * 3 + (mb < ks ? mb : mb - 1))) * 64 + lane] = acc[t][mb];
         __syncthreads();
+        f32x4 sum[T];
         auto sum_kept = [&](auto ks_c) {
             constexpr int KS = decltype(ks_c)::value;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                const int tb = th * T + t;
-                if (tb >= ntiles) continue;
                 f32x4 v;
 #pragma unroll
                 for (int s = 0; s < NKS; ++s) {
                     const f32x4 term = (s == KS) ? acc[t][KS] : red[((size_t)((th * NKS + s) * (T * 3) + t * 3 + (KS < s ? KS : KS - 1))) * 64 + lane];
                     v = (s == 0) ? term : v + term;
                 }
-                finish(v, tb, KS);
+                sum[t] = v;
             }
         };
         if (ks == 0) sum_kept(std::integral_constant<int, 0>{});
         else if (ks == 1) sum_kept(std::integral_constant<int, 1>{});
         else if (ks == 2) sum_kept(std::integral_constant<int, 2>{});
         else sum_kept(std::integral_constant<int, MB - 1>{});
+        // one copy of the store's code (4 T of them, each run once per block by one wave, were 30 KB that no instruction cache held): gate_up of 64 rows 29.9 -> 29.3 us
+#pragma unroll 1
+        for (int t = 0; t < T; ++t) {
+            if (th * T + t >= ntiles) break;
+            f32x4 v = sum[0];
+#pragma unroll
+            for (int j = 1; j < T; ++j)
+                if (t == j) v = sum[j];
+            finish(v, th * T + t, ks);
+        }
     } else {
 #pragma unroll
         for (int r0 = 0; r0 < T; r0 += TR) {
