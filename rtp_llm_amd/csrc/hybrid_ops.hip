@@ -1468,7 +1468,7 @@ __global__ __launch_bounds__(1024) void hy_scan_kernel(ScanParams p) {
 }
 
 // ------------------------------------------------------------------------------------------------ gated recurrence, patches of rows and columns
-// The same recurrence (modes HGRN2, GLA and the fixed ones) with keys of at most 8 RPL channels: a lane holds RPL key rows x 4 value columns of the state, a wave all rows of
+// The same recurrence (modes HGRN2 and GLA) with keys of at most 8 RPL channels: a lane holds RPL key rows x 4 value columns of the state, a wave all rows of
 // 32 columns, a block 128 columns.  What bounded hy_scan_kernel is the LDS: its threads hold 8 rows of ONE column, so every wave reads 24 broadcast floats per 24
 // multiply-adds.  Here 7 (RPL 8) wave reads of 16 bytes feed 96 multiply-adds, the gates of a token are formed once per head instead of once per 64 columns,
 // and the sum over the row groups is a three-step exchange between eight lanes (each ends with one column; no LDS, no barrier).
@@ -1534,13 +1534,7 @@ __global__ __launch_bounds__(256) void hy_walk_kernel(ScanParams p, float* cdeca
             for (int c = 0; c < 4; ++c) {
                 if (d + c >= p.dim) continue;
                 const int hd = h * p.dim + d + c;
-                if (p.mode == SCAN_FIXED) {
-                    if (OUT) qv[c] = rq[e][c];
-                    kv[c] = rk[e][c]; av[c] = ((const float*)p.lower)[h];
-                } else if (p.mode == SCAN_FIXED_SILU) {
-                    if (OUT) qv[c] = hy_silu(rq[e][c]);
-                    kv[c] = hy_silu(rk[e][c]); av[c] = ((const float*)p.lower)[h];
-                } else if (p.mode == SCAN_HGRN2) {
+                if (p.mode == SCAN_HGRN2) {
                     const float lw = (float)((const T*)p.lower)[hd];
                     const float f = lw + (1.f - lw) * hy_sigmoid(rk[e][c] + (float)((const T*)p.fbias)[hd]);
                     if (OUT) qv[c] = hy_silu(rq[e][c]);
@@ -1556,13 +1550,7 @@ __global__ __launch_bounds__(256) void hy_walk_kernel(ScanParams p, float* cdeca
             k_s[i] = kv; a_s[i] = av;
         }
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            if (p.mode == SCAN_FIXED_SILU) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) rv[e][c] = hy_silu(rv[e][c]);
-            }
-            v_s[tid + e * 256] = rv[e];
-        }
+        for (int e = 0; e < 2; ++e) v_s[tid + e * 256] = rv[e];
         __syncthreads();
         if (t0 + TOK < r1) fetch(t0 + TOK);
         if (!idle) {
@@ -2745,14 +2733,13 @@ extern "C" int mi355_hy_chunk_prefix_rows(const int32_t* cs, const int32_t* sc, 
     return MI355_OK;
 }
 
-// The recurrence of mi355_hy_scan (modes 0 to 3) on patches of rows and columns (hy_walk_kernel): dim <= 128, MI355_ERR_UNSUPPORTED beyond.  out null: only the states (and
+// The gated recurrences of mi355_hy_scan (modes 0 and 1: HGRN2, GLA) on patches of rows and columns (hy_walk_kernel): dim <= 128, MI355_ERR_UNSUPPORTED beyond.  out null: only the states (and
 // cdecay fp32 [nseq, H, dim], the product of the sequence's decays per key row, unless null).  keep_state 0: the states are read, not written back.
 extern "C" int mi355_hy_walk(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, const float* z, int32_t ldz, const void* lower,
                              const void* fbias, float tau, float qscale, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start, const int32_t* slot,
                              const int32_t* first_pos, int32_t nseq, float* state, float* out, float* cdecay, int32_t keep_state, int32_t act_dtype, mi355_stream_t stream) {
     MI355_CHECK_ARG(proj && row_start && slot && first_pos && state && nseq > 0 && H > 0 && dim > 0 && vdim > 0, "hy_walk: bad argument");
-    MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : (mode == SCAN_FIXED || mode == SCAN_FIXED_SILU) ? lower != nullptr : (mode == SCAN_GLA && z && tau > 0.f),
-                    "hy_walk: mode %d lacks its gate inputs", mode);
+    MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : (mode == SCAN_GLA && z && tau > 0.f), "hy_walk: mode %d lacks its gate inputs", mode);
     if (dim > 128) return MI355_ERR_UNSUPPORTED;
     auto al = [](const void* q) { return (uintptr_t)q % 16 == 0; };
     const int vec = dim % 4 == 0 && vdim % 4 == 0 && ld % 4 == 0 && qo % 4 == 0 && ko % 4 == 0 && vo % 4 == 0 && al(proj) && al(state) &&

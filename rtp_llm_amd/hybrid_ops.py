@@ -447,8 +447,8 @@ WALK_MAX_DIM = 128         # key channels of mi355_hy_walk
 def walk_chunk(T: int, nseq: int, max_rows: int, heads: int, vdim: int) -> int:
     """Chunk size of the gated recurrence over prompt portions, 0: walked whole.  A model of both in us: the whole walk takes 0.33 a token of the longest
     sequence for every 512 blocks of 64 columns; the chunks (of 32, 64 or 128 tokens, so that their blocks fill the chip once) two walks of a chunk behind 30 of
-    launches and prefix, or 1.85e-3 a token and head where the chip is full.  Measured, heads of 64 x 128, whole / chunks: 4 x 2048 tokens 16 heads 680 / 253,
-    1 x 2048 16 heads 665 / 103, 1 x 1537 8 heads 504 / 64, 2 x 300 8 heads 100 / 46, 16 x 512 16 heads 225 / 254, 8 x 96 16 heads 38 / 55."""
+    launches and prefix, or 1.85e-3 a token and head where the chip is full.  Measured, heads of 64 x 128, whole / chunks: 4 x 2048 tokens 16 heads 683 / 265,
+    1 x 2048 16 heads 668 / 105, 1 x 1537 8 heads 504 / 65, 2 x 300 8 heads 100 / 46, 16 x 512 16 heads 232 / 253, 8 x 96 16 heads 38 / 57."""
     longest = max_rows if max_rows > 0 else T - (nseq - 1)
     work = T * heads * ((vdim + 127) // 128)
     C = 32 if work < 50000 else 64 if work < 100000 else 128

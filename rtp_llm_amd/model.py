@@ -588,7 +588,7 @@ class DecoderEngine:
             counts = [max(0, min(q_len, len(p) - c0)) for p in prompts]
             first = [sum(counts[:b]) for b in range(nseq + 1)]
             T = first[nseq]
-            toks = torch.cat([torch.as_tensor(p[c0:c0 + n], dtype=torch.int32) for p, n in zip(prompts, counts)])
+            toks = torch.cat([torch.as_tensor(p[c0:c0 + n], dtype=torch.int32).cpu() for p, n in zip(prompts, counts)])
             pos = torch.cat([torch.arange(start[b] + c0, start[b] + c0 + n, dtype=torch.int32) for b, n in enumerate(counts)])
             ending = [b for b, p in enumerate(prompts) if counts[b] and c0 + counts[b] == len(p)]
             last = torch.zeros(nseq, dtype=torch.int32)
