@@ -43,6 +43,7 @@ struct AttnParams {
     float*         tmp_out; // [B][nh][P][hd]
     float*         tmp_ml;  // [B][nh][P][2]
     int32_t*       done;    // non-null (zeros before and after): [row tile of a sequence][kv head], the partitions that have left their part; the last one merges
+    int            done_step;  // int32 from one counter to the next (32: a cache line of its own each)
     int B, nh, nkv, G, page, max_blocks, P, PS, seq_add, max_seq, num_blocks;
     int q_len, R, ntile;   // rows per sequence (of the longest, with row_start), rows per 16-column tile (16 / G), row tiles per sequence
     const int32_t* row_start; // non-null (the two-tile instances): sequence b has rows row_start[b] .. row_start[b + 1] - 1, no padding rows between
@@ -562,40 +563,71 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     // written through to where the other XCDs see it before the block counts itself; the last block sees all counts, then reads all parts from there.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's part has arrived
     __syncthreads();
-    if (tid == 0) s_m[0][0] = __builtin_bit_cast(float, __hip_atomic_fetch_add(p.done + (size_t)blockIdx.z * p.nkv + kh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (tid == 0) s_m[0][0] = __builtin_bit_cast(float, __hip_atomic_fetch_add(p.done + ((size_t)blockIdx.z * p.nkv + kh) * p.done_step, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     __syncthreads();
     if (__builtin_bit_cast(int, s_m[0][0]) != nparts - 1) return;
-    for (int idx = tid; idx < nrows * p.G * (HD / 4); idx += NTHR) {
-        const int col = idx / (HD / 4), d0 = (idx - col * (HD / 4)) * 4, rl = col / p.G, row = row0 + rl, h = kh * p.G + (col - rl * p.G);
-        const int np = (min(max(p.seq_lens[row] + p.seq_add, 0), p.max_seq) + p.PS - 1) / p.PS;      // partitions that saw this row
-        const size_t slot = ((size_t)row * p.nh + h) * p.P;
-        const float* ml = p.tmp_ml + slot * 2;
-        const float* po = p.tmp_out + slot * HD + d0;
-        float mstar = NEG_BIG, l = 0.f;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int i0 = 0; i0 < np; i0 += 8) {                     // eight parts in flight, summed in partition order
-            float2 v[8], oa[8], ob[8];
+    // Up to eight parts: a thread takes four channels of a row's head through all of them in one round trip.  More: eight or sixteen in flight by 16-byte loads, and where
+    // the rows leave threads without channels (7 heads of 64: 112 of 256) the waves split the parts and meet in LDS.  Against the merge in a launch of its own, us per call,
+    // before / now / launch: 14 over 2 heads of 64, 8 sequences, 8 parts 8.0 / 7.0 / 7.5, 16 parts 10.4 / 7.8 / 7.7, 1 sequence, 32 parts 9.9 / 8.3 / 11.6; 28 over 4 heads of
+    // 128, 4 sequences, 8 parts 9.3 / 8.2 / 8.7, 16 parts 12.0 / 9.6 / 9.5, 1 sequence, 16 parts 9.6 / 9.2 / 9.0, 32 parts 12.9 / 11.4 / 13.2.  Most of it was the counters:
+    // side by side, up to 256 arrivals went through one cache line (8 sequences of 16 parts: 8.1 with nothing changed but their distance).
+    auto merge = [&](auto in_flight, auto split) {
+        constexpr int U = decltype(in_flight)::value;
+        const int items = nrows * p.G * (HD / 4), share = !decltype(split)::value ? 1 : items <= 64 ? NW : items <= 64 * NW / 2 ? 2 : 1, span = NTHR / share;
+        const int sw = wave / (NW / share);                          // which of the waves that share an item
+        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void*)p.tmp_out, 0, 0x7FFFFFFC, 0x00020000);
+        const uint32_t mlo = (uint32_t)(p.tmp_ml - p.tmp_out) * 4u;
+        f32x4* x_o = reinterpret_cast<f32x4*>(&s_o[0][0][0]);
+        float2* x_ml = reinterpret_cast<float2*>(x_o + (share - 1) * span);
+        for (int at = tid - sw * span; at < (share > 1 ? span : items); at += NTHR) {
+            const int idx = share > 1 ? min(at, items - 1) : at, col = idx / (HD / 4), d0 = (idx - col * (HD / 4)) * 4, rl = col / p.G, row = row0 + rl, h = kh * p.G + (col - rl * p.G);
+            const int np = (min(max(p.seq_lens[row] + p.seq_add, 0), p.max_seq) + p.PS - 1) / p.PS;      // partitions that saw this row
+            const size_t slot = ((size_t)row * p.nh + h) * p.P;
+            const float* ml = p.tmp_ml + slot * 2;
+            const float* po = p.tmp_out + slot * HD + d0;
+            float mstar = NEG_BIG, l = 0.f;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            for (int i0 = sw * U; i0 < np; i0 += share * U) {        // U parts in flight, summed in partition order
+                float2 v[U], oa[U], ob[U];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int i = min(i0 + u, np - 1);
-                v[u] = get2(ml + i * 2); oa[u] = get2(po + (size_t)i * HD); ob[u] = get2(po + (size_t)i * HD + 2);
+                for (int u = 0; u < U; ++u) {
+                    const int i = min(i0 + u, np - 1);
+                    if constexpr (decltype(split)::value) {
+                        const u32x4 o4 = __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)((slot + i) * HD + d0) * 4u, 0, 16 /* sc1 */);
+                        v[u] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rp, mlo + (uint32_t)(slot + i) * 8u, 0, 16));
+                        oa[u] = __builtin_bit_cast(float2, u32x2{o4[0], o4[1]}); ob[u] = __builtin_bit_cast(float2, u32x2{o4[2], o4[3]});
+                    } else { v[u] = get2(ml + i * 2); oa[u] = get2(po + (size_t)i * HD); ob[u] = get2(po + (size_t)i * HD + 2); }
+                }
+                float mnew = mstar;
+#pragma unroll
+                for (int u = 0; u < U; ++u) mnew = fmaxf(mnew, v[u].x);
+                const float resc = __builtin_amdgcn_exp2f(mstar - mnew);
+                l *= resc; acc *= resc; mstar = mnew;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (i0 + u >= np) continue;
+                    const float f = __builtin_amdgcn_exp2f(v[u].x - mstar);
+                    l += v[u].y * f;
+                    acc += f32x4{oa[u].x, oa[u].y, ob[u].x, ob[u].y} * f;
+                }
             }
-            float mnew = mstar;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) mnew = fmaxf(mnew, v[u].x);
-            const float resc = __builtin_amdgcn_exp2f(mstar - mnew);
-            l *= resc; acc *= resc; mstar = mnew;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (i0 + u >= np) continue;
-                const float f = __builtin_amdgcn_exp2f(v[u].x - mstar);
-                l += v[u].y * f;
-                acc += f32x4{oa[u].x, oa[u].y, ob[u].x, ob[u].y} * f;
+            if (share > 1) {                                         // one pass of the loop for every wave
+                if (sw > 0) { x_o[(sw - 1) * span + at] = acc; x_ml[(sw - 1) * span + at] = make_float2(mstar, l); }
+                __syncthreads();
+                if (sw > 0 || at >= items) break;
+                for (int k = 0; k < share - 1; ++k) {
+                    const float2 o_ml = x_ml[k * span + at];
+                    const float mnew = fmaxf(mstar, o_ml.x), fa = __builtin_amdgcn_exp2f(mstar - mnew), fb = __builtin_amdgcn_exp2f(o_ml.x - mnew);
+                    l = l * fa + o_ml.y * fb; acc = acc * fa + x_o[k * span + at] * fb; mstar = mnew;
+                }
             }
+            store_out(row, h * HD + d0, acc, l);
         }
-        store_out(row, h * HD + d0, acc, l);
-    }
-    if (tid == 0) __hip_atomic_store(p.done + (size_t)blockIdx.z * p.nkv + kh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (nparts <= 8) merge(std::integral_constant<int, 8>{}, std::false_type{});
+    else if (nparts <= 16 && nrows * p.G * (HD / 4) <= 64 * NW / 2) merge(std::integral_constant<int, 8>{}, std::true_type{});
+    else merge(std::integral_constant<int, 16>{}, std::true_type{});
+    if (tid == 0) __hip_atomic_store(p.done + ((size_t)blockIdx.z * p.nkv + kh) * p.done_step, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ------------------------------------------------------------------------------------------------ prompt rows (16-bit cache)
@@ -871,7 +903,7 @@ namespace {
 int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table, int32_t max_blocks_per_seq,
                 const int32_t* seq_lens, int32_t seq_lens_minus_one, int32_t B, int32_t q_len, int32_t nh, float scale,
                 int32_t max_seq_len, void* out, void* workspace, size_t workspace_bytes, mi355_stream_t stream, int img_mblk = 0,
-                const int32_t* row_start = nullptr, int32_t total_rows = 0, int32_t* done = nullptr) {
+                const int32_t* row_start = nullptr, int32_t total_rows = 0, int32_t* done = nullptr, int done_step = 1) {
     MI355_CHECK_ARG(q && kv && kv->kv_base && block_table && seq_lens && out, "paged_attn: null pointer");
     MI355_CHECK_ARG(kv->hd == 64 || kv->hd == 128, "paged_attn: hd=%d (64 or 128)", kv->hd);
     MI355_CHECK_ARG(kv->page >= 16 && kv->page % 8 == 0, "paged_attn: page=%d (>= 16, multiple of 8)", kv->page);
@@ -926,7 +958,7 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
         mi355_set_error("paged_attn: workspace %zu < %zu", workspace_bytes, need);
         return MI355_ERR_WORKSPACE;
     }
-    p.done = p.P > 1 ? done : nullptr;
+    p.done = p.P > 1 ? done : nullptr; p.done_step = done_step;
     p.tmp_out = (float*)workspace;
     p.tmp_ml  = p.tmp_out + rows * nh * p.P * kv->hd;
     hipStream_t st = (hipStream_t)stream;
@@ -1007,12 +1039,13 @@ extern "C" int mi355_paged_attn_rows_img(const void* q, const mi355_kv_layer_t* 
                        workspace_bytes, stream, cdiv(B * q_len, 16));
 }
 
-// What the step driver calls: out row-major or (img) an activation image; done: [B * row tiles][nkv] counters that are zero (B * q_len * nkv of them suffice), left at zero.
-// Calls that share them must not overlap.
+// What the step driver calls.  form: MI355_ATTN_IMG = out is an activation image (else row-major), MI355_ATTN_DONE_APART = the counters lie 128 bytes apart (else side by
+// side).  done: [B * row tiles][nkv] counters that are zero (B * q_len * nkv of them suffice), left at zero.  Calls that share them must not overlap.
 extern "C" int mi355_paged_attn_step(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table, int32_t max_blocks_per_seq, const int32_t* positions,
-                                     int32_t B, int32_t q_len, int32_t nh, float scale, int32_t max_seq_len, void* out, int32_t img, void* workspace, size_t workspace_bytes,
+                                     int32_t B, int32_t q_len, int32_t nh, float scale, int32_t max_seq_len, void* out, int32_t form, void* workspace, size_t workspace_bytes,
                                      int32_t* done, mi355_stream_t stream) {
+    const bool img = form & MI355_ATTN_IMG;
     MI355_CHECK_ARG(!img || (B > 0 && q_len > 0 && B * q_len <= 64 && kv && (nh * kv->hd) % 32 == 0), "paged_attn_step: %d x %d rows (<= 64)", B, q_len);
     return launch_attn(q, kv, block_table, max_blocks_per_seq, positions, 1, B, q_len, nh, scale, max_seq_len, out, workspace, workspace_bytes, stream,
-                       img ? cdiv(B * q_len, 16) : 0, nullptr, 0, done);
+                       img ? cdiv(B * q_len, 16) : 0, nullptr, 0, done, form & MI355_ATTN_DONE_APART ? 32 : 1);
 }

@@ -50,7 +50,7 @@ struct mi355_decoder {
     // carved workspace
     void *resid, *xn, *q_buf, *attn_out, *act, *attn_ws, *argmax_ws;
     void *xn_img, *attn_img;   // activation images (mi355_act_image_*) of the normed hidden rows / the attention output, 5-64-row steps
-    int32_t* attn_done; // counters of the attention's last-partition merge, zero between launches: [64 rows][nkv]
+    int32_t* attn_done; // counters of the attention's last-partition merge, zero between launches: [64 rows][nkv], 128 bytes apart
     int32_t* oob_count; // tokens refused by the KV writer (stale position / block id)
     const float* prefill_cos_sin = nullptr;   // mi355_decoder_set_prefill_rope_table: {cos, sin} rows of the NEXT prefill chunks (dynamic-NTK prompts past the original context), or null
     mi355_allreduce_t* ar; // attached all-reduce context (tp_size > 1): the TP step runs entirely from C++
@@ -155,7 +155,7 @@ size_t carve_all(mi355_decoder* d, const mi355_model_config_t& c, void* base) {
     const size_t gw = (size_t)c.max_batch * 64 * 8;
     void* argmax_ws = cv.take(gw);
     void* oob = cv.take(256);
-    void* done = cv.take(MB_ * c.nkv * 4);
+    void* done = cv.take(MB_ * c.nkv * 128);
     void* ssq = cv.take((size_t)16 * ((c.hidden / 16 + 3) & ~3) * 4);   // per-tile sums of squares of the residual rows (fused norm, <= 16 rows)
     void* xn_img = cv.take(mi355_act_image_bytes(64, c.hidden));
     void* xg_img = cv.take(mi355_act_image_bytes(64, c.hidden));
@@ -353,7 +353,7 @@ extern "C" mi355_decoder_t* mi355_decoder_create(const mi355_model_config_t* cfg
     }
     std::vector<int32_t> iota_h(cfg->max_batch);
     for (int i = 0; i < cfg->max_batch; ++i) iota_h[i] = i;
-    if (hipMemset(d->oob_count, 0, 256) != hipSuccess || hipMemset(d->attn_done, 0, (size_t)(cfg->max_batch < 64 ? cfg->max_batch : 64) * cfg->nkv * 4) != hipSuccess ||
+    if (hipMemset(d->oob_count, 0, 256) != hipSuccess || hipMemset(d->attn_done, 0, (size_t)(cfg->max_batch < 64 ? cfg->max_batch : 64) * cfg->nkv * 128) != hipSuccess ||
         hipMemcpy(d->iota, iota_h.data(), iota_h.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
         mi355_set_error("decoder_create: cannot initialise the workspace"); delete d; return nullptr;
     }
@@ -597,7 +597,7 @@ extern "C" int mi355_decoder_layer_attn(mi355_decoder_t* d, int32_t l, mi355_str
     // q_len > 1: rows of one sequence share a pass over its KV, causal mask inside the page walk (is_target_verify)
     if (tp_img && d->tp_pub_o && B <= 64 && pub_ready(d, B)) {   // TP: attention image -> O shard published in the all-reduce buffer -> exchange + residual + norm
         RUN(MI355_KC_ATTN, mi355_paged_attn_step(d->q_buf, &kv, d->bufs.block_table, c.max_blocks_per_seq, d->bufs.positions,
-                                                 B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_img, 1,
+                                                 B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_img, MI355_ATTN_IMG | MI355_ATTN_DONE_APART,
                                                  d->attn_ws, d->attn_ws_bytes, d->attn_done, st));
         if (int e = pf_join(d, st)) return e;
         RUN(MI355_KC_GEMM_QUANT, mi355_linear_publish_img(d->attn_img, B, &L.o, nullptr, d->ar, st));
@@ -608,7 +608,7 @@ extern "C" int mi355_decoder_layer_attn(mi355_decoder_t* d, int32_t l, mi355_str
     }
     if (mid_o) {   // the attention output as an image: what the O projection's full-K launch reads
         RUN(MI355_KC_ATTN, mi355_paged_attn_step(d->q_buf, &kv, d->bufs.block_table, c.max_blocks_per_seq, d->bufs.positions,
-                                                 B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_img, 1,
+                                                 B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_img, MI355_ATTN_IMG | MI355_ATTN_DONE_APART,
                                                  d->attn_ws, d->attn_ws_bytes, d->attn_done, st));
         if (int e = pf_join(d, st)) return e;
         if (d->img_gate_up) {   // no norm launch: gate_up finishes the RMSNorm on its accumulators
@@ -622,7 +622,7 @@ extern "C" int mi355_decoder_layer_attn(mi355_decoder_t* d, int32_t l, mi355_str
         return MI355_OK;
     }
     RUN(MI355_KC_ATTN, mi355_paged_attn_step(d->q_buf, &kv, d->bufs.block_table, c.max_blocks_per_seq, d->bufs.positions,
-                                             B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_out, 0,
+                                             B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_out, MI355_ATTN_DONE_APART,
                                              d->attn_ws, d->attn_ws_bytes, d->attn_done, st));
     if (int e = pf_join(d, st)) return e;
     if (d->fuse_o && small) {     // h += fp16(attn W_o) in the GEMM's epilogue: no slabs; the norm moves into gate_up (or stays a launch)

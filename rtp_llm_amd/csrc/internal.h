@@ -15,9 +15,10 @@ int mi355_paged_decode_attn_ex(const void* q, const mi355_kv_layer_t* kv, const 
                                int32_t max_blocks_per_seq, const int32_t* seq_lens, int32_t seq_lens_minus_one, int32_t B,
                                int32_t nh, float scale, int32_t max_seq_len, void* out, void* workspace,
                                size_t workspace_bytes, mi355_stream_t stream);
-/* attention.hip: mi355_paged_attn_rows / _img whose last partition merges (done: [B * q_len][nkv] int32 counters, zero before and after) */
+/* attention.hip: mi355_paged_attn_rows / _img whose last partition merges (done: [B * q_len][nkv] int32 counters, zero before and after; form: the flags below) */
+enum { MI355_ATTN_IMG = 1, MI355_ATTN_DONE_APART = 2 };
 int mi355_paged_attn_step(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_table, int32_t max_blocks_per_seq, const int32_t* positions,
-                          int32_t B, int32_t q_len, int32_t nh, float scale, int32_t max_seq_len, void* out, int32_t img, void* workspace, size_t workspace_bytes,
+                          int32_t B, int32_t q_len, int32_t nh, float scale, int32_t max_seq_len, void* out, int32_t form, void* workspace, size_t workspace_bytes,
                           int32_t* done, mi355_stream_t stream);
 int mi355_fullk_weight_ok(const mi355_weight_t* w);
 int mi355_fullk64_weight_ok(const mi355_weight_t* w);     /* gemm.hip: the full-K launches on activation images (gemm_fullk64.hip) take this linear */
