@@ -627,14 +627,20 @@ __device__ __forceinline__ int search_histogram(const float* q, int V, bool vec,
     const double m_lane = __shfl_up(mi, 1);
     if (lane > 0) m_at += m_lane;
     if (use_p) use_p = total > (double)tp;                                      // nothing to drop when even the mass above 0 fits
+    // The prefix up to a thread's bins and the sum over the bins of the thread before it round differently: both may see p crossed.  The larger values' bin has it, with the sum
+    // of the thread that it belongs to.
+    int mine_q = -1;
+    double mine_above = 0.0;
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
         const int bin = kBins - 1 - (tx * PB + i);
         if (use_k && c_at < (uint32_t)k && c_at + c[i] >= (uint32_t)k) { sh.bin_k = bin; sh.above_k = c_at; }
-        if (use_p && m_at <= (double)tp && m_at + m[i] > (double)tp) { sh.bin_q = bin; sh.above_q = m_at; }
+        if (use_p && m_at <= (double)tp && m_at + m[i] > (double)tp) { mine_q = bin; mine_above = m_at; }
         c_at += c[i]; m_at += m[i];
     }
+    if (mine_q >= 0) atomicMax(&sh.bin_q, mine_q);
     __syncthreads();
+    if (mine_q >= 0 && mine_q == sh.bin_q) sh.above_q = mine_above;             // read behind the candidates' barrier
     const int bin_k = use_k ? sh.bin_k : -1, bin_q = use_p ? sh.bin_q : -1;     // bin_k -1: fewer than k entries are above zero
     if (use_p && bin_q < 0) return 0;                                           // the sums crossed p between a thread's last bin and the next thread's first
     kb = 0; vbits = 0;
