@@ -1,4 +1,4 @@
-"""The sampler where its arithmetic or its grid is at an edge: a top-p that falls on the rounding of the bins' 64-bit sums."""
+"""The sampler where its arithmetic or its grid is at an edge: a top-p that falls on the rounding of the bins' 64-bit sums, more rows than the 65535 of many grids' second dimension."""
 from fractions import Fraction
 
 import pytest
@@ -27,3 +27,23 @@ def test_top_p_within_a_rounding_of_a_bin_border(V):
     assert int(want.sum()) == 5
     ids, out = ops.top_k_top_p_sample(probs.to(DEV), torch.zeros(3, dtype=torch.int32), torch.full((3,), 0.75), torch.tensor([0.1, 0.5, 0.9]).to(DEV), return_probs=True)
     assert torch.equal(out.cpu() > 0, want.expand(3, V)) and bool(want[ids.cpu().long()].all())
+
+
+@pytest.mark.parametrize("V", [3, 8])
+def test_more_than_65536_rows(V):
+    """65536 + 5 rows: temperature alone, temperature and penalties, and the joint form, against each row's own arithmetic (2^-22 of a value: a division and a product)."""
+    B = (1 << 16) + 5
+    g = torch.Generator(device=DEV).manual_seed(V)
+    x, t = torch.randn(B, V, device=DEV, generator=g) * 3, torch.rand(B, device=DEV, generator=g) + 0.5
+    want = x * (1.0 / (t + 1e-6))[:, None]
+    got = ops.apply_penalties(x.clone(), temperature=t)
+    assert bool(((got - want).abs() <= 2.0 ** -22 * want.abs()).all())
+    ids = torch.randint(0, V, (B, 2), device=DEV, generator=g, dtype=torch.int32)
+    pen = dict(repetition_penalty=torch.full((B,), 1.5, device=DEV), presence_penalty=torch.full((B,), 0.25, device=DEV), frequency_penalty=torch.full((B,), 0.5, device=DEV))
+    count = torch.zeros_like(x).scatter_add_(1, ids.long(), torch.ones(B, 2, device=DEV))
+    full = torch.where(count > 0, torch.where(want < 0, want * 1.5, want / 1.5) - 0.25 - 0.5 * count, want)
+    lens = torch.full((B,), 2, dtype=torch.int32, device=DEV)
+    got = ops.apply_penalties(x.clone(), temperature=t, output_ids=ids.t().contiguous(), input_lengths=lens, max_input_length=2, step=2, **pen)
+    assert bool(((got - full).abs() <= 2.0 ** -21 * (full.abs() + 2)).all())
+    got = ops.sampling_probs(x.clone(), t, token_ids=ids, input_lengths=lens, max_input_length=2, step=2, **pen)
+    assert bool(((got - full.double().softmax(-1)).abs() <= 2.0 ** -18).all())
