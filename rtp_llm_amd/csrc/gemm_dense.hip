@@ -6,7 +6,8 @@
 //   * tile kernels, bf16: block tiles of 64 x 128 up to 256 x 256, both operands through LDS by DMA, MFMA 16x16x32; one that stages 64 x 128 through registers
 //     for operands without 16-byte alignment;
 //   * tile kernel, fp32:  64 x 64 block tile, 4 x 4 register micro-tiles, true fp32 FMAs (no reduced-precision matrix mode);
-//   * skinny kernel, bf16, 2 <= M <= 16: one block per 16 outputs, its waves split K, MFMA fragments loaded straight from memory;
+//   * skinny kernel, bf16, 2 <= M <= 16: one block per 16 outputs (8 of few outputs and rows, with the same partial sums), its waves split K, MFMA fragments loaded
+//     straight from memory;
 //   * row kernel (M = 1; fp32 up to M = 16): a wave per output column streams its weight row once, 16-byte loads, wave reduction at the end.
 //   * grouped forms of these kernels (per-head or per-branch weights over column slices; rows sorted by expert with a gather and a tile
 //     list; the few rows of a decode step, each with its own expert's weight): mi355_dense_grouped.
@@ -694,35 +695,37 @@ void launch_rows(const DenseParams& p, hipStream_t st) {
 // the A operand and 16 weight rows as B, both fragments loaded straight from memory (8 consecutive k per lane, no LDS staging).  The weight
 // stream is read once whatever M is; the waves' partial tiles are summed through LDS.  Under GATED a tile is 16 channels: their gate rows and
 // their up rows share the A fragments.
-// HALF (M <= 8, K % 64 == 0): 8 outputs per block.  Rows 0 to 7 of the first operand are x over the first half of K, rows 8 to 15 x over the second, the second
-// operand likewise: of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are the halves of the result, the rest is not used.
+// HALF (M <= 8): 8 outputs per block and half the waves, each with the k-steps of two of them: rows 0 to 7 of the first operand are x in the steps of wave w, rows 8 to 15 x in
+// those of wave w + NW, the second operand likewise.  Of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are what the two waves would hold, the rest is not used;
+// the partial sums and their order are those of 16 outputs, a row's bits do not depend on how many rows (2 to 16) there are.
 template <bool GATED, bool HALF>
 __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, int mbase) {
     __shared__ f32x4 red[8][2][64];
     constexpr int NO = HALF ? 8 : 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, NW = blockDim.x >> 6;
     const int nout = GATED ? p.N / 2 : p.N, grp = blockIdx.y;
-    const int r = lane & (NO - 1), K = HALF ? p.K / 2 : p.K, kq = (lane >> 4) * 8, kh = HALF && (lane & 8) ? K : 0;
+    const int r = lane & (NO - 1), chains = HALF ? 2 * NW : NW, kq = (lane >> 4) * 8 + (HALF && (lane & 8) ? NW * 32 : 0);
     const int o = min((int)blockIdx.x * NO + r, nout - 1);
     const int n = GATED ? (o >> 5) * 64 + (o & 31) : o;
-    const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kh + kq;
+    const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kq;
     const bf16* wu = wg + (size_t)32 * p.K;
-    const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(mbase + r, p.M - 1) * p.ldx + kh + kq;
+    const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(mbase + r, p.M - 1) * p.ldx + kq;
     f32x4 ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
     const bf16x8 zero = {};
-    const int stride = NW * 32;
-    for (int k0 = wave * 32; k0 < K; k0 += 4 * stride) {
-        bf16x8 a[4], b[4], c[4];
+    constexpr int U = HALF ? 8 : 4;                          // steps in flight: the same bytes per compute unit in both forms
+    const int stride = chains * 32;
+    for (int k0 = wave * 32; k0 < p.K; k0 += U * stride) {
+        bf16x8 a[U], b[U], c[U];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int k = k0 + u * stride;
-            const bool ok = k + kq < K;
+            const bool ok = k + kq < p.K;
             a[u] = ok ? *(const bf16x8*)(xr + k) : zero;
             b[u] = ok ? *(const bf16x8*)(wg + k) : zero;
             if (GATED) c[u] = ok ? *(const bf16x8*)(wu + k) : zero;
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < U; ++u) {
             ag = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], ag, 0, 0, 0);
             if (GATED) au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], c[u], au, 0, 0, 0);
         }
@@ -735,16 +738,13 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
         ag += red[w][0][lane];
         if (GATED) au += red[w][1][lane];
     }
-    // C fragment: lane holds output (lane & 15), rows 4 * (lane >> 4) + e; HALF: the second half's sum of (output, row) lies at (output + 8, row + 8), 40 lanes on
+    // C fragment: lane holds output (lane & 15), rows 4 * (lane >> 4) + e; HALF: the second wave's sum of (output, row) lies at (output + 8, row + 8), 40 lanes on
     if constexpr (HALF) {
         if ((lane & 8) || lane >= 32) return;
-        f32x4 g2 = red[0][0][lane + 40], u2 = GATED ? red[0][1][lane + 40] : g2;
-        for (int w = 1; w < NW; ++w) {
-            g2 += red[w][0][lane + 40];
-            if (GATED) u2 += red[w][1][lane + 40];
+        for (int w = 0; w < NW; ++w) {
+            ag += red[w][0][lane + 40];
+            if (GATED) au += red[w][1][lane + 40];
         }
-        ag += g2;
-        if (GATED) au += u2;
     }
     const int oc = blockIdx.x * NO + r;
     if (oc >= nout) return;
@@ -759,13 +759,12 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
     }
 }
 
-// M of 2 to 16, p.vec.  Few outputs (2048 make 128 blocks of 16): 8 per block where M allows it, so that all compute units pull weights; narrow outputs: more waves per
-// tile keep the memory system busy.  M = 8, weights from memory, us with 16 / 8 outputs: 2048 x 5632 12.5 / 9.5, 2048 x 2048 6.3 / 5.6, 16 x 2048 5.3 / 4.8,
-// 1024 x 1024 4.5 / 4.1 (4 waves), 4096 x 2048 7.4 / 8.2.
+// M of 2 to 16, p.vec.  Few outputs: 8 per block where M allows it, so that all compute units pull weights; narrow outputs: more waves per tile keep the memory system
+// busy.  M = 8, weights from memory, us with 16 / 8 outputs: 2048 x 5632 12.8 / 10.7, 2048 x 2048 6.4 / 5.6, 16 x 2048 5.3 / 4.4, 1024 x 1024 4.8 / 4.4, 4096 x 2048 7.4 / 8.2.
 void launch_skinny(const DenseParams& p, hipStream_t st) {
     const int nout = p.gated ? p.N / 2 : p.N, tiles = (nout + 15) / 16;
-    if (p.M <= 8 && p.K % 64 == 0 && p.K >= 128 && tiles * p.G <= 192) {
-        const dim3 grid((nout + 7) / 8, p.G), block(p.K < 2048 ? 256 : 512);
+    if (p.M <= 8 && p.K >= 128 && tiles * p.G <= 192) {
+        const dim3 grid((nout + 7) / 8, p.G), block(p.K < 1024 ? 128 : 256);
         if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, true>), grid, block, 0, st, p, 0);
         else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, true>), grid, block, 0, st, p, 0);
         return;
