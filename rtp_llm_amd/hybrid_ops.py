@@ -444,16 +444,28 @@ SCAN_BLOCKS_AT_ONCE = 512  # blocks of the scan kernel the chip runs side by sid
 WALK_MAX_DIM = 128         # key channels of mi355_hy_walk
 
 
-def walk_chunk(T: int, nseq: int, max_rows: int, heads: int, vdim: int) -> int:
-    """Chunk size of the gated recurrence over prompt portions, 0: walked whole.  A model of both in us: the whole walk takes 0.33 a token of the longest
-    sequence for every 512 blocks of 64 columns; the chunks (of 32, 64 or 128 tokens, so that their blocks fill the chip once) two walks of a chunk behind 30 of
-    launches and prefix, or 1.85e-3 a token and head where the chip is full.  Measured, heads of 64 x 128, whole / chunks: 4 x 2048 tokens 16 heads 683 / 265,
-    1 x 2048 16 heads 668 / 105, 1 x 1537 8 heads 504 / 65, 2 x 300 8 heads 100 / 46, 16 x 512 16 heads 232 / 253, 8 x 96 16 heads 38 / 57."""
+def gated_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int) -> Optional[int]:
+    """How a gated recurrence of keys up to WALK_MAX_DIM channels runs: a chunk size (hy_walk over chunks), 0 (hy_walk, whole) or None (hy_scan, whole).
+    A model of the three in us, fitted to 460 calls of 2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64 sequences of 1 to 2048 rows: a call takes what its
+    longest sequence (chunk) walks in series, or the rounds of its blocks if that is more.  hy_scan: blocks of 64 columns and a wave for 8 key rows, 16 waves on a compute unit,
+    0.28 (keys of 32) to 0.45 (128) a token.  hy_walk: blocks of 128 columns, 0.42 a token, or 0.75 and one block on a compute unit from 65 key channels on; with few blocks, or
+    values of 64 that leave half a block idle, that loses to hy_scan.  Chunks: two passes of it, launches and the chunk states.  In those calls the pick is never slower
+    than hy_scan by more than 2 %, 4 % off the fastest in the mean.
+    Measured, us, hy_scan / whole / chunks: 16 heads of 64 x 128, 4 x 2048 rows 684 / 683 / 265, 1 x 2048 668 / - / 105; 4 heads of 96 x 64, 37 sequences of up to 317
+    141 / 237 / 286; 8 heads of 128 x 256, 8 x 195 105 / 137 / 181; 32 heads of 128 x 128, 9 x 136 208 / 331 / -, 16 x 339 694 / 495 / -."""
     longest = max_rows if max_rows > 0 else T - (nseq - 1)
-    work = T * heads * ((vdim + 127) // 128)
-    C = 32 if work < 50000 else 64 if work < 100000 else 128
-    whole = 0.33 * longest * -(-nseq * heads * ((vdim + 63) // 64) // 512)
-    return C if longest > C and max(30.0 + 0.6 * C, 12.0 + 1.85e-3 * work) < whole else 0
+    waves = -(-dim // 8)
+    scan_us = 5.5 + (0.22 + 0.0145 * waves) * max(longest, -(-nseq * heads * -(-vdim // 64) // (256 * (16 // waves))) * T / nseq)
+    blocks, wide = heads * -(-vdim // 128), dim > 64
+    work = T * blocks
+    best, us = 0, 8.0 + 0.75 * max(longest, -(-nseq * blocks // 256) * T / nseq) if wide else 5.6 + 0.42 * max(longest, work / 420)
+    for C in (32, 64, 128):
+        if longest > C:
+            states = (T / C + 0.5 * nseq) * heads * dim * vdim * 1e-6
+            t = 20.0 + 1.14 * max(C, work / 170) + 1.9 * states if wide else 14.0 + 0.67 * max(C, work / 395) + 4.3 * states
+            if t < us:
+                best, us = C, t
+    return best if 1.05 * us < scan_us else None
 
 
 def scan_prefers_chunks(T: int, nseq: int, max_rows: int, heads: int, vdim: int, C: int) -> bool:
@@ -487,7 +499,7 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
     Long prompt portions run in chunks that are walked side by side, the same sums in another order, when that is expected to be faster (few long sequences;
     max_rows = the rows of the step's longest sequence when the caller knows it).  The modes with a constant decay per head (SCAN_FIXED, SCAN_FIXED_SILU):
     every chunk from a zero state, a prefix over each sequence's chunks, then the chunk-start states' share of the outputs (scan_prefers_chunks).
-    The gated modes: what every chunk leaves from a zero state and its total decays, the prefix, then the tokens again from the chunk-start states (walk_chunk).
+    The gated modes: what every chunk leaves from a zero state and its total decays, the prefix, then the tokens again from the chunk-start states (gated_form).
     plans: a dict that keeps the step's chunk plan between calls (the layers of one step share it); chunked forces the choice."""
     _dev(proj, torch.float32, "scan.proj"); _dev(state, torch.float32, "scan.state")
     T = proj.shape[0]
@@ -509,8 +521,8 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
                                               float(qscale), heads, dim, vdim, rs.data_ptr(), sl.data_ptr(), fp.data_ptr(), n, st.data_ptr(), _p(dst), _p(cdecay), keep,
                                               act_code(act), _stream()), "hy_walk")
 
-        C = walk_chunk(T, nseq, max_rows, heads, vdim)
-        if not C and nseq * heads * ((vdim + 127) // 128) < 192:                            # few blocks: the walk with more of them takes 0.33 us a token, not 0.41
+        C = gated_form(T, nseq, max_rows, heads, dim, vdim)
+        if C is None:
             run(mode, row_start, slot, first_pos, nseq, state)
             return out
         if not C:
