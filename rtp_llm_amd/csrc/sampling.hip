@@ -252,60 +252,57 @@ __device__ __forceinline__ float penalised(const PenaltyParams& p, int row, floa
     return logit;
 }
 
-// History of at most kShortHistory entries, one block per row: the entries lie in LDS, the first entry of an id counts its equals and penalises it.  No
-// [batch][V] counters to clear (39 MB at 64 rows of 152064, more than all the other work of the launch).
+// A history of at most kShortHistory entries is counted in LDS: a table of at least twice as many slots, hashed by the id, probed in line.  No [batch][V] counters to clear (39 MB at
+// 64 rows of 152064, more than all the other work of the launch), and no entry is compared with every other.
+// us with such comparisons / here / with counters in memory: 16 rows of 1627 entries 343 / 7.7 / 15, 1 row of 300 20 / 3.1 / 5.5, 64 rows of 256 11.5 / 5.7 / 12.4; in the joint
+// launches below 64 rows of 2000 253 / 32.
 constexpr int kShortHistory = 2048;
-__global__ __launch_bounds__(256) void penalties_short_kernel(const PenaltyParams p) {
-    __shared__ __attribute__((aligned(16))) int s_tok[kShortHistory];
-    const int row = blockIdx.x, tx = threadIdx.x;
-    float* x = p.logits + (size_t)row * p.ld;
+struct HistoryTable { int key[2 * kShortHistory], count[2 * kShortHistory]; };      // key -1: free
+
+// Penalises the history's ids in [lo, lo + n) once each, x = the row from lo on.  Whole block of NT threads; ends without a barrier.
+template <int NT>
+__device__ __forceinline__ void penalise_history(const PenaltyParams& p, HistoryTable& t, int row, int id_step, int id_row, int lo, int n, float* x) {
+    const int tx = threadIdx.x;
+    int bits = 6;
+    while ((1 << bits) < 2 * p.step) ++bits;
+    const int size = 1 << bits;
+    for (int i = tx; i < size; i += NT) { t.key[i] = -1; t.count[i] = 0; }
+    __threadfence_block();
+    __syncthreads();                                        // also: the row's scaling by other threads is done
     const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
-    const int padded = (p.step + 3) & ~3;
-    for (int i = tx; i < padded; i += 256) {
-        int tok = -1;                                       // nothing to penalise: padding, or an id outside the vocabulary
-        if (i < p.step && !(i >= input_length && i < p.max_input_length)) {
-            tok = p.output_ids[(size_t)i * p.batch + row];
-            if (tok >= p.V || tok < 0) tok = -1;
+    for (int i = tx; i < p.step; i += NT) {
+        if (i >= input_length && i < p.max_input_length) continue;                  // padding
+        const int tok = p.output_ids[(size_t)i * id_step + (size_t)row * id_row];
+        if (tok < lo || tok >= lo + n) continue;
+        int at = (int)(((uint32_t)tok * 2654435761u) >> (32 - bits));
+        for (int probe = 0; probe < size; ++probe) {        // ends: there are more slots than entries
+            const int was = atomicCAS(&t.key[at], -1, tok);
+            if (was == -1 || was == tok) { atomicAdd(&t.count[at], 1); break; }
+            at = (at + 1) & (size - 1);
         }
-        s_tok[i] = tok;
     }
     __syncthreads();
-    for (int i = tx; i < p.step; i += 256) {
-        const int tok = s_tok[i];
-        if (tok < 0) continue;
-        int count = 0, before = 0;
-        for (int j = 0; j < padded; j += 4) {
-            const int4 t = *reinterpret_cast<const int4*>(&s_tok[j]);
-            const int c = (t.x == tok) + (t.y == tok) + (t.z == tok) + (t.w == tok);
-            count += c;
-            if (j + 3 < i) before += c;
-            else before += (j < i && t.x == tok) + (j + 1 < i && t.y == tok) + (j + 2 < i && t.z == tok);
-        }
-        if (before == 0) x[tok] = penalised(p, row, x[tok], count);
+    for (int i = tx; i < size; i += NT) {
+        const int tok = t.key[i];
+        if (tok >= 0) x[tok - lo] = penalised(p, row, x[tok - lo], t.count[i]);
     }
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void penalties_short_kernel(const PenaltyParams p) {
+    __shared__ HistoryTable table;
+    penalise_history<NT>(p, table, blockIdx.x, p.batch, 1, 0, p.V, p.logits + (size_t)blockIdx.x * p.ld);
 }
 
 // Temperature, penalties and softmax of the sampler in two launches, every row split over blocks.  One block per row, the softmax alone took 36 us of 64 rows of 152064 (its
 // three passes at what one CU pulls), behind 14 of temperature and 14 of penalties; the two take 29 and 11.
-// Prepare: a block scales its slice, penalises the history's ids that lie in it (as penalties_short_kernel) and leaves the slice's maximum and sum of exponentials.
+// Prepare: a block scales its slice, penalises the history's ids that lie in it and leaves the slice's maximum and sum of exponentials.
 __global__ __launch_bounds__(kThreads) void sampling_prepare_kernel(const PenaltyParams p, float2* parts, int id_step, int id_row, int slice) {
-    __shared__ __attribute__((aligned(16))) int s_tok[kShortHistory];
+    __shared__ HistoryTable table;
     __shared__ float s_red[kThreads / 64];
     const int row = blockIdx.y, tx = threadIdx.x, lo = min(p.V, (int)blockIdx.x * slice), n = min(p.V, lo + slice) - lo;
     float* x = p.logits + (size_t)row * p.ld + lo;
     const bool vec = (p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;       // lo is a multiple of 4
-    const int padded = p.output_ids ? (p.step + 3) & ~3 : 0;
-    if (padded) {
-        const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
-        for (int i = tx; i < padded; i += kThreads) {
-            int tok = -1;                                   // nothing to penalise: padding, or an id outside the vocabulary
-            if (i < p.step && !(i >= input_length && i < p.max_input_length)) {
-                tok = p.output_ids[(size_t)i * id_step + (size_t)row * id_row];
-                if (tok >= p.V || tok < 0) tok = -1;
-            }
-            s_tok[i] = tok;
-        }
-    }
     if (p.temperature) {
         const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
         int done = 0;
@@ -321,25 +318,9 @@ __global__ __launch_bounds__(kThreads) void sampling_prepare_kernel(const Penalt
         }
         for (int j = done + tx; j < n; j += kThreads) x[j] *= inv_t;
     }
+    if (p.output_ids) penalise_history<kThreads>(p, table, row, id_step, id_row, lo, n, x);
     __threadfence_block();
     __syncthreads();
-    if (padded) {
-        for (int i = tx; i < p.step; i += kThreads) {
-            const int tok = s_tok[i];
-            if (tok < lo || tok >= lo + n) continue;
-            int count = 0, before = 0;
-            for (int j = 0; j < padded; j += 4) {
-                const int4 t = *reinterpret_cast<const int4*>(&s_tok[j]);
-                const int c = (t.x == tok) + (t.y == tok) + (t.z == tok) + (t.w == tok);
-                count += c;
-                if (j + 3 < i) before += c;
-                else before += (j < i && t.x == tok) + (j + 1 < i && t.y == tok) + (j + 2 < i && t.z == tok);
-            }
-            if (before == 0) x[tok - lo] = penalised(p, row, x[tok - lo], count);
-        }
-        __threadfence_block();
-        __syncthreads();
-    }
     float m = -3.0e38f;
     row_pass(x, n, vec, [&](float v) { m = fmaxf(m, v); });
     m = wave_max(m);
@@ -870,7 +851,8 @@ extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t 
         hipLaunchKernelGGL(penalties_kernel, dim3(batch_size), dim3(kThreads), 0, st, p);
         MI355_CHECK_LAUNCH("penalties_kernel");
     } else if (pen && step > 0) {
-        hipLaunchKernelGGL(penalties_short_kernel, dim3(batch_size), dim3(256), 0, st, p);
+        if (step <= 256) hipLaunchKernelGGL(penalties_short_kernel<256>, dim3(batch_size), dim3(256), 0, st, p);
+        else             hipLaunchKernelGGL(penalties_short_kernel<kThreads>, dim3(batch_size), dim3(kThreads), 0, st, p);
         MI355_CHECK_LAUNCH("penalties_short_kernel");
     }
     return MI355_OK;

@@ -4,6 +4,7 @@ from fractions import Fraction
 import pytest
 import torch
 
+from oracle import oracle
 from rtp_llm_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +48,26 @@ def test_more_than_65536_rows(V):
     assert bool(((got - full).abs() <= 2.0 ** -21 * (full.abs() + 2)).all())
     got = ops.sampling_probs(x.clone(), t, token_ids=ids, input_lengths=lens, max_input_length=2, step=2, **pen)
     assert bool(((got - full.double().softmax(-1)).abs() <= 2.0 ** -18).all())
+
+
+@pytest.mark.parametrize("step", [1, 31, 33, 700, 2048])
+@pytest.mark.parametrize("kind", ["one hash", "last hash", "few ids", "one id", "outside"])
+def test_history_counts(kind, step):
+    """Histories whose ids share a slot of the on-chip table (probing, also over its end), repeat, or lie outside the vocabulary; every id once, by its count, in both launches that count."""
+    V, B = 40000, 3
+    bits = max(6, (2 * step - 1).bit_length())
+    g = torch.Generator().manual_seed(step)
+    ids = torch.arange(V, dtype=torch.int64)
+    slot = (ids * 2654435761 % 2 ** 32) >> (32 - bits)
+    pool = {"one hash": ids[slot == slot[77]], "last hash": ids[slot >= (1 << bits) - 2], "few ids": ids[5:12], "one id": ids[9:10], "outside": torch.tensor([-1, -7, 3, V, V + 9, 2 ** 31 - 1])}[kind]
+    hist = pool[torch.randint(0, pool.numel(), (step, B), generator=g)].int()
+    x = torch.randn(B, V, generator=g) * 3
+    pen = dict(repetition_penalty=torch.tensor([1.0, 1.3, 0.7]), presence_penalty=torch.tensor([0.5, 0.0, 0.25]), frequency_penalty=torch.tensor([0.125, 0.5, 0.0]))
+    lens = torch.full((B,), step, dtype=torch.int32)
+    want = oracle.apply_penalties(x, output_ids=hist, input_lengths=lens, max_input_length=step, step=step, **pen)
+    got = ops.apply_penalties(x.clone().to(DEV), output_ids=hist.to(DEV), input_lengths=lens, max_input_length=step, step=step, **pen)
+    assert torch.equal(got.cpu(), want)
+    dev = {k: v.to(DEV) for k, v in pen.items()}
+    got = ops.sampling_probs(x.clone().to(DEV), token_ids=hist.t().contiguous().to(DEV), input_lengths=lens.to(DEV), max_input_length=step, step=step, **dev)
+    soft = want.double().softmax(-1)            # exp2 of an argument rounded to 24 bits, |x - max| < 40 where the result counts: 40 * 2^-24 = 2.4e-6, and the sum
+    assert bool(((got.cpu() - soft).abs() <= 5e-6 * soft + 1e-12).all())
