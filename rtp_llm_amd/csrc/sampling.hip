@@ -225,9 +225,10 @@ struct PenaltyParams {
     int32_t*       counts;         // [batch][V]: histories of more than kShortHistory entries
 };
 
-// Temperature alone: blockIdx.x splits the row.  64 rows of 152064: 14 us, the copy rate of their 78 MB.
+// Temperature alone: blockIdx.x splits the row.
+template <bool WHOLE>
 __global__ __launch_bounds__(kThreads) void temperature_kernel(const PenaltyParams p) {
-    const int row = blockIdx.y, start = blockIdx.x * kThreads + threadIdx.x, stride = gridDim.x * kThreads;
+    const int row = WHOLE ? blockIdx.x : blockIdx.y, start = (WHOLE ? 0 : blockIdx.x * kThreads) + threadIdx.x, stride = WHOLE ? kThreads : gridDim.x * kThreads;
     float* x = p.logits + (size_t)row * p.ld;
     const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
     int done = 0;
@@ -826,6 +827,20 @@ extern "C" int mi355_rejection_sample(const float* draft_probs, const int32_t* d
     return MI355_OK;
 }
 
+// Blocks of a row: about one block per compute unit in all, none with less than a pass of its threads.  Temperature alone, us with 1 / 2 / 4 / 8 / 16 blocks a row:
+// 1 x 152064 11.9 / 6.6 / 4.3 / 3.2 / 2.7, 64 x 152064 18.3 / 12.5 / 11.6 / 12.2 / 12.4, 64 x 6952 2.8 / 2.8 / 2.9 / 3.6 / 4.5, 237 x 32000 8.3 / 8.2 / 8.8 / 9.6 / 13.1.
+constexpr int kMostSplits = 16;
+static int row_splits(int rows, int V) {
+    const int most = rows >= 256 ? 1 : 256 / rows < kMostSplits ? 256 / rows : kMostSplits, full = (V + 4 * kThreads - 1) / (4 * kThreads);
+    return most < full ? most : full;
+}
+// The joint launches walk a slice three times: of long rows more blocks, so that a slice of 64 KB stays near its compute unit.  Us with row_splits / these: 64 x 152064 31.7 / 28.1,
+// 237 x 152064 127.5 / 97.8; 237 x 32000 21.7 / 30.0 with 8 blocks a row, 237 x 1695 7.2 / 20.7.
+static int joint_splits(int rows, int V) {
+    const int least = row_splits(rows, V), near = V / 16384 < kMostSplits ? V / 16384 : kMostSplits;
+    return least > near ? least : near;
+}
+
 extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t V, int32_t ld, const float* temperature,
                                      const float* repetition_penalty, const float* presence_penalty, const float* frequency_penalty,
                                      const int32_t* output_ids, const int32_t* input_lengths, int32_t max_input_length,
@@ -840,8 +855,9 @@ extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t 
                     pen ? output_ids : nullptr, input_lengths, batch_size, max_input_length, step, penalty_ws};
     hipStream_t st = (hipStream_t)stream;
     if (temperature) {
-        const int split = batch_size >= 256 ? 1 : batch_size >= 32 ? 8 : 16;
-        hipLaunchKernelGGL(temperature_kernel, dim3(split, batch_size), dim3(kThreads), 0, st, p);
+        const int split = row_splits(batch_size, V);
+        if (split > 1) hipLaunchKernelGGL(temperature_kernel<false>, dim3(split, batch_size), dim3(kThreads), 0, st, p);
+        else           hipLaunchKernelGGL(temperature_kernel<true>, dim3(batch_size), dim3(kThreads), 0, st, p);
         MI355_CHECK_LAUNCH("temperature_kernel");
     }
     if (pen && step > kShortHistory) {
@@ -858,10 +874,7 @@ extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t 
     return MI355_OK;
 }
 
-// splits of a row: enough blocks for the chip, no more than kSamplingSplits
-static int sampling_splits(int rows) { return rows >= 256 ? 1 : rows >= 32 ? 8 : 16; }
-
-extern "C" size_t mi355_sampling_probs_workspace_bytes(int32_t rows) { return rows > 0 ? (size_t)rows * sampling_splits(rows) * sizeof(float2) : 0; }
+extern "C" size_t mi355_sampling_probs_workspace_bytes(int32_t rows) { return rows > 0 ? (size_t)rows * kMostSplits * sizeof(float2) : 0; }
 
 extern "C" int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
                                     const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
@@ -869,7 +882,7 @@ extern "C" int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int3
     MI355_CHECK_ARG(logits && workspace && rows > 0 && V > 0 && ld >= V && step >= 0 && (uintptr_t)workspace % 8 == 0, "sampling_probs: bad args");
     if (output_ids && step > kShortHistory) return MI355_ERR_UNSUPPORTED;      // apply_penalties counts those in memory
     const bool pen = output_ids && step > 0 && (repetition || presence || frequency);
-    const int S = sampling_splits(rows), slice = ((V + S - 1) / S + 3) & ~3;
+    const int S = joint_splits(rows, V), slice = ((V + S - 1) / S + 3) & ~3;
     const PenaltyParams p{logits, V, ld, temperature, repetition, presence, frequency, pen ? output_ids : nullptr, input_lengths, rows, max_input_length, step, nullptr};
     hipLaunchKernelGGL(sampling_prepare_kernel, dim3(S, rows), dim3(kThreads), 0, (hipStream_t)stream, p, (float2*)workspace, id_step, id_row, slice);
     MI355_CHECK_LAUNCH("sampling_prepare_kernel");
