@@ -407,9 +407,10 @@ __global__ __launch_bounds__(kThreads) void penalties_kernel(const PenaltyParams
 // two thresholds took 31 passes of 24 us over 152064 values on one CU.  A histogram of the pattern's top 12 bits (a sixteenth of an octave per bin) with the
 // count and the mass of every bin names the one bin each threshold lies in; the values of those two bins go to LDS and the low 19 bits are searched there.  The
 // values of a bin share their exponent, so its mass is a sum of integers, exact whatever the order of the atomics, and packs with the count into one 64-bit
-// word: one LDS atomic a value.  The draw reads the row twice more, a wave per contiguous sixteenth.  Rows whose boundary bin holds more than kSet values (flat
-// rows, long runs of one value) are searched bit by bit as before.
-// 64 rows of 152064, top-k 0..100, top-p 0.8..0.95 of a distribution with a heavy tail: 827 -> 97 us.
+// word: one LDS atomic a value.  The draw reads the row twice more, a wave per contiguous sixteenth.  Where a bin holds more than kSet values (flat rows), a second
+// histogram of it gives the next 12 bits; runs of more than kSet equal values are searched bit by bit over the row for the
+// last 7.  Infinities, p < 0 and rows of more than 2^20 values are searched bit by bit as a whole.
+// 64 rows of 152064, top-k 0..100, top-p 0.8..0.95 of a distribution with a heavy tail: 827 -> 97 us; flat ones (softmax of logits of deviation 0.5) 508 -> 134.
 struct TopKPParams {
     const float*   probs;
     int            V, ld;
@@ -423,19 +424,23 @@ struct TopKPParams {
 
 constexpr int kSet = 4096, kBinShift = 19, kBins = 1 << (31 - kBinShift), kWaves = kThreads / 64;
 
-struct DrawShared { float red[kWaves]; int found; };
+// (16-byte aligned, so that a wave reads the sixteen waves' results 16 bytes at a time: 31 against 38 us for a row of 1001)
+#define ALIGN16 __attribute__((aligned(16)))
+struct DrawShared { ALIGN16 float red[kWaves]; int found; };
 struct SampleShared : DrawShared {
-    float    pair[kWaves][2];
-    float    scan[kThreads];
-    unsigned long long hist[kBins];          // count << 40 | sum of the low 19 bits
-    uint32_t set_k[kSet], set_q[kSet];
+    ALIGN16 float    pair[kWaves][2];
+    ALIGN16 float    scan[kThreads];
+    ALIGN16 unsigned long long hist[kBins];  // count << 40 | sum of the bits below the bin's
+    ALIGN16 uint32_t set_k[kSet];
+    ALIGN16 uint32_t set_q[kSet];
+    ALIGN16 uint32_t wave_n[kWaves];
+    ALIGN16 unsigned long long wave_m[kWaves];
+    ALIGN16 double   wave_d[kWaves];
     int      n_k, n_q, bin_k, bin_q;
     uint32_t above_k;                        // entries in the bins above bin_k
     double   above_q;                        // mass in the bins above bin_q
-    uint32_t wave_n[kWaves];
-    unsigned long long wave_m[kWaves];
-    double   wave_d[kWaves];
 };
+#undef ALIGN16
 
 __device__ __forceinline__ float sample_pos(float v) { return v > 0.f ? v : 0.f; }   // +0 for -0, negatives and NaN: the bit pattern is the order
 
@@ -568,130 +573,191 @@ __device__ __forceinline__ void filter_and_draw(const float* q, int V, uint32_t 
 __device__ __forceinline__ int search_histogram(const float* q, int V, bool vec, bool use_k, int k, bool& use_p, float tp, uint32_t& kb, uint32_t& vbits,
                                                 SampleShared& sh) {
     const int tx = threadIdx.x, lane = tx & 63, wave = tx >> 6;
-    constexpr uint32_t LOW = (1u << kBinShift) - 1u;
     if (V > (1 << 20) || (use_p && tp < 0.f)) return 0;                         // the packed sums hold 2^21 values
-    for (int i = tx; i < kBins; i += kThreads) sh.hist[i] = 0ull;
-    if (tx == 0) { sh.n_k = sh.n_q = 0; sh.bin_k = sh.bin_q = -1; }
-    __syncthreads();
-    row_pass(q, V, vec, [&](float x) {
-        const uint32_t b = __float_as_uint(sample_pos(x));
-        if (b != 0u) atomicAdd(&sh.hist[b >> kBinShift], (1ull << 40) + (unsigned long long)(b & LOW));
-    });
-    __syncthreads();
-    // from the largest values down: a thread takes kBins / kThreads bins, prefixes over the lanes and the waves
-    constexpr int PB = kBins / kThreads;
-    uint32_t c[PB], ci = 0;
-    double m[PB], mi = 0.0;
+    auto bits_of = [](float x) { return __float_as_uint(sample_pos(x)); };
+    // the values above zero whose bits from `up` on are `top`, by their bits [shift, up)
+    auto count = [&](int shift, int up, uint32_t top) {
+        for (int i = tx; i < kBins; i += kThreads) sh.hist[i] = 0ull;
+        if (tx == 0) { sh.bin_k = sh.bin_q = -1; sh.n_k = sh.n_q = 0; }
+        __syncthreads();
+        const uint32_t low = (1u << shift) - 1u;
+        row_pass(q, V, vec, [&](float x) {
+            const uint32_t b = bits_of(x);
+            if (b != 0u && b >> up == top) atomicAdd(&sh.hist[b >> shift & (kBins - 1)], (1ull << 40) + (unsigned long long)(b & low));
+        });
+        __syncthreads();
+    };
+    // The bins that hold the k-th largest value (sh.bin_k) and the crossing of p (sh.bin_q), c0 values and m0 mass above the histogram: from the largest values down, a thread takes
+    // kBins / kThreads bins, prefixes over the lanes and the waves.  Returns the histogram's mass.
+    auto locate = [&](int shift, uint32_t base, bool want_k, uint32_t c0, bool want_p, double m0, bool only_above_p) {
+        constexpr int PB = kBins / kThreads;
+        uint32_t c[PB], ci = 0;
+        double m[PB], mi = 0.0;
 #pragma unroll
-    for (int i = 0; i < PB; ++i) {
-        const int bin = kBins - 1 - (tx * PB + i), e = bin >> (23 - kBinShift);
-        const unsigned long long h = sh.hist[bin];
-        c[i] = (uint32_t)(h >> 40);
-        m[i] = (double)c[i] * (double)__uint_as_float((uint32_t)bin << kBinShift) + (double)(h & ((1ull << 40) - 1ull)) * __builtin_ldexp(1.0, (e ? e : 1) - 150);
-        if (c[i] == 0u) m[i] = 0.0;
-        if (bin >= (0x7F800000 >> kBinShift) && c[i]) sh.bin_k = -2;            // an infinity
-        ci += c[i]; mi += m[i];
-    }
-    const uint32_t c_own = ci;
+        for (int i = 0; i < PB; ++i) {
+            const uint32_t bin = kBins - 1 - (tx * PB + i), at = base | bin << shift, e = at >> 23;
+            const unsigned long long h = sh.hist[bin], mant = (at & 0x7FFFFFu) | (e ? 0x800000u : 0u);
+            c[i] = (uint32_t)(h >> 40);
+            m[i] = (double)(c[i] * mant + (h & ((1ull << 40) - 1ull))) * __builtin_ldexp(1.0, (int)(e ? e : 1) - 150);
+            if (at >= 0x7F800000u) { if (c[i]) sh.bin_k = -2; m[i] = 0.0; }         // an infinity
+            ci += c[i]; mi += m[i];
+        }
+        const uint32_t c_own = ci;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t yc = __shfl_up(ci, o);
-        const double ym = __shfl_up(mi, o);
-        if (lane >= o) { ci += yc; mi += ym; }
-    }
-    if (lane == 63) { sh.wave_n[wave] = ci; sh.wave_d[wave] = mi; }
-    __syncthreads();
-    if (sh.bin_k == -2) return 0;
-    uint32_t c_at = ci - c_own;
-    double m_at = 0.0, total = 0.0;
-    for (int w = 0; w < kWaves; ++w) {
-        if (w < wave) c_at += sh.wave_n[w];
-        if (w == wave) m_at = total;
-        total += sh.wave_d[w];
-    }
-    const double m_lane = __shfl_up(mi, 1);
-    if (lane > 0) m_at += m_lane;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t yc = __shfl_up(ci, o);
+            const double ym = __shfl_up(mi, o);
+            if (lane >= o) { ci += yc; mi += ym; }
+        }
+        if (lane == 63) { sh.wave_n[wave] = ci; sh.wave_d[wave] = mi; }
+        __syncthreads();
+        if (sh.bin_k == -2) return -1.0;
+        uint32_t c_at = c0 + ci - c_own;
+        double m_at = 0.0, total = 0.0;
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) c_at += sh.wave_n[w];
+            if (w == wave) m_at = total;
+            total += sh.wave_d[w];
+        }
+        const double m_lane = __shfl_up(mi, 1);
+        if (lane > 0) m_at += m_lane;
+        m_at += m0;
+        if (only_above_p) want_p = want_p && total > (double)tp;
+        // The prefix up to a thread's bins and the sum over the bins of the thread before it round differently: both may see p crossed.  The larger values' bin has it, with the sum
+        // of the thread that it belongs to.
+        int mine_q = -1;
+        double mine_above = 0.0;
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+            const int bin = kBins - 1 - (tx * PB + i);
+            if (want_k && c_at < (uint32_t)k && c_at + c[i] >= (uint32_t)k) { sh.bin_k = bin; sh.above_k = c_at; }
+            if (want_p && m_at <= (double)tp && m_at + m[i] > (double)tp) { mine_q = bin; mine_above = m_at; }
+            c_at += c[i]; m_at += m[i];
+        }
+        if (mine_q >= 0) atomicMax(&sh.bin_q, mine_q);
+        __syncthreads();
+        if (mine_q >= 0 && mine_q == sh.bin_q) sh.above_q = mine_above;             // to be read behind another barrier
+        return total;
+    };
+    count(kBinShift, 31, 0);
+    const double total = locate(kBinShift, 0, use_k, 0, use_p, 0.0, true);
+    if (total < 0.0) return 0;
     if (use_p) use_p = total > (double)tp;                                      // nothing to drop when even the mass above 0 fits
-    // The prefix up to a thread's bins and the sum over the bins of the thread before it round differently: both may see p crossed.  The larger values' bin has it, with the sum
-    // of the thread that it belongs to.
-    int mine_q = -1;
-    double mine_above = 0.0;
-#pragma unroll
-    for (int i = 0; i < PB; ++i) {
-        const int bin = kBins - 1 - (tx * PB + i);
-        if (use_k && c_at < (uint32_t)k && c_at + c[i] >= (uint32_t)k) { sh.bin_k = bin; sh.above_k = c_at; }
-        if (use_p && m_at <= (double)tp && m_at + m[i] > (double)tp) { mine_q = bin; mine_above = m_at; }
-        c_at += c[i]; m_at += m[i];
-    }
-    if (mine_q >= 0) atomicMax(&sh.bin_q, mine_q);
-    __syncthreads();
-    if (mine_q >= 0 && mine_q == sh.bin_q) sh.above_q = mine_above;             // read behind the candidates' barrier
     const int bin_k = use_k ? sh.bin_k : -1, bin_q = use_p ? sh.bin_q : -1;     // bin_k -1: fewer than k entries are above zero
     if (use_p && bin_q < 0) return 0;                                           // the sums crossed p between a thread's last bin and the next thread's first
     kb = 0; vbits = 0;
     if (bin_k < 0 && bin_q < 0) return 1;
-    row_pass(q, V, vec, [&](float x) {
-        const uint32_t b = __float_as_uint(sample_pos(x));
-        const int bin = (int)(b >> kBinShift);
-        if (b == 0u) return;
-        if (bin == bin_k) { const int at = atomicAdd(&sh.n_k, 1); if (at < kSet) sh.set_k[at] = b; }
-        if (bin == bin_q) { const int at = atomicAdd(&sh.n_q, 1); if (at < kSet) sh.set_q[at] = b; }
-    });
-    __syncthreads();
+    int left_k = kBinShift, left_q = kBinShift;                                 // bits of the thresholds that are not known
+    if (bin_k >= 0) kb = (uint32_t)bin_k << kBinShift; else left_k = 0;
+    if (bin_q >= 0) vbits = (uint32_t)bin_q << kBinShift; else left_q = 0;
+    auto in_k = [&](uint32_t b) { return bin_k >= 0 && b != 0u && b >> left_k == kb >> left_k; };
+    auto in_q = [&](uint32_t b) { return bin_q >= 0 && b != 0u && b >> left_q == vbits >> left_q; };
+    auto gather = [&]() {                                                       // the values that share a threshold's known bits
+        row_pass(q, V, vec, [&](float x) {
+            const uint32_t b = bits_of(x);
+            if (in_k(b)) { const int at = atomicAdd(&sh.n_k, 1); if (at < kSet) sh.set_k[at] = b; }
+            if (in_q(b)) { const int at = atomicAdd(&sh.n_q, 1); if (at < kSet) sh.set_q[at] = b; }
+        });
+        __syncthreads();
+    };
+    gather();
+    uint32_t above_k = sh.above_k;
+    double above_q = sh.above_q;
+    if (sh.n_k > kSet || sh.n_q > kSet) {                                       // flat rows: the next 12 bits from a histogram of the bin
+        const bool again_k = sh.n_k > kSet, again_q = sh.n_q > kSet;
+        constexpr int REST = kBinShift - 12;
+        __syncthreads();                                                        // the counts have been read
+        if (again_k) {
+            count(REST, kBinShift, (uint32_t)bin_k);
+            locate(REST, kb, true, above_k, false, 0.0, false);
+            kb |= (uint32_t)sh.bin_k << REST; above_k = sh.above_k; left_k = REST;
+        }
+        if (again_q) {
+            __syncthreads();                                                    // bin_k has been read
+            count(REST, kBinShift, (uint32_t)bin_q);
+            locate(REST, vbits, false, 0, true, above_q, false);
+            if (sh.bin_q < 0) return 0;                                         // rounding took the crossing out of the bin
+            __syncthreads();
+            vbits |= (uint32_t)sh.bin_q << REST; above_q = sh.above_q; left_q = REST;
+        }
+        __syncthreads();
+        gather();
+    }
     const int n_k = sh.n_k, n_q = sh.n_q;
-    if (n_k > kSet || n_q > kSet) return 0;
-    // low bits, most significant first: the largest threshold that leaves k entries (more mass than p) at or above it.  The sets lie in registers.
-    constexpr int PT = kSet / kThreads;
-    const int e_q = max(bin_q, 0) >> (23 - kBinShift);
+    const bool whole = n_k > kSet || n_q > kSet;                                // long runs of one value: the last bits from the row
+    const int e_q = (int)(vbits >> 23);
     const uint32_t implicit = e_q ? 0x800000u : 0u;
     const double unit = __builtin_ldexp(1.0, (e_q ? e_q : 1) - 150);
-    uint32_t vk[PT], vq[PT];
-#pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        const int j = tx + i * kThreads;
-        vk[i] = j < n_k ? sh.set_k[j] : 0u;
-        vq[i] = j < n_q ? sh.set_q[j] : 0u;
-    }
     auto mantissa = [&](uint32_t b) { return (unsigned long long)((b & 0x7FFFFFu) | implicit); };
-    if (bin_k >= 0) kb = (uint32_t)bin_k << kBinShift;
-    if (bin_q >= 0) vbits = (uint32_t)bin_q << kBinShift;
-    const uint32_t above_k = sh.above_k;
-    const double above_q = sh.above_q;
-    for (int bit = kBinShift - 1; bit >= 0; --bit) {
-        const uint32_t ck = kb | (1u << bit), cq = vbits | (1u << bit);
-        uint32_t cnt = 0;
-        unsigned long long mass = 0;
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-            cnt += (uint32_t)__popcll(__ballot(vk[i] >= ck));
-            if (vq[i] >= cq) mass += mantissa(vq[i]);
-        }
+    auto over_waves = [&](uint32_t& cnt, unsigned long long& mass) {            // of every wave's sums
         if (bin_q >= 0) mass = wave_sum_u64(mass);
         if (lane == 0) { sh.wave_n[wave] = cnt; sh.wave_m[wave] = mass; }
         __syncthreads();
-        cnt = above_k; mass = 0;
+        cnt = 0; mass = 0;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) { cnt += sh.wave_n[w]; mass += sh.wave_m[w]; }
         __syncthreads();
-        if (bin_k >= 0 && cnt >= (uint32_t)k) kb = ck;
-        if (bin_q >= 0 && above_q + (double)mass * unit > (double)tp) vbits = cq;
-    }
-    if (bin_q < 0) return 1;
-    // equals of the boundary value: the j-th of T stays while S + j v <= p, S = the mass above it
+    };
+    // the rest, most significant bit first: the largest threshold that leaves k entries (more mass than p) at or above it
     uint32_t ties = 0;
     unsigned long long mass = 0;
+    if (!whole) {                                                               // the sets lie in registers
+        constexpr int PT = kSet / kThreads;
+        uint32_t vk[PT], vq[PT];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-        ties += (uint32_t)__popcll(__ballot(vq[i] == vbits && vq[i] != 0u));
-        if (vq[i] > vbits) mass += mantissa(vq[i]);
+        for (int i = 0; i < PT; ++i) {
+            const int j = tx + i * kThreads;
+            vk[i] = j < n_k ? sh.set_k[j] : 0u;
+            vq[i] = j < n_q ? sh.set_q[j] : 0u;
+        }
+        for (int bit = max(left_k, left_q) - 1; bit >= 0; --bit) {
+            const uint32_t ck = kb | (1u << bit), cq = vbits | (1u << bit);
+            uint32_t cnt = 0;
+            mass = 0;
+#pragma unroll
+            for (int i = 0; i < PT; ++i) {
+                cnt += (uint32_t)__popcll(__ballot(vk[i] >= ck));
+                if (vq[i] >= cq) mass += mantissa(vq[i]);
+            }
+            over_waves(cnt, mass);
+            if (bin_k >= 0 && bit < left_k && above_k + cnt >= (uint32_t)k) kb = ck;
+            if (bin_q >= 0 && bit < left_q && above_q + (double)mass * unit > (double)tp) vbits = cq;
+        }
+        if (bin_q < 0) return 1;
+        mass = 0;
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+            ties += (uint32_t)__popcll(__ballot(vq[i] == vbits && vq[i] != 0u));
+            if (vq[i] > vbits) mass += mantissa(vq[i]);
+        }
+        over_waves(ties, mass);
+    } else {
+        const uint32_t top_k = bin_k >= 0 ? kb >> left_k : ~0u, top_q = bin_q >= 0 ? vbits >> left_q : ~0u;
+        for (int bit = max(left_k, left_q) - 1; bit >= 0; --bit) {
+            const uint32_t ck = kb | (1u << bit), cq = vbits | (1u << bit);
+            uint32_t cnt = 0;
+            mass = 0;
+            row_pass(q, V, vec, [&](float x) {
+                const uint32_t b = bits_of(x);
+                if (b >> left_k == top_k && b >= ck) ++cnt;
+                if (b >> left_q == top_q && b >= cq) mass += mantissa(b);
+            });
+            cnt = (uint32_t)wave_sum_u64(cnt);
+            over_waves(cnt, mass);
+            if (bin_k >= 0 && bit < left_k && above_k + cnt >= (uint32_t)k) kb = ck;
+            if (bin_q >= 0 && bit < left_q && above_q + (double)mass * unit > (double)tp) vbits = cq;
+        }
+        if (bin_q < 0) return 1;
+        mass = 0;
+        row_pass(q, V, vec, [&](float x) {
+            const uint32_t b = bits_of(x);
+            if (b == vbits && b != 0u) ++ties;
+            if (b >> left_q == top_q && b > vbits) mass += mantissa(b);
+        });
+        ties = (uint32_t)wave_sum_u64(ties);
+        over_waves(ties, mass);
     }
-    mass = wave_sum_u64(mass);
-    if (lane == 0) { sh.wave_n[wave] = ties; sh.wave_m[wave] = mass; }
-    __syncthreads();
-    ties = 0; mass = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) { ties += sh.wave_n[w]; mass += sh.wave_m[w]; }
-    __syncthreads();
+    // equals of the boundary value: the j-th of T stays while S + j v <= p, S = the mass above it
     return ties <= 1u || above_q + (double)(mass + (unsigned long long)(ties - 1u) * mantissa(vbits)) * unit <= (double)tp ? 1 : 2;
 }
 

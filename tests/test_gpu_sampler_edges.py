@@ -71,3 +71,50 @@ def test_history_counts(kind, step):
     got = ops.sampling_probs(x.clone().to(DEV), token_ids=hist.t().contiguous().to(DEV), input_lengths=lens.to(DEV), max_input_length=step, step=step, **dev)
     soft = want.double().softmax(-1)            # exp2 of an argument rounded to 24 bits, |x - max| < 40 where the result counts: 40 * 2^-24 = 2.4e-6, and the sum
     assert bool(((got.cpu() - soft).abs() <= 5e-6 * soft + 1e-12).all())
+
+
+@pytest.mark.parametrize("V", [700, 5001, 70001, 152064])
+@pytest.mark.parametrize("kind", ["flat", "crowded k", "crowded p", "one value", "two values"])
+def test_rows_with_more_values_in_a_bin_than_the_sets_hold(V, kind):
+    """Multiples of 2^-34 inside one or two bins, and runs of one value: the first histogram, the second one of a bin, and the last bits over the row.  Kept sets against exact integers (the masses are
+    sums of integers below 2^53)."""
+    g = torch.Generator().manual_seed(V)
+    n = min(V, 60000)
+    if kind in ("flat", "crowded k", "crowded p"):
+        # 2^18 units of 2^-34 = 2^-16 and up to 2^14 units more: a sixteenth of an octave is one bin
+        units = (torch.randperm(16384, generator=g).repeat(4)[:n] if n > 16384 else torch.randperm(16384, generator=g)[:n]).long() + 262144
+        if kind == "crowded k":
+            units[: n // 2] = units[: n // 2] * 32 + 7
+        elif kind == "crowded p":
+            units[: n // 50] = units[: n // 50] * 32 + 3
+    else:
+        units = torch.full((n,), 262144 + 777, dtype=torch.long)
+        if kind == "two values":
+            units[::3] = 262144 + 778
+    at = torch.randperm(V, generator=g)[:n]
+    R = 4
+    value = torch.zeros(V, dtype=torch.long)
+    value[at] = units
+    probs = (value.double() * 2.0 ** -34).float()[None].repeat(R, 1)
+    assert torch.equal((probs[0].double() * 2.0 ** 34).long(), value)
+    order = torch.argsort(value, descending=True, stable=True)
+    before = value[order].cumsum(0) - value[order]                       # mass in front of each entry, in units
+    top_k = torch.tensor([0, n // 3, n - 1, 5], dtype=torch.int32)
+    want = torch.zeros(R, V, dtype=torch.bool)
+    top_p = torch.empty(R)
+    for r, share in enumerate((0.4, 1.0, 0.9, 0.97)):
+        top_p[r] = 1.0 if share == 1.0 else float(torch.tensor(float(before[int(share * n)]) * 2.0 ** -34).float())
+        keep = torch.ones(V, dtype=torch.bool)
+        if 0 < int(top_k[r]) < V:
+            keep &= value >= value[order[int(top_k[r]) - 1]]
+        if share != 1.0:
+            limit = int(round(float(top_p[r].double()) * 2 ** 34))
+            inside = torch.zeros(V, dtype=torch.bool)
+            inside[order[before <= limit]] = True
+            keep &= inside
+        want[r] = keep & (value > 0) if bool((value[keep] > 0).any()) else keep
+    ids, out = ops.top_k_top_p_sample(probs.to(DEV), top_k, top_p, torch.tensor([0.0, 0.3, 0.6, 0.95]).to(DEV), return_probs=True)
+    got = out.cpu() > 0
+    # where equals of the border value go, the index from which they do is found from fp32 sums: their rounding (20 steps of 2^-24 of a mass of 1 to 16) is below an entry (2^-16 and up, 2^-11 there)
+    assert int((got != want).sum(-1).max()) <= 1
+    assert bool(got[torch.arange(R), ids.cpu().long()].all())
