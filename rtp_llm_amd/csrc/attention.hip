@@ -94,7 +94,9 @@ __device__ __forceinline__ f16x8 widen_kv8(uint32_t lo, uint32_t hi) {
 // BF: Q, a 16-bit cache and the output are bf16 (kv_dtype MI355_KV_BF16): bf16 MFMAs for S = K q^T and O = V^T P, P rounded to
 // bf16.  The INT8 cache serves both activation dtypes: its bytes are widened to fp16 (widen_kv8, bias 1152) or to bf16
 // (widen_u8_bf16, bias 128).
-template <int HD, bool INT8, int NT, int NW, int NG, bool BF = false>
+// MERGE (p.done): the block that is done last merges the partitions' parts.  RAGGED (p.row_start): rows without padding between.  Instances of their own: with both as run-time cases
+// a small call of prompt rows took 3 to 5 % longer.
+template <int HD, bool INT8, int NT, int NW, int NG, bool BF, bool MERGE, bool RAGGED>
 __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p) {
     constexpr float KVB = BF ? 128.f : 1152.f;     // INT8: what a widened cache byte carries on top of its code (see widen_kv8 / _bf16)
     constexpr int NTHR = 64 * NW, GS = 32 * NW;    // threads; tokens one round of the block's waves covers
@@ -104,9 +106,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     const int b = blockIdx.z / p.ntile, tile = blockIdx.z - b * p.ntile;
     const int RT = NT * p.R;                       // query rows of this block
     int base = b * p.q_len, len = p.q_len;
-    if constexpr (NT == 2) {
-        if (p.row_start) { base = p.row_start[b]; len = p.row_start[b + 1] - base; if (tile * RT >= len) return; }
-    }
+    if constexpr (RAGGED) { base = p.row_start[b]; len = p.row_start[b + 1] - base; if (tile * RT >= len) return; }
     const int row0 = base + tile * RT;             // first row (index into q / positions / out)
     const int nrows = min(RT, len - tile * RT);
     // context of a row = its position + 1 (seq_add = 1: positions hold tokens already cached) or seq_lens[row] itself;
@@ -139,8 +139,8 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     }
     if (pstart >= seq_len) return;
     const int pend = min(seq_len, pstart + p.PS);
-    // partitions of this tile that write (1: the outputs themselves; without `done` attn_reduce_kernel merges whatever their number)
-    const int nparts = p.P == 1 ? 1 : p.done ? (seq_len + p.PS - 1) / p.PS : p.P;
+    // partitions of this tile that write (1: the outputs themselves; without MERGE attn_reduce_kernel merges whatever their number)
+    const int nparts = MERGE ? (seq_len + p.PS - 1) / p.PS : p.P;
     auto store_out = [&](int row, int col, const f32x4& acc, float l) {
         const float inv = l > 0.f ? 1.f / l : 0.f;                  // padding row / empty context: zeros, not NaN
         u32x2 ov;
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
                 store_out(row, h * HD + d0, acc, l);
             } else {
                 const size_t slot = ((size_t)row * p.nh + h) * p.P + part;
-                if (p.done) {      // seen by the other XCDs without a write-back of the whole L2 (a release fence: 3 to 13 us here)
+                if (MERGE) {       // seen by the other XCDs without a write-back of the whole L2 (a release fence: 3 to 13 us here)
                     put2(p.tmp_out + slot * HD + d0, acc[0], acc[1]);
                     put2(p.tmp_out + slot * HD + d0 + 2, acc[2], acc[3]);
                     if (d0 == 0) put2(p.tmp_ml + slot * 2, mstar, l);
@@ -558,7 +558,8 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
         }
     }
     AT_STAMP(5);
-    if (!p.done || nparts == 1) return;
+    if constexpr (MERGE) {
+    if (nparts == 1) return;
     // The partition that is done last merges: its own launch (attn_reduce_kernel) costs 3 to 5 us behind an attention of 4 to 6 at one sequence.  Every thread's part is
     // written through to where the other XCDs see it before the block counts itself; the last block sees all counts, then reads all parts from there.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's part has arrived
@@ -628,6 +629,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     else if (nparts <= 16 && nrows * p.G * (HD / 4) <= 64 * NW / 2) merge(std::integral_constant<int, 8>{}, std::true_type{});
     else merge(std::integral_constant<int, 16>{}, std::true_type{});
     if (tid == 0) __hip_atomic_store(p.done + ((size_t)blockIdx.z * p.nkv + kh) * p.done_step, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ prompt rows (16-bit cache)
@@ -963,7 +965,10 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     p.tmp_ml  = p.tmp_out + rows * nh * p.P * kv->hd;
     hipStream_t st = (hipStream_t)stream;
     dim3 grid(p.P, kv->nkv, B * p.ntile);
-#define L_(HD_, I8_, NT_, NW_, NG_) hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, NT_, NW_, NG_>), grid, dim3(64 * NW_), 0, st, p)
+#define LI_(HD_, I8_, NT_, NW_, NG_, BF_, M_, R_) hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, NT_, NW_, NG_, BF_, M_, R_>), grid, dim3(64 * NW_), 0, st, p)
+#define LM_(HD_, I8_, NT_, NW_, NG_, BF_) do { if (p.done) LI_(HD_, I8_, NT_, NW_, NG_, BF_, true, false); else if (row_start) LI_(HD_, I8_, 2, NW_, 2, BF_, false, true); \
+                                              else LI_(HD_, I8_, NT_, NW_, NG_, BF_, false, false); } while (0)
+#define L_(HD_, I8_, NT_, NW_, NG_) LM_(HD_, I8_, NT_, NW_, NG_, false)
 #ifdef MI355_TUNING
 #define L2_(HD_, I8_) do { if (NT == 1) { if (TUNE(6) == 3) L_(HD_, I8_, 1, 4, 3); else if (TUNE(6) == 4) L_(HD_, I8_, 1, 4, 4); else if (TUNE(6) == 2) L_(HD_, I8_, 1, 4, 2); \
                                             else if (TUNE(6) == 8) L_(HD_, I8_, 1, 8, 2); else if (TUNE(6) == 9) L_(HD_, I8_, 1, 8, 3); else L_(HD_, I8_, 1, 4, (I8_ ? 4 : 2)); } else L_(HD_, I8_, 2, 4, 2); } while (0)
@@ -972,14 +977,15 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
 // (NG = 3: 72.7), ctx 1024 unchanged; fp16 loses with more than two (28.4 -> 30.6 us at ctx 1024)
 #define L2_(HD_, I8_) do { if (NT == 1) L_(HD_, I8_, 1, 4, (I8_ ? 4 : 2)); else L_(HD_, I8_, 2, 4, 2); } while (0)
 #endif
-#define LB_(HD_, I8_) do { if (NT == 1) hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, 1, 4, (I8_ ? 4 : 2), true>), grid, dim3(256), 0, st, p); \
-                           else         hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, 2, 4, 2, true>), grid, dim3(256), 0, st, p); } while (0)
+#define LB_(HD_, I8_) do { if (NT == 1) LM_(HD_, I8_, 1, 4, (I8_ ? 4 : 2), true); else LM_(HD_, I8_, 2, 4, 2, true); } while (0)
     if (bf)            { if (kv->hd == 128) { if (int8) LB_(128, true); else LB_(128, false); } else { if (int8) LB_(64, true); else LB_(64, false); } }
     else if (kv->hd == 128) { if (int8) L2_(128, true); else L2_(128, false); }
     else               { if (int8) L2_(64, true);  else L2_(64, false); }
 #undef LB_
 #undef L2_
 #undef L_
+#undef LM_
+#undef LI_
     MI355_CHECK_LAUNCH("paged_attn_kernel");
     if (p.P > 1 && !p.done) {
         const int nblk = cdiv((int)rows * nh, 4);
