@@ -936,12 +936,14 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     int HW = p.G < 8 ? p.G : 8;
     while (p.G % HW) --HW;                                  // heads of a key/value head per block
     const int TW = 8 / HW, NW = HW * TW, JT = (kv->hd / 8 + NW - 1) / NW;
-    const dim3 pgrid(cdiv(q_len, 16 * TW), nh / HW, B);
-    // Prompt rows: where the blocks fill the chip; with fewer of them the other kernel's smaller row tiles and split contexts win (28 over 4 heads of 128, us there / here:
+    // tiles that have rows: of ragged sequences the lengths are on the device, each is taken to end in the middle of a tile
+    const long tile_rows = 16 * TW, most = (long)B * cdiv(q_len, tile_rows), mean = ((long)total_rows + (long)B * (tile_rows - 1) / 2 + tile_rows - 1) / tile_rows;
+    const long live = row_start && mean < most ? mean : most;
+    // Prompt rows: where the blocks with rows fill the chip; with fewer of them the other kernel's smaller row tiles and split contexts win (28 over 4 heads of 128, us there / here:
     // 8 x 512 rows 179 / 86, 3 x 352 72 / 52, 1 x 1500 137 / 106, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100)
-    if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)pgrid.x * pgrid.y * pgrid.z >= 256 && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
+    if (!int8 && img_mblk == 0 && q_len >= 16 && !done && live * (nh / HW) >= 256 && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
         constexpr int NS = 3;
-        const dim3 grid = pgrid;
+        const dim3 grid(cdiv(q_len, 16 * TW), nh / HW, B);
         const size_t lds = (size_t)NS * JT * NW * 1024 + 16;
         hipStream_t st = (hipStream_t)stream;
         if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS);

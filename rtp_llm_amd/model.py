@@ -584,34 +584,36 @@ class DecoderEngine:
         longest = max(len(p) for p in prompts)
         logits = torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
         for c0 in range(0, longest, chunk):
-            q_len = min(chunk, longest - c0)
-            counts = [max(0, min(q_len, len(p) - c0)) for p in prompts]
-            first = [sum(counts[:b]) for b in range(nseq + 1)]
-            T = first[nseq]
-            toks = torch.cat([torch.as_tensor(p[c0:c0 + n], dtype=torch.int32).cpu() for p, n in zip(prompts, counts)])
-            pos = torch.cat([torch.arange(start[b] + c0, start[b] + c0 + n, dtype=torch.int32) for b, n in enumerate(counts)])
-            ending = [b for b, p in enumerate(prompts) if counts[b] and c0 + counts[b] == len(p)]
-            last = torch.zeros(nseq, dtype=torch.int32)
-            for b in ending:
-                last[b] = first[b] + counts[b] - 1
-            # the chunk's integers in one copy: tokens, positions, logit rows and, unless every sequence has q_len rows, where each sequence's rows lie
-            parts = [toks, pos, last]
-            if T < nseq * q_len:
-                parts += [torch.repeat_interleave(torch.arange(nseq, dtype=torch.int32), torch.tensor(counts)), torch.tensor(first, dtype=torch.int32)]
-            td, pd, ld, *ragged = torch.cat(parts).to(dev).split([p.numel() for p in parts])
-            ws_bytes = self.lib.mi355_decoder_prefill_workspace_bytes(self.handle, T, nseq)
+            # the sequences that still have tokens; what has ended takes no blocks, logit rows or table rows of the pass
+            live = [b for b, p in enumerate(prompts) if len(p) > c0]
+            counts = [min(chunk, len(prompts[b]) - c0) for b in live]
+            n, q_len = len(live), max(counts)
+            first = [sum(counts[:i]) for i in range(n + 1)]
+            T = first[n]
+            toks = torch.cat([torch.as_tensor(prompts[b][c0:c0 + k], dtype=torch.int32).cpu() for b, k in zip(live, counts)])
+            pos = torch.cat([torch.arange(start[b] + c0, start[b] + c0 + k, dtype=torch.int32) for b, k in zip(live, counts)])
+            ending = [i for i, b in enumerate(live) if c0 + counts[i] == len(prompts[b])]
+            last = torch.zeros(n, dtype=torch.int32)
+            for i in ending:
+                last[i] = first[i] + counts[i] - 1
+            # the chunk's integers in one copy: tokens, positions, logit rows, the sequences and, unless every sequence has q_len rows, where each sequence's rows lie
+            parts = [toks, pos, last, torch.tensor(live, dtype=torch.int32)]
+            if T < n * q_len:
+                parts += [torch.repeat_interleave(torch.arange(n, dtype=torch.int32), torch.tensor(counts)), torch.tensor(first, dtype=torch.int32)]
+            td, pd, ld, lived, *ragged = torch.cat(parts).to(dev).split([p.numel() for p in parts])
+            table = btd if n == nseq else btd.index_select(0, lived)
+            ws_bytes = self.lib.mi355_decoder_prefill_workspace_bytes(self.handle, T, n)
             if getattr(self, "_prefill_ws", None) is None or self._prefill_ws.numel() < ws_bytes:
                 self._prefill_ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            tmp_logits = torch.empty(nseq, self.cfg.vocab, dtype=torch.float32, device=dev) if ending else None
+            tmp_logits = torch.empty(n, self.cfg.vocab, dtype=torch.float32, device=dev) if ending else None
             seqd, firstd = (r.data_ptr() for r in ragged) if ragged else (None, None)
-            _C.check(self.lib.mi355_decoder_prefill_ragged(self.handle, td.data_ptr(), pd.data_ptr(), seqd, firstd, btd.data_ptr(), nseq, q_len, T,
+            _C.check(self.lib.mi355_decoder_prefill_ragged(self.handle, td.data_ptr(), pd.data_ptr(), seqd, firstd, table.data_ptr(), n, q_len, T,
                                                            ld.data_ptr() if ending else None, tmp_logits.data_ptr() if ending else None,
                                                            self._prefill_ws.data_ptr(), self._prefill_ws.numel(), st), "decoder_prefill")
             if len(ending) == nseq:
                 logits = tmp_logits
             elif ending:
-                sel = torch.tensor(ending, device=dev)
-                logits[sel] = tmp_logits[sel]
+                logits[torch.tensor([live[i] for i in ending], device=dev)] = tmp_logits[torch.tensor(ending, device=dev)]
         return logits
 
     def generate(self, prompts: List[List[int]], block_table, max_new_tokens: int, prefill_chunk: int = 512) -> List[List[int]]:
