@@ -761,10 +761,11 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
 
 // M of 2 to 16, p.vec.  Few outputs (blocks of 8 still one for every compute unit): 8 per block where M allows it, so that all compute units pull weights; narrow outputs:
 // more waves per tile keep the memory system busy.  M = 8, weights from memory, us with 16 / 8 outputs: 2048 x 5632 12.8 / 10.7, 2048 x 2048 6.4 / 5.5, 16 x 2048 5.3 / 4.4,
-// 1024 x 1024 4.8 / 4.4; past the line, where some compute units get a second block: 2176 x 2048 6.3 / 7.1, 2560 x 5632 13.5 / 15.4, gated 2304 x 1024 6.3 / 6.9.
+// 1024 x 1024 4.8 / 4.4; past the line, where some compute units get a second block: 2176 x 2048 6.3 / 7.1, 2560 x 5632 13.5 / 15.4, gated 2304 x 1024 6.3 / 6.9;
+// short K, of which a wave has a step or two: 1536 x 512 3.9 / 3.7, 48 x 192 2.6 / 3.0, gated 512 x 152 2.8 / 3.3.
 void launch_skinny(const DenseParams& p, hipStream_t st) {
     const int nout = p.gated ? p.N / 2 : p.N, tiles = (nout + 15) / 16;
-    if (p.M <= 8 && p.K >= 128 && tiles * p.G <= 128) {
+    if (p.M <= 8 && p.K >= 512 && tiles * p.G <= 128) {
         const dim3 grid((nout + 7) / 8, p.G), block(p.K < 1024 ? 128 : 256);
         if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, true>), grid, block, 0, st, p, 0);
         else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, true>), grid, block, 0, st, p, 0);
