@@ -936,12 +936,11 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     int HW = p.G < 8 ? p.G : 8;
     while (p.G % HW) --HW;                                  // heads of a key/value head per block
     const int TW = 8 / HW, NW = HW * TW, JT = (kv->hd / 8 + NW - 1) / NW;
-    // tiles that have rows: of ragged sequences the lengths are on the device, each is taken to end in the middle of a tile
-    const long tile_rows = 16 * TW, most = (long)B * cdiv(q_len, tile_rows), mean = ((long)total_rows + (long)B * (tile_rows - 1) / 2 + tile_rows - 1) / tile_rows;
-    const long live = row_start && mean < most ? mean : most;
-    // Prompt rows: where the blocks with rows fill the chip; with fewer of them the other kernel's smaller row tiles and split contexts win (28 over 4 heads of 128, us there / here:
-    // 8 x 512 rows 179 / 86, 3 x 352 72 / 52, 1 x 1500 137 / 106, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100)
-    if (!int8 && img_mblk == 0 && q_len >= 16 && !done && live * (nh / HW) >= 256 && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
+    // Prompt rows: where the rows fill the waves of about as many blocks as the chip has compute units (a third more where heads share no keys: a block then holds 128 rows of one
+    // head); with fewer the other kernel's smaller row tiles and split contexts win.  us there / here: 28 over 4 heads of 128, 8 x 512 rows 179 / 86, 3 x 352 72 / 52, 1 x 1500 137 /
+    // 106, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100, 37 x 20 behind 3477 188 / 250; 16 over 16 heads of 64, 16 x 34 behind 3628 75 / 117; 32 over 32 of 128, 38 x 23 behind
+    // 3378 409 / 603.  Over 300 random calls the pick is 1.7 x faster than the other kernel, 3 of them slower (by up to a fifth, at contexts of thousands).
+    if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)p.rows * nh >= 16L * NW * (HW == 1 ? 310 : 240) && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
         constexpr int NS = 3;
         const dim3 grid(cdiv(q_len, 16 * TW), nh / HW, B);
         const size_t lds = (size_t)NS * JT * NW * 1024 + 16;

@@ -51,7 +51,7 @@ def _check(nh, nkv, hd, page, dtype, lens, start):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,hd,page", [(28, 4, 128, 16), (14, 2, 64, 64), (8, 8, 128, 24), (8, 2, 64, 16), (10, 2, 128, 40)])
 def test_many_rows(nh, nkv, hd, page, dtype):
-    lens = [300, 1, 0, 17, 16, 0, 255, 2, 129, 33] * 8                       # 752 rows in ten sequences, eight times: at least 256 blocks for every grouping of heads
+    lens = [300, 1, 0, 17, 16, 0, 255, 2, 129, 33] * 10                      # 753 rows in ten sequences, ten times: enough waves with rows for every grouping of heads
     _check(nh, nkv, hd, page, dtype, lens, [(7 * i) % 90 if i % 3 else 0 for i in range(len(lens))])
 
 
@@ -60,6 +60,14 @@ def test_many_rows(nh, nkv, hd, page, dtype):
 @pytest.mark.parametrize("lens,start", [([0] * 15 + [64], [0] * 15 + [2048]), ([64] + [0] * 31, [700] * 32), ([1] * 40 + [40], [300] * 41), ([0, 500, 0], [0, 20, 0])])
 def test_few_sequences_with_rows(nh, nkv, hd, page, dtype, lens, start):
     _check(nh, nkv, hd, page, dtype, lens, start)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 8, 128), (8, 2, 64), (6, 2, 64)])
+@pytest.mark.parametrize("q_len", [16, 33])
+def test_many_short_portions(nh, nkv, hd, q_len):
+    """Blocks of which some waves have no rows."""
+    B = 40960 // (nh * q_len) + 1                                             # rows for 310 blocks' waves and more
+    _check(nh, nkv, hd, 16, torch.float16, [q_len] * B, [40 if i % 2 else 0 for i in range(B)])
 
 
 def test_prefill_when_most_prompts_have_ended():
