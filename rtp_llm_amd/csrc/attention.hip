@@ -641,27 +641,10 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
 // key, a value row (one channel, 32 tokens) is 64 bytes and needs none.
 // 8 x 512 rows, 28 over 4 heads of 128: 179 -> 86 us; 3 ragged of 389: 51 -> 29.
 // What bounds it: a step of one wave, about 1.4 us of product, softmax and product in series whatever the depth of the staging (3 to 6 stages measured the same).
-// 16 bytes per lane to LDS at `lds` + 16 lane, from base + voff
-__device__ __forceinline__ void pr_dma16(uint32_t lds, uint32_t voff, const void* base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-}
-template <int VM> __device__ __forceinline__ void pr_wait() {     // at most VM vector-memory operations of the wave left, no LDS operation
-    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
-}
-__device__ __forceinline__ void pr_wait(int left) {
-    asm volatile("" ::: "memory");
-    switch (left) {
-        case 0: pr_wait<0>(); break;    case 1: pr_wait<1>(); break;    case 2: pr_wait<2>(); break;    case 3: pr_wait<3>(); break;
-        case 4: pr_wait<4>(); break;    case 5: pr_wait<5>(); break;    case 6: pr_wait<6>(); break;    case 7: pr_wait<7>(); break;
-        case 8: pr_wait<8>(); break;    case 9: pr_wait<9>(); break;    case 10: pr_wait<10>(); break;  case 11: pr_wait<11>(); break;
-        case 12: pr_wait<12>(); break;  case 13: pr_wait<13>(); break;  case 14: pr_wait<14>(); break;  case 15: pr_wait<15>(); break;
-        default: pr_wait<16>(); break;
-    }
-    asm volatile("" ::: "memory");
-}
-
+constexpr int PR_STAGES = 3;
 template <int HD, bool BF>
-__global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p, int HW, int TW, int NS) {
+__global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p, int HW, int TW) {
+    constexpr int NS = PR_STAGES;
     constexpr int NSTEP = HD / 32, NDB = HD / 16, KL = HD / 16, LOADS = 2 * KL;     // 1 KB loads of a key tile (32 rows), of a step
     constexpr int CK = HD / 8;
     extern __shared__ __attribute__((aligned(16))) char pr_sm[];
@@ -724,16 +707,16 @@ __global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p,
                 const int wt = min(st * 32 + win[j] * 8, lastw), ti = wt - page_of(wt) * p.page, blk = min(max(id[j], 0), p.num_blocks - 1);
                 const uint32_t hk = (uint32_t)blk * (uint32_t)(2 * p.nkv) + (uint32_t)(isv[j] ? p.nkv + kh : kh);
                 const uint16_t* src = (const uint16_t*)p.kv_base + (uint64_t)hk * (uint32_t)(p.page * HD) + (uint32_t)(isv[j] ? ti : (ti + koff[j]) * HD);
-                pr_dma16(__builtin_amdgcn_readfirstlane(lds0 + buf * stage + (j * NW + wave) * 1024), voff[j], src);
+                dma16(__builtin_amdgcn_readfirstlane(lds0 + buf * stage + (j * NW + wave) * 1024), voff[j], src);
             }
         };
-        pr_wait(0);                                               // the rows' queries are here: no wait for them (and with it for the DMA) inside the loop
+        wait_vm<0>();                                             // the rows' queries are here: no wait for them (and with it for the DMA) inside the loop
         for (int st = 0; st < min(NS - 1, nsteps); ++st) { fetch(st); issue(st, st); }
         fetch(NS - 1);
         int buf = 0;
         const int kswz = lr & 3;                                  // key of the lane's row: (lr >> 2) * 8 + tau * 4 + (lr & 3)
         for (int st = 0; st < nsteps; ++st) {
-            pr_wait(JT * min(NS - 2, nsteps - 1 - st));           // all but the later steps' loads of this wave
+            wait_vm(JT * min(NS - 2, nsteps - 1 - st));           // all but the later steps' loads of this wave
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             const int t0 = st * 32;
@@ -941,14 +924,13 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     // 106, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100, 37 x 20 behind 3477 188 / 250; 16 over 16 heads of 64, 16 x 34 behind 3628 75 / 117; 32 over 32 of 128, 38 x 23 behind
     // 3378 409 / 603.  Over 300 random calls the pick is 1.7 x faster than the other kernel, 3 of them slower (by up to a fifth, at contexts of thousands).
     if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)p.rows * nh >= 16L * NW * (HW == 1 ? 310 : 240) && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
-        constexpr int NS = 3;
         const dim3 grid(cdiv(q_len, 16 * TW), nh / HW, B);
-        const size_t lds = (size_t)NS * JT * NW * 1024 + 16;
+        const size_t lds = (size_t)PR_STAGES * JT * NW * 1024 + 16;
         hipStream_t st = (hipStream_t)stream;
-        if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS);
-                             else          hipLaunchKernelGGL((prompt_attn_kernel<128, false>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS); }
-        else               { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<64, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS);
-                             else          hipLaunchKernelGGL((prompt_attn_kernel<64, false>), grid, dim3(64 * NW), lds, st, p, HW, TW, NS); }
+        if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW);
+                             else          hipLaunchKernelGGL((prompt_attn_kernel<128, false>), grid, dim3(64 * NW), lds, st, p, HW, TW); }
+        else               { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<64, true>), grid, dim3(64 * NW), lds, st, p, HW, TW);
+                             else          hipLaunchKernelGGL((prompt_attn_kernel<64, false>), grid, dim3(64 * NW), lds, st, p, HW, TW); }
         MI355_CHECK_LAUNCH("prompt_attn_kernel");
         return MI355_OK;
     }

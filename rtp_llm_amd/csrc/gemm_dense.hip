@@ -241,17 +241,6 @@ __global__ __launch_bounds__(256) void dense_tile_bf16_kernel(DenseParams p) {
 //   M x N x K       8192x2048x2048 62 / 71 / 82 / 86 / 112, 118    6148x1408x1024 gated 33 / 31 / 29 / 32 / 37, 43     768x11264x2048 gated 50 / 52 / 49 / 53 / 61, 73
 //                   1537x2176x1024 30 / 15 / 14 / 13 /  17,  25    1537x1024x1024       29 / 15 / 13 / 11 / 10, 21     768x2048x5632       109 / 57 / 52 / 36 / 34, 77
 //                   1537x3072x1024 30 / 20 / 18 / 21 /  22,  30    1537x1024x2816       60 / 32 / 29 / 21 / 20, 45      70x2048x2048        42 / 23 / 20 / 16 / 12, 32
-__device__ __forceinline__ void dn_dma16(uint32_t lds, uint32_t voff, const void* base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-}
-
-// waits until at most VM of the wave's vector-memory operations and none of its LDS operations are left.  (A builtin, not asm: the compiler's own counting sees it.)
-template <int VM> __device__ __forceinline__ void dn_wait() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-
 template <int BM, int BN, int WM, int WN, int BK, int NS>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_kernel(DenseParams p) {
     constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, MI = WM / 16, NJ = WN / 16;
@@ -289,7 +278,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
     auto issue = [&](int buf, int kt) {
 #pragma unroll
         for (int u = 0; u < ULD; ++u)
-            dn_dma16(lds0 + buf * STAGE + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024, voff[u], u < ULA ? X + kt * BK : W + kt * BK);
+            dma16(lds0 + buf * STAGE + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024, voff[u], u < ULA ? X + kt * BK : W + kt * BK);
     };
     f32x4 acc[MI][NJ];
 #pragma unroll
@@ -321,7 +310,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
         int at = 0;
         for (int kt = 0; kt < nk; ++kt) {
             // this wave's part of tile kt is in LDS, its reads of tile kt - 1 are done
-            if (NS == 2 || kt + NS - 2 >= nk) dn_wait<0>(); else dn_wait<ULD * (NS - 2)>();
+            if (NS == 2 || kt + NS - 2 >= nk) wait_vm<0>(); else wait_vm<ULD * (NS - 2)>();
             __builtin_amdgcn_s_barrier();
             if (kt + NS - 1 < nk) issue(at == 0 ? NS - 1 : at - 1, kt + NS - 1);
 #pragma unroll
@@ -330,7 +319,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
         }
     } else {
         if (nk > 0) {
-            if (nk >= NS - 1) dn_wait<ULD * (NS - 2)>(); else dn_wait<0>();
+            if (nk >= NS - 1) wait_vm<ULD * (NS - 2)>(); else wait_vm<0>();
             __builtin_amdgcn_s_barrier();
             load(fa, 0, 0);
         }
@@ -338,7 +327,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
         // IN_FLIGHT: tile kt + 1 is in LDS once at most that many of the wave's loads are left; its reads of tile kt are done by then, so behind the barrier
         // tile kt + NS - 1 may go over tile kt - 1
         auto advance = [&](Frags& nxt, auto in_flight, bool more) {
-            dn_wait<decltype(in_flight)::value>();
+            wait_vm<decltype(in_flight)::value>();
             __builtin_amdgcn_s_barrier();
             if (more) issue(ahead, kt + NS - 1);
             load(nxt, next, 0);

@@ -96,8 +96,7 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
         if (dma && c * 128 + 128 <= p.K) {
 #pragma unroll
             for (int u = 0; u < UPT; ++u)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                             :: "s"(lds0 + (buf * XSLOTS + (u * NWN + wave % NWN) * 64) * 16), "v"(xoff[u]), "s"((const char*)p.x + (size_t)c * 256) : "memory", "m0");
+                dma16(lds0 + (buf * XSLOTS + (u * NWN + wave % NWN) * 64) * 16, xoff[u], (const char*)p.x + (size_t)c * 256);
         } else {                                              // the last chunk of a K that is no multiple of 128 (columns past K are zero), a tensor off 16 bytes
 #pragma unroll
             for (int u = 0; u < UPT; ++u) {
@@ -234,8 +233,7 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     // Chunk c lies in buffer and ring d.  One barrier: behind it every wave's part of chunk c is in LDS and chunk c - KS is done with, so that the DMA of chunk c + KS may
     // go over it.  At most the weights of chunk c + KS are younger than the DMA of chunk c.
     auto chunk = [&](int c, int d) {
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt((WLD & 15) | (7 << 4) | ((WLD >> 4) << 14));
+        wait_vm<WLD>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (c + KS < KC) load_x(c + KS, d ^ 1);

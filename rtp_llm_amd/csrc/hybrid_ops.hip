@@ -872,17 +872,6 @@ __device__ __forceinline__ float hy_sum_groups(float v) {
     hy_swap<32>(v, a, b); v = a + b;
     hy_swap<16>(v, a, b); return a + b;
 }
-// 16 bytes per lane straight into LDS, at `lds` + 16 lane
-__device__ __forceinline__ void hy_dma16(uint32_t lds, const void* src) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(src) : "memory", "m0");
-}
-// until at most VM of the wave's vector-memory operations and none of its LDS operations are left (a builtin, which the compiler's own counting sees)
-template <int VM> __device__ __forceinline__ void hy_wait() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-
 constexpr int AT_STAGES = 3, AT_PAGES = 1024;     // block-table entries of the walked range held in LDS
 
 // DK: 32-channel steps of a key row.  NCBM: 16-channel fragments of a value row the instance holds; they are multiplied by fours (fragments past the row's end hold what lies
@@ -982,7 +971,7 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
             };
             const uint32_t base = buf * stage + wave * 1024;
             auto piece = [&](uint32_t at, const bf16* src) {
-                if (vec & 2) { hy_dma16(lds0 + at, src); return; }
+                if (vec & 2) { dma16(lds0 + at, src); return; }
                 bf16x8 v;                                     // a cache that is not on 16 bytes
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = src[i];
@@ -1005,17 +994,8 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
         int buf = 0;
         for (int st = 0; st < nsteps; ++st) {
             if (st + 1 < nsteps) {                            // all but the next step's loads of this wave
-                switch (JK + JV) {
-                    case 1: hy_wait<1>(); break;
-                    case 2: hy_wait<2>(); break;
-                    case 3: hy_wait<3>(); break;
-                    case 4: hy_wait<4>(); break;
-                    case 5: hy_wait<5>(); break;
-                    case 6: hy_wait<6>(); break;
-                    case 7: hy_wait<7>(); break;
-                    default: hy_wait<8>(); break;
-                }
-            } else hy_wait<0>();
+                wait_vm(JK + JV);
+            } else wait_vm<0>();
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             const int t0 = step_key(st), cur = buf * stage;

@@ -33,13 +33,13 @@ __device__ __forceinline__ float block_sum(float v, float* s_red) {
 }
 
 // Inverse-CDF draw from the unnormalised non-negative weights f(0..V-1): the first index j with f(j) > 0 whose inclusive
-// prefix sum, taken in index order, exceeds u01 * sum (`none` when rounding leaves none; V - 1 in the reference: sampling.cu:418).  Thread tx owns
+// prefix sum, taken in index order, exceeds u01 * sum (V - 1 when rounding leaves none: sampling.cu:418).  Thread tx owns
 // the contiguous segment [lo, hi) (a multiple of 4 long: segments start on 16-byte boundaries of an aligned row), so the block-level
 // prefix over threads is the prefix over indices.  Result in *s_found (valid for every thread after the call); returns sum.
 __device__ __forceinline__ int draw_segment(int V) { return (((V + kThreads - 1) / kThreads) + 3) & ~3; }
 
 template <class F>
-__device__ __forceinline__ float block_draw(F&& f, int V, float u01, float* s_red, float* s_scan, int* s_found, int none) {
+__device__ __forceinline__ float block_draw(F&& f, int V, float u01, float* s_red, float* s_scan, int* s_found) {
     const int tx = threadIdx.x;
     const int seg = draw_segment(V);
     const int lo = min(V, tx * seg), hi = min(V, lo + seg);
@@ -50,7 +50,7 @@ __device__ __forceinline__ float block_draw(F&& f, int V, float u01, float* s_re
     const float u = u01 * total;
     // inclusive prefix over threads (Hillis-Steele in LDS; 1024 entries)
     s_scan[tx] = local;
-    if (tx == 0) *s_found = none;
+    if (tx == 0) *s_found = V - 1;
     __syncthreads();
     for (int off = 1; off < kThreads; off <<= 1) {
         const float add = (tx >= off) ? s_scan[tx - off] : 0.f;
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kThreads) void rejection_sample_kernel(const Reject
         const float pv = dp ? dp[j] : (j == dtok ? 1.0f : 0.0f);
         return fmaxf(q[j] - pv, 0.f);
     };
-    block_draw(resid, p.V, p.uniform[row * G1 + min(pos + 1, G)], s_red, s_scan, &s_found, p.V - 1);
+    block_draw(resid, p.V, p.uniform[row * G1 + min(pos + 1, G)], s_red, s_scan, &s_found);
     if (tx == 0) {
         p.out_ids[row * G1 + pos] = s_found;
         for (int n = pos + 1; n < G1; ++n) p.out_ids[row * G1 + n] = -1;
@@ -564,7 +564,7 @@ __device__ __forceinline__ void filter_and_draw(const float* q, int V, uint32_t 
         const uint32_t b = __float_as_uint(v);
         return (b >= kb && (b > vbits || (b == vbits && j < cut))) ? v : 0.f;
     };
-    const float total = block_draw(kept, V, u, sh.red, sh.scan, &sh.found, V - 1);
+    const float total = block_draw(kept, V, u, sh.red, sh.scan, &sh.found);
     out(kept, lo, hi, total);
 }
 
