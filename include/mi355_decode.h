@@ -129,6 +129,10 @@ int mi355_linear_forward(const void* x, int32_t M, const mi355_weight_t* w, cons
                          void* y, int32_t epilogue, void* workspace, size_t workspace_bytes,
                          mi355_stream_t stream);
 
+/* The block shape of a linear over more than 64 rows (N_pad / 16 weight tiles, K_pad / 128 chunks): 0 128x512, 1 128x256, 2 64x256, 3 64x128, 4 64x64, 5 32x64,
+ * 6 32x32.  Host only. */
+int mi355_gemm_prefill_shape(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits);
+
 /*
  * Split-K half of the same GEMM: writes fp32 partial slabs
  * partials[split][M][N_pad] and returns the slab count (>0) — consumed by

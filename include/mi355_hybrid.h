@@ -87,6 +87,8 @@ int mi355_hy_delta_scan(const float* proj, int32_t ld, int32_t ro, int32_t ko, i
                         float decay_mult, float unit_eps, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start, const int32_t* slot,
                         const int32_t* first_pos, int32_t nseq, float* state, float* out, mi355_stream_t stream);
 
+/* The tile shape that a bf16 call of M x N x K takes (groups weights, row_tiles tiles of 64 sorted rows or 0): 0 64x64, 1 and 2 64x128, 3 128x128, 4 256x256.  Host only. */
+int mi355_dense_tile_shape(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t row_tiles);
 
 /* Further extended forms: an activation with a parameter (act 5: clamped gated form g' sigmoid(1.702 g') (u' + 1)), routers that score by sigmoids, rank
  * groups by their two best experts and scale the weights, a query / key norm over all heads at once, an embedding with a multiplier, and the end of a

@@ -79,6 +79,7 @@ SIGNATURES = {
     "mi355_last_error": (C.c_char_p, []),
     "mi355_linear_workspace_bytes": (sz, [i32, C.POINTER(Weight)]),
     "mi355_linear_forward": (i32, [vp, i32, C.POINTER(Weight), vp, vp, i32, vp, sz, vp]),
+    "mi355_gemm_prefill_shape": (i32, [i32] * 5),
     "mi355_linear_partial": (i32, [vp, i32, C.POINTER(Weight), vp, i32, vp]),
     "mi355_rmsnorm": (i32, [vp, vp, f32, i32, i32, vp, vp]),
     "mi355_add_rmsnorm": (i32, [vp, vp, i32, i32, vp, vp, vp, vp, f32, i32, i32, vp, vp]),
@@ -170,6 +171,7 @@ ip = C.POINTER(i32)
 HYBRID_SIGNATURES = {
     "mi355_abi_version": (i32, []),
     "mi355_last_error": (C.c_char_p, []),
+    "mi355_dense_tile_shape": (i32, [i32] * 5),
     "mi355_dense_linear": (i32, [vp, i32, i32, vp, i32, i32, vp, vp, i32, i32, i32, i32, f32, i32, vp]),
     "mi355_hy_embed": (i32, [vp, i32, vp, i32, i32, vp, i32, vp]),
     "mi355_hy_residual_norm": (i32, [vp, vp, vp, f32, vp, i32, i32, vp, vp, f32, f32, vp, vp, i32, vp]),

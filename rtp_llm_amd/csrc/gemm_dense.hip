@@ -18,6 +18,19 @@
 #include "common.h"
 #include "../../include/mi355_hybrid.h"
 
+// The tile shape of a bf16 call of M x N x K through `groups` weights (64-row tiles of sorted rows in `row_tiles`, 0: all M rows through each): 0 64x64, 1 64x128 in three stages,
+// 2 64x128 in two, 3 128x128, 4 256x256.  The one with the least expected time, us per 32 columns of k: a constant and the blocks per CU times what one costs a busy CU (256 x 256:
+// whole rounds count half, one block fills a CU; 64x128 in three stages: two blocks fill one).  Measured at M = 70..8192, N = 16..32000, K = 16..5632: within 10 % of the fastest.
+// Grouped rows come in tiles of 64.
+extern "C" int mi355_dense_tile_shape(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t row_tiles) {
+    auto share = [&](int bm, int bn) { return (double)((N + bn - 1) / bn) * (row_tiles ? row_tiles : (M + bm - 1) / bm) * groups / 256.0; };
+    const double sa = share(256, 256), sb = share(128, 128), sc = share(64, 128), se = share(64, 64), k = K / 32.0;
+    const double ta = row_tiles ? 1e30 : k * fmax(0.65, 0.475 * (sa + ceil(sa))) + 12.0, tb = row_tiles ? 1e30 : k * fmax(0.34, 0.255 * sb + 0.13) + 5.0;
+    const double tc = k * fmax(0.27, 0.15 * sc + 0.09) + 4.0, td = k * (sc <= 2.0 ? 0.18 + 0.06 * sc : 0.15 * sc + 0.22) + 4.0;
+    const double te = k * fmax(0.125, 0.105 * se + 0.02) + 4.0, t = fmin(fmin(ta, tb), fmin(tc, fmin(td, te)));
+    return t == te ? 0 : t == td ? 1 : t == tc ? 2 : t == tb ? 3 : 4;
+}
+
 namespace {
 
 constexpr int DN_ACT_NONE = 0, DN_ACT_RELU = 1, DN_ACT_SILU = 2, DN_ACT_GELU_TANH = 3, DN_ACT_TANH = 4, DN_ACT_SWIGLU_CLAMP = 5, DN_ACT_RELU2 = 6;
@@ -650,20 +663,13 @@ void launch_tiles_bf16(const DenseParams& p, int gy64, int gz, hipStream_t st) {
         hipLaunchKernelGGL(dense_tile_bf16_kernel, dim3((p.N + TB_N - 1) / TB_N, gy64, gz), dim3(256), 0, st, p);
         return;
     }
-    // the shape with the least expected time, us per 32 columns of k: a constant and the blocks per CU times what one costs a busy CU (256 x 256: whole rounds
-    // count half, one block fills a CU; 64x128 in three stages: two blocks fill one).  Measured at M = 70..8192, N = 16..32000, K = 16..5632: within 10 % of the fastest.
-    // Grouped rows come in tiles of 64.
-    auto share = [&](int bm, int bn) { return (double)((p.N + bn - 1) / bn) * (p.offs ? gy64 : (p.M + bm - 1) / bm) * gz / 256.0; };
-    const double sa = share(256, 256), sb = share(128, 128), sc = share(64, 128), se = share(64, 64), k = p.K / 32.0;
-    const double ta = p.offs ? 1e30 : k * fmax(0.65, 0.475 * (sa + ceil(sa))) + 12.0, tb = p.offs ? 1e30 : k * fmax(0.34, 0.255 * sb + 0.13) + 5.0;
-    const double tc = k * fmax(0.27, 0.15 * sc + 0.09) + 4.0, td = k * (sc <= 2.0 ? 0.18 + 0.06 * sc : 0.15 * sc + 0.22) + 4.0;
-    const double te = k * fmax(0.125, 0.105 * se + 0.02) + 4.0, t = fmin(fmin(ta, tb), fmin(tc, fmin(td, te)));
+    const int shape = mi355_dense_tile_shape(p.M, p.N, p.K, gz, p.offs ? gy64 : 0);
     const int gn = (p.N + 127) / 128;
-    if (t == te)      hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 64, 16, 64, 64, 4>), dim3((p.N + 63) / 64, gy64, gz), dim3(256), 0, st, p);
-    else if (t == td) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 3>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
-    else if (t == tc) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 2>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
-    else if (t == tb) hipLaunchKernelGGL((dense_dma_bf16_kernel<128, 128, 32, 64, 64, 2>), dim3(gn, (p.M + 127) / 128, gz), dim3(512), 0, st, p);
-    else              hipLaunchKernelGGL((dense_dma_bf16_kernel<256, 256, 128, 64, 32, 4>), dim3((p.N + 255) / 256, (p.M + 255) / 256, gz), dim3(512), 0, st, p);
+    if (shape == 0)      hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 64, 16, 64, 64, 4>), dim3((p.N + 63) / 64, gy64, gz), dim3(256), 0, st, p);
+    else if (shape == 1) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 3>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
+    else if (shape == 2) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 2>), dim3(gn, gy64, gz), dim3(256), 0, st, p);
+    else if (shape == 3) hipLaunchKernelGGL((dense_dma_bf16_kernel<128, 128, 32, 64, 64, 2>), dim3(gn, (p.M + 127) / 128, gz), dim3(512), 0, st, p);
+    else                 hipLaunchKernelGGL((dense_dma_bf16_kernel<256, 256, 128, 64, 32, 4>), dim3((p.N + 255) / 256, (p.M + 255) / 256, gz), dim3(512), 0, st, p);
 }
 
 template <typename T, bool GATED>

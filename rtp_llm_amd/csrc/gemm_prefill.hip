@@ -305,15 +305,15 @@ constexpr PrefillCost kPrefillCost[3][kPrefillShapeCount] = {
     {{1e9, 1e9},   {2.16, 2.45}, {1.52, 1.32}, {0.94, 0.708}, {0.98, 0.856}, {0.72, 0.507}, {0.69, 0.708}},      // bf16 under group scales: two sets of accumulators
     {{1e9, 1e9},   {1.41, 2.82}, {0.92, 1.84}, {0.49, 0.856}, {0.49, 0.779}, {0.45, 0.532}, {0.37, 0.742}},     // 16-bit weights
 };
-int pick_shape(const GemmParams& p, int wbits, double* t_best) {
-    const PrefillCost* cost = kPrefillCost[wbits == 16 ? 2 : (p.bf16 && wbits == 4) ? 1 : 0];
+int pick_shape(int M, int NT, int KC, bool bf, int wbits, double* t_best) {
+    const PrefillCost* cost = kPrefillCost[wbits == 16 ? 2 : (bf && wbits == 4) ? 1 : 0];
     int best = 1;
     *t_best = 1e30;
-    for (int i = (p.bf16 || wbits == 16) ? 1 : 0; i < kPrefillShapeCount; ++i) {
+    for (int i = (bf || wbits == 16) ? 1 : 0; i < kPrefillShapeCount; ++i) {
         const PrefillShape s = kPrefillShapes[i];
-        const double full = (double)cdiv(p.NT, 8 / s.ks * s.tpw) * cdiv(p.M, 16 * s.mb) / 256.0;
+        const double full = (double)cdiv(NT, 8 / s.ks * s.tpw) * cdiv(M, 16 * s.mb) / 256.0;
         const double whole = (double)(long)(full + 0.9999), share = cost[i].sat * 0.5 * (full + whole);
-        const double t = cdiv(p.KC, s.ks) * (share > cost[i].lat ? share : cost[i].lat) + 2.5;
+        const double t = cdiv(KC, s.ks) * (share > cost[i].lat ? share : cost[i].lat) + 2.5;
         if (t < *t_best) { *t_best = t; best = i; }
     }
     return best;
@@ -343,6 +343,12 @@ int launch_shape(int i, const GemmParams& p, hipStream_t st) {
 
 } // namespace
 
+// The block shape of a call, by its place in kPrefillShapes: NT = N_pad / 16, KC = K_pad / 128.
+extern "C" int mi355_gemm_prefill_shape(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits) {
+    double t;
+    return pick_shape(M, NT, KC, bf16 != 0, wbits, &t);
+}
+
 // Direct-mode launch (fused epilogue in p.mode).  MI355_ERR_UNSUPPORTED: shape / format not covered, caller falls back.
 // t_limit: the caller's estimate (us) for its other path; a launch expected to take longer is not made (MI355_ERR_UNSUPPORTED).
 extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, double t_limit, mi355_stream_t stream) {
@@ -352,7 +358,7 @@ extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, dou
     hipStream_t st = (hipStream_t)stream;
     const bool bf = g.bf16 != 0;
     double t;
-    const int s = pick_shape(g, wbits, &t);
+    const int s = pick_shape(g.M, g.NT, g.KC, bf, wbits, &t);
     if (t > t_limit) return MI355_ERR_UNSUPPORTED;
     if (wbits == 16) return bf ? launch_shape<16, 0, true>(s, g, st) : launch_shape<16, 0, false>(s, g, st);
     if (wbits == 8 && group_size == 0) return bf ? launch_shape<8, 0, true>(s, g, st) : launch_shape<8, 0, false>(s, g, st);

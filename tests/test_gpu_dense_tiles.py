@@ -14,9 +14,10 @@ def _rand(g, *shape, k=1.0):
     return (torch.randn(*shape, device=DEV, generator=g) * k).bfloat16()
 
 
-# rows x outputs x K: 64 x 128 tiles on one and two blocks per CU, 128 x 128, 256 x 256; K below, at and between the K tiles of 32 and 64
+# rows x outputs x K: 64 x 64 tiles, 64 x 128 in two and in three stages, 128 x 128, 256 x 256 (test_tile_shapes.py holds the list to that); K below, at and between the K tiles
+# of 32 and 64, and an even and an odd count of them with a remainder
 SHAPES = [(17, 8, 8), (63, 24, 40), (65, 130, 64), (129, 200, 72), (300, 1000, 32), (700, 2050, 200), (1537, 1028, 96), (2300, 4100, 136), (4700, 4360, 104), (513, 12, 2056),
-          (5000, 5000, 24)]
+          (5000, 5000, 24), (1537, 2172, 1032), (2304, 1028, 520), (6000, 1024, 264), (4700, 4360, 200), (6145, 1400, 1032), (6148, 4032, 232), (8190, 2044, 2056), (8190, 2044, 2088)]
 
 
 @pytest.mark.parametrize("f32", [True, False])
@@ -36,8 +37,11 @@ def test_dense_tiles(M, N, K, f32):
         assert torch.equal(hops.dense_linear(x[lo:lo + 17], w, bias, out_dtype=torch.float32 if f32 else None)[r - lo], y[r])
 
 
+GATED = [(65, 64, 40), (700, 1344, 72), (2300, 4160, 136), (4700, 4416, 104), (1537, 2176, 1032), (4700, 4352, 200), (8190, 2048, 2056)]
+
+
 @pytest.mark.parametrize("act", [hops.ACT_RELU, hops.ACT_SILU, hops.ACT_GELU_TANH])
-@pytest.mark.parametrize("M,N,K", [(65, 64, 40), (700, 1344, 72), (2300, 4160, 136), (4700, 4416, 104)])
+@pytest.mark.parametrize("M,N,K", GATED)
 def test_dense_tiles_gated(M, N, K, act):
     g = torch.Generator(device=DEV).manual_seed(M + N + K + act)
     gate, up, x = _rand(g, N // 2, K, k=K ** -0.5), _rand(g, N // 2, K, k=K ** -0.5), _rand(g, M, K)

@@ -23,8 +23,10 @@ def _dense64(c):
     return ((c.q.double().view(-1, g, c.N) - c.z_eff.double()[:, None]) * c.scales.double()[:, None]).view(c.K, c.N)
 
 
-# the shapes of a call go from 32 x 32 tiles on four K slices (narrow, deep, few rows) to 128 x 512 (many rows, wide)
-SHAPES = [(65, 136, 24), (66, 4864, 64), (129, 1280, 200), (130, 896, 1152), (257, 640, 4096), (513, 384, 9728), (1100, 256, 8208)]
+# every tile shape that a call of its class can take, from 32 x 32 on four K slices (narrow, deep, few rows) to 128 x 512 (many rows, wide; codes under fp16): test_tile_shapes.py
+# holds the list to that
+SHAPES = [(65, 136, 24), (66, 4864, 64), (129, 1280, 200), (130, 896, 1152), (257, 640, 4096), (513, 384, 9728), (1100, 256, 8208),
+          (131, 200, 37880), (201, 136, 37880), (300, 2048, 4104), (1537, 136, 4104), (2050, 136, 24), (517, 384, 37880)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

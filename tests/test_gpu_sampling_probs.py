@@ -40,3 +40,22 @@ def test_long_histories_are_refused():
     one = torch.ones(1, device=DEV)
     with pytest.raises(_C.Mi355Error):
         ops.sampling_probs(x, None, one, one, one, torch.zeros(1, 2049, dtype=torch.int32, device=DEV), None, 0, 2049)
+
+
+@pytest.mark.parametrize("V", [3, 67, 4096, 32003, 152064])
+def test_rows_with_infinities_and_nans(V):
+    """+infinity or NaN among a row's logits, wherever its slice lies, and a row without a finite value: NaN all over the row, as from the launches of their own; the other rows
+    are what they are without them, and a draw stays in the vocabulary."""
+    g = torch.Generator(device=DEV).manual_seed(V)
+    clean = torch.randn(9, V, device=DEV, generator=g) * 4
+    x, t = clean.clone(), torch.rand(9, device=DEV, generator=g) + 0.5
+    x[1, 0], x[2, V - 1], x[3, V // 2] = float("inf"), float("inf"), float("nan")
+    x[5, V - 1], x[5, 0], x[6], x[7] = float("nan"), float("inf"), float("-inf"), float("nan")
+    ref = x.clone()
+    ops.apply_penalties(ref, temperature=t)
+    ref = ops.softmax_rows(ref)
+    got, want = ops.sampling_probs(x.clone(), t), ops.sampling_probs(clean.clone(), t)
+    bad = torch.tensor([r in (1, 2, 3, 5, 6, 7) for r in range(9)], device=DEV)
+    assert bool(ref[bad].isnan().all()) and bool(got[bad].isnan().all()) and torch.equal(got[~bad], want[~bad])
+    ids = [ops.top_k_top_p_sample(p.clone(), torch.full((9,), 5, dtype=torch.int32), torch.full((9,), 0.9), torch.full((9,), 0.4, device=DEV)) for p in (got, want)]
+    assert torch.equal(ids[0][~bad], ids[1][~bad]) and bool(((ids[0] >= 0) & (ids[0] < V)).all())

@@ -1,0 +1,31 @@
+"""The lists of the tile tests reach every tile shape that a call can take: the shape chosen for each listed call, against all shapes chosen over a grid of sizes."""
+import pytest
+import test_gpu_dense_tiles as dense
+import test_gpu_prefill_gemm as prefill
+
+from rtp_llm_amd import _C
+
+
+def _prefill(M, K, N, bf16, wbits):
+    return _C.lib().mi355_gemm_prefill_shape(M, -(-N // 16), -(-K // 128), bf16, wbits)
+
+
+@pytest.mark.parametrize("wbits", [4, 8, 16])
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_prefill_shapes(bf16, wbits):
+    can = {_prefill(M, K, N, bf16, wbits) for M in (65, 96, 129, 200, 257, 300, 513, 1024, 1537, 2050, 3000, 4096, 8192) for K in (128, 256, 384, 640, 896, 1280, 3584, 4864, 18944)
+           for N in (24, 64, 200, 512, 1152, 3584, 4608, 9728, 18944, 37888, 151936)}
+    assert len(can) >= 5
+    assert {_prefill(M, K, N, bf16, wbits) for M, K, N in prefill.SHAPES} == can
+
+
+def test_dense_shapes():
+    pick = _C.hybrid_lib().mi355_dense_tile_shape
+    can = {pick(M, N, K, 1, 0) for M in (17, 65, 300, 768, 1537, 2304, 4700, 6000, 8190) for N in (8, 200, 1032, 2044, 4100, 16400) for K in (8, 40, 136, 264, 1032, 2056)}
+    assert can == {0, 1, 2, 3, 4}
+    assert {pick(M, N, K, 1, 0) for M, N, K in dense.SHAPES} == can
+    # gated calls: the small tile, both middle ones that they are given in practice, the largest
+    assert {0, 1, 4} <= {pick(M, N, K, 1, 0) for M, N, K in dense.GATED}
+    # the largest tile with an even and an odd count of K tiles of 32, both with a remainder
+    assert {K // 32 % 2 for M, N, K in dense.SHAPES if pick(M, N, K, 1, 0) == 4 and K % 32} == {0, 1}
+    assert {pick(M, N, K, 1, 64) for M, N, K in dense.SHAPES} <= {0, 1, 2}           # sorted rows: tiles of 64
