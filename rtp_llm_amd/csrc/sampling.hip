@@ -225,25 +225,28 @@ struct PenaltyParams {
     int32_t*       counts;         // [batch][V]: histories of more than kShortHistory entries
 };
 
-// Temperature alone: blockIdx.x splits the row.
-template <bool WHOLE>
-__global__ __launch_bounds__(kThreads) void temperature_kernel(const PenaltyParams p) {
-    const int row = WHOLE ? blockIdx.x : blockIdx.y, start = (WHOLE ? 0 : blockIdx.x * kThreads) + threadIdx.x, stride = WHOLE ? kThreads : gridDim.x * kThreads;
-    float* x = p.logits + (size_t)row * p.ld;
+// Of the n values of x a thread's own (start, start + stride, ..) by its row's temperature; vec: x lies on 16 bytes, start and stride count fours there.
+__device__ __forceinline__ void scale_row(const PenaltyParams& p, int row, float* x, int n, bool vec, int start, int stride) {
     const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
     int done = 0;
-    if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0) {
+    if (vec) {
         f32x4* x4 = reinterpret_cast<f32x4*>(x);
-        const int V4 = p.V >> 2;
+        done = n & ~3;
 #pragma unroll 4
-        for (int j = start; j < V4; j += stride) {
+        for (int j = start; j < n >> 2; j += stride) {
             f32x4 v = x4[j];
             v[0] *= inv_t; v[1] *= inv_t; v[2] *= inv_t; v[3] *= inv_t;
             x4[j] = v;
         }
-        done = V4 << 2;
     }
-    for (int j = done + start; j < p.V; j += stride) x[j] *= inv_t;
+    for (int j = done + start; j < n; j += stride) x[j] *= inv_t;
+}
+
+// Temperature alone: blockIdx.x splits the row.
+template <bool WHOLE>
+__global__ __launch_bounds__(kThreads) void temperature_kernel(const PenaltyParams p) {
+    const int row = WHOLE ? blockIdx.x : blockIdx.y, start = (WHOLE ? 0 : blockIdx.x * kThreads) + threadIdx.x, stride = WHOLE ? kThreads : gridDim.x * kThreads;
+    scale_row(p, row, p.logits + (size_t)row * p.ld, p.V, (p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0, start, stride);
 }
 
 __device__ __forceinline__ float penalised(const PenaltyParams& p, int row, float logit, int count) {
@@ -304,21 +307,7 @@ __global__ __launch_bounds__(kThreads) void sampling_prepare_kernel(const Penalt
     const int row = blockIdx.y, tx = threadIdx.x, lo = min(p.V, (int)blockIdx.x * slice), n = min(p.V, lo + slice) - lo;
     float* x = p.logits + (size_t)row * p.ld + lo;
     const bool vec = (p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;       // lo is a multiple of 4
-    if (p.temperature) {
-        const float inv_t = 1.0f / (p.temperature[row] + 1e-6f);
-        int done = 0;
-        if (vec) {
-            f32x4* x4 = reinterpret_cast<f32x4*>(x);
-#pragma unroll 4
-            for (int j = tx; j < n >> 2; j += kThreads) {
-                f32x4 v = x4[j];
-                v[0] *= inv_t; v[1] *= inv_t; v[2] *= inv_t; v[3] *= inv_t;
-                x4[j] = v;
-            }
-            done = n & ~3;
-        }
-        for (int j = done + tx; j < n; j += kThreads) x[j] *= inv_t;
-    }
+    if (p.temperature) scale_row(p, row, x, n, vec, tx, kThreads);
     if (p.output_ids) penalise_history<kThreads>(p, table, row, id_step, id_row, lo, n, x);
     __threadfence_block();
     __syncthreads();
