@@ -567,11 +567,11 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     if (tid == 0) s_m[0][0] = __builtin_bit_cast(float, __hip_atomic_fetch_add(p.done + ((size_t)blockIdx.z * p.nkv + kh) * p.done_step, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     __syncthreads();
     if (__builtin_bit_cast(int, s_m[0][0]) != nparts - 1) return;
-    // Up to eight parts: a thread takes four channels of a row's head through all of them in one round trip.  More: eight or sixteen in flight by 16-byte loads, and where
-    // the rows leave threads without channels (7 heads of 64: 112 of 256) the waves split the parts and meet in LDS.  Against the merge in a launch of its own, us per call,
-    // before / now / launch: 14 over 2 heads of 64, 8 sequences, 8 parts 8.0 / 7.0 / 7.5, 16 parts 10.4 / 7.8 / 7.7, 1 sequence, 32 parts 9.9 / 8.3 / 11.6; 28 over 4 heads of
-    // 128, 4 sequences, 8 parts 9.3 / 8.2 / 8.7, 16 parts 12.0 / 9.6 / 9.5, 1 sequence, 16 parts 9.6 / 9.2 / 9.0, 32 parts 12.9 / 11.4 / 13.2.  Most of it was the counters:
-    // side by side, up to 256 arrivals went through one cache line (8 sequences of 16 parts: 8.1 with nothing changed but their distance).
+    // A thread takes four channels of a row's head (the host sees to it that the block has a thread for each), up to eight parts in one round trip.  More: eight or sixteen in flight by
+    // 16-byte loads, and where the rows leave threads without channels (7 heads of 64: 112 of 256) the waves split the parts and meet in LDS.  Against the merge in a launch of
+    // its own, us per call, before / now / launch: 14 over 2 heads of 64, 8 sequences, 8 parts 8.0 / 7.0 / 7.5, 16 parts 10.4 / 7.8 / 7.7, 1 sequence, 32 parts 9.9 / 8.3 / 11.6;
+    // 28 over 4 heads of 128, 4 sequences, 8 parts 9.3 / 8.2 / 8.7, 16 parts 12.0 / 9.6 / 9.5, 1 sequence, 16 parts 9.6 / 9.2 / 9.0, 32 parts 12.9 / 11.4 / 13.2.  Most of it was
+    // the counters: side by side, up to 256 arrivals went through one cache line (8 sequences of 16 parts: 8.1 with nothing changed but their distance).
     auto merge = [&](auto in_flight, auto split) {
         constexpr int U = decltype(in_flight)::value;
         const int items = nrows * p.G * (HD / 4), share = !decltype(split)::value ? 1 : items <= 64 ? NW : items <= 64 * NW / 2 ? 2 : 1, span = NTHR / share;
@@ -580,50 +580,49 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
         const uint32_t mlo = (uint32_t)(p.tmp_ml - p.tmp_out) * 4u;
         f32x4* x_o = reinterpret_cast<f32x4*>(&s_o[0][0][0]);
         float2* x_ml = reinterpret_cast<float2*>(x_o + (share - 1) * span);
-        for (int at = tid - sw * span; at < (share > 1 ? span : items); at += NTHR) {
-            const int idx = share > 1 ? min(at, items - 1) : at, col = idx / (HD / 4), d0 = (idx - col * (HD / 4)) * 4, rl = col / p.G, row = row0 + rl, h = kh * p.G + (col - rl * p.G);
-            const int np = (min(max(p.seq_lens[row] + p.seq_add, 0), p.max_seq) + p.PS - 1) / p.PS;      // partitions that saw this row
-            const size_t slot = ((size_t)row * p.nh + h) * p.P;
-            const float* ml = p.tmp_ml + slot * 2;
-            const float* po = p.tmp_out + slot * HD + d0;
-            float mstar = NEG_BIG, l = 0.f;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            for (int i0 = sw * U; i0 < np; i0 += share * U) {        // U parts in flight, summed in partition order
-                float2 v[U], oa[U], ob[U];
+        const int at = tid - sw * span, idx = min(at, items - 1), col = idx / (HD / 4), d0 = (idx - col * (HD / 4)) * 4, rl = col / p.G, row = row0 + rl, h = kh * p.G + (col - rl * p.G);
+        if (share == 1 && at >= items) return;
+        const int np = (min(max(p.seq_lens[row] + p.seq_add, 0), p.max_seq) + p.PS - 1) / p.PS;      // partitions that saw this row
+        const size_t slot = ((size_t)row * p.nh + h) * p.P;
+        const float* ml = p.tmp_ml + slot * 2;
+        const float* po = p.tmp_out + slot * HD + d0;
+        float mstar = NEG_BIG, l = 0.f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int i0 = sw * U; i0 < np; i0 += share * U) {        // U parts in flight, summed in partition order
+            float2 v[U], oa[U], ob[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int i = min(i0 + u, np - 1);
-                    if constexpr (decltype(split)::value) {
-                        const u32x4 o4 = __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)((slot + i) * HD + d0) * 4u, 0, 16 /* sc1 */);
-                        v[u] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rp, mlo + (uint32_t)(slot + i) * 8u, 0, 16));
-                        oa[u] = __builtin_bit_cast(float2, u32x2{o4[0], o4[1]}); ob[u] = __builtin_bit_cast(float2, u32x2{o4[2], o4[3]});
-                    } else { v[u] = get2(ml + i * 2); oa[u] = get2(po + (size_t)i * HD); ob[u] = get2(po + (size_t)i * HD + 2); }
-                }
-                float mnew = mstar;
-#pragma unroll
-                for (int u = 0; u < U; ++u) mnew = fmaxf(mnew, v[u].x);
-                const float resc = __builtin_amdgcn_exp2f(mstar - mnew);
-                l *= resc; acc *= resc; mstar = mnew;
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if (i0 + u >= np) continue;
-                    const float f = __builtin_amdgcn_exp2f(v[u].x - mstar);
-                    l += v[u].y * f;
-                    acc += f32x4{oa[u].x, oa[u].y, ob[u].x, ob[u].y} * f;
-                }
+            for (int u = 0; u < U; ++u) {
+                const int i = min(i0 + u, np - 1);
+                if constexpr (decltype(split)::value) {
+                    const u32x4 o4 = __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)((slot + i) * HD + d0) * 4u, 0, 16 /* sc1 */);
+                    v[u] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rp, mlo + (uint32_t)(slot + i) * 8u, 0, 16));
+                    oa[u] = __builtin_bit_cast(float2, u32x2{o4[0], o4[1]}); ob[u] = __builtin_bit_cast(float2, u32x2{o4[2], o4[3]});
+                } else { v[u] = get2(ml + i * 2); oa[u] = get2(po + (size_t)i * HD); ob[u] = get2(po + (size_t)i * HD + 2); }
             }
-            if (share > 1) {                                         // one pass of the loop for every wave
-                if (sw > 0) { x_o[(sw - 1) * span + at] = acc; x_ml[(sw - 1) * span + at] = make_float2(mstar, l); }
-                __syncthreads();
-                if (sw > 0 || at >= items) break;
-                for (int k = 0; k < share - 1; ++k) {
-                    const float2 o_ml = x_ml[k * span + at];
-                    const float mnew = fmaxf(mstar, o_ml.x), fa = __builtin_amdgcn_exp2f(mstar - mnew), fb = __builtin_amdgcn_exp2f(o_ml.x - mnew);
-                    l = l * fa + o_ml.y * fb; acc = acc * fa + x_o[k * span + at] * fb; mstar = mnew;
-                }
+            float mnew = mstar;
+#pragma unroll
+            for (int u = 0; u < U; ++u) mnew = fmaxf(mnew, v[u].x);
+            const float resc = __builtin_amdgcn_exp2f(mstar - mnew);
+            l *= resc; acc *= resc; mstar = mnew;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (i0 + u >= np) continue;
+                const float f = __builtin_amdgcn_exp2f(v[u].x - mstar);
+                l += v[u].y * f;
+                acc += f32x4{oa[u].x, oa[u].y, ob[u].x, ob[u].y} * f;
             }
-            store_out(row, h * HD + d0, acc, l);
         }
+        if (share > 1) {
+            if (sw > 0) { x_o[(sw - 1) * span + at] = acc; x_ml[(sw - 1) * span + at] = make_float2(mstar, l); }
+            __syncthreads();
+            if (sw > 0) return;
+            for (int k = 0; k < share - 1; ++k) {
+                const float2 o_ml = x_ml[k * span + at];
+                const float mnew = fmaxf(mstar, o_ml.x), fa = __builtin_amdgcn_exp2f(mstar - mnew), fb = __builtin_amdgcn_exp2f(o_ml.x - mnew);
+                l = l * fa + o_ml.y * fb; acc = acc * fa + x_o[k * span + at] * fb; mstar = mnew;
+            }
+        }
+        if (at < items) store_out(row, h * HD + d0, acc, l);
     };
     if (nparts <= 8) merge(std::integral_constant<int, 8>{}, std::false_type{});
     else if (nparts <= 16 && nrows * p.G * (HD / 4) <= 64 * NW / 2) merge(std::integral_constant<int, 8>{}, std::true_type{});
@@ -943,13 +942,18 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
         mi355_set_error("paged_attn: workspace %zu < %zu", workspace_bytes, need);
         return MI355_ERR_WORKSPACE;
     }
-    p.done = p.P > 1 ? done : nullptr; p.done_step = done_step;
+    // The last partition merges where its block has a thread for every four channels of the tile's rows (one row of up to 8 heads of 128, 16 of 64 per key/value head; never two tiles
+    // of rows): one trip past the L2 of about 2 us against 3 for a launch.  With more outputs than threads the trips add up: us with the launch / in the block, 28 over 4 heads of 128,
+    // 6 sequences of 4 rows, 2 parts 11.9 / 15.6, 2 of 8 rows, 12 parts 15.1 / 22.0; 7 over 1 of 64, 9 of 4 rows, 17 parts 9.6 / 15.0; 16 over 2 of 128, 4 of 2 rows, 24 parts
+    // 13.4 / 17.2.  Heads of 64, whose launch is the cheaper one, only with half the threads or few parts: 24 over 2, 1 row, 18 parts 8.2 / 9.6, 7 over 1, 15 of 2 rows, 15 parts 9.6 / 10.4.
+    const int outs = (q_len < p.R ? q_len : p.R) * p.G * (kv->hd / 4);
+    p.done = p.P > 1 && NT == 1 && outs <= (kv->hd == 128 || p.P <= 8 ? 256 : 128) ? done : nullptr; p.done_step = done_step;
     p.tmp_out = (float*)workspace;
     p.tmp_ml  = p.tmp_out + rows * nh * p.P * kv->hd;
     hipStream_t st = (hipStream_t)stream;
     dim3 grid(p.P, kv->nkv, B * p.ntile);
 #define LI_(HD_, I8_, NT_, NW_, NG_, BF_, M_, R_) hipLaunchKernelGGL((paged_attn_kernel<HD_, I8_, NT_, NW_, NG_, BF_, M_, R_>), grid, dim3(64 * NW_), 0, st, p)
-#define LM_(HD_, I8_, NT_, NW_, NG_, BF_) do { if (p.done) LI_(HD_, I8_, NT_, NW_, NG_, BF_, true, false); else if (row_start) LI_(HD_, I8_, 2, NW_, 2, BF_, false, true); \
+#define LM_(HD_, I8_, NT_, NW_, NG_, BF_) do { if (p.done) LI_(HD_, I8_, 1, NW_, (I8_ ? 4 : 2), BF_, true, false); else if (row_start) LI_(HD_, I8_, 2, NW_, 2, BF_, false, true); \
                                               else LI_(HD_, I8_, NT_, NW_, NG_, BF_, false, false); } while (0)
 #define L_(HD_, I8_, NT_, NW_, NG_) LM_(HD_, I8_, NT_, NW_, NG_, false)
 #ifdef MI355_TUNING

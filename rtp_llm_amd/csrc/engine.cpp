@@ -10,7 +10,8 @@
 //
 // Launches per layer (tp = 1):
 //   * 5-64 rows (bf16 and per-channel W8: 1-64), W4 group-wise or W8 per-channel weights, 16-bit cache (rounds 4-5): SIX launches, activations handed over as fragment-ordered images
-//     (common.h act_img_index): QKV + bias + RoPE + KV write (gemm_fullk64.hip) -> paged attention (the partition that is done last merges) ->
+//     (common.h act_img_index): QKV + bias + RoPE + KV write (gemm_fullk64.hip) -> paged attention (partitions are
+//     merged by the one that is done last, by a launch of their own where a block has fewer threads than outputs) ->
 //     O + residual, leaving gamma 2^-e h' as an image and the sums of squares -> gate_up + SiLU with the RMSNorm finished on its
 //     accumulators (gemm_wide.hip) -> down as 4 K-quarters (gemm_splitk64.hip) -> fold: slabs + residual + RMSNorm -> image;
 //   * up to 4 rows every GEMM is a full-K launch with its consumer fused (gemm_fullk.hip), 5 launches:
