@@ -67,6 +67,12 @@ __device__ __forceinline__ size_t out_index(const AttnParams& p, int row, int co
 
 constexpr float NEG_BIG = -1e30f;
 
+// The block table, which no launch of this file writes, as constant memory: reads at a wave-uniform index are scalar loads then.  As global memory the compiler took vector loads for the
+// reads inside the loops, behind the loads of keys and values in the in-order counter, and each of them waited for everything in flight.  Us before / now, 28 over 4 heads of 128, 16-bit
+// cache, pages of 16: 36 sequences of 3225 tokens 62.2 / 52.1, 33 of 1500 32.8 / 27.7, 24 of 3225 40.6 / 36.7, 64 of 3225 83.1 / 77.4; 8-bit, 36 of 1000 16.6 / 15.0; 14 over 2 of 64, 64
+// of 3000 26.4 / 24.9; prompts: 8 x 512 rows 83.6 / 78.8, 16 x 512 over 16 heads of 64 52.0 / 44.4.
+typedef const __attribute__((address_space(4))) int32_t* table_ptr;
+
 // two floats written through to, read from where all XCDs see them
 __device__ __forceinline__ void put2(float* p, float a, float b) {
     __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, make_float2(a, b)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -116,7 +122,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
     // their table slots depend on the partition only.  Slots past a short context hold whatever the table holds -- the ids are
     // clamped where they are used and those tokens carry p = 0.  (They used to wait for seq_len: a second dependent round trip
     // in front of the first K/V request; tools/attn_stamps.py.)
-    const int32_t* bt = p.block_table + (size_t)b * p.max_blocks;
+    const table_ptr bt = (table_ptr)(uintptr_t)(p.block_table + (size_t)b * p.max_blocks);
     const int wave_pre = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int first_ids[4];
     {
@@ -638,7 +644,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
 // step.  Products transposed as there (a lane owns one row: its maximum, sum and rescaling are its own; the weights are the second product's operand where they
 // are: the keys of a step are handed to the first product in an order that leaves every lane eight consecutive ones).  16-byte pieces of a key row are swizzled by the
 // key, a value row (one channel, 32 tokens) is 64 bytes and needs none.
-// 8 x 512 rows, 28 over 4 heads of 128: 179 -> 86 us; 3 ragged of 389: 51 -> 29.
+// 8 x 512 rows, 28 over 4 heads of 128: 169 -> 79 us; 3 of 389: 51 -> 30.
 // What bounds it: a step of one wave, about 1.4 us of product, softmax and product in series whatever the depth of the staging (3 to 6 stages measured the same).
 constexpr int PR_STAGES = 3;
 template <int HD, bool BF>
@@ -675,7 +681,7 @@ __global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p,
     for (int db = 0; db < NDB; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float m = NEG_BIG, l = 0.f;
     if (klim > 0) {
-        const int32_t* bt = p.block_table + (size_t)b * p.max_blocks;
+        const table_ptr bt = (table_ptr)(uintptr_t)(p.block_table + (size_t)b * p.max_blocks);
         const int last = klim - 1, lastw = last & ~7, nsteps = (last >> 5) + 1;
         const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)pr_sm;
         auto page_of = [&](int t) { return (int)__builtin_amdgcn_readfirstlane((int)(((unsigned long long)(unsigned)t * p.page_magic) >> 32)); };
@@ -919,8 +925,8 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     while (p.G % HW) --HW;                                  // heads of a key/value head per block
     const int TW = 8 / HW, NW = HW * TW, JT = (kv->hd / 8 + NW - 1) / NW;
     // Prompt rows: where the rows fill the waves of about as many blocks as the chip has compute units (a third more where heads share no keys: a block then holds 128 rows of one
-    // head); with fewer the other kernel's smaller row tiles and split contexts win.  us there / here: 28 over 4 heads of 128, 8 x 512 rows 179 / 86, 3 x 352 72 / 52, 1 x 1500 137 /
-    // 106, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100, 37 x 20 behind 3477 188 / 250; 16 over 16 heads of 64, 16 x 34 behind 3628 75 / 117; 32 over 32 of 128, 38 x 23 behind
+    // head); with fewer the other kernel's smaller row tiles and split contexts win.  us there / here: 28 over 4 heads of 128, 8 x 512 rows 169 / 79, 3 x 352 72 / 52, 1 x 1500 108 /
+    // 92, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100, 37 x 20 behind 3477 188 / 250; 16 over 16 heads of 64, 16 x 34 behind 3628 75 / 117; 32 over 32 of 128, 38 x 23 behind
     // 3378 409 / 603.  Over 300 random calls the pick is 1.7 x faster than the other kernel, 3 of them slower (by up to a fifth, at contexts of thousands).
     if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)p.rows * nh >= 16L * NW * (HW == 1 ? 310 : 240) && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
         const dim3 grid(cdiv(q_len, 16 * TW), nh / HW, B);
