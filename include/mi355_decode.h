@@ -404,6 +404,11 @@ size_t mi355_sampling_probs_workspace_bytes(int32_t rows);
 int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
                          const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
                          int32_t step, void* workspace, mi355_stream_t stream);
+/* mi355_sampling_probs, then mi355_top_k_top_p_sample on the probabilities (which replace the logits): ids[row].  workspace: 16-byte aligned. */
+size_t mi355_sampling_draw_workspace_bytes(int32_t rows, int32_t V);
+int mi355_sampling_draw(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
+                        const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
+                        int32_t step, const int32_t* top_k, const float* top_p, const float* uniform_samples, int32_t* ids, void* workspace, mi355_stream_t stream);
 /* ids[r] = first index whose inclusive fp32 prefix sum of probs[r, :] (index order) exceeds uniform_samples[r] * sum --
  * sampling from the probabilities, the top_k = 0 / top_p = 1 branch of the sampler (bindings/core/CudaSampleOp.cc:702-737);
  * gives the target model's own sampled token per verify row (target_token_ids of mi355_rejection_sample). */

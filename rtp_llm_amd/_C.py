@@ -112,6 +112,8 @@ SIGNATURES = {
     "mi355_argmax": (i32, [vp, i32, i32, i32, vp, vp, sz, vp]),
     "mi355_sampling_probs_workspace_bytes": (sz, [i32]),
     "mi355_sampling_probs": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp]),
+    "mi355_sampling_draw_workspace_bytes": (sz, [i32, i32]),
+    "mi355_sampling_draw": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp, vp, vp, vp, vp]),
     "mi355_softmax_rows": (i32, [vp, i32, i32, i32, f32, vp, vp]),
     "mi355_sample_rows": (i32, [vp, i32, i32, i32, vp, vp, vp]),
     "mi355_apply_penalties": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp]),

@@ -10,11 +10,14 @@
 // One 1024-thread block per row: the accept chain is serial in one lane (gamma <= 16 dependent reads), the residual
 // draw is two passes over the vocabulary row (sum, then locate), each thread owning a contiguous segment so that the
 // block-level prefix over threads is the prefix over indices.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
 
 constexpr int kThreads = 1024;
+constexpr int kMostSplits = 16;              // blocks of a row at most, in the launches that split rows
 
 __device__ __forceinline__ float block_sum(float v, float* s_red) {
     v = wave_sum(v);
@@ -272,20 +275,30 @@ __device__ __forceinline__ float penalised(const PenaltyParams& p, int row, floa
 constexpr int kShortHistory = 2048;
 struct HistoryTable { int key[2 * kShortHistory], count[2 * kShortHistory]; };      // key -1: free
 
-// Penalises the history's ids in [lo, lo + n) once each, x = the row from lo on.  Whole block of NT threads; ends without a barrier.
+// A thread's entries of the row's history, -1: padding or none.
 template <int NT>
-__device__ __forceinline__ void penalise_history(const PenaltyParams& p, HistoryTable& t, int row, int id_step, int id_row, int lo, int n, float* x) {
-    const int tx = threadIdx.x;
-    int bits = 6;
-    while ((1 << bits) < 2 * p.step) ++bits;
+struct HistoryIds {
+    static constexpr int E = (kShortHistory + NT - 1) / NT;
+    int tok[E];
+    __device__ __forceinline__ void load(const PenaltyParams& p, int row, int id_step, int id_row) {
+        const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = threadIdx.x + e * NT;
+            tok[e] = i < p.step && !(i >= input_length && i < p.max_input_length) ? p.output_ids[(size_t)i * id_step + (size_t)row * id_row] : -1;
+        }
+    }
+};
+// Counts the ids in [lo, lo + n), 2^bits slots; seen(i) for each entry, i = its id - lo.  Whole block of NT threads; ends with a barrier.
+template <int NT, class Seen>
+__device__ __forceinline__ void count_history(const HistoryIds<NT>& ids, HistoryTable& t, int bits, int lo, int n, Seen&& seen) {
     const int size = 1 << bits;
-    for (int i = tx; i < size; i += NT) { t.key[i] = -1; t.count[i] = 0; }
+    for (int i = threadIdx.x; i < size; i += NT) { t.key[i] = -1; t.count[i] = 0; }
     __threadfence_block();
     __syncthreads();                                        // also: the row's scaling by other threads is done
-    const int input_length = p.input_lengths ? p.input_lengths[row] : p.max_input_length;
-    for (int i = tx; i < p.step; i += NT) {
-        if (i >= input_length && i < p.max_input_length) continue;                  // padding
-        const int tok = p.output_ids[(size_t)i * id_step + (size_t)row * id_row];
+#pragma unroll
+    for (int e = 0; e < HistoryIds<NT>::E; ++e) {
+        const int tok = ids.tok[e];
         if (tok < lo || tok >= lo + n) continue;
         int at = (int)(((uint32_t)tok * 2654435761u) >> (32 - bits));
         for (int probe = 0; probe < size; ++probe) {        // ends: there are more slots than entries
@@ -293,9 +306,36 @@ __device__ __forceinline__ void penalise_history(const PenaltyParams& p, History
             if (was == -1 || was == tok) { atomicAdd(&t.count[at], 1); break; }
             at = (at + 1) & (size - 1);
         }
+        seen(tok - lo);
     }
     __syncthreads();
-    for (int i = tx; i < size; i += NT) {
+}
+__device__ __forceinline__ int history_bits(int step) {
+    int bits = 6;
+    while ((1 << bits) < 2 * step) ++bits;
+    return bits;
+}
+// how often the id is in the history
+__device__ __forceinline__ int history_count(const HistoryTable& t, int bits, int tok) {
+    const int size = 1 << bits;
+    int at = (int)(((uint32_t)tok * 2654435761u) >> (32 - bits));
+    for (int probe = 0; probe < size; ++probe) {
+        const int key = t.key[at];
+        if (key == tok) return t.count[at];
+        if (key == -1) break;
+        at = (at + 1) & (size - 1);
+    }
+    return 0;
+}
+
+// Penalises the history's ids in [lo, lo + n) once each, x = the row from lo on.  Whole block of NT threads; ends without a barrier.
+template <int NT>
+__device__ __forceinline__ void penalise_history(const PenaltyParams& p, HistoryTable& t, int row, int id_step, int id_row, int lo, int n, float* x) {
+    const int bits = history_bits(p.step);
+    HistoryIds<NT> ids;
+    ids.load(p, row, id_step, id_row);
+    count_history<NT>(ids, t, bits, lo, n, [](int) {});
+    for (int i = threadIdx.x; i < 1 << bits; i += NT) {
         const int tok = t.key[i];
         if (tok >= 0) x[tok - lo] = penalised(p, row, x[tok - lo], t.count[i]);
     }
@@ -309,19 +349,80 @@ __global__ __launch_bounds__(NT) void penalties_short_kernel(const PenaltyParams
 
 // Temperature, penalties and softmax of the sampler in two launches, every row split over blocks.  One block per row, the softmax alone took 36 us of 64 rows of 152064 (its
 // three passes at what one CU pulls), behind 14 of temperature and 14 of penalties; the two take 29 and 11.
-// Prepare: a block scales its slice, penalises the history's ids that lie in it and leaves the slice's maximum and sum of exponentials.
+// A slice of up to kHeld aligned values stays in registers between its uses.  The history is counted while the slice is on its way; a bitmap names the fours with an id of it, whose
+// threads look their ids up.  64 rows of 152064: 24.7 us walked three times, with the penalties behind the scaled values in memory; held 22.4 (without the writing, and the same
+// again in the next launch: 18.6, and 18.3 there in place of 12.6).
+constexpr int kHeld = 20 * kThreads, kHeldRounds = kHeld / (4 * kThreads);
+struct HeldShared { HistoryTable table; uint32_t seen[kHeld / 128]; };      // a bit per four values
+struct HeldSlice {
+    f32x4 v[kHeldRounds];
+    float tail;                                                             // the last n % 4 values: threads 0 to 2
+    int n, n4;
+    __device__ __forceinline__ bool has(int i) const { return (int)threadIdx.x + i * kThreads < n4; }
+    __device__ __forceinline__ bool has_tail() const { return (n4 << 2) + (int)threadIdx.x < n; }
+    __device__ __forceinline__ void load(const PenaltyParams& p, HeldShared& sh, int row, int id_step, int id_row, int lo, float* x) {
+        const int tx = threadIdx.x, rest = (n4 << 2) + tx;
+        f32x4* x4 = reinterpret_cast<f32x4*>(x);
+        HistoryIds<kThreads> ids;                                           // in front of the slice: loads come back in order
+        if (p.output_ids) { ids.load(p, row, id_step, id_row); __builtin_amdgcn_sched_barrier(0); }
+#pragma unroll
+        for (int i = 0; i < kHeldRounds; ++i) v[i] = has(i) ? x4[tx + i * kThreads] : f32x4{0.f, 0.f, 0.f, 0.f};
+        tail = has_tail() ? x[rest] : 0.f;
+        const int bits = history_bits(p.step);
+        if (p.output_ids) {
+            for (int i = tx; i < kHeld / 128; i += kThreads) sh.seen[i] = 0u;
+            count_history<kThreads>(ids, sh.table, bits, lo, n, [&](int at) { atomicOr(&sh.seen[at >> 7], 1u << (at >> 2 & 31)); });
+        }
+        const float scale = p.temperature ? 1.0f / (p.temperature[row] + 1e-6f) : 1.f;
+        auto penalise = [&](float f, int at) { const int c = history_count(sh.table, bits, lo + at); return c ? penalised(p, row, f, c) : f; };
+#pragma unroll
+        for (int i = 0; i < kHeldRounds; ++i) {
+            const int j = tx + i * kThreads;
+            if (!has(i)) continue;
+            if (p.temperature) v[i] *= scale;
+            const bool seen = p.output_ids && (sh.seen[j >> 5] >> (j & 31) & 1u);
+            if (seen) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[i][r] = penalise(v[i][r], 4 * j + r);
+            }
+            if (p.temperature || seen) x4[j] = v[i];
+        }
+        if (has_tail()) {
+            if (p.temperature) tail *= scale;
+            if (p.output_ids) tail = penalise(tail, rest);
+            x[rest] = tail;
+        }
+    }
+};
+
+// Prepare: scales and penalises the slice, leaves its maximum and sum of exponentials.
+template <bool HELD>
 __global__ __launch_bounds__(kThreads) void sampling_prepare_kernel(const PenaltyParams p, float2* parts, int id_step, int id_row, int slice) {
-    __shared__ HistoryTable table;
+    __shared__ std::conditional_t<HELD, HeldShared, HistoryTable> sh;
     __shared__ float s_red[kThreads / 64];
     const int row = blockIdx.y, tx = threadIdx.x, lo = min(p.V, (int)blockIdx.x * slice), n = min(p.V, lo + slice) - lo;
     float* x = p.logits + (size_t)row * p.ld + lo;
     const bool vec = (p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;       // lo is a multiple of 4
-    if (p.temperature) scale_row(p, row, x, n, vec, tx, kThreads);
-    if (p.output_ids) penalise_history<kThreads>(p, table, row, id_step, id_row, lo, n, x);
-    __threadfence_block();
-    __syncthreads();
+    HeldSlice held;
+    if constexpr (HELD) {
+        held.n = n; held.n4 = n >> 2;
+        held.load(p, sh, row, id_step, id_row, lo, x);
+    } else {
+        if (p.temperature) scale_row(p, row, x, n, vec, tx, kThreads);
+        if (p.output_ids) penalise_history<kThreads>(p, sh, row, id_step, id_row, lo, n, x);
+        __threadfence_block();
+        __syncthreads();
+    }
+    auto each = [&](auto&& g) {
+        if constexpr (HELD) {
+#pragma unroll
+            for (int i = 0; i < kHeldRounds; ++i)
+                if (held.has(i)) { g(held.v[i][0]); g(held.v[i][1]); g(held.v[i][2]); g(held.v[i][3]); }
+            if (held.has_tail()) g(held.tail);
+        } else row_pass(x, n, vec, g);
+    };
     float m = -3.0e38f;
-    row_pass(x, n, vec, [&](float v) { m = fmaxf(m, v); });
+    each([&](float f) { m = fmaxf(m, f); });
     m = wave_max(m);
     if ((tx & 63) == 0) s_red[tx >> 6] = m;
     __syncthreads();
@@ -329,33 +430,56 @@ __global__ __launch_bounds__(kThreads) void sampling_prepare_kernel(const Penalt
     for (int w = 1; w < kThreads / 64; ++w) m = fmaxf(m, s_red[w]);
     __syncthreads();
     float s = 0.f;
-    row_pass(x, n, vec, [&](float v) { s += __expf(v - m); });
+    each([&](float f) { s += __expf(f - m); });
     s = block_sum(s, s_red);
     if (tx == 0) parts[(size_t)row * gridDim.x + blockIdx.x] = make_float2(m, s);
 }
 
-// Probabilities in place: exp(x - m) / sum from the slices' maxima and sums.
-__global__ __launch_bounds__(kThreads) void sampling_probs_kernel(float* logits, int V, int ld, const float2* parts, int slice) {
+// A probability's place among kDrawBins bins of a sixteenth of an octave down from 1, 0: below them (2^-32 and less, negative, NaN); and its exact value in units of 2^-56.
+constexpr int kDrawBins = 512, kDrawShift = 19, kDrawBase = (127 << 4) - (kDrawBins - 1);
+__device__ __forceinline__ int draw_bin(uint32_t b) { return min(max((int)(b >> kDrawShift) - kDrawBase, 0), kDrawBins - 1); }
+__device__ __forceinline__ unsigned long long draw_fixed(uint32_t b) { return (unsigned long long)((b & 0x7FFFFFu) | 0x800000u) << ((b >> 23) - 94u); }
+
+// Probabilities in place: exp(x - m) / sum from the slices' maxima and sums.  HIST: with a histogram of the slice's probabilities, count << 40 | sum of the bits below the bin's.
+template <bool HIST>
+__global__ __launch_bounds__(kThreads) void sampling_probs_kernel(float* logits, int V, int ld, const float2* parts, int slice, unsigned long long* hist) {
+    __shared__ unsigned long long s_hist[HIST ? kDrawBins : 1];
     const int row = blockIdx.y, tx = threadIdx.x, lo = min(V, (int)blockIdx.x * slice), n = min(V, lo + slice) - lo;
     float* x = logits + (size_t)row * ld + lo;
+    if (HIST) { for (int i = tx; i < kDrawBins; i += kThreads) s_hist[i] = 0ull; __syncthreads(); }
     const float2* pr = parts + (size_t)row * gridDim.x;
     float m = pr[0].x, s = 0.f;
     for (int i = 1; i < (int)gridDim.x; ++i) m = fmaxf(m, pr[i].x);
     for (int i = 0; i < (int)gridDim.x; ++i) s += pr[i].y * __expf(pr[i].x - m);
     const float inv = 1.f / s;
+    auto count = [&](float v) {
+        const uint32_t b = v > 0.f ? __float_as_uint(v) : 0u;
+        const int bin = draw_bin(b);
+        if (bin > 0) atomicAdd(&s_hist[bin], (1ull << 40) + (unsigned long long)(b & ((1u << kDrawShift) - 1u)));
+    };
+    auto four = [&](f32x4 v) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = __expf(v[r] - m) * inv;
+        if (HIST) { count(v[0]); count(v[1]); count(v[2]); count(v[3]); }
+        return v;
+    };
+    auto one = [&](float f) {
+        const float v = __expf(f - m) * inv;
+        if (HIST) count(v);
+        return v;
+    };
     int done = 0;
     if ((ld & 3) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0) {
         f32x4* x4 = reinterpret_cast<f32x4*>(x);
 #pragma unroll 4
-        for (int j = tx; j < n >> 2; j += kThreads) {
-            f32x4 v = x4[j];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = __expf(v[r] - m) * inv;
-            x4[j] = v;
-        }
+        for (int j = tx; j < n >> 2; j += kThreads) x4[j] = four(x4[j]);
         done = n & ~3;
     }
-    for (int j = done + tx; j < n; j += kThreads) x[j] = __expf(x[j] - m) * inv;
+    for (int j = done + tx; j < n; j += kThreads) x[j] = one(x[j]);
+    if constexpr (HIST) {
+        __syncthreads();
+        for (int i = tx; i < kDrawBins; i += kThreads) hist[((size_t)row * gridDim.x + blockIdx.x) * kDrawBins + i] = s_hist[i];
+    }
 }
 
 // Longer histories: counters in memory, cleared by the first of two launches.
@@ -759,9 +883,8 @@ __device__ __forceinline__ int search_histogram(const float* q, int V, bool vec,
     return ties <= 1u || above_q + (double)(mass + (unsigned long long)(ties - 1u) * mantissa(vbits)) * unit <= (double)tp ? 1 : 2;
 }
 
-__global__ __launch_bounds__(kThreads) void top_k_top_p_sample_kernel(const TopKPParams p) {
-    __shared__ SampleShared sh;
-    const int row = blockIdx.x, tx = threadIdx.x, V = p.V;
+__device__ __forceinline__ void sample_row(const TopKPParams& p, int row, SampleShared& sh) {
+    const int tx = threadIdx.x, V = p.V;
     const float* q = p.probs + (size_t)row * p.ld;
     const int k = p.top_k ? p.top_k[row] : 0;
     const bool use_k = k > 0 && k < V;
@@ -818,6 +941,238 @@ __global__ __launch_bounds__(kThreads) void top_k_top_p_sample_kernel(const TopK
             const float den = fmaxf(total, 1e-10f);
             for (int j = lo; j < hi; ++j) y[j] = kept(j) / den;
         });
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void top_k_top_p_sample_kernel(const TopKPParams p) {
+    __shared__ SampleShared sh;
+    sample_row(p, blockIdx.x, sh);
+}
+
+// The same behind sampling_probs_kernel<true>.  Its histograms name the bin that the higher of the two thresholds lies in, and give every slice's mass above it; the values of
+// that bin (1300 of 152064 where logits have a deviation of 2) are copied to the row's list by sampling_list_kernel, every row split over blocks as in the launches before.
+// draw_listed_kernel, one block per row, finds the threshold among them, with it every slice's mass and the slice that the draw falls into, and walks that slice alone.
+// Counts and masses are integers (units of 2^-56): exact, whatever the order.  Rows without such a bin (no filter, a threshold below 2^-32) or with more than kList values
+// in it take sample_row.
+// 64 rows of 152064, top-k 0..100, top-p 0.8..0.95: 103 us of top_k_top_p_sample_kernel (one compute unit pulls a row three times) -> 12.8 and 16.8.
+constexpr int kList = 8 * kThreads;
+
+struct DrawFilter { int k; bool use_k, use_p; float tp; };
+__device__ __forceinline__ DrawFilter draw_filter(const TopKPParams& p, int row) {
+    DrawFilter f;
+    f.k = p.top_k ? p.top_k[row] : 0;
+    f.use_k = f.k > 0 && f.k < p.V;
+    f.tp = p.top_p ? p.top_p[row] : 1.0f;
+    if (fabsf(f.tp) < 1e-7f) f.tp = 1.0f;
+    f.use_p = !(fabsf(f.tp - 1.0f) < 1e-7f);
+    return f;
+}
+// mass <= p as mass <= draw_limit(p), p >= 0
+__device__ __forceinline__ unsigned long long draw_limit(float tp) { return tp >= 64.f ? ~0ull >> 1 : (unsigned long long)((double)tp * 72057594037927936.0); }
+// The mass of c values that share the exponent and the four bits behind it, at = those, low = the sum of the bits below; c at most 2^20.  In 32 bits: of c times the whole mantissa
+// in 64 bits the compiler (hipcc 7.2) lost the mantissa's mask.
+__device__ __forceinline__ unsigned long long draw_mass(uint32_t at, uint32_t c, unsigned long long low) {
+    return (((unsigned long long)(c * (16u + (at & 15u))) << kDrawShift) + low) << ((at >> 4) - 94u);
+}
+
+struct DrawRow { int n; uint32_t low, above; unsigned long long mass; };        // values in the list (-1: none is made), their top bits, how many and how much lies above them
+
+struct DrawScan {                                                               // where the filter's thresholds cross, from the largest values down, a bin a thread
+    uint32_t c[kWaves];
+    unsigned long long m[kWaves];
+    int bin;
+};
+// ci / mi: the bin's count and mass with all above it, from c0 and m0 on.  Returns the higher crossing's bin (0 to `most`, -1: none).  Whole block.
+__device__ __forceinline__ int draw_cross(const DrawFilter& f, unsigned long long limit, int bin, uint32_t c, unsigned long long m, uint32_t c0, unsigned long long m0, uint32_t& ci,
+                                          unsigned long long& mi, bool& of_p, DrawScan& sc) {
+    const int tx = threadIdx.x, lane = tx & 63, wave = tx >> 6;
+    if (tx == 0) sc.bin = -1;
+    ci = c; mi = m;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t yc = __shfl_up(ci, o);
+        const unsigned long long ym = __shfl_up(mi, o);
+        if (lane >= o) { ci += yc; mi += ym; }
+    }
+    if (lane == 63) { sc.c[wave] = ci; sc.m[wave] = mi; }
+    __syncthreads();
+    ci += c0; mi += m0;
+    for (int w = 0; w < wave; ++w) { ci += sc.c[w]; mi += sc.m[w]; }
+    const bool of_k = f.use_k && ci - c < (uint32_t)f.k && ci >= (uint32_t)f.k;
+    of_p = f.use_p && mi - m <= limit && mi > limit;
+    if (bin >= 0 && (of_k || of_p)) atomicMax(&sc.bin, bin);
+    __syncthreads();
+    return sc.bin;
+}
+
+__global__ __launch_bounds__(kThreads) void sampling_list_kernel(const TopKPParams p, const unsigned long long* hist, int slice, DrawRow* rows, unsigned long long* above, uint2* list) {
+    __shared__ DrawScan sc;
+    __shared__ unsigned long long s_mass, s_above;
+    __shared__ uint32_t s_over;
+    __shared__ int s_n, s_base, s_at;
+    const int row = blockIdx.y, S = gridDim.x, tx = threadIdx.x, lane = tx & 63, wave = tx >> 6;
+    const DrawFilter f = draw_filter(p, row);
+    const unsigned long long* hr = hist + (size_t)row * S * kDrawBins;
+    if (tx == 0) { s_n = -1; s_base = 0; s_at = 0; s_above = 0; }
+    uint32_t c = 0, ci;
+    unsigned long long m = 0, mi, own = 0;                                      // the row's bin, what of its mass lies in this slice
+    bool of_p;
+    const int bin = kDrawBins - 1 - tx;
+    if (bin > 0) {
+        unsigned long long h = 0;
+#pragma unroll 4
+        for (int s = 0; s < S; ++s) h += hr[s * kDrawBins + bin];
+        c = (uint32_t)(h >> 40);
+        m = draw_mass((uint32_t)(bin + kDrawBase), c, h & ((1ull << 40) - 1ull));
+        h = hr[blockIdx.x * kDrawBins + bin];
+        own = draw_mass((uint32_t)(bin + kDrawBase), (uint32_t)(h >> 40), h & ((1ull << 40) - 1ull));
+    }
+    const bool negative = f.use_p && !(f.tp >= 0.f);
+    const int low = draw_cross(f, f.use_p && !negative ? draw_limit(f.tp) : 0ull, bin > 0 ? bin : -1, c, m, 0u, 0ull, ci, mi, of_p, sc);
+    if (bin == low && low > 0 && !negative && c <= (uint32_t)kList) { s_n = (int)c; s_over = ci - c; s_mass = mi - m; }
+    if (low > 0) {
+        own = wave_sum_u64(bin > low ? own : 0ull);
+        if (lane == 0 && own) atomicAdd(&s_above, own);
+    }
+    for (int s = wave; s < (int)blockIdx.x; s += kWaves)                        // where the slice's part of the list begins
+        if (lane == 0 && low > 0) atomicAdd(&s_base, (int)(hr[s * kDrawBins + low] >> 40));
+    __syncthreads();
+    if (tx == 0) {
+        if (blockIdx.x == 0) rows[row] = DrawRow{s_n, (uint32_t)(max(low, 0) + kDrawBase), s_over, s_mass};
+        above[(size_t)row * S + blockIdx.x] = s_above;
+    }
+    if (s_n < 0) return;
+    uint2* out = list + (size_t)row * kList + s_base;
+    const int lo = min(p.V, (int)blockIdx.x * slice), n = min(p.V, lo + slice) - lo;
+    const float* x = p.probs + (size_t)row * p.ld + lo;
+    const float least = __uint_as_float((uint32_t)(low + kDrawBase) << kDrawShift), next = __uint_as_float((uint32_t)(low + 1 + kDrawBase) << kDrawShift);
+    auto take = [&](float v, int j) {
+        if (v >= least && (v < next || low == kDrawBins - 1)) out[atomicAdd(&s_at, 1)] = make_uint2(__float_as_uint(v), (uint32_t)(lo + j));
+    };
+    int done = 0;
+    if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.probs) & 15) == 0) {
+        const f32x4* x4 = reinterpret_cast<const f32x4*>(x);
+#pragma unroll 4
+        for (int j = tx; j < n >> 2; j += kThreads) {
+            const f32x4 v = x4[j];
+            take(v[0], 4 * j); take(v[1], 4 * j + 1); take(v[2], 4 * j + 2); take(v[3], 4 * j + 3);
+        }
+        done = n & ~3;
+    }
+    for (int j = done + tx; j < n; j += kThreads) take(x[j], j);
+}
+
+__global__ __launch_bounds__(kThreads) void draw_listed_kernel(const TopKPParams p, int S, int slice, const DrawRow* rows, const unsigned long long* above, const uint2* list) {
+    __shared__ SampleShared sh;
+    __shared__ DrawScan sc;
+    __shared__ unsigned long long s_slice[kMostSplits], s_over;
+    __shared__ uint32_t s_ties, s_stay;
+    const int row = blockIdx.x, tx = threadIdx.x, lane = tx & 63, wave = tx >> 6;
+    const DrawRow r = rows[row];
+    if (r.n < 0) { sample_row(p, row, sh); return; }
+    const DrawFilter f = draw_filter(p, row);
+    const unsigned long long limit = f.use_p ? draw_limit(f.tp) : 0ull;
+    constexpr int PT = kList / kThreads, REST = 9;                              // values of a thread; bits behind the first 10 of the 19 that the list's values differ in
+    uint2 e[PT];
+#pragma unroll
+    for (int i = 0; i < PT; ++i) e[i] = tx + i * kThreads < r.n ? list[(size_t)row * kList + tx + i * kThreads] : make_uint2(0u, 0u);
+    sh.hist[tx] = 0ull; sh.hist[kThreads + tx] = 0ull;
+    if (tx < S) s_slice[tx] = above[(size_t)row * S + tx];
+    __syncthreads();
+    constexpr uint32_t LOW = (1u << kDrawShift) - 1u;
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+        if (e[i].x) atomicAdd(&sh.hist[(e[i].x & LOW) >> REST], (1ull << 40) + (unsigned long long)(e[i].x & LOW));
+    __syncthreads();
+    uint32_t ci;
+    unsigned long long mi;
+    bool of_p;
+    unsigned long long h = sh.hist[kThreads - 1 - tx];
+    uint32_t c = (uint32_t)(h >> 40);
+    unsigned long long m = draw_mass(r.low, c, h & ((1ull << 40) - 1ull));
+    const int first = draw_cross(f, limit, kThreads - 1 - tx, c, m, r.above, r.mass, ci, mi, of_p, sc);
+    if (kThreads - 1 - tx == first) { s_ties = ci - c; s_over = mi - m; }       // counted so far, and their mass
+    __syncthreads();
+    const uint32_t c1 = s_ties;
+    const unsigned long long m1 = s_over;
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+        if (e[i].x && (int)((e[i].x & LOW) >> REST) == first) atomicAdd(&sh.hist[kThreads + (e[i].x & ((1u << REST) - 1u))], 1ull);
+    __syncthreads();
+    const int bin = (1 << REST) - 1 - tx;
+    c = bin >= 0 ? (uint32_t)sh.hist[kThreads + bin] : 0u;
+    const uint32_t mine = r.low << kDrawShift | (uint32_t)(first << REST) | (uint32_t)max(bin, 0);      // the bits of the bin's value
+    m = c * draw_fixed(mine);
+    const int last = draw_cross(f, limit, bin, c, m, c1, m1, ci, mi, of_p, sc);
+    if (bin == last) {                                                          // equals of the boundary value: the j-th stays while S + j v <= p, S = the mass above it
+        s_ties = c;
+        s_stay = of_p ? (uint32_t)min((unsigned long long)c, (limit - (mi - m)) / draw_fixed(mine) + 1ull) : c;
+    }
+    __syncthreads();
+    const uint32_t bound = r.low << kDrawShift | (uint32_t)(first << REST) | (uint32_t)last, ties = s_ties, stay = s_stay;
+    uint32_t cut = (uint32_t)p.V;                                               // equals from this index on go
+    if (stay < ties) {                                                          // the largest index with at most `stay` of them in front of it
+        cut = 0;
+        for (int bit = 31 - __clz(p.V); bit >= 0; --bit) {
+            const uint32_t at = cut | 1u << bit;
+            uint32_t before = 0;
+#pragma unroll
+            for (int i = 0; i < PT; ++i) before += (uint32_t)__popcll(__ballot(e[i].x == bound && e[i].y < at));
+            if (lane == 0) sc.c[wave] = before;
+            __syncthreads();
+            before = 0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) before += sc.c[w];
+            __syncthreads();
+            if (before <= stay) cut = at;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+        if (e[i].x && (e[i].x > bound || (e[i].x == bound && e[i].y < cut))) atomicAdd(&s_slice[e[i].y / (uint32_t)slice], draw_fixed(e[i].x));
+    __syncthreads();
+    unsigned long long total = 0, front = 0;                                    // mass in front of the slice with the draw
+    for (int s = 0; s < S; ++s) total += s_slice[s];
+    const double u = (double)p.uniform[row] * (double)total;
+    int hit = 0;
+    while (hit < S && !((double)(front + s_slice[hit]) > u)) front += s_slice[hit++];
+    if (hit == S || !(u >= 0.0)) {
+        if (tx == 0) p.ids[row] = p.V - 1;
+        return;
+    }
+    // the slice: a contiguous run of it a thread, the runs' masses, their prefix, the run that u lies in
+    const int lo = hit * slice, end = min(p.V, lo + slice), run = ((slice / 4 + kThreads - 1) / kThreads) * 4, j0 = min(end, lo + tx * run), j1 = min(end, j0 + run);
+    const float* q = p.probs + (size_t)row * p.ld;
+    auto weight = [&](float v, int j) -> unsigned long long {
+        const uint32_t b = v > 0.f ? __float_as_uint(v) : 0u;
+        return b > bound || (b == bound && (uint32_t)j < cut) ? draw_fixed(b) : 0ull;
+    };
+    unsigned long long sum = 0;
+    int j = j0;
+    if ((p.ld & 3) == 0 && (reinterpret_cast<uintptr_t>(p.probs) & 15) == 0) {
+#pragma unroll 4
+        for (; j + 3 < j1; j += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(q + j);
+            sum += (weight(v[0], j) + weight(v[1], j + 1)) + (weight(v[2], j + 2) + weight(v[3], j + 3));
+        }
+    }
+    for (; j < j1; ++j) sum += weight(q[j], j);
+    unsigned long long incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+    }
+    if (lane == 63) sc.m[wave] = incl;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) incl += sc.m[w];
+    incl += front;
+    if (sum && !((double)(incl - sum) > u) && (double)incl > u) {
+        unsigned long long at = incl - sum;
+        for (j = j0; j < j1; ++j) {
+            at += weight(q[j], j);
+            if ((double)at > u) { p.ids[row] = j; break; }
+        }
     }
 }
 
@@ -898,15 +1253,14 @@ extern "C" int mi355_rejection_sample(const float* draft_probs, const int32_t* d
 
 // Blocks of a row: about one block per compute unit in all, none with less than a pass of its threads.  Temperature alone, us with 1 / 2 / 4 / 8 / 16 blocks a row:
 // 1 x 152064 11.9 / 6.6 / 4.3 / 3.2 / 2.7, 64 x 152064 18.3 / 12.5 / 11.6 / 12.2 / 12.4, 64 x 6952 2.8 / 2.8 / 2.9 / 3.6 / 4.5, 237 x 32000 8.3 / 8.2 / 8.8 / 9.6 / 13.1.
-constexpr int kMostSplits = 16;
 static int row_splits(int rows, int V) {
     const int most = rows >= 256 ? 1 : 256 / rows < kMostSplits ? 256 / rows : kMostSplits, full = (V + 4 * kThreads - 1) / (4 * kThreads);
     return most < full ? most : full;
 }
-// The joint launches walk a slice three times: of long rows more blocks, so that a slice of 64 KB stays near its compute unit.  Us with row_splits / these: 64 x 152064 31.7 / 28.1,
-// 237 x 152064 127.5 / 97.8; 237 x 32000 21.7 / 30.0 with 8 blocks a row, 237 x 1695 7.2 / 20.7.
+// The joint launches: of long rows as many blocks as hold their slices in registers.  64 x 152064, us of prepare, probabilities and list with 8 blocks a row (one round of two a compute
+// unit) 21.8 + 12.7 + 12.9, with 9 24.2 + 14.8 + 14.3; with 4, walked from memory, the first two took 31.7 before against 28.1 with 9.
 static int joint_splits(int rows, int V) {
-    const int least = row_splits(rows, V), near = V / 16384 < kMostSplits ? V / 16384 : kMostSplits;
+    const int least = row_splits(rows, V), held = (V + kHeld - 1) / kHeld, near = held < kMostSplits ? held : kMostSplits;
     return least > near ? least : near;
 }
 
@@ -943,6 +1297,20 @@ extern "C" int mi355_apply_penalties(float* logits, int32_t batch_size, int32_t 
     return MI355_OK;
 }
 
+namespace {
+template <bool HIST>
+int launch_probs(const PenaltyParams& p, void* parts, int id_step, int id_row, int S, int slice, unsigned long long* hist, hipStream_t st) {
+    const dim3 grid(S, p.batch), block(kThreads);
+    const bool held = slice <= kHeld && p.ld % 4 == 0 && (uintptr_t)p.logits % 16 == 0;
+    if (held) hipLaunchKernelGGL(sampling_prepare_kernel<true>, grid, block, 0, st, p, (float2*)parts, id_step, id_row, slice);
+    else      hipLaunchKernelGGL(sampling_prepare_kernel<false>, grid, block, 0, st, p, (float2*)parts, id_step, id_row, slice);
+    MI355_CHECK_LAUNCH("sampling_prepare_kernel");
+    hipLaunchKernelGGL(sampling_probs_kernel<HIST>, grid, block, 0, st, p.logits, p.V, p.ld, (const float2*)parts, slice, hist);
+    MI355_CHECK_LAUNCH("sampling_probs_kernel");
+    return MI355_OK;
+}
+} // namespace
+
 extern "C" size_t mi355_sampling_probs_workspace_bytes(int32_t rows) { return rows > 0 ? (size_t)rows * kMostSplits * sizeof(float2) : 0; }
 
 extern "C" int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
@@ -953,10 +1321,46 @@ extern "C" int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int3
     const bool pen = output_ids && step > 0 && (repetition || presence || frequency);
     const int S = joint_splits(rows, V), slice = ((V + S - 1) / S + 3) & ~3;
     const PenaltyParams p{logits, V, ld, temperature, repetition, presence, frequency, pen ? output_ids : nullptr, input_lengths, rows, max_input_length, step, nullptr};
-    hipLaunchKernelGGL(sampling_prepare_kernel, dim3(S, rows), dim3(kThreads), 0, (hipStream_t)stream, p, (float2*)workspace, id_step, id_row, slice);
-    MI355_CHECK_LAUNCH("sampling_prepare_kernel");
-    hipLaunchKernelGGL(sampling_probs_kernel, dim3(S, rows), dim3(kThreads), 0, (hipStream_t)stream, logits, V, ld, (const float2*)workspace, slice);
-    MI355_CHECK_LAUNCH("sampling_probs_kernel");
+    return launch_probs<false>(p, workspace, id_step, id_row, S, slice, nullptr, (hipStream_t)stream);
+}
+
+// mi355_sampling_probs and mi355_top_k_top_p_sample (without its probabilities) in one: the logits become the probabilities, ids[row] is drawn from what the filter leaves.
+namespace {
+struct DrawWorkspace { size_t hist, above, list, listed, bytes; };                     // the slices' (maximum, sum) lie in front
+DrawWorkspace draw_workspace(int rows, int S) {
+    DrawWorkspace w;
+    w.hist = ((size_t)rows * kMostSplits * sizeof(float2) + 15) & ~(size_t)15;
+    w.above = w.hist + (size_t)rows * S * kDrawBins * sizeof(unsigned long long);
+    w.list = w.above + (size_t)rows * S * sizeof(unsigned long long);
+    w.listed = w.list + (size_t)rows * kList * sizeof(uint2);
+    w.bytes = w.listed + (size_t)rows * sizeof(DrawRow);
+    return w;
+}
+} // namespace
+extern "C" size_t mi355_sampling_draw_workspace_bytes(int32_t rows, int32_t V) { return rows > 0 && V > 0 ? draw_workspace(rows, joint_splits(rows, V)).bytes : 0; }
+
+extern "C" int mi355_sampling_draw(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
+                                   const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
+                                   int32_t step, const int32_t* top_k, const float* top_p, const float* uniform_samples, int32_t* ids, void* workspace, mi355_stream_t stream) {
+    MI355_CHECK_ARG(logits && workspace && rows > 0 && V > 0 && ld >= V && step >= 0 && (uintptr_t)workspace % 16 == 0 && uniform_samples && ids, "sampling_draw: bad args");
+    if (V > 1 << 20) {                                                          // the packed sums of a bin
+        if (int e = mi355_sampling_probs(logits, rows, V, ld, temperature, repetition, presence, frequency, output_ids, id_step, id_row, input_lengths, max_input_length, step, workspace, stream)) return e;
+        return mi355_top_k_top_p_sample(logits, rows, V, ld, top_k, top_p, uniform_samples, ids, nullptr, 0, stream);
+    }
+    if (output_ids && step > kShortHistory) return MI355_ERR_UNSUPPORTED;
+    const bool pen = output_ids && step > 0 && (repetition || presence || frequency);
+    const int S = joint_splits(rows, V), slice = ((V + S - 1) / S + 3) & ~3;
+    const DrawWorkspace w = draw_workspace(rows, S);
+    char* ws = (char*)workspace;
+    hipStream_t st = (hipStream_t)stream;
+    const PenaltyParams p{logits, V, ld, temperature, repetition, presence, frequency, pen ? output_ids : nullptr, input_lengths, rows, max_input_length, step, nullptr};
+    if (int e = launch_probs<true>(p, workspace, id_step, id_row, S, slice, (unsigned long long*)(ws + w.hist), st)) return e;
+    const TopKPParams t{logits, V, ld, top_k, top_p, uniform_samples, ids, nullptr, 0};
+    auto* above = (unsigned long long*)(ws + w.above);
+    hipLaunchKernelGGL(sampling_list_kernel, dim3(S, rows), dim3(kThreads), 0, st, t, (const unsigned long long*)(ws + w.hist), slice, (DrawRow*)(ws + w.listed), above, (uint2*)(ws + w.list));
+    MI355_CHECK_LAUNCH("sampling_list_kernel");
+    hipLaunchKernelGGL(draw_listed_kernel, dim3(rows), dim3(kThreads), 0, st, t, S, slice, (const DrawRow*)(ws + w.listed), above, (const uint2*)(ws + w.list));
+    MI355_CHECK_LAUNCH("draw_listed_kernel");
     return MI355_OK;
 }
 

@@ -500,6 +500,22 @@ def apply_penalties(logits: torch.Tensor, temperature: Optional[torch.Tensor] = 
     return logits
 
 
+def _sampling_vectors(what, logits, floats, token_ids, ints, step) -> int:
+    """Checks the vectors of the joint sampler launches; the row stride of the history."""
+    B = logits.shape[0]
+    for t, dt in [(t, torch.float32) for t in floats] + [(t, torch.int32) for t in ints]:
+        if t is not None:
+            _chk(t, dt, what)
+            if t.numel() != B:
+                raise _C.Mi355Error(f"{what}: one value per row")
+    if token_ids is None:
+        return 0
+    _chk(token_ids, torch.int32, f"{what}.token_ids")
+    if token_ids.dim() != 2 or token_ids.shape[0] != B or token_ids.shape[1] < step:
+        raise _C.Mi355Error(f"{what}: token_ids must be [B, >= step]")
+    return token_ids.shape[1]
+
+
 def sampling_probs(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None, repetition_penalty: Optional[torch.Tensor] = None,
                    presence_penalty: Optional[torch.Tensor] = None, frequency_penalty: Optional[torch.Tensor] = None, token_ids: Optional[torch.Tensor] = None,
                    input_lengths: Optional[torch.Tensor] = None, max_input_length: int = 0, step: int = 0) -> torch.Tensor:
@@ -507,23 +523,34 @@ def sampling_probs(logits: torch.Tensor, temperature: Optional[torch.Tensor] = N
     history is token_ids [B, >= step] int32, step <= 2048."""
     _chk(logits, torch.float32, "sampling_probs.logits")
     B, V = logits.shape
-    for t, dt in ((temperature, torch.float32), (repetition_penalty, torch.float32), (presence_penalty, torch.float32), (frequency_penalty, torch.float32), (input_lengths, torch.int32)):
-        if t is not None:
-            _chk(t, dt, "sampling_probs")
-            if t.numel() != B:
-                raise _C.Mi355Error("sampling_probs: one value per row")
-    if token_ids is not None:
-        _chk(token_ids, torch.int32, "sampling_probs.token_ids")
-        if token_ids.dim() != 2 or token_ids.shape[0] != B or token_ids.shape[1] < step:
-            raise _C.Mi355Error("sampling_probs: token_ids must be [B, >= step]")
-    elif repetition_penalty is not None or presence_penalty is not None or frequency_penalty is not None:
+    stride = _sampling_vectors("sampling_probs", logits, (temperature, repetition_penalty, presence_penalty, frequency_penalty), token_ids, (input_lengths,), step)
+    if token_ids is None and (repetition_penalty is not None or presence_penalty is not None or frequency_penalty is not None):
         raise _C.Mi355Error("sampling_probs: penalties need the token history token_ids [B, step]")
     lib = _C.lib()
     ws = torch.empty(max(8, lib.mi355_sampling_probs_workspace_bytes(B)), dtype=torch.uint8, device=logits.device)
     _C.check(lib.mi355_sampling_probs(logits.data_ptr(), B, V, V, _p(temperature), _p(repetition_penalty), _p(presence_penalty), _p(frequency_penalty), _p(token_ids),
-                                      1, 0 if token_ids is None else token_ids.shape[1], _p(input_lengths), int(max_input_length), int(step), ws.data_ptr(), _stream()),
+                                      1, stride, _p(input_lengths), int(max_input_length), int(step), ws.data_ptr(), _stream()),
              "sampling_probs")
     return logits
+
+
+def sampling_draw(logits: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Optional[torch.Tensor], uniform: torch.Tensor, temperature: Optional[torch.Tensor] = None,
+                  repetition_penalty: Optional[torch.Tensor] = None, presence_penalty: Optional[torch.Tensor] = None, frequency_penalty: Optional[torch.Tensor] = None,
+                  token_ids: Optional[torch.Tensor] = None, input_lengths: Optional[torch.Tensor] = None, max_input_length: int = 0, step: int = 0) -> torch.Tensor:
+    """sampling_probs in place on the logits, then top_k_top_p_sample on the probabilities, in four launches -> ids [B] int32.  All vectors as sampling_probs takes them."""
+    _chk(logits, torch.float32, "sampling_draw.logits")
+    B, V = logits.shape
+    stride = _sampling_vectors("sampling_draw", logits, (temperature, repetition_penalty, presence_penalty, frequency_penalty, top_p, uniform), token_ids,
+                               (input_lengths, top_k), step)
+    if token_ids is None and (repetition_penalty is not None or presence_penalty is not None or frequency_penalty is not None):
+        raise _C.Mi355Error("sampling_draw: penalties need the token history token_ids [B, step]")
+    lib = _C.lib()
+    ws = torch.empty(lib.mi355_sampling_draw_workspace_bytes(B, V), dtype=torch.uint8, device=logits.device)
+    ids = torch.empty(B, dtype=torch.int32, device=logits.device)
+    _C.check(lib.mi355_sampling_draw(logits.data_ptr(), B, V, V, _p(temperature), _p(repetition_penalty), _p(presence_penalty), _p(frequency_penalty), _p(token_ids),
+                                     1, stride, _p(input_lengths), int(max_input_length), int(step), _p(top_k), _p(top_p), uniform.data_ptr(), ids.data_ptr(),
+                                     ws.data_ptr(), _stream()), "sampling_draw")
+    return ids
 
 
 def ban_repeat_ngram(logits: torch.Tensor, token_ids: torch.Tensor, sequence_last_index: torch.Tensor,

@@ -123,6 +123,11 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
         if penalise:
             vectors = dict(repetition_penalty=up["rep"], presence_penalty=up["pres"], frequency_penalty=up["freq"], input_lengths=up["lengths"], max_input_length=step + 1,
                            step=step + 1, token_ids=up["history"] if "history" in up else params.token_ids.to(device=dev, dtype=torch.int32).contiguous())
+        if not all_greedy and params.output_all_probs is None:                            # and the draw behind them
+            u = up["uniform"] if "uniform" in up else params.uniform.to(device=dev, dtype=torch.float32).contiguous()
+            ids = ops.sampling_draw(logits, up["top_k"], up["top_p"], u, up.get("temperature"), **vectors)
+            params.token_ids[:, step] = ids.to(params.token_ids.device)
+            return ids
         probs = ops.sampling_probs(logits, up.get("temperature"), **vectors)
     else:
         if scale:

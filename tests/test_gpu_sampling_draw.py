@@ -1,0 +1,59 @@
+"""The sampler's four joint launches against its two separate ones (softmax of the penalised logits, then the filter and the draw on whole rows)."""
+import pytest
+import torch
+
+from rtp_llm_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _logits(kind, B, V, g):
+    x = torch.randn(B, V, device=DEV, generator=g) * 2.0
+    if kind == "peaked":                      # a few dozen candidates above a bulk
+        n = min(V, 48)
+        x.scatter_(1, torch.rand(B, V, device=DEV, generator=g).topk(n).indices, 8.0 + 2.5 * torch.randn(B, n, device=DEV, generator=g))
+    elif kind == "flat":                      # more values than a list holds
+        x *= 0.05
+    elif kind == "ties":
+        x = x.round()
+    elif kind == "masked":                    # -inf and the type's lowest value beside few finite ones
+        x[torch.rand(B, V, device=DEV, generator=g) < 0.5] = float("-inf")
+        x[torch.rand(B, V, device=DEV, generator=g) < 0.5] = torch.finfo(torch.float32).min
+        x[:, V // 2] = 3.0
+    elif kind == "spike":                     # one token has all the mass that a float holds
+        x[:, V // 3] = 200.0
+    return x
+
+
+# rows of one slice and of sixteen, slices held in registers (up to 20480 values) and walked, rows off 16 bytes, a vocabulary below one load
+@pytest.mark.parametrize("B,V", [(1, 7), (3, 1000), (2, 8191), (5, 32001), (1, 152064), (64, 20484), (300, 4099), (2, 400003)])
+@pytest.mark.parametrize("kind", ["peaked", "flat", "ties", "masked", "spike"])
+def test_joint_draw_equals_separate_launches(B, V, kind):
+    g = torch.Generator(device=DEV).manual_seed(B * 1000 + V)
+    x = _logits(kind, B, V, g)
+    pick = lambda values, dt: torch.tensor(values, dtype=dt, device=DEV)[torch.randint(0, len(values), (B,), device=DEV, generator=g)]
+    k, p = pick([0, 1, 7, 50, 3000, V], torch.int32), pick([0.0, 0.3, 0.8, 0.95, 0.999999, 1.0, -0.5], torch.float32)
+    u = torch.rand(B, device=DEV, generator=g) * 0.996 + 0.002
+    hist = torch.randint(-1, V + 2, (B, 40), dtype=torch.int32, device=DEV, generator=g)
+    pen = dict(repetition_penalty=pick([1.0, 1.2], torch.float32), presence_penalty=pick([0.0, 0.4], torch.float32), frequency_penalty=pick([0.0, 0.1], torch.float32),
+               token_ids=hist, input_lengths=torch.full((B,), 40, dtype=torch.int32, device=DEV), max_input_length=40, step=40)
+    for t, kw in ((None, {}), (pick([0.6, 1.0], torch.float32), pen)):
+        want = ops.sampling_probs(x.clone(), t, **kw)
+        want_ids = ops.top_k_top_p_sample(want, k, p, u)
+        got = x.clone()
+        ids = ops.sampling_draw(got, k, p, u, t, **kw)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), "the probabilities are the same launch's"
+        # a draw may land on the neighbour where the fp32 sums of whole rows and the exact ones of the list differ in the last bit; none does at these seeds
+        assert torch.equal(ids, want_ids), (k[ids != want_ids], p[ids != want_ids])
+
+
+def test_joint_draw_takes_kept_tokens_only():
+    """Uniforms at both ends of the range: the first and the last token that the filter keeps, of a row with a known order."""
+    V, B = 5000, 4
+    x = torch.full((B, V), -20.0, device=DEV)
+    x[:, 1234], x[:, 77], x[:, 4000], x[:, 9] = 5.0, 4.0, 3.0, 2.0
+    k = torch.tensor([3, 3, 0, 0], dtype=torch.int32, device=DEV)
+    p = torch.tensor([1.0, 1.0, 0.85, 0.85], device=DEV)          # 0.644, 0.237, 0.087, 0.032: the third starts above 0.85
+    u = torch.tensor([0.0, 0.9999999, 0.0, 0.9999999], device=DEV)
+    assert ops.sampling_draw(x, k, p, u).tolist() == [77, 4000, 77, 1234]
