@@ -14,6 +14,9 @@
 // One ragged batch of rows serves prefill portions and decode tokens alike: every row carries its position and the index of its
 // sequence; a sequence carries its block-table row, its state slot and the range of its rows.  What the model states as 32-bit is fp32
 // here whatever the activation type T (bf16 or float): positions and angles, scores and softmax, norms, gates, decays, states, residual.
+#include <algorithm>
+#include <cstdlib>
+
 #include "common.h"
 #include "../../include/mi355_hybrid.h"
 
@@ -841,10 +844,11 @@ __global__ __launch_bounds__(256) void hy_attn_merge_kernel(const float* parts, 
 // Key and value rows come by DMA into three LDS stages, two steps ahead, pieces of 16 bytes swizzled by the key so that fragment reads meet no bank twice; values are read
 // through the transposing LDS load.  One barrier a step.  A latent cache (one row that is key and, with its leading channels, value) is staged once.
 // What bounded the kernel before was the chain of a step: one wave per SIMD (234 to 512 registers, keys and values of the next step in them), page lookups, a transpose
-// through 2-byte LDS writes, 16-lane reductions and two barriers in series: 2.8 us per 32 keys at 128 channels, 6 us at 256.  Before / now, 16 query over 4 key heads of
-// 128: 4 x 2048 rows under a block mask of 1024 319 / 176 us, 8 x 96 rows 26 / 15 us; 8 heads over a latent row of 256 (192), 1537 rows: 281 / 98 us; 8 heads of
-// 128 without sharing, 2048 rows: 294 / 100 us; 2 x 1024 rows, 28 over 4: 335 / 113 us.  What bounds it now: a wave's own chain of products, softmax and products, with
-// two or three waves on a SIMD; the matrix units alone would take 30 us of the 176.
+// through 2-byte LDS writes, 16-lane reductions and two barriers in series: 2.8 us per 32 keys at 128 channels, 6 us at 256.  Then the addresses of the DMA, a page lookup and
+// 64-bit products a lane and load (a step inside one page takes one of the scalar unit: 100 -> 84 us below), and LDS latencies between fragments and their products
+// (84 -> 76).  First / before these / now, 8 heads over a latent row of 256 (192), 1537 rows: 281 / 100 / 55 us with two groups of waves on the keys; 16 query over 4 key
+// heads of 128, 4 x 2048 rows under a block mask of 1024 319 / 172 / 157, 8 x 100 rows 26 / 12.8 / 10.8.  What bounds it now: a wave's own chain of products, softmax and
+// products, with two or three waves on a SIMD; the matrix units alone would take 30 us of the 157.
 __device__ __forceinline__ void hy_split_bf16(float x, bf16& hi, bf16& lo) { hi = (bf16)x; lo = (bf16)(x - (float)hi); }
 // reductions over the 16 lanes of a DPP row: quad swaps, then the half-row and row mirrors
 template <int CTRL> __device__ __forceinline__ float hy_dpp(float v) {
@@ -876,13 +880,15 @@ constexpr int AT_STAGES = 3, AT_PAGES = 1024;     // block-table entries of the 
 
 // DK: 32-channel steps of a key row.  NCBM: 16-channel fragments of a value row the instance holds; they are multiplied by fours (fragments past the row's end hold what lies
 // behind it in LDS and are never stored).
+// KG groups of four waves share a block's tiles: group k takes the steps st with st % KG == k, into stages of its own, and their maxima, denominators and sums meet in LDS.
+constexpr int at_groups(int DK, int NCBM) { return DK >= 5 && NCBM == 16 ? 1 : 2; }                  // most of them: the instances with 16 value fragments take more than 256 registers
 template <int DK, int NCBM>
-__global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_tiles_kernel(const float* q, int ldq, float scale, AttnGeom g, int chunk, const float* sink, const float* vfreq,
+__global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3 : at_groups(DK, NCBM)) void hy_attn_tiles_kernel(const float* q, int ldq, float scale, AttnGeom g, int chunk, const float* sink, const float* vfreq,
                                                                            const int32_t* pos, const int32_t* seq, const int32_t* block_table, const int32_t* tile_row0,
                                                                            const int32_t* tile_n, int ntiles, const bf16* kcache, const bf16* vcache, bf16* out, AttnExtra ex,
-                                                                           int HW, int same, int vec) {
-    extern __shared__ __attribute__((aligned(16))) char at_sm[];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
+                                                                           int HW, int same, int vec, int KG) {
+    extern __shared__ __attribute__((aligned(16))) char at_smem[];
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6 & 3), lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
     const int TW = 4 / HW, h = blockIdx.y * HW + wave % HW, tw = wave / HW;
     const int kvh = (int)blockIdx.y * HW / (g.H / g.G);
     const int NCB = g.vdim / 16;
@@ -891,11 +897,12 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
     const int CV = same ? CK : NCB * 2, JV = same ? 0 : (CV + 7) / 8;
     const int mk = ((CK & -CK) - 1) & 15, mv = same ? mk : ((CV & -CV) - 1) & 15;
     const int kbytes = JK * 4096, stage = kbytes + JV * 4096;
-    int32_t* bt_s = (int32_t*)(at_sm + AT_STAGES * stage);
+    int32_t* bt_s = (int32_t*)(at_smem + KG * AT_STAGES * stage);
+    char* at_sm = at_smem + group * AT_STAGES * stage;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)at_sm;
     // long (late) tiles of a prompt first
     const int first_tile = ((int)gridDim.x - 1 - (int)blockIdx.x) * TW, ntw = min(TW, ntiles - first_tile);
-    const bool has = tw < ntw;
+    bool has = tw < ntw;
     const int tile = first_tile + min(tw, ntw - 1), r0 = __builtin_amdgcn_readfirstlane(tile_row0[tile]), n = __builtin_amdgcn_readfirstlane(tile_n[tile]);
     const int p0 = __builtin_amdgcn_readfirstlane(pos[r0]), plast = p0 + n - 1;
     const int psh = (g.page & (g.page - 1)) == 0 ? __builtin_ctz(g.page) : -1;       // page size a power of two: shifts instead of divisions
@@ -919,7 +926,8 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
 #pragma unroll
         for (int i = 0; i < 8; ++i) { bf16 a, b; hy_split_bf16(v[i] * scale2, a, b); qh[ks][i] = a; ql[ks][i] = b; }
     }
-    float m = sink ? sink[h] * 1.44269504088896340736f : -INFINITY, l = sink && lq == 0 ? 1.f : 0.f;      // l: the lane's share of the row's denominator
+    const bool sunk = sink && group == 0;
+    float m = sunk ? sink[h] * 1.44269504088896340736f : -INFINITY, l = sunk && lq == 0 ? 1.f : 0.f;      // l: the lane's share of the row's denominator
     f32x4 o[NCBM];                                            // fragment element e: channel cb * 16 + 4 lq + e of row lr
 #pragma unroll
     for (int cb = 0; cb < NCBM; ++cb) o[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -937,6 +945,16 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
         const int slot = (j * 4 + wave) * 64 + lane, key = min(slot / CV, 31), c = slot % CV;
         vpiece[j] = key | (c ^ (key & mv)) << 8;
     }
+    // A step of 32 keys that lie in one page: the page's address is the scalar unit's, a lane's offsets from it stay.
+    const bool whole = (vec & 2) && g.page % 32 == 0;
+    uint32_t koff[JK], voff[JVM];
+#pragma unroll
+    for (int j = 0; j < JK; ++j) {
+        const int slot = (j * 4 + wave) * 64 + lane, key = min(slot / CK, 31), c = slot % CK;
+        koff[j] = (uint32_t)(key * g.dim + ((c ^ (key & mk)) << 3)) * 2u;
+    }
+#pragma unroll
+    for (int j = 0; j < JVM; ++j) voff[j] = (uint32_t)((vpiece[j] & 31) * g.v_ld + (vpiece[j] >> 5)) * 2u;
     // the tiles of the block in runs of one sequence (one run unless a block's tiles belong to several): the run's keys are staged for all its tiles
     for (int ft = 0; ft < ntw;) {
         const int fr = tile_row0[first_tile + ft], sq = seq[fr];
@@ -957,19 +975,35 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
         auto step_key = [&](int st) { return (st < nkept ? 0 : kstart - 32 * nkept) + 32 * st; };
         auto page_of = [&](int k) { return psh >= 0 ? k >> psh : k / g.page; };
         int bt0 = INT_MIN;                                    // first block-table entry in LDS
-        auto issue = [&](int st, int buf) {
-            const int t0 = step_key(st), plo = page_of(t0), phi = page_of(min(t0 + 31, klast));
+        const int rounds = (nsteps + KG - 1) / KG;
+        auto issue = [&](int round, int buf) {                // KG steps, one a group (several only without kept tokens: their keys follow each other)
+            const int plo = page_of(step_key(round * KG)), phi = page_of(min(step_key(round * KG) + 32 * KG - 1, klast));
             if (bt0 == INT_MIN || plo < bt0 || phi >= bt0 + AT_PAGES) {        // seldom: the same for the whole block
                 __syncthreads();
                 bt0 = plo;
-                for (int i = threadIdx.x; i < AT_PAGES; i += 256) if (bt0 + i <= page_of(klast)) bt_s[i] = bt[bt0 + i];
+                for (int i = threadIdx.x; i < AT_PAGES; i += 256 * KG) if (bt0 + i <= page_of(klast)) bt_s[i] = bt[bt0 + i];
                 __syncthreads();
+            }
+            if (round * KG + group >= nsteps) return;
+            const int t0 = step_key(round * KG + group);
+            const uint32_t base = buf * stage + wave * 1024;
+            if (whole && t0 + 31 <= klast) {
+                const int pi = page_of(t0), po = psh >= 0 ? t0 & (g.page - 1) : t0 - pi * g.page;
+                const size_t first = (size_t)(__builtin_amdgcn_readfirstlane(bt_s[pi - bt0]) * g.G + kvh) * g.page + po;
+                const uint32_t to = __builtin_amdgcn_readfirstlane(lds0 + base);
+#pragma unroll
+                for (int j = 0; j < JK; ++j) dma16(to + j * 4096, koff[j], kcache + first * g.dim);
+#pragma unroll
+                for (int j = 0; j < JVM; ++j) {
+                    if (j >= JV) break;
+                    dma16(to + kbytes + j * 4096, voff[j], vcache + first * g.v_ld);
+                }
+                return;
             }
             auto row = [&](int key) {
                 const int kc = min(t0 + key, klast), pi = page_of(kc), po = psh >= 0 ? kc & (g.page - 1) : kc - pi * g.page;
                 return (size_t)(bt_s[pi - bt0] * g.G + kvh) * g.page + po;
             };
-            const uint32_t base = buf * stage + wave * 1024;
             auto piece = [&](uint32_t at, const bf16* src) {
                 if (vec & 2) { dma16(lds0 + at, src); return; }
                 bf16x8 v;                                     // a cache that is not on 16 bytes
@@ -990,28 +1024,48 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
         };
         __syncthreads();                                      // the stages and bt_s are free
         issue(0, 0);
-        if (nsteps > 1) issue(1, 1);
+        if (rounds > 1) issue(1, 1);
         int buf = 0;
-        for (int st = 0; st < nsteps; ++st) {
-            if (st + 1 < nsteps) {                            // all but the next step's loads of this wave
+        for (int round = 0; round < rounds; ++round) {
+            const int st = round * KG + group;
+            if (st + KG < nsteps) {                           // all but the next step's loads of this wave
                 wait_vm(JK + JV);
             } else wait_vm<0>();
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             const int t0 = step_key(st), cur = buf * stage;
-            if (st + 2 < nsteps) issue(st + 2, buf == 0 ? 2 : buf - 1);
+            if (round + 2 < rounds) issue(round + 2, buf == 0 ? 2 : buf - 1);
             buf = buf == 2 ? 0 : buf + 1;
-            if (!mine || t0 > plast || (t0 + 31 < rlo_first && t0 >= keep)) continue;
+            if (!mine || st >= nsteps || t0 > plast || (t0 + 31 < rlo_first && t0 >= keep)) continue;
+            // all key fragments are asked for in front of the products, all value fragments in front of the softmax: left alone the compiler waits for each pair
             f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            {
+                bf16x8 k0[DK], k1[DK];
 #pragma unroll
-            for (int ks = 0; ks < DK; ++ks) {
-                        const char* kp = at_sm + cur + krow + (((ks * 4 + lq) ^ kx) << 4);
-                const bf16x8 k0 = *(const bf16x8*)kp, k1 = *(const bf16x8*)(kp + 256 * CK);
-                s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qh[ks], s[0], 0, 0, 0);
-                s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qh[ks], s[1], 0, 0, 0);
-                s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, ql[ks], s[0], 0, 0, 0);
-                s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, ql[ks], s[1], 0, 0, 0);
+                for (int ks = 0; ks < DK; ++ks) {
+                    const char* kp = at_sm + cur + krow + (((ks * 4 + lq) ^ kx) << 4);
+                    k0[ks] = *(const bf16x8*)kp; k1[ks] = *(const bf16x8*)(kp + 256 * CK);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int ks = 0; ks < DK; ++ks) {
+                    s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0[ks], qh[ks], s[0], 0, 0, 0);
+                    s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1[ks], qh[ks], s[1], 0, 0, 0);
+                    s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0[ks], ql[ks], s[0], 0, 0, 0);
+                    s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1[ks], ql[ks], s[1], 0, 0, 0);
+                }
             }
+            typedef short s16x4 __attribute__((ext_vector_type(4)));
+            typedef short s16x8 __attribute__((ext_vector_type(8)));
+            bf16x8 vf[NCBM];                                  // past the row's end (never in its last four) whatever lies there
+#pragma unroll
+            for (int i = 0; i < NCBM; ++i) {
+                const char* vp = at_sm + cur + VJ + vrow + (((i * 2 + vhi) ^ vx) << 4);
+                const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)vp);
+                const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vp + 256 * CV));
+                vf[i] = __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+            }
+            __builtin_amdgcn_sched_barrier(0);
             if (ex.softcap > 0.f) {       // cap tanh(s / cap) = cap (t - 1) / (t + 1), t = 2^(2 s log2(e) / cap), the exponent kept inside fp32's range
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
@@ -1050,27 +1104,35 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
                 ph[i] = a; pl[i] = b;
             }
             l += sum;
-            typedef short s16x4 __attribute__((ext_vector_type(4)));
-            typedef short s16x8 __attribute__((ext_vector_type(8)));
 #pragma unroll
             for (int c0 = 0; c0 < NCBM; c0 += 4) {
-                if (c0 >= NCB) continue;
-                bf16x8 vf[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const char* vp = at_sm + cur + VJ + vrow + ((((c0 + i) * 2 + vhi) ^ vx) << 4);
-                    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)vp);
-                    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vp + 256 * CV));
-                    vf[i] = __builtin_bit_cast(bf16x8, s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
-                }
+                for (int i = 0; i < 4; ++i) o[c0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[c0 + i], ph, o[c0 + i], 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[c0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i], ph, o[c0 + i], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) o[c0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i], pl, o[c0 + i], 0, 0, 0);
+                for (int i = 0; i < 4; ++i) o[c0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[c0 + i], pl, o[c0 + i], 0, 0, 0);
             }
         }
     }
-    const float lt = hy_sum_groups(l);
+    float lt = hy_sum_groups(l);
+    if (KG > 1) {                                             // the first group takes the others' parts over
+        __syncthreads();
+        constexpr int PART = (NCBM * 16 + 8) * 64;
+        char* part = at_smem + wave * PART;
+        if (group > 0) {
+#pragma unroll
+            for (int cb = 0; cb < NCBM; ++cb) *(f32x4*)(part + (cb * 64 + lane) * 16) = o[cb];
+            *(float2*)(part + NCBM * 1024 + lane * 8) = make_float2(m, lt);
+            has = false;
+        }
+        __syncthreads();
+        if (group == 0) {
+            const float2 ml = *(const float2*)(part + NCBM * 1024 + lane * 8);
+            const float mn = fmaxf(m, ml.x), ms = mn == -INFINITY ? 0.f : mn, fa = __builtin_amdgcn_exp2f(m - ms), fb = __builtin_amdgcn_exp2f(ml.x - ms);
+            lt = lt * fa + ml.y * fb;
+#pragma unroll
+            for (int cb = 0; cb < NCBM; ++cb) o[cb] = o[cb] * fa + *(const f32x4*)(part + (cb * 64 + lane) * 16) * fb;
+        }
+    }
     float inv = lt > 0.f ? 1.f / lt : 0.f;
     if (ex.ogate && !ex.gate_channels && lr < n) inv *= hy_sigmoid(ex.ogate[(size_t)(r0 + lr) * ex.ldg + h]);
     bf16* od = out + ((size_t)r0 * g.H + h) * g.vdim;
@@ -1079,7 +1141,7 @@ __global__ __launch_bounds__(256, DK <= 4 && NCBM <= 8 ? 3 : 1) void hy_attn_til
         __syncthreads();
         if (!has) return;
         const int ldr = g.vdim + 4, pairs = g.vdim / 2;
-        float* rows = (float*)at_sm + wave * 16 * ldr;
+        float* rows = (float*)at_smem + wave * 16 * ldr;
 #pragma unroll
         for (int cb = 0; cb < NCBM; ++cb)
             if (cb < NCB) *(f32x4*)(rows + lr * ldr + cb * 16 + lq * 4) = o[cb] * inv;
@@ -2566,11 +2628,18 @@ extern "C" int mi355_hy_attn_tiles_ex3(const float* q, int32_t ldq, float scale,
     const int gq = g.H / g.G, HW = gq % 4 == 0 ? 4 : gq % 2 == 0 ? 2 : 1;       // query heads of one key/value head per block, 4 / HW tiles each
     const int same = kcache == vcache && g.v_ld == g.dim && g.vdim <= g.dim;    // the value is a part of the staged key row
     const int vec = ((uintptr_t)q % 16 == 0 && ldq % 4 == 0 ? 1 : 0) | (((uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 ? 2 : 0) | ((uintptr_t)out % 8 == 0 ? 4 : 0);
-    const int staged = AT_STAGES * 4096 * ((g.dim / 8 + 7) / 8 + (same ? 0 : (g.vdim / 8 + 7) / 8)) + 4 * AT_PAGES, turned = vfreq ? 4 * 16 * (g.vdim + 4) * 4 : 0;
-    const int lds = staged > turned ? staged : turned;
+    const int staged = AT_STAGES * 4096 * ((g.dim / 8 + 7) / 8 + (same ? 0 : (g.vdim / 8 + 7) / 8)), turned = vfreq ? 4 * 16 * (g.vdim + 4) * 4 : 0;
+    const dim3 grid((tiles + 4 / HW - 1) / (4 / HW), g.H / HW);
+    // Two groups of waves walk the keys of a block where the grid leaves them compute units: us with one / two, 8 heads over a latent row of 256 (192) 64 rows 10.3 / 11.9, 131 14.4 / 14.5,
+    // 256 18.7 / 17.5, 512 30.2 / 24.8, 1024 52.4 / 39.4, 1537 76.5 / 55.3, 2048 (256 blocks) 99.5 / 71.2, 2 x 2048 (512) 127.2 / 127.5; 16 over 4 heads of 128 131 rows 12.5 / 11.5,
+    // 777 37.7 / 27.8, 1024 (256 blocks) 46.9 / 33.6, 1537 (388) 52.1 / 51.6, 2048 (512) 56.7 / 64.7.
+    const bool two = grid.x * grid.y <= 320 && keep == 0 && 2 * staged + 4 * AT_PAGES <= 160 * 1024;
 #define HY_TILES(DK_, NCBM_)                                                                                                                                     \
-    hipLaunchKernelGGL((hy_attn_tiles_kernel<DK_, NCBM_>), dim3((tiles + 4 / HW - 1) / (4 / HW), g.H / HW), dim3(256), lds, (hipStream_t)stream, q, ldq, scale, g, chunk, \
-                       sink, vfreq, pos, seq, block_table, tile_row0, tile_n, tiles, (const bf16*)kcache, (const bf16*)vcache, (bf16*)out, ex, HW, same, vec)
+    do {                                                                                                                                                         \
+        const int KG = two ? at_groups(DK_, NCBM_) : 1, part = KG > 1 ? 4 * (NCBM_ * 16 + 8) * 64 : 0, lds = std::max(KG * staged + 4 * AT_PAGES, std::max(part, turned)); \
+        hipLaunchKernelGGL((hy_attn_tiles_kernel<DK_, NCBM_>), grid, dim3(256 * KG), lds, (hipStream_t)stream, q, ldq, scale, g, chunk, sink, vfreq, pos, seq, block_table, \
+                           tile_row0, tile_n, tiles, (const bf16*)kcache, (const bf16*)vcache, (bf16*)out, ex, HW, same, vec, KG);                               \
+    } while (0)
 #define HY_TILES_V(DK_) \
     case DK_: if (g.vdim <= 64) HY_TILES(DK_, 4); else if (g.vdim <= 128) HY_TILES(DK_, 8); else if (g.vdim <= 192) HY_TILES(DK_, 12); else HY_TILES(DK_, 16); break
     switch (g.dim / 32) { HY_TILES_V(1); HY_TILES_V(2); HY_TILES_V(3); HY_TILES_V(4); HY_TILES_V(5); HY_TILES_V(6); HY_TILES_V(7); HY_TILES_V(8); }

@@ -76,3 +76,9 @@ def test_portions(dim, vdim, H, G, page, opt, starts, counts):
         got = out[r:r + c].double().view(c, H, vdim)
         assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * v.abs().max()).all()), float((got - ref).abs().max())
         r += c
+
+
+# grids of more than 320 blocks: one group of waves walks the keys (above, two do)
+@pytest.mark.parametrize("dim,vdim,H,G,page,opt", [(128, 128, 16, 4, 64, {"chunk": 512}), (256, 192, 16, 1, 48, {"latent": True, "sink": True}), (64, 64, 16, 16, 16, {"window": 100})])
+def test_portions_of_large_grids(dim, vdim, H, G, page, opt):
+    test_portions(dim, vdim, H, G, page, opt, [0, 5], [1300, 70])
