@@ -63,6 +63,11 @@ class StepBuffers(C.Structure):  # mi355_step_buffers_t
                 ("ar_buf", vp), ("workspace", vp), ("workspace_bytes", sz)]
 
 
+class PrefillPass(C.Structure):  # mi355_prefill_pass_t
+    _fields_ = [("token_ids", vp), ("positions", vp), ("row_seq", vp), ("row_start", vp), ("block_table", vp), ("nseq", i32), ("q_len", i32), ("rows", i32),
+                ("logit_rows", vp), ("logits_out", vp), ("workspace", vp), ("workspace_bytes", sz)]
+
+
 ALL_REDUCE_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
 ALL_GATHER_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
 
@@ -159,6 +164,8 @@ SIGNATURES = {
     "mi355_decoder_prefill_workspace_bytes": (sz, [vp, i32, i32]),
     "mi355_decoder_prefill": (i32, [vp, vp, vp, vp, i32, i32, vp, vp, vp, sz, vp]),
     "mi355_decoder_prefill_ragged": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, sz, vp]),
+    "mi355_decoder_prefill_overlaps": (i32, [vp, i32]),
+    "mi355_decoder_prefill_passes": (i32, [vp, C.POINTER(PrefillPass), i32, vp]),
     "mi355_decoder_set_prefill_rope_table": (i32, [vp, vp]),
     "mi355_decoder_capture": (i32, [vp, i32]),
     "mi355_decoder_replay": (i32, [vp, i32, i32, vp]),

@@ -26,6 +26,7 @@
 // Multi-row: the 16 MFMA columns of a tile hold (row, head) pairs -- R = 16 / G rows of one sequence x its G query heads --
 // and a block carries NT such tiles against the same K/V fragments, so a sequence's KV is streamed once per NT*R query rows
 // instead of once per row; column j masks tokens beyond ITS row's position (causality), nothing else changes.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -885,7 +886,8 @@ extern "C" void mi355_debug_attn_stamps(void* p) { g_attn_stamps = (unsigned lon
 
 extern "C" size_t mi355_paged_attn_workspace_bytes(int32_t B, int32_t nh, int32_t hd, int32_t max_seq_len) {
     if (B <= 0 || nh <= 0 || hd <= 0 || max_seq_len <= 0) return 0;
-    const int P = cdiv(max_seq_len, 128); // upper bound over every plan
+    // upper bound over every plan of up to B rows: plan_partitions splits no further than to 256 blocks, a block has at most 32 rows (never less for more rows: a step may have fewer)
+    const int P = std::min(cdiv(max_seq_len, 128), cdiv(256 * 32, B));
     return (size_t)B * nh * P * (hd + 2) * sizeof(float);
 }
 

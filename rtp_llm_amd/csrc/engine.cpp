@@ -113,6 +113,9 @@ struct mi355_decoder {
     void*  xg_img;                    // image of gamma 2^-e h'
     float* ssq64;                     // [64][hidden / 16 rounded up to 4]
     float* ssq;      // [16 rows][hidden / 16]: the producer GEMM's per-tile sums of h^2, consumed by the next GEMM's on-the-fly RMSNorm
+    // prefill passes in flight beside the caller's stream: see prefill_overlapped
+    hipStream_t              pass_stream = nullptr;
+    std::vector<hipEvent_t>  pass_ev;
     // graphs
     hipStream_t                    cap_stream;
     std::map<int, hipGraphExec_t>  graphs;
@@ -369,6 +372,8 @@ extern "C" void mi355_decoder_destroy(mi355_decoder_t* d) {
     if (d->ev_fork) hipEventDestroy(d->ev_fork);
     if (d->ev_join) hipEventDestroy(d->ev_join);
     for (auto e : d->ev) hipEventDestroy(e);
+    if (d->pass_stream) hipStreamDestroy(d->pass_stream);
+    for (auto e : d->pass_ev) hipEventDestroy(e);
     if (d->pairs_local) hipFree(d->pairs_local);
     delete d;
 }
@@ -789,74 +794,166 @@ extern "C" size_t mi355_decoder_prefill_workspace_bytes(mi355_decoder_t* d, int3
     return carve_prefill(d->cfg, max_tokens, max_seqs, nullptr, nullptr);
 }
 
+namespace {
+// One pass of prompt tokens (mi355_prefill_pass_t) in the pieces that two passes in flight are interleaved by.
+int prefill_check(mi355_decoder_t* d, const mi355_prefill_pass_t& p, PrefillBufs* b) {
+    if (!p.token_ids || !p.positions || !p.block_table || p.nseq <= 0 || p.q_len <= 0 || !p.workspace || (p.row_seq != nullptr) != (p.row_start != nullptr) || p.rows <= 0 ||
+        (long)p.rows > (long)p.nseq * p.q_len || (!p.row_seq && p.rows != p.nseq * p.q_len)) {
+        mi355_set_error("decoder_prefill: bad arguments"); return MI355_ERR_ARG;
+    }
+    if (d->cfg.tp_size > 1 && !d->ar && !d->has_ext) {
+        mi355_set_error("decoder_prefill: tp_size > 1 needs mi355_decoder_attach_allreduce or _attach_collective"); return MI355_ERR_ARG;
+    }
+    const size_t need = carve_prefill(d->cfg, p.rows, p.nseq, p.workspace, b);
+    if (need > p.workspace_bytes) { mi355_set_error("decoder_prefill: workspace %zu < %zu", p.workspace_bytes, need); return MI355_ERR_WORKSPACE; }
+    return MI355_OK;
+}
+
+int prefill_begin(mi355_decoder_t* d, const mi355_prefill_pass_t& p, const PrefillBufs& b, hipStream_t st) {
+    const auto& c = d->cfg;
+    const int T = p.rows;
+    if (d->embed_split) {
+        const int n = c.hidden / c.tp_size;
+        RUN(MI355_KC_OTHER, mi355_embedding(p.token_ids, T, d->model.embedding, n, d->model.vocab_full, b.tmp, st));
+        RUN(MI355_KC_COMM, mi355_allgather_hidden(d->ar, b.tmp, b.resid, T, n, st));
+    } else {
+        RUN(MI355_KC_OTHER, mi355_embedding(p.token_ids, T, d->model.embedding, c.hidden, d->model.vocab_full, b.resid, st));
+    }
+    RUN(MI355_KC_NORM, mi355_rmsnorm_dt(b.resid, d->layers[0].input_norm, c.rms_eps, T, c.hidden, b.xn, ADT, st));
+    return MI355_OK;
+}
+
+// up to the keys and values of the pass in the cache
+int prefill_layer_kv(mi355_decoder_t* d, const mi355_prefill_pass_t& p, const PrefillBufs& b, int l, hipStream_t st) {
+    const auto& c = d->cfg;
+    const auto& L = d->layers[l];
+    mi355_kv_layer_t kv = kv_of(d, l);
+    RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.xn, p.rows, &L.qkv, L.qkv_bias, b.qkv, MI355_EPI_NONE, b.gemm_ws, b.gemm_ws_bytes, st));
+    RUN(MI355_KC_ROPE_KV, mi355_rope_kv_write_rows_ragged(b.qkv, nullptr, 0, L.qkv.N, nullptr, d->prefill_cos_sin ? d->prefill_cos_sin : d->model.cos_sin, c.rope_dim,
+                                                          c.max_pos, p.positions, p.row_seq, p.block_table, c.max_blocks_per_seq, p.rows, p.row_seq ? 1 : p.q_len, c.nh, &kv,
+                                                          b.q, d->oob_count, st));
+    return MI355_OK;
+}
+
+// the rest of the layer, from the attention over the cache on
+int prefill_layer_rest(mi355_decoder_t* d, const mi355_prefill_pass_t& p, const PrefillBufs& b, int l, hipStream_t st) {
+    const auto& c = d->cfg;
+    const auto& L = d->layers[l];
+    const int T = p.rows;
+    const float scale = 1.0f / sqrtf((float)c.hd);
+    mi355_kv_layer_t kv = kv_of(d, l);
+    if (p.row_start)
+        RUN(MI355_KC_ATTN, mi355_paged_attn_rows_ragged(b.q, &kv, p.block_table, c.max_blocks_per_seq, p.positions, p.row_start, p.nseq, p.q_len, T, c.nh, scale,
+                                                        c.max_seq_len, b.attn, b.attn_ws, b.attn_ws_bytes, st));
+    else
+        RUN(MI355_KC_ATTN, mi355_paged_attn_rows(b.q, &kv, p.block_table, c.max_blocks_per_seq, p.positions, p.nseq, p.q_len, c.nh, scale,
+                                                 c.max_seq_len, b.attn, b.attn_ws, b.attn_ws_bytes, st));
+    RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.attn, T, &L.o, nullptr, b.tmp, MI355_EPI_NONE, b.gemm_ws, b.gemm_ws_bytes, st));
+    if (c.tp_size > 1 && !d->ar) RUN(MI355_KC_COMM, ext_all_reduce(d, b.tmp, (size_t)T * c.hidden, st));
+    if (c.tp_size == 1 || !d->ar) {
+        RUN(MI355_KC_NORM, mi355_add_rmsnorm_dt(b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, L.post_norm, c.rms_eps, T, c.hidden, b.xn, ADT, st));
+    } else {
+        RUN(MI355_KC_COMM, mi355_allreduce_fused_dt(d->ar, b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, L.post_norm, c.rms_eps, T,
+                                                 c.hidden, b.xn, ADT, st));
+    }
+    RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.xn, T, &L.gate_up, nullptr, b.act, MI355_EPI_SILU_MUL, b.gemm_ws, b.gemm_ws_bytes, st));
+    RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.act, T, &L.down, nullptr, b.tmp, MI355_EPI_NONE, b.gemm_ws, b.gemm_ws_bytes, st));
+    const void* next_norm = (l + 1 < c.num_layers) ? d->layers[l + 1].input_norm : d->model.final_norm;
+    if (c.tp_size > 1 && !d->ar) RUN(MI355_KC_COMM, ext_all_reduce(d, b.tmp, (size_t)T * c.hidden, st));
+    if (c.tp_size == 1 || !d->ar) {
+        RUN(MI355_KC_NORM, mi355_add_rmsnorm_dt(b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, next_norm, c.rms_eps, T, c.hidden, b.xn, ADT, st));
+    } else {
+        RUN(MI355_KC_COMM, mi355_allreduce_fused_dt(d->ar, b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, next_norm, c.rms_eps, T,
+                                                 c.hidden, b.xn, ADT, st));
+    }
+    return MI355_OK;
+}
+
+int prefill_end(mi355_decoder_t* d, const mi355_prefill_pass_t& p, const PrefillBufs& b, hipStream_t st) {
+    const auto& c = d->cfg;
+    if (!p.logit_rows || !p.logits_out) return MI355_OK;
+    // gather the requested rows of the final normed hidden state, then lm_head on nseq rows
+    RUN(MI355_KC_OTHER, mi355_embedding(p.logit_rows, p.nseq, b.xn, c.hidden, p.rows, b.last_h, st));
+    for (int r0 = 0; r0 < p.nseq; r0 += 64) {
+        const int n = p.nseq - r0 < 64 ? p.nseq - r0 : 64;
+        RUN(MI355_KC_GEMM_LMHEAD, mi355_linear_direct((const char*)b.last_h + (size_t)r0 * c.hidden * 2, n, &d->model.lm_head, nullptr,
+                                                      p.logits_out + (size_t)r0 * c.vocab, MI355_EPI_OUT_F32, nullptr, 0, st));
+    }
+    return MI355_OK;
+}
+
+int prefill_one(mi355_decoder_t* d, const mi355_prefill_pass_t& p, const PrefillBufs& b, hipStream_t st) {
+    int rc = prefill_begin(d, p, b, st);
+    for (int l = 0; rc >= 0 && l < d->cfg.num_layers; ++l) {
+        rc = prefill_layer_kv(d, p, b, l, st);
+        if (rc >= 0) rc = prefill_layer_rest(d, p, b, l, st);
+    }
+    return rc < 0 ? rc : prefill_end(d, p, b, st);
+}
+
+// Passes of which two are in flight: the second runs on a stream of the decoder's one layer behind the first (its attention waits for the first's keys and values), so that the
+// launches of one fill the compute units that those of the other leave idle.
+int prefill_overlapped(mi355_decoder_t* d, const mi355_prefill_pass_t* ps, const PrefillBufs* bs, int n, hipStream_t st) {
+    const int layers = d->cfg.num_layers;
+    auto ok = [](hipError_t e) { if (e != hipSuccess) mi355_set_error("decoder_prefill: %s", hipGetErrorString(e)); return e == hipSuccess; };
+    if (!d->pass_stream && !ok(hipStreamCreateWithFlags(&d->pass_stream, hipStreamNonBlocking))) return MI355_ERR_HIP;
+    while (d->pass_ev.size() < (size_t)2 * layers + 2) {                        // keys and values of layer l of the even / odd pass; fork; join
+        hipEvent_t e;
+        if (!ok(hipEventCreateWithFlags(&e, hipEventDisableTiming))) return MI355_ERR_HIP;
+        d->pass_ev.push_back(e);
+    }
+    hipEvent_t fork = d->pass_ev[2 * layers], join = d->pass_ev[2 * layers + 1];
+    if (!ok(hipEventRecord(fork, st)) || !ok(hipStreamWaitEvent(d->pass_stream, fork, 0))) return MI355_ERR_HIP;
+    int rc = MI355_OK;
+    for (int p0 = 0; rc >= 0 && p0 < n; p0 += 2)
+        for (int l = 0; rc >= 0 && l < layers; ++l)
+            for (int p = p0; rc >= 0 && p < n && p < p0 + 2; ++p) {
+                hipStream_t s = p & 1 ? d->pass_stream : st;
+                if (l == 0) rc = prefill_begin(d, ps[p], bs[p], s);
+                if (rc >= 0) rc = prefill_layer_kv(d, ps[p], bs[p], l, s);
+                if (rc >= 0 && p + 1 < n && !ok(hipEventRecord(d->pass_ev[(p & 1) * layers + l], s))) rc = MI355_ERR_HIP;
+                if (rc >= 0 && p > 0 && !ok(hipStreamWaitEvent(s, d->pass_ev[(~p & 1) * layers + l], 0))) rc = MI355_ERR_HIP;
+                if (rc >= 0) rc = prefill_layer_rest(d, ps[p], bs[p], l, s);
+                if (rc >= 0 && l + 1 == layers) rc = prefill_end(d, ps[p], bs[p], s);
+            }
+    // whatever happened: what the stream has in flight uses the caller's buffers
+    if (!ok(hipEventRecord(join, d->pass_stream)) || !ok(hipStreamWaitEvent(st, join, 0))) { hipStreamSynchronize(d->pass_stream); return MI355_ERR_HIP; }
+    return rc;
+}
+} // namespace
+
 // Ragged chunks: the sequences' rows lie back to back (row_seq [rows], row_start [nseq + 1], device), the linears and norms run over what is there.
 // Padding every sequence to the longest made three prompts of up to 389 tokens (7B, 8-bit weights) cost what three of 389 do: 21.0 ms, now 19.6; attention blocks
 // past a sequence's rows end at once.
 extern "C" int mi355_decoder_prefill_ragged(mi355_decoder_t* d, const int32_t* token_ids, const int32_t* positions, const int32_t* row_seq,
                                             const int32_t* row_start, const int32_t* block_table, int32_t nseq, int32_t q_len, int32_t rows,
                                             const int32_t* logit_rows, float* logits_out, void* workspace, size_t workspace_bytes, mi355_stream_t stream) {
-    if (!d || !token_ids || !positions || !block_table || nseq <= 0 || q_len <= 0 || !workspace || (row_seq != nullptr) != (row_start != nullptr) || rows <= 0 ||
-        (long)rows > (long)nseq * q_len || (!row_seq && rows != nseq * q_len)) {
-        mi355_set_error("decoder_prefill: bad arguments"); return MI355_ERR_ARG;
+    const mi355_prefill_pass_t p{token_ids, positions, row_seq, row_start, block_table, nseq, q_len, rows, logit_rows, logits_out, workspace, workspace_bytes};
+    return mi355_decoder_prefill_passes(d, &p, 1, stream);
+}
+
+// Us of a call one pass after the other / overlapped (the 0.5B model in passes of 512 tokens a prompt, 16-bit weights: 1 x 777 3571 / 2931, 1 x 1500 6477 / 5295, 4 x 1000 9363 / 7541;
+// 4 bits: 1 x 3000 12148 / 8552; the 7B model, 4 bits: 1 x 600 15288 / 14095, 2 x 1024 35701 / 30655, 8 x 1024 111971 / 105304; 8 bits: 1 x 1024 21701 / 18653).  Larger passes were
+// not measured, and want a second workspace of their size.  Under tensor parallelism two passes would meet in the collectives' buffers.
+extern "C" int mi355_decoder_prefill_overlaps(mi355_decoder_t* d, int32_t rows) { return d && d->cfg.tp_size == 1 && rows <= 4096; }
+
+extern "C" int mi355_decoder_prefill_passes(mi355_decoder_t* d, const mi355_prefill_pass_t* passes, int32_t n, mi355_stream_t stream) {
+    if (!d || !passes || n <= 0) { mi355_set_error("decoder_prefill: bad arguments"); return MI355_ERR_ARG; }
+    std::vector<PrefillBufs> bufs(n);
+    bool overlap = n > 1 && !d->prof_on, apart = true;
+    for (int i = 0; i < n; ++i) {
+        if (int e = prefill_check(d, passes[i], &bufs[i])) return e;
+        overlap = overlap && mi355_decoder_prefill_overlaps(d, passes[i].rows);
+        if (i > 0) {
+            const char *a = (const char*)passes[i - 1].workspace, *b = (const char*)passes[i].workspace;
+            apart = apart && (a + passes[i - 1].workspace_bytes <= b || b + passes[i].workspace_bytes <= a);
+        }
     }
-    const auto& c = d->cfg;
-    const int T = rows;
-    if (c.tp_size > 1 && !d->ar && !d->has_ext) {
-        mi355_set_error("decoder_prefill: tp_size > 1 needs mi355_decoder_attach_allreduce or _attach_collective"); return MI355_ERR_ARG;
-    }
-    PrefillBufs b;
-    const size_t need = carve_prefill(c, T, nseq, workspace, &b);
-    if (need > workspace_bytes) { mi355_set_error("decoder_prefill: workspace %zu < %zu", workspace_bytes, need); return MI355_ERR_WORKSPACE; }
     hipStream_t st = (hipStream_t)stream;
-    const float scale = 1.0f / sqrtf((float)c.hd);
-    if (d->embed_split) {
-        const int n = c.hidden / c.tp_size;
-        RUN(MI355_KC_OTHER, mi355_embedding(token_ids, T, d->model.embedding, n, d->model.vocab_full, b.tmp, st));
-        RUN(MI355_KC_COMM, mi355_allgather_hidden(d->ar, b.tmp, b.resid, T, n, st));
-    } else {
-        RUN(MI355_KC_OTHER, mi355_embedding(token_ids, T, d->model.embedding, c.hidden, d->model.vocab_full, b.resid, st));
-    }
-    RUN(MI355_KC_NORM, mi355_rmsnorm_dt(b.resid, d->layers[0].input_norm, c.rms_eps, T, c.hidden, b.xn, ADT, st));
-    for (int l = 0; l < c.num_layers; ++l) {
-        const auto& L = d->layers[l];
-        mi355_kv_layer_t kv = kv_of(d, l);
-        RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.xn, T, &L.qkv, L.qkv_bias, b.qkv, MI355_EPI_NONE, b.gemm_ws, b.gemm_ws_bytes, st));
-        RUN(MI355_KC_ROPE_KV, mi355_rope_kv_write_rows_ragged(b.qkv, nullptr, 0, L.qkv.N, nullptr, d->prefill_cos_sin ? d->prefill_cos_sin : d->model.cos_sin, c.rope_dim,
-                                                              c.max_pos, positions, row_seq, block_table, c.max_blocks_per_seq, T, row_seq ? 1 : q_len, c.nh, &kv, b.q,
-                                                              d->oob_count, st));
-        if (row_start)
-            RUN(MI355_KC_ATTN, mi355_paged_attn_rows_ragged(b.q, &kv, block_table, c.max_blocks_per_seq, positions, row_start, nseq, q_len, T, c.nh, scale,
-                                                            c.max_seq_len, b.attn, b.attn_ws, b.attn_ws_bytes, st));
-        else
-            RUN(MI355_KC_ATTN, mi355_paged_attn_rows(b.q, &kv, block_table, c.max_blocks_per_seq, positions, nseq, q_len, c.nh, scale,
-                                                     c.max_seq_len, b.attn, b.attn_ws, b.attn_ws_bytes, st));
-        RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.attn, T, &L.o, nullptr, b.tmp, MI355_EPI_NONE, b.gemm_ws, b.gemm_ws_bytes, st));
-        if (c.tp_size > 1 && !d->ar) RUN(MI355_KC_COMM, ext_all_reduce(d, b.tmp, (size_t)T * c.hidden, st));
-        if (c.tp_size == 1 || !d->ar) {
-            RUN(MI355_KC_NORM, mi355_add_rmsnorm_dt(b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, L.post_norm, c.rms_eps, T, c.hidden, b.xn, ADT, st));
-        } else {
-            RUN(MI355_KC_COMM, mi355_allreduce_fused_dt(d->ar, b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, L.post_norm, c.rms_eps, T,
-                                                     c.hidden, b.xn, ADT, st));
-        }
-        RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.xn, T, &L.gate_up, nullptr, b.act, MI355_EPI_SILU_MUL, b.gemm_ws, b.gemm_ws_bytes, st));
-        RUN(MI355_KC_GEMM_QUANT, mi355_linear_forward(b.act, T, &L.down, nullptr, b.tmp, MI355_EPI_NONE, b.gemm_ws, b.gemm_ws_bytes, st));
-        const void* next_norm = (l + 1 < c.num_layers) ? d->layers[l + 1].input_norm : d->model.final_norm;
-        if (c.tp_size > 1 && !d->ar) RUN(MI355_KC_COMM, ext_all_reduce(d, b.tmp, (size_t)T * c.hidden, st));
-        if (c.tp_size == 1 || !d->ar) {
-            RUN(MI355_KC_NORM, mi355_add_rmsnorm_dt(b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, next_norm, c.rms_eps, T, c.hidden, b.xn, ADT, st));
-        } else {
-            RUN(MI355_KC_COMM, mi355_allreduce_fused_dt(d->ar, b.tmp, nullptr, 0, 0, nullptr, b.resid, b.resid, next_norm, c.rms_eps, T,
-                                                     c.hidden, b.xn, ADT, st));
-        }
-    }
-    if (logit_rows && logits_out) {   // gather the requested rows of the final normed hidden state, then lm_head on nseq rows
-        RUN(MI355_KC_OTHER, mi355_embedding(logit_rows, nseq, b.xn, c.hidden, T, b.last_h, st));
-        for (int r0 = 0; r0 < nseq; r0 += 64) {
-            const int n = nseq - r0 < 64 ? nseq - r0 : 64;
-            RUN(MI355_KC_GEMM_LMHEAD, mi355_linear_direct((const char*)b.last_h + (size_t)r0 * c.hidden * 2, n, &d->model.lm_head, nullptr,
-                                                          logits_out + (size_t)r0 * c.vocab, MI355_EPI_OUT_F32, nullptr, 0, st));
-        }
-    }
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (overlap && apart && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return prefill_overlapped(d, passes, bufs.data(), n, st);
+    for (int i = 0; i < n; ++i)
+        if (int e = prefill_one(d, passes[i], bufs[i], st); e < 0) return e;
     return MI355_OK;
 }
 

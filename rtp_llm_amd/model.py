@@ -582,38 +582,52 @@ class DecoderEngine:
         btd = torch.zeros(nseq, self.max_blocks_per_seq, dtype=torch.int32, device=dev)
         btd[:, : bt.shape[1]].copy_(bt)
         longest = max(len(p) for p in prompts)
-        logits = torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
+        # pass by pass the sequences that still have tokens, their counts and the pass's integers: tokens, positions, logit rows, the sequences and, unless every sequence has
+        # q_len rows, where each sequence's rows lie.  What has ended takes no blocks, logit rows or table rows of a pass.
+        plan, ints = [], []
         for c0 in range(0, longest, chunk):
-            # the sequences that still have tokens; what has ended takes no blocks, logit rows or table rows of the pass
             live = [b for b, p in enumerate(prompts) if len(p) > c0]
             counts = [min(chunk, len(prompts[b]) - c0) for b in live]
             n, q_len = len(live), max(counts)
             first = [sum(counts[:i]) for i in range(n + 1)]
-            T = first[n]
-            toks = torch.cat([torch.as_tensor(prompts[b][c0:c0 + k], dtype=torch.int32).cpu() for b, k in zip(live, counts)])
-            pos = torch.cat([torch.arange(start[b] + c0, start[b] + c0 + k, dtype=torch.int32) for b, k in zip(live, counts)])
             ending = [i for i, b in enumerate(live) if c0 + counts[i] == len(prompts[b])]
             last = torch.zeros(n, dtype=torch.int32)
             for i in ending:
                 last[i] = first[i] + counts[i] - 1
-            # the chunk's integers in one copy: tokens, positions, logit rows, the sequences and, unless every sequence has q_len rows, where each sequence's rows lie
-            parts = [toks, pos, last, torch.tensor(live, dtype=torch.int32)]
-            if T < n * q_len:
+            parts = [torch.cat([torch.as_tensor(prompts[b][c0:c0 + k], dtype=torch.int32).cpu() for b, k in zip(live, counts)]),
+                     torch.cat([torch.arange(start[b] + c0, start[b] + c0 + k, dtype=torch.int32) for b, k in zip(live, counts)]), last, torch.tensor(live, dtype=torch.int32)]
+            if first[n] < n * q_len:
                 parts += [torch.repeat_interleave(torch.arange(n, dtype=torch.int32), torch.tensor(counts)), torch.tensor(first, dtype=torch.int32)]
-            td, pd, ld, lived, *ragged = torch.cat(parts).to(dev).split([p.numel() for p in parts])
+            plan.append((live, n, q_len, first[n], ending, [p.numel() for p in parts]))
+            ints += parts
+        if not plan:
+            return torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
+        on_device = torch.cat(ints).to(dev).split([k for pl in plan for k in pl[-1]])       # one copy
+        # two workspaces, taken in turn, where two passes may be in flight
+        need = [self.lib.mi355_decoder_prefill_workspace_bytes(self.handle, T, n) for _, n, _, T, _, _ in plan]
+        two = len(plan) > 1 and all(self.lib.mi355_decoder_prefill_overlaps(self.handle, pl[3]) for pl in plan)
+        sizes = [max(need[0::2]), max(need[1::2])] if two else [max(need)]
+        sizes = [(b + 255) // 256 * 256 for b in sizes]
+        if getattr(self, "_prefill_ws", None) is None or self._prefill_ws.numel() < sum(sizes):
+            self._prefill_ws = torch.empty(sum(sizes), dtype=torch.uint8, device=dev)
+        passes, held, at = (_C.PrefillPass * len(plan))(), [], 0
+        for i, (live, n, q_len, T, ending, lens) in enumerate(plan):
+            td, pd, ld, lived, *ragged = on_device[at:at + len(lens)]
+            at += len(lens)
             table = btd if n == nseq else btd.index_select(0, lived)
-            ws_bytes = self.lib.mi355_decoder_prefill_workspace_bytes(self.handle, T, n)
-            if getattr(self, "_prefill_ws", None) is None or self._prefill_ws.numel() < ws_bytes:
-                self._prefill_ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            tmp_logits = torch.empty(n, self.cfg.vocab, dtype=torch.float32, device=dev) if ending else None
+            out = torch.empty(n, self.cfg.vocab, dtype=torch.float32, device=dev) if ending else None
+            held.append((table, out))
             seqd, firstd = (r.data_ptr() for r in ragged) if ragged else (None, None)
-            _C.check(self.lib.mi355_decoder_prefill_ragged(self.handle, td.data_ptr(), pd.data_ptr(), seqd, firstd, table.data_ptr(), n, q_len, T,
-                                                           ld.data_ptr() if ending else None, tmp_logits.data_ptr() if ending else None,
-                                                           self._prefill_ws.data_ptr(), self._prefill_ws.numel(), st), "decoder_prefill")
-            if len(ending) == nseq:
-                logits = tmp_logits
-            elif ending:
-                logits[torch.tensor([live[i] for i in ending], device=dev)] = tmp_logits[torch.tensor(ending, device=dev)]
+            side = i % len(sizes)
+            passes[i] = _C.PrefillPass(td.data_ptr(), pd.data_ptr(), seqd, firstd, table.data_ptr(), n, q_len, T, ld.data_ptr() if ending else None,
+                                       out.data_ptr() if ending else None, self._prefill_ws.data_ptr() + side * sizes[0], sizes[side])
+        _C.check(self.lib.mi355_decoder_prefill_passes(self.handle, passes, len(plan), st), "decoder_prefill")
+        if len(plan[-1][4]) == nseq:
+            return held[-1][1]
+        logits = torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
+        for (live, _, _, _, ending, _), (_, out) in zip(plan, held):
+            if ending:
+                logits[torch.tensor([live[i] for i in ending], device=dev)] = out[torch.tensor(ending, device=dev)]
         return logits
 
     def generate(self, prompts: List[List[int]], block_table, max_new_tokens: int, prefill_chunk: int = 512) -> List[List[int]]:

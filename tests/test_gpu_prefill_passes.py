@@ -1,0 +1,41 @@
+"""Prompts in several passes: two of them in flight and one after the other are the same launches, so everything they leave is the same bits."""
+import pytest
+import torch
+
+from rtp_llm_amd import model
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+class _OneAtATime:
+    """The library as it answers where passes do not overlap (they then share one workspace)."""
+
+    def __init__(self, lib):
+        self._lib = lib
+
+    def __getattr__(self, name):
+        return (lambda handle, rows: 0) if name == "mi355_decoder_prefill_overlaps" else getattr(self._lib, name)
+
+
+# one prompt of 2 and of 7 passes, prompts that end in different passes, on top of cached tokens; few rows (decode kernels) and many
+@pytest.mark.parametrize("lens,start,chunk", [([40], [0], 32), ([200], [0], 32), ([3, 200, 32, 64, 1, 31], [0] * 6, 32), ([150, 90], [40, 7], 16), ([230, 230], [0, 0], 100)])
+@pytest.mark.parametrize("kv_int8,dtype", [(False, torch.float16), (True, torch.bfloat16)])
+def test_passes_in_flight_change_nothing(lens, start, chunk, kv_int8, dtype):
+    cfg = model.ModelConfig("tiny-passes", 3, 512, 8, 2, 64, 1024, 2048, max_pos=512)
+    eng = model.DecoderEngine(cfg, model.weights_to(model.synth_model(cfg, "w4", "cpu", seed=3, zeros="centered"), DEV), kv_int8=kv_int8, page=16, num_blocks=96,
+                              max_batch=6, max_seq_len=256, device=DEV, dtype=dtype)
+    g = torch.Generator().manual_seed(2)
+    prompts = [torch.randint(0, cfg.vocab, (n,), generator=g).tolist() for n in lens]
+    bt = torch.randperm(96, generator=g).reshape(6, 16).int()[:len(lens)]
+    lib = eng.lib
+    runs = []
+    for turn in range(4):                                       # the second and fourth: streams, events and workspaces that have been used
+        for t in eng.kv + [s for s in eng.kv_scale if s is not None]:
+            t.zero_()
+        eng.lib = _OneAtATime(lib) if turn == 2 else lib
+        logits = eng.prefill(prompts, bt, chunk=chunk, start=start)
+        runs.append([logits.clone()] + [t.clone() for t in eng.kv] + [s.clone() for s in eng.kv_scale if s is not None])
+    eng.lib = lib
+    for other in runs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(runs[0], other))
