@@ -90,6 +90,22 @@ int mi355_hy_delta_scan(const float* proj, int32_t ld, int32_t ro, int32_t ko, i
 /* The tile shape that a bf16 call of M x N x K takes (groups weights, row_tiles tiles of 64 sorted rows or 0): 0 64x64, 1 and 2 64x128, 3 128x128, 4 256x256.  Host only. */
 int mi355_dense_tile_shape(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t row_tiles);
 
+/* Two linears of a few bf16 rows (2 to 16) in one launch: see mi355_dense_linear_ex for the arguments. */
+typedef struct {
+    const void* x; int32_t ldx, M;
+    const void* w; int32_t N, K;
+    const void* bias;
+    void*       y; int32_t ldy, out_f32, gated, act;
+    float       act_param;
+} mi355_dense_args_t;
+int mi355_dense_linear_pair(const mi355_dense_args_t* two, mi355_stream_t stream);
+/* mi355_hy_scan over a few rows and mi355_hy_head_norm_ex2 (weight, gate through silu) in one launch, a block per sequence and head.  mode, projections, state and gates as
+ * there; with ao >= 0 the decay pre-activations of mode 1 are formed here: column hd is b2[hd] + sum over j < rank of w2[hd, j] (act type) times proj[:, ao + j] rounded to the
+ * act type.  w null: unit RMS only; go < 0: no gate.  out [rows, H * vdim] of the act type.  MI355_ERR_UNSUPPORTED: vdim % 4, vdim > 256, dim > 256 or dim * vdim > 32768. */
+int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, int32_t go, int32_t ao, int32_t rank, const void* w2, const void* b2,
+                        const float* z, int32_t ldz, const void* lower, const void* fbias, float tau, float qscale, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start,
+                        const int32_t* slot, const int32_t* first_pos, int32_t nseq, float* state, const void* w, int32_t w_heads, float eps, void* out, int32_t act_dtype,
+                        mi355_stream_t stream);
 /* Further extended forms: an activation with a parameter (act 5: clamped gated form g' sigmoid(1.702 g') (u' + 1)), routers that score by sigmoids, rank
  * groups by their two best experts and scale the weights, a query / key norm over all heads at once, an embedding with a multiplier, and the end of a
  * sublayer whose output is normed before it joins the stream (layer norm or RMS norm), also as the last norm on gathered rows. */

@@ -68,6 +68,11 @@ class PrefillPass(C.Structure):  # mi355_prefill_pass_t
                 ("logit_rows", vp), ("logits_out", vp), ("workspace", vp), ("workspace_bytes", sz)]
 
 
+class DenseArgs(C.Structure):  # mi355_dense_args_t
+    _fields_ = [("x", vp), ("ldx", i32), ("M", i32), ("w", vp), ("N", i32), ("K", i32), ("bias", vp), ("y", vp), ("ldy", i32), ("out_f32", i32), ("gated", i32), ("act", i32),
+                ("act_param", f32)]
+
+
 ALL_REDUCE_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
 ALL_GATHER_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
 
@@ -202,6 +207,8 @@ HYBRID_SIGNATURES = {
     "mi355_hy_depth_mix_norm": (i32, [vp, vp, vp, C.c_int64, i32, vp, vp, i32, i32, vp, f32, f32, vp, i32, vp]),
     "mi355_hy_attn_prep_ex": (i32, [vp, i32, i32, i32, ip, vp, vp, i32, f32, vp, vp, vp, i32, vp, vp, vp, vp, f32, f32, i32, i32, vp]),
     "mi355_hy_attn_rows_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, f32, vp, i32, i32, vp]),
+    "mi355_dense_linear_pair": (i32, [C.POINTER(DenseArgs), vp]),
+    "mi355_hy_recur_step": (i32, [i32, vp] + [i32] * 7 + [vp, vp, vp, i32, vp, vp, f32, f32, i32, i32, i32, vp, vp, vp, i32, vp, vp, i32, f32, vp, i32, vp]),
     "mi355_hy_attn_tiles_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, f32, vp, i32, i32, vp]),
     "mi355_hy_head_norm_ex": (i32, [vp, i32, i32, i32, vp, f32, vp, i32, i32, vp, i32, i32, i32, vp]),
     "mi355_hy_delta_scan": (i32, [vp, i32, i32, i32, i32, i32, vp, i32, f32, f32, i32, i32, i32, vp, vp, vp, i32, vp, vp, vp]),

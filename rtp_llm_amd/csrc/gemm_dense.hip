@@ -693,14 +693,15 @@ void launch_rows(const DenseParams& p, hipStream_t st) {
 // HALF (M <= 8): 8 outputs per block and half the waves, each with the k-steps of two of them: rows 0 to 7 of the first operand are x in the steps of wave w, rows 8 to 15 x in
 // those of wave w + NW, the second operand likewise.  Of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are what the two waves would hold, the rest is not used;
 // the partial sums and their order are those of 16 outputs, a row's bits do not depend on how many rows (2 to 16) there are.
+// The tile's block bx of group grp; the first NW of the block's waves take part.  Whole block.
+typedef f32x4 SkinnySums[8][2][64];
 template <bool GATED, bool HALF>
-__global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, int mbase) {
-    __shared__ f32x4 red[8][2][64];
+__device__ __forceinline__ void dense_skinny_tile(const DenseParams& p, int bx, int grp, int NW, int mbase, SkinnySums& red) {
     constexpr int NO = HALF ? 8 : 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, NW = blockDim.x >> 6;
-    const int nout = GATED ? p.N / 2 : p.N, grp = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nout = GATED ? p.N / 2 : p.N;
     const int r = lane & (NO - 1), chains = HALF ? 2 * NW : NW, kq = (lane >> 4) * 8 + (HALF && (lane & 8) ? NW * 32 : 0);
-    const int o = min((int)blockIdx.x * NO + r, nout - 1);
+    const int o = min(bx * NO + r, nout - 1);
     const int n = GATED ? (o >> 5) * 64 + (o & 31) : o;
     const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kq;
     const bf16* wu = wg + (size_t)32 * p.K;
@@ -709,7 +710,7 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
     const bf16x8 zero = {};
     constexpr int U = HALF ? 8 : 4;                          // steps in flight: the same bytes per compute unit in both forms
     const int stride = chains * 32;
-    for (int k0 = wave * 32; k0 < p.K; k0 += U * stride) {
+    for (int k0 = wave < NW ? wave * 32 : p.K; k0 < p.K; k0 += U * stride) {
         bf16x8 a[U], b[U], c[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -741,7 +742,7 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
             if (GATED) au += red[w][1][lane + 40];
         }
     }
-    const int oc = blockIdx.x * NO + r;
+    const int oc = bx * NO + r;
     if (oc >= nout) return;
     const int nb = GATED ? (oc >> 5) * 64 + (oc & 31) : oc;
 #pragma unroll
@@ -754,10 +755,32 @@ __global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, i
     }
 }
 
+template <bool GATED, bool HALF>
+__global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, int mbase) {
+    __shared__ SkinnySums red;
+    dense_skinny_tile<GATED, HALF>(p, blockIdx.x, blockIdx.y, blockDim.x >> 6, mbase, red);
+}
+
+// Two of them in one launch, the second's blocks behind the first's: a launch of few rows costs 4 to 5 us whatever it reads, and the weights of the two keep each other's compute
+// units busy.  NW: the waves that each takes, as in a launch of its own, so that the bits are the same.
+template <bool HALF>
+__global__ __launch_bounds__(512) void dense_skinny_pair_kernel(DenseParams p0, DenseParams p1, int blocks0, int nw0, int nw1) {
+    __shared__ SkinnySums red;
+    if ((int)blockIdx.x < blocks0) {
+        if (p0.gated) dense_skinny_tile<true, HALF>(p0, blockIdx.x, 0, nw0, 0, red);
+        else          dense_skinny_tile<false, HALF>(p0, blockIdx.x, 0, nw0, 0, red);
+    } else {
+        if (p1.gated) dense_skinny_tile<true, HALF>(p1, blockIdx.x - blocks0, 0, nw1, 0, red);
+        else          dense_skinny_tile<false, HALF>(p1, blockIdx.x - blocks0, 0, nw1, 0, red);
+    }
+}
+
 // M of 2 to 16, p.vec.  Few outputs (blocks of 8 still one for every compute unit): 8 per block where M allows it, so that all compute units pull weights; narrow outputs:
 // more waves per tile keep the memory system busy.  M = 8, weights from memory, us with 16 / 8 outputs: 2048 x 5632 12.8 / 10.7, 2048 x 2048 6.4 / 5.5, 16 x 2048 5.3 / 4.4,
 // 1024 x 1024 4.8 / 4.4; past the line, where some compute units get a second block: 2176 x 2048 6.3 / 7.1, 2560 x 5632 13.5 / 15.4, gated 2304 x 1024 6.3 / 6.9;
 // short K, of which a wave has a step or two: 1536 x 512 3.9 / 3.7, 48 x 192 2.6 / 3.0, gated 512 x 152 2.8 / 3.3.
+// The partial sums that K is split into.
+int skinny_chains(const DenseParams& p, int tiles) { return tiles * p.G >= 1024 || p.K < 1024 ? 4 : 8; }
 void launch_skinny(const DenseParams& p, hipStream_t st) {
     const int nout = p.gated ? p.N / 2 : p.N, tiles = (nout + 15) / 16;
     if (p.M <= 8 && p.K >= 512 && tiles * p.G <= 128) {
@@ -766,7 +789,7 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, true>), grid, block, 0, st, p, 0);
         return;
     }
-    const dim3 grid(tiles, p.G), block((tiles * p.G >= 1024 || p.K < 1024) ? 256 : 512);
+    const dim3 grid(tiles, p.G), block(64 * skinny_chains(p, tiles));
     if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, false>), grid, block, 0, st, p, 0);
     else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, false>), grid, block, 0, st, p, 0);
 }
@@ -822,6 +845,40 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
         hipLaunchKernelGGL(dense_tile_f32_kernel, grid, dim3(256), 0, st, p);
         MI355_CHECK_LAUNCH("dense_tile_f32_kernel");
     }
+    return MI355_OK;
+}
+
+// Two linears of bf16 rows in one launch, arguments as in mi355_dense_linear_ex each (M of 2 to 16 rows, whole 16-byte pieces): the results are those of two calls, bit for bit.
+// MI355_ERR_UNSUPPORTED: other forms, which take two calls.
+extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream_t stream) {
+    MI355_CHECK_ARG(a, "dense_linear_pair: null arguments");
+    DenseParams p[2];
+    int tiles[2], nw[2];
+    for (int i = 0; i < 2; ++i) {
+        const mi355_dense_args_t& d = a[i];
+        MI355_CHECK_ARG(d.x && d.w && d.y && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && (!d.gated || d.N % 64 == 0) && d.ldy >= (d.gated ? d.N / 2 : d.N) && d.act >= 0 &&
+                            d.act <= DN_ACT_RELU2 && (d.act != DN_ACT_SWIGLU_CLAMP || (d.gated && d.act_param > 0.f)),
+                        "dense_linear_pair: M=%d N=%d K=%d ldx=%d ldy=%d gated=%d act=%d", d.M, d.N, d.K, d.ldx, d.ldy, d.gated, d.act);
+        if (d.M < 2 || d.M > 16 || d.K % 8 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16) return MI355_ERR_UNSUPPORTED;
+        DenseParams& q = p[i];
+        q.x = d.x; q.w = d.w; q.bias = d.bias; q.y = d.y; q.M = d.M; q.N = d.N; q.K = d.K; q.ldx = d.ldx; q.ldy = d.ldy;
+        q.gated = d.gated; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
+        q.yvec = (d.ldy % 4 == 0) && ((uintptr_t)d.y % (d.out_f32 ? 16 : 8) == 0);
+        q.G = 1; q.xs = q.ws = q.ys = 0; q.offs = nullptr; q.gather = nullptr; q.tiles = nullptr; q.egate = nullptr; q.ldg = q.goff = 0;
+        tiles[i] = ((d.gated ? d.N / 2 : d.N) + 15) / 16;
+        nw[i] = skinny_chains(q, tiles[i]);
+    }
+    hipStream_t st = (hipStream_t)stream;
+    // 8 outputs a block where both together leave a compute unit two of them.  M = 8, weights from memory, us of 16 outputs a block / 8: 1024 x 1024 + 1024 x 2816 7.4 / 6.4,
+    // 2048 x 2048 + 2048 x 5632 12.9 / 11.9, 3072 x 2048 + 1024 x 2048 6.6 / 7.2; past the line 2560 x 2560 + 2560 x 6912 20.7 / 22.4, 6160 x 2048 + gated 11264 x 2048 21.0 / 22.5
+    // (in two launches the second takes 5.2 + 9.9, the last 10.4 + 16.6).
+    if (p[0].M <= 8 && p[1].M <= 8 && p[0].K >= 512 && p[1].K >= 512 && tiles[0] + tiles[1] <= 256) {
+        const int b0 = ((p[0].gated ? p[0].N / 2 : p[0].N) + 7) / 8, b1 = ((p[1].gated ? p[1].N / 2 : p[1].N) + 7) / 8;
+        hipLaunchKernelGGL(dense_skinny_pair_kernel<true>, dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, nw[0] / 2, nw[1] / 2);
+    } else {
+        hipLaunchKernelGGL(dense_skinny_pair_kernel<false>, dim3(tiles[0] + tiles[1]), dim3(512), 0, st, p[0], p[1], tiles[0], nw[0], nw[1]);
+    }
+    MI355_CHECK_LAUNCH("dense_skinny_pair_kernel");
     return MI355_OK;
 }
 

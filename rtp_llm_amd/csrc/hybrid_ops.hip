@@ -653,16 +653,19 @@ __global__ __launch_bounds__(1024) void hy_attn_rows_kernel(const float* q, int 
     float qv[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) qv[i] = (coop && kl_ok) ? q_s[kl * 8 + i] : 0.f;
-    for (int t0 = (sp * NW + wave) * 64; t0 < nvis; t0 += 64 * NW * S) {
+    // 64 keys a wave and trip; of short contexts 16 or 32, so that all waves have some: 8 rows of 16 heads over about 100 keys 15.7 us on two
+    // of sixteen waves, 12.3 on seven
+    const int tile = nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;
+    for (int t0 = (sp * NW + wave) * tile; t0 < nvis; t0 += tile * NW * S) {
         const int kj = t0 + lane < kept ? t0 + lane : t0 + lane - kept + lo;
-        const bool valid = kj <= p;
+        const bool valid = lane < tile && kj <= p;
         float s = -INFINITY;
         int rowi = 0;                                              // row of the key inside the cache tensors: (page * G + kv head) * page size + offset
         if (valid) rowi = (bt[kj / g.page] * g.G + kvh) * g.page + (kj % g.page);
         if (coop) {
             // LK lanes share a key row (8 channels = one 16- or 32-byte piece each), so a load instruction reads KK whole rows instead of one
             // piece of 64 rows; the partial products are summed over the LK lanes and handed to the lane that owns the key
-            const int nk = min(64, nvis - t0);
+            const int nk = min(tile, nvis - t0);
             float sc = 0.f;
             constexpr int UB = 8;                                  // load instructions in flight
             for (int it0 = 0; it0 * KK < nk; it0 += UB) {
@@ -699,7 +702,7 @@ __global__ __launch_bounds__(1024) void hy_attn_rows_kernel(const float* q, int 
         const float corr = (m == -INFINITY) ? 0.f : expf(m - mn);
         l = l * corr + hy_wave_sum(pj);
         m = mn;
-        const int nv = min(64, nvis - t0);
+        const int nv = min(tile, nvis - t0);
         if (fast) {
             // LPK lanes share one key's value row (8 channels = 16 bytes each), so one load instruction covers KPI keys
 #pragma unroll
@@ -2030,6 +2033,120 @@ __global__ __launch_bounds__(1024) void hy_head_norm_kernel(const float* o, int 
 }
 
 
+// ------------------------------------------------------------------------------------------------ recurrences of a few rows: gates, update, output, norm and output gate in one launch
+// A decode step's recurrence took four launches (the low-rank decay's second linear, the scan over blocks of 64 value columns, the norm over whole heads, and the launch of the
+// first low-rank linear, now a part of the input linear) of 4 to 6 us each for a state of a few MB.  Here a block has a head of one sequence: thread (kg, cg) holds four value
+// columns of the key rows kg, kg + KG, .., loaded while the gates are formed.  16 heads of 64 x 128, 8 sequences: 8.3 us under a low-rank decay, with 6.1 + 2.8 of the scan and the
+// norm and 2.8 of that decay's second linear before; what is left is a chain of four trips to memory.
+struct RecurStep {
+    const float* proj; int ld, qo, ko, vo, go, ao, rank;
+    const void* w2; const void* b2;
+    const float* z; int ldz;
+    const void* lower; const void* fbias;
+    float tau, qscale;
+    int mode, H, dim, vdim;
+    const int32_t* row_start; const int32_t* slot; const int32_t* first_pos;
+    float* state;
+    const void* w; int w_heads;
+    float eps;
+    void* out;
+};
+template <typename T, int RPT>
+__global__ __launch_bounds__(256) void hy_recur_step_kernel(RecurStep p) {
+    __shared__ float q_s[256], k_s[256], a_s[256], red[8];
+    __shared__ __attribute__((aligned(16))) float part[1024];
+    const int sq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, CG = p.vdim >> 2, KG = 256 / CG, cg = tid % CG, kg = tid / CG;
+    const int r0 = p.row_start[sq], r1 = p.row_start[sq + 1];
+    const bool on = kg < KG;
+    float* st = p.state + ((size_t)p.slot[sq] * p.H + h) * p.dim * p.vdim + cg * 4;
+    f32x4 s[RPT];
+    const bool fresh = p.first_pos[sq] == 0;
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const int d = kg + j * KG;
+        s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (on && !fresh && d < p.dim) s[j] = *(const f32x4*)(st + (size_t)d * p.vdim);
+    }
+    const int hd = h * p.dim + min(tid, p.dim - 1), hv = h * p.vdim + min(tid, p.vdim - 1);
+    const float norm = p.w ? (float)((const T*)p.w)[p.w_heads ? hv : min(tid, p.vdim - 1)] : 1.f;
+    const bool low = p.mode == SCAN_GLA && p.ao >= 0;
+    for (int t = r0; t < r1; ++t) {
+        // everything the token needs is asked for at once: a later load is another trip to memory in a launch of a few microseconds
+        const float* row = p.proj + (size_t)t * p.ld;
+        float qv = row[p.qo + hd], kv = row[p.ko + hd], av = 0.f, zz = 0.f, lr = 0.f;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = row[p.vo + h * p.vdim + cg * 4 + e];
+        const float gz = p.go >= 0 ? row[p.go + hv] : 0.f;
+        if (low) {
+            lr = (float)(T)row[p.ao + min(tid & 63, p.rank - 1)];
+            zz = p.b2 ? (float)((const T*)p.b2)[hd] : 0.f;
+            const T* w2 = (const T*)p.w2 + (size_t)hd * p.rank;
+            float dot = 0.f;
+            if (p.rank % 8 == 0 && (uintptr_t)p.w2 % 32 == 0)
+                for (int j = 0; j < p.rank; j += 8) {
+                    float w8[8];
+                    hy_load8<T>(w2 + j, w8);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(w8[e], __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lr), j + e)), dot);
+                }
+            else
+                for (int j = 0; j < p.rank; ++j)
+                    dot = __builtin_fmaf((float)w2[j], __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lr), j)), dot);
+            zz += dot;
+        } else if (p.mode == SCAN_GLA) zz = p.z[(size_t)t * p.ldz + hd];
+        if (p.mode == SCAN_HGRN2) {
+            const float lw = (float)((const T*)p.lower)[hd], f = lw + (1.f - lw) * hy_sigmoid(kv + (float)((const T*)p.fbias)[hd]);
+            qv = hy_silu(qv); av = f; kv = 1.f - f;
+        } else if (p.mode == SCAN_GLA) {
+            qv *= p.qscale;
+            av = expf((fminf(zz, 0.f) - log1pf(expf(-fabsf(zz)))) / p.tau);
+        } else {
+            if (p.mode == SCAN_FIXED_SILU) {
+                qv = hy_silu(qv); kv = hy_silu(kv);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = hy_silu(v[e]);
+            }
+            av = ((const float*)p.lower)[h];
+        }
+        if (tid < p.dim) { q_s[tid] = qv; k_s[tid] = kv; a_s[tid] = av; }
+        __syncthreads();
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+        if (on) {
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                const int d = kg + j * KG;
+                if (d >= p.dim) continue;
+                const float a = a_s[d], k = k_s[d], q = q_s[d];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { s[j][e] = __builtin_fmaf(a, s[j][e], k * v[e]); o[e] = __builtin_fmaf(s[j][e], q, o[e]); }
+            }
+            *(f32x4*)(part + (kg * CG + cg) * 4) = o;
+        }
+        __syncthreads();
+        float y = 0.f;
+        if (tid < p.vdim)
+            for (int g = 0; g < KG; ++g) y += part[g * p.vdim + tid];
+        const float ss = hy_wave_sum(y * y);
+        if ((tid & 63) == 0) red[(t & 1) * 4 + (tid >> 6)] = ss;
+        __syncthreads();
+        if (tid < p.vdim) {
+            const float* rd = red + (t & 1) * 4;
+            y *= 1.f / sqrtf(((rd[0] + rd[1]) + (rd[2] + rd[3])) / (float)p.vdim + p.eps);
+            if (p.w) y *= norm;
+            if (p.go >= 0) y *= hy_silu(gz);
+            ((T*)p.out)[((size_t)t * p.H + h) * p.vdim + tid] = (T)y;
+        }
+    }
+    if (r0 < r1) {
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            const int d = kg + j * KG;
+            if (on && d < p.dim) *(f32x4*)(st + (size_t)d * p.vdim) = s[j];
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ latent attention: normed latent + shared rotated key -> page; queries split
 // A token caches ONE row [c (R) | rotated shared key part (dr) | zeros up to dpad] for all heads: c = unit-RMS(first R outputs of the down
 // projection) * w, the key part is the remaining dr outputs with their first `rdims` channels turned by the position (pair layout as hy_pair,
@@ -2680,6 +2797,32 @@ extern "C" int mi355_hy_scan(int32_t mode, const float* proj, int32_t ld, int32_
     else if (RD == 16) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_scan_kernel<T, 16>), grid, dim3(64 * DS), lds, (hipStream_t)stream, p));
     else               HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_scan_kernel<T, 32>), grid, dim3(64 * DS), lds, (hipStream_t)stream, p));
     MI355_CHECK_LAUNCH("hy_scan_kernel");
+    return MI355_OK;
+}
+
+// mi355_hy_scan over few rows with the head norm and output gate behind it: see the header.
+extern "C" int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, int32_t go, int32_t ao, int32_t rank, const void* w2,
+                                   const void* b2, const float* z, int32_t ldz, const void* lower, const void* fbias, float tau, float qscale, int32_t H, int32_t dim,
+                                   int32_t vdim, const int32_t* row_start, const int32_t* slot, const int32_t* first_pos, int32_t nseq, float* state, const void* w,
+                                   int32_t w_heads, float eps, void* out, int32_t act_dtype, mi355_stream_t stream) {
+    MI355_CHECK_ARG(proj && row_start && slot && first_pos && state && out && nseq > 0 && H > 0 && dim > 0 && vdim > 0, "hy_recur_step: bad argument");
+    MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : (mode == SCAN_FIXED || mode == SCAN_FIXED_SILU) ? lower != nullptr
+                                                          : (mode == SCAN_GLA && tau > 0.f && (ao >= 0 ? (w2 && rank > 0 && rank <= 64) : z != nullptr)),
+                    "hy_recur_step: mode %d lacks its gate inputs", mode);
+    if (vdim % 4 || vdim > 256 || dim > 256 || dim * vdim > 32768 || (uintptr_t)state % 16) {
+        mi355_set_error("hy_recur_step: heads of %d x %d", dim, vdim);
+        return MI355_ERR_UNSUPPORTED;
+    }
+    const RecurStep p{proj, ld, qo, ko, vo, go, ao, rank, w2, b2, z, ldz, lower, fbias, tau, qscale, mode, H, dim, vdim, row_start, slot, first_pos, state, w, w_heads, eps, out};
+    const int KG = 256 / (vdim / 4), rows = (dim + KG - 1) / KG;
+    const dim3 grid(nseq, H);
+    hipStream_t st = (hipStream_t)stream;
+    if (rows <= 4)       HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 4>), grid, dim3(256), 0, st, p));
+    else if (rows <= 8)  HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 8>), grid, dim3(256), 0, st, p));
+    else if (rows <= 16) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 16>), grid, dim3(256), 0, st, p));
+    else if (rows <= 36) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 36>), grid, dim3(256), 0, st, p));
+    else { mi355_set_error("hy_recur_step: %d key rows a thread", rows); return MI355_ERR_UNSUPPORTED; }
+    MI355_CHECK_LAUNCH("hy_recur_step_kernel");
     return MI355_OK;
 }
 

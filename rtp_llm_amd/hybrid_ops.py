@@ -84,6 +84,38 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
     return out
 
 
+FEW_ROWS = 16              # rows up to which the linears are bound by their weights' stream and every launch by its own cost
+
+
+def dense_pair(first: dict, second: dict):
+    """Two dense_linear calls (keywords x, w, bias, out_dtype, gated, act, act_param) as one launch where both are bf16 with 2 to FEW_ROWS rows, else as two; the same bits either way."""
+    args, outs = (_C.DenseArgs * 2)(), []
+    for a, d in zip(args, (first, second)):
+        x, w, bias = d["x"], d["w"], d.get("bias")
+        M, K = x.shape
+        if w.dtype != torch.bfloat16 or not 2 <= M <= FEW_ROWS:
+            return dense_linear(**first), dense_linear(**second)
+        _dev(x, w.dtype, "dense_pair.x"); _dev(w, w.dtype, "dense_pair.w")
+        N, gated = w.shape[0], bool(d.get("gated"))
+        if w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or (gated and N % 64) or (bias is not None and (bias.numel() != N or not bias.is_contiguous())):
+            raise _C.Mi355Error(f"dense_pair: x {tuple(x.shape)} against w {tuple(w.shape)}")
+        if bias is not None:
+            _dev(bias, w.dtype, "dense_pair.bias")
+        od = d.get("out_dtype") or w.dtype
+        if od not in (torch.float32, w.dtype):
+            raise _C.Mi355Error(f"dense_pair: output {od} from {w.dtype} operands")
+        n_out = N // 2 if gated else N
+        out = torch.empty(M, n_out, dtype=od, device=x.device)
+        outs.append(out)
+        a.x, a.ldx, a.M, a.w, a.N, a.K, a.bias, a.y, a.ldy = x.data_ptr(), _rows(x, "dense_pair.x"), M, w.data_ptr(), N, K, _p(bias), out.data_ptr(), n_out
+        a.out_f32, a.gated, a.act, a.act_param = int(od == torch.float32), int(gated), int(d.get("act", ACT_NONE)), float(d.get("act_param", 0.0))
+    rc = _C.hybrid_lib().mi355_dense_linear_pair(args, _stream())
+    if rc == _C.ERR_UNSUPPORTED:               # operands off 16 bytes, K % 8
+        return dense_linear(**first), dense_linear(**second)
+    _C.check_hybrid(rc, "dense_pair")
+    return tuple(outs)
+
+
 def group_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """[ff, K] gate and up weights -> the [2 ff, K] weight of a gated dense_linear: per 32 channels, 32 gate rows then 32 up rows
     (ff % 32 == 0)."""
@@ -551,6 +583,41 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
     _C.check_hybrid(lib.mi355_hy_chunk_prefix(plan.cs.data_ptr(), plan.sc.data_ptr(), slot.data_ptr(), first_pos.data_ptr(), nseq, lower.data_ptr(), heads,
                                               dim * vdim, cstate.data_ptr(), state.data_ptr(), _stream()), "hy_chunk_prefix")        # 2: states at the chunks' starts
     run(mode + 4, plan.cs, plan.ids, plan.ones, plan.max_chunks, cstate)                    # 3: their share of the outputs
+    return out
+
+
+STEP_MAX_RANK = 64         # of the low-rank decay that recur_step forms
+
+
+def recur_step_supported(dim: int, vdim: int) -> bool:
+    """Heads that recur_step takes."""
+    return vdim % 4 == 0 and vdim <= 256 and dim <= 256 and dim * vdim <= 32768
+
+
+def recur_step(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, go: Optional[int], low_rank, z: Optional[torch.Tensor], lower, fbias, tau: float, qscale: float, heads: int,
+               dim: int, vdim: int, row_start, slot, first_pos, state: torch.Tensor, w: Optional[torch.Tensor], eps: float, act: torch.dtype) -> torch.Tensor:
+    """scan and head_norm (weight w, gate through silu at column go) over few rows in one launch -> act type [T, heads * vdim].  low_rank: None, or (column of proj, w2
+    [heads * dim, rank], b2 or None) that SCAN_GLA forms its decay pre-activations from instead of z."""
+    _dev(proj, torch.float32, "recur_step.proj"); _dev(state, torch.float32, "recur_step.state")
+    if not state.is_contiguous() or state.shape[1:] != (heads, dim, vdim):
+        raise _C.Mi355Error(f"recur_step: state {tuple(state.shape)} for {heads} heads of {dim} x {vdim}")
+    T, nseq = proj.shape[0], slot.numel()
+    out = torch.empty(T, heads * vdim, dtype=act, device=proj.device)
+    if not (T and nseq):
+        return out
+    ao, w2, b2 = low_rank if low_rank is not None else (-1, None, None)
+    for t, n in ((w2, None), (b2, heads * dim), (w, None)):
+        if t is not None:
+            _dev(t, act, "recur_step.weights")
+            if not t.is_contiguous() or (n and t.numel() != n):
+                raise _C.Mi355Error(f"recur_step: weight {tuple(t.shape)}")
+    if (w2 is not None and (w2.dim() != 2 or w2.shape[0] != heads * dim)) or (w is not None and w.numel() not in (vdim, heads * vdim)):
+        raise _C.Mi355Error("recur_step: weights do not fit the heads")
+    _C.check_hybrid(_C.hybrid_lib().mi355_hy_recur_step(mode, proj.data_ptr(), _rows(proj, "recur_step.proj"), qo, ko, vo, -1 if go is None else go, ao,
+                                                        0 if w2 is None else w2.shape[1], _p(w2), _p(b2), _p(z), 0 if z is None else _rows(z, "recur_step.z"), _p(lower),
+                                                        _p(fbias), float(tau), float(qscale), heads, dim, vdim, row_start.data_ptr(), slot.data_ptr(), first_pos.data_ptr(),
+                                                        nseq, state.data_ptr(), _p(w), int(w is not None and w.numel() == heads * vdim and heads > 1), float(eps),
+                                                        out.data_ptr(), act_code(act), _stream()), "hy_recur_step")
     return out
 
 

@@ -242,6 +242,10 @@ class PagedChunkAttention:
                                                   num_pages))
         return self._geom[1]
 
+    def few_rows(self, T: int):
+        """(weight, bias) of the input linear of a step of few rows; None: not such a step."""
+        return (self.w_in, self.b_in) if T <= hops.FEW_ROWS else None
+
     def forward(self, h: torch.Tensor, batch: StepBatch, kcache: torch.Tensor, vcache: torch.Tensor, proj: Optional[torch.Tensor] = None,
                 out_proj: bool = True) -> torch.Tensor:
         """proj: h w_in^T (+ b_in) in fp32 when the caller has computed it (as columns of a linear shared with other projections of h; the query
@@ -309,9 +313,12 @@ class GatedLinearRecurrence:
             self.w_in = torch.cat([weights["q"], weights["f"], weights["v"]], 0).contiguous()
             self.lower, self.fbias = weights["lower"].contiguous(), weights["f.b"].contiguous()
             self.qo, self.ko, self.vo, self.go = 0, hd, 2 * hd, None
+            self.w_few = self.w_in
             self.mode = hops.SCAN_HGRN2
         elif s.kind == "gla":
-            self.w_in = torch.cat([weights["q"], weights["k"], weights["v"], weights["g"]], 0).contiguous()
+            whole = torch.cat([weights["q"], weights["k"], weights["v"], weights["g"], weights["a1"]], 0).contiguous()
+            n = whole.shape[0] - weights["a1"].shape[0]
+            self.w_few, self.w_in, self.ao = whole, whole[:n], n                # few rows take the low-rank decay's first linear along
             self.w_a1, self.w_a2, self.b_a2 = weights["a1"].contiguous(), weights["a2"].contiguous(), weights["a2.b"].contiguous()
             self.qo, self.ko, self.vo, self.go = 0, hd, 2 * hd, 2 * hd + s.heads * s.vdim
             self.lower = self.fbias = None
@@ -325,8 +332,23 @@ class GatedLinearRecurrence:
         s = self.spec
         return (s.heads, s.dim, s.vdim)
 
-    def forward(self, h: torch.Tensor, batch: StepBatch, state: torch.Tensor) -> torch.Tensor:
+    def few_rows(self, T: int):
+        """(weight, bias) of the input linear of a step of few rows, whose fp32 result `forward` takes as proj; None: not such a step."""
+        if T > hops.FEW_ROWS or not hops.recur_step_supported(self.spec.dim, self.spec.vdim) or (self.mode == hops.SCAN_GLA and self.w_a2.shape[1] > hops.STEP_MAX_RANK):
+            return None
+        return self.w_few, None
+
+    def forward(self, h: torch.Tensor, batch: StepBatch, state: torch.Tensor, proj: Optional[torch.Tensor] = None, out_proj: bool = True) -> torch.Tensor:
+        """proj: h w^T for the weight that few_rows names, when the caller has computed it.  out_proj False: without the output projection."""
         s = self.spec
+        few = self.few_rows(h.shape[0])
+        if few is not None:
+            if proj is None:
+                proj = hops.dense_linear(h, self.w_few, out_dtype=torch.float32)
+            low_rank = (self.ao, self.w_a2, self.b_a2) if self.mode == hops.SCAN_GLA else None
+            o = hops.recur_step(self.mode, proj, self.qo, self.ko, self.vo, self.go, low_rank, None, self.lower, self.fbias, s.tau, 1.0 / math.sqrt(s.dim), s.heads, s.dim,
+                                s.vdim, batch.row_start, batch.slot, batch.first_pos, state, self.norm, self.eps, self.act)
+            return hops.dense_linear(o, self.w_o, out_dtype=torch.float32) if out_proj else o
         proj = hops.dense_linear(h, self.w_in, out_dtype=torch.float32)
         z = None
         if self.mode == hops.SCAN_GLA:
@@ -334,7 +356,7 @@ class GatedLinearRecurrence:
         o = hops.scan(self.mode, proj, self.qo, self.ko, self.vo, z, self.lower, self.fbias, s.tau, 1.0 / math.sqrt(s.dim), s.heads, s.dim, s.vdim,
                       batch.row_start, batch.slot, batch.first_pos, state, self.act, plans=batch.plans, max_rows=batch.max_rows)
         o = hops.head_norm(o, s.heads, s.vdim, self.norm, self.eps, proj if self.go is not None else None, self.go or 0)
-        return hops.dense_linear(o, self.w_o, out_dtype=torch.float32)
+        return hops.dense_linear(o, self.w_o, out_dtype=torch.float32) if out_proj else o
 
 
 @dataclass
@@ -474,6 +496,10 @@ class Retention:
         rot = s.rot
         hops.rotary(proj, [(self.qo, s.heads, s.dim, 1.0), (self.ko, s.heads, s.dim, 1.0 / math.sqrt(s.dim))], rot.dims if rot else 0,
                     hops.LAYOUTS[rot.layout] if rot else 0, self.freq, self.mag, batch.pos)
+        if h.shape[0] <= hops.FEW_ROWS and hops.recur_step_supported(s.dim, s.vdim):
+            o = hops.recur_step(hops.SCAN_FIXED, proj, self.qo, self.ko, self.vo, self.go, None, None, self.decay, None, 1.0, 1.0, s.heads, s.dim, s.vdim, batch.row_start,
+                                batch.slot, batch.first_pos, state, None, self.eps, self.act)
+            return hops.dense_linear(o, self.w_o, out_dtype=torch.float32)
         o = hops.scan(hops.SCAN_FIXED, proj, self.qo, self.ko, self.vo, None, self.decay, None, 1.0, 1.0, s.heads, s.dim, s.vdim,
                       batch.row_start, batch.slot, batch.first_pos, state, self.act, plans=batch.plans, max_rows=batch.max_rows)
         o = hops.head_norm(o, s.heads, s.vdim, None, self.eps, proj, self.go, out_dtype=self.act)
