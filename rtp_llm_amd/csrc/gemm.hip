@@ -582,7 +582,33 @@ int launch_gemm_bf16_t(const GemmParams& p, int cfg, hipStream_t st) {
     return MI355_OK;
 }
 
+// 16-bit weights where the shapes above leave most of the chip without a block, or a wave with two of its chunks in flight: four n-waves of one tile (two up to 64 blocks), as many chunks
+// in flight as a block has, up to 8 of 4 KB a wave (4 from 17 rows on).  The same sums: a wave's tiles and chunks are what they were.  One step of the 0.5B model, us before / now:
+// 1 row 845 / 751, 12 (bf16) 921 / 896, 20 1155 / 949, 32 (bf16) 1186 / 974, 40 1651 / 1108, 64 1875 / 1288, 64 (bf16) 1598 / 1242; with four waves everywhere 1 row 773, 64 rows 1327.
+// Shapes that fill the chip stay: the 7B model with 16-bit weights, these everywhere / the others, 1 row 3259 / 3100, 16 (bf16) 3621 / 3463, 40 4158 / 3978, 64 4453 / 4340, 64 (bf16)
+// 4474 / 4291; only from 17 to 32 rows 24 rows 3748 / 3851, with lm_heads (1187 blocks of 128 columns) the other way: 0.5B, 18 rows 53.4 / 49.0, 7B, 30 rows 189.8 / 185.7.
+template <int MB, int NWN, bool BF>
+void launch_gemm_w16_t(const GemmParams& p, hipStream_t st) {
+    const dim3 grid(cdiv(p.NT, NWN), p.nsplit), block(64 * NWN);
+    if (p.cps <= 2)                hipLaunchKernelGGL((gemm_wq_kernel<16, MB, 1, 0, 2, NWN, 1, BF>), grid, block, 0, st, p);
+    else if (MB > 1 || p.cps <= 4) hipLaunchKernelGGL((gemm_wq_kernel<16, MB, 1, 0, 4, NWN, 1, BF>), grid, block, 0, st, p);
+    else if constexpr (MB == 1)    hipLaunchKernelGGL((gemm_wq_kernel<16, MB, 1, 0, 8, NWN, 1, BF>), grid, block, 0, st, p);
+}
+template <int MB, bool BF>
+int launch_gemm_w16(const GemmParams& p, hipStream_t st) {
+    if (cdiv(p.NT, 4) * p.nsplit <= 64) launch_gemm_w16_t<MB, 2, BF>(p, st);
+    else                                launch_gemm_w16_t<MB, 4, BF>(p, st);
+    MI355_CHECK_LAUNCH("gemm_wq_kernel");
+    return MI355_OK;
+}
+
 int launch_gemm(const GemmParams& p, int wbits, int group_size, int cfg, hipStream_t st) {
+    if (wbits == 16) {
+        const int blocks = cdiv(p.NT * 16, kCfgBN[cfg]) * p.nsplit;
+        if (cfg == 5 && blocks <= 256) return p.bf16 ? launch_gemm_w16<1, true>(p, st) : launch_gemm_w16<1, false>(p, st);
+        if (cfg == 2 && blocks <= 512) return p.bf16 ? launch_gemm_w16<2, true>(p, st) : launch_gemm_w16<2, false>(p, st);
+        if ((cfg == 4 || cfg == 6 || cfg == 8) && blocks <= 96) return p.bf16 ? launch_gemm_w16<4, true>(p, st) : launch_gemm_w16<4, false>(p, st);
+    }
     if (p.bf16) {
         if (wbits == 16) return launch_gemm_bf16_t<16, 0, 2, 2, 2>(p, cfg, st);
         if (wbits == 4 && group_size == 128) return launch_gemm_bf16_t<4, 4, 4, 4, 4>(p, cfg, st);
