@@ -160,7 +160,7 @@ int mi355_hy_chunk_prefix_ex(const int32_t* cs, const int32_t* sc, const int32_t
 int mi355_hy_chunk_prefix_rows(const int32_t* cs, const int32_t* sc, const int32_t* slot, const int32_t* first_pos, int32_t nseq, const float* decay,
                                const float* cdecay, int32_t row_len, int32_t H, int32_t per_head, float* chunk_state, float* state, mi355_stream_t stream);
 
-/* The gated recurrences of mi355_hy_scan (modes 0 and 1) for keys of at most 128 channels, whole or as the two passes of the chunked form (out null: states and total
+/* The recurrences of mi355_hy_scan for keys of at most 128 channels, whole or as the two passes of the chunked form (out null: states and total
  * decays of the chunks; then, behind mi355_hy_chunk_prefix_rows, the walk from the chunk-start states, which are not written back: keep_state 0). */
 int mi355_hy_walk(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, const float* z, int32_t ldz, const void* lower,
                   const void* fbias, float tau, float qscale, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start, const int32_t* slot,

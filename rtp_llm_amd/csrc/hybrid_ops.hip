@@ -857,6 +857,11 @@ __device__ __forceinline__ void hy_split_bf16(float x, bf16& hi, bf16& lo) { hi 
 template <int CTRL> __device__ __forceinline__ float hy_dpp(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
+template <int CTRL> __device__ __forceinline__ double hy_dpp(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const float lo = hy_dpp<CTRL>(__builtin_bit_cast(float, (uint32_t)b)), hi = hy_dpp<CTRL>(__builtin_bit_cast(float, (uint32_t)(b >> 32)));
+    return __builtin_bit_cast(double, (uint64_t)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo));
+}
 __device__ __forceinline__ float hy_sum16(float v) {
     v += hy_dpp<0xB1>(v);      // quad_perm [1,0,3,2]
     v += hy_dpp<0x4E>(v);      // quad_perm [2,3,0,1]
@@ -1208,6 +1213,7 @@ __global__ __launch_bounds__(256) void hy_chunk_plan_kernel(const int32_t* row_s
     for (int i = threadIdx.x; i < max_chunks; i += 256) { ids[i] = i; zeros[i] = 0; ones[i] = 1; }
 }
 
+template <int AHEAD>
 __global__ __launch_bounds__(256) void hy_chunk_prefix_kernel(const int32_t* cs, const int32_t* sc, const int32_t* slot, const int32_t* first_pos, const float* decay,
                                                               int H, int per_head, float* chunk_state, float* state, const float* cdecay, int row_len) {
     const int sq = blockIdx.x, h = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
@@ -1217,11 +1223,22 @@ __global__ __launch_bounds__(256) void hy_chunk_prefix_kernel(const int32_t* cs,
     const int rows = row_len > 0 ? per_head / row_len : 1, row = row_len > 0 ? e / row_len : 0;
     float* st = state + ((size_t)slot[sq] * H + h) * per_head + e;
     float S = first_pos[sq] == 0 ? 0.f : *st;
-    for (int c = sc[sq]; c < sc[sq + 1]; ++c) {
-        float* cp = chunk_state + ((size_t)c * H + h) * per_head + e;
-        const float L = *cp;
-        *cp = S;
-        S = __builtin_fmaf(cdecay ? cdecay[((size_t)c * H + h) * rows + row] : hy_decay_pow(a, cs[c + 1] - cs[c]), S, L);
+    // AHEAD chunks' loads before their stores, which the compiler cannot tell apart
+    for (int c0 = sc[sq], n = sc[sq + 1]; c0 < n; c0 += AHEAD) {
+        float L[AHEAD], f[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int c = c0 + i;
+            if (c >= n) break;
+            L[i] = chunk_state[((size_t)c * H + h) * per_head + e];
+            f[i] = cdecay ? cdecay[((size_t)c * H + h) * rows + row] : hy_decay_pow(a, cs[c + 1] - cs[c]);
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            if (c0 + i < n) {
+                chunk_state[((size_t)(c0 + i) * H + h) * per_head + e] = S;
+                S = __builtin_fmaf(f[i], S, L[i]);
+            }
     }
     *st = S;
 }
@@ -1512,159 +1529,308 @@ __global__ __launch_bounds__(1024) void hy_scan_kernel(ScanParams p) {
     }
 }
 
-// ------------------------------------------------------------------------------------------------ gated recurrence, patches of rows and columns
-// The same recurrence (modes HGRN2 and GLA) with keys of at most 8 RPL channels: a lane holds RPL key rows x 4 value columns of the state, a wave all rows of
-// 32 columns, a block 128 columns.  What bounded hy_scan_kernel is the LDS: its threads hold 8 rows of ONE column, so every wave reads 24 broadcast floats per 24
-// multiply-adds.  Here 7 (RPL 8) wave reads of 16 bytes feed 96 multiply-adds, the gates of a token are formed once per head instead of once per 64 columns,
-// and the sum over the row groups is a three-step exchange between eight lanes (each ends with one column; no LDS, no barrier).
-// Tokens are still walked in order.  OUT: outputs are formed; without them (the first of the two passes over chunks) only the state each chunk leaves
-// from zero and, in cdecay [sequences, H, dim], the product of its decays.
-// 16 heads of 64 x 128, four sequences of 2048 tokens: 684 us as hy_scan_kernel, 683 us walked whole (64 blocks: one chain
-// of 2048 tokens each), 265 us in chunks of 128; one sequence of 1537, 8 heads: 504 us and in chunks of 32 65 us.  The error against a 64-bit walk is 2.7e-7 of the
-// state's norm, 2.8e-7 before (a chunk's carried state is rounded once per chunk, not per token).
-__device__ __forceinline__ f32x4 hy_ld4(const float* p, int n, int vec) {
-    if (vec && n >= 4) return *(const f32x4*)p;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) if (e < n) v[e] = p[e];
-    return v;
+// ------------------------------------------------------------------------------------------------ gated recurrence, tiles of 16 tokens on the matrix units
+// The same recurrence with keys of at most 64 CH channels, S_t = diag(a_t) S_(t-1) + k_t v_t^T, o_t = S_t^T q_t, 16 tokens at a time: with c_t = a_1 .. a_t inside the tile
+// and e_t = a_(t+1) .. a_16,
+//     o_t = (q_t c_t)^T S_0 + sum_(s <= t) P_ts v_s,   P_ts = sum_d q_td k_sd a_(s+1)d .. a_td,      S_16 = diag(c_16) S_0 + sum_s (k_s e_s) v_s^T.
+// Every product of decays is formed by multiplication, so a small decay underflows to what it is worth and nothing is divided.  The contractions are fp32 MFMA 16 x 16 x 4; a wave
+// holds all key rows of 32 value columns as accumulators, whose layout (row 4 (lane / 16) + r, column lane % 16) is that of the B operand over the key rows 4 (lane / 16) + r, so
+// the state is never moved; a block is 128 columns.  P (136 of 256 pairs) is formed by the vector units once per head.  Walking token by token took 5 vector operations per state
+// value and token in the two passes over chunks and was bound by them.  OUT: outputs are formed; without them (the first of the two passes over chunks) only the state each
+// chunk leaves from zero and, in cdecay [sequences, H, dim], the product of its decays.
+// 16 heads of 64 x 128, four sequences of 2048 tokens in chunks of 128: states 106.7 -> 49 us, outputs 136.5 -> 86; one sequence of 1537, 8 heads, chunks of 32: all 60.5 -> 42 us.
+// A block alone takes 4 us a tile, of which 2304 cycles are products; the rest is its chain of two barriers, LDS and exponentials, which four blocks of a compute unit hide (128
+// registers; HGRN2's outputs three).  Products of decays are formed in 64 bits (a constant decay's powers would carry one rounding from tile to tile), sums as short chains and trees.
+// Error of the outputs against a 64-bit walk, root mean square over that of the outputs, 2048 tokens of 16 heads, here / token by token: GLA 3.16e-7 / 3.47e-7, HGRN2 1.09e-7 / 1.10e-7,
+// constant decays 1.12e-7 / 1.27e-7; of the states 3.12e-7 / 3.46e-7, 2.46e-7 / 2.43e-7, 0.86e-7 / 1.08e-7.
+// sigmoid(z)^(1 / tau).  From tau = 4 on by the exponential and logarithm of the vector unit: what they and the rounding of 1 + e^-|z| put on the logarithm, about 2^-23 of
+// max(1, |z|), is divided by tau, and the exponent's own rounding is that of a decay that has left nothing (20 operations a value instead of 170: 716 of a tile's 1300 instructions).
+__device__ __forceinline__ float hy_gla_decay(float z, float tau, float itau) {
+    if (tau < 4.f) return expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) / tau);
+    const float l2e = 1.44269504f, l = __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(z) * l2e));         // base 2
+    return __builtin_amdgcn_exp2f((fminf(z, 0.f) * l2e - l) * itau);
 }
-template <typename T, int RPL, bool OUT>
-__global__ __launch_bounds__(256) void hy_walk_kernel(ScanParams p, float* cdecay, int keep_state, int vec) {
-    constexpr int DP = 8 * RPL, TOK = 16, D4 = DP / 4, QV = TOK * D4 / 256, J = RPL / 4;
-    __shared__ f32x4 q_s[OUT ? TOK * D4 : 1], k_s[TOK * D4], a_s[TOK * D4], v_s[TOK * 32];
+using f64x4 = __attribute__((ext_vector_type(4))) double;
+template <typename T, int MODE, int CH, bool OUT>
+__global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4) void hy_walk_kernel(ScanParams p, float* cdecay, int keep_state) {
+    constexpr int TOK = 16, DP = 64 * CH, DB = DP / 16, QS = DP + 4, KS = TOK + 4;
+    constexpr bool LOW = OUT && MODE == SCAN_HGRN2;     // P in two parts: its k = 1 - a and silu(q) lean to one side, so that P's own rounding and the
+                                                        // sums' show in the outputs: 1.19e-7 without, 1.15e-7 with, 1.09e-7 with 64-bit sums as well; 86 -> 107 us
+    __shared__ __attribute__((aligned(16))) float q_s[OUT ? (TOK + 3) * DP : 4], k_s[OUT ? TOK * DP : 4], a_s[OUT ? (TOK + 3) * DP : 4];      // as they are, [token][channel]; three rows of q and a are read past the tile, unused
+    __shared__ __attribute__((aligned(16))) float qc_s[OUT ? TOK * QS : 4], ke_s[DP * KS], P_s[OUT ? TOK * KS : 4], Pl_s[LOW ? TOK * KS : 4];               // q c [token][channel], k e [channel][token], P [t][s]
+    __shared__ double part_s[4][DP];                                                                                              // products of the decays of four tokens ...
+    __shared__ __attribute__((aligned(16))) float all_s[DP];                                                                      // ... and of all
     const int sq = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * 128;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rg = lane & 7, cg = lane >> 3;
-    const int r0 = p.row_start[sq], r1 = p.row_start[sq + 1], vcol = v0 + wave * 32 + cg * 4, vn = p.vdim - vcol;
-    float* st = p.state + ((size_t)p.slot[sq] * p.H + h) * p.dim * p.vdim + vcol;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+    const int r0 = p.row_start[sq], r1 = p.row_start[sq + 1], vcol = v0 + wave * 32 + c;
+    float* st = p.state + ((size_t)p.slot[sq] * p.H + h) * p.dim * p.vdim;
     const bool fresh = p.first_pos[sq] == 0, idle = v0 + wave * 32 >= p.vdim;
-    f32x4 S[RPL], A[OUT ? 1 : J];                       // row j * 32 + rg * 4 + e of the state in S[4 j + e]
+    constexpr uint32_t NONE = 0x80000000u;
+    const uint32_t vb = (uint32_t)p.vdim * 4u;
+    uint32_t s_o[2];
 #pragma unroll
-    for (int i = 0; i < RPL; ++i) {
-        const int d = (i >> 2) * 32 + rg * 4 + (i & 3);
-        S[i] = !fresh && d < p.dim ? hy_ld4(st + (size_t)d * p.vdim, vn, vec) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    if constexpr (!OUT) {
+    for (int cb = 0; cb < 2; ++cb) s_o[cb] = vcol + 16 * cb < p.vdim ? 4 * g * vb + (vcol + 16 * cb) * 4u : NONE;
+    auto ldf = [](__amdgpu_buffer_rsrc_t r, uint32_t at, uint32_t row) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, at, row, 0)); };
+    f32x4 S[DB][2];                                     // row 16 db + 4 g + r, column vcol + 16 cb
+    {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)st, 0, fresh ? 0 : (int)(p.dim * vb), 0x00020000);     // rows past the last: out of range, zeros
 #pragma unroll
-        for (int j = 0; j < J; ++j) A[j] = f32x4{1.f, 1.f, 1.f, 1.f};
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) S[db][cb][r] = ldf(rs, s_o[cb] + (16 * db + r) * vb, 0);
     }
-    f32x4 rq[QV], rk[QV], rz[QV], rv[2];                // the next pass's raw projections
+    if (OUT) for (int i = tid; i < TOK * KS; i += 256) { P_s[i] = 0.f; if (LOW) Pl_s[i] = 0.f; }             // s > t stays so
+    double A[CH];
+    // per head and channel, the same for every token
+    float lw[CH], fb[CH], fixed = 1.f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        A[j] = 1.; lw[j] = fb[j] = 0.f;
+        const int d = lane + 64 * j;
+        if (MODE == SCAN_HGRN2 && d < p.dim) { lw[j] = (float)((const T*)p.lower)[h * p.dim + d]; fb[j] = (float)((const T*)p.fbias)[h * p.dim + d]; }
+    }
+    if constexpr (MODE == SCAN_FIXED || MODE == SCAN_FIXED_SILU) fixed = ((const float*)p.lower)[h];
+    // the next tile's projections: q, k, z of tokens 4 wave + i and channel lane + 64 j (tokens past the last read the last), v of tokens 4 g + r and column vcol + 16 cb.
+    // Lanes without a channel, column or token lie out of their descriptor's range: zeros without a branch
+    float rq[CH][4], rk[CH][4], rz[CH][4];
+    f32x4 rv[2];
+    const uint32_t ldb = (uint32_t)p.ld * 4u, zb = (uint32_t)p.ldz * 4u, ob = (uint32_t)(p.H * p.vdim) * 4u;
+    uint32_t ch_o[CH], v_o[2], o_o[2];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) ch_o[j] = lane + 64 * j < p.dim ? (uint32_t)(h * p.dim + lane + 64 * j) * 4u : NONE;
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+        const bool ok = vcol + 16 * cb < p.vdim;
+        v_o[cb] = ok ? (uint32_t)(h * p.vdim + vcol + 16 * cb) * 4u + 4 * g * ldb : NONE;
+        o_o[cb] = ok ? (uint32_t)(h * p.vdim + vcol + 16 * cb) * 4u + 4 * g * ob : NONE;
+    }
+    const float itau = MODE == SCAN_GLA ? 1.f / p.tau : 1.f;
+    auto rows_of = [](const float* base, size_t row, uint32_t bytes, int n) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)base + row * bytes), 0, (int)(n * bytes), 0x00020000);
+    };
     auto fetch = [&](int t0) {
+        const int nt = min(TOK, r1 - t0);
+        const __amdgpu_buffer_rsrc_t rp = rows_of(p.proj, t0, ldb, nt), rzp = MODE == SCAN_GLA ? rows_of(p.z, t0, zb, nt) : rp;
 #pragma unroll
-        for (int e = 0; e < QV; ++e) {
-            const int i = tid + e * 256, t = t0 + i / D4, d = i % D4 * 4;
-            if (t >= r1 || d >= p.dim) continue;
-            const float* row = p.proj + (size_t)t * p.ld;
-            const int hd = h * p.dim + d, n = p.dim - d;
-            if (OUT) rq[e] = hy_ld4(row + p.qo + hd, n, vec);
-            rk[e] = hy_ld4(row + p.ko + hd, n, vec);
-            if (p.mode == SCAN_GLA) rz[e] = hy_ld4(p.z + (size_t)t * p.ldz + hd, n, vec);
+        for (int i = 0; i < 4; ++i) {
+            const int t = min(4 * wave + i, nt - 1);
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                if (OUT) rq[j][i] = ldf(rp, ch_o[j], t * ldb + p.qo * 4u);
+                rk[j][i] = ldf(rp, ch_o[j], t * ldb + p.ko * 4u);
+                if (MODE == SCAN_GLA) rz[j][i] = ldf(rzp, ch_o[j], t * zb);
+            }
         }
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int i = tid + e * 256, t = t0 + (i >> 5), c = v0 + (i & 31) * 4;
-            rv[e] = t < r1 && c < p.vdim ? hy_ld4(p.proj + (size_t)t * p.ld + p.vo + h * p.vdim + c, p.vdim - c, vec) : f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb) rv[cb][r] = ldf(rp, 4 * g + r < nt ? v_o[cb] : NONE, r * ldb + p.vo * 4u);
     };
     if (r0 < r1) fetch(r0);
-    const bool b0 = lane & 1, b1 = lane & 2;
     for (int t0 = r0; t0 < r1; t0 += TOK) {
         const int nt = min(TOK, r1 - t0);
+        float qv[CH][4], kv[CH][4], av[CH][4];
+        f32x4 v[2];
 #pragma unroll
-        for (int e = 0; e < QV; ++e) {
-            const int i = tid + e * 256, d = i % D4 * 4;
-            if (i / D4 >= nt) continue;
-            f32x4 qv = {0.f, 0.f, 0.f, 0.f}, kv = qv, av = {1.f, 1.f, 1.f, 1.f};
+        for (int j = 0; j < CH; ++j) {
+            double m = 1.;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if (d + c >= p.dim) continue;
-                const int hd = h * p.dim + d + c;
-                if (p.mode == SCAN_HGRN2) {
-                    const float lw = (float)((const T*)p.lower)[hd];
-                    const float f = lw + (1.f - lw) * hy_sigmoid(rk[e][c] + (float)((const T*)p.fbias)[hd]);
-                    if (OUT) qv[c] = hy_silu(rq[e][c]);
-                    av[c] = f; kv[c] = 1.f - f;
-                } else {
-                    const float zz = rz[e][c];
-                    const float ls = fminf(zz, 0.f) - log1pf(expf(-fabsf(zz)));       // log sigmoid(z)
-                    if (OUT) qv[c] = rq[e][c] * p.qscale;
-                    kv[c] = rk[e][c]; av[c] = expf(ls / p.tau);
+            for (int i = 0; i < 4; ++i) {
+                const int t = 4 * wave + i;
+                float x = OUT ? rq[j][i] : 0.f, k = rk[j][i], a = fixed;
+                if constexpr (MODE == SCAN_HGRN2) {
+                    a = lw[j] + (1.f - lw[j]) * hy_sigmoid(k + fb[j]);
+                    if (OUT) x = hy_silu(x);
+                    k = 1.f - a;
+                } else if constexpr (MODE == SCAN_GLA) {
+                    x *= p.qscale; a = hy_gla_decay(rz[j][i], p.tau, itau);
+                } else if constexpr (MODE == SCAN_FIXED_SILU) {
+                    if (OUT) x = hy_silu(x);
+                    k = hy_silu(k);
+                }
+                if (t >= nt || lane + 64 * j >= p.dim) { x = 0.f; k = 0.f; a = 1.f; }
+                qv[j][i] = x; kv[j][i] = k; av[j][i] = a; m *= (double)a;
+                if (OUT) {
+                    const int at = t * DP + lane + 64 * j;
+                    q_s[at] = x; k_s[at] = k; a_s[at] = a;
                 }
             }
-            if (OUT) q_s[i] = qv;
-            k_s[i] = kv; a_s[i] = av;
+            part_s[wave][lane + 64 * j] = m;
         }
 #pragma unroll
-        for (int e = 0; e < 2; ++e) v_s[tid + e * 256] = rv[e];
+        for (int cb = 0; cb < 2; ++cb) {
+            v[cb] = rv[cb];
+            if constexpr (MODE == SCAN_FIXED_SILU) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[cb][r] = hy_silu(v[cb][r]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const int d = lane + 64 * j;
+            double before = 1., behind = 1.;         // 64 bits: a constant decay's powers would carry the same rounding from tile to tile
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const double m = part_s[w][d];
+                if (w < wave) before *= m;
+                if (w > wave) behind *= m;
+            }
+            f32x4 ke;
+#pragma unroll
+            for (int i = 3; i >= 0; --i) { ke[i] = kv[j][i] * (float)behind; behind *= (double)av[j][i]; }
+            *(f32x4*)(ke_s + d * KS + 4 * wave) = ke;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                before *= (double)av[j][i];
+                if (OUT) qc_s[(4 * wave + i) * QS + d] = qv[j][i] * (float)before;
+            }
+            if (wave == 3) all_s[d] = (float)before;
+            if (!OUT) A[j] *= before;                   // the last wave's is the product of all
+        }
+        if constexpr (OUT) {
+            // lane (s = 4 wave + g, c): channels 4 c .. of P_(s + u) s, u = 0 .. 15 - s; then the sums over the 16 lanes, lane c keeps u = c
+            const int s = 4 * wave + g;
+            f32x4 kr[CH];
+            float pt[16];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) kr[j] = *(const f32x4*)(k_s + s * DP + 4 * c + 64 * j);
+#pragma unroll
+            for (int u4 = 0; u4 < 16; u4 += 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pt[u4 + e] = 0.f;
+                if (u4 > 15 - 4 * wave) continue;       // no lane of this wave
+#pragma unroll
+                for (int u = u4; u < u4 + 4; ++u)
+#pragma unroll
+                    for (int j = 0; j < CH; ++j) {
+                        const int at = (s + u) * DP + 4 * c + 64 * j;
+                        if (u) kr[j] *= *(const f32x4*)(a_s + at);
+                        const f32x4 q4 = *(const f32x4*)(q_s + at);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) pt[u] = __builtin_fmaf(kr[j][e], q4[e], pt[u]);
+                    }
+            }
+            const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+            using Sum = std::conditional_t<LOW, double, float>;
+            float p8[8];
+            Sum p4[4], p2[2];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) p8[u] = (b3 ? pt[u + 8] : pt[u]) + hy_dpp<0x140>(b3 ? pt[u] : pt[u + 8]);                   // lane 15 - i of the 16: the other half of u
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p4[u] = (Sum)(b2 ? p8[u + 4] : p8[u]) + (Sum)hy_dpp<0x141>(b2 ? p8[u] : p8[u + 4]);         // lane 7 - i of the 8
+#pragma unroll
+            for (int u = 0; u < 2; ++u) p2[u] = (b1 ? p4[u + 2] : p4[u]) + hy_dpp<0x1B>(b1 ? p4[u] : p4[u + 2]);                    // lane 3 - i of the 4
+            const Sum p1 = (b0 ? p2[1] : p2[0]) + hy_dpp<0xB1>(b0 ? p2[0] : p2[1]);
+            if (s + c < 16) {
+                P_s[(s + c) * KS + s] = (float)p1;
+                if constexpr (LOW) Pl_s[(s + c) * KS + s] = (float)(p1 - (double)(float)p1);
+            }
+        }
         __syncthreads();
         if (t0 + TOK < r1) fetch(t0 + TOK);
-        if (!idle) {
-            // stores through a descriptor over the pass's rows, lanes without a column out of its range: no branch in the walk, so that the reads of later tokens
-            // move up between the products of earlier ones
-            const uint32_t row_bytes = (uint32_t)p.H * p.vdim * 4u;
-            const int oc = vcol + (b0 ? 2 : 0) + (b1 ? 1 : 0);
-            const uint32_t voff = !(lane & 4) && oc < p.vdim ? (uint32_t)(h * p.vdim + oc) * 4u : 0x80000000u;
-            __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(OUT ? (void*)(p.out + (size_t)t0 * p.H * p.vdim) : (void*)p.state, 0, OUT ? (int)(nt * row_bytes) : 0, 0x00020000);
-            auto token = [&](int t) {
-                const f32x4 vt = v_s[t * 32 + wave * 8 + cg];
-                f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int j = 0; j < J; ++j) {
-                    const f32x4 a4 = a_s[t * D4 + j * 8 + rg], k4 = k_s[t * D4 + j * 8 + rg];
-                    f32x4 q4 = a4;
-                    if constexpr (OUT) q4 = q_s[t * D4 + j * 8 + rg];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            S[j * 4 + e][c] = __builtin_fmaf(a4[e], S[j * 4 + e][c], k4[e] * vt[c]);      // rounds the small product and the sum, not the decayed state as well
-                            if constexpr (OUT) o[c] = __builtin_fmaf(S[j * 4 + e][c], q4[e], o[c]);
-                        }
-                    if constexpr (!OUT) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) A[j][e] *= a4[e];
-                    }
-                }
-                if constexpr (OUT) {
-                    // sum over the eight row groups: halves of the columns to the neighbour, then a quarter, then the other four lanes' sums
-                    float k0 = b0 ? o[2] : o[0], k1 = b0 ? o[3] : o[1];
-                    k0 += hy_dpp<0xB1>(b0 ? o[0] : o[2]);
-                    k1 += hy_dpp<0xB1>(b0 ? o[1] : o[3]);
-                    float k = b1 ? k1 : k0;
-                    k += hy_dpp<0x4E>(b1 ? k0 : k1);
-                    k += hy_dpp<0x104>(k);                                  // lane + 4
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, k), ro, voff, (uint32_t)t * row_bytes, 0);
-                }
+        if (idle) continue;
+        if constexpr (OUT) {
+            const __amdgpu_buffer_rsrc_t ro = rows_of(p.out, t0, ob, nt);
+            // sums of eight products, then a tree: one chain of 80 would round a tenth more than the token-by-token walk's short sums did
+            auto pair = [](float a0, float a1, float b0, float b1) {
+                const f32x4 x = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                return __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, x, 0, 0, 0);
             };
-            if (nt == TOK) {
-#pragma unroll 4
-                for (int t = 0; t < TOK; ++t) token(t);
+            using Acc = std::conditional_t<LOW, f64x4, f32x4>;
+            auto wide = [](const f32x4& x) { return __builtin_convertvector(x, Acc); };
+            // P times a tile of values
+            auto within = [&](const f32x4& x, const f32x4& ph, const f32x4& pq) {
+                Acc y = wide(pair(ph[0], ph[1], x[0], x[1])) + wide(pair(ph[2], ph[3], x[2], x[3]));
+                if constexpr (LOW) y += wide(__builtin_amdgcn_mfma_f32_16x16x4f32(pq[3], x[3], __builtin_amdgcn_mfma_f32_16x16x4f32(pq[2], x[2], pair(pq[0], pq[1], x[0], x[1]), 0, 0, 0), 0, 0, 0));
+                return y;
+            };
+            Acc o[2], two[2], four[2];
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                if (db % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+                const f32x4 q4 = *(const f32x4*)(qc_s + c * QS + 16 * db + 4 * g);
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) {
+                    const f32x4 x = pair(q4[0], q4[1], S[db][cb][0], S[db][cb][1]), y = pair(q4[2], q4[3], S[db][cb][2], S[db][cb][3]);
+                    const Acc xy = wide(x) + wide(y);
+                    if (db % 2 == 0) two[cb] = xy;
+                    else if (db % 4 == 1) four[cb] = two[cb] + xy;
+                    else if (db == 3) o[cb] = four[cb] + (two[cb] + xy);
+                    else o[cb] += four[cb] + (two[cb] + xy);
+                }
+            }
+            // an infinite or undefined value of a later token must not meet the zeros of P: those tiles sum token by token
+            const f32x4 p4 = *(const f32x4*)(P_s + c * KS + 4 * g);
+            f32x4 pl = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (LOW) pl = *(const f32x4*)(Pl_s + c * KS + 4 * g);
+            float odd = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) odd += v[0][r] * 0.f + v[1][r] * 0.f;
+            if (!__any(odd != 0.f)) {
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) o[cb] += within(v[cb], p4, pl);
             } else {
-                for (int t = 0; t < nt; ++t) token(t);
+#pragma unroll 1
+                for (int t = 0; t < TOK; ++t) {
+                    Acc x[2];
+#pragma unroll
+                    for (int cb = 0; cb < 2; ++cb) {
+                        f32x4 u;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) u[r] = 4 * g + r <= t ? v[cb][r] : 0.f;
+                        x[cb] = o[cb] + within(u, p4, pl);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int cb = 0; cb < 2; ++cb) o[cb][r] = 4 * g + r == t ? x[cb][r] : o[cb][r];
+                }
             }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) {
+                    const float x = (float)o[cb][r];
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), ro, 4 * g + r < nt ? o_o[cb] : NONE, r * ob, 0);
+                }
         }
-        __syncthreads();
+        // the tile's own sum by itself, then one rounding at the state's magnitude instead of sixteen
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            if (db % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+            const f32x4 k4 = *(const f32x4*)(ke_s + (16 * db + c) * KS + 4 * g), all = *(const f32x4*)(all_s + 16 * db + 4 * g);
+            f32x4 own[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) own[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[r], v[cb][r], own[cb], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) S[db][cb][r] = __builtin_fmaf(all[r], S[db][cb][r], own[cb][r]);
+        }
     }
-    if (keep_state && vn > 0) {
+    if (keep_state) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)st, 0, (int)(p.dim * vb), 0x00020000);
+        asm volatile("" : "+v"(s_o[0]), "+v"(s_o[1]));   // the addresses are formed again: not held in registers since the loads
 #pragma unroll
-        for (int i = 0; i < RPL; ++i) {
-            const int d = (i >> 2) * 32 + rg * 4 + (i & 3);
-            if (d >= p.dim) continue;
-            float* to = st + (size_t)d * p.vdim;
-            if (vec && vn >= 4) *(f32x4*)to = S[i];
-            else {
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) if (c < vn) to[c] = S[i][c];
-            }
-        }
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) {
+                    const float x = S[db][cb][r];
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), rs, s_o[cb] + (16 * db + r) * vb, 0, 0);
+                }
     }
     if constexpr (!OUT) {
-        if (cdecay && wave == 0 && cg == 0 && blockIdx.z == 0) {
+        if (cdecay && wave == 3 && blockIdx.z == 0) {
 #pragma unroll
-            for (int j = 0; j < J; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (j * 32 + rg * 4 + e < p.dim) cdecay[((size_t)sq * p.H + h) * p.dim + j * 32 + rg * 4 + e] = A[j][e];
+            for (int j = 0; j < CH; ++j)
+                if (lane + 64 * j < p.dim) cdecay[((size_t)sq * p.H + h) * p.dim + lane + 64 * j] = (float)A[j];
         }
     }
 }
@@ -2919,28 +3085,37 @@ extern "C" int mi355_hy_chunk_prefix_rows(const int32_t* cs, const int32_t* sc, 
                                           const float* cdecay, int32_t row_len, int32_t H, int32_t per_head, float* chunk_state, float* state, mi355_stream_t stream) {
     MI355_CHECK_ARG(cs && sc && slot && first_pos && (decay || cdecay) && chunk_state && state && nseq > 0 && H > 0 && per_head > 0, "hy_chunk_prefix: nseq=%d H=%d", nseq, H);
     MI355_CHECK_ARG(row_len == 0 || (row_len > 0 && per_head % row_len == 0 && cdecay), "hy_chunk_prefix: rows of %d in %d", row_len, per_head);
-    hipLaunchKernelGGL(hy_chunk_prefix_kernel, dim3(nseq, H, (per_head + 255) / 256), dim3(256), 0, (hipStream_t)stream, cs, sc, slot, first_pos, decay, H, per_head,
-                       chunk_state, state, cdecay, row_len);
+    // A few blocks wait for one chunk after the other; a chip full of them is bound by the states' bytes and wants the smaller loop: 48 chunks of 8 heads of 64 x 128 18.5 us one at a
+    // time, 11.0 in eights; 4 sequences of 16 chunks of 16 heads 13.9 / 14.4, 8 of 3 chunks 9.1 / 10.4.
+    const dim3 grid(nseq, H, (per_head + 255) / 256);
+    if ((uint64_t)grid.x * grid.y * grid.z <= 1024)
+        hipLaunchKernelGGL(hy_chunk_prefix_kernel<8>, grid, dim3(256), 0, (hipStream_t)stream, cs, sc, slot, first_pos, decay, H, per_head, chunk_state, state, cdecay, row_len);
+    else
+        hipLaunchKernelGGL(hy_chunk_prefix_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, cs, sc, slot, first_pos, decay, H, per_head, chunk_state, state, cdecay, row_len);
     MI355_CHECK_LAUNCH("hy_chunk_prefix_kernel");
     return MI355_OK;
 }
 
-// The gated recurrences of mi355_hy_scan (modes 0 and 1: HGRN2, GLA) on patches of rows and columns (hy_walk_kernel): dim <= 128, MI355_ERR_UNSUPPORTED beyond.  out null: only the states (and
+// The recurrences of mi355_hy_scan on tiles of 16 tokens (hy_walk_kernel): dim <= 128, MI355_ERR_UNSUPPORTED beyond.  out null: only the states (and
 // cdecay fp32 [nseq, H, dim], the product of the sequence's decays per key row, unless null).  keep_state 0: the states are read, not written back.
 extern "C" int mi355_hy_walk(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, const float* z, int32_t ldz, const void* lower,
                              const void* fbias, float tau, float qscale, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start, const int32_t* slot,
                              const int32_t* first_pos, int32_t nseq, float* state, float* out, float* cdecay, int32_t keep_state, int32_t act_dtype, mi355_stream_t stream) {
     MI355_CHECK_ARG(proj && row_start && slot && first_pos && state && nseq > 0 && H > 0 && dim > 0 && vdim > 0, "hy_walk: bad argument");
-    MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : (mode == SCAN_GLA && z && tau > 0.f), "hy_walk: mode %d lacks its gate inputs", mode);
+    MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : mode == SCAN_GLA ? (z && tau > 0.f) : ((mode == SCAN_FIXED || mode == SCAN_FIXED_SILU) && lower),
+                    "hy_walk: mode %d lacks its gate inputs", mode);
     if (dim > 128) return MI355_ERR_UNSUPPORTED;
-    auto al = [](const void* q) { return (uintptr_t)q % 16 == 0; };
-    const int vec = dim % 4 == 0 && vdim % 4 == 0 && ld % 4 == 0 && qo % 4 == 0 && ko % 4 == 0 && vo % 4 == 0 && al(proj) && al(state) &&
-                    (mode != SCAN_GLA || (al(z) && ldz % 4 == 0));
     const ScanParams p{proj, ld, qo, ko, vo, z, ldz, lower, fbias, tau, qscale, mode, H, dim, vdim, row_start, slot, first_pos, state, out, 16, 0, {}};
     const dim3 grid(nseq, H, (vdim + 127) / 128);
-#define HY_WALK(RPL_, OUT_) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_walk_kernel<T, RPL_, OUT_>), grid, dim3(256), 0, (hipStream_t)stream, p, cdecay, keep_state, vec))
-    if (dim <= 64) { if (out) HY_WALK(8, true); else HY_WALK(8, false); }
-    else           { if (out) HY_WALK(16, true); else HY_WALK(16, false); }
+#define HY_WALK(T_, MODE_) do { \
+        if (dim <= 64) { if (out) hipLaunchKernelGGL((hy_walk_kernel<T_, MODE_, 1, true>), grid, dim3(256), 0, (hipStream_t)stream, p, cdecay, keep_state); \
+                         else     hipLaunchKernelGGL((hy_walk_kernel<T_, MODE_, 1, false>), grid, dim3(256), 0, (hipStream_t)stream, p, cdecay, keep_state); } \
+        else           { if (out) hipLaunchKernelGGL((hy_walk_kernel<T_, MODE_, 2, true>), grid, dim3(256), 0, (hipStream_t)stream, p, cdecay, keep_state); \
+                         else     hipLaunchKernelGGL((hy_walk_kernel<T_, MODE_, 2, false>), grid, dim3(256), 0, (hipStream_t)stream, p, cdecay, keep_state); } } while (0)
+    if (mode == SCAN_HGRN2)     HY_DISPATCH(act_dtype, HY_WALK(T, SCAN_HGRN2));
+    else if (mode == SCAN_GLA)  HY_WALK(float, SCAN_GLA);                          // T is that of the gate's own tensors
+    else if (mode == SCAN_FIXED) HY_WALK(float, SCAN_FIXED);
+    else                        HY_WALK(float, SCAN_FIXED_SILU);
 #undef HY_WALK
     MI355_CHECK_LAUNCH("hy_walk_kernel");
     return MI355_OK;

@@ -3,6 +3,7 @@ family (csrc/gemm_dense.hip, csrc/hybrid_ops.hip).  As in ``ops``: PyTorch suppl
 function enqueues hand-written HIP kernels and never falls back.  Activations and weights are bfloat16 or float32 (`act`); what the
 family keeps in 32-bit (residual stream, projections that feed gates and rotations, recurrent state, logits) is float32 in both."""
 import ctypes as C
+import functools
 from typing import Optional
 
 import torch
@@ -476,15 +477,10 @@ SCAN_BLOCKS_AT_ONCE = 512  # blocks of the scan kernel the chip runs side by sid
 WALK_MAX_DIM = 128         # key channels of mi355_hy_walk
 
 
+@functools.lru_cache(maxsize=64)      # the layers of a step ask for the same
 def gated_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int) -> Optional[int]:
-    """How a gated recurrence of keys up to WALK_MAX_DIM channels runs: a chunk size (hy_walk over chunks), 0 (hy_walk, whole) or None (hy_scan, whole).
-    A model of the three in us, fitted to 460 calls of 2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64 sequences of 1 to 2048 rows: a call takes what its
-    longest sequence (chunk) walks in series, or the rounds of its blocks if that is more.  hy_scan: blocks of 64 columns and a wave for 8 key rows, 16 waves on a compute unit,
-    0.28 (keys of 32) to 0.45 (128) a token.  hy_walk: blocks of 128 columns, 0.42 a token, or 0.75 and one block on a compute unit from 65 key channels on; with few blocks, or
-    values of 64 that leave half a block idle, that loses to hy_scan.  Chunks: two passes of it, launches and the chunk states.  In those calls the pick is never slower
-    than hy_scan by more than 2 %, 4 % off the fastest in the mean.
-    Measured, us, hy_scan / whole / chunks: 16 heads of 64 x 128, 4 x 2048 rows 684 / 683 / 265, 1 x 2048 668 / - / 105; 4 heads of 96 x 64, 37 sequences of up to 317
-    141 / 237 / 286; 8 heads of 128 x 256, 8 x 195 105 / 137 / 181; 32 heads of 128 x 128, 9 x 136 208 / 331 / -, 16 x 339 694 / 495 / -."""
+    """How a gated recurrence of keys up to WALK_MAX_DIM channels runs where even a walk token by token gains on hy_scan: a chunk size, 0 (whole) or None (no gain; tiles_form looks
+    again).  A model of the forms in us, fitted to 460 calls of such a walk: 2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64 sequences of 1 to 2048 rows."""
     longest = max_rows if max_rows > 0 else T - (nseq - 1)
     waves = -(-dim // 8)
     scan_us = 5.5 + (0.22 + 0.0145 * waves) * max(longest, -(-nseq * heads * -(-vdim // 64) // (256 * (16 // waves))) * T / nseq)
@@ -498,6 +494,30 @@ def gated_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int
             if t < us:
                 best, us = C, t
     return best if 1.05 * us < scan_us else None
+
+
+CHUNKS_HOST_US = 25        # two more launches and two buffers of a call in chunks: shows where launches bound a step (two prompts of 99 rows, 8 layers: 940 us, 1087 in chunks)
+
+
+@functools.lru_cache(maxsize=64)
+def tiles_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int, margin: float = 1.05) -> Optional[int]:
+    """How a recurrence of keys up to WALK_MAX_DIM channels runs: hy_walk over chunks of the size returned, hy_walk whole (0) or hy_scan (None).  A model of the forms in us: what the
+    longest sequence (chunk) takes in series, or what the chip takes for all tokens if that is more.  Fitted to 120 calls of 2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64
+    sequences of 2 to 2048 rows: 10 to 13 % off in the root mean square; the pick is 2 % off the fastest in the mean (chunks with their host time), at most 35 %, and 1 %
+    behind hy_scan at worst.  HGRN2 asks for a wider margin: hy_scan is 10 % faster there and the tiles, with 64-bit sums, 15 to 20 % slower.
+    Measured, us, hy_scan / whole / chunks: 16 heads of 64 x 128, 4 x 2048 rows 673 / 581 / 156 (128), 8 x 40 20 / 19 / 32 (32); 32 heads of 128 x 128, 9 x 136 227 / 83 / 138 (64);
+    8 heads of 128 x 256, 8 x 195 115 / 81 / 82 (64); 16 heads of 32 x 64, 16 x 2 7.6 / 10.4 / -."""
+    longest = max_rows if max_rows > 0 else T - (nseq - 1)
+    waves, work, wide = -(-dim // 8), T * heads * -(-vdim // 128), dim > 64
+    scan_us = 7.1 + (0.254 + 0.0108 * waves) * max(longest, 2.51 * T * heads * -(-vdim // 64) / (256 * (16 // waves)))
+    best, us = 0, 10.0 + 0.34 * max(longest, work / 170) if wide else 9.0 + 0.26 * max(longest, work / 200)
+    for C in (32, 64, 128):
+        if longest > C:
+            states = (T / C + 0.5 * nseq) * heads * dim * vdim * 1e-6
+            t = CHUNKS_HOST_US + (11.4 + 0.512 * max(C, work / 333) + 4.2 * states if wide else 11.8 + 0.348 * max(C, work / 384) + 5.5 * states)
+            if t < us:
+                best, us = C, t
+    return best if margin * us < scan_us else None
 
 
 def scan_prefers_chunks(T: int, nseq: int, max_rows: int, heads: int, vdim: int, C: int) -> bool:
@@ -528,10 +548,10 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
          heads: int, dim: int, vdim: int, row_start, slot, first_pos, state: torch.Tensor, act: torch.dtype, *, plans: Optional[dict] = None,
          chunked: Optional[bool] = None, max_rows: int = 0) -> torch.Tensor:
     """Gated linear recurrence over the rows of every sequence, continuing (and leaving) the fp32 state of its slot -> fp32 [T, heads * vdim].
-    Long prompt portions run in chunks that are walked side by side, the same sums in another order, when that is expected to be faster (few long sequences;
-    max_rows = the rows of the step's longest sequence when the caller knows it).  The modes with a constant decay per head (SCAN_FIXED, SCAN_FIXED_SILU):
-    every chunk from a zero state, a prefix over each sequence's chunks, then the chunk-start states' share of the outputs (scan_prefers_chunks).
-    The gated modes: what every chunk leaves from a zero state and its total decays, the prefix, then the tokens again from the chunk-start states (gated_form).
+    Keys of up to WALK_MAX_DIM channels run on tiles of tokens (hy_walk) where that is expected to be faster (gated_form, tiles_form; max_rows = the rows of the step's longest
+    sequence when the caller knows it), long portions in chunks side by side, the same sums in another order: what every chunk leaves from a zero state and its total decays, a prefix
+    over each sequence's chunks, then the tokens again from the chunk-start states.  Longer keys under a constant decay per head (SCAN_FIXED, SCAN_FIXED_SILU) walk token by token,
+    in chunks where that pays (scan_prefers_chunks): every chunk from a zero state, the prefix, then the chunk-start states' share of the outputs.
     plans: a dict that keeps the step's chunk plan between calls (the layers of one step share it); chunked forces the choice."""
     _dev(proj, torch.float32, "scan.proj"); _dev(state, torch.float32, "scan.state")
     T = proj.shape[0]
@@ -547,13 +567,15 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
                                           act_code(act), _stream()), "hy_scan")
 
     fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
-    if not fixed and chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim):
+    if chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim):
         def walk(rs, sl, fp, n, st, dst, cdecay, keep):
             _C.check_hybrid(lib.mi355_hy_walk(mode, proj.data_ptr(), ld, qo, ko, vo, _p(z), 0 if z is None else _rows(z, "scan.z"), _p(lower), _p(fbias), float(tau),
                                               float(qscale), heads, dim, vdim, rs.data_ptr(), sl.data_ptr(), fp.data_ptr(), n, st.data_ptr(), _p(dst), _p(cdecay), keep,
                                               act_code(act), _stream()), "hy_walk")
 
-        C = gated_form(T, nseq, max_rows, heads, dim, vdim)
+        C = None if fixed else gated_form(T, nseq, max_rows, heads, dim, vdim)
+        if C is None:
+            C = tiles_form(T, nseq, max_rows, heads, dim, vdim, 1.35 if mode == SCAN_HGRN2 else 1.05)       # HGRN2: hy_scan 10 % faster, the tiles (64-bit sums) 15 to 20 % slower
         if C is None:
             run(mode, row_start, slot, first_pos, nseq, state)
             return out

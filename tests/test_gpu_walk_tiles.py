@@ -1,0 +1,89 @@
+"""hy_walk's tiles of 16 tokens in the forms that scan may pick, forced here: whole and in chunks, every mode, around the tile's and the chunk's edges, keys and values that fill no
+16 or 64.  Errors as in test_gpu_walk.py: the 2-norm over that of the same walk of absolute values, 3 sqrt(32) 2^-24 = 1e-6; a constant decay of at most 0.96 remembers 32 tokens too.
+An infinite or undefined value reaches its own token's outputs and later ones, no earlier ones and no other head or column."""
+import pytest
+import torch
+
+from rtp_llm_amd import hybrid_ops as hops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _run(monkeypatch, C, mode, proj, qo, ko, vo, z, lower, fbias, tau, H, dim, vdim, starts, slot, first, state, longest):
+    monkeypatch.setattr(hops, "gated_form", lambda *a: C)
+    monkeypatch.setattr(hops, "tiles_form", lambda *a: C)
+    return hops.scan(mode, proj, qo, ko, vo, z, lower, fbias, tau, dim ** -0.5, H, dim, vdim, starts, slot, first, state, torch.bfloat16, plans={}, max_rows=longest)
+
+
+@pytest.mark.parametrize("mode,tau", [(hops.SCAN_GLA, 16.0), (hops.SCAN_GLA, 1.0), (hops.SCAN_HGRN2, 1.0), (hops.SCAN_FIXED, 1.0), (hops.SCAN_FIXED_SILU, 1.0)])
+@pytest.mark.parametrize("H,dim,vdim,off", [(2, 64, 128, 0), (1, 5, 3, 1), (3, 17, 48, 2), (2, 65, 33, 1), (1, 128, 144, 0)])
+@pytest.mark.parametrize("C", [0, 32])
+def test_forms(monkeypatch, mode, tau, H, dim, vdim, off, C):
+    lens = [1, 15, 16, 17, 33, 65, 97]
+    g = torch.Generator(device=DEV).manual_seed(dim + vdim)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    T, n = sum(lens), len(lens)
+    proj, z = r(T, off + 2 * H * dim + H * vdim + 3), r(T, H * dim) + 2
+    fixed = mode in (hops.SCAN_FIXED, hops.SCAN_FIXED_SILU)
+    lower = torch.linspace(0.5, 0.96, H, device=DEV) if fixed else torch.rand(H * dim, device=DEV, generator=g).bfloat16()
+    fbias = r(H * dim).bfloat16()
+    qo, ko, vo = off, off + H * dim, off + 2 * H * dim
+    slot = torch.randperm(n + 1, device=DEV, generator=g)[:n].int()
+    first = torch.tensor([0 if i % 2 else 9 for i in range(n)], dtype=torch.int32, device=DEV)
+    starts = torch.tensor([sum(lens[:i]) for i in range(n + 1)], dtype=torch.int32, device=DEV)
+    state = r(n + 1, H, dim, vdim)
+    before = state.clone()
+    out = _run(monkeypatch, C, mode, proj, qo, ko, vo, z, lower, fbias, tau, H, dim, vdim, starts, slot, first, state, max(lens))
+    d = lambda o, c: proj[:, o:o + H * c].double().view(T, H, c)
+    silu = torch.nn.functional.silu
+    q, k, v = d(qo, dim), d(ko, dim), d(vo, vdim)
+    if mode == hops.SCAN_GLA:
+        q, a = q * dim ** -0.5, torch.exp(torch.nn.functional.logsigmoid(z.double()) / tau).view(T, H, dim)
+    elif mode == hops.SCAN_HGRN2:
+        low = lower.double().view(H, dim)
+        a = low + (1 - low) * torch.sigmoid(k + fbias.double().view(H, dim))
+        q, k = silu(q), 1 - a
+    else:
+        a = lower.double()[None, :, None].expand(T, H, dim)
+        if mode == hops.SCAN_FIXED_SILU:
+            q, k, v = silu(q), silu(k), silu(v)
+
+    def walk(q, k, v, S):
+        o = []
+        for t in range(lo, hi):
+            S = S * a[t][:, :, None] + k[t][:, :, None] * v[t][:, None, :]
+            o.append((S * q[t][:, :, None]).sum(1))
+        return torch.stack(o), S
+
+    rel = lambda x, y, scale: float((x.double() - y).norm() / scale.norm())
+    for i in range(n):
+        lo, hi = int(starts[i]), int(starts[i + 1])
+        S0 = before[int(slot[i])].double() * (int(first[i]) > 0)
+        o, S = walk(q, k, v, S0)
+        o_abs, S_abs = walk(q.abs(), k.abs() + (mode == hops.SCAN_HGRN2), v.abs(), S0.abs())
+        assert rel(out[lo:hi].view(hi - lo, H, vdim), o, o_abs) < 1e-6
+        assert rel(state[int(slot[i])], S, S_abs) < 1e-6
+    unused = [i for i in range(n + 1) if i not in slot.tolist()]
+    assert torch.equal(state[unused], before[unused])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("C", [0, 32])
+def test_undefined_values_stay_behind_their_token(monkeypatch, C, bad):
+    H, dim, vdim, T, at = 2, 64, 64, 70, 41
+    g = torch.Generator(device=DEV).manual_seed(1)
+    proj, z = torch.randn(T, 2 * H * dim + H * vdim, device=DEV, generator=g), torch.randn(T, H * dim, device=DEV, generator=g) + 2
+    index = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    outs = []
+    for x in (None, bad):
+        p = proj.clone()
+        if x is not None:
+            p[at, 2 * H * dim + 5] = x                     # head 0, column 5
+        outs.append(_run(monkeypatch, C, hops.SCAN_GLA, p, 0, H * dim, 2 * H * dim, z, None, None, 16.0, H, dim, vdim, index(0, T), index(0), index(0),
+                         torch.zeros(1, H, dim, vdim, device=DEV), T))
+    good, odd = outs
+    assert torch.equal(good[:at], odd[:at]) and not torch.isfinite(odd[at:, 5]).any()
+    rest = [c for c in range(H * vdim) if c != 5]
+    tol = 1e-6 * float(good.abs().max()) * dim ** 0.5      # the tile with the bad value sums its products in another order
+    assert float((good[:, rest] - odd[:, rest]).abs().max()) < tol
