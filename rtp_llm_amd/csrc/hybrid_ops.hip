@@ -2199,6 +2199,37 @@ __global__ __launch_bounds__(1024) void hy_head_norm_kernel(const float* o, int 
 }
 
 
+// The same for heads of up to 4 G channels whose rows lie on 16 bytes: G lanes have four channels each of one head, all loads at once, one trip to memory where the kernel above makes two
+// of 4 bytes a lane.  8192 rows of 16 heads of 128 with gate: 77.3 -> 36.4 us (4.6 TB/s).
+template <typename T, int G>
+__global__ __launch_bounds__(256) void hy_head_norm4_kernel(const float* o, int ldo, int H, int vdim, const T* w, float eps, const float* gate, int ldg, int goff, T* out,
+                                                            int w_heads, int gate_sigmoid, const float* den, int heads) {
+    using T4 = __attribute__((ext_vector_type(4))) T;
+    const int i = blockIdx.x * (256 / G) + threadIdx.x / G, c = threadIdx.x % G * 4;
+    if (i >= heads) return;                             // whole groups of G lanes
+    const int r = i / H, h = i - r * H;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f}, gz = v, wv = {1.f, 1.f, 1.f, 1.f};
+    if (c < vdim) {
+        v = *(const f32x4*)(o + (size_t)r * ldo + (size_t)h * vdim + c);
+        if (gate) gz = *(const f32x4*)(gate + (size_t)r * ldg + goff + h * vdim + c);
+        if (w) wv = __builtin_convertvector(*(const T4*)(w + (w_heads ? h * vdim : 0) + c), f32x4);
+    }
+    if (den) v *= 1.f / den[i];
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(v[e], v[e], ss);
+#pragma unroll
+    for (int m = G / 2; m; m >>= 1) ss += __shfl_xor(ss, m, G);
+    if (c >= vdim) return;
+    v *= 1.f / sqrtf(ss / (float)vdim + eps);
+    if (w) v *= wv;
+    if (gate) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= gate_sigmoid ? hy_sigmoid(gz[e]) : hy_silu(gz[e]);
+    }
+    *(T4*)(out + (size_t)i * vdim + c) = __builtin_convertvector(v, T4);
+}
+
 // ------------------------------------------------------------------------------------------------ recurrences of a few rows: gates, update, output, norm and output gate in one launch
 // A decode step's recurrence took four launches (the low-rank decay's second linear, the scan over blocks of 64 value columns, the norm over whole heads, and the launch of the
 // first low-rank linear, now a part of the input linear) of 4 to 6 us each for a state of a few MB.  Here a block has a head of one sequence: thread (kg, cg) holds four value
@@ -3180,6 +3211,18 @@ extern "C" int mi355_hy_head_norm_ex3(const float* o, int32_t ldo, int32_t rows,
                                       int32_t goff, void* out, int32_t w_heads, int32_t gate_sigmoid, const float* den, int32_t act_dtype,
                                       mi355_stream_t stream) {
     MI355_CHECK_ARG(o && out && rows > 0 && H > 0 && vdim > 0 && ldo >= H * vdim, "hy_head_norm: bad argument");
+    const size_t tb = act_dtype == MI355_ACT_F32 ? 16 : 8;
+    auto on = [](const void* q, size_t b) { return (uintptr_t)q % b == 0; };
+    if (vdim % 4 == 0 && vdim <= 256 && ldo % 4 == 0 && on(o, 16) && on(out, tb) && (!w || on(w, tb)) && (!gate || (ldg % 4 == 0 && goff % 4 == 0 && on(gate, 16))) &&
+        (int64_t)rows * H <= INT32_MAX - 256) {
+        const int n = rows * H, G = vdim <= 32 ? 8 : vdim <= 64 ? 16 : vdim <= 128 ? 32 : 64;
+#define HY_HEAD_NORM4(G_) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_head_norm4_kernel<T, G_>), dim3((n + 256 / G_ - 1) / (256 / G_)), dim3(256), 0, (hipStream_t)stream, o, ldo, H, \
+                                      vdim, (const T*)w, eps, gate, ldg, goff, (T*)out, w_heads, gate_sigmoid, den, n))
+        if (G == 8) HY_HEAD_NORM4(8); else if (G == 16) HY_HEAD_NORM4(16); else if (G == 32) HY_HEAD_NORM4(32); else HY_HEAD_NORM4(64);
+#undef HY_HEAD_NORM4
+        MI355_CHECK_LAUNCH("hy_head_norm4_kernel");
+        return MI355_OK;
+    }
     HY_DISPATCH(act_dtype, hipLaunchKernelGGL(hy_head_norm_kernel<T>, dim3(rows, H), dim3(vdim > 256 ? std::min(1024, (vdim + 255) / 256 * 64) : 64), 0, (hipStream_t)stream, o, ldo, H, vdim, (const T*)w, eps,
                                               gate, ldg, goff, (T*)out, w_heads, gate_sigmoid, den));
     MI355_CHECK_LAUNCH("hy_head_norm_kernel");
