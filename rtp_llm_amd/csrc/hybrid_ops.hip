@@ -15,8 +15,6 @@
 // sequence; a sequence carries its block-table row, its state slot and the range of its rows.  What the model states as 32-bit is fp32
 // here whatever the activation type T (bf16 or float): positions and angles, scores and softmax, norms, gates, decays, states, residual.
 #include <algorithm>
-#include <cstdlib>
-
 #include "common.h"
 #include "../../include/mi355_hybrid.h"
 
@@ -655,7 +653,7 @@ __global__ __launch_bounds__(1024) void hy_attn_rows_kernel(const float* q, int 
     for (int i = 0; i < 8; ++i) qv[i] = (coop && kl_ok) ? q_s[kl * 8 + i] : 0.f;
     // 64 keys a wave and trip; of short contexts 16 or 32, so that all waves have some: 8 rows of 16 heads over about 100 keys 15.7 us on two
     // of sixteen waves, 12.3 on seven
-    const int tile = nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;
+    const int tile = (const void*)kcache == (const void*)vcache ? 64 : nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;        // a latent cache's rows: 64 as ever
     for (int t0 = (sp * NW + wave) * tile; t0 < nvis; t0 += tile * NW * S) {
         const int kj = t0 + lane < kept ? t0 + lane : t0 + lane - kept + lo;
         const bool valid = lane < tile && kj <= p;
@@ -884,6 +882,7 @@ __device__ __forceinline__ float hy_sum_groups(float v) {
     hy_swap<32>(v, a, b); v = a + b;
     hy_swap<16>(v, a, b); return a + b;
 }
+constexpr int AT_SOLO = 20;                       // walks of up to this many steps (640 keys) gain little from a second group (18.7 / 17.5 us at 256 rows) and keep one group's sums
 constexpr int AT_STAGES = 3, AT_PAGES = 1024;     // block-table entries of the walked range held in LDS
 
 // DK: 32-channel steps of a key row.  NCBM: 16-channel fragments of a value row the instance holds; they are multiplied by fours (fragments past the row's end hold what lies
@@ -983,17 +982,18 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
         auto step_key = [&](int st) { return (st < nkept ? 0 : kstart - 32 * nkept) + 32 * st; };
         auto page_of = [&](int k) { return psh >= 0 ? k >> psh : k / g.page; };
         int bt0 = INT_MIN;                                    // first block-table entry in LDS
-        const int rounds = (nsteps + KG - 1) / KG;
+        const int ks = nsteps > AT_SOLO ? KG : 1;             // groups at work on this run; the others keep to the barriers
+        const int rounds = (nsteps + ks - 1) / ks;
         auto issue = [&](int round, int buf) {                // KG steps, one a group (several only without kept tokens: their keys follow each other)
-            const int plo = page_of(step_key(round * KG)), phi = page_of(min(step_key(round * KG) + 32 * KG - 1, klast));
+            const int plo = page_of(step_key(round * ks)), phi = page_of(min(step_key(round * ks) + 32 * ks - 1, klast));
             if (bt0 == INT_MIN || plo < bt0 || phi >= bt0 + AT_PAGES) {        // seldom: the same for the whole block
                 __syncthreads();
                 bt0 = plo;
                 for (int i = threadIdx.x; i < AT_PAGES; i += 256 * KG) if (bt0 + i <= page_of(klast)) bt_s[i] = bt[bt0 + i];
                 __syncthreads();
             }
-            if (round * KG + group >= nsteps) return;
-            const int t0 = step_key(round * KG + group);
+            if (group >= ks || round * ks + group >= nsteps) return;
+            const int t0 = step_key(round * ks + group);
             const uint32_t base = buf * stage + wave * 1024;
             if (whole && t0 + 31 <= klast) {
                 const int pi = page_of(t0), po = psh >= 0 ? t0 & (g.page - 1) : t0 - pi * g.page;
@@ -1035,8 +1035,8 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
         if (rounds > 1) issue(1, 1);
         int buf = 0;
         for (int round = 0; round < rounds; ++round) {
-            const int st = round * KG + group;
-            if (st + KG < nsteps) {                           // all but the next step's loads of this wave
+            const int st = round * ks + group;
+            if (st + ks < nsteps) {                           // all but the next step's loads of this wave
                 wait_vm(JK + JV);
             } else wait_vm<0>();
             __builtin_amdgcn_s_barrier();
@@ -1044,7 +1044,7 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
             const int t0 = step_key(st), cur = buf * stage;
             if (round + 2 < rounds) issue(round + 2, buf == 0 ? 2 : buf - 1);
             buf = buf == 2 ? 0 : buf + 1;
-            if (!mine || st >= nsteps || t0 > plast || (t0 + 31 < rlo_first && t0 >= keep)) continue;
+            if (!mine || group >= ks || st >= nsteps || t0 > plast || (t0 + 31 < rlo_first && t0 >= keep)) continue;
             // all key fragments are asked for in front of the products, all value fragments in front of the softmax: left alone the compiler waits for each pair
             f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
             {
@@ -2199,35 +2199,44 @@ __global__ __launch_bounds__(1024) void hy_head_norm_kernel(const float* o, int 
 }
 
 
-// The same for heads of up to 4 G channels whose rows lie on 16 bytes: G lanes have four channels each of one head, all loads at once, one trip to memory where the kernel above makes two
-// of 4 bytes a lane.  8192 rows of 16 heads of 128 with gate: 77.3 -> 36.4 us (4.6 TB/s).
+// The same, with the same sums, for heads of up to 4 G channels: lane l of G has channels l + G e of one head, all loads at once: one trip to memory and several heads a block.
+// 8192 rows of 16 heads of 128 with gate: 77.3 -> 44.6 us (36.4 with four adjacent channels a lane, whose sums differ).
 template <typename T, int G>
 __global__ __launch_bounds__(256) void hy_head_norm4_kernel(const float* o, int ldo, int H, int vdim, const T* w, float eps, const float* gate, int ldg, int goff, T* out,
                                                             int w_heads, int gate_sigmoid, const float* den, int heads) {
-    using T4 = __attribute__((ext_vector_type(4))) T;
-    const int i = blockIdx.x * (256 / G) + threadIdx.x / G, c = threadIdx.x % G * 4;
+    const int i = blockIdx.x * (256 / G) + threadIdx.x / G, l = threadIdx.x % G;
     if (i >= heads) return;                             // whole groups of G lanes
     const int r = i / H, h = i - r * H;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f}, gz = v, wv = {1.f, 1.f, 1.f, 1.f};
-    if (c < vdim) {
-        v = *(const f32x4*)(o + (size_t)r * ldo + (size_t)h * vdim + c);
-        if (gate) gz = *(const f32x4*)(gate + (size_t)r * ldg + goff + h * vdim + c);
-        if (w) wv = __builtin_convertvector(*(const T4*)(w + (w_heads ? h * vdim : 0) + c), f32x4);
-    }
-    if (den) v *= 1.f / den[i];
-    float ss = 0.f;
+    float v[4], gz[4], wv[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(v[e], v[e], ss);
+    for (int e = 0; e < 4; ++e) {
+        const int c = l + G * e;
+        const bool ok = c < vdim;
+        v[e] = ok ? o[(size_t)r * ldo + (size_t)h * vdim + c] : 0.f;
+        gz[e] = gate && ok ? gate[(size_t)r * ldg + goff + h * vdim + c] : 0.f;
+        wv[e] = w && ok ? (float)w[w_heads ? h * vdim + c : c] : 1.f;
+    }
+    if (den) {
+        const float sc = 1.f / den[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= sc;
+    }
+    // channels 64 apart one after the other, then a tree over 32, 16, .. apart
+    float ss;
+    if (G == 64)      ss = __builtin_fmaf(v[3], v[3], __builtin_fmaf(v[2], v[2], __builtin_fmaf(v[1], v[1], v[0] * v[0])));
+    else if (G == 32) ss = __builtin_fmaf(v[2], v[2], v[0] * v[0]) + __builtin_fmaf(v[3], v[3], v[1] * v[1]);
+    else              ss = (v[0] * v[0] + v[2] * v[2]) + (v[1] * v[1] + v[3] * v[3]);
 #pragma unroll
     for (int m = G / 2; m; m >>= 1) ss += __shfl_xor(ss, m, G);
-    if (c >= vdim) return;
-    v *= 1.f / sqrtf(ss / (float)vdim + eps);
-    if (w) v *= wv;
-    if (gate) {
+    const float inv = 1.f / sqrtf(ss / (float)vdim + eps);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= gate_sigmoid ? hy_sigmoid(gz[e]) : hy_silu(gz[e]);
+    for (int e = 0; e < 4; ++e) {
+        const int c = l + G * e;
+        float y = v[e] * inv;
+        if (w) y *= wv[e];
+        if (gate) y *= gate_sigmoid ? hy_sigmoid(gz[e]) : hy_silu(gz[e]);
+        if (c < vdim) out[(size_t)i * vdim + c] = (T)y;
     }
-    *(T4*)(out + (size_t)i * vdim + c) = __builtin_convertvector(v, T4);
 }
 
 // ------------------------------------------------------------------------------------------------ recurrences of a few rows: gates, update, output, norm and output gate in one launch
@@ -3211,10 +3220,7 @@ extern "C" int mi355_hy_head_norm_ex3(const float* o, int32_t ldo, int32_t rows,
                                       int32_t goff, void* out, int32_t w_heads, int32_t gate_sigmoid, const float* den, int32_t act_dtype,
                                       mi355_stream_t stream) {
     MI355_CHECK_ARG(o && out && rows > 0 && H > 0 && vdim > 0 && ldo >= H * vdim, "hy_head_norm: bad argument");
-    const size_t tb = act_dtype == MI355_ACT_F32 ? 16 : 8;
-    auto on = [](const void* q, size_t b) { return (uintptr_t)q % b == 0; };
-    if (vdim % 4 == 0 && vdim <= 256 && ldo % 4 == 0 && on(o, 16) && on(out, tb) && (!w || on(w, tb)) && (!gate || (ldg % 4 == 0 && goff % 4 == 0 && on(gate, 16))) &&
-        (int64_t)rows * H <= INT32_MAX - 256) {
+    if (vdim <= 256 && (int64_t)rows * H <= INT32_MAX - 256) {
         const int n = rows * H, G = vdim <= 32 ? 8 : vdim <= 64 ? 16 : vdim <= 128 ? 32 : 64;
 #define HY_HEAD_NORM4(G_) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_head_norm4_kernel<T, G_>), dim3((n + 256 / G_ - 1) / (256 / G_)), dim3(256), 0, (hipStream_t)stream, o, ldo, H, \
                                       vdim, (const T*)w, eps, gate, ldg, goff, (T*)out, w_heads, gate_sigmoid, den, n))

@@ -496,6 +496,7 @@ def gated_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int
     return best if 1.05 * us < scan_us else None
 
 
+FIXED_TILES_FROM = 640     # rows of the longest sequence: shorter walks under a constant decay gain a few us and keep the sums of hy_scan
 CHUNKS_HOST_US = 25        # two more launches and two buffers of a call in chunks: shows where launches bound a step (two prompts of 99 rows, 8 layers: 940 us, 1087 in chunks)
 
 
@@ -567,7 +568,7 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
                                           act_code(act), _stream()), "hy_scan")
 
     fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
-    if chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim):
+    if chunked is None and dim <= WALK_MAX_DIM and (not fixed or max_rows > FIXED_TILES_FROM) and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim):
         def walk(rs, sl, fp, n, st, dst, cdecay, keep):
             _C.check_hybrid(lib.mi355_hy_walk(mode, proj.data_ptr(), ld, qo, ko, vo, _p(z), 0 if z is None else _rows(z, "scan.z"), _p(lower), _p(fbias), float(tau),
                                               float(qscale), heads, dim, vdim, rs.data_ptr(), sl.data_ptr(), fp.data_ptr(), n, st.data_ptr(), _p(dst), _p(cdecay), keep,

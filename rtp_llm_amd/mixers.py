@@ -496,10 +496,6 @@ class Retention:
         rot = s.rot
         hops.rotary(proj, [(self.qo, s.heads, s.dim, 1.0), (self.ko, s.heads, s.dim, 1.0 / math.sqrt(s.dim))], rot.dims if rot else 0,
                     hops.LAYOUTS[rot.layout] if rot else 0, self.freq, self.mag, batch.pos)
-        if h.shape[0] <= hops.FEW_ROWS and hops.recur_step_supported(s.dim, s.vdim):
-            o = hops.recur_step(hops.SCAN_FIXED, proj, self.qo, self.ko, self.vo, self.go, None, None, self.decay, None, 1.0, 1.0, s.heads, s.dim, s.vdim, batch.row_start,
-                                batch.slot, batch.first_pos, state, None, self.eps, self.act)
-            return hops.dense_linear(o, self.w_o, out_dtype=torch.float32)
         o = hops.scan(hops.SCAN_FIXED, proj, self.qo, self.ko, self.vo, None, self.decay, None, 1.0, 1.0, s.heads, s.dim, s.vdim,
                       batch.row_start, batch.slot, batch.first_pos, state, self.act, plans=batch.plans, max_rows=batch.max_rows)
         o = hops.head_norm(o, s.heads, s.vdim, None, self.eps, proj, self.go, out_dtype=self.act)

@@ -1,4 +1,4 @@
-"""Head norms where the heads' rows lie on 16 bytes (four channels a lane) and where they do not, against 64-bit arithmetic.  Error: sums of at most 1024 squares, one reciprocal root and the gate,
+"""Head norms of several heads a block (up to 256 channels) and of one, against 64-bit arithmetic.  Error: sums of at most 1024 squares, one reciprocal root and the gate,
 a few roundings of 2^-24 each, then one rounding to the activation type."""
 import pytest
 import torch

@@ -13,6 +13,7 @@ DEV = "cuda:0"
 def _run(monkeypatch, C, mode, proj, qo, ko, vo, z, lower, fbias, tau, H, dim, vdim, starts, slot, first, state, longest):
     monkeypatch.setattr(hops, "gated_form", lambda *a: C)
     monkeypatch.setattr(hops, "tiles_form", lambda *a: C)
+    monkeypatch.setattr(hops, "FIXED_TILES_FROM", 0)
     return hops.scan(mode, proj, qo, ko, vo, z, lower, fbias, tau, dim ** -0.5, H, dim, vdim, starts, slot, first, state, torch.bfloat16, plans={}, max_rows=longest)
 
 
