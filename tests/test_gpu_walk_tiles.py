@@ -4,7 +4,7 @@ An infinite or undefined value reaches its own token's outputs and later ones, n
 import pytest
 import torch
 
-from rtp_llm_amd import hybrid_ops as hops
+from rtp_llm_amd import _C, hybrid_ops as hops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -88,3 +88,35 @@ def test_undefined_values_stay_behind_their_token(monkeypatch, C, bad):
     rest = [c for c in range(H * vdim) if c != 5]
     tol = 1e-6 * float(good.abs().max()) * dim ** 0.5      # the tile with the bad value sums its products in another order
     assert float((good[:, rest] - odd[:, rest]).abs().max()) < tol
+
+
+@pytest.mark.parametrize("tau", [4.0, 16.0, 64.0])
+@pytest.mark.parametrize("lo,hi", [(-90.0, -30.0), (-30.0, -2.0), (-2.0, 8.0)])
+def test_decay_of_a_token(tau, lo, hi):
+    """sigmoid(z)^(1 / tau), tau a power of two so that the division is exact.  Bound in units of 2^-24: the exponential's last place 2, log(1 + e^-|z|) below 0.7 to two of its places
+    3 / tau, and where it is not lost beside z (above -18) the rounding of their sum |z| / tau."""
+    H, dim, n = 2, 64, 500
+    z = torch.rand(n, H * dim, device=DEV, dtype=torch.float64, generator=torch.Generator(device=DEV).manual_seed(int(tau))).mul(hi - lo).add(lo).float()
+    proj, state, decay = torch.ones(n, 2 * H * dim + H * 8, device=DEV), torch.zeros(n, H, dim, 8, device=DEV), torch.zeros(n, H, dim, device=DEV)
+    at = torch.arange(n + 1, dtype=torch.int32, device=DEV)              # a sequence each: the product of its decays is that of its token
+    first = torch.zeros(n, dtype=torch.int32, device=DEV)
+    _C.check_hybrid(_C.hybrid_lib().mi355_hy_walk(hops.SCAN_GLA, proj.data_ptr(), proj.stride(0), 0, H * dim, 2 * H * dim, z.data_ptr(), H * dim, None, None, tau, 1.0, H, dim, 8,
+                                                  at.data_ptr(), at.data_ptr(), first.data_ptr(), n, state.data_ptr(), None, decay.data_ptr(), 0, hops.act_code(torch.bfloat16),
+                                                  torch.cuda.current_stream().cuda_stream), "hy_walk")
+    ref = torch.exp(torch.nn.functional.logsigmoid(z.double()) / tau)
+    bound = 2.0 ** -24 * (2 + 3 / tau + torch.where(z > -18, z.abs(), 0.0).double() / tau)
+    off = (decay.view(n, H * dim).double() / ref - 1).abs()
+    assert bool((off <= bound)[ref > 1e-30].all())
+
+
+def test_decay_at_the_ends():
+    n, dim = 6, 4
+    z = torch.tensor([float("inf"), float("-inf"), -1e30, 1e30, 0.0, float("nan")], device=DEV)[:, None].expand(n, dim).contiguous()
+    proj, state, decay = torch.ones(n, 12, device=DEV), torch.zeros(n, 1, dim, 4, device=DEV), torch.zeros(n, dim, device=DEV)
+    at, first = torch.arange(n + 1, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+    for tau in (1.0, 16.0):
+        _C.check_hybrid(_C.hybrid_lib().mi355_hy_walk(hops.SCAN_GLA, proj.data_ptr(), 12, 0, 4, 8, z.data_ptr(), dim, None, None, tau, 1.0, 1, dim, 4, at.data_ptr(), at.data_ptr(),
+                                                      first.data_ptr(), n, state.data_ptr(), None, decay.data_ptr(), 0, hops.act_code(torch.bfloat16),
+                                                      torch.cuda.current_stream().cuda_stream), "hy_walk")
+        got = decay[:, 0].tolist()
+        assert got[:4] == [1.0, 0.0, 0.0, 1.0] and abs(got[4] - 0.5 ** (1 / tau)) < 1e-6 and got[5] != got[5]
