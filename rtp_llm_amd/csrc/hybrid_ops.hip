@@ -1540,9 +1540,11 @@ __global__ __launch_bounds__(1024) void hy_scan_kernel(ScanParams p) {
 // chunk leaves from zero and, in cdecay [sequences, H, dim], the product of its decays.
 // 16 heads of 64 x 128, four sequences of 2048 tokens in chunks of 128: states 106.7 -> 49 us, outputs 136.5 -> 86; one sequence of 1537, 8 heads, chunks of 32: all 60.5 -> 42 us.
 // A block alone takes 4 us a tile, of which 2304 cycles are products; the rest is its chain of two barriers, LDS and exponentials, which four blocks of a compute unit hide (128
-// registers; HGRN2's outputs three).  Products of decays are formed in 64 bits (a constant decay's powers would carry one rounding from tile to tile), sums as short chains and trees.
-// Error of the outputs against a 64-bit walk, root mean square over that of the outputs, 2048 tokens of 16 heads, here / token by token: GLA 3.16e-7 / 3.47e-7, HGRN2 1.09e-7 / 1.10e-7,
-// constant decays 1.12e-7 / 1.27e-7; of the states 3.12e-7 / 3.46e-7, 2.46e-7 / 2.43e-7, 0.86e-7 / 1.08e-7.
+// registers; HGRN2's outputs three).  Products of decays are formed in 64 bits (a constant decay's powers would carry one rounding from tile to tile), sums as short chains and trees,
+// P's tree over the lanes in 64 bits under gates.
+// Error against a 64-bit walk, root mean square over that of the result, 2048 tokens of 16 heads, here / token by token: outputs GLA 3.17e-7 / 3.47e-7 (tau 16, z 3 +- 2), 1.14e-7 / 1.20e-7
+// (z 0 +- 2), 7.55e-8 / 8.46e-8 (z -10 +- 6), 8.77e-8 / 9.28e-8 (tau 1, z 2 +- 2), HGRN2 1.124e-7 / 1.128e-7, constant decays 1.09e-7 / 1.27e-7; states 3.14e-7 / 3.44e-7, 9.52e-8 / 1.00e-7,
+// 4.02e-8 / 4.51e-8, 5.79e-8 / 5.98e-8, 2.50e-7 / 2.52e-7, 0.80e-7 / 1.07e-7.
 // sigmoid(z)^(1 / tau).  From tau = 16 on log(1 + e^-|z|) by the vector unit's exponential and logarithm, with what 1 + e^-|z| rounds off put back: they leave about 2^-24 on it, which tau
 // divides; the quotient is corrected to a division's and the outer exponential is expf, so that the error is that of the plain form (root mean square, tau 16, z in (-2, 2) 1.87e-8 both,
 // (-10, 0) 2.72e-8 both, (-90, -30) 2.64e-8 both) in a quarter of its operations.  Smaller tau: the plain form (tau 4, z in (0, 8) 1.847e-8 against 1.854e-8).
@@ -1560,7 +1562,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
     constexpr bool LOW = OUT && MODE == SCAN_HGRN2;     // P in two parts: its k = 1 - a and silu(q) lean to one side, so that P's own rounding and the
                                                         // sums' show in the outputs: 1.19e-7 without, 1.15e-7 with, 1.09e-7 with 64-bit sums as well; 86 -> 107 us
     __shared__ __attribute__((aligned(16))) float q_s[OUT ? (TOK + 3) * DP : 4], k_s[OUT ? TOK * DP : 4], a_s[OUT ? (TOK + 3) * DP : 4];      // as they are, [token][channel]; three rows of q and a are read past the tile, unused
-    __shared__ __attribute__((aligned(16))) float qc_s[OUT ? TOK * QS : 4], ke_s[DP * KS], P_s[OUT ? TOK * KS : 4], Pl_s[LOW ? TOK * KS : 4];               // q c [token][channel], k e [channel][token], P [t][s]
+    __shared__ __attribute__((aligned(16))) float qc_s[OUT ? TOK * QS : 4], ke_s[DP * KS], P_s[OUT ? TOK * KS : 4], Pl_s[LOW ? TOK * KS : 4];               // q c [token][channel], k e [channel][token] and P [t][s], tokens s at 4 (s % 4) + s / 4: the products add them in order
     __shared__ double part_s[4][DP];                                                                                              // products of the decays of four tokens ...
     __shared__ __attribute__((aligned(16))) float all_s[DP];                                                                      // ... and of all
     const int sq = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * 128;
@@ -1595,7 +1597,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
         if (MODE == SCAN_HGRN2 && d < p.dim) { lw[j] = (float)((const T*)p.lower)[h * p.dim + d]; fb[j] = (float)((const T*)p.fbias)[h * p.dim + d]; }
     }
     if constexpr (MODE == SCAN_FIXED || MODE == SCAN_FIXED_SILU) fixed = ((const float*)p.lower)[h];
-    // the next tile's projections: q, k, z of tokens 4 wave + i and channel lane + 64 j (tokens past the last read the last), v of tokens 4 g + r and column vcol + 16 cb.
+    // the next tile's projections: q, k, z of tokens 4 wave + i and channel lane + 64 j (tokens past the last read the last), v of tokens 4 r + g and column vcol + 16 cb.
     // Lanes without a channel, column or token lie out of their descriptor's range: zeros without a branch
     float rq[CH][4], rk[CH][4], rz[CH][4];
     f32x4 rv[2];
@@ -1606,7 +1608,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
         const bool ok = vcol + 16 * cb < p.vdim;
-        v_o[cb] = ok ? (uint32_t)(h * p.vdim + vcol + 16 * cb) * 4u + 4 * g * ldb : NONE;
+        v_o[cb] = ok ? (uint32_t)(h * p.vdim + vcol + 16 * cb) * 4u + g * ldb : NONE;
         o_o[cb] = ok ? (uint32_t)(h * p.vdim + vcol + 16 * cb) * 4u + 4 * g * ob : NONE;
     }
     const float itau = MODE == SCAN_GLA ? 1.f / p.tau : 1.f;
@@ -1629,7 +1631,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int cb = 0; cb < 2; ++cb) rv[cb][r] = ldf(rp, 4 * g + r < nt ? v_o[cb] : NONE, r * ldb + p.vo * 4u);
+            for (int cb = 0; cb < 2; ++cb) rv[cb][r] = ldf(rp, 4 * r + g < nt ? v_o[cb] : NONE, 4 * r * ldb + p.vo * 4u);
     };
     if (r0 < r1) fetch(r0);
     for (int t0 = r0; t0 < r1; t0 += TOK) {
@@ -1681,14 +1683,12 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
                 if (w < wave) before *= m;
                 if (w > wave) behind *= m;
             }
-            f32x4 ke;
 #pragma unroll
-            for (int i = 3; i >= 0; --i) { ke[i] = kv[j][i] * (float)behind; behind *= (double)av[j][i]; }
-            *(f32x4*)(ke_s + d * KS + 4 * wave) = ke;
+            for (int i = 3; i >= 0; --i) { ke_s[d * KS + 4 * i + wave] = (float)((double)kv[j][i] * behind); behind *= (double)av[j][i]; }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 before *= (double)av[j][i];
-                if (OUT) qc_s[(4 * wave + i) * QS + d] = qv[j][i] * (float)before;
+                if (OUT) qc_s[(4 * wave + i) * QS + d] = (float)((double)qv[j][i] * before);
             }
             if (wave == 3) all_s[d] = (float)before;
             if (!OUT) A[j] *= before;                   // the last wave's is the product of all
@@ -1717,7 +1717,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
                     }
             }
             const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
-            using Sum = std::conditional_t<LOW, double, float>;
+            using Sum = std::conditional_t<LOW || MODE == SCAN_GLA, double, float>;
             float p8[8];
             Sum p4[4], p2[2];
 #pragma unroll
@@ -1728,8 +1728,8 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
             for (int u = 0; u < 2; ++u) p2[u] = (b1 ? p4[u + 2] : p4[u]) + hy_dpp<0x1B>(b1 ? p4[u] : p4[u + 2]);                    // lane 3 - i of the 4
             const Sum p1 = (b0 ? p2[1] : p2[0]) + hy_dpp<0xB1>(b0 ? p2[0] : p2[1]);
             if (s + c < 16) {
-                P_s[(s + c) * KS + s] = (float)p1;
-                if constexpr (LOW) Pl_s[(s + c) * KS + s] = (float)(p1 - (double)(float)p1);
+                P_s[(s + c) * KS + 4 * g + wave] = (float)p1;
+                if constexpr (LOW) Pl_s[(s + c) * KS + 4 * g + wave] = (float)(p1 - (double)(float)p1);
             }
         }
         __syncthreads();
@@ -1783,7 +1783,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
                     for (int cb = 0; cb < 2; ++cb) {
                         f32x4 u;
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) u[r] = 4 * g + r <= t ? v[cb][r] : 0.f;
+                        for (int r = 0; r < 4; ++r) u[r] = 4 * r + g <= t ? v[cb][r] : 0.f;
                         x[cb] = o[cb] + within(u, p4, pl);
                     }
 #pragma unroll
@@ -1800,12 +1800,17 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
                     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), ro, 4 * g + r < nt ? o_o[cb] : NONE, r * ob, 0);
                 }
         }
-        // the tile's own sum by itself, then one rounding at the state's magnitude instead of sixteen
+        // The tile's own sum by itself, then one rounding at the state's magnitude instead of sixteen; where the decays leave less than a quarter the last of the sixteen stand alone, and
+        // the decayed state goes in front of them (a row's sum by itself saves 17 all^2 of a rounding's square and costs one)
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             if (db % 2 == 0) __builtin_amdgcn_sched_barrier(0);
             const f32x4 k4 = *(const f32x4*)(ke_s + (16 * db + c) * KS + 4 * g), all = *(const f32x4*)(all_s + 16 * db + 4 * g);
-            f32x4 own[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            f32x4 own[2];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) own[cb][r] = all[r] < 0.25f ? all[r] * S[db][cb][r] : 0.f;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -1813,7 +1818,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int cb = 0; cb < 2; ++cb) S[db][cb][r] = __builtin_fmaf(all[r], S[db][cb][r], own[cb][r]);
+                for (int cb = 0; cb < 2; ++cb) S[db][cb][r] = all[r] < 0.25f ? own[cb][r] : __builtin_fmaf(all[r], S[db][cb][r], own[cb][r]);
         }
     }
     if (keep_state) {
