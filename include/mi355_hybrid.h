@@ -101,7 +101,9 @@ typedef struct {
 int mi355_dense_linear_pair(const mi355_dense_args_t* two, mi355_stream_t stream);
 /* mi355_hy_scan over a few rows and mi355_hy_head_norm_ex2 (weight, gate through silu) in one launch, a block per sequence and head.  mode, projections, state and gates as
  * there; with ao >= 0 the decay pre-activations of mode 1 are formed here: column hd is b2[hd] + sum over j < rank of w2[hd, j] (act type) times proj[:, ao + j] rounded to the
- * act type.  w null: unit RMS only; go < 0: no gate.  out [rows, H * vdim] of the act type.  MI355_ERR_UNSUPPORTED: vdim % 4, vdim > 256, dim > 256 or dim * vdim > 32768. */
+ * act type.  w null: unit RMS only; go < 0: no gate.  out [rows, H * vdim] of the act type.  MI355_ERR_UNSUPPORTED: a state off 16 bytes, and heads
+ * that mi355_hy_recur_step_fits refuses (host only): vdim % 4, vdim > 256, dim > 256, dim * vdim > 32768 or more than 36 key rows for each of the 256 / (vdim / 4) threads of a column. */
+int mi355_hy_recur_step_fits(int32_t dim, int32_t vdim);
 int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, int32_t go, int32_t ao, int32_t rank, const void* w2, const void* b2,
                         const float* z, int32_t ldz, const void* lower, const void* fbias, float tau, float qscale, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start,
                         const int32_t* slot, const int32_t* first_pos, int32_t nseq, float* state, const void* w, int32_t w_heads, float eps, void* out, int32_t act_dtype,

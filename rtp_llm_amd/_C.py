@@ -208,6 +208,7 @@ HYBRID_SIGNATURES = {
     "mi355_hy_attn_prep_ex": (i32, [vp, i32, i32, i32, ip, vp, vp, i32, f32, vp, vp, vp, i32, vp, vp, vp, vp, f32, f32, i32, i32, vp]),
     "mi355_hy_attn_rows_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, f32, vp, i32, i32, vp]),
     "mi355_dense_linear_pair": (i32, [C.POINTER(DenseArgs), vp]),
+    "mi355_hy_recur_step_fits": (i32, [i32, i32]),
     "mi355_hy_recur_step": (i32, [i32, vp] + [i32] * 7 + [vp, vp, vp, i32, vp, vp, f32, f32, i32, i32, i32, vp, vp, vp, i32, vp, vp, i32, f32, vp, i32, vp]),
     "mi355_hy_attn_tiles_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, f32, vp, i32, i32, vp]),
     "mi355_hy_head_norm_ex": (i32, [vp, i32, i32, i32, vp, f32, vp, i32, i32, vp, i32, i32, i32, vp]),

@@ -3014,6 +3014,13 @@ extern "C" int mi355_hy_scan(int32_t mode, const float* proj, int32_t ld, int32_
     return MI355_OK;
 }
 
+// Heads that hy_recur_step_kernel takes: four value columns a thread, the key rows that each of its threads then holds at most 36 (registers).
+extern "C" int mi355_hy_recur_step_fits(int32_t dim, int32_t vdim) {
+    if (dim <= 0 || vdim <= 0 || vdim % 4 || vdim > 256 || dim > 256 || dim * vdim > 32768) return 0;
+    const int KG = 256 / (vdim / 4);
+    return (dim + KG - 1) / KG <= 36;
+}
+
 // mi355_hy_scan over few rows with the head norm and output gate behind it: see the header.
 extern "C" int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, int32_t qo, int32_t ko, int32_t vo, int32_t go, int32_t ao, int32_t rank, const void* w2,
                                    const void* b2, const float* z, int32_t ldz, const void* lower, const void* fbias, float tau, float qscale, int32_t H, int32_t dim,
@@ -3023,7 +3030,7 @@ extern "C" int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, 
     MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : (mode == SCAN_FIXED || mode == SCAN_FIXED_SILU) ? lower != nullptr
                                                           : (mode == SCAN_GLA && tau > 0.f && (ao >= 0 ? (w2 && rank > 0 && rank <= 64) : z != nullptr)),
                     "hy_recur_step: mode %d lacks its gate inputs", mode);
-    if (vdim % 4 || vdim > 256 || dim > 256 || dim * vdim > 32768 || (uintptr_t)state % 16) {
+    if (!mi355_hy_recur_step_fits(dim, vdim) || (uintptr_t)state % 16) {
         mi355_set_error("hy_recur_step: heads of %d x %d", dim, vdim);
         return MI355_ERR_UNSUPPORTED;
     }
@@ -3034,8 +3041,7 @@ extern "C" int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, 
     if (rows <= 4)       HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 4>), grid, dim3(256), 0, st, p));
     else if (rows <= 8)  HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 8>), grid, dim3(256), 0, st, p));
     else if (rows <= 16) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 16>), grid, dim3(256), 0, st, p));
-    else if (rows <= 36) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 36>), grid, dim3(256), 0, st, p));
-    else { mi355_set_error("hy_recur_step: %d key rows a thread", rows); return MI355_ERR_UNSUPPORTED; }
+    else                 HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 36>), grid, dim3(256), 0, st, p));
     MI355_CHECK_LAUNCH("hy_recur_step_kernel");
     return MI355_OK;
 }

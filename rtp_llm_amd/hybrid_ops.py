@@ -612,9 +612,10 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
 STEP_MAX_RANK = 64         # of the low-rank decay that recur_step forms
 
 
+@functools.lru_cache(maxsize=64)
 def recur_step_supported(dim: int, vdim: int) -> bool:
     """Heads that recur_step takes."""
-    return vdim % 4 == 0 and vdim <= 256 and dim <= 256 and dim * vdim <= 32768
+    return bool(_C.hybrid_lib().mi355_hy_recur_step_fits(dim, vdim))
 
 
 def recur_step(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, go: Optional[int], low_rank, z: Optional[torch.Tensor], lower, fbias, tau: float, qscale: float, heads: int,

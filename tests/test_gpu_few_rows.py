@@ -1,8 +1,10 @@
 """Launches of steps of few rows: two linears in one (the bits of two calls), and a recurrence with its norm and output gate in one against the same in 64 bits."""
+import types
+
 import pytest
 import torch
 
-from rtp_llm_amd import hybrid_ops as hops
+from rtp_llm_amd import hybrid_ops as hops, mixers
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -24,7 +26,7 @@ def test_pair_is_two_calls(M, K0, N0, K1, N1, gated):
 
 
 @pytest.mark.parametrize("mode", ["hgrn2", "gla", "gla-z", "fixed", "fixed-silu"])
-@pytest.mark.parametrize("H,dim,vdim,rank", [(16, 64, 128, 16), (3, 32, 64, 4), (2, 128, 256, 16), (2, 256, 128, 24), (5, 40, 96, 3), (1, 7, 4, 1), (4, 100, 100, 8)])
+@pytest.mark.parametrize("H,dim,vdim,rank", [(16, 64, 128, 16), (3, 32, 64, 4), (2, 128, 256, 16), (2, 256, 128, 24), (5, 40, 96, 3), (1, 7, 4, 1), (4, 100, 100, 8), (1, 144, 208, 8)])
 @pytest.mark.parametrize("counts", [[1], [1, 1, 1, 1, 1, 1, 1, 1], [3, 1, 12]])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_recurrence_of_few_rows(mode, H, dim, vdim, rank, counts, dtype):
@@ -74,3 +76,43 @@ def test_recurrence_of_few_rows(mode, H, dim, vdim, rank, counts, dtype):
                           dim ** -0.5, H, dim, vdim, start, slot, first, state, w, 1e-5, dtype)
     assert float((state.double() - S).abs().max()) <= 2.0 ** -18 * float(S.abs().max())
     assert bool(((out.double().view(T, H, vdim) - ref).abs() <= off + (2.0 ** -20 if dtype == torch.float32 else 2.0 ** -8) * ref.abs()).all())
+
+
+# heads on both sides of the recurrence step's limits: 36 and 37 key rows a thread, value columns that are no multiple of 4
+@pytest.mark.parametrize("kind", ["gla", "hgrn2"])
+@pytest.mark.parametrize("dim,vdim,fits", [(180, 176, True), (184, 176, False), (144, 208, True), (152, 208, False), (64, 130, False), (128, 256, True)])
+def test_a_decode_step_serves_every_head(kind, dim, vdim, fits):
+    """What the recurrence step refuses walks as before it was there.  Against 64 bits from the same bf16 weights, the low-rank decay's middle rounded to bf16 as there: the outputs are
+    rounded to bf16 twice (2^-8 each of the largest), the states differ by what the middle's rounding may flip (2^-8 of a pre-activation of about 1 over tau, of a state of about 1)."""
+    assert hops.recur_step_supported(dim, vdim) is fits
+    H, W, T, tau = 2, 64, 3, 16.0
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    weight = lambda n, k=W: (r(n, k) * k ** -0.5).bfloat16()
+    hd, hv = H * dim, H * vdim
+    w = {"q": weight(hd), "v": weight(hv), "o": torch.eye(hv, device=DEV).bfloat16(), "norm": (1 + 0.1 * r(hv if kind == "gla" else vdim)).bfloat16()}
+    if kind == "gla":
+        w.update({"k": weight(hd), "g": weight(hv), "a1": weight(16), "a2": weight(hd, 16), "a2.b": r(hd).bfloat16()})
+    else:
+        w.update({"f": weight(hd), "lower": torch.sigmoid(r(hd)).bfloat16(), "f.b": r(hd).bfloat16()})
+    mixer = mixers.GatedLinearRecurrence(mixers.RecurrenceSpec(kind=kind, heads=H, dim=dim, vdim=vdim, tau=tau), w, 1e-5)
+    index = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    batch = types.SimpleNamespace(row_start=index(0, 1, 2, 3), slot=index(2, 0, 1), first_pos=index(4, 0, 9), plans={}, max_rows=1)
+    state, h = r(3, H, dim, vdim), r(T, W).bfloat16()
+    lin = lambda n, c: (h.double() @ w[n].double().t()).view(T, H, c)
+    q, v = lin("q", dim), lin("v", vdim)
+    if kind == "gla":
+        k, z = lin("k", dim), (h.double() @ w["a1"].double().t()).bfloat16().double() @ w["a2"].double().t() + w["a2.b"].double()
+        q, a = q * dim ** -0.5, torch.exp(torch.nn.functional.logsigmoid(z) / tau).view(T, H, dim)
+    else:
+        low = w["lower"].double().view(H, dim)
+        a = low + (1 - low) * torch.sigmoid(lin("f", dim) + w["f.b"].double().view(H, dim))
+        q, k = torch.nn.functional.silu(q), 1 - a
+    S = state.double()[batch.slot.long()] * (batch.first_pos > 0).double()[:, None, None, None] * a[..., None] + k[..., None] * v[:, :, None]
+    o = (S * q[..., None]).sum(2)
+    o = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5) * w["norm"].double().view(-1, vdim)
+    if kind == "gla":
+        o = o * torch.nn.functional.silu(lin("g", vdim))
+    got = mixer.forward(h, batch, state).double().view(T, H, vdim)
+    assert float((got - o).abs().max()) <= 2.0 ** -7 * float(o.abs().max())
+    assert float((state.double()[batch.slot.long()] - S).abs().max()) <= 2.0 ** -8 / tau * float(S.abs().max())
