@@ -886,9 +886,10 @@ extern "C" void mi355_debug_attn_stamps(void* p) { g_attn_stamps = (unsigned lon
 
 extern "C" size_t mi355_paged_attn_workspace_bytes(int32_t B, int32_t nh, int32_t hd, int32_t max_seq_len) {
     if (B <= 0 || nh <= 0 || hd <= 0 || max_seq_len <= 0) return 0;
-    // upper bound over every plan of up to B rows: plan_partitions splits no further than to 256 blocks, a block has at most 32 rows (never less for more rows: a step may have fewer)
-    const int P = std::min(cdiv(max_seq_len, 128), cdiv(256 * 32, B));
-    return (size_t)B * nh * P * (hd + 2) * sizeof(float);
+    // Upper bound over every plan of B rows, and of fewer (it grows with B): partitions have 128 tokens or more; a plan that splits at all (one that does not needs no workspace) has at
+    // most 256 blocks over the (tile of rows, key/value head) pairs, a tile at most 32 rows.
+    const size_t parts = std::min((size_t)B * cdiv(max_seq_len, 128), (size_t)256 * 32);
+    return parts * nh * (hd + 2) * sizeof(float);
 }
 
 namespace {

@@ -430,3 +430,13 @@ def test_bench_gpus_n_without_a_launcher_spawns_its_own_ranks(tmp_path):
     assert "rank 1 of 3" in ok.stderr and "rank 2 of 3" in ok.stderr
     bad = subprocess.run([sys.executable, "-c", drv], env={**env, "FAIL_RANK": "2"}, capture_output=True, text=True, timeout=120)
     assert bad.returncode == 3, (bad.returncode, bad.stderr[-500:])
+
+
+@pytest.mark.parametrize("max_seq", [100, 1088, 4096, 32768])
+def test_attention_workspace_of_fewer_rows_is_no_larger(max_seq):
+    """A caller sizes it once for the most rows a step may have.  Every plan of r rows fits: up to ceil(max_seq / 128) partitions a row, and 256 blocks of 32 rows."""
+    l = _C.lib()
+    one = 28 * 130 * 4
+    sizes = [l.mi355_paged_attn_workspace_bytes(B, 28, 128, max_seq) for B in range(1, 8300)]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+    assert all(s == min(B * -(-max_seq // 128), 8192) * one for B, s in enumerate(sizes, 1))
