@@ -643,8 +643,9 @@ int    mi355_decoder_prefill_ragged(mi355_decoder_t* d, const int32_t* token_ids
                                     const int32_t* row_start, const int32_t* block_table, int32_t nseq, int32_t q_len, int32_t rows,
                                     const int32_t* logit_rows, float* logits_out, void* workspace, size_t workspace_bytes, mi355_stream_t stream);
 /* Several passes in order, with the arguments of mi355_decoder_prefill_ragged each: pass i may attend to what the passes before it cached.  Passes for which
- * mi355_decoder_prefill_overlaps(rows) holds may run two at a time, the second on a stream of the decoder's that the caller's stream waits for at the end: a pass and the
- * next one need workspaces of their own (passes further apart may share one), or they run one after the other.  The same results either way. */
+ * mi355_decoder_prefill_overlaps(rows) holds may run two at a time, the second on a stream of the decoder's that the caller's stream waits for at the end: every
+ * even pass's workspace and logits must lie apart from every odd pass's (mi355_prefill_passes_apart, host only; passes of one parity may share), or they run one after the
+ * other.  The same results either way. */
 typedef struct {
     const int32_t *token_ids, *positions, *row_seq, *row_start, *block_table;
     int32_t        nseq, q_len, rows;
@@ -653,6 +654,7 @@ typedef struct {
     void*          workspace;
     size_t         workspace_bytes;
 } mi355_prefill_pass_t;
+int    mi355_prefill_passes_apart(const mi355_prefill_pass_t* passes, int32_t n, int32_t vocab);
 int    mi355_decoder_prefill_overlaps(mi355_decoder_t* d, int32_t rows);
 int    mi355_decoder_prefill_passes(mi355_decoder_t* d, const mi355_prefill_pass_t* passes, int32_t n, mi355_stream_t stream);
 /* Dynamic-NTK RoPE styles only: {cos, sin} rows [max_pos][rope_dim / 2][2] (fp32, device) the prefill chunks that follow rotate with, or NULL for the model's

@@ -169,6 +169,7 @@ SIGNATURES = {
     "mi355_decoder_prefill_workspace_bytes": (sz, [vp, i32, i32]),
     "mi355_decoder_prefill": (i32, [vp, vp, vp, vp, i32, i32, vp, vp, vp, sz, vp]),
     "mi355_decoder_prefill_ragged": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, sz, vp]),
+    "mi355_prefill_passes_apart": (i32, [C.POINTER(PrefillPass), i32, i32]),
     "mi355_decoder_prefill_overlaps": (i32, [vp, i32]),
     "mi355_decoder_prefill_passes": (i32, [vp, C.POINTER(PrefillPass), i32, vp]),
     "mi355_decoder_set_prefill_rope_table": (i32, [vp, vp]),

@@ -937,21 +937,30 @@ extern "C" int mi355_decoder_prefill_ragged(mi355_decoder_t* d, const int32_t* t
 // not measured, and want a second workspace of their size.  Under tensor parallelism two passes would meet in the collectives' buffers.
 extern "C" int mi355_decoder_prefill_overlaps(mi355_decoder_t* d, int32_t rows) { return d && d->cfg.tp_size == 1 && rows <= 4096; }
 
+// Even passes run on the caller's stream and odd ones beside it; only passes of one stream wait for each other's ends.
+extern "C" int mi355_prefill_passes_apart(const mi355_prefill_pass_t* passes, int32_t n, int32_t vocab) {
+    auto meet = [](const void* a, size_t na, const void* b, size_t nb) { return a && b && (const char*)a < (const char*)b + nb && (const char*)b < (const char*)a + na; };
+    for (int i = 0; i < n; ++i)
+        for (int j = i + 1; j < n; j += 2) {
+            const mi355_prefill_pass_t &a = passes[i], &b = passes[j];
+            if (meet(a.workspace, a.workspace_bytes, b.workspace, b.workspace_bytes)) return 0;
+            if (meet(a.logits_out, (size_t)a.nseq * vocab * 4, b.logits_out, (size_t)b.nseq * vocab * 4)) return 0;
+        }
+    return 1;
+}
+
 extern "C" int mi355_decoder_prefill_passes(mi355_decoder_t* d, const mi355_prefill_pass_t* passes, int32_t n, mi355_stream_t stream) {
     if (!d || !passes || n <= 0) { mi355_set_error("decoder_prefill: bad arguments"); return MI355_ERR_ARG; }
     std::vector<PrefillBufs> bufs(n);
-    bool overlap = n > 1 && !d->prof_on, apart = true;
+    bool overlap = n > 1 && !d->prof_on;
     for (int i = 0; i < n; ++i) {
         if (int e = prefill_check(d, passes[i], &bufs[i])) return e;
         overlap = overlap && mi355_decoder_prefill_overlaps(d, passes[i].rows);
-        if (i > 0) {
-            const char *a = (const char*)passes[i - 1].workspace, *b = (const char*)passes[i].workspace;
-            apart = apart && (a + passes[i - 1].workspace_bytes <= b || b + passes[i].workspace_bytes <= a);
-        }
     }
     hipStream_t st = (hipStream_t)stream;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (overlap && apart && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return prefill_overlapped(d, passes, bufs.data(), n, st);
+    if (overlap && mi355_prefill_passes_apart(passes, n, d->cfg.vocab) && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone)
+        return prefill_overlapped(d, passes, bufs.data(), n, st);
     for (int i = 0; i < n; ++i)
         if (int e = prefill_one(d, passes[i], bufs[i], st); e < 0) return e;
     return MI355_OK;
