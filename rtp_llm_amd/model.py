@@ -610,24 +610,32 @@ class DecoderEngine:
         sizes = [(b + 255) // 256 * 256 for b in sizes]
         if getattr(self, "_prefill_ws", None) is None or self._prefill_ws.numel() < sum(sizes):
             self._prefill_ws = torch.empty(sum(sizes), dtype=torch.uint8, device=dev)
-        passes, held, at = (_C.PrefillPass * len(plan))(), [], 0
+        logits, run, at = None, [], 0
+
+        def issue():                                                # the passes of `run`; the logits rows of what ended in them
+            nonlocal logits
+            _C.check(self.lib.mi355_decoder_prefill_passes(self.handle, (_C.PrefillPass * len(run))(*(r[0] for r in run)), len(run), st), "decoder_prefill")
+            for _, live, ending, _, out in run:
+                if len(ending) == nseq:
+                    logits = out
+                elif ending:
+                    if logits is None:
+                        logits = torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
+                    logits[torch.tensor([live[i] for i in ending], device=dev)] = out[torch.tensor(ending, device=dev)]
+            run.clear()
+
         for i, (live, n, q_len, T, ending, lens) in enumerate(plan):
+            if ending and sum(r[4].shape[0] for r in run if r[2]) + n > 4 * nseq:             # their logits are held meanwhile: at most four times the result
+                issue()
             td, pd, ld, lived, *ragged = on_device[at:at + len(lens)]
             at += len(lens)
             table = btd if n == nseq else btd.index_select(0, lived)
             out = torch.empty(n, self.cfg.vocab, dtype=torch.float32, device=dev) if ending else None
-            held.append((table, out))
             seqd, firstd = (r.data_ptr() for r in ragged) if ragged else (None, None)
             side = i % len(sizes)
-            passes[i] = _C.PrefillPass(td.data_ptr(), pd.data_ptr(), seqd, firstd, table.data_ptr(), n, q_len, T, ld.data_ptr() if ending else None,
-                                       out.data_ptr() if ending else None, self._prefill_ws.data_ptr() + side * sizes[0], sizes[side])
-        _C.check(self.lib.mi355_decoder_prefill_passes(self.handle, passes, len(plan), st), "decoder_prefill")
-        if len(plan[-1][4]) == nseq:
-            return held[-1][1]
-        logits = torch.zeros(nseq, self.cfg.vocab, dtype=torch.float32, device=dev)
-        for (live, _, _, _, ending, _), (_, out) in zip(plan, held):
-            if ending:
-                logits[torch.tensor([live[i] for i in ending], device=dev)] = out[torch.tensor(ending, device=dev)]
+            run.append((_C.PrefillPass(td.data_ptr(), pd.data_ptr(), seqd, firstd, table.data_ptr(), n, q_len, T, ld.data_ptr() if ending else None,
+                                       out.data_ptr() if ending else None, self._prefill_ws.data_ptr() + side * sizes[0], sizes[side]), live, ending, table, out))
+        issue()
         return logits
 
     def generate(self, prompts: List[List[int]], block_table, max_new_tokens: int, prefill_chunk: int = 512) -> List[List[int]]:

@@ -39,3 +39,25 @@ def test_passes_in_flight_change_nothing(lens, start, chunk, kv_int8, dtype):
     eng.lib = lib
     for other in runs[1:]:
         assert all(torch.equal(a, b) for a, b in zip(runs[0], other))
+
+
+def test_logits_held_are_bounded():
+    """Prompts that end one after the other: the passes' logits [live sequences, vocab] are not held all together (528 rows here), and every prompt's row is
+    that of its own last pass."""
+    cfg = model.ModelConfig("tiny-endings", 2, 512, 8, 2, 64, 1024, 4096, max_pos=1024)
+    n = 32
+    eng = model.DecoderEngine(cfg, model.weights_to(model.synth_model(cfg, "w4", "cpu", seed=3, zeros="centered"), DEV), kv_int8=False, page=16, num_blocks=n * (n + 1),
+                              max_batch=n, max_seq_len=16 * (n + 1), device=DEV)
+    g = torch.Generator().manual_seed(5)
+    prompts = [torch.randint(0, cfg.vocab, (16 * (b + 1),), generator=g).tolist() for b in range(n)]
+    bt = torch.arange(n * (n + 1)).reshape(n, n + 1).int()
+    eng.prefill(prompts, bt, chunk=16)                          # the workspace
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    logits = eng.prefill(prompts, bt, chunk=16)
+    torch.cuda.synchronize()
+    one = n * cfg.vocab * 4
+    assert torch.cuda.max_memory_allocated() - before <= 6 * one                          # the result, four times as much, tables and integers
+    eng.lib = _OneAtATime(eng.lib)
+    assert torch.equal(logits, eng.prefill(prompts, bt, chunk=16))
