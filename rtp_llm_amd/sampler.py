@@ -113,6 +113,7 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
     if draw:
         top_p = _host(params.top_p, torch.float32).clone()
         top_p[top_p.abs() < 1e-7] = 1.0
+        filtered = _off(top_p, 1.0) or (_off(top_k, 0) and bool(((top_k.numpy() > 0) & (top_k.numpy() < V)).any()))
         up.update(top_k=top_k, top_p=top_p)
         if params.uniform.device.type == "cpu":
             up["uniform"] = params.uniform.to(torch.float32)
@@ -123,7 +124,9 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
         if penalise:
             vectors = dict(repetition_penalty=up["rep"], presence_penalty=up["pres"], frequency_penalty=up["freq"], input_lengths=up["lengths"], max_input_length=step + 1,
                            step=step + 1, token_ids=up["history"] if "history" in up else params.token_ids.to(device=dev, dtype=torch.int32).contiguous())
-        if not all_greedy and params.output_all_probs is None:                            # and the draw behind them
+        # and the draw behind them, where a row has a filter: with none the histograms that name its threshold are for nothing (64 rows of 152064 56 us in two calls, 65 in one; with
+        # top-p 0.8 to 0.95 125 and 52)
+        if not all_greedy and filtered and params.output_all_probs is None:
             u = up["uniform"] if "uniform" in up else params.uniform.to(device=dev, dtype=torch.float32).contiguous()
             ids = ops.sampling_draw(logits, up["top_k"], up["top_p"], u, up.get("temperature"), **vectors)
             params.token_ids[:, step] = ids.to(params.token_ids.device)

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from rtp_llm_amd import ops
+from rtp_llm_amd import ops, sampler
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -57,3 +57,21 @@ def test_joint_draw_takes_kept_tokens_only():
     p = torch.tensor([1.0, 1.0, 0.85, 0.85], device=DEV)          # 0.644, 0.237, 0.087, 0.032: the third starts above 0.85
     u = torch.tensor([0.0, 0.9999999, 0.0, 0.9999999], device=DEV)
     assert ops.sampling_draw(x, k, p, u).tolist() == [77, 4000, 77, 1234]
+
+
+@pytest.mark.parametrize("top_k,top_p,joint", [(0, 1.0, False), (300, 1.0, False), (0, 0.0, False), (50, 1.0, True), (0, 0.9, True), (299, 1.0, True)])
+def test_rows_without_a_filter_take_the_separate_launches(monkeypatch, top_k, top_p, joint):
+    """sample_greedy: top-k of 0 or the whole row and top-p of 1 (0 means that too) keep everything; one row with a filter is enough for the joint draw."""
+    B, V = 3, 300
+    x = torch.randn(B, V, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)) * 2
+    calls = []
+    one, two = ops.sampling_draw, ops.top_k_top_p_sample
+    monkeypatch.setattr(ops, "sampling_draw", lambda *a, **k: calls.append("joint") or one(*a, **k))
+    monkeypatch.setattr(ops, "top_k_top_p_sample", lambda *a, **k: calls.append("separate") or two(*a, **k))
+    k, p, u = torch.tensor([0, top_k, 0], dtype=torch.int32), torch.tensor([1.0, top_p, 1.0]), torch.tensor([0.2, 0.5, 0.9])
+    logits = x.clone()
+    ids = sampler.sample_greedy(sampler.GreedyParams(logits=logits, input_lengths=torch.ones(B, dtype=torch.int32), sequence_lengths=torch.ones(B, dtype=torch.int32),
+                                                     token_ids=torch.zeros(B, 2, dtype=torch.int32), step=1, top_k=k, top_p=p, temperature=torch.ones(B), uniform=u))
+    assert calls == ["joint" if joint else "separate"]
+    probs = ops.sampling_probs(x.clone())
+    assert torch.equal(logits, probs) and torch.equal(ids, two(probs, k.to(DEV), p.to(DEV), u.to(DEV)))
