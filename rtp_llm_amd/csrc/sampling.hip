@@ -956,6 +956,7 @@ __global__ __launch_bounds__(kThreads) void top_k_top_p_sample_kernel(const TopK
 // in it take sample_row.
 // 64 rows of 152064, top-k 0..100, top-p 0.8..0.95: 103 us of top_k_top_p_sample_kernel (one compute unit pulls a row three times) -> 12.8 and 16.8.
 constexpr int kList = 8 * kThreads;
+__device__ __host__ __forceinline__ int draw_list(int V) { return V < kList ? V : kList; }        // a row's list
 
 struct DrawFilter { int k; bool use_k, use_p; float tp; };
 __device__ __forceinline__ DrawFilter draw_filter(const TopKPParams& p, int row) {
@@ -1042,7 +1043,7 @@ __global__ __launch_bounds__(kThreads) void sampling_list_kernel(const TopKPPara
         above[(size_t)row * S + blockIdx.x] = s_above;
     }
     if (s_n < 0) return;
-    uint2* out = list + (size_t)row * kList + s_base;
+    uint2* out = list + (size_t)row * draw_list(p.V) + s_base;
     const int lo = min(p.V, (int)blockIdx.x * slice), n = min(p.V, lo + slice) - lo;
     const float* x = p.probs + (size_t)row * p.ld + lo;
     const float least = __uint_as_float((uint32_t)(low + kDrawBase) << kDrawShift), next = __uint_as_float((uint32_t)(low + 1 + kDrawBase) << kDrawShift);
@@ -1075,7 +1076,7 @@ __global__ __launch_bounds__(kThreads) void draw_listed_kernel(const TopKPParams
     constexpr int PT = kList / kThreads, REST = 9;                              // values of a thread; bits behind the first 10 of the 19 that the list's values differ in
     uint2 e[PT];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) e[i] = tx + i * kThreads < r.n ? list[(size_t)row * kList + tx + i * kThreads] : make_uint2(0u, 0u);
+    for (int i = 0; i < PT; ++i) e[i] = tx + i * kThreads < r.n ? list[(size_t)row * draw_list(p.V) + tx + i * kThreads] : make_uint2(0u, 0u);
     sh.hist[tx] = 0ull; sh.hist[kThreads + tx] = 0ull;
     if (tx < S) s_slice[tx] = above[(size_t)row * S + tx];
     __syncthreads();
@@ -1259,8 +1260,9 @@ static int row_splits(int rows, int V) {
 }
 // The joint launches: of long rows as many blocks as hold their slices in registers.  64 x 152064, us of prepare, probabilities and list with 8 blocks a row (one round of two a compute
 // unit) 21.8 + 12.7 + 12.9, with 9 24.2 + 14.8 + 14.3; with 4, walked from memory, the first two took 31.7 before against 28.1 with 9.
+static int held_splits(int V) { const int held = (V + kHeld - 1) / kHeld; return held < kMostSplits ? held : kMostSplits; }
 static int joint_splits(int rows, int V) {
-    const int least = row_splits(rows, V), held = (V + kHeld - 1) / kHeld, near = held < kMostSplits ? held : kMostSplits;
+    const int least = row_splits(rows, V), near = held_splits(V);
     return least > near ? least : near;
 }
 
@@ -1327,17 +1329,20 @@ extern "C" int mi355_sampling_probs(float* logits, int32_t rows, int32_t V, int3
 // mi355_sampling_probs and mi355_top_k_top_p_sample (without its probabilities) in one: the logits become the probabilities, ids[row] is drawn from what the filter leaves.
 namespace {
 struct DrawWorkspace { size_t hist, above, list, listed, bytes; };                     // the slices' (maximum, sum) lie in front
-DrawWorkspace draw_workspace(int rows, int S) {
+constexpr int kDrawRows = 1024;                                                       // rows of a round of launches: four blocks a compute unit and more, at most 130 MB
+DrawWorkspace draw_workspace(int rows, int V) {                                       // no smaller for more rows
     DrawWorkspace w;
+    rows = rows < kDrawRows ? rows : kDrawRows;
+    const int most = rows * held_splits(V) > 256 ? rows * held_splits(V) : 256, slices = rows * kMostSplits < most ? rows * kMostSplits : most;         // rows * joint_splits at most
     w.hist = ((size_t)rows * kMostSplits * sizeof(float2) + 15) & ~(size_t)15;
-    w.above = w.hist + (size_t)rows * S * kDrawBins * sizeof(unsigned long long);
-    w.list = w.above + (size_t)rows * S * sizeof(unsigned long long);
-    w.listed = w.list + (size_t)rows * kList * sizeof(uint2);
+    w.above = w.hist + (size_t)slices * kDrawBins * sizeof(unsigned long long);
+    w.list = w.above + (size_t)slices * sizeof(unsigned long long);
+    w.listed = w.list + (size_t)rows * draw_list(V) * sizeof(uint2);
     w.bytes = w.listed + (size_t)rows * sizeof(DrawRow);
     return w;
 }
 } // namespace
-extern "C" size_t mi355_sampling_draw_workspace_bytes(int32_t rows, int32_t V) { return rows > 0 && V > 0 ? draw_workspace(rows, joint_splits(rows, V)).bytes : 0; }
+extern "C" size_t mi355_sampling_draw_workspace_bytes(int32_t rows, int32_t V) { return rows > 0 && V > 0 ? draw_workspace(rows, V).bytes : 0; }
 
 extern "C" int mi355_sampling_draw(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
                                    const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
@@ -1350,17 +1355,23 @@ extern "C" int mi355_sampling_draw(float* logits, int32_t rows, int32_t V, int32
     if (output_ids && step > kShortHistory) return MI355_ERR_UNSUPPORTED;
     const bool pen = output_ids && step > 0 && (repetition || presence || frequency);
     const int S = joint_splits(rows, V), slice = ((V + S - 1) / S + 3) & ~3;
-    const DrawWorkspace w = draw_workspace(rows, S);
+    const DrawWorkspace w = draw_workspace(rows, V);
     char* ws = (char*)workspace;
     hipStream_t st = (hipStream_t)stream;
-    const PenaltyParams p{logits, V, ld, temperature, repetition, presence, frequency, pen ? output_ids : nullptr, input_lengths, rows, max_input_length, step, nullptr};
-    if (int e = launch_probs<true>(p, workspace, id_step, id_row, S, slice, (unsigned long long*)(ws + w.hist), st)) return e;
-    const TopKPParams t{logits, V, ld, top_k, top_p, uniform_samples, ids, nullptr, 0};
-    auto* above = (unsigned long long*)(ws + w.above);
-    hipLaunchKernelGGL(sampling_list_kernel, dim3(S, rows), dim3(kThreads), 0, st, t, (const unsigned long long*)(ws + w.hist), slice, (DrawRow*)(ws + w.listed), above, (uint2*)(ws + w.list));
-    MI355_CHECK_LAUNCH("sampling_list_kernel");
-    hipLaunchKernelGGL(draw_listed_kernel, dim3(rows), dim3(kThreads), 0, st, t, S, slice, (const DrawRow*)(ws + w.listed), above, (const uint2*)(ws + w.list));
-    MI355_CHECK_LAUNCH("draw_listed_kernel");
+    for (int r0 = 0; r0 < rows; r0 += kDrawRows) {
+        const int n = rows - r0 < kDrawRows ? rows - r0 : kDrawRows;
+        auto from = [r0](auto* v) { return v ? v + r0 : v; };
+        float* x = logits + (size_t)r0 * ld;
+        const PenaltyParams p{x, V, ld, from(temperature), from(repetition), from(presence), from(frequency), pen ? output_ids + (size_t)r0 * id_row : nullptr, from(input_lengths), n,
+                              max_input_length, step, nullptr};
+        if (int e = launch_probs<true>(p, workspace, id_step, id_row, S, slice, (unsigned long long*)(ws + w.hist), st)) return e;
+        const TopKPParams t{x, V, ld, from(top_k), from(top_p), uniform_samples + r0, ids + r0, nullptr, 0};
+        auto* above = (unsigned long long*)(ws + w.above);
+        hipLaunchKernelGGL(sampling_list_kernel, dim3(S, n), dim3(kThreads), 0, st, t, (const unsigned long long*)(ws + w.hist), slice, (DrawRow*)(ws + w.listed), above, (uint2*)(ws + w.list));
+        MI355_CHECK_LAUNCH("sampling_list_kernel");
+        hipLaunchKernelGGL(draw_listed_kernel, dim3(n), dim3(kThreads), 0, st, t, S, slice, (const DrawRow*)(ws + w.listed), above, (const uint2*)(ws + w.list));
+        MI355_CHECK_LAUNCH("draw_listed_kernel");
+    }
     return MI355_OK;
 }
 

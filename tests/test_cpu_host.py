@@ -440,3 +440,14 @@ def test_attention_workspace_of_fewer_rows_is_no_larger(max_seq):
     sizes = [l.mi355_paged_attn_workspace_bytes(B, 28, 128, max_seq) for B in range(1, 8300)]
     assert all(a <= b for a, b in zip(sizes, sizes[1:]))
     assert all(s == min(B * -(-max_seq // 128), 8192) * one for B, s in enumerate(sizes, 1))
+
+
+@pytest.mark.parametrize("V", [1, 100, 8192, 32000, 152064, 1 << 20])
+def test_sampler_workspace_is_bounded(V):
+    """The joint draw: lists no longer than the row, and what 1024 rows take however many there are."""
+    l = _C.lib()
+    sizes = {rows: l.mi355_sampling_draw_workspace_bytes(rows, V) for rows in (1, 64, 1024, 1025, 65535)}
+    assert sizes[65535] <= 150 << 20 and sizes[1025] <= sizes[1024] <= 1024 * (8 * min(V, 8192) + 16 * (4096 + 16) + 64)
+    assert sizes[64] <= 64 * (8 * min(V, 8192) + 16 * (4096 + 16) + 64)
+    grow = [l.mi355_sampling_draw_workspace_bytes(rows, V) for rows in range(1, 1400)]
+    assert all(a <= b for a, b in zip(grow, grow[1:]))           # a caller may size it once for the most rows

@@ -26,8 +26,9 @@ def _logits(kind, B, V, g):
     return x
 
 
-# rows of one slice and of sixteen, slices held in registers (up to 20480 values) and walked, rows off 16 bytes, a vocabulary below one load
-@pytest.mark.parametrize("B,V", [(1, 7), (3, 1000), (2, 8191), (5, 32001), (1, 152064), (64, 20484), (300, 4099), (2, 400003)])
+# rows of one slice and of sixteen, slices held in registers (up to 20480 values) and walked, rows off 16 bytes, a vocabulary below one load, rows of one round of
+# launches and one more, of three
+@pytest.mark.parametrize("B,V", [(1, 7), (3, 1000), (2, 8191), (5, 32001), (1, 152064), (64, 20484), (300, 4099), (2, 400003), (1025, 100), (2100, 33)])
 @pytest.mark.parametrize("kind", ["peaked", "flat", "ties", "masked", "spike"])
 def test_joint_draw_equals_separate_launches(B, V, kind):
     g = torch.Generator(device=DEV).manual_seed(B * 1000 + V)
