@@ -76,3 +76,23 @@ def test_rows_without_a_filter_take_the_separate_launches(monkeypatch, top_k, to
     assert calls == ["joint" if joint else "separate"]
     probs = ops.sampling_probs(x.clone())
     assert torch.equal(logits, probs) and torch.equal(ids, two(probs, k.to(DEV), p.to(DEV), u.to(DEV)))
+
+
+# a row is not counted from 8193 values on, where they are equal; one more value here and there, half of a row masked
+@pytest.mark.parametrize("B,V", [(2, 8192), (2, 8193), (70, 8200), (3, 32001), (2, 152064)])
+@pytest.mark.parametrize("kind", ["equal", "one above", "half masked", "beside others"])
+def test_rows_too_flat_to_count(B, V, kind):
+    x = torch.full((B, V), 1.5, device=DEV)
+    if kind == "one above":
+        x[:, V // 3] = 2.0
+    elif kind == "half masked":
+        x[:, ::2] = float("-inf")
+    elif kind == "beside others":
+        x[1:] = torch.randn(B - 1, V, device=DEV, generator=torch.Generator(device=DEV).manual_seed(V)) * 3
+    k, u = torch.zeros(B, dtype=torch.int32, device=DEV), torch.linspace(0.01, 0.99, B, device=DEV)
+    for p in (0.3141, 0.9017):                # between two prefixes of equal values: their fp32 and exact sums keep as many
+        p = torch.full((B,), p, device=DEV)
+        want = ops.sampling_probs(x.clone())
+        got = x.clone()
+        ids = ops.sampling_draw(got, k, p, u)
+        assert torch.equal(got, want) and torch.equal(ids, ops.top_k_top_p_sample(want, k, p, u))
