@@ -652,8 +652,9 @@ __global__ __launch_bounds__(1024) void hy_attn_rows_kernel(const float* q, int 
 #pragma unroll
     for (int i = 0; i < 8; ++i) qv[i] = (coop && kl_ok) ? q_s[kl * 8 + i] : 0.f;
     // 64 keys a wave and trip; of short contexts 16 or 32, so that all waves have some: 8 rows of 16 heads over about 100 keys 15.7 us on two
-    // of sixteen waves, 12.3 on seven
-    const int tile = (const void*)kcache == (const void*)vcache ? 64 : nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;        // a latent cache's rows: 64 as ever
+    // of sixteen waves, 12.3 on seven.  Not over a latent cache (one tensor for keys and values), which is what the models with routers have: they keep the sums they had (eight
+    // sequences served by one 7.8 ms, 7.3 with short tiles)
+    const int tile = (const void*)kcache == (const void*)vcache ? 64 : nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;
     for (int t0 = (sp * NW + wave) * tile; t0 < nvis; t0 += tile * NW * S) {
         const int kj = t0 + lane < kept ? t0 + lane : t0 + lane - kept + lo;
         const bool valid = lane < tile && kj <= p;
@@ -882,7 +883,9 @@ __device__ __forceinline__ float hy_sum_groups(float v) {
     hy_swap<32>(v, a, b); v = a + b;
     hy_swap<16>(v, a, b); return a + b;
 }
-constexpr int AT_SOLO = 20;                       // walks of up to this many steps (640 keys) gain little from a second group (18.7 / 17.5 us at 256 rows) and keep one group's sums
+// Walks of up to this many steps (640 keys) keep one group's sums.  A second group would gain there too (us with one / two, 512 rows 30.2 / 24.8, 256 18.7 / 17.5), but models with routers
+// are served over such contexts, and another rounding in front of a router sends a token between two experts to the other one.
+constexpr int AT_SOLO = 20;
 constexpr int AT_STAGES = 3, AT_PAGES = 1024;     // block-table entries of the walked range held in LDS
 
 // DK: 32-channel steps of a key row.  NCBM: 16-channel fragments of a value row the instance holds; they are multiplied by fours (fragments past the row's end hold what lies
