@@ -479,8 +479,8 @@ WALK_MAX_DIM = 128         # key channels of mi355_hy_walk
 
 @functools.lru_cache(maxsize=64)      # the layers of a step ask for the same
 def gated_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int) -> Optional[int]:
-    """How a gated recurrence of keys up to WALK_MAX_DIM channels runs where even a walk token by token gains on hy_scan: a chunk size, 0 (whole) or None (no gain; tiles_form looks
-    again).  A model of the forms in us, fitted to 460 calls of such a walk: 2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64 sequences of 1 to 2048 rows."""
+    """How a gated recurrence of keys up to WALK_MAX_DIM channels runs where even a slower walk than hy_walk's would gain on hy_scan: a chunk size, 0 (whole) or None (no such gain).  A
+    model of the forms in us, fitted to 460 calls of a walk token by token (2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64 sequences of 1 to 2048 rows)."""
     longest = max_rows if max_rows > 0 else T - (nseq - 1)
     waves = -(-dim // 8)
     scan_us = 5.5 + (0.22 + 0.0145 * waves) * max(longest, -(-nseq * heads * -(-vdim // 64) // (256 * (16 // waves))) * T / nseq)
@@ -496,7 +496,10 @@ def gated_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int
     return best if 1.05 * us < scan_us else None
 
 
-FIXED_TILES_FROM = 640     # rows of the longest sequence: shorter walks under a constant decay gain a few us and keep the sums of hy_scan
+# Rows of the longest sequence up to which a constant decay keeps hy_scan and its sums.  Not for its cost (8 heads of 64 x 128, 512 rows 45.4 us, 23.7 on tiles; 16 heads, 4 x 512 rows
+# 118 and 57): models with such a recurrence have routers behind it, where another rounding sends a token between two experts to the other one, and steps of this length are what
+# such models are served in.  There some batches' logits moved by 4e-2 and 1e-1, as far as they are from 64 bits; longer prompts are scored, and theirs did not.
+FIXED_TILES_FROM = 640
 CHUNKS_HOST_US = 25        # two more launches and two buffers of a call in chunks: shows where launches bound a step (two prompts of 99 rows, 8 layers: 940 us, 1087 in chunks)
 
 
@@ -519,6 +522,18 @@ def tiles_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int
             if t < us:
                 best, us = C, t
     return best if margin * us < scan_us else None
+
+
+def scan_form(mode: int, T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int) -> Optional[int]:
+    """How `scan` runs keys of up to WALK_MAX_DIM channels when the choice is its own: hy_walk over chunks of the size returned, hy_walk whole (0) or hy_scan (None).  Gated recurrences
+    that gated_form answers keep its form: over 112 such calls it is 4 % off the fastest on the GPU in the mean, at most half as much again, and takes 0.36 of hy_scan's time (at most
+    0.83).  tiles_form, which counts the host's time for chunks as well, would leave half of them (most of the 112 are calls where the two differ) whole or to hy_scan, at up to 2.6
+    times the time on the GPU.  The rest is tiles_form's, HGRN2 with a wider margin: hy_scan is 10 % faster there, the tiles with their 64-bit sums up to 15 % slower."""
+    fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
+    if fixed and max_rows <= FIXED_TILES_FROM:
+        return None
+    C = None if fixed else gated_form(T, nseq, max_rows, heads, dim, vdim)
+    return tiles_form(T, nseq, max_rows, heads, dim, vdim, 1.35 if mode == SCAN_HGRN2 else 1.05) if C is None else C
 
 
 def scan_prefers_chunks(T: int, nseq: int, max_rows: int, heads: int, vdim: int, C: int) -> bool:
@@ -549,7 +564,7 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
          heads: int, dim: int, vdim: int, row_start, slot, first_pos, state: torch.Tensor, act: torch.dtype, *, plans: Optional[dict] = None,
          chunked: Optional[bool] = None, max_rows: int = 0) -> torch.Tensor:
     """Gated linear recurrence over the rows of every sequence, continuing (and leaving) the fp32 state of its slot -> fp32 [T, heads * vdim].
-    Keys of up to WALK_MAX_DIM channels run on tiles of tokens (hy_walk) where that is expected to be faster (gated_form, tiles_form; max_rows = the rows of the step's longest
+    Keys of up to WALK_MAX_DIM channels run on tiles of tokens (hy_walk) where that is expected to be faster (scan_form; max_rows = the rows of the step's longest
     sequence when the caller knows it), long portions in chunks side by side, the same sums in another order: what every chunk leaves from a zero state and its total decays, a prefix
     over each sequence's chunks, then the tokens again from the chunk-start states.  Longer keys under a constant decay per head (SCAN_FIXED, SCAN_FIXED_SILU) walk token by token,
     in chunks where that pays (scan_prefers_chunks): every chunk from a zero state, the prefix, then the chunk-start states' share of the outputs.
@@ -568,18 +583,13 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
                                           act_code(act), _stream()), "hy_scan")
 
     fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
-    if chunked is None and dim <= WALK_MAX_DIM and (not fixed or max_rows > FIXED_TILES_FROM) and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim):
+    C = scan_form(mode, T, nseq, max_rows, heads, dim, vdim) if chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim) else None
+    if C is not None:
         def walk(rs, sl, fp, n, st, dst, cdecay, keep):
             _C.check_hybrid(lib.mi355_hy_walk(mode, proj.data_ptr(), ld, qo, ko, vo, _p(z), 0 if z is None else _rows(z, "scan.z"), _p(lower), _p(fbias), float(tau),
                                               float(qscale), heads, dim, vdim, rs.data_ptr(), sl.data_ptr(), fp.data_ptr(), n, st.data_ptr(), _p(dst), _p(cdecay), keep,
                                               act_code(act), _stream()), "hy_walk")
 
-        C = None if fixed else gated_form(T, nseq, max_rows, heads, dim, vdim)
-        if C is None:
-            C = tiles_form(T, nseq, max_rows, heads, dim, vdim, 1.35 if mode == SCAN_HGRN2 else 1.05)       # HGRN2: hy_scan 10 % faster, the tiles (64-bit sums) 15 to 20 % slower
-        if C is None:
-            run(mode, row_start, slot, first_pos, nseq, state)
-            return out
         if not C:
             walk(row_start, slot, first_pos, nseq, state, out, None, 1)
             return out

@@ -1,5 +1,5 @@
-"""Which form the gated recurrences take: in calls whose forms were all measured (us on one MI355X) the pick costs no more than the walk that every call took once, and at most a third more
-than the fastest (the model's own error)."""
+"""What gated_form answers, against the times that it was fitted to: those of a walk token by token (us on one MI355X).  The pick costs no more than hy_scan, and at most a third more than
+the fastest (the model's own error).  What hy_walk's tiles take, and the rule in use, is in test_scan_form.py."""
 import pytest
 
 from rtp_llm_amd import hybrid_ops as hops
