@@ -933,8 +933,9 @@ extern "C" int mi355_decoder_prefill_ragged(mi355_decoder_t* d, const int32_t* t
 }
 
 // Us of a call one pass after the other / overlapped (the 0.5B model in passes of 512 tokens a prompt, 16-bit weights: 1 x 777 3571 / 2931, 1 x 1500 6477 / 5295, 4 x 1000 9363 / 7541;
-// 4 bits: 1 x 3000 12148 / 8552; the 7B model, 4 bits: 1 x 600 15288 / 14095, 2 x 1024 35701 / 30655, 8 x 1024 111971 / 105304; 8 bits: 1 x 1024 21701 / 18653).  Larger passes were
-// not measured, and want a second workspace of their size.  Under tensor parallelism two passes would meet in the collectives' buffers.
+// 4 bits: 1 x 3000 12148 / 8552; the 7B model, 4 bits: 1 x 600 15288 / 14095, 2 x 1024 35701 / 30655, 8 x 1024 111971 / 105304; 8 bits: 1 x 1024 21701 / 18653).  Short tails too: one
+// row behind 512 3256 / 2392 and 12798 / 11722 (0.5B, 7B), 8 behind 2 x 512 5504 / 4292, 8 x (512 + 8) 57805 / 55773; and short passes, 512 rows in 16s 42610 / 38452 and 86074 / 58133.
+// Larger passes were not measured, and want a second workspace of their size.  Under tensor parallelism two passes would meet in the collectives' buffers.
 extern "C" int mi355_decoder_prefill_overlaps(mi355_decoder_t* d, int32_t rows) { return d && d->cfg.tp_size == 1 && rows <= 4096; }
 
 // Even passes run on the caller's stream and odd ones beside it; only passes of one stream wait for each other's ends.

@@ -3246,7 +3246,7 @@ extern "C" int mi355_hy_head_norm_ex3(const float* o, int32_t ldo, int32_t rows,
         MI355_CHECK_LAUNCH("hy_head_norm4_kernel");
         return MI355_OK;
     }
-    HY_DISPATCH(act_dtype, hipLaunchKernelGGL(hy_head_norm_kernel<T>, dim3(rows, H), dim3(vdim > 256 ? std::min(1024, (vdim + 255) / 256 * 64) : 64), 0, (hipStream_t)stream, o, ldo, H, vdim, (const T*)w, eps,
+    HY_DISPATCH(act_dtype, hipLaunchKernelGGL(hy_head_norm_kernel<T>, dim3(rows, H), dim3(std::min(1024, (vdim + 255) / 256 * 64)), 0, (hipStream_t)stream, o, ldo, H, vdim, (const T*)w, eps,
                                               gate, ldg, goff, (T*)out, w_heads, gate_sigmoid, den));
     MI355_CHECK_LAUNCH("hy_head_norm_kernel");
     return MI355_OK;
