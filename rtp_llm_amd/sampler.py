@@ -112,8 +112,9 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
             up["history"] = history if together else history.t()
     if draw:
         top_p = _host(params.top_p, torch.float32).clone()
-        top_p[top_p.abs() < 1e-7] = 1.0
-        filtered = _off(top_p, 1.0) or (_off(top_k, 0) and bool(((top_k.numpy() > 0) & (top_k.numpy() < V)).any()))
+        p = top_p.numpy()
+        p[np.abs(p) < 1e-7] = 1.0
+        filtered = bool((p != 1.0).any()) or (_off(top_k, 0) and bool(((top_k.numpy() > 0) & (top_k.numpy() < V)).any()))
         up.update(top_k=top_k, top_p=top_p)
         if params.uniform.device.type == "cpu":
             up["uniform"] = params.uniform.to(torch.float32)
