@@ -1541,7 +1541,7 @@ __global__ __launch_bounds__(1024) void hy_scan_kernel(ScanParams p) {
 // the state is never moved; a block is 128 columns.  P (136 of 256 pairs) is formed by the vector units once per head.  Walking token by token took 5 vector operations per state
 // value and token in the two passes over chunks and was bound by them.  OUT: outputs are formed; without them (the first of the two passes over chunks) only the state each
 // chunk leaves from zero and, in cdecay [sequences, H, dim], the product of its decays.
-// 16 heads of 64 x 128, four sequences of 2048 tokens in chunks of 128: states 106.7 -> 49 us, outputs 136.5 -> 86; one sequence of 1537, 8 heads, chunks of 32: all 60.5 -> 42 us.
+// 16 heads of 64 x 128, four sequences of 2048 tokens in chunks of 128: states 106.7 -> 48 us, outputs 136.5 -> 97 (HGRN2 44 and 110); one sequence of 1537, 8 heads, chunks of 32: all 60.5 -> 42 us.
 // A block alone takes 4 us a tile, of which 2304 cycles are products; the rest is its chain of two barriers, LDS and exponentials, which four blocks of a compute unit hide (128
 // registers; HGRN2's outputs three).  Products of decays are formed in 64 bits (a constant decay's powers would carry one rounding from tile to tile), sums as short chains and trees,
 // P's tree over the lanes in 64 bits under gates.
