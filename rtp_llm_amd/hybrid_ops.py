@@ -508,12 +508,14 @@ def tiles_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int
     """How a recurrence of keys up to WALK_MAX_DIM channels runs: hy_walk over chunks of the size returned, hy_walk whole (0) or hy_scan (None).  A model of the forms in us: what the
     longest sequence (chunk) takes in series, or what the chip takes for all tokens if that is more.  Fitted to 120 calls of 2 to 32 heads, keys of 32 to 128, values of 64 to 256, 1 to 64
     sequences of 2 to 2048 rows: 10 to 13 % off in the root mean square; the pick is 2 % off the fastest in the mean (chunks with their host time), at most 35 %, and 1 %
-    behind hy_scan at worst.  HGRN2 asks for a wider margin: hy_scan is 10 % faster there and the tiles, with 64-bit sums, 15 to 20 % slower.
+    behind hy_scan at worst.  HGRN2 asks for a wider margin: hy_scan is 10 % faster there and the tiles, with 64-bit sums, 15 to 20 % slower.  Keys of 65 to 127 channels are not whole
+    in what either kernel does at once; hy_scan's throughput there is put at its best (1.5): with that of narrow keys (2.51) 13 of 117 calls lost up to 20 % to it (32 sequences of up to
+    38 rows, 4 heads of 80 x 128 20.2 / 23.5 us, now hy_scan), with 1.5 one of 247 loses 4 %, and the pick is 4 % off the fastest in the mean.
     Measured, us, hy_scan / whole / chunks: 16 heads of 64 x 128, 4 x 2048 rows 673 / 581 / 156 (128), 8 x 40 20 / 19 / 32 (32); 32 heads of 128 x 128, 9 x 136 227 / 83 / 138 (64);
     8 heads of 128 x 256, 8 x 195 115 / 81 / 82 (64); 16 heads of 32 x 64, 16 x 2 7.6 / 10.4 / -."""
     longest = max_rows if max_rows > 0 else T - (nseq - 1)
     waves, work, wide = -(-dim // 8), T * heads * -(-vdim // 128), dim > 64
-    scan_us = 7.1 + (0.254 + 0.0108 * waves) * max(longest, 2.51 * T * heads * -(-vdim // 64) / (256 * (16 // waves)))
+    scan_us = 7.1 + (0.254 + 0.0108 * waves) * max(longest, (1.5 if wide else 2.51) * T * heads * -(-vdim // 64) / (256 * (16 // waves)))
     best, us = 0, 10.0 + 0.34 * max(longest, work / 170) if wide else 9.0 + 0.26 * max(longest, work / 200)
     for C in (32, 64, 128):
         if longest > C:

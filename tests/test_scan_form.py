@@ -61,6 +61,11 @@ CALLS = {
                                HGRN2: dict(scan=37.9, walk=36.1, c32=21.0, c64=32.2)},
     (906, 8, 171, 16, 64, 128): {GLA: dict(scan=62.4, walk=54.9, c32=47.2, c64=53.1, c128=68.5),
                                  HGRN2: dict(scan=57.6, walk=52.1, c32=48.0, c64=54.2, c128=65.4)},
+    (375, 8, 68, 8, 96, 256): {HGRN2: dict(scan=32.4, walk=39.0)},
+    (54, 1, 54, 32, 80, 256): {GLA: dict(scan=25.9, walk=29.9)},
+    (776, 32, 38, 4, 80, 128): {GLA: dict(scan=20.2, walk=23.5)},
+    (5486, 64, 131, 2, 80, 128): {GLA: dict(scan=55.0, walk=61.2)},
+    (5840, 32, 282, 4, 128, 256): {GLA: dict(scan=287.8, walk=119.5)},
 }
 
 
