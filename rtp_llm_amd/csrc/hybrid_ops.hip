@@ -3237,7 +3237,10 @@ extern "C" int mi355_hy_head_norm_ex3(const float* o, int32_t ldo, int32_t rows,
                                       int32_t goff, void* out, int32_t w_heads, int32_t gate_sigmoid, const float* den, int32_t act_dtype,
                                       mi355_stream_t stream) {
     MI355_CHECK_ARG(o && out && rows > 0 && H > 0 && vdim > 0 && ldo >= H * vdim, "hy_head_norm: bad argument");
-    if (vdim <= 256 && (int64_t)rows * H <= INT32_MAX - 256) {
+    // Several heads a block: from 129 channels on, where a wave by itself makes a second trip, and of shorter heads where they fill the chip; a few of them are done sooner by a wave each.
+    // Us of a wave each / several a block, with gate: 128 heads of 64 2.6 / 3.4, 2048 2.9 / 3.5, 4096 3.5 / 3.5, 8192 4.6 / 3.9; 128 heads of 128 3.1 / 3.6,
+    // 2048 3.5 / 3.6, 4096 4.1 / 3.9, 32768 18.4 / 11.4; 16 heads of 192 3.6 / 3.0.
+    if (vdim <= 256 && (int64_t)rows * H <= INT32_MAX - 256 && (vdim > 128 || rows * H >= 4096)) {
         const int n = rows * H, G = vdim <= 32 ? 8 : vdim <= 64 ? 16 : vdim <= 128 ? 32 : 64;
 #define HY_HEAD_NORM4(G_) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_head_norm4_kernel<T, G_>), dim3((n + 256 / G_ - 1) / (256 / G_)), dim3(256), 0, (hipStream_t)stream, o, ldo, H, \
                                       vdim, (const T*)w, eps, gate, ldg, goff, (T*)out, w_heads, gate_sigmoid, den, n))

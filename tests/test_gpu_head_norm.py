@@ -1,4 +1,4 @@
-"""Head norms of several heads a block (up to 256 channels) and of one, against 64-bit arithmetic.  Error: sums of at most 1024 squares, one reciprocal root and the gate,
+"""Head norms of several heads a block (129 to 256 channels, and shorter ones from 4096 heads on) and of one, against 64-bit arithmetic.  Error: sums of at most 1024 squares, one reciprocal root and the gate,
 a few roundings of 2^-24 each, then one rounding to the activation type."""
 import pytest
 import torch
@@ -10,7 +10,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,H,vdim", [(1, 1, 4), (3, 5, 32), (7, 3, 36), (33, 2, 64), (5, 16, 128), (9, 3, 132), (2, 7, 256), (3, 2, 260), (5, 3, 30), (65, 1, 128)])
+@pytest.mark.parametrize("rows,H,vdim", [(1, 1, 4), (3, 5, 32), (7, 3, 36), (33, 2, 64), (5, 16, 128), (9, 3, 132), (2, 7, 256), (3, 2, 260), (5, 3, 30), (65, 1, 128), (512, 8, 4), (1024, 4, 32), (585, 7, 36), (1365, 3, 64), (4097, 1, 30), (257, 16, 100), (64, 64, 128)])
 @pytest.mark.parametrize("goff,gate_act,per_head", [(None, "silu", False), (4, "silu", True), (3, "sigmoid", False), (8, "sigmoid", True)])
 def test_head_norm(rows, H, vdim, goff, gate_act, per_head, dtype):
     g = torch.Generator(device=DEV).manual_seed(rows + vdim)
