@@ -3142,10 +3142,10 @@ extern "C" int mi355_hy_chunk_prefix_rows(const int32_t* cs, const int32_t* sc, 
                                           const float* cdecay, int32_t row_len, int32_t H, int32_t per_head, float* chunk_state, float* state, mi355_stream_t stream) {
     MI355_CHECK_ARG(cs && sc && slot && first_pos && (decay || cdecay) && chunk_state && state && nseq > 0 && H > 0 && per_head > 0, "hy_chunk_prefix: nseq=%d H=%d", nseq, H);
     MI355_CHECK_ARG(row_len == 0 || (row_len > 0 && per_head % row_len == 0 && cdecay), "hy_chunk_prefix: rows of %d in %d", row_len, per_head);
-    // A few blocks wait for one chunk after the other; a chip full of them is bound by the states' bytes and wants the smaller loop: 48 chunks of 8 heads of 64 x 128 18.5 us one at a
-    // time, 11.0 in eights; 4 sequences of 16 chunks of 16 heads 13.9 / 14.4, 8 of 3 chunks 9.1 / 10.4.
+    // A few blocks wait for one chunk after the other; a chip full of them is bound by the states' bytes and wants the smaller loop.  Us one at a time / in eights, heads of 64 x 128: 256
+    // blocks of 32 chunks 8.5 / 7.2, of 8 4.0 / 3.8; 512 of 32 9.7 / 9.2, of 3 3.3 / 3.3; 1024 of 16 7.6 / 8.6, of 3 3.8 / 4.0, of 32 15.5 / 13.7.
     const dim3 grid(nseq, H, (per_head + 255) / 256);
-    if ((uint64_t)grid.x * grid.y * grid.z <= 1024)
+    if ((uint64_t)grid.x * grid.y * grid.z <= 512)
         hipLaunchKernelGGL(hy_chunk_prefix_kernel<8>, grid, dim3(256), 0, (hipStream_t)stream, cs, sc, slot, first_pos, decay, H, per_head, chunk_state, state, cdecay, row_len);
     else
         hipLaunchKernelGGL(hy_chunk_prefix_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, cs, sc, slot, first_pos, decay, H, per_head, chunk_state, state, cdecay, row_len);
