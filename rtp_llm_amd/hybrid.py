@@ -592,10 +592,10 @@ class HybridModel:
                     proj = hops.dense_linear(h1, gate_w[:n_in], out_dtype=torch.float32)
                     g = hops.dense_linear(h1, gate_w[n_pad:], gate_b[n_pad:], out_dtype=torch.float32)
                 a = mixer.forward(h1, batch, *cache, proj=proj) if isinstance(cache, tuple) else mixer.forward(h1, batch, cache, proj=proj)
-            elif gate_w is None and isinstance(mlp, GatedMLP) and hasattr(mixer, "few_rows") and mixer.few_rows(T) is not None:
+            elif gate_w is None and isinstance(mlp, GatedMLP) and hasattr(mixer, "few_rows") and mixer.few_rows(T, batch) is not None:
                 # few rows: the two branches read the same stream, so their input linears are one launch, and their output linears another
                 g = None
-                w, bias = mixer.few_rows(T)
+                w, bias = mixer.few_rows(T, batch)
                 proj, up = hops.dense_pair(dict(x=h1, w=w, bias=bias, out_dtype=torch.float32),
                                            dict(x=h2, w=mlp.w_gate_up, gated=True, act=mlp.act, act_param=mlp.act_param))
                 o = mixer.forward(h1, batch, *(cache if isinstance(cache, tuple) else (cache,)), proj=proj, out_proj=False)

@@ -242,7 +242,7 @@ class PagedChunkAttention:
                                                   num_pages))
         return self._geom[1]
 
-    def few_rows(self, T: int):
+    def few_rows(self, T: int, batch: StepBatch):
         """(weight, bias) of the input linear of a step of few rows; None: not such a step."""
         return (self.w_in, self.b_in) if T <= hops.FEW_ROWS else None
 
@@ -332,16 +332,25 @@ class GatedLinearRecurrence:
         s = self.spec
         return (s.heads, s.dim, s.vdim)
 
-    def few_rows(self, T: int):
-        """(weight, bias) of the input linear of a step of few rows, whose fp32 result `forward` takes as proj; None: not such a step."""
-        if T > hops.FEW_ROWS or not hops.recur_step_supported(self.spec.dim, self.spec.vdim) or (self.mode == hops.SCAN_GLA and self.w_a2.shape[1] > hops.STEP_MAX_RANK):
+    def few_rows(self, T: int, batch: StepBatch):
+        """(weight, bias) of the input linear of a step of few rows, whose fp32 result `forward` takes as proj; None: not such a step.
+        recur_step pays a trip to memory for every token of a sequence, hy_scan one for sixteen.  Mixers alone, us of scan and norm / recur_step, sequences x rows: GLA, 8 heads of
+        64 x 128 8 x 1 27 / 16, 8 x 2 27 / 19, 1 x 8 28 / 32, of 128 x 256 1 x 2 27 / 27, 1 x 3 41 / 45, 1 x 16 39 / 94; HGRN2 of 64 x 128 8 x 1 17 / 15, 1 x 2 15 / 15, 1 x 4 17 / 19, 1 x 16
+        21 / 41, and at one row 256 x 128 22 / 20, 64 x 256 17 / 16, 128 x 192 17 / 19, 128 x 256 18 / 21 (a thread then holds 26 and 32 key rows)."""
+        s = self.spec
+        if T > hops.FEW_ROWS or not hops.recur_step_supported(s.dim, s.vdim):
             return None
-        return self.w_few, None
+        longest = batch.max_rows if batch.max_rows > 0 else T - (batch.slot.numel() - 1)
+        if self.mode == hops.SCAN_GLA:
+            few = longest <= 2 and self.w_a2.shape[1] <= hops.STEP_MAX_RANK
+        else:
+            few = longest <= 1 and (s.vdim <= 128 or s.dim * s.vdim <= 16384)
+        return (self.w_few, None) if few else None
 
     def forward(self, h: torch.Tensor, batch: StepBatch, state: torch.Tensor, proj: Optional[torch.Tensor] = None, out_proj: bool = True) -> torch.Tensor:
         """proj: h w^T for the weight that few_rows names, when the caller has computed it.  out_proj False: without the output projection."""
         s = self.spec
-        few = self.few_rows(h.shape[0])
+        few = self.few_rows(h.shape[0], batch)
         if few is not None:
             if proj is None:
                 proj = hops.dense_linear(h, self.w_few, out_dtype=torch.float32)
