@@ -652,9 +652,10 @@ __global__ __launch_bounds__(1024) void hy_attn_rows_kernel(const float* q, int 
 #pragma unroll
     for (int i = 0; i < 8; ++i) qv[i] = (coop && kl_ok) ? q_s[kl * 8 + i] : 0.f;
     // 64 keys a wave and trip; of short contexts 16 or 32, so that all waves have some: 8 rows of 16 heads over about 100 keys 15.7 us on two
-    // of sixteen waves, 12.3 on seven.  Not over a latent cache (one tensor for keys and values), which is what the models with routers have: they keep the sums they had (eight
+    // of sixteen waves, 12.3 on seven.  Not for keys of up to 64 channels, of which eight loads bring 64 anyway (16 rows of 14 heads over 260 keys 11.4 us, 13.6 with short tiles), and
+    // not over a latent cache (one tensor for keys and values), which is what the models with routers have: they keep the sums they had (eight
     // sequences served by one 7.8 ms, 7.3 with short tiles)
-    const int tile = (const void*)kcache == (const void*)vcache ? 64 : nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;
+    const int tile = (const void*)kcache == (const void*)vcache || g.dim <= 64 ? 64 : nvis <= 16 * NW * S ? 16 : nvis <= 32 * NW * S ? 32 : 64;
     for (int t0 = (sp * NW + wave) * tile; t0 < nvis; t0 += tile * NW * S) {
         const int kj = t0 + lane < kept ? t0 + lane : t0 + lane - kept + lo;
         const bool valid = lane < tile && kj <= p;
