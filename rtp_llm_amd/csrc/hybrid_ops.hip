@@ -966,6 +966,7 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
     }
 #pragma unroll
     for (int j = 0; j < JVM; ++j) voff[j] = (uint32_t)((vpiece[j] & 31) * g.v_ld + (vpiece[j] >> 5)) * 2u;
+    bool shared = false;                                      // a run's steps were dealt over the groups
     // the tiles of the block in runs of one sequence (one run unless a block's tiles belong to several): the run's keys are staged for all its tiles
     for (int ft = 0; ft < ntw;) {
         const int fr = tile_row0[first_tile + ft], sq = seq[fr];
@@ -988,6 +989,7 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
         int bt0 = INT_MIN;                                    // first block-table entry in LDS
         const int ks = nsteps > AT_SOLO ? KG : 1;             // groups at work on this run; the others keep to the barriers
         const int rounds = (nsteps + ks - 1) / ks;
+        shared |= ks > 1;
         auto issue = [&](int round, int buf) {                // KG steps, one a group (several only without kept tokens: their keys follow each other)
             const int plo = page_of(step_key(round * ks)), phi = page_of(min(step_key(round * ks) + 32 * ks - 1, klast));
             if (bt0 == INT_MIN || plo < bt0 || phi >= bt0 + AT_PAGES) {        // seldom: the same for the whole block
@@ -1126,7 +1128,8 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
         }
     }
     float lt = hy_sum_groups(l);
-    if (KG > 1) {                                             // the first group takes the others' parts over
+    if (group > 0) has = false;
+    if (shared) {                                             // the first group takes the others' parts over
         __syncthreads();
         constexpr int PART = (NCBM * 16 + 8) * 64;
         char* part = at_smem + wave * PART;
@@ -1134,7 +1137,6 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
 #pragma unroll
             for (int cb = 0; cb < NCBM; ++cb) *(f32x4*)(part + (cb * 64 + lane) * 16) = o[cb];
             *(float2*)(part + NCBM * 1024 + lane * 8) = make_float2(m, lt);
-            has = false;
         }
         __syncthreads();
         if (group == 0) {
@@ -2968,7 +2970,11 @@ extern "C" int mi355_hy_attn_tiles_ex3(const float* q, int32_t ldq, float scale,
     // Two groups of waves walk the keys of a block where the grid leaves them compute units: us with one / two, 8 heads over a latent row of 256 (192) 64 rows 10.3 / 11.9, 131 14.4 / 14.5,
     // 256 18.7 / 17.5, 512 30.2 / 24.8, 1024 52.4 / 39.4, 1537 76.5 / 55.3, 2048 (256 blocks) 99.5 / 71.2, 2 x 2048 (512) 127.2 / 127.5; 16 over 4 heads of 128 131 rows 12.5 / 11.5,
     // 777 37.7 / 27.8, 1024 (256 blocks) 46.9 / 33.6, 1537 (388) 52.1 / 51.6, 2048 (512) 56.7 / 64.7.
-    const bool two = grid.x * grid.y <= 320 && keep == 0 && 2 * staged + 4 * AT_PAGES <= 160 * 1024;
+    // Not where no block can have a walk that the groups would share (AT_SOLO): 4 sequences of up to 1568 rows, 4 heads of 128 in a window of 64 16.2 us, 24.4 with the second group idle.
+    int keys = g.max_blocks * (int64_t)g.page > INT_MAX ? INT_MAX : g.max_blocks * g.page;
+    const int span = chunk > 0 ? chunk : window;
+    if (span > 0 && span < keys - 64 / HW - 32) keys = span + 64 / HW + 32;     // of the first row's first key's step to the last row
+    const bool two = grid.x * grid.y <= 320 && keep == 0 && keys > 32 * AT_SOLO && 2 * staged + 4 * AT_PAGES <= 160 * 1024;
 #define HY_TILES(DK_, NCBM_)                                                                                                                                     \
     do {                                                                                                                                                         \
         const int KG = two ? at_groups(DK_, NCBM_) : 1, part = KG > 1 ? 4 * (NCBM_ * 16 + 8) * 64 : 0, lds = std::max(KG * staged + 4 * AT_PAGES, std::max(part, turned)); \

@@ -21,7 +21,8 @@ CASES = [  # dim, vdim, heads, kv_heads, page, options
 
 
 @pytest.mark.parametrize("dim,vdim,H,G,page,opt", CASES)
-@pytest.mark.parametrize("starts,counts", [([0], [7]), ([0, 70, 250], [45, 130, 17]), ([3, 0, 0, 1, 0], [1, 2, 31, 16, 33]), ([1300], [40])])
+# the last: walks that two groups of waves share and such that one keeps, also in one block
+@pytest.mark.parametrize("starts,counts", [([0], [7]), ([0, 70, 250], [45, 130, 17]), ([3, 0, 0, 1, 0], [1, 2, 31, 16, 33]), ([1300], [40]), ([1300, 3, 700, 0, 590], [20, 9, 5, 16, 40])])
 def test_portions(dim, vdim, H, G, page, opt, starts, counts):
     g = torch.Generator(device=DEV).manual_seed(dim + vdim + H + len(starts))
     off, n = opt.get("off", 0), len(starts)
