@@ -32,7 +32,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E spec peak (/opt/skills/guides/MI355X_MICROARCH.md)
-TRAFFIC_FILE = "r06_traffic.json"   # profiles/: PMC traffic of the engine's linears, tools/engine_traffic.sh
+TRAFFIC_FILE = "engine_traffic.json"   # profiles/: PMC traffic of the engine's linears, tools/engine_traffic.sh
 
 WORKLOADS = {
     # name: (model, weight kind, kv_int8, default batch, default ctx, page)
@@ -401,7 +401,7 @@ def main():
         traffic, traffic_src, kernel_us = None, None, None
         if traffic_ok:
             try:  # HBM read + write bytes per launch of THESE launches (the engine's four linears per layer), from the committed
-                # rocprofv3 --pmc passes over `bench.py --no-graph` (tools/engine_traffic.sh -> profiles/r05_traffic.json); PMC
+                # rocprofv3 --pmc passes over `bench.py --no-graph` (tools/engine_traffic.sh -> profiles/engine_traffic.json); PMC
                 # collection needs its own profiled runs, so it cannot happen inside this timed invocation: the value is static --
                 # and only quoted while the GEMM sources still hash to what was measured (a stale file reports null)
                 tj = json.load(open(os.path.join(ROOT, "profiles", TRAFFIC_FILE))).get(args.workload)
