@@ -1551,11 +1551,12 @@ __global__ __launch_bounds__(1024) void hy_scan_kernel(ScanParams p) {
 // Error against a 64-bit walk, root mean square over that of the result, 2048 tokens of 16 heads, here / token by token: outputs GLA 3.17e-7 / 3.47e-7 (tau 16, z 3 +- 2), 1.14e-7 / 1.20e-7
 // (z 0 +- 2), 7.55e-8 / 8.46e-8 (z -10 +- 6), 8.77e-8 / 9.28e-8 (tau 1, z 2 +- 2), HGRN2 1.124e-7 / 1.128e-7, constant decays 1.09e-7 / 1.27e-7; states 3.14e-7 / 3.44e-7, 9.52e-8 / 1.00e-7,
 // 4.02e-8 / 4.51e-8, 5.79e-8 / 5.98e-8, 2.50e-7 / 2.52e-7, 0.80e-7 / 1.07e-7.
-// sigmoid(z)^(1 / tau).  From tau = 16 on log(1 + e^-|z|) by the vector unit's exponential and logarithm, with what 1 + e^-|z| rounds off put back: they leave about 2^-24 on it, which tau
+// sigmoid(z)^(1 / tau).  From tau = 4 on log(1 + e^-|z|) by the vector unit's exponential and logarithm, with what 1 + e^-|z| rounds off put back: they leave about 2^-24 on it, which tau
 // divides; the quotient is corrected to a division's and the outer exponential is expf, so that the error is that of the plain form (root mean square, tau 16, z in (-2, 2) 1.87e-8 both,
-// (-10, 0) 2.72e-8 both, (-90, -30) 2.64e-8 both) in a quarter of its operations.  Smaller tau: the plain form (tau 4, z in (0, 8) 1.847e-8 against 1.854e-8).
+// (-10, 0) 2.72e-8 both, (-90, -30) 2.64e-8 both; at most 0.4 % more: tau 4, z in (0, 8) 1.854e-8 against 1.847e-8) in a quarter of its operations.  Smaller tau: the plain form (tau 1, z in
+// (-2, 2) 3.84e-8 against 4.05e-8).
 __device__ __forceinline__ float hy_gla_decay(float z, float tau, float itau) {
-    if (!(tau >= 16.f && tau <= 1e6f)) return expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) / tau);
+    if (!(tau >= 4.f && tau <= 1e6f)) return expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) / tau);
     const float u = __builtin_amdgcn_exp2f(-fabsf(z) * 1.44269504f), w = 1.f + u, c = u - (w - 1.f);
     const float l = __builtin_fmaf(__builtin_amdgcn_logf(w), 0.69314718f, c * __builtin_amdgcn_rcpf(w));        // v_log_f32: base 2
     const float n = fmaxf(fminf(z, 0.f), -1e30f) - l, q = n * itau;                                             // -inf would leave inf - inf in the correction
