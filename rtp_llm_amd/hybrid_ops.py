@@ -526,16 +526,17 @@ def tiles_form(T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int
     return best if margin * us < scan_us else None
 
 
-def scan_form(mode: int, T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int) -> Optional[int]:
+def scan_form(mode: int, T: int, nseq: int, max_rows: int, heads: int, dim: int, vdim: int, tau: float = 16.0) -> Optional[int]:
     """How `scan` runs keys of up to WALK_MAX_DIM channels when the choice is its own: hy_walk over chunks of the size returned, hy_walk whole (0) or hy_scan (None).  Gated recurrences
     that gated_form answers keep its form: over 112 such calls it is 4 % off the fastest on the GPU in the mean, at most half as much again, and takes 0.36 of hy_scan's time (at most
     0.83).  tiles_form, which counts the host's time for chunks as well, would leave half of them (most of the 112 are calls where the two differ) whole or to hy_scan, at up to 2.6
-    times the time on the GPU.  The rest is tiles_form's, HGRN2 with a wider margin: hy_scan is 10 % faster there, the tiles with their 64-bit sums up to 15 % slower."""
+    times the time on the GPU.  The rest is tiles_form's, HGRN2 with a wider margin: hy_scan is 10 % faster there, the tiles with their 64-bit sums up to 15 % slower.  So for decays of tau below 4, whose
+    plain form costs the tiles a quarter (of 140 such calls 12 lost up to 18 % to hy_scan without: 8 sequences of up to 59 rows, 8 heads of 96 x 256 32 / 38 us; none with)."""
     fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
     if fixed and max_rows <= FIXED_TILES_FROM:
         return None
     C = None if fixed else gated_form(T, nseq, max_rows, heads, dim, vdim)
-    return tiles_form(T, nseq, max_rows, heads, dim, vdim, 1.35 if mode == SCAN_HGRN2 else 1.05) if C is None else C
+    return tiles_form(T, nseq, max_rows, heads, dim, vdim, 1.35 if mode == SCAN_HGRN2 or (mode == SCAN_GLA and tau < 4) else 1.05) if C is None else C
 
 
 def scan_prefers_chunks(T: int, nseq: int, max_rows: int, heads: int, vdim: int, C: int) -> bool:
@@ -585,7 +586,7 @@ def scan(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, z: Optional[t
                                           act_code(act), _stream()), "hy_scan")
 
     fixed = mode in (SCAN_FIXED, SCAN_FIXED_SILU)
-    C = scan_form(mode, T, nseq, max_rows, heads, dim, vdim) if chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim) else None
+    C = scan_form(mode, T, nseq, max_rows, heads, dim, vdim, tau) if chunked is None and dim <= WALK_MAX_DIM and state.is_contiguous() and state.shape[1:] == (heads, dim, vdim) else None
     if C is not None:
         def walk(rs, sl, fp, n, st, dst, cdecay, keep):
             _C.check_hybrid(lib.mi355_hy_walk(mode, proj.data_ptr(), ld, qo, ko, vo, _p(z), 0 if z is None else _rows(z, "scan.z"), _p(lower), _p(fbias), float(tau),

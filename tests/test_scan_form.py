@@ -85,3 +85,11 @@ def test_unknown_longest():
     """max_rows 0: the longest is taken to be what the other sequences leave, a constant decay keeps hy_scan."""
     assert hops.scan_form(FIXED, 4096, 1, 0, 8, 64, 128) is None
     assert hops.scan_form(GLA, 4096, 1, 0, 8, 64, 128) == hops.scan_form(GLA, 4096, 1, 4096, 8, 64, 128)
+
+
+@pytest.mark.parametrize("call,scan,walk", [((350, 8, 59, 8, 96, 256), 32.2, 38.0), ((171, 4, 65, 8, 64, 64), 26.0, 28.7), ((706, 16, 82, 8, 128, 128), 48.2, 53.4),
+                                            ((1815, 16, 176, 16, 128, 192), 267.9, 103.0)])
+def test_small_tau(call, scan, walk):
+    """Decays of tau 1 cost the tiles more (the last is of tau 16, far from the line)."""
+    C = hops.scan_form(GLA, *call, tau=1.0)
+    assert C == (0 if walk < scan else None)
