@@ -1547,7 +1547,7 @@ __global__ __launch_bounds__(1024) void hy_scan_kernel(ScanParams p) {
 // 16 heads of 64 x 128, four sequences of 2048 tokens in chunks of 128: states 106.7 -> 48 us, outputs 136.5 -> 97 (HGRN2 44 and 110); one sequence of 1537, 8 heads, chunks of 32: all 60.5 -> 42 us.
 // A block alone takes 4 us a tile, of which 2304 cycles are products; the rest is its chain of two barriers, LDS and exponentials, which four blocks of a compute unit hide (128
 // registers; HGRN2's outputs three).  Products of decays are formed in 64 bits (a constant decay's powers would carry one rounding from tile to tile), sums as short chains and trees,
-// P's tree over the lanes in 64 bits under gates.
+// P's tree over the lanes in 64 bits under gates (GLA: of up to 64 channels; the token walk's chains over more of them round more, and so may the tree: 0.87 to 0.97 of its error).
 // Error against a 64-bit walk, root mean square over that of the result, 2048 tokens of 16 heads, here / token by token: outputs GLA 3.17e-7 / 3.47e-7 (tau 16, z 3 +- 2), 1.14e-7 / 1.20e-7
 // (z 0 +- 2), 7.55e-8 / 8.46e-8 (z -10 +- 6), 8.77e-8 / 9.28e-8 (tau 1, z 2 +- 2), HGRN2 1.124e-7 / 1.128e-7, constant decays 1.09e-7 / 1.27e-7; states 3.14e-7 / 3.44e-7, 9.52e-8 / 1.00e-7,
 // 4.02e-8 / 4.51e-8, 5.79e-8 / 5.98e-8, 2.50e-7 / 2.52e-7, 0.80e-7 / 1.07e-7.
@@ -1724,7 +1724,7 @@ __global__ __launch_bounds__(256, CH > 1 ? 2 : OUT && MODE == SCAN_HGRN2 ? 3 : 4
                     }
             }
             const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
-            using Sum = std::conditional_t<LOW || MODE == SCAN_GLA, double, float>;
+            using Sum = std::conditional_t<LOW || (MODE == SCAN_GLA && CH == 1), double, float>;
             float p8[8];
             Sum p4[4], p2[2];
 #pragma unroll
