@@ -586,7 +586,11 @@ int launch_gemm_bf16_t(const GemmParams& p, int cfg, hipStream_t st) {
 // in flight as a block has, up to 8 of 4 KB a wave (4 from 17 rows on).  The same sums: a wave's tiles and chunks are what they were.  One step of the 0.5B model, us before / now:
 // 1 row 845 / 751, 12 (bf16) 921 / 896, 20 1155 / 949, 32 (bf16) 1186 / 974, 40 1651 / 1108, 64 1875 / 1288, 64 (bf16) 1598 / 1242; with four waves everywhere 1 row 773, 64 rows 1327.
 // Shapes that fill the chip stay: the 7B model with 16-bit weights, these everywhere / the others, 1 row 3259 / 3100, 16 (bf16) 3621 / 3463, 40 4158 / 3978, 64 4453 / 4340, 64 (bf16)
-// 4474 / 4291; only from 17 to 32 rows 24 rows 3748 / 3851, with lm_heads (1187 blocks of 128 columns) the other way: 0.5B, 18 rows 53.4 / 49.0, 7B, 30 rows 189.8 / 185.7.
+// 4474 / 4291; lm_heads of 17 to 32 rows (1187 blocks of 128 columns) 0.5B, 18 rows 53.4 / 49.0, 7B, 30 rows 189.8 / 185.7.
+// From 17 to 32 rows by how the blocks of 128 columns fill the chip: half as wide ones even it out where the last round has at most 128 (214 random linears, cold weights, time over the
+// others': 0.82 for up to 128 blocks, 0.95 for 257 to 384) and only add blocks where it has more (1.05 for 129 to 256, 1.06 for 385 to 512, up to 22.0 -> 25.0 us).  With two chunks a
+// block the 129 to 256 cost nothing (1.02 cold, 0.97 warm; a step of the 0.5B model, 24 rows, down_proj of 133 blocks, 930 without them / 921).  A step of the 7B model, the others / these
+// up to 512 blocks / this rule: 18 rows 3601 / 3511 / 3412, 24 (bf16) 3705 / 3615 / 3535.
 template <int MB, int NWN, bool BF>
 void launch_gemm_w16_t(const GemmParams& p, hipStream_t st) {
     const dim3 grid(cdiv(p.NT, NWN), p.nsplit), block(64 * NWN);
@@ -606,7 +610,7 @@ int launch_gemm(const GemmParams& p, int wbits, int group_size, int cfg, hipStre
     if (wbits == 16) {
         const int blocks = cdiv(p.NT * 16, kCfgBN[cfg]) * p.nsplit;
         if (cfg == 5 && blocks <= 256) return p.bf16 ? launch_gemm_w16<1, true>(p, st) : launch_gemm_w16<1, false>(p, st);
-        if (cfg == 2 && blocks <= 512) return p.bf16 ? launch_gemm_w16<2, true>(p, st) : launch_gemm_w16<2, false>(p, st);
+        if (cfg == 2 && (blocks <= (p.cps <= 2 ? 256 : 128) || (blocks > 256 && blocks <= 384))) return p.bf16 ? launch_gemm_w16<2, true>(p, st) : launch_gemm_w16<2, false>(p, st);
         if ((cfg == 4 || cfg == 6 || cfg == 8) && blocks <= 96) return p.bf16 ? launch_gemm_w16<4, true>(p, st) : launch_gemm_w16<4, false>(p, st);
     }
     if (p.bf16) {

@@ -11,7 +11,8 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 48, 64])
-@pytest.mark.parametrize("K,N", [(64, 16), (128, 48), (896, 1152), (896, 9728), (640, 33 * 16), (1152, 8 * 16), (4864, 896), (1024, 20000)])
+@pytest.mark.parametrize("K,N", [(64, 16), (128, 48), (896, 1152), (896, 9728), (640, 33 * 16), (1152, 8 * 16), (4864, 896), (1024, 20000), (440, 16384), (312, 17256),
+                                 (4864, 1800), (624, 17160), (1184, 8480), (1848, 11208)])
 def test_few_rows_of_16_bit_weights(M, K, N, dtype):
     g = torch.Generator(device=DEV).manual_seed(K + N + M)
     x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
