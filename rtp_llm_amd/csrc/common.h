@@ -61,6 +61,10 @@ __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const void* b
 __device__ __forceinline__ void dma16(uint32_t lds, const void* src) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(src) : "memory", "m0");
 }
+// the same for bytes that are read once: not kept in the caches
+__device__ __forceinline__ void dma16_nt(uint32_t lds, uint32_t voff, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
 // until at most VM of the wave's vector-memory operations (such loads among them) and none of its LDS operations are left.  A builtin, not asm: the compiler's own
 // counting sees it.
 template <int VM> __device__ __forceinline__ void wait_vm() {

@@ -6,8 +6,7 @@
 //   * tile kernels, bf16: block tiles of 64 x 128 up to 256 x 256, both operands through LDS by DMA, MFMA 16x16x32; one that stages 64 x 128 through registers
 //     for operands without 16-byte alignment;
 //   * tile kernel, fp32:  64 x 64 block tile, 4 x 4 register micro-tiles, true fp32 FMAs (no reduced-precision matrix mode);
-//   * skinny kernel, bf16, 2 <= M <= 16: one block per 16 outputs (8 of few outputs and rows, with the same partial sums), its waves split K, MFMA fragments loaded
-//     straight from memory;
+//   * skinny kernel, bf16, 2 <= M <= 16: one block per 8 weight rows, its waves split K, both operands through LDS in runs of 1 KB a row;
 //   * row kernel (M = 1; fp32 up to M = 16): a wave per output column streams its weight row once, 16-byte loads, wave reduction at the end.
 //   * grouped forms of these kernels (per-head or per-branch weights over column slices; rows sorted by expert with a gather and a tile
 //     list; the few rows of a decode step, each with its own expert's weight): mi355_dense_grouped.
@@ -686,35 +685,133 @@ void launch_rows(const DenseParams& p, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------------------------------------ skinny kernel (bf16, M <= 16)
-// One block per 16 outputs; its NW waves split K in interleaved steps of 32 and each wave runs MFMA 16x16x32 with the (up to) 16 rows of x as
-// the A operand and 16 weight rows as B, both fragments loaded straight from memory (8 consecutive k per lane, no LDS staging).  The weight
-// stream is read once whatever M is; the waves' partial tiles are summed through LDS.  Under GATED a tile is 16 channels: their gate rows and
-// their up rows share the A fragments.
-// HALF (M <= 8): 8 outputs per block and half the waves, each with the k-steps of two of them: rows 0 to 7 of the first operand are x in the steps of wave w, rows 8 to 15 x in
-// those of wave w + NW, the second operand likewise.  Of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are what the two waves would hold, the rest is not used;
-// the partial sums and their order are those of 16 outputs, a row's bits do not depend on how many rows (2 to 16) there are.
-// The tile's block bx of group grp; the first NW of the block's waves take part.  Whole block.
-typedef f32x4 SkinnySums[8][2][64];
-template <bool GATED, bool HALF>
-__device__ __forceinline__ void dense_skinny_tile(const DenseParams& p, int bx, int grp, int NW, int mbase, SkinnySums& red) {
-    constexpr int NO = HALF ? 8 : 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nout = GATED ? p.N / 2 : p.N;
-    const int r = lane & (NO - 1), chains = HALF ? 2 * NW : NW, kq = (lane >> 4) * 8 + (HALF && (lane & 8) ? NW * 32 : 0);
-    const int o = min(bx * NO + r, nout - 1);
-    const int n = GATED ? (o >> 5) * 64 + (o & 31) : o;
+// One block of four waves per 8 weight rows: 8 outputs, or the gate and up rows of 4 channels.  What bounds it is how the weight comes out of memory: 8 rows of a row-major weight
+// lie side by side, and read as MFMA fragments (16 rows by 64 bytes a wave load) they came at 3.2 TB/s however the steps were ordered.  Here every wave load is one
+// row's run of 1 KB, by DMA into LDS, three stages of 512 columns; the rows of x beside them the same way, so that nothing but the fragments passes through registers.  8 weight rows a
+// block and 48 KB (M <= 8): three blocks a compute unit, 96 KB of loads in flight.  More rows a block, more waves, more or fewer stages and narrower runs are all slower.
+// Weights from memory, M = 8, us before / now: 17408 x 2048 22.4 / 14.4, 32000 x 2048 35.1 / 24.3, 4096 x 2048 7.5 / 5.2, 2048 x 5632 13.6 / 6.5, 2048 x 2048 5.4 / 3.6.
+// Sums: k in steps of 32, step s into chain s mod skinny_chains (4 or 8), the chains added in order: bits that depend on N, K and G only.
+// 16-byte pieces are permuted by the row (applied to the source address), so that the 8 or 16 rows of a fragment read hit different banks.
+constexpr int SK_RB = 8;
+template <int XR_, int KC_, int NS_> struct SkinnyForm {                      // rows of x that are staged (M <= XR), columns of a stage, stages
+    static constexpr int XR = XR_, KC = KC_, NS = NS_, STAGE = (SK_RB + XR) * KC * 2, BYTES = NS * STAGE;
+};
+
+// The weight rows bx * 8 .. of group grp.  NCH: chains.  NT: the weight is not kept in the caches.  Whole block of 256.
+template <class F, int NCH, bool NT>
+__device__ __forceinline__ void dense_skinny_tile(const DenseParams& p, int bx, int grp, char* smem) {
+    constexpr int XR = F::XR, KC = F::KC, NS = F::NS, STAGE = F::STAGE, RB = KC * 2, NW = 4, PPR = KC / 8;   // PPR: 16-byte pieces of a row
+    constexpr int LW = SK_RB * PPR / (64 * NW), LX = XR * PPR / (64 * NW), LD = LW + LX;                                   // loads per wave and stage
+    static_assert((NCH == 4 || NCH == 8) && LX * 64 * NW == XR * PPR, "a wave adds one or two chains; whole wave loads");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem);
+    const int no = p.gated ? SK_RB / 2 : SK_RB, nout = p.gated ? p.N / 2 : p.N, o0 = bx * no;   // the block's outputs
+    const bf16* X = (const bf16*)p.x + p.xs * grp;
+    // gated: rows 0 to 3 are the gates of channels o0 .., 4 to 7 their up rows, 32 further on; a row past the end repeats the last one and is not stored
+    const int first = p.gated ? (o0 >> 5) * 64 + (o0 & 31) : o0;
+    const bf16* W = (const bf16*)p.w + p.ws * grp + (size_t)first * p.K;
+    uint32_t row[LD], pc[LD];                                              // byte offset of the lane's row, its piece of it
+#pragma unroll
+    for (int u = 0; u < LD; ++u) {
+        const int at = ((u < LW ? u : u - LW) * NW + wave) * 64 + lane, r = at / PPR;
+        if (u < LW) row[u] = (uint32_t)(p.gated ? (r & 3) + (r >> 2) * 32 : min(r, nout - 1 - o0)) * (uint32_t)p.K * 2u;
+        else        row[u] = (uint32_t)min(r, p.M - 1) * (uint32_t)p.ldx * 2u;
+        pc[u] = (at % PPR) ^ (r & 15);
+    }
+    auto issue = [&](int buf, int c) {
+        const uint32_t last = (uint32_t)min(KC, p.K - c * KC) / 8 - 1;  // pieces past the end of K repeat the last one
+#pragma unroll
+        for (int u = 0; u < LD; ++u) {
+            const uint32_t to = lds0 + buf * STAGE + (u < LW ? 0 : SK_RB * RB) + ((u < LW ? u : u - LW) * NW + wave) * 1024, from = row[u] + min(pc[u], last) * 16u;
+            if (u < LW && NT) dma16_nt(to, from, W + c * KC);
+            else              dma16(to, from, (u < LW ? W : X) + c * KC);
+        }
+    };
+    const int nc = (p.K + KC - 1) / KC, fr = lane & 15, q = lane >> 4, wr = fr & (SK_RB - 1), xr = fr & (XR - 1);
+    f32x4 acc[NCH / 4];
+#pragma unroll
+    for (int i = 0; i < NCH / 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NS - 1; ++c) if (c < nc) issue(c, c);
+    int at = 0;
+    for (int c = 0; c < nc; ++c) {
+        if (c + NS - 2 < nc) wait_vm<LD * (NS - 2)>(); else wait_vm<0>();    // this wave's part of the columns is in LDS, its reads of the stage before are done
+        __builtin_amdgcn_s_barrier();
+        if (c + NS - 1 < nc) issue(at == 0 ? NS - 1 : at - 1, c + NS - 1);
+        const char* wb = smem + at * STAGE + wr * RB;
+        const char* xb = smem + at * STAGE + (SK_RB + xr) * RB;
+        auto step = [&](int s, bool tail) {                                   // the wave's step s of the stage
+            const int piece = (s * NW + wave) * 4 + q;
+            bf16x8 b = *(const bf16x8*)(wb + ((piece ^ wr) << 4)), a = *(const bf16x8*)(xb + ((piece ^ xr) << 4));
+            if (tail && c * KC + piece * 8 >= p.K) { a = bf16x8{}; b = bf16x8{}; }
+            acc[NCH == 8 ? s & 1 : 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[NCH == 8 ? s & 1 : 0], 0, 0, 0);
+        };
+        if ((c + 1) * KC <= p.K) {
+#pragma unroll
+            for (int s = 0; s < KC / 32 / NW; ++s) step(s, false);
+        } else {
+#pragma unroll
+            for (int s = 0; s < KC / 32 / NW; ++s) if (c * KC + (s * NW + wave) * 32 < p.K) step(s, true);
+        }
+        at = at + 1 == NS ? 0 : at + 1;
+    }
+    // the chains meet in a stage that no wave reads any more: not the last one's, and behind its barrier all others are done with
+    f32x4* red = (f32x4*)(smem + (at + 1 == NS ? 0 : at + 1) * STAGE);
+    static_assert(NCH * 64 * 16 <= STAGE && NS >= 3, "room for the chains beside the stage that is still read");
+#pragma unroll
+    for (int i = 0; i < NCH / 4; ++i) red[(i * 4 + wave) * 64 + lane] = acc[i];
+    __syncthreads();
+    // C fragment: lane holds weight row (lane & 15), rows 4 * (lane >> 4) + e of x; wave e takes the rows of its e
+    if (fr >= no || o0 + fr >= nout) return;
+    const int m = q * 4 + wave, oc = o0 + fr;
+    if (m >= p.M) return;
+    const float* mine = (const float*)(red + lane) + wave;
+    float g = mine[0], v = p.gated ? mine[16] : 0.f;                          // the up row's lane is four on
+#pragma unroll
+    for (int i = 1; i < NCH; ++i) {
+        g += mine[i * 256];
+        if (p.gated) v += mine[i * 256 + 16];
+    }
+    if (p.bias) { const bf16* Bi = (const bf16*)p.bias + (size_t)grp * p.N + first + fr; g += dn_ld(Bi); if (p.gated) v += dn_ld(Bi + 32); }
+    dn_store<bf16>(p, m, (int)(p.ys * grp) + oc, p.gated ? dn_gated(g, v, p.act, p.act_param) : dn_act(g, p.act));
+}
+
+template <class F, int NCH, bool NT>
+__global__ __launch_bounds__(256) void dense_skinny_bf16_kernel(DenseParams p) {
+    __shared__ __attribute__((aligned(1024))) char smem[F::BYTES];
+    dense_skinny_tile<F, NCH, NT>(p, blockIdx.x, blockIdx.y, smem);
+}
+
+// Two of them in one launch, the second's blocks behind the first's: a launch of few rows costs 2 to 3 us whatever it reads, and the weights of the two keep each other's compute
+// units busy.  Chains as in a launch of its own, so that the bits are the same.
+template <class F, bool NT>
+__global__ __launch_bounds__(256) void dense_skinny_pair_kernel(DenseParams p0, DenseParams p1, int blocks0, int chains0, int chains1) {
+    __shared__ __attribute__((aligned(1024))) char smem[F::BYTES];
+    const int b = blockIdx.x;
+    if (b < blocks0) {
+        if (chains0 == 8) dense_skinny_tile<F, 8, NT>(p0, b, 0, smem); else dense_skinny_tile<F, 4, NT>(p0, b, 0, smem);
+    } else {
+        if (chains1 == 8) dense_skinny_tile<F, 8, NT>(p1, b - blocks0, 0, smem); else dense_skinny_tile<F, 4, NT>(p1, b - blocks0, 0, smem);
+    }
+}
+
+// Short K through many outputs: a block of 8 weight rows would end before it has begun, so 16 outputs a block, fragments straight from memory, the four waves a chain each: the same sums.
+typedef f32x4 SkinnySums[4][2][64];
+template <bool GATED>
+__device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, int bx, int grp, SkinnySums& red) {
+    constexpr int NW = 4, U = 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nout = GATED ? p.N / 2 : p.N;
+    const int r = lane & 15, kq = (lane >> 4) * 8, o = min(bx * 16 + r, nout - 1), n = GATED ? (o >> 5) * 64 + (o & 31) : o;
     const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kq;
     const bf16* wu = wg + (size_t)32 * p.K;
-    const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(mbase + r, p.M - 1) * p.ldx + kq;
+    const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(r, p.M - 1) * p.ldx + kq;
     f32x4 ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
     const bf16x8 zero = {};
-    constexpr int U = HALF ? 8 : 4;                          // steps in flight: the same bytes per compute unit in both forms
-    const int stride = chains * 32;
-    for (int k0 = wave < NW ? wave * 32 : p.K; k0 < p.K; k0 += U * stride) {
+    for (int k0 = wave * 32; k0 < p.K; k0 += U * NW * 32) {
         bf16x8 a[U], b[U], c[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = k0 + u * stride;
+            const int k = k0 + u * NW * 32;
             const bool ok = k + kq < p.K;
             a[u] = ok ? *(const bf16x8*)(xr + k) : zero;
             b[u] = ok ? *(const bf16x8*)(wg + k) : zero;
@@ -734,64 +831,85 @@ __device__ __forceinline__ void dense_skinny_tile(const DenseParams& p, int bx, 
         ag += red[w][0][lane];
         if (GATED) au += red[w][1][lane];
     }
-    // C fragment: lane holds output (lane & 15), rows 4 * (lane >> 4) + e; HALF: the second wave's sum of (output, row) lies at (output + 8, row + 8), 40 lanes on
-    if constexpr (HALF) {
-        if ((lane & 8) || lane >= 32) return;
-        for (int w = 0; w < NW; ++w) {
-            ag += red[w][0][lane + 40];
-            if (GATED) au += red[w][1][lane + 40];
-        }
-    }
-    const int oc = bx * NO + r;
-    if (oc >= nout) return;
-    const int nb = GATED ? (oc >> 5) * 64 + (oc & 31) : oc;
+    if (bx * 16 + r >= nout) return;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const int row = mbase + (lane >> 4) * 4 + e;
+        const int row = (lane >> 4) * 4 + e;
         if (row >= p.M) continue;
         float g = ag[e], u = au[e];
-        if (p.bias) { const bf16* Bi = (const bf16*)p.bias + (size_t)grp * p.N; g += dn_ld(Bi + nb); if (GATED) u += dn_ld(Bi + nb + 32); }
-        dn_store<bf16>(p, row, (int)(p.ys * grp) + oc, GATED ? dn_gated(g, u, p.act, p.act_param) : dn_act(g, p.act));
+        if (p.bias) { const bf16* Bi = (const bf16*)p.bias + (size_t)grp * p.N; g += dn_ld(Bi + n); if (GATED) u += dn_ld(Bi + n + 32); }
+        dn_store<bf16>(p, row, (int)(p.ys * grp) + bx * 16 + r, GATED ? dn_gated(g, u, p.act, p.act_param) : dn_act(g, p.act));
     }
 }
-
-template <bool GATED, bool HALF>
-__global__ __launch_bounds__(512) void dense_skinny_bf16_kernel(DenseParams p, int mbase) {
+template <bool GATED>
+__global__ __launch_bounds__(256) void dense_skinny_short_kernel(DenseParams p) {
     __shared__ SkinnySums red;
-    dense_skinny_tile<GATED, HALF>(p, blockIdx.x, blockIdx.y, blockDim.x >> 6, mbase, red);
+    dense_skinny_short_tile<GATED>(p, blockIdx.x, blockIdx.y, red);
 }
-
-// Two of them in one launch, the second's blocks behind the first's: a launch of few rows costs 4 to 5 us whatever it reads, and the weights of the two keep each other's compute
-// units busy.  NW: the waves that each takes, as in a launch of its own, so that the bits are the same.
-template <bool HALF>
-__global__ __launch_bounds__(512) void dense_skinny_pair_kernel(DenseParams p0, DenseParams p1, int blocks0, int nw0, int nw1) {
+template <bool GATED0, bool GATED1>
+__global__ __launch_bounds__(256) void dense_skinny_short_pair_kernel(DenseParams p0, DenseParams p1, int blocks0) {
     __shared__ SkinnySums red;
-    if ((int)blockIdx.x < blocks0) {
-        if (p0.gated) dense_skinny_tile<true, HALF>(p0, blockIdx.x, 0, nw0, 0, red);
-        else          dense_skinny_tile<false, HALF>(p0, blockIdx.x, 0, nw0, 0, red);
-    } else {
-        if (p1.gated) dense_skinny_tile<true, HALF>(p1, blockIdx.x - blocks0, 0, nw1, 0, red);
-        else          dense_skinny_tile<false, HALF>(p1, blockIdx.x - blocks0, 0, nw1, 0, red);
-    }
+    if ((int)blockIdx.x < blocks0) dense_skinny_short_tile<GATED0>(p0, blockIdx.x, 0, red);
+    else                           dense_skinny_short_tile<GATED1>(p1, blockIdx.x - blocks0, 0, red);
 }
+// us in the form above / in this one: 16 x 6720 gated x 872 7.2 / 6.4, 8 x 8706 x 584 5.6 / 5.2, 12 x 13952 x 232 6.3 / 4.2, two groups of 2519 x 80 3.1 / 2.9; below the line 9 x 3648 gated x 64
+// 3.2 / 3.3, 8 x 3090 x 344 3.9 / 3.8.
+bool skinny_short(int K, long long weight_rows) { return K < 1024 && weight_rows > 4096; }
 
-// M of 2 to 16, p.vec.  Few outputs (blocks of 8 still one for every compute unit): 8 per block where M allows it, so that all compute units pull weights; narrow outputs:
-// more waves per tile keep the memory system busy.  M = 8, weights from memory, us with 16 / 8 outputs: 2048 x 5632 12.8 / 10.7, 2048 x 2048 6.4 / 5.5, 16 x 2048 5.3 / 4.4,
-// 1024 x 1024 4.8 / 4.4; past the line, where some compute units get a second block: 2176 x 2048 6.3 / 7.1, 2560 x 5632 13.5 / 15.4, gated 2304 x 1024 6.3 / 6.9;
-// short K, of which a wave has a step or two: 1536 x 512 3.9 / 3.7, 48 x 192 2.6 / 3.0, gated 512 x 152 2.8 / 3.3.
-// The partial sums that K is split into.
-int skinny_chains(const DenseParams& p, int tiles) { return tiles * p.G >= 1024 || p.K < 1024 ? 4 : 8; }
+// The partial sums that K is split into (part of a result's bits): eight, four of many outputs or short K.
+int skinny_chains(const DenseParams& p) { return (((p.gated ? p.N / 2 : p.N) + 15) / 16) * p.G >= 1024 || p.K < 1024 ? 4 : 8; }
+int skinny_blocks(const DenseParams& p) { return (p.N + SK_RB - 1) / SK_RB; }
+// A weight that one launch reads 24 MB or more of belongs to a layer, and so to a model, that the 256 MB memory-side cache does not hold from one step to the next: it is read past the caches.
+// Weights from memory, us without / with the hint: 17408 x 2048 15.5 / 14.4, 32000 x 2048 26.5 / 24.3; in 128 MB that are read again and again 12.0 / 13.4, 19.7 / 23.0.
+bool skinny_nt(size_t weights) { return weights * 2 >= (size_t)24 << 20; }
+
+// launch(form) with the form for M rows of K columns (the shorter of two) in `blocks` blocks.  As few rows of x staged as there are: they come from the L2, but pass through the same loads
+// as the weights (32000 x 2048 with 4 / 8 / 16: 21.2 / 24.3 / 28.6 us).  Stages of half the columns, and so more blocks a compute unit, for short K, of which a stage of 512 would be
+// mostly empty, and for 9 to 16 rows in many blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2).  Stages of twice the columns, half the barriers, where no compute unit
+// has a second block to hide them (2 rows, 384 x 5960, six stages of 512 / three of 1024: 7.1 / 6.3).
+template <class L>
+void skinny_form(int M, int K, long long blocks, L&& launch) {
+    auto rows = [&](auto kc, auto ns) {
+        constexpr int KC = decltype(kc)::value, NS = decltype(ns)::value;
+        if (M > 8) launch(SkinnyForm<16, KC, NS>{});
+        else if (M > 4 || KC < 512) launch(SkinnyForm<8, KC, NS>{});
+        else if constexpr (KC >= 512) launch(SkinnyForm<4, KC, NS>{});
+    };
+    if (K < 1024 || (M > 8 && blocks >= 1024)) rows(std::integral_constant<int, 256>{}, std::integral_constant<int, 4>{});
+    else if (blocks <= 256)                    rows(std::integral_constant<int, 1024>{}, std::integral_constant<int, 3>{});
+    else                                       rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 3>{});
+}
+// M of 2 to 16, p.vec
 void launch_skinny(const DenseParams& p, hipStream_t st) {
-    const int nout = p.gated ? p.N / 2 : p.N, tiles = (nout + 15) / 16;
-    if (p.M <= 8 && p.K >= 512 && tiles * p.G <= 128) {
-        const dim3 grid((nout + 7) / 8, p.G), block(p.K < 1024 ? 128 : 256);
-        if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, true>), grid, block, 0, st, p, 0);
-        else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, true>), grid, block, 0, st, p, 0);
+    if (skinny_short(p.K, (long long)p.N * p.G)) {
+        const int b = ((p.gated ? p.N / 2 : p.N) + 15) / 16;
+        if (p.gated) hipLaunchKernelGGL(dense_skinny_short_kernel<true>, dim3(b, p.G), dim3(256), 0, st, p);
+        else         hipLaunchKernelGGL(dense_skinny_short_kernel<false>, dim3(b, p.G), dim3(256), 0, st, p);
         return;
     }
-    const dim3 grid(tiles, p.G), block(64 * skinny_chains(p, tiles));
-    if (p.gated) hipLaunchKernelGGL((dense_skinny_bf16_kernel<true, false>), grid, block, 0, st, p, 0);
-    else         hipLaunchKernelGGL((dense_skinny_bf16_kernel<false, false>), grid, block, 0, st, p, 0);
+    const dim3 grid(skinny_blocks(p), p.G), block(256);
+    const bool nt = skinny_nt((size_t)p.N * p.K * p.G), eight = skinny_chains(p) == 8;
+    skinny_form(p.M, p.K, (long long)grid.x * grid.y, [&](auto f) {
+        using F = decltype(f);
+        if (eight) { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, false>), grid, block, 0, st, p); }
+        else       { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, false>), grid, block, 0, st, p); }
+    });
+}
+void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
+    if (skinny_short(p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N)) {
+        const int s0 = ((p[0].gated ? p[0].N / 2 : p[0].N) + 15) / 16, s1 = ((p[1].gated ? p[1].N / 2 : p[1].N) + 15) / 16;
+        const dim3 grid(s0 + s1), block(256);
+        if (p[0].gated) { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, true>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, false>), grid, block, 0, st, p[0], p[1], s0); }
+        else            { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, true>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, false>), grid, block, 0, st, p[0], p[1], s0); }
+        return;
+    }
+    const int b0 = skinny_blocks(p[0]), b1 = skinny_blocks(p[1]), c0 = skinny_chains(p[0]), c1 = skinny_chains(p[1]);
+    const bool nt = skinny_nt((size_t)p[0].N * p[0].K + (size_t)p[1].N * p[1].K);
+    skinny_form(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K < p[1].K ? p[0].K : p[1].K, (long long)b0 + b1, [&](auto f) {
+        using F = decltype(f);
+        if (nt) hipLaunchKernelGGL((dense_skinny_pair_kernel<F, true>), dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, c0, c1);
+        else    hipLaunchKernelGGL((dense_skinny_pair_kernel<F, false>), dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, c0, c1);
+    });
 }
 
 } // namespace
@@ -853,7 +971,6 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
 extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream_t stream) {
     MI355_CHECK_ARG(a, "dense_linear_pair: null arguments");
     DenseParams p[2];
-    int tiles[2], nw[2];
     for (int i = 0; i < 2; ++i) {
         const mi355_dense_args_t& d = a[i];
         MI355_CHECK_ARG(d.x && d.w && d.y && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && (!d.gated || d.N % 64 == 0) && d.ldy >= (d.gated ? d.N / 2 : d.N) && d.act >= 0 &&
@@ -865,19 +982,9 @@ extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream
         q.gated = d.gated; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
         q.yvec = (d.ldy % 4 == 0) && ((uintptr_t)d.y % (d.out_f32 ? 16 : 8) == 0);
         q.G = 1; q.xs = q.ws = q.ys = 0; q.offs = nullptr; q.gather = nullptr; q.tiles = nullptr; q.egate = nullptr; q.ldg = q.goff = 0;
-        tiles[i] = ((d.gated ? d.N / 2 : d.N) + 15) / 16;
-        nw[i] = skinny_chains(q, tiles[i]);
     }
     hipStream_t st = (hipStream_t)stream;
-    // 8 outputs a block where both together leave a compute unit two of them.  M = 8, weights from memory, us of 16 outputs a block / 8: 1024 x 1024 + 1024 x 2816 7.4 / 6.4,
-    // 2048 x 2048 + 2048 x 5632 12.9 / 11.9, 3072 x 2048 + 1024 x 2048 6.6 / 7.2; past the line 2560 x 2560 + 2560 x 6912 20.7 / 22.4, 6160 x 2048 + gated 11264 x 2048 21.0 / 22.5
-    // (in two launches the second takes 5.2 + 9.9, the last 10.4 + 16.6).
-    if (p[0].M <= 8 && p[1].M <= 8 && p[0].K >= 512 && p[1].K >= 512 && tiles[0] + tiles[1] <= 256) {
-        const int b0 = ((p[0].gated ? p[0].N / 2 : p[0].N) + 7) / 8, b1 = ((p[1].gated ? p[1].N / 2 : p[1].N) + 7) / 8;
-        hipLaunchKernelGGL(dense_skinny_pair_kernel<true>, dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, nw[0] / 2, nw[1] / 2);
-    } else {
-        hipLaunchKernelGGL(dense_skinny_pair_kernel<false>, dim3(tiles[0] + tiles[1]), dim3(512), 0, st, p[0], p[1], tiles[0], nw[0], nw[1]);
-    }
+    launch_skinny_pair(p, st);
     MI355_CHECK_LAUNCH("dense_skinny_pair_kernel");
     return MI355_OK;
 }

@@ -39,3 +39,21 @@ def test_few_rows_through_every_group():
     y = hops.dense_grouped(x, w, x_step=128, y_step=24, out_dtype=torch.float32).double()
     ref = torch.cat([x[:, i * 128:(i + 1) * 128].double() @ w[i].double().t() for i in range(3)], 1)
     assert float((y - ref).abs().max()) <= 2.0 ** -17 * 128 * 4
+
+
+@pytest.mark.parametrize("N,K", [(2048, 1016), (2048, 1024), (2050, 1032), (4096, 1016), (4097, 1016), (8184, 1024), (8200, 1160), (6152, 2056), (6136, 2048), (64, 5640)])
+def test_few_rows_forms(N, K):
+    """Either side of each rule that picks stages, columns of a stage and rows of a block (K 1024, 256 and 1024 blocks, 4096 weight rows, 24 MB), a last stage with one piece: against a
+    64-bit product, the same bits for any number of rows, alone and in a launch of two."""
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x, w = torch.randn(16, K, device=DEV, generator=g).bfloat16(), (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
+    x2, w2 = torch.randn(16, 72, device=DEV, generator=g).bfloat16(), torch.randn(64, 72, device=DEV, generator=g).bfloat16()
+    y = hops.dense_linear(x, w, out_dtype=torch.float32)
+    ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert float(((y.double() - ref).abs() / (2.0 ** -24 * 1.01 * ref.abs() + 2.0 ** -17 * mag)).max()) <= 1.0
+    gated = hops.dense_linear(x2, w2, gated=True, act=hops.ACT_SILU)
+    for M in (2, 4, 5, 8, 9, 16):
+        a, b = hops.dense_pair(dict(x=x[:M], w=w, out_dtype=torch.float32), dict(x=x2[:M], w=w2, gated=True, act=hops.ACT_SILU))
+        assert torch.equal(hops.dense_linear(x[:M], w, out_dtype=torch.float32), y[:M]) and torch.equal(a, y[:M]) and torch.equal(b, gated[:M]), M
+    a, b = hops.dense_pair(dict(x=x2, w=w2, gated=True, act=hops.ACT_SILU), dict(x=x, w=w, out_dtype=torch.float32))
+    assert torch.equal(a, gated) and torch.equal(b, y)
