@@ -409,6 +409,21 @@ size_t mi355_sampling_draw_workspace_bytes(int32_t rows, int32_t V);
 int mi355_sampling_draw(float* logits, int32_t rows, int32_t V, int32_t ld, const float* temperature, const float* repetition, const float* presence,
                         const float* frequency, const int32_t* output_ids, int32_t id_step, int32_t id_row, const int32_t* input_lengths, int32_t max_input_length,
                         int32_t step, const int32_t* top_k, const float* top_p, const float* uniform_samples, int32_t* ids, void* workspace, mi355_stream_t stream);
+/* A sampler step whose vectors lie in host memory: what mi355_sampling_draw takes is chosen (a temperature of 1 everywhere or penalties that do nothing are left out, top_p 0 reads as 1),
+ * packed and sent in one copy; on return the drawn ids are in ids (device) and in token_ids[row][step] (host, rows of step + 1).  pinned (page-locked host memory) and device: stage_bytes
+ * each, 16-byte aligned, both free again on return.  _takes: 1 if some row has a filter and is not greedy, step < 2048, rows <= 65535; else, from mi355_sampler_step, MI355_ERR_UNSUPPORTED
+ * before anything is done. */
+typedef struct {
+    const float *temperature, *repetition, *presence, *frequency;   /* [rows]; the penalties together or all null */
+    const int32_t* top_k;                                           /* [rows] */
+    const float *top_p, *uniform;                                   /* [rows] */
+    const int32_t *input_lengths, *sequence_lengths;                /* [rows], [n_sequences <= rows]: the history's length, of a sequence that decodes the second */
+    int32_t n_sequences, step;
+    int32_t* token_ids;
+} mi355_sampler_host_t;
+size_t mi355_sampler_step_stage_bytes(int32_t rows, int32_t step);
+int mi355_sampler_step_takes(const mi355_sampler_host_t* host, int32_t rows, int32_t V);
+int mi355_sampler_step(float* logits, int32_t rows, int32_t V, int32_t ld, const mi355_sampler_host_t* host, void* pinned, void* device, int32_t* ids, void* workspace, mi355_stream_t stream);
 /* ids[r] = first index whose inclusive fp32 prefix sum of probs[r, :] (index order) exceeds uniform_samples[r] * sum --
  * sampling from the probabilities, the top_k = 0 / top_p = 1 branch of the sampler (bindings/core/CudaSampleOp.cc:702-737);
  * gives the target model's own sampled token per verify row (target_token_ids of mi355_rejection_sample). */

@@ -68,6 +68,11 @@ class PrefillPass(C.Structure):  # mi355_prefill_pass_t
                 ("logit_rows", vp), ("logits_out", vp), ("workspace", vp), ("workspace_bytes", sz)]
 
 
+class SamplerHost(C.Structure):  # mi355_sampler_host_t
+    _fields_ = [(n, vp) for n in ("temperature", "repetition", "presence", "frequency", "top_k", "top_p", "uniform", "input_lengths", "sequence_lengths")] + [
+        ("n_sequences", i32), ("step", i32), ("token_ids", vp)]
+
+
 class DenseArgs(C.Structure):  # mi355_dense_args_t
     _fields_ = [("x", vp), ("ldx", i32), ("M", i32), ("w", vp), ("N", i32), ("K", i32), ("bias", vp), ("y", vp), ("ldy", i32), ("out_f32", i32), ("gated", i32), ("act", i32),
                 ("act_param", f32)]
@@ -124,6 +129,9 @@ SIGNATURES = {
     "mi355_sampling_probs": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp]),
     "mi355_sampling_draw_workspace_bytes": (sz, [i32, i32]),
     "mi355_sampling_draw": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp, vp, vp, vp, vp]),
+    "mi355_sampler_step_stage_bytes": (sz, [i32, i32]),
+    "mi355_sampler_step_takes": (i32, [C.POINTER(SamplerHost), i32, i32]),
+    "mi355_sampler_step": (i32, [vp, i32, i32, i32, C.POINTER(SamplerHost), vp, vp, vp, vp, vp]),
     "mi355_softmax_rows": (i32, [vp, i32, i32, i32, f32, vp, vp]),
     "mi355_sample_rows": (i32, [vp, i32, i32, i32, vp, vp, vp]),
     "mi355_apply_penalties": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, i32, vp, vp]),

@@ -536,10 +536,20 @@ def sampling_probs(logits: torch.Tensor, temperature: Optional[torch.Tensor] = N
 
 def sampling_draw(logits: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Optional[torch.Tensor], uniform: torch.Tensor, temperature: Optional[torch.Tensor] = None,
                   repetition_penalty: Optional[torch.Tensor] = None, presence_penalty: Optional[torch.Tensor] = None, frequency_penalty: Optional[torch.Tensor] = None,
-                  token_ids: Optional[torch.Tensor] = None, input_lengths: Optional[torch.Tensor] = None, max_input_length: int = 0, step: int = 0) -> torch.Tensor:
-    """sampling_probs in place on the logits, then top_k_top_p_sample on the probabilities, in four launches -> ids [B] int32.  All vectors as sampling_probs takes them."""
+                  token_ids: Optional[torch.Tensor] = None, input_lengths: Optional[torch.Tensor] = None, max_input_length: int = 0, step: int = 0, host=None) -> torch.Tensor:
+    """sampling_probs in place on the logits, then top_k_top_p_sample on the probabilities, in four launches -> ids [B] int32.  All vectors as sampling_probs takes them.  host: of
+    sampler_vectors, in place of the vectors, which the caller holds until the call returns; the ids are then in the history's last column too."""
     _chk(logits, torch.float32, "sampling_draw.logits")
     B, V = logits.shape
+    if host is not None:
+        lib = _C.lib()
+        stage = lib.mi355_sampler_step_stage_bytes(B, host.step)
+        pinned = torch.empty(stage, dtype=torch.uint8, pin_memory=True)
+        work = (lib.mi355_sampling_draw_workspace_bytes(B, V) + 255) // 256 * 256
+        ws = torch.empty(work + stage, dtype=torch.uint8, device=logits.device)
+        ids = torch.empty(B, dtype=torch.int32, device=logits.device)
+        _C.check(lib.mi355_sampler_step(logits.data_ptr(), B, V, V, host, pinned.data_ptr(), ws.data_ptr() + work, ids.data_ptr(), ws.data_ptr(), _stream()), "sampling_draw")
+        return ids
     stride = _sampling_vectors("sampling_draw", logits, (temperature, repetition_penalty, presence_penalty, frequency_penalty, top_p, uniform), token_ids,
                                (input_lengths, top_k), step)
     if token_ids is None and (repetition_penalty is not None or presence_penalty is not None or frequency_penalty is not None):
@@ -551,6 +561,32 @@ def sampling_draw(logits: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Op
                                      1, stride, _p(input_lengths), int(max_input_length), int(step), _p(top_k), _p(top_p), uniform.data_ptr(), ids.data_ptr(),
                                      ws.data_ptr(), _stream()), "sampling_draw")
     return ids
+
+
+def sampler_vectors(logits: torch.Tensor, token_ids: torch.Tensor, temperature: torch.Tensor, penalties, top_k: torch.Tensor, top_p: torch.Tensor, uniform: torch.Tensor,
+                    input_lengths: torch.Tensor, sequence_lengths: torch.Tensor):
+    """What sampling_draw takes as `host`: the vectors of a whole step, penalties (repetition, presence, frequency) or None, history token_ids [B, step + 1].  None where mi355_sampler_step
+    does not take the step, or a tensor is not contiguous host memory of its kernel's type with one value per row."""
+    f32, i32 = torch.float32, torch.int32
+    if logits.dim() != 2 or logits.dtype != f32 or not logits.is_contiguous() or token_ids.dim() != 2:
+        return None
+    B, V = logits.shape
+    vectors = [(temperature, f32), (top_p, f32), (uniform, f32), (top_k, i32)]
+    if penalties is not None:
+        vectors += [(t, f32) for t in penalties] + [(input_lengths, i32)]
+        if sequence_lengths.numel() > B or sequence_lengths.dtype != i32 or not sequence_lengths.is_cpu or not sequence_lengths.is_contiguous():
+            return None
+    for t, dt in vectors:
+        if t.dtype != dt or not t.is_cpu or t.numel() != B or not t.is_contiguous():
+            return None
+    if B == 0 or token_ids.dtype != i32 or not token_ids.is_cpu or not token_ids.is_contiguous() or token_ids.shape[0] != B or token_ids.shape[1] == 0:
+        return None
+    host = _C.SamplerHost(temperature=temperature.data_ptr(), top_k=top_k.data_ptr(), top_p=top_p.data_ptr(), uniform=uniform.data_ptr(), step=token_ids.shape[1] - 1,
+                          token_ids=token_ids.data_ptr())
+    if penalties is not None:
+        host.repetition, host.presence, host.frequency = (t.data_ptr() for t in penalties)
+        host.input_lengths, host.sequence_lengths, host.n_sequences = input_lengths.data_ptr(), sequence_lengths.data_ptr(), sequence_lengths.numel()
+    return host if _C.lib().mi355_sampler_step_takes(host, B, V) else None
 
 
 def ban_repeat_ngram(logits: torch.Tensor, token_ids: torch.Tensor, sequence_last_index: torch.Tensor,

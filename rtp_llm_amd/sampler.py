@@ -76,6 +76,14 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
     step = int(params.step)
     if params.token_ids.shape != (B, step + 1):
         raise ValueError("sample_greedy: token_ids must be [batch_size, step + 1]")
+    # vectors and history on the host, nothing between the penalties and the draw: the whole step in one native call, where some row has a filter
+    penalties = (params.repetition_penalty, params.presence_penalty, params.frequency_penalty)
+    if logits.is_cuda and params.uniform is not None and params.output_all_probs is None and (params.no_repeat_ngram_size is None or params.sequence_lengths.numel() == 0) and \
+            (penalties[0] is None or (penalties[1] is not None and penalties[2] is not None)):
+        host = ops.sampler_vectors(logits, params.token_ids, params.temperature, None if penalties[0] is None else penalties, params.top_k, params.top_p, params.uniform,
+                                   params.input_lengths, params.sequence_lengths)
+        if host is not None:
+            return ops.sampling_draw(logits, None, None, params.uniform, host=host)
     temperature = _host(params.temperature, torch.float32)
     scale = _off(temperature, 1.0)
     penalise = False

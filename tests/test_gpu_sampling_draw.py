@@ -96,3 +96,39 @@ def test_rows_too_flat_to_count(B, V, kind):
         got = x.clone()
         ids = ops.sampling_draw(got, k, p, u)
         assert torch.equal(got, want) and torch.equal(ids, ops.top_k_top_p_sample(want, k, p, u))
+
+
+def _step_params(B, V, n, pen, plain_t, seed):
+    g = torch.Generator().manual_seed(seed)
+    pick = lambda values: torch.tensor(values)[torch.randint(0, len(values), (B,), generator=g)]
+    p = dict(top_k=pick([0, 1, 5, V, V + 3]).int(), top_p=pick([0.0, 1e-8, -1e-8, 0.4, 0.9, 1.0]).float(), temperature=torch.ones(B) if plain_t else pick([0.5, 1.0, 1.5]).float(),
+             uniform=torch.rand(B, generator=g))
+    p["top_k"][0], p["top_p"][0] = 7, 0.8                         # one row at least has a filter
+    if pen != "none":
+        on = pen == "on"
+        p.update(repetition_penalty=pick([1.0, 1.3] if on else [1.0]).float(), presence_penalty=pick([0.0, 0.4] if on else [0.0]).float(), frequency_penalty=pick([0.0, -0.2] if on else [0.0]).float())
+    lens = torch.randint(0, n + 1, (B,), generator=g, dtype=torch.int32)
+    return p, torch.randint(0, V, (B, n + 1), generator=g, dtype=torch.int32), lens, torch.randint(0, n + 1, (B // 2,), generator=g, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("B,V,n", [(1, 50, 0), (3, 1000, 1), (64, 4099, 40), (5, 300, 2047), (7, 300, 2048)])
+@pytest.mark.parametrize("pen", ["none", "neutral", "on"])
+@pytest.mark.parametrize("plain_t", [True, False])
+def test_step_from_host_vectors(monkeypatch, B, V, n, pen, plain_t):
+    """sample_greedy on host vectors, in one native call up to a history of 2047, against its general path: the same ids, probabilities and history, also where a tensor has another type or
+    strides (which the native call leaves to that path)."""
+    x = torch.randn(B, V, device=DEV, generator=torch.Generator(device=DEV).manual_seed(n)) * 3
+    vectors, taken = ops.sampler_vectors, []
+
+    def run(native, change=lambda p: p):
+        monkeypatch.setattr(ops, "sampler_vectors", (lambda *a: taken.append(vectors(*a)) or taken[-1]) if native else (lambda *a: None))
+        p, tokens, lens, seqs = _step_params(B, V, n, pen, plain_t, B + n)
+        logits = x.clone()
+        ids = sampler.sample_greedy(sampler.GreedyParams(logits=logits, input_lengths=lens, sequence_lengths=seqs, token_ids=tokens, step=n, **change(p)))
+        return ids.tolist(), logits, tokens
+
+    want = run(False)
+    for change in (lambda p: p, lambda p: {**p, "top_p": p["top_p"].double()}, lambda p: {**p, "top_k": torch.stack([p["top_k"], p["top_k"]], 1)[:, 0]}):
+        got = run(True, change)
+        assert got[0] == want[0] and torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    assert [t is not None for t in taken] == [n < 2048, False, B == 1 and n < 2048]
