@@ -17,6 +17,7 @@
 //   * up to 4 rows every GEMM is a full-K launch with its consumer fused (gemm_fullk.hip), 5 launches:
 //     [RMSNorm on load +] QKV + bias + RoPE + KV write -> attention -> O + residual (leaves the
 //     per-tile sums of squares) -> RMSNorm on load + gate_up + SiLU-gate -> down + residual;
+//   * up to 8 rows, 16-bit weights whose K slices are short (small models): five launches as well, gemm_rows16.hip (six with an INT8 cache);
 //   * other formats / TP (above 12 rows): QKV GEMM (split-K slabs) -> reduce+bias+RoPE+KV-write -> paged attention
 //     -> O GEMM (slabs) -> reduce+residual+RMSNorm -> gate_up GEMM with fused SiLU-gate -> down GEMM (slabs) ->
 //     reduce+residual+RMSNorm (already the next layer's input norm).  No standalone reduce / add / activation kernels.
@@ -86,6 +87,7 @@ struct mi355_decoder {
     // at 64 (measured M = 64: qkv+rope 20.8 vs 9.0 + 4.9 us, o 18.6 vs 9.7 + slab fold; M = 1: 6.8 vs 7.3 + 3.1 us)
     bool   fuse_qkv, fuse_o, fuse_down, fuse_norm;
     int    fuse_rows;
+    bool   rows16[9];    // [rows]: 16-bit weights, a step of that many rows on the launches of gemm_rows16.hip
     // 1-64 rows (tp = 1): QKV + bias + RoPE + KV write and O + residual as one full-K launch each (gemm_fullk64.hip), their
     // activations handed over as images by the producing launches (RMSNorm fold, attention): 7 launches per layer instead of 8 + no slabs
     bool   img_qkv, img_o;
@@ -355,6 +357,12 @@ extern "C" mi355_decoder_t* mi355_decoder_create(const mi355_model_config_t* cfg
             d->post_norm_exp.push_back(bf_act ? (ex + 8 > 14 ? 14 : ex + 8) : ex);
         }
     }
+    // 16-bit weights, few rows, one rank: norms, RoPE, cache write and residual adds inside the linears (the same bits as the launches they replace)
+    for (int M = 1; M <= 8; ++M) {
+        d->rows16[M] = cfg->tp_size == 1 && cfg->rope_dim == cfg->hd;
+        for (const auto& L : d->layers)
+            d->rows16[M] = d->rows16[M] && mi355_rows16_ok(M, &L.qkv, &L.o, &L.gate_up, &L.down, cfg->kv_dtype == MI355_KV_INT8, kMaxSplits) != 0;
+    }
     std::vector<int32_t> iota_h(cfg->max_batch);
     for (int i = 0; i < cfg->max_batch; ++i) iota_h[i] = i;
     if (hipMemset(d->oob_count, 0, 256) != hipSuccess || hipMemset(d->attn_done, 0, (size_t)(cfg->max_batch < 64 ? cfg->max_batch : 64) * cfg->nkv * 128) != hipSuccess ||
@@ -378,6 +386,8 @@ extern "C" void mi355_decoder_destroy(mi355_decoder_t* d) {
     delete d;
 }
 
+static bool on_rows16(const mi355_decoder_t* d) { return d->B <= 8 && d->rows16[d->B]; }
+
 extern "C" int mi355_decoder_begin(mi355_decoder_t* d, int32_t B, mi355_stream_t stream) {
     return mi355_decoder_begin_rows(d, B, 1, stream);
 }
@@ -399,7 +409,7 @@ extern "C" int mi355_decoder_begin_rows(mi355_decoder_t* d, int32_t nseq, int32_
     } else {
         RUN(MI355_KC_OTHER, mi355_embedding(d->bufs.token_ids, B, d->model.embedding, c.hidden, d->model.vocab_full, d->resid, st));
     }
-    if (c.tp_size == 1 || d->ar) {
+    if ((c.tp_size == 1 || d->ar) && !on_rows16(d)) {
         if ((d->img_qkv && B > d->fuse_rows) || (d->tp_img_qkv && d->ar && B > d->tp_fuse_rows))
             RUN(MI355_KC_NORM, mi355_add_rmsnorm_img(d->resid, nullptr, 0, 0, nullptr, nullptr, nullptr, d->layers[0].input_norm, c.rms_eps, B,
                                                      c.hidden, d->xn_img, ADT, st));
@@ -578,7 +588,14 @@ extern "C" int mi355_decoder_layer_attn(mi355_decoder_t* d, int32_t l, mi355_str
     const int pf = c.tp_size == 1 ? d->pf_mask : 0;       // (tp > 1: the side stream belongs to comm_with_prefetch)
     if (int e = pf_join(d, st)) return e;                  // this layer's QKV weights, requested behind the previous down GEMM
     const bool mid_qkv = (d->img_qkv && B > d->fuse_rows) || tp_img, mid_o = d->img_o && B > d->fuse_rows;   // 1-64 rows: full-K launches on activation images
-    if (mid_qkv) {
+    if (on_rows16(d)) {                                    // the layer's norm, the rotation and (16-bit caches) the cache write inside
+        const bool write = c.kv_dtype != MI355_KV_INT8;
+        RUN(MI355_KC_GEMM_QUANT, mi355_rows16_norm_qkv(d->resid, B, &L.qkv, L.input_norm, c.rms_eps, L.qkv_bias, d->model.cos_sin, c.max_pos, d->bufs.positions, d->bufs.block_table,
+                                                       c.max_blocks_per_seq, d->q_len, c.nh, write ? &kv : nullptr, d->q_buf, d->oob_count, d->partials, kMaxSplits, st));
+        if (!write)
+            RUN(MI355_KC_ROPE_KV, mi355_rope_kv_write_rows(nullptr, d->partials, 1, L.qkv.N_pad, L.qkv_bias, d->model.cos_sin, c.rope_dim, c.max_pos, d->bufs.positions,
+                                                           d->bufs.block_table, c.max_blocks_per_seq, B, d->q_len, c.nh, &kv, d->q_buf, d->oob_count, st));
+    } else if (mid_qkv) {
         RUN(MI355_KC_GEMM_QUANT, mi355_qkv_rope_kv_write_img(d->xn_img, B, &L.qkv, L.qkv_bias, d->model.cos_sin, c.rope_dim, c.max_pos,
                                                              d->bufs.positions, d->bufs.block_table, c.max_blocks_per_seq, d->q_len, c.nh,
                                                              &kv, d->q_buf, d->oob_count, st));
@@ -631,6 +648,10 @@ extern "C" int mi355_decoder_layer_attn(mi355_decoder_t* d, int32_t l, mi355_str
                                              B / d->q_len, d->q_len, c.nh, 1.0f / sqrtf((float)c.hd), c.max_seq_len, d->attn_out, MI355_ATTN_DONE_APART,
                                              d->attn_ws, d->attn_ws_bytes, d->attn_done, st));
     if (int e = pf_join(d, st)) return e;
+    if (on_rows16(d)) {
+        RUN(MI355_KC_GEMM_QUANT, mi355_rows16_residual(d->attn_out, B, &L.o, d->resid, kMaxSplits, st));
+        return MI355_OK;
+    }
     if (d->fuse_o && small) {     // h += fp16(attn W_o) in the GEMM's epilogue: no slabs; the norm moves into gate_up (or stays a launch)
         RUN(MI355_KC_GEMM_QUANT, mi355_linear_residual(d->attn_out, B, &L.o, nullptr, d->resid, d->resid, normed ? d->ssq : nullptr, (c.hidden / 16 + 3) & ~3, st));
         if (!normed) {
@@ -671,6 +692,12 @@ extern "C" int mi355_decoder_layer_mlp(mi355_decoder_t* d, int32_t l, mi355_stre
     const bool normed = small && d->fuse_norm && d->fuse_o;
     const int pf = c.tp_size == 1 ? d->pf_mask : 0;
     if (int e = pf_join(d, st)) return e;
+    if (on_rows16(d)) {
+        RUN(MI355_KC_GEMM_QUANT, mi355_rows16_norm_silu(d->resid, B, &L.gate_up, L.post_norm, c.rms_eps, d->act, st));
+        RUN(MI355_KC_GEMM_QUANT, mi355_rows16_residual(d->act, B, &L.down, d->resid, kMaxSplits, st));
+        if (l + 1 == c.num_layers) RUN(MI355_KC_NORM, mi355_rmsnorm_dt(d->resid, d->model.final_norm, c.rms_eps, B, c.hidden, d->xn, ADT, st));   // feeds lm_head
+        return MI355_OK;
+    }
     if (d->img_o && d->img_gate_up && B > d->fuse_rows) {   // the O launch left gamma 2^-e h' and the sums of h'^2: RMSNorm finished on gate_up's accumulators
         const mi355_deferred_norm_t dn = {d->ssq64, c.hidden / 16, (c.hidden / 16 + 3) & ~3, c.rms_eps, ldexpf(1.f, d->post_norm_exp[l])};
         const bool down_img = d->img_down;                 // gate_up's SiLU epilogue writes the image down_proj's K-quarter launch reads

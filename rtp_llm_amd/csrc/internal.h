@@ -26,6 +26,13 @@ int mi355_fullk64_qkv_ok(const mi355_weight_t* w, int32_t hd);   /* ... as the Q
 int mi355_gemm_wide_direct_ok(const mi355_weight_t* w);   /* gemm_wide.hip: the one-launch form takes this linear (N fills the chip) */
 int mi355_gemm_splitk64_plan(int M, int NT, int KC, int wbits, int group_size, int max_splits, int* cps_out);   /* gemm_splitk64.hip: slabs, or < 0 */
 int mi355_gemm_splitk64_direct_plan(int M, int NT, int KC, int wbits, int group_size);   /* gemm_splitk64.hip, direct form: tiles per block, or < 0 */
+/* gemm_rows16.hip: 16-bit weights, up to 8 rows, a layer's norms, rotation, cache write and residual adds inside its linears */
+int mi355_rows16_ok(int M, const mi355_weight_t* qkv, const mi355_weight_t* o, const mi355_weight_t* gate_up, const mi355_weight_t* down, int quantised_cache, int max_splits);
+int mi355_rows16_norm_qkv(const void* h, int M, const mi355_weight_t* w, const void* norm_weight, float eps, const void* bias, const float* cos_sin, int max_pos, const int32_t* positions,
+                          const int32_t* block_table, int max_blocks_per_seq, int q_len, int nh, const mi355_kv_layer_t* kv, void* q_out, int32_t* oob_count, float* slab, int max_splits,
+                          mi355_stream_t stream);
+int mi355_rows16_residual(const void* x, int M, const mi355_weight_t* w, void* h, int max_splits, mi355_stream_t stream);
+int mi355_rows16_norm_silu(const void* h, int M, const mi355_weight_t* w, const void* norm_weight, float eps, void* y, mi355_stream_t stream);
 int mi355_prefetch(const void* ptr, size_t bytes, void* sink, mi355_stream_t stream);
 /* Touch plan: the blocks a latency-bound launch has to spare (the slab fold in front of a QKV launch: 64 blocks on 256 CUs) read one dword per
  * 128-byte line of the weights the NEXT launch streams, so that its first requests are served by the Infinity Cache (or the XCD's L2)
