@@ -287,10 +287,12 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
         }
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem);
+    auto issue1 = [&](int buf, int kt, int u) {
+        dma16(lds0 + buf * STAGE + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024, voff[u], u < ULA ? X + kt * BK : W + kt * BK);
+    };
     auto issue = [&](int buf, int kt) {
 #pragma unroll
-        for (int u = 0; u < ULD; ++u)
-            dma16(lds0 + buf * STAGE + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024, voff[u], u < ULA ? X + kt * BK : W + kt * BK);
+        for (int u = 0; u < ULD; ++u) issue1(buf, kt, u);
     };
     f32x4 acc[MI][NJ];
 #pragma unroll
@@ -346,24 +348,44 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
             next = next + 1 == NS ? 0 : next + 1;
             ahead = ahead + 1 == NS ? 0 : ahead + 1;
         };
-        auto interleave = [&]() {      // reads between products, nothing across the tile's end (left alone, the scheduler puts the reads in front of the barrier's wait)
-#pragma unroll
-            for (int g = 0; g < MI + NJ; ++g) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, MI * NJ / (MI + NJ), 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, MI * NJ, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        };
         constexpr std::integral_constant<int, ULD * (NS - 3)> steady{};
-        for (; kt + NS < nk; ++kt) {                                        // no conditions inside: the compiler's own waits stay as late as they can be
-            advance(fb, steady, true);
-            multiply(fa);
-            interleave();
+        // One tile in ULD parts: a load of tile kt + NS - 1, its share of the reads of tile kt + 1, its share of tile kt's products, and nothing across a part's end.  Asked for at once behind the
+        // barrier, the block's 32 loads of 16 cycles each stood in front of every wave's products: 1720 cycles a tile instead of the 1024 of the products.
+        constexpr int RP = (MI + NJ + ULD - 1) / ULD, MP = MI / ULD;
+        static_assert(!AHEAD || MI % ULD == 0, "whole rows of products a part");
+        auto tile = [&](const Frags& cur, Frags& nxt) {
+            wait_vm<decltype(steady)::value>();
+            __builtin_amdgcn_s_barrier();
+            const int foff = ((q ^ swizzle(fr)) << 4) + fr * RB;
+            const char* xs = smem + next * STAGE + wm * WM * RB + foff;
+            const char* ws = smem + next * STAGE + (BM + wn * WN) * RB + foff;
+#pragma unroll
+            for (int u = 0; u < ULD; ++u) {
+                issue1(ahead, kt + NS - 1, u);
+#pragma unroll
+                for (int g = u * RP; g < (u + 1) * RP && g < MI + NJ; ++g) {
+                    if (g < NJ) nxt.w[g] = *(const bf16x8*)(ws + g * 16 * RB);
+                    else        nxt.x[g - NJ] = *(const bf16x8*)(xs + (g - NJ) * 16 * RB);
+                }
+#pragma unroll
+                for (int i = u * MP; i < (u + 1) * MP; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.w[j], cur.x[i], acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int g = 0; g < RP; ++g) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, MP * NJ / RP, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x008, MP * NJ, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            next = next + 1 == NS ? 0 : next + 1;
+            ahead = ahead + 1 == NS ? 0 : ahead + 1;
             ++kt;
-            advance(fa, steady, true);
-            multiply(fb);
-            interleave();
+        };
+        while (kt + NS < nk) {                                              // no conditions inside: the compiler's own waits stay as late as they can be
+            tile(fa, fb);
+            tile(fb, fa);
         }
         for (; kt < nk; ++kt) {
             if (kt + 1 < nk) {
