@@ -11,7 +11,7 @@
 //     by the row (conflict-free ds_read_b128); two buffers, one barrier a chunk.  Through registers, as before, the chunk cost 16 of them, and with them the reach of the
 //     fragment reads: 3 fragments are now read ahead of their products.  37888 x 3584 in fp16 W4 at 4096 rows 1066 -> 1002 us, 3584 x 18944 493 -> 459 us (at the rate of
 //     a large dense product on the 224 of 256 CUs that have a block); 8 bits at 1055 rows 343 -> 315 and 159 -> 157 us; bf16 W16 9728 x 896 at 512 rows 20.3 -> 17.8 us;
-//   * weights stream from HBM/L2 once per row tile (the row tiles of a column tile run back to back on different CUs and meet in L2 / Infinity Cache),
+//   * weights stream from HBM/L2 once per row tile (an XCD's blocks walk a column tile's row tiles together and meet in its L2: prefill_tile),
 //     through a 2-deep register ring, buffer range checks instead of tail branches.
 #include "gemm_common.h"
 
@@ -39,6 +39,21 @@ __device__ __forceinline__ void store_bf16(const GemmParams& p, f32x4 v, int m, 
     }
 }
 
+// The chip deals consecutive blocks to its eight XCDs in turn, each with an L2 of its own.  Dealt row by row, the 32 blocks of an XCD read 32 column tiles of the weights
+// and hardly share one: at 128 x 512 tiles 2 MB of 8-bit codes per XCD and 128-k chunk from the Infinity Cache, 5.7 TB/s over the chip.  So an XCD takes a contiguous run
+// of tiles in an order of bands of up to PF_BAND row tiles, column by column: per chunk 4 column tiles and 8 row tiles, a quarter of the bytes.  Column counts that eight
+// divides stay in rows: there an XCD has its columns to itself anyway, and their weights stay in its L2 from one row tile to the next (72 columns 1.6 % faster so, 32
+// columns 2 to 3 %).  us in rows / in bands: 8 bits 37888 x 3584 at 1055 rows 300 / 266, W4 at 4096 rows 1005 / 985, W16 11008 x 4096 at 2667 rows 418 / 315, 896 x 4864 at
+// 1753 rows 42 / 36; 110 random calls 0.97 of the time in rows; bands of 6, 8 and 12 alike, 24 1 % slower.
+constexpr int PF_XCD = 8, PF_BAND = 8;
+__host__ __device__ __forceinline__ void prefill_tile(int id, int rows, int cols, int& bx, int& by) {
+    if (cols % PF_XCD == 0) { bx = id % cols; by = id / cols; return; }
+    const int nb = rows * cols, k = id % PF_XCD, j = k * (nb / PF_XCD) + (k < nb % PF_XCD ? k : nb % PF_XCD) + id / PF_XCD;
+    const int bands = (rows + PF_BAND - 1) / PF_BAND, band = (rows + bands - 1) / bands;      // of even height
+    const int r0 = j / (band * cols) * band, i = j - r0 * cols, h = band < rows - r0 ? band : rows - r0;
+    bx = i / h; by = r0 + i % h;
+}
+
 // One block = 8 waves: NWN = 8 / KS of them side by side along N, KS of them along K (slice ks takes the chunks c with c % KS == ks; the slices' sums meet in
 // LDS at the end).  TPW = weight tiles per wave, MB = 16-row blocks of the tile, so the tile is 16 MB rows x 16 TPW NWN columns.
 //   TPW = 4, MB = 8 (128 x 512, one block per CU): one B-fragment read from LDS feeds four MFMAs.  At TPW = 2 (128 x 256, two blocks per CU) the 8 waves of a
@@ -47,7 +62,7 @@ __device__ __forceinline__ void store_bf16(const GemmParams& p, f32x4 v, int m, 
 // BF: bf16 activations.  16-bit weights are the MFMA operand as they are; a 4-bit code enters it as the exact integer u - z and the group's scale multiplies the
 // group's fp32 sums (a bf16 product s (u - z) would round the weight to 8 bits); an 8-bit code as the exact u - 128, its column scale on the finished sums.
 template <int WBITS, int GS, bool BF, int MB, int TPW, int KS>
-__global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p) {
+__global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p, const int rows, const int cols) {
     constexpr int BM = 16 * MB, NWN = 8 / KS;                 // rows, waves side by side
     constexpr int LPC  = WBITS / 4;
     constexpr int NSUB = (GS > 0) ? 4 / GS : 1;
@@ -64,8 +79,10 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave / NWN;
     const int jj = lane & 15, q = lane >> 4;
-    const int m0 = blockIdx.y * BM;
-    const int nt_base = (blockIdx.x * NWN + wave % NWN) * TPW;
+    int bx, by;
+    prefill_tile((int)blockIdx.x, rows, cols, bx, by);
+    const int m0 = by * BM;
+    const int nt_base = (bx * NWN + wave % NWN) * TPW;
     const int KC = p.KC;
 
     constexpr uint32_t FLAGS = 0x00020000u;
@@ -322,8 +339,8 @@ int pick_shape(int M, int NT, int KC, bool bf, int wbits, double* t_best) {
 template <int WBITS, int GS, bool BF, int I>
 void launch_shape_t(const GemmParams& p, hipStream_t st) {
     constexpr PrefillShape s = kPrefillShapes[I];
-    const dim3 grid(cdiv(p.NT, 8 / s.ks * s.tpw), cdiv(p.M, 16 * s.mb));
-    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks>), grid, dim3(512), 0, st, p);
+    const int rows = cdiv(p.M, 16 * s.mb), cols = cdiv(p.NT, 8 / s.ks * s.tpw);
+    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks>), dim3(rows * cols), dim3(512), 0, st, p, rows, cols);
 }
 template <int WBITS, int GS, bool BF>
 int launch_shape(int i, const GemmParams& p, hipStream_t st) {
@@ -342,6 +359,13 @@ int launch_shape(int i, const GemmParams& p, hipStream_t st) {
 }
 
 } // namespace
+
+// The tile that block id of a rows x cols grid of tiles takes: column tile in the low half, row tile in the high half (for the tests: every tile once).
+extern "C" int64_t mi355_gemm_prefill_tile(int32_t id, int32_t rows, int32_t cols) {
+    int bx, by;
+    prefill_tile(id, rows, cols, bx, by);
+    return (int64_t)by << 32 | bx;
+}
 
 // The block shape of a call, by its place in kPrefillShapes: NT = N_pad / 16, KC = K_pad / 128.
 extern "C" int mi355_gemm_prefill_shape(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits) {

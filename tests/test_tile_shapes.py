@@ -19,6 +19,20 @@ def test_prefill_shapes(bf16, wbits):
     assert {_prefill(M, K, N, bf16, wbits) for M, K, N in prefill.SHAPES} == can
 
 
+@pytest.mark.parametrize("cols", [1, 2, 7, 8, 14, 43, 72, 74])
+@pytest.mark.parametrize("rows", [1, 2, 7, 8, 9, 16, 17, 25, 65])
+def test_prefill_tiles_once(rows, cols):
+    """Whatever the order in which the blocks take the tiles: each tile once; the blocks of an XCD take a run of whole columns of at most 8 row tiles."""
+    tile = _C.lib().mi355_gemm_prefill_tile
+    got = [(t & 0xffffffff, t >> 32) for t in (tile(i, rows, cols) for i in range(rows * cols))]
+    assert sorted(got) == [(c, r) for c in range(cols) for r in range(rows)]
+    if cols % 8 == 0:
+        assert got == [(c, r) for r in range(rows) for c in range(cols)]
+    elif rows <= 8:
+        run = [t for x in range(8) for t in got[x::8]]
+        assert run == [(c, r) for c in range(cols) for r in range(rows)]
+
+
 def test_dense_shapes():
     pick = _C.hybrid_lib().mi355_dense_tile_shape
     can = {pick(M, N, K, 1, 0) for M in (17, 65, 300, 768, 1537, 2304, 4700, 6000, 8190) for N in (8, 200, 1032, 2044, 4100, 16400) for K in (8, 40, 136, 264, 1032, 2056)}
