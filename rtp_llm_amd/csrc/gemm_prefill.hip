@@ -12,7 +12,8 @@
 //     fragment reads: 3 fragments are now read ahead of their products.  37888 x 3584 in fp16 W4 at 4096 rows 1066 -> 1002 us, 3584 x 18944 493 -> 459 us (at the rate of
 //     a large dense product on the 224 of 256 CUs that have a block); 8 bits at 1055 rows 343 -> 315 and 159 -> 157 us; bf16 W16 9728 x 896 at 512 rows 20.3 -> 17.8 us;
 //   * weights stream from HBM/L2 once per row tile (an XCD's blocks walk a column tile's row tiles together and meet in its L2: prefill_tile),
-//     through a 2-deep register ring, buffer range checks instead of tail branches.
+//     through a 2-deep register ring (128 x 512: half a chunk at a time, see WHOLE), buffer range checks instead of tail branches.
+#include <type_traits>
 #include "gemm_common.h"
 
 namespace {
@@ -61,7 +62,28 @@ __host__ __device__ __forceinline__ void prefill_tile(int id, int rows, int cols
 //   MB = 4 and the K-sliced forms are for grids that would leave most CUs without a block (narrow outputs, short prompts): see launch_prefill_t.
 // BF: bf16 activations.  16-bit weights are the MFMA operand as they are; a 4-bit code enters it as the exact integer u - z and the group's scale multiplies the
 // group's fp32 sums (a bf16 product s (u - z) would round the weight to 8 bits); an 8-bit code as the exact u - 128, its column scale on the finished sums.
-template <int WBITS, int GS, bool BF, int MB, int TPW, int KS>
+// WHOLE: K is a multiple of 128 and x lies on 16 bytes, so that every chunk comes by DMA and the loop has no branch.  With the branches of the general loop the
+// compiler's count of loads in flight, taken over all paths, made the products wait for the DMA of the chunk after (37 to 42 % of the waves' time at 128 x 512 went into
+// waits), and the first three fragment reads of a chunk waited one by one.  In front of the last chunk of a straight loop lies one DMA too many (K sliced: left out);
+// it reads a chunk again that is there, and is waited for.
+// us general / WHOLE, same bits: 8 bits 37888 x 3584 at 1055 rows 279 / 263 (128 x 512), 3584 x 18944 155 / 136 (64 x 256); fp16 W4 37888 x 3584 at 4096 rows 1060 / 1004
+// (power), 3584 x 3584 at 512 rows 36 / 32 (64 x 256), 26.6 / 22.7 (64 x 128); bf16 W4 37888 x 3584 at 4096 rows 1257 / 1091 (128 x 256); W16 896 x 4864 at 777 rows
+// 21.3 / 19.1 (64 x 64), 9728 x 896 39 / 34 (32 x 64).
+// The 128 x 512 form has 128 registers of sums and none for two chunks of weights: it holds one chunk's, each half loaded again as soon as its last operand is formed
+// (a little more than half a chunk, 1.4 us, ahead of its use; the other row tiles of the XCD's band have most of them in L2).  230 and 236 registers; a ring of two spills.
+template <int WBITS, int TPW, int MB, int AHEAD>
+__device__ __forceinline__ void pace(int i0, int n) {         // the order of fragment reads, products and operand arithmetic of fragments i0 .. i0 + n - 1 of a chunk
+#pragma unroll
+    for (int i = i0; i < i0 + n; ++i) {
+        if (i + AHEAD < 4 * MB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if constexpr (WBITS != 16) __builtin_amdgcn_sched_group_barrier(0x002, (14 + MB - 1) / MB, 0);
+        }
+    }
+}
+template <int WBITS, int GS, bool BF, int MB, int TPW, int KS, bool WHOLE>
 __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p, const int rows, const int cols) {
     constexpr int BM = 16 * MB, NWN = 8 / KS;                 // rows, waves side by side
     constexpr int LPC  = WBITS / 4;
@@ -71,7 +93,9 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     constexpr bool CSCALE = BF && GROUPED;                    // the group's scale on the accumulator side
     constexpr int XSLOTS = 256 * MB;                          // 16-byte pieces of an x chunk tile
     constexpr int UPT = XSLOTS / (64 * NWN);                  // staging loads per wave
-    constexpr int WLD = TPW * (LPC + (GS > 0 ? NSUB : 0));    // weight loads per wave and chunk
+    constexpr bool HALVES = WHOLE && TPW == 4;                // the weights of half a chunk in registers, not of two chunks
+    constexpr int WLD = TPW * ((HALVES ? 2 : LPC) + (GS > 0 ? NSUB : 0));     // weight loads per wave and chunk
+    static_assert(!HALVES || (WBITS != 16 && !CSCALE && NSUB == 1 && KS == 1), "one scale a chunk");
     __shared__ u32x4 xs[KS][2][XSLOTS];
     static_assert(KS == 1 || (size_t)(KS - 1) * NWN * TPW * MB * 1024 <= sizeof(u32x4) * 2 * KS * XSLOTS, "the slices' sums meet in the x buffers");
 
@@ -107,10 +131,20 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
         const int pi = (u * NWN + wave % NWN) * 64 + lane, j = pi >> 4, pp = (pi & 15) ^ (j & 15);
         xoff[u] = (uint32_t)(((size_t)min(m0 + j, p.M - 1) * p.K + pp * 8) * 2);      // rows past M repeat the last one: their sums are never stored
     }
+    if constexpr (HALVES) {                                   // load u starts 32 u rows further down, at most at the last row: two registers for all
+        const int j = wave * 4 + (lane >> 4), pp = (lane & 15) ^ (j & 15);
+        xoff[0] = (uint32_t)(m0 + j) * (uint32_t)p.K * 2u + pp * 16u;
+        xoff[1] = (uint32_t)(p.M - 1) * (uint32_t)p.K * 2u + pp * 16u;
+    }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&xs[ks][0][0];
-    const bool dma = (uintptr_t)p.x % 16 == 0 && p.K % 8 == 0;
-    auto load_x = [&](int c, int buf) {
-        if (dma && c * 128 + 128 <= p.K) {
+    const bool dma = WHOLE || ((uintptr_t)p.x % 16 == 0 && p.K % 8 == 0);
+    auto load_x = [&](int c, int buf) __attribute__((always_inline)) {
+        if constexpr (HALVES) {
+            asm volatile("" : "+v"(xoff[0]));                 // the sums are formed here, not kept through the loop
+#pragma unroll
+            for (int u = 0; u < UPT; ++u)
+                dma16(lds0 + (buf * XSLOTS + (u * NWN + wave % NWN) * 64) * 16, min(xoff[0] + (uint32_t)u * 64u * (uint32_t)p.K, xoff[1]), (const char*)p.x + (size_t)c * 256);
+        } else if (WHOLE || (dma && c * 128 + 128 <= p.K)) {
 #pragma unroll
             for (int u = 0; u < UPT; ++u)
                 dma16(lds0 + (buf * XSLOTS + (u * NWN + wave % NWN) * 64) * 16, xoff[u], (const char*)p.x + (size_t)c * 256);
@@ -124,9 +158,25 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     };
 
     const uint32_t lane16 = lane * 16u, jj4 = jj * 4u;
-    u32x4    wr[2][TPW][LPC];
+    u32x4    wr[2][TPW][LPC];                                 // HALVES: wr[0][t][h] (8 bits) or the half-filled wr[0][t][0] (4 bits) are the chunk at work
     uint32_t mr[2][TPW][NSUB];
-    auto load_w = [&](int d, int c) {
+    auto load_half = [&](int h, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            if constexpr (WBITS == 8) wr[0][t][h % LPC] = bload128<0>(rw[t], lane16, (uint32_t)(c * LPC + h) * 1024u);
+            else {
+                const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw[t], lane16 + h * 8, (uint32_t)c * 1024u, 0));
+                wr[0][t][0][2 * h] = v[0]; wr[0][t][0][2 * h + 1] = v[1];
+            }
+        }
+    };
+    auto load_meta = [&](int d, int c) __attribute__((always_inline)) {
+        if (GROUPED) {
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) mr[d][t][0] = __builtin_amdgcn_raw_buffer_load_b32(rm[t], jj4, (uint32_t)c * (uint32_t)p.N_pad * 4u, 0);
+        }
+    };
+    auto load_w = [&](int d, int c) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TPW; ++t) {
 #pragma unroll
@@ -152,15 +202,23 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     const W4Consts w4c = w4_consts();
     const f16x2 c960 = {(f16)960.f, (f16)960.f};
 
-    load_x(ks, 0);
-    load_w(0, ks);
-    load_w(1, ks + KS);
+    load_x(WHOLE ? min(ks, KC - 1) : ks, 0);
+    if constexpr (HALVES) {
+        load_half(0, 0); load_half(1, 0); load_meta(0, 0);
+    } else {
+        load_w(0, ks);
+        load_w(1, ks + KS);
+    }
 
-    auto dq = [&](int d, int t, int s) -> u32x4 {
+    auto dq = [&](int d, int t, int s) __attribute__((always_inline)) -> u32x4 {
         if constexpr (WBITS == 16) return wr[d][t][s];
         const uint32_t m = GROUPED ? mr[d][t][s / SPG] : mch[t];
-        const f16x2 zn = as_h2(__builtin_amdgcn_perm(m, m, 0x05040504u));
-        const f16x2 sc = as_h2(__builtin_amdgcn_perm(m, m, 0x07060706u));
+        f16x2 zn, sc;
+        if constexpr (HALVES) {      // halves that the packed operations pick themselves: eight registers less
+            zn = (f16x2){as_h2(m)[0], as_h2(m)[0]}; sc = (f16x2){as_h2(m)[1], as_h2(m)[1]};
+        } else {
+            zn = as_h2(__builtin_amdgcn_perm(m, m, 0x05040504u)); sc = as_h2(__builtin_amdgcn_perm(m, m, 0x07060706u));
+        }
         if constexpr (BF) {          // small integers: exact in fp16, in fp32 and in bf16 (the high half of the fp32)
             f16x8 v;
             if constexpr (WBITS == 4) {
@@ -176,18 +234,25 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
                 r[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, (float)v[2 * i + 1]), __builtin_bit_cast(uint32_t, (float)v[2 * i]), 0x07060302u);
             return r;
         } else {
-            if constexpr (WBITS == 4) return __builtin_bit_cast(u32x4, dequant_w4_vc(wr[d][t][0][s], zn, zn + c960, sc, w4c));
-            const u32x4 w = wr[d][t][(s >> 1) % LPC];   // per-channel int8: exact (u - z) operand, the column scale is applied in fp32 in the epilogue
+            const int r = HALVES ? 0 : d;
+            if constexpr (WBITS == 4) return __builtin_bit_cast(u32x4, dequant_w4_vc(wr[r][t][0][s], zn, zn + c960, sc, w4c));
+            const u32x4 w = wr[r][t][(s >> 1) % LPC];   // per-channel int8: exact (u - z) operand, the column scale is applied in fp32 in the epilogue
             return __builtin_bit_cast(u32x4, dequant_w8<GROUPED>(w[(s & 1) * 2], w[(s & 1) * 2 + 1], zn, sc));
         }
     };
-    auto frag = [&](int buf, int s, int mb) { return xs[ks][buf][mb * 256 + jj * 16 + ((s * 4 + q) ^ jj)]; };
+    uint32_t fo[4];                                           // HALVES: this lane's first fragment of each k-step in the buffer at work
+#pragma unroll
+    for (int s = 0; s < 4; ++s) fo[s] = lds0 + (jj * 16 + ((s * 4 + q) ^ jj)) * 16;
+    auto frag = [&](int buf, int s, int mb) __attribute__((always_inline)) {
+        if constexpr (HALVES) return *(const __attribute__((address_space(3))) u32x4*)(fo[s] + mb * 4096);
+        else return xs[ks][buf][mb * 256 + jj * 16 + ((s * 4 + q) ^ jj)];
+    };
     u32x4 an[TPW];                                            // operands of the next k-step (a chunk starts with those the one before left)
-    auto next = [&](int d, int s) {
+    auto next = [&](int d, int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TPW; ++t) an[t] = dq(d, t, s);
     };
-    auto compute = [&](int d, int buf) {
+    auto compute = [&](int c, int d, int buf) __attribute__((always_inline)) {
         if constexpr (CSCALE) {              // a group's sums on accumulators of their own, scaled as they join the tile's
 #pragma unroll
             for (int gi = 0; gi < NSUB; ++gi) {
@@ -216,10 +281,12 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
         } else {
             // Fragment i + AHEAD is read while fragment i is multiplied, the next k-step's operands are formed between the products: left to itself the compiler
             // reads two fragments, waits for them and multiplies (one LDS latency per 8 products and wave)
-            constexpr int AHEAD = WBITS == 8 && TPW == 4 ? 1 : 3, N = 4 * MB;
+            constexpr int AHEAD = WBITS == 8 && TPW == 4 && !HALVES ? 1 : 3, N = 4 * MB;
             u32x4 b[AHEAD + 1];
 #pragma unroll
             for (int i = 0; i < AHEAD; ++i) b[i] = frag(buf, i / MB, i % MB);
+            if (WHOLE) __builtin_amdgcn_sched_barrier(0);
+            else       __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 u32x4 a[TPW];
@@ -233,34 +300,64 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
 #pragma unroll
                     for (int t = 0; t < TPW; ++t) acc[t][mb] = mfma_act<BF>(a[t], b[i % (AHEAD + 1)], acc[t][mb]);
                 }
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                if (i + AHEAD < N) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-#pragma unroll
-                for (int t = 0; t < TPW; ++t) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    if constexpr (WBITS != 16) __builtin_amdgcn_sched_group_barrier(0x002, (14 + MB - 1) / MB, 0);
+                if constexpr (HALVES) {
+                    pace<WBITS, TPW, MB, AHEAD>(s * MB, MB);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (s == 0) { load_half(0, c + 1); load_meta(d ^ 1, c + 1); }
+                    if (s == 2) load_half(1, c + 1);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
+            if constexpr (!HALVES) pace<WBITS, TPW, MB, AHEAD>(0, N);
         }
     };
 
     // Chunk c lies in buffer and ring d.  One barrier: behind it every wave's part of chunk c is in LDS and chunk c - KS is done with, so that the DMA of chunk c + KS may
-    // go over it.  At most the weights of chunk c + KS are younger than the DMA of chunk c.
-    auto chunk = [&](int c, int d) {
-        wait_vm<WLD>();
+    // go over it.  At most the weights of chunk c + KS are younger than the DMA of chunk c; in front of a last chunk nothing is (its loads of weights past the end are
+    // unused, and the compiler leaves them out).
+    const std::true_type more{};                     // WHOLE: a chunk follows, or is loaded all the same
+    const std::false_type last{};
+    auto chunk = [&](int c, int d, int buf, auto follows) __attribute__((always_inline)) {
+        if (WHOLE && !decltype(follows)::value) wait_vm<0>();
+        else wait_vm<WLD>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (c + KS < KC) load_x(c + KS, d ^ 1);
-        if (c < KC) compute(d, d);                   // slices past the end have nothing left
-        load_w(d, c + 2 * KS);
+        if constexpr (WHOLE) {
+            if (decltype(follows)::value) load_x(min(c + KS, KC - 1), buf ^ 1);
+        } else if (c + KS < KC) load_x(c + KS, buf ^ 1);
+        if ((WHOLE && KS == 1) || c < KC) compute(c, d, buf);    // slices past the end have nothing left
+        if (!HALVES) load_w(d, c + 2 * KS);
+        if (WHOLE) __builtin_amdgcn_sched_barrier(0);
     };
     if constexpr (!CSCALE) next(0, 0);
-    for (int c = ks; c - ks < KC; c += 2 * KS) {     // the same number of rounds for every slice
-        chunk(c, 0);
-        if (c - ks + KS < KC) chunk(c + KS, 1);
+    if constexpr (HALVES) {
+        for (int c = 0; c < KC; ++c) {
+            chunk(c, 0, c & 1, more);
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) mr[0][t][0] = mr[1][t][0];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                fo[s] += c & 1 ? -XSLOTS * 16 : XSLOTS * 16;
+                asm volatile("" : "+v"(fo[s]));
+            }
+        }
+        wait_vm<0>();
+    } else if constexpr (WHOLE) {
+        int c = ks, left = (KC + KS - 1) / KS;       // the same number of rounds for every slice
+        for (; left > (KS > 1 ? 2 : 1); left -= 2, c += 2 * KS) {
+            chunk(c, 0, 0, more);
+            chunk(c + KS, 1, 1, more);
+        }
+        if (KS > 1 && left == 2) {
+            chunk(c, 0, 0, more);
+            chunk(c + KS, 1, 1, last);
+        } else if (left) chunk(c, 0, 0, last);
+        wait_vm<0>();
+    } else {
+        for (int c = ks; c - ks < KC; c += 2 * KS) { // the same number of rounds for every slice
+            chunk(c, 0, 0, last);
+            if (c - ks + KS < KC) chunk(c + KS, 1, 1, last);
+        }
     }
     if constexpr (KS > 1) __syncthreads();
 
@@ -336,11 +433,21 @@ int pick_shape(int M, int NT, int KC, bool bf, int wbits, double* t_best) {
     return best;
 }
 
+// The loop without branches where x allows it.  Not for 128 x 512 under groups of 32 or 64 (two or four scales a chunk and tile have no registers left), nor for 64 x 256
+// in groups of 32 and the 64-row forms of bf16 W4 (held in one piece the compiler takes more than 128 or 80 registers for them and a block less fits a CU: 37888 x 3584 at
+// 4096 rows 1293 -> 1485 us).  K below 2^23: the 128 x 512 form's row offsets are formed past the last row, in 32 bits.
 template <int WBITS, int GS, bool BF, int I>
 void launch_shape_t(const GemmParams& p, hipStream_t st) {
     constexpr PrefillShape s = kPrefillShapes[I];
     const int rows = cdiv(p.M, 16 * s.mb), cols = cdiv(p.NT, 8 / s.ks * s.tpw);
-    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks>), dim3(rows * cols), dim3(512), 0, st, p, rows, cols);
+    constexpr bool straight = !(I == 0 && (GS == 1 || GS == 2)) && !(I == 2 && GS == 1) && !(BF && WBITS == 4 && s.mb == 4 && s.ks == 1);
+    if constexpr (straight) {
+        if ((uintptr_t)p.x % 16 == 0 && p.K % 128 == 0 && p.K < 1 << 23) {
+            hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, true>), dim3(rows * cols), dim3(512), 0, st, p, rows, cols);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, false>), dim3(rows * cols), dim3(512), 0, st, p, rows, cols);
 }
 template <int WBITS, int GS, bool BF>
 int launch_shape(int i, const GemmParams& p, hipStream_t st) {

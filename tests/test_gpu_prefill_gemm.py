@@ -50,6 +50,31 @@ def test_prefill_gemm_shapes(kind, group, dtype, M, K, N):
     assert float(over.max()) <= 1.0, (float(over.max()), float((y - ref).abs().max()))
 
 
+# K a multiple of 128 (1 to 9 chunks, odd and even, fewer than the slices of K), every tile shape, the last row tile full, of one row, of some
+WHOLE = [(65, 128, 48), (100, 256, 1152), (130, 384, 896), (300, 512, 896), (577, 640, 1152), (129, 1152, 4600), (513, 384, 9728), (640, 1024, 4104), (1100, 256, 8208), (2049, 384, 4104),
+         (300, 896, 37880), (1537, 1152, 4104), (150, 384, 37880), (400, 896, 4104)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,group", [("w4", 128), ("w4", 64), ("w4", 32), ("int8", 0), ("fp16", 0)])
+def test_prefill_gemm_straight_loop(kind, group, dtype):
+    """x on 16 bytes (the loop without branches) and off them (the general loop): the same bits."""
+    seen = set()
+    for M, K, N in WHOLE:
+        c = model.synth_linear(K, N, kind, "cpu", _gen(K + N), group or 128)
+        if kind == "fp16":
+            c.w = c.w.to(dtype)
+        w = c.pack(dtype=dtype).to(DEV)
+        buf = torch.zeros(M * K + 8, dtype=dtype, device=DEV)
+        x = (torch.randn(M, K, generator=_gen(M)) * 0.5).to(dtype).to(DEV)
+        off = buf[4:4 + M * K].view(M, K).copy_(x)
+        assert x.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 8
+        assert torch.equal(ops.linear(x, w).view(torch.int16), ops.linear(off, w).view(torch.int16)), (M, K, N)
+        seen.add(_C.lib().mi355_gemm_prefill_shape(M, -(-N // 16), K // 128, int(dtype == torch.bfloat16), w.wbits))
+    can = {0, 1, 2, 3, 4, 5, 6} - ({0} if kind == "fp16" or dtype == torch.bfloat16 else set()) - ({2} if kind == "fp16" else set())
+    assert seen >= can, seen
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("kind", ["w4", "int8", "fp16"])
 def test_prefill_gemm_silu_pairs(kind, dtype):
