@@ -117,8 +117,15 @@ int mi355_dense_grouped_ex(const void* x, int32_t ldx, int32_t M, const void* w,
                            int32_t out_f32, int32_t gated, int32_t act, float act_param, int32_t act_dtype, int32_t G, int64_t xs, int64_t ys,
                            const int32_t* offs, const int32_t* gather, const int32_t* tiles, int32_t max_tiles, const float* egate, int32_t ldg,
                            int32_t goff, mi355_stream_t stream);
+int mi355_dense_grouped_ahead(const void* x, int32_t ldx, int32_t M, const void* w, int32_t N, int32_t K, const void* bias, void* y, int32_t ldy,
+                              int32_t out_f32, int32_t gated, int32_t act, float act_param, int32_t act_dtype, int32_t G, int64_t xs, int64_t ys,
+                              const int32_t* offs, const int32_t* gather, const int32_t* tiles, int32_t max_tiles, const float* egate, int32_t ldg,
+                              int32_t goff, const void* ahead, int64_t ahead_bytes, mi355_stream_t stream);
 int mi355_hy_moe_route_ex(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
                           int32_t score, int32_t group_top, float wscale, mi355_stream_t stream);
+int mi355_hy_moe_route_sorted(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
+                              int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top, float wscale,
+                              const void* ahead, int64_t ahead_bytes, mi355_stream_t stream);
 int mi355_hy_moe_route_align_ex(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
                                 int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top,
                                 float wscale, mi355_stream_t stream);

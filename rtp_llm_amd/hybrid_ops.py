@@ -824,13 +824,15 @@ def head_norm(o: torch.Tensor, heads: int, vdim: int, w: Optional[torch.Tensor],
 
 def dense_grouped(x: torch.Tensor, w: torch.Tensor, *, x_step: int = 0, y_step: int = 0, offs: Optional[torch.Tensor] = None,
                   gather: Optional[torch.Tensor] = None, tiles: Optional[torch.Tensor] = None, rows: Optional[int] = None, out_dtype: Optional[torch.dtype] = None, gated: bool = False,
-                  act: int = ACT_NONE, out: Optional[torch.Tensor] = None, mul_sigmoid: Optional[torch.Tensor] = None, act_param: float = 0.0) -> torch.Tensor:
+                  act: int = ACT_NONE, out: Optional[torch.Tensor] = None, mul_sigmoid: Optional[torch.Tensor] = None, act_param: float = 0.0,
+                  ahead: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One launch of G = w.shape[0] linears with the weights w [G, N, K].  mul_sigmoid: fp32 [M, width of the output] pre-activations (a column
     slice of a wider buffer is fine); every output is multiplied by the sigmoid of its entry before it is stored.
     Without offs every group takes all rows of x, reads its K inputs from column g * x_step and writes its outputs from column g * y_step
     (per-head projections).  With offs (int32 [G + 1] on the device) the `rows` rows of the output are sorted by group, group g owns rows
     offs[g] .. offs[g + 1] - 1, and sorted row r reads x[gather[r]] (x[r] without gather): the experts of a mixture.  tiles: the list of
-    64-row tiles that hold rows, as moe_align writes it (without it every group is launched over all row tiles)."""
+    64-row tiles that hold rows, as moe_align writes it (without it every group is launched over all row tiles).  ahead (with tiles): a contiguous weight
+    that a later launch streams, which the blocks past the list read into the caches."""
     _dev(x, w.dtype, "dense_grouped.x"); _dev(w, w.dtype, "dense_grouped.w")
     if w.dim() != 3 or not w.is_contiguous():
         raise _C.Mi355Error(f"dense_grouped: weights {tuple(w.shape)} must be contiguous [G, N, K]")
@@ -864,10 +866,10 @@ def dense_grouped(x: torch.Tensor, w: torch.Tensor, *, x_step: int = 0, y_step: 
         if mul_sigmoid.shape != (M, width):
             raise _C.Mi355Error(f"dense_grouped: gate {tuple(mul_sigmoid.shape)} for outputs [{M}, {width}]")
     if M:
-        _C.check_hybrid(_C.hybrid_lib().mi355_dense_grouped_ex(x.data_ptr(), ldx, M, w.data_ptr(), N, K, None, out.data_ptr(), _rows(out, "dense_grouped.out"),
+        _C.check_hybrid(_C.hybrid_lib().mi355_dense_grouped_ahead(x.data_ptr(), ldx, M, w.data_ptr(), N, K, None, out.data_ptr(), _rows(out, "dense_grouped.out"),
                                                                1 if od == torch.float32 else 0, 1 if gated else 0, act, float(act_param), act_code(w.dtype), G, x_step,
                                                                y_step, _p(offs), _p(gather), _p(tiles), 0 if tiles is None else (tiles.numel() - 1) // 2,
-                                                               _p(mul_sigmoid), ldg, 0, _stream()),
+                                                               _p(mul_sigmoid), ldg, 0, *_ahead(ahead, "dense_grouped.ahead"), _stream()),
                         "dense_grouped")
     return out
 
@@ -959,22 +961,38 @@ def moe_align(ids: torch.Tensor, experts: int):
     return offs, src, place, tiles
 
 
-def moe_route_sorted(z: torch.Tensor, experts: int, groups: int, keep: int, top: int, *, sigmoid: bool = False, chosen: bool = False, group_top: int = 1, scale: float = 1.0):
-    """moe_route followed by moe_align -> (ids, wts, offs, src_row, place_of, tiles); a few tokens (a decode step) take one launch for both."""
+def _ahead(t: Optional[torch.Tensor], name: str):
+    """(address, bytes) of a weight that is read ahead of its use."""
+    if t is None:
+        return 0, 0
+    _dev(t, t.dtype, name)
+    if not t.is_contiguous():
+        raise _C.Mi355Error(f"{name}: must be contiguous")
+    return t.data_ptr(), t.numel() * t.element_size()
+
+
+def moe_route_sorted(z: torch.Tensor, experts: int, groups: int, keep: int, top: int, *, sigmoid: bool = False, chosen: bool = False, group_top: int = 1, scale: float = 1.0,
+                     ahead: Optional[torch.Tensor] = None):
+    """moe_route followed by moe_align -> (ids, wts, offs, src_row, place_of, tiles); a few tokens (a decode step) take one launch for both.  ahead: the
+    contiguous weight of the grouped linear behind, which the sort of many tokens reads into the caches on the way."""
     _dev(z, torch.float32, "moe_route_sorted.z")
     T = z.shape[0]
     if z.shape[1] != experts:
         raise _C.Mi355Error(f"moe_route_sorted: logits {tuple(z.shape)} for {experts} experts")
-    if not 0 < T <= 64 or 16 * (experts + groups) * 4 + experts * 8 > 48 * 1024:
+    many = not 0 < T <= 64 or 16 * (experts + groups) * 4 + experts * 8 > 48 * 1024
+    if T == 0:
         ids, wts = moe_route(z, groups, keep, top, sigmoid=sigmoid, chosen=chosen, group_top=group_top, scale=scale)
         return (ids, wts) + moe_align(ids, experts)
     dev = z.device
     ids, wts = torch.empty(T, top, dtype=torch.int32, device=dev), torch.empty(T, top, dtype=torch.float32, device=dev)
     offs, src, place = torch.empty(experts + 1, dtype=torch.int32, device=dev), torch.empty(T * top, dtype=torch.int32, device=dev), torch.empty(T * top, dtype=torch.int32, device=dev)
     tiles = torch.empty(1 + 2 * (T * top // 64 + experts), dtype=torch.int32, device=dev)
-    _C.check_hybrid(_C.hybrid_lib().mi355_hy_moe_route_align_ex(z.data_ptr(), _rows(z, "moe_route_sorted.z"), T, experts, groups, keep, top, ids.data_ptr(),
-                                                                wts.data_ptr(), offs.data_ptr(), src.data_ptr(), place.data_ptr(), tiles.data_ptr(),
-                                                                2 if chosen else 1 if sigmoid else 0, int(group_top), float(scale), _stream()), "hy_moe_route_align")
+    args = (z.data_ptr(), _rows(z, "moe_route_sorted.z"), T, experts, groups, keep, top, ids.data_ptr(), wts.data_ptr(), offs.data_ptr(), src.data_ptr(), place.data_ptr(),
+            tiles.data_ptr(), 2 if chosen else 1 if sigmoid else 0, int(group_top), float(scale))
+    if many:
+        _C.check_hybrid(_C.hybrid_lib().mi355_hy_moe_route_sorted(*args, *_ahead(ahead, "moe_route_sorted.ahead"), _stream()), "hy_moe_route_sorted")
+    else:
+        _C.check_hybrid(_C.hybrid_lib().mi355_hy_moe_route_align_ex(*args, _stream()), "hy_moe_route_align")
     return ids, wts, offs, src, place, tiles
 
 

@@ -795,10 +795,12 @@ class RoutedExperts:
             logits = hops.dense_linear(h, self.w_router, out_dtype=torch.float32)
             if self.shared_gated:
                 logits, sgate = logits[:, :self.n_router], logits[:, self.n_router]
+        most = logits.shape[0] * r.top >= 4 * r.experts      # nearly every expert will have rows (98 % under even routing): their weights are read ahead
         ids, wts, offs, src, place, tiles = hops.moe_route_sorted(logits, r.experts, r.groups, r.keep, r.top, sigmoid=r.score == "sigmoid", chosen=r.score == "softmax_chosen",
-                                                                  group_top=r.group_top, scale=r.scale)
+                                                                  group_top=r.group_top, scale=r.scale, ahead=self.w_gate_up if most else None)
         n = ids.numel()
-        a = hops.dense_grouped(h, self.w_gate_up, offs=offs, gather=src, tiles=tiles, rows=n, gated=self.gated, act=self.act, act_param=self.act_param)
+        a = hops.dense_grouped(h, self.w_gate_up, offs=offs, gather=src, tiles=tiles, rows=n, gated=self.gated, act=self.act, act_param=self.act_param,
+                               ahead=self.w_down if most else None)
         y = hops.dense_grouped(a, self.w_down, offs=offs, tiles=tiles, rows=n, out_dtype=torch.float32)
         parts = hops.MoeSum(y, place, wts, self.shared.forward(h) if self.shared is not None else None, sgate)
         if self.shared_gated and not defer:
