@@ -421,14 +421,14 @@ constexpr PrefillCost kPrefillCost[3][kPrefillShapeCount] = {
 };
 // The same for the shapes that do not slice K, in the loop without branches and with the tiles dealt in bands, per operand class: fp16 W4, fp16 and bf16 8 bits, 16-bit weights
 // (bf16 W4: as above).  One round of blocks takes `lat`, however few they are.  These shapes choose among each other only: whether K is sliced stays with the table above, so
-// that a call's sums keep their order.  Fitted to 290 random calls of M = 65..4096: the pick takes 1.003 of the fastest shape's time on average, at worst 1.09, where
-// the table above took 1.024 and 1.2 (8 bits, 4608 x 3584 at 1055 rows: 52 -> 45 us).
+// that a call's sums keep their order.  Fitted to times and picks of 290 random calls of M = 65..4096: the pick takes 1.004 of the fastest shape's time on average, at worst 1.09,
+// where the table above took 1.024 and 1.2 (8 bits, 4608 x 3584 at 1055 rows: 52 -> 45 us).
 constexpr int kWholeShapes = 4;
 constexpr PrefillCost kWholeCost[4][kWholeShapes] = {
-    {{3.17, 3.99}, {1.74, 2.19}, {0.92, 1.114}, {0.58, 0.607}},
-    {{3.41, 3.93}, {1.75, 2.11}, {0.86, 1.12},  {0.69, 0.62}},
-    {{1e9, 1e9},   {1.66, 1.90}, {1.40, 1.01},  {0.78, 0.522}},
-    {{1e9, 1e9},   {1.99, 2.24}, {0.95, 1.133}, {0.43, 0.601}},
+    {{3.12, 3.94}, {1.81, 2.08}, {1.10, 1.087}, {0.62, 0.635}},
+    {{3.16, 3.40}, {1.69, 1.81}, {1.01, 0.997}, {0.70, 0.583}},
+    {{1e9, 1e9},   {2.07, 2.28}, {1.27, 1.213}, {0.75, 0.668}},
+    {{1e9, 1e9},   {1.94, 2.65}, {0.89, 1.368}, {0.56, 0.737}},
 };
 int pick_among(const PrefillCost* cost, int first, int count, bool round, int M, int NT, int KC, double* t_best) {
     int best = 1;
