@@ -45,13 +45,16 @@ __device__ __forceinline__ void store_bf16(const GemmParams& p, f32x4 v, int m, 
 // of tiles in an order of bands of up to PF_BAND row tiles, column by column: per chunk 4 column tiles and 8 row tiles, a quarter of the bytes.  Column counts that eight
 // divides stay in rows: there an XCD has its columns to itself anyway, and their weights stay in its L2 from one row tile to the next (72 columns 1.6 % faster so, 32
 // columns 2 to 3 %).  us in rows / in bands: 8 bits 37888 x 3584 at 1055 rows 300 / 266, W4 at 4096 rows 1005 / 985, W16 11008 x 4096 at 2667 rows 418 / 315, 896 x 4864 at
-// 1753 rows 42 / 36; 110 random calls 0.97 of the time in rows; bands of 6, 8 and 12 alike, 24 1 % slower.
+// 1753 rows 42 / 36; 110 random calls 0.97 of the time in rows; bands of 6, 8 and 12 alike, 24 1 % slower.  Tiles that stay in rows are the launch's own blocks: the divisions that
+// find a tile stand in front of a block's first load, 0.9 us of 15.
 constexpr int PF_XCD = 8, PF_BAND = 8;
-__host__ __device__ __forceinline__ void prefill_tile(int id, int rows, int cols, int& bx, int& by) {
-    if (cols % PF_XCD == 0) { bx = id % cols; by = id / cols; return; }
+int prefill_band(int rows, int cols) {                        // 0: in rows; else the height of all bands but the last
+    const int bands = (rows + PF_BAND - 1) / PF_BAND;
+    return cols % PF_XCD == 0 ? 0 : (rows + bands - 1) / bands;
+}
+__host__ __device__ __forceinline__ void prefill_tile(int id, int rows, int cols, int band, int& bx, int& by) {
     const int nb = rows * cols, k = id % PF_XCD, j = k * (nb / PF_XCD) + (k < nb % PF_XCD ? k : nb % PF_XCD) + id / PF_XCD;
-    const int bands = (rows + PF_BAND - 1) / PF_BAND, band = (rows + bands - 1) / bands;      // of even height
-    const int r0 = j / (band * cols) * band, i = j - r0 * cols, h = band < rows - r0 ? band : rows - r0;
+    const int r0 = band >= rows ? 0 : j / (band * cols) * band, i = j - r0 * cols, h = band < rows - r0 ? band : rows - r0;
     bx = i / h; by = r0 + i % h;
 }
 
@@ -84,7 +87,7 @@ __device__ __forceinline__ void pace(int i0, int n) {         // the order of fr
     }
 }
 template <int WBITS, int GS, bool BF, int MB, int TPW, int KS, bool WHOLE>
-__global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p, const int rows, const int cols) {
+__global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p, const int band) {
     constexpr int BM = 16 * MB, NWN = 8 / KS;                 // rows, waves side by side
     constexpr int LPC  = WBITS / 4;
     constexpr int NSUB = (GS > 0) ? 4 / GS : 1;
@@ -103,8 +106,8 @@ __global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBIT
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave / NWN;
     const int jj = lane & 15, q = lane >> 4;
-    int bx, by;
-    prefill_tile((int)blockIdx.x, rows, cols, bx, by);
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (band) prefill_tile(by * (int)gridDim.x + bx, gridDim.y, gridDim.x, band, bx, by);
     const int m0 = by * BM;
     const int nt_base = (bx * NWN + wave % NWN) * TPW;
     const int KC = p.KC;
@@ -452,19 +455,21 @@ int pick_shape(int M, int NT, int KC, bool bf, int wbits, double* t_best) {
 
 // The loop without branches where x allows it.  Not for 128 x 512 under groups of 32 or 64 (two or four scales a chunk and tile have no registers left), nor for 64 x 256
 // in groups of 32 and the 64-row forms of bf16 W4 (held in one piece the compiler takes more than 128 or 80 registers for them and a block less fits a CU: 37888 x 3584 at
-// 4096 rows 1293 -> 1485 us).  K below 2^23: the 128 x 512 form's row offsets are formed past the last row, in 32 bits.
+// 4096 rows 1293 -> 1485 us), nor for 4-bit weights under sliced K (8 or 16 products and 56 operand instructions a wave and chunk: 2 % either way, 3584 x 18944 at 104 rows
+// 59 -> 60 to 62 us).  K below 2^23: the 128 x 512 form's row offsets are formed past the last row, in 32 bits.
 template <int WBITS, int GS, bool BF, int I>
 void launch_shape_t(const GemmParams& p, hipStream_t st) {
     constexpr PrefillShape s = kPrefillShapes[I];
-    const int rows = cdiv(p.M, 16 * s.mb), cols = cdiv(p.NT, 8 / s.ks * s.tpw);
-    constexpr bool straight = !(I == 0 && (GS == 1 || GS == 2)) && !(I == 2 && GS == 1) && !(BF && WBITS == 4 && s.mb == 4 && s.ks == 1);
+    const dim3 grid(cdiv(p.NT, 8 / s.ks * s.tpw), cdiv(p.M, 16 * s.mb));
+    const int band = prefill_band(grid.y, grid.x);
+    constexpr bool straight = !(I == 0 && (GS == 1 || GS == 2)) && !(I == 2 && GS == 1) && !(BF && WBITS == 4 && s.mb == 4) && !(WBITS == 4 && s.ks > 1);
     if constexpr (straight) {
         if ((uintptr_t)p.x % 16 == 0 && p.K % 128 == 0 && p.K < 1 << 23) {
-            hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, true>), dim3(rows * cols), dim3(512), 0, st, p, rows, cols);
+            hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, true>), grid, dim3(512), 0, st, p, band);
             return;
         }
     }
-    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, false>), dim3(rows * cols), dim3(512), 0, st, p, rows, cols);
+    hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, false>), grid, dim3(512), 0, st, p, band);
 }
 template <int WBITS, int GS, bool BF>
 int launch_shape(int i, const GemmParams& p, hipStream_t st) {
@@ -486,8 +491,8 @@ int launch_shape(int i, const GemmParams& p, hipStream_t st) {
 
 // The tile that block id of a rows x cols grid of tiles takes: column tile in the low half, row tile in the high half (for the tests: every tile once).
 extern "C" int64_t mi355_gemm_prefill_tile(int32_t id, int32_t rows, int32_t cols) {
-    int bx, by;
-    prefill_tile(id, rows, cols, bx, by);
+    int bx = id % cols, by = id / cols;
+    if (const int band = prefill_band(rows, cols)) prefill_tile(id, rows, cols, band, bx, by);
     return (int64_t)by << 32 | bx;
 }
 
