@@ -920,8 +920,25 @@ void skinny_form(int M, int K, long long blocks, L&& launch) {
     else if (blocks <= 256)                    rows(std::integral_constant<int, 1024>{}, std::integral_constant<int, 3>{});
     else                                       rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 3>{});
 }
-// M of 2 to 16, p.vec
+// The DMA form adds 32-bit byte offsets to the first row of x and of a block's weight rows.  Rows of x further apart than that reaches (15 steps of 143 million elements: the last tokens of eight
+// sequences of 131072 x 2048) go in launches of fewer rows, the same bits; a K that the 35 rows between a gate and the last up row of a block do not reach has no such form.
+constexpr long long SK_REACH = 0xFFFFFFFFll - 2 * 1024;                        // in front of a stage's columns
+bool skinny_weight_reach(int K) { return 35ll * K * 2 <= SK_REACH; }
+int skinny_rows_reach(int ldx) { return (int)(SK_REACH / (2ll * ldx)) + 1; }
+// M of 2 to 16, p.vec, skinny_weight_reach
 void launch_skinny(const DenseParams& p, hipStream_t st) {
+    const int reach = skinny_rows_reach(p.ldx);
+    if (p.M > reach) {
+        for (int m = 0; m < p.M; m += reach) {
+            DenseParams q = p;
+            q.M = p.M - m < reach ? p.M - m : reach;
+            q.x = (const bf16*)p.x + (size_t)m * p.ldx;
+            q.y = (char*)p.y + (size_t)m * p.ldy * (p.out_f32 ? 4 : 2);
+            if (p.egate) q.egate = p.egate + (size_t)m * p.ldg;
+            launch_skinny(q, st);
+        }
+        return;
+    }
     if (skinny_short(p.K, (long long)p.N * p.G)) {
         const int b = ((p.gated ? p.N / 2 : p.N) + 15) / 16;
         if (p.gated) hipLaunchKernelGGL(dense_skinny_short_kernel<true>, dim3(b, p.G), dim3(256), 0, st, p);
@@ -985,7 +1002,7 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
     p.G = 1; p.xs = p.ws = p.ys = 0; p.offs = nullptr; p.gather = nullptr; p.tiles = nullptr; p.egate = nullptr; p.ldg = p.goff = 0;
     (void)es;
     hipStream_t st = (hipStream_t)stream;
-    if (bf && M > 1 && M <= 16 && p.vec) {
+    if (bf && M > 1 && M <= 16 && p.vec && skinny_weight_reach(K)) {
         launch_skinny(p, st);
         MI355_CHECK_LAUNCH("dense_skinny_bf16_kernel");
         return MI355_OK;
@@ -1007,7 +1024,7 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
     return MI355_OK;
 }
 
-// Two linears of bf16 rows in one launch, arguments as in mi355_dense_linear_ex each (M of 2 to 16 rows, whole 16-byte pieces): the results are those of two calls, bit for bit.
+// Two linears of bf16 rows in one launch, arguments as in mi355_dense_linear_ex each (M of 2 to 16 rows, whole 16-byte pieces, rows within reach of 32-bit offsets): the results are those of two calls, bit for bit.
 // MI355_ERR_UNSUPPORTED: other forms, which take two calls.
 extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream_t stream) {
     MI355_CHECK_ARG(a, "dense_linear_pair: null arguments");
@@ -1017,7 +1034,7 @@ extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream
         MI355_CHECK_ARG(d.x && d.w && d.y && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && (!d.gated || d.N % 64 == 0) && d.ldy >= (d.gated ? d.N / 2 : d.N) && d.act >= 0 &&
                             d.act <= DN_ACT_RELU2 && (d.act != DN_ACT_SWIGLU_CLAMP || (d.gated && d.act_param > 0.f)),
                         "dense_linear_pair: M=%d N=%d K=%d ldx=%d ldy=%d gated=%d act=%d", d.M, d.N, d.K, d.ldx, d.ldy, d.gated, d.act);
-        if (d.M < 2 || d.M > 16 || d.K % 8 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16) return MI355_ERR_UNSUPPORTED;
+        if (d.M < 2 || d.M > 16 || d.K % 8 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16 || !skinny_weight_reach(d.K) || d.M > skinny_rows_reach(d.ldx)) return MI355_ERR_UNSUPPORTED;
         DenseParams& q = p[i];
         q.x = d.x; q.w = d.w; q.bias = d.bias; q.y = d.y; q.M = d.M; q.N = d.N; q.K = d.K; q.ldx = d.ldx; q.ldy = d.ldy;
         q.gated = d.gated; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
@@ -1090,7 +1107,7 @@ extern "C" int mi355_dense_grouped_ahead(const void* x, int32_t ldx, int32_t M, 
         return MI355_OK;
     }
     if (!offs && M <= 16) {                    // a decode step's rows through every group: the kernels of the plain linear, groups in the grid
-        if (bf && M > 1 && p.vec) {
+        if (bf && M > 1 && p.vec && skinny_weight_reach(K)) {
             launch_skinny(p, st);
             MI355_CHECK_LAUNCH("dense_skinny_bf16_kernel");
             return MI355_OK;

@@ -57,3 +57,21 @@ def test_few_rows_forms(N, K):
         assert torch.equal(hops.dense_linear(x[:M], w, out_dtype=torch.float32), y[:M]) and torch.equal(a, y[:M]) and torch.equal(b, gated[:M]), M
     a, b = hops.dense_pair(dict(x=x2, w=w2, gated=True, act=hops.ACT_SILU), dict(x=x, w=w, out_dtype=torch.float32))
     assert torch.equal(a, gated) and torch.equal(b, y)
+
+
+@pytest.mark.parametrize("M,ldx", [(3, 1 << 30), (16, 143165608), (9, (1 << 29) + 8)])
+def test_few_rows_far_apart(M, ldx):
+    """Rows of x whose offsets do not fit 32 bits: the bits of the same rows side by side, alone, in a launch of two and through groups."""
+    K, g = 1032, torch.Generator(device=DEV).manual_seed(M)
+    flat = torch.empty((M - 1) * ldx + 2 * K, dtype=torch.bfloat16, device=DEV)
+    far, x = flat.as_strided((M, 2 * K), (ldx, 1)), torch.randn(M, 2 * K, device=DEV, generator=g).bfloat16()
+    far.copy_(x)
+    w, wg = (torch.randn(*s, device=DEV, generator=g).bfloat16() * K ** -0.5 for s in ((72, K), (64, K)))
+    for a, b in ((x[:, :K], far[:, :K]), (x[:, K:], far[:, K:])):
+        for out in (torch.float32, torch.bfloat16):
+            assert torch.equal(hops.dense_linear(b, w, out_dtype=out), hops.dense_linear(a, w, out_dtype=out))
+        want = [hops.dense_linear(a, wg, gated=True, act=hops.ACT_SILU), hops.dense_linear(a, w)]
+        assert all(torch.equal(p, q) for p, q in zip(hops.dense_pair(dict(x=b, w=wg, gated=True, act=hops.ACT_SILU), dict(x=b, w=w)), want))
+    w2, gate = torch.stack([w, w.flip(0)]), torch.randn(M, 2 * 72, device=DEV, generator=g)
+    run = lambda v: hops.dense_grouped(v, w2, x_step=K, y_step=72, mul_sigmoid=gate)
+    assert torch.equal(run(far), run(x))
