@@ -89,13 +89,19 @@ __device__ __forceinline__ DnGroup dn_group(const DenseParams& p, int tile_rows)
 
 // A block past the list of tiles (of one group only in z): its share of the lines of p.ahead, four loads at a time.  The list is bounded by rows / 64 + groups tiles, so about half
 // as many rows of blocks as there are groups are left over, and they run while the launch multiplies and HBM is idle: 16 experts 1024 -> 704 -> 1024 over 6148 rows, the second linear
-// 31.6 -> 24.2 us, the first no slower.
+// 31.6 -> 24.2 us, the first no slower.  They are dealt last, and of few experts there may be one row of them or none, so a thread reads DN_AHEAD_ROUNDS times four lines and no more: shared
+// out over however many blocks are left, one row of 16 read 3 MB a CU behind a finished product (64 experts of 384, 364 pairs: sort and linears 49.7 us without, 66.7 so, 51.2 so bounded).
+constexpr int DN_AHEAD_ROUNDS = 4;
 __device__ __forceinline__ void dn_read_ahead(const DenseParams& p) {
     const uint32_t used = gridDim.x * (uint32_t)p.tiles[0], n = (gridDim.x * gridDim.y - used) * blockDim.x;
-    for (uint32_t i = (blockIdx.y * gridDim.x + blockIdx.x - used) * blockDim.x + threadIdx.x; i < p.ahead_lines; i += 4 * n) {
+    const uint32_t first = (blockIdx.y * gridDim.x + blockIdx.x - used) * blockDim.x + threadIdx.x;
+    for (int r = 0; r < DN_AHEAD_ROUNDS; ++r) {
         uint32_t v[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = i + k * n < p.ahead_lines ? *(const uint32_t*)(p.ahead + (size_t)(i + k * n) * 128) : 0u;
+        for (int k = 0; k < 4; ++k) {
+            const uint64_t i = first + (uint64_t)(4 * r + k) * n;
+            v[k] = i < p.ahead_lines ? *(const uint32_t*)(p.ahead + i * 128) : 0u;
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k) asm volatile("" :: "v"(v[k]));
     }
@@ -1071,7 +1077,7 @@ extern "C" int mi355_dense_grouped_ex(const void* x, int32_t ldx, int32_t M, con
                                      nullptr, 0, stream);
 }
 
-// The same, and a weight that a later launch streams (ahead_bytes of ahead; at most 48 MB of it): read by blocks past the list of tiles.
+// The same, and a weight that a later launch streams (ahead_bytes of ahead; at most 48 MB of it, and 2 KB a thread): read by blocks past the list of tiles.
 extern "C" int mi355_dense_grouped_ahead(const void* x, int32_t ldx, int32_t M, const void* w, int32_t N, int32_t K, const void* bias, void* y,
                                          int32_t ldy, int32_t out_f32, int32_t gated, int32_t act, float act_param, int32_t act_dtype, int32_t G,
                                          int64_t xs, int64_t ys, const int32_t* offs, const int32_t* gather, const int32_t* tiles, int32_t max_tiles,
