@@ -94,14 +94,12 @@ __device__ __forceinline__ DnGroup dn_group(const DenseParams& p, int tile_rows)
 constexpr int DN_AHEAD_ROUNDS = 4;
 __device__ __forceinline__ void dn_read_ahead(const DenseParams& p) {
     const uint32_t used = gridDim.x * (uint32_t)p.tiles[0], n = (gridDim.x * gridDim.y - used) * blockDim.x;
-    const uint32_t first = (blockIdx.y * gridDim.x + blockIdx.x - used) * blockDim.x + threadIdx.x;
-    for (int r = 0; r < DN_AHEAD_ROUNDS; ++r) {
+    uint32_t i = (blockIdx.y * gridDim.x + blockIdx.x - used) * blockDim.x + threadIdx.x;
+#pragma unroll 1
+    for (int r = 0; r < DN_AHEAD_ROUNDS && i < p.ahead_lines; ++r, i += 4 * n) {
         uint32_t v[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint64_t i = first + (uint64_t)(4 * r + k) * n;
-            v[k] = i < p.ahead_lines ? *(const uint32_t*)(p.ahead + i * 128) : 0u;
-        }
+        for (int k = 0; k < 4; ++k) v[k] = i + k * n < p.ahead_lines ? *(const uint32_t*)(p.ahead + (size_t)(i + k * n) * 128) : 0u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) asm volatile("" :: "v"(v[k]));
     }

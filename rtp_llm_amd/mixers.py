@@ -748,12 +748,12 @@ class RouterSpec:
     scale: float = 1.0                   # the chosen experts weigh score * scale
 
 
-def reads_ahead(pairs: int, experts: int, nbytes: int) -> bool:
-    """Is a weight of all experts read into the memory-side cache ahead of its grouped linear?  Where nearly every expert will have rows (98 % under even routing), the sort of the (token,
-    choice) pairs is long enough to read behind, and the weight is read whole.  Sort and both linears, weights from memory, time with / without the reads: 39 layers inside these lines 0.92
-    (0.83 to 1.02); 80 of fewer than 1000 pairs 1.12, at worst 1.32 (the spare blocks outlast a short sort by 3 us), 55 of 1000 to 2000 1.03, 50 of 2000 to 4096 0.99 (0.84 to 1.15); 11 whose
+def ahead_from(experts: int, nbytes: int) -> float:
+    """The (token, choice) pairs from which a weight of all experts is read into the memory-side cache ahead of its grouped linear: where nearly every expert will have rows (98 % under even
+    routing), the sort of the pairs is long enough to read behind, and the weight is read whole.  Sort and both linears, weights from memory, time with / without the reads: 39 layers inside
+    these lines 0.92 (0.83 to 1.02); 80 of fewer than 1000 pairs 1.12, at worst 1.32 (the spare blocks outlast a short sort by 3 us), 55 of 1000 to 2000 1.03, 50 of 2000 to 4096 0.99 (0.84 to 1.15); 11 whose
     weight is over 96 MB, of which 48 are read, 1.01."""
-    return pairs >= max(4096, 4 * experts) and (2 << 20) <= nbytes <= (48 << 20)
+    return max(4096, 4 * experts) if (2 << 20) <= nbytes <= (48 << 20) else float("inf")
 
 
 class RoutedExperts:
@@ -791,6 +791,7 @@ class RoutedExperts:
                 d = torch.cat([d, torch.zeros(d.shape[0], pad, dtype=d.dtype, device=d.device)], 1)
             gu.append(hops.group_gate_up(g, u) if self.gated else u); dn.append(d)
         self.w_gate_up, self.w_down = torch.stack(gu).contiguous(), torch.stack(dn).contiguous()
+        self.ahead_from = [ahead_from(r.experts, w.numel() * w.element_size()) for w in (self.w_gate_up, self.w_down)]
         self.shared, self.act, self.act_param = shared, hops.ACTIVATIONS[act], float(act_param)
 
     def forward(self, h: torch.Tensor, logits: Optional[torch.Tensor] = None, defer: bool = False):
@@ -803,11 +804,12 @@ class RoutedExperts:
             logits = hops.dense_linear(h, self.w_router, out_dtype=torch.float32)
             if self.shared_gated:
                 logits, sgate = logits[:, :self.n_router], logits[:, self.n_router]
-        ahead = [w if reads_ahead(logits.shape[0] * r.top, r.experts, w.numel() * w.element_size()) else None for w in (self.w_gate_up, self.w_down)]
+        pairs = logits.shape[0] * r.top
         ids, wts, offs, src, place, tiles = hops.moe_route_sorted(logits, r.experts, r.groups, r.keep, r.top, sigmoid=r.score == "sigmoid", chosen=r.score == "softmax_chosen",
-                                                                  group_top=r.group_top, scale=r.scale, ahead=ahead[0])
+                                                                  group_top=r.group_top, scale=r.scale, ahead=self.w_gate_up if pairs >= self.ahead_from[0] else None)
         n = ids.numel()
-        a = hops.dense_grouped(h, self.w_gate_up, offs=offs, gather=src, tiles=tiles, rows=n, gated=self.gated, act=self.act, act_param=self.act_param, ahead=ahead[1])
+        a = hops.dense_grouped(h, self.w_gate_up, offs=offs, gather=src, tiles=tiles, rows=n, gated=self.gated, act=self.act, act_param=self.act_param,
+                               ahead=self.w_down if pairs >= self.ahead_from[1] else None)
         y = hops.dense_grouped(a, self.w_down, offs=offs, tiles=tiles, rows=n, out_dtype=torch.float32)
         parts = hops.MoeSum(y, place, wts, self.shared.forward(h) if self.shared is not None else None, sgate)
         if self.shared_gated and not defer:

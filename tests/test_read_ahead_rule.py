@@ -2,7 +2,7 @@
 loses more than 3 % by it, and the ones that gain most."""
 import pytest
 
-from rtp_llm_amd.mixers import reads_ahead
+from rtp_llm_amd.mixers import ahead_from
 
 MB = 1 << 20
 # pairs, experts, MB of the gate and up weights (the down weights are half), us without / with
@@ -13,7 +13,7 @@ LAYERS = [(71, 8, 40, 32.0, 40.4), (131 * 2, 16, 82, 48.0, 56.9), (186, 8, 36, 3
 
 @pytest.mark.parametrize("pairs,experts,mb,off,on", LAYERS)
 def test_read_ahead_rule(pairs, experts, mb, off, on):
-    takes = reads_ahead(pairs, experts, int(mb * MB)), reads_ahead(pairs, experts, int(mb * MB / 2))
+    takes = pairs >= ahead_from(experts, int(mb * MB)), pairs >= ahead_from(experts, int(mb * MB / 2))
     if on > 1.03 * off:
         assert not takes[0] and (not takes[1] or mb > 96)
     if on < 0.95 * off and pairs >= 4096:
@@ -21,5 +21,5 @@ def test_read_ahead_rule(pairs, experts, mb, off, on):
 
 
 def test_read_ahead_edges():
-    assert reads_ahead(4096, 16, 2 * MB) and reads_ahead(4096, 1024, 48 * MB)
-    assert not reads_ahead(4095, 16, 2 * MB) and not reads_ahead(4099, 1025, 48 * MB) and not reads_ahead(4096, 16, 2 * MB - 1) and not reads_ahead(4096, 16, 48 * MB + 1)
+    assert ahead_from(16, 2 * MB) == 4096 and ahead_from(1025, 48 * MB) == 4100
+    assert ahead_from(16, 2 * MB - 1) == ahead_from(16, 48 * MB + 1) == float("inf")
