@@ -733,7 +733,8 @@ void launch_rows(const DenseParams& p, hipStream_t st) {
 // One block of four waves per 8 weight rows: 8 outputs, or the gate and up rows of 4 channels.  What bounds it is how the weight comes out of memory: 8 rows of a row-major weight
 // lie side by side, and read as MFMA fragments (16 rows by 64 bytes a wave load) they came at 3.2 TB/s however the steps were ordered.  Here every wave load is one
 // row's run of 1 KB, by DMA into LDS, three stages of 512 columns; the rows of x beside them the same way, so that nothing but the fragments passes through registers.  8 weight rows a
-// block and 48 KB (M <= 8): three blocks a compute unit, 96 KB of loads in flight.  More rows a block, more waves, more or fewer stages and narrower runs are all slower.
+// block and 48 KB (M <= 8): three blocks a compute unit, 96 KB of loads in flight.  More rows a block and more waves are slower; which stages
+// pay is in skinny_form, which shapes are better off without LDS in skinny_short.
 // Weights from memory, M = 8, us before / now: 17408 x 2048 22.4 / 14.4, 32000 x 2048 35.1 / 24.3, 4096 x 2048 7.5 / 5.2, 2048 x 5632 13.6 / 6.5, 2048 x 2048 5.4 / 3.6.
 // Sums: k in steps of 32, step s into chain s mod skinny_chains (4 or 8), the chains added in order: bits that depend on N, K and G only.
 // 16-byte pieces are permuted by the row (applied to the source address), so that the 8 or 16 rows of a fragment read hit different banks.
@@ -840,11 +841,11 @@ __global__ __launch_bounds__(256) void dense_skinny_pair_kernel(DenseParams p0, 
     }
 }
 
-// Short K through many outputs: a block of 8 weight rows would end before it has begun, so 16 outputs a block, fragments straight from memory, the four waves a chain each: the same sums.
-typedef f32x4 SkinnySums[4][2][64];
-template <bool GATED>
-__device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, int bx, int grp, SkinnySums& red) {
-    constexpr int NW = 4, U = 4;
+// Short K through many outputs: a block of 8 weight rows would end before it has begun, so 16 outputs a block, fragments straight from memory, a wave for each of the NW chains: the same sums.
+template <int NW> struct SkinnySums { f32x4 at[NW][2][64]; };
+template <bool GATED, int NW>
+__device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, int bx, int grp, SkinnySums<NW>& red) {
+    constexpr int U = 4;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nout = GATED ? p.N / 2 : p.N;
     const int r = lane & 15, kq = (lane >> 4) * 8, o = min(bx * 16 + r, nout - 1), n = GATED ? (o >> 5) * 64 + (o & 31) : o;
     const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kq;
@@ -868,13 +869,13 @@ __device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, in
             if (GATED) au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], c[u], au, 0, 0, 0);
         }
     }
-    red[wave][0][lane] = ag;
-    if (GATED) red[wave][1][lane] = au;
+    red.at[wave][0][lane] = ag;
+    if (GATED) red.at[wave][1][lane] = au;
     __syncthreads();
     if (wave != 0) return;
     for (int w = 1; w < NW; ++w) {
-        ag += red[w][0][lane];
-        if (GATED) au += red[w][1][lane];
+        ag += red.at[w][0][lane];
+        if (GATED) au += red.at[w][1][lane];
     }
     if (bx * 16 + r >= nout) return;
 #pragma unroll
@@ -886,20 +887,24 @@ __device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, in
         dn_store<bf16>(p, row, (int)(p.ys * grp) + bx * 16 + r, GATED ? dn_gated(g, u, p.act, p.act_param) : dn_act(g, p.act));
     }
 }
-template <bool GATED>
-__global__ __launch_bounds__(256) void dense_skinny_short_kernel(DenseParams p) {
-    __shared__ SkinnySums red;
-    dense_skinny_short_tile<GATED>(p, blockIdx.x, blockIdx.y, red);
+template <bool GATED, int NW>
+__global__ __launch_bounds__(64 * NW) void dense_skinny_short_kernel(DenseParams p) {
+    __shared__ SkinnySums<NW> red;
+    dense_skinny_short_tile<GATED, NW>(p, blockIdx.x, blockIdx.y, red);
 }
-template <bool GATED0, bool GATED1>
-__global__ __launch_bounds__(256) void dense_skinny_short_pair_kernel(DenseParams p0, DenseParams p1, int blocks0) {
-    __shared__ SkinnySums red;
-    if ((int)blockIdx.x < blocks0) dense_skinny_short_tile<GATED0>(p0, blockIdx.x, 0, red);
-    else                           dense_skinny_short_tile<GATED1>(p1, blockIdx.x - blocks0, 0, red);
+template <bool GATED0, bool GATED1, int NW>
+__global__ __launch_bounds__(64 * NW) void dense_skinny_short_pair_kernel(DenseParams p0, DenseParams p1, int blocks0) {
+    __shared__ SkinnySums<NW> red;
+    if ((int)blockIdx.x < blocks0) dense_skinny_short_tile<GATED0, NW>(p0, blockIdx.x, 0, red);
+    else                           dense_skinny_short_tile<GATED1, NW>(p1, blockIdx.x - blocks0, 0, red);
 }
-// us in the form above / in this one: 16 x 6720 gated x 872 7.2 / 6.4, 8 x 8706 x 584 5.6 / 5.2, 12 x 13952 x 232 6.3 / 4.2, two groups of 2519 x 80 3.1 / 2.9; below the line 9 x 3648 gated x 64
-// 3.2 / 3.3, 8 x 3090 x 344 3.9 / 3.8.
-bool skinny_short(int K, long long weight_rows) { return K < 1024 && weight_rows > 4096; }
+// Where that form is taken.  It has no stages to fill and half the blocks, but its wave loads are 16 rows by 64 bytes, which the weights' stream of long K pays for.  Random calls of 2 to 16 rows,
+// us of the DMA form / this one, weights from memory: 11 x 1024 x 47616 gated 29.1 / 24.5, 10 x 1024 x 22784 gated 16.4 / 13.1, 16 x 6720 gated x 872 7.2 / 6.4; read again and again from the
+// memory-side cache: 11 x 1352 x 34880 22.8 / 18.8, 7 x 1048 x 9344 8.3 / 6.9, 2 x 1176 x 4096 5.1 / 4.4; past the lines, from memory: 11 x 1728 x 10368 gated 13.0 / 14.0,
+// 12 x 1832 x 4224 8.3 / 9.5, 4 x 2048 x 30464 22.8 / 29.6, 5 x 2000 x 4160 7.4 / 8.3.
+bool skinny_short(int M, int K, long long weight_rows) {
+    return (K <= 1152 && weight_rows >= 6144) || (K <= (M > 4 ? 1792 : 1280) && weight_rows >= (M > 8 ? 12288 : 4096));
+}
 
 // The partial sums that K is split into (part of a result's bits): eight, four of many outputs or short K.
 int skinny_chains(const DenseParams& p) { return (((p.gated ? p.N / 2 : p.N) + 15) / 16) * p.G >= 1024 || p.K < 1024 ? 4 : 8; }
@@ -909,9 +914,14 @@ int skinny_blocks(const DenseParams& p) { return (p.N + SK_RB - 1) / SK_RB; }
 bool skinny_nt(size_t weights) { return weights * 2 >= (size_t)24 << 20; }
 
 // launch(form) with the form for M rows of K columns (the shorter of two) in `blocks` blocks.  As few rows of x staged as there are: they come from the L2, but pass through the same loads
-// as the weights (32000 x 2048 with 4 / 8 / 16: 21.2 / 24.3 / 28.6 us).  Stages of half the columns, and so more blocks a compute unit, for short K, of which a stage of 512 would be
-// mostly empty, and for 9 to 16 rows in many blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2).  Stages of twice the columns, half the barriers, where no compute unit
-// has a second block to hide them (2 rows, 384 x 5960, six stages of 512 / three of 1024: 7.1 / 6.3).
+// as the weights (32000 x 2048 with 4 / 8 / 16: 21.2 / 24.3 / 28.6 us).  Stages of 512 columns, three of them, except:
+//   stages of 256, four of them, and so more blocks a compute unit, for short K, of which a stage of 512 would be mostly empty; where many blocks would load a tenth more columns than there are with
+//   512 (a stage's loads past K cost what the others do); and for 9 to 16 rows in more than 256 blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2);
+//   stages of 1024, half the barriers, in up to 192 blocks, where no compute unit has a second block to hide them (2 rows, 384 x 5960, six stages of 512 / three of 1024: 7.1 / 6.3) and the last
+//   stage is not mostly empty.
+// 400 random calls of 2 to 16 rows, weights from memory and from the memory-side cache, time over that of the fastest of the four forms: 1.010 with these lines and skinny_short's, 1.021 with
+// stages of 256 and 1024 for K < 1024 and up to 256 blocks alone.  34 of the 800 times are more than 3 % over those of 16 outputs a block throughout, 24 of them from the memory-side cache, the
+// worst 1.14; the others are 0.5 to 1.03.
 template <class L>
 void skinny_form(int M, int K, long long blocks, L&& launch) {
     auto rows = [&](auto kc, auto ns) {
@@ -920,9 +930,10 @@ void skinny_form(int M, int K, long long blocks, L&& launch) {
         else if (M > 4 || KC < 512) launch(SkinnyForm<8, KC, NS>{});
         else if constexpr (KC >= 512) launch(SkinnyForm<4, KC, NS>{});
     };
-    if (K < 1024 || (M > 8 && blocks >= 1024)) rows(std::integral_constant<int, 256>{}, std::integral_constant<int, 4>{});
-    else if (blocks <= 256)                    rows(std::integral_constant<int, 1024>{}, std::integral_constant<int, 3>{});
-    else                                       rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 3>{});
+    auto padded = [&](int kc) { return ((long long)K + kc - 1) / kc * kc; };
+    if (K < 1024 || (blocks > 256 && (M > 8 || padded(512) * 10 > padded(256) * 11))) rows(std::integral_constant<int, 256>{}, std::integral_constant<int, 4>{});
+    else if (blocks <= 192 && padded(1024) * 10 <= padded(512) * 12)                    rows(std::integral_constant<int, 1024>{}, std::integral_constant<int, 3>{});
+    else                                                                                rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 3>{});
 }
 // The DMA form adds 32-bit byte offsets to the first row of x and of a block's weight rows.  Rows of x further apart than that reaches (15 steps of 143 million elements: the last tokens of eight
 // sequences of 131072 x 2048) go in launches of fewer rows, the same bits; a K that the 35 rows between a gate and the last up row of a block do not reach has no such form.
@@ -943,26 +954,32 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         }
         return;
     }
-    if (skinny_short(p.K, (long long)p.N * p.G)) {
-        const int b = ((p.gated ? p.N / 2 : p.N) + 15) / 16;
-        if (p.gated) hipLaunchKernelGGL(dense_skinny_short_kernel<true>, dim3(b, p.G), dim3(256), 0, st, p);
-        else         hipLaunchKernelGGL(dense_skinny_short_kernel<false>, dim3(b, p.G), dim3(256), 0, st, p);
+    const bool eight = skinny_chains(p) == 8;
+    if (skinny_short(p.M, p.K, (long long)p.N * p.G)) {
+        const dim3 grid(((p.gated ? p.N / 2 : p.N) + 15) / 16, p.G), block(eight ? 512 : 256);
+        if (eight) { if (p.gated) hipLaunchKernelGGL((dense_skinny_short_kernel<true, 8>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_short_kernel<false, 8>), grid, block, 0, st, p); }
+        else       { if (p.gated) hipLaunchKernelGGL((dense_skinny_short_kernel<true, 4>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_short_kernel<false, 4>), grid, block, 0, st, p); }
         return;
     }
     const dim3 grid(skinny_blocks(p), p.G), block(256);
-    const bool nt = skinny_nt((size_t)p.N * p.K * p.G), eight = skinny_chains(p) == 8;
+    const bool nt = skinny_nt((size_t)p.N * p.K * p.G);
     skinny_form(p.M, p.K, (long long)grid.x * grid.y, [&](auto f) {
         using F = decltype(f);
         if (eight) { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, false>), grid, block, 0, st, p); }
         else       { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, false>), grid, block, 0, st, p); }
     });
 }
+template <int NW>
+void launch_skinny_short_pair(const DenseParams (&p)[2], hipStream_t st) {
+    const int s0 = ((p[0].gated ? p[0].N / 2 : p[0].N) + 15) / 16, s1 = ((p[1].gated ? p[1].N / 2 : p[1].N) + 15) / 16;
+    const dim3 grid(s0 + s1), block(64 * NW);
+    if (p[0].gated) { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, true, NW>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, false, NW>), grid, block, 0, st, p[0], p[1], s0); }
+    else            { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, true, NW>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, false, NW>), grid, block, 0, st, p[0], p[1], s0); }
+}
 void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
-    if (skinny_short(p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N)) {
-        const int s0 = ((p[0].gated ? p[0].N / 2 : p[0].N) + 15) / 16, s1 = ((p[1].gated ? p[1].N / 2 : p[1].N) + 15) / 16;
-        const dim3 grid(s0 + s1), block(256);
-        if (p[0].gated) { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, true>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, false>), grid, block, 0, st, p[0], p[1], s0); }
-        else            { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, true>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, false>), grid, block, 0, st, p[0], p[1], s0); }
+    const int chains = skinny_chains(p[0]);
+    if (skinny_chains(p[1]) == chains && skinny_short(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N)) {
+        if (chains == 8) launch_skinny_short_pair<8>(p, st); else launch_skinny_short_pair<4>(p, st);
         return;
     }
     const int b0 = skinny_blocks(p[0]), b1 = skinny_blocks(p[1]), c0 = skinny_chains(p[0]), c1 = skinny_chains(p[1]);

@@ -41,10 +41,12 @@ def test_few_rows_through_every_group():
     assert float((y - ref).abs().max()) <= 2.0 ** -17 * 128 * 4
 
 
-@pytest.mark.parametrize("N,K", [(2048, 1016), (2048, 1024), (2050, 1032), (4096, 1016), (4097, 1016), (8184, 1024), (8200, 1160), (6152, 2056), (6136, 2048), (64, 5640)])
+@pytest.mark.parametrize("N,K", [(2048, 1016), (2048, 1024), (2050, 1032), (4096, 1016), (4097, 1016), (8184, 1024), (8200, 1160), (6152, 2056), (6136, 2048), (64, 5640),
+                                 (6144, 1152), (6136, 1152), (6144, 1160), (4096, 1280), (4096, 1288), (4088, 1280), (4096, 1792), (4096, 1800), (12288, 1792), (12280, 1792), (16400, 1024), (16384, 1792),
+                                 (1536, 2048), (1544, 2048), (1536, 1032), (2048, 1056), (2056, 1056), (2056, 1288)])
 def test_few_rows_forms(N, K):
-    """Either side of each rule that picks stages, columns of a stage and rows of a block (K 1024, 256 and 1024 blocks, 4096 weight rows, 24 MB), a last stage with one piece: against a
-    64-bit product, the same bits for any number of rows, alone and in a launch of two."""
+    """Either side of each rule that picks the form (K 1024, 1152, 1280, 1792; 4096, 6144, 12288 weight rows; four chains and eight), stages and columns of a stage (192 and 256 blocks, columns
+    loaded for nothing, 24 MB), a last stage with one piece: against a 64-bit product, the same bits for any number of rows, alone and in a launch of two."""
     g = torch.Generator(device=DEV).manual_seed(N + K)
     x, w = torch.randn(16, K, device=DEV, generator=g).bfloat16(), (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
     x2, w2 = torch.randn(16, 72, device=DEV, generator=g).bfloat16(), torch.randn(64, 72, device=DEV, generator=g).bfloat16()
