@@ -19,6 +19,9 @@ extern "C" {
  * per-head output gates and normed queries and keys, a generalized delta-rule recurrence, hashed bigram embedding rows, a weighted
  * average over the depth of the stack).  act_dtype is MI355_ACT_BF16 or MI355_ACT_F32.  Sources: csrc/gemm_dense.hip,
  * csrc/hybrid_ops.hip; the argument conventions are documented at the definitions. */
+/* With `gated` of the dense linears: the weight is one of more than the 256 MB memory-side cache holds from one use to the next; the kernels of 2 to 16 bf16 rows then read it past the
+ * caches where a launch reads 24 MB or more. */
+enum { MI355_DENSE_STREAMED = 1 << 30 };
 int mi355_dense_linear(const void* x, int32_t ldx, int32_t M, const void* w, int32_t N, int32_t K, const void* bias, void* y, int32_t ldy,
                        int32_t out_f32, int32_t gated, int32_t act, float softcap, int32_t act_dtype, mi355_stream_t stream);
 int mi355_hy_embed(const int32_t* ids, int32_t rows, const void* table, int32_t W, int32_t vocab, float* out, int32_t act_dtype, mi355_stream_t stream);

@@ -38,6 +38,7 @@ struct DenseParams {
     const void* x; const void* w; const void* bias; void* y;
     int M, N, K, ldx, ldy;
     int gated;       // 0: N outputs; 1: rows of w are [32 gate | 32 up] groups, N / 2 outputs
+    int streamed;    // MI355_DENSE_STREAMED
     int act;         // DN_ACT_* applied to the gate
     float act_param; // DN_ACT_SWIGLU_CLAMP: the limit of the gate (from above) and of the up value (both sides)
     int out_f32;
@@ -909,9 +910,10 @@ bool skinny_short(int M, int K, long long weight_rows) {
 // The partial sums that K is split into (part of a result's bits): eight, four of many outputs or short K.
 int skinny_chains(const DenseParams& p) { return (((p.gated ? p.N / 2 : p.N) + 15) / 16) * p.G >= 1024 || p.K < 1024 ? 4 : 8; }
 int skinny_blocks(const DenseParams& p) { return (p.N + SK_RB - 1) / SK_RB; }
-// A weight that one launch reads 24 MB or more of belongs to a layer, and so to a model, that the 256 MB memory-side cache does not hold from one step to the next: it is read past the caches.
-// Weights from memory, us without / with the hint: 17408 x 2048 15.5 / 14.4, 32000 x 2048 26.5 / 24.3; in 128 MB that are read again and again 12.0 / 13.4, 19.7 / 23.0.
-bool skinny_nt(size_t weights) { return weights * 2 >= (size_t)24 << 20; }
+// A weight that the 256 MB memory-side cache does not hold from one step to the next is read past the caches where a launch reads 24 MB or more.  Only the caller knows: the same weight in a
+// small model, or under a draft's head, comes from that cache.  40 random weights of 24 to 130 MB, time with / without the hint: 0.97 (0.91 to 1.01) in a footprint of 1 GB, 0.96 in 400 MB,
+// 1.12 (0.99 to 1.37) in 256 MB, 1.10 in 128 MB.  17408 x 2048 from memory 15.5 / 14.4 us, 32000 x 2048 26.5 / 24.3; eight prompts and eight steps of a 16-layer model of width 2048 8920 / 8400 us.
+bool skinny_nt(bool streamed, size_t weights) { return streamed && weights * 2 >= (size_t)24 << 20; }
 
 // launch(form) with the form for M rows of K columns (the shorter of two) in `blocks` blocks.  As few rows of x staged as there are: they come from the L2, but pass through the same loads
 // as the weights (32000 x 2048 with 4 / 8 / 16: 21.2 / 24.3 / 28.6 us).  Stages of 512 columns, three of them, except:
@@ -962,7 +964,7 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         return;
     }
     const dim3 grid(skinny_blocks(p), p.G), block(256);
-    const bool nt = skinny_nt((size_t)p.N * p.K * p.G);
+    const bool nt = skinny_nt(p.streamed, (size_t)p.N * p.K * p.G);
     skinny_form(p.M, p.K, (long long)grid.x * grid.y, [&](auto f) {
         using F = decltype(f);
         if (eight) { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, false>), grid, block, 0, st, p); }
@@ -983,7 +985,7 @@ void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
         return;
     }
     const int b0 = skinny_blocks(p[0]), b1 = skinny_blocks(p[1]), c0 = skinny_chains(p[0]), c1 = skinny_chains(p[1]);
-    const bool nt = skinny_nt((size_t)p[0].N * p[0].K + (size_t)p[1].N * p[1].K);
+    const bool nt = skinny_nt(p[0].streamed && p[1].streamed, (size_t)p[0].N * p[0].K + (size_t)p[1].N * p[1].K);
     skinny_form(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K < p[1].K ? p[0].K : p[1].K, (long long)b0 + b1, [&](auto f) {
         using F = decltype(f);
         if (nt) hipLaunchKernelGGL((dense_skinny_pair_kernel<F, true>), dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, c0, c1);
@@ -1008,6 +1010,7 @@ extern "C" int mi355_dense_linear(const void* x, int32_t ldx, int32_t M, const v
 extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, const void* w, int32_t N, int32_t K, const void* bias,
                                      void* y, int32_t ldy, int32_t out_f32, int32_t gated, int32_t act, float act_param, float softcap,
                                      int32_t act_dtype, mi355_stream_t stream) {
+    const int streamed = (gated & MI355_DENSE_STREAMED) != 0; gated &= ~MI355_DENSE_STREAMED;
     MI355_CHECK_ARG(x && w && y && M > 0 && N > 0 && K > 0 && ldx >= K, "dense_linear: M=%d N=%d K=%d ldx=%d", M, N, K, ldx);
     MI355_CHECK_ARG(act_dtype == MI355_ACT_BF16 || act_dtype == MI355_ACT_F32, "dense_linear: act_dtype=%d (bf16 or fp32)", act_dtype);
     MI355_CHECK_ARG(!gated || N % 64 == 0, "dense_linear: gated needs N %% 64 == 0 (N=%d)", N);
@@ -1017,7 +1020,7 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
     const size_t es = bf ? 2 : 4;
     DenseParams p;
     p.x = x; p.w = w; p.bias = bias; p.y = y; p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = ldy;
-    p.gated = gated; p.act = act; p.act_param = act_param; p.out_f32 = bf ? out_f32 : 1; p.softcap = softcap;
+    p.gated = gated; p.streamed = streamed; p.act = act; p.act_param = act_param; p.out_f32 = bf ? out_f32 : 1; p.softcap = softcap;
     p.vec = (K % 8 == 0) && (ldx % 8 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
     p.yvec = (ldy % 4 == 0) && ((uintptr_t)y % (p.out_f32 ? 16 : 8) == 0);
     p.G = 1; p.xs = p.ws = p.ys = 0; p.offs = nullptr; p.gather = nullptr; p.tiles = nullptr; p.egate = nullptr; p.ldg = p.goff = 0;
@@ -1051,14 +1054,15 @@ extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream
     MI355_CHECK_ARG(a, "dense_linear_pair: null arguments");
     DenseParams p[2];
     for (int i = 0; i < 2; ++i) {
-        const mi355_dense_args_t& d = a[i];
+        mi355_dense_args_t d = a[i];
+        const int streamed = (d.gated & MI355_DENSE_STREAMED) != 0; d.gated &= ~MI355_DENSE_STREAMED;
         MI355_CHECK_ARG(d.x && d.w && d.y && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && (!d.gated || d.N % 64 == 0) && d.ldy >= (d.gated ? d.N / 2 : d.N) && d.act >= 0 &&
                             d.act <= DN_ACT_RELU2 && (d.act != DN_ACT_SWIGLU_CLAMP || (d.gated && d.act_param > 0.f)),
                         "dense_linear_pair: M=%d N=%d K=%d ldx=%d ldy=%d gated=%d act=%d", d.M, d.N, d.K, d.ldx, d.ldy, d.gated, d.act);
         if (d.M < 2 || d.M > 16 || d.K % 8 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16 || !skinny_weight_reach(d.K) || d.M > skinny_rows_reach(d.ldx)) return MI355_ERR_UNSUPPORTED;
         DenseParams& q = p[i];
         q.x = d.x; q.w = d.w; q.bias = d.bias; q.y = d.y; q.M = d.M; q.N = d.N; q.K = d.K; q.ldx = d.ldx; q.ldy = d.ldy;
-        q.gated = d.gated; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
+        q.gated = d.gated; q.streamed = streamed; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
         q.yvec = (d.ldy % 4 == 0) && ((uintptr_t)d.y % (d.out_f32 ? 16 : 8) == 0);
         q.G = 1; q.xs = q.ws = q.ys = 0; q.offs = nullptr; q.gather = nullptr; q.tiles = nullptr; q.egate = nullptr; q.ldg = q.goff = 0;
     }
@@ -1097,6 +1101,7 @@ extern "C" int mi355_dense_grouped_ahead(const void* x, int32_t ldx, int32_t M, 
                                          int32_t ldy, int32_t out_f32, int32_t gated, int32_t act, float act_param, int32_t act_dtype, int32_t G,
                                          int64_t xs, int64_t ys, const int32_t* offs, const int32_t* gather, const int32_t* tiles, int32_t max_tiles,
                                          const float* egate, int32_t ldg, int32_t goff, const void* ahead, int64_t ahead_bytes, mi355_stream_t stream) {
+    const int streamed = (gated & MI355_DENSE_STREAMED) != 0; gated &= ~MI355_DENSE_STREAMED;
     MI355_CHECK_ARG(x && w && y && M > 0 && N > 0 && K > 0 && G > 0 && xs >= 0 && ys >= 0, "dense_grouped: M=%d N=%d K=%d G=%d", M, N, K, G);
     MI355_CHECK_ARG(ldx >= xs * (G - 1) + K, "dense_grouped: ldx=%d for %d groups of K=%d at step %lld", ldx, G, K, (long long)xs);
     MI355_CHECK_ARG(act_dtype == MI355_ACT_BF16 || act_dtype == MI355_ACT_F32, "dense_grouped: act_dtype=%d (bf16 or fp32)", act_dtype);
@@ -1107,7 +1112,7 @@ extern "C" int mi355_dense_grouped_ahead(const void* x, int32_t ldx, int32_t M, 
     const bool bf = act_dtype == MI355_ACT_BF16;
     DenseParams p;
     p.x = x; p.w = w; p.bias = bias; p.y = y; p.M = M; p.N = N; p.K = K; p.ldx = ldx; p.ldy = ldy;
-    p.gated = gated; p.act = act; p.act_param = act_param; p.out_f32 = bf ? out_f32 : 1; p.softcap = 0.f;
+    p.gated = gated; p.streamed = streamed; p.act = act; p.act_param = act_param; p.out_f32 = bf ? out_f32 : 1; p.softcap = 0.f;
     p.vec = (K % 8 == 0) && (ldx % 8 == 0) && (xs % 8 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
     p.yvec = (ldy % 4 == 0) && ((uintptr_t)y % (p.out_f32 ? 16 : 8) == 0);
     p.G = G; p.xs = xs; p.ws = (long long)N * K; p.ys = ys; p.offs = offs; p.gather = gather; p.tiles = tiles;

@@ -363,10 +363,15 @@ class HybridModel:
         hops.act_code(dtype)
         self.cfg, self.dtype, self.device, self.page = cfg, dtype, torch.device(device), page
 
+        step_bytes = 0                                 # of the weights that a step reads whole
+
         def get(name):
+            nonlocal step_bytes
             if name not in tensors:
                 raise KeyError(f"checkpoint has no tensor {name!r}")
-            return tensors[name].to(device=self.device, dtype=dtype).contiguous()
+            t = tensors[name].to(device=self.device, dtype=dtype).contiguous()
+            step_bytes += 0 if name == "bigram" or (name == "embed" and not cfg.tied_head) else t.numel() * t.element_size()
+            return t
 
         def sub(prefix, names):
             return {n: get(prefix + n) for n in names}
@@ -503,6 +508,7 @@ class HybridModel:
         self.norm_center = cfg.norm_kind == "layer"
         if cfg.norm_kind not in ("rms", "layer") or (cfg.norm_kind == "layer" and not cfg.out_norm):
             raise NotImplementedError(f"norm kind {cfg.norm_kind!r} (layer norms are built for stacks that norm the sublayers' outputs)")
+        hops.mark_streamed([self.head, self.layers, self.loop_in], step_bytes)
 
     # ---- what an engine has to allocate
     def cache_layout(self):

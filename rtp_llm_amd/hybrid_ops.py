@@ -80,9 +80,41 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
     if M == 0:
         return out
     _C.check_hybrid(_C.hybrid_lib().mi355_dense_linear_ex(x.data_ptr(), ldx, M, w.data_ptr(), N, K, _p(bias), out.data_ptr(), ldy,
-                                                          1 if od == torch.float32 else 0, 1 if gated else 0, act, float(act_param), float(softcap),
+                                                          1 if od == torch.float32 else 0, _gated(w, M, gated), act, float(act_param), float(softcap),
                                                           act_code(w.dtype), _stream()), "dense_linear")
     return out
+
+
+_STREAMED = 1 << 30         # MI355_DENSE_STREAMED
+
+
+def mark_streamed(weights, nbytes: int, cached: int = 256 << 20) -> bool:
+    """A model's weights (tensors, or objects, lists and dicts that hold some) get the attribute `streamed` where the nbytes that a step reads are more than the memory-side cache keeps for the
+    next: the linears of a few rows then read the large ones past the caches.  -> whether they did."""
+    seen = set()
+
+    def walk(o):
+        if id(o) in seen:
+            return
+        seen.add(id(o))
+        if isinstance(o, torch.Tensor):
+            o.streamed = True
+        elif isinstance(o, dict):
+            for v in o.values():
+                walk(v)
+        elif isinstance(o, (list, tuple, set)):
+            for v in o:
+                walk(v)
+        elif type(o).__module__.startswith(__name__.rpartition(".")[0]) and hasattr(o, "__dict__"):
+            walk(vars(o))
+
+    if nbytes > cached:
+        walk(weights)
+    return nbytes > cached
+
+
+def _gated(w: torch.Tensor, rows: int, gated: bool) -> int:
+    return int(gated) | (_STREAMED if 2 <= rows <= FEW_ROWS and getattr(w, "streamed", False) else 0)
 
 
 FEW_ROWS = 16              # rows up to which the linears are bound by their weights' stream and every launch by its own cost
@@ -109,7 +141,7 @@ def dense_pair(first: dict, second: dict):
         out = torch.empty(M, n_out, dtype=od, device=x.device)
         outs.append(out)
         a.x, a.ldx, a.M, a.w, a.N, a.K, a.bias, a.y, a.ldy = x.data_ptr(), _rows(x, "dense_pair.x"), M, w.data_ptr(), N, K, _p(bias), out.data_ptr(), n_out
-        a.out_f32, a.gated, a.act, a.act_param = int(od == torch.float32), int(gated), int(d.get("act", ACT_NONE)), float(d.get("act_param", 0.0))
+        a.out_f32, a.gated, a.act, a.act_param = int(od == torch.float32), _gated(w, M, gated), int(d.get("act", ACT_NONE)), float(d.get("act_param", 0.0))
     rc = _C.hybrid_lib().mi355_dense_linear_pair(args, _stream())
     if rc == _C.ERR_UNSUPPORTED:               # operands off 16 bytes, K % 8
         return dense_linear(**first), dense_linear(**second)
@@ -867,7 +899,7 @@ def dense_grouped(x: torch.Tensor, w: torch.Tensor, *, x_step: int = 0, y_step: 
             raise _C.Mi355Error(f"dense_grouped: gate {tuple(mul_sigmoid.shape)} for outputs [{M}, {width}]")
     if M:
         _C.check_hybrid(_C.hybrid_lib().mi355_dense_grouped_ahead(x.data_ptr(), ldx, M, w.data_ptr(), N, K, None, out.data_ptr(), _rows(out, "dense_grouped.out"),
-                                                               1 if od == torch.float32 else 0, 1 if gated else 0, act, float(act_param), act_code(w.dtype), G, x_step,
+                                                               1 if od == torch.float32 else 0, _gated(w, M, gated), act, float(act_param), act_code(w.dtype), G, x_step,
                                                                y_step, _p(offs), _p(gather), _p(tiles), 0 if tiles is None else (tiles.numel() - 1) // 2,
                                                                _p(mul_sigmoid), ldg, 0, *_ahead(ahead, "dense_grouped.ahead"), _stream()),
                         "dense_grouped")

@@ -77,3 +77,23 @@ def test_few_rows_far_apart(M, ldx):
     w2, gate = torch.stack([w, w.flip(0)]), torch.randn(M, 2 * 72, device=DEV, generator=g)
     run = lambda v: hops.dense_grouped(v, w2, x_step=K, y_step=72, mul_sigmoid=gate)
     assert torch.equal(run(far), run(x))
+
+
+@pytest.mark.parametrize("N,K", [(6144, 2048), (6136, 2048), (13000, 968), (13008, 968)])
+def test_few_rows_streamed(N, K):
+    """Weights marked as streamed, on either side of 24 MB: the same bits, alone, in a launch of two and through groups."""
+    g = torch.Generator(device=DEV).manual_seed(N)
+    w = torch.randn(N, K, device=DEV, generator=g).bfloat16()
+    s, small, smalls = w.clone(), w[:64].clone(), w[:64].clone()
+    s.streamed = smalls.streamed = True
+    for M in (2, 8, 16):
+        x = torch.randn(M, K, device=DEV, generator=g).bfloat16()
+        y = hops.dense_linear(x, w)
+        assert torch.equal(hops.dense_linear(x, s), y)
+        for a, b in ((s, smalls), (s, small), (w, smalls)):
+            p, q = hops.dense_pair(dict(x=x, w=a), dict(x=x, w=b, gated=True, act=hops.ACT_SILU))
+            assert torch.equal(p, y) and torch.equal(q, hops.dense_linear(x, small, gated=True, act=hops.ACT_SILU))
+        gs = w[:N // 8 * 8].view(4, N // 8 * 2, K).clone()
+        z = hops.dense_grouped(x, gs, y_step=N // 8 * 2)
+        gs.streamed = True
+        assert torch.equal(hops.dense_grouped(x, gs, y_step=N // 8 * 2), z)
