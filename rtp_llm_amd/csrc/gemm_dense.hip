@@ -842,13 +842,15 @@ __global__ __launch_bounds__(256) void dense_skinny_pair_kernel(DenseParams p0, 
     }
 }
 
-// Short K through many outputs: a block of 8 weight rows would end before it has begun, so 16 outputs a block, fragments straight from memory, a wave for each of the NW chains: the same sums.
+// Where that costs more than it gains (skinny_short): fragments straight from memory, the same sums.  16 outputs a block, a wave for each of the NW chains, U steps of it in flight.
+// HALF (M <= 8): 8 outputs a block and half the waves, each with two chains: rows 0 to 7 of the first operand are x in the steps of chain w, rows 8 to 15 x in those of chain w + NW / 2, the second
+// operand likewise; of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are the two chains, the rest is not used.
 template <int NW> struct SkinnySums { f32x4 at[NW][2][64]; };
-template <bool GATED, int NW>
+template <bool GATED, int NW, int U, bool HALF>
 __device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, int bx, int grp, SkinnySums<NW>& red) {
-    constexpr int U = 4;
+    constexpr int NO = HALF ? 8 : 16, WAVES = HALF ? NW / 2 : NW;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nout = GATED ? p.N / 2 : p.N;
-    const int r = lane & 15, kq = (lane >> 4) * 8, o = min(bx * 16 + r, nout - 1), n = GATED ? (o >> 5) * 64 + (o & 31) : o;
+    const int r = lane & (NO - 1), kq = (lane >> 4) * 8 + (HALF && (lane & 8) ? WAVES * 32 : 0), o = min(bx * NO + r, nout - 1), n = GATED ? (o >> 5) * 64 + (o & 31) : o;
     const bf16* wg = (const bf16*)p.w + p.ws * grp + (size_t)n * p.K + kq;
     const bf16* wu = wg + (size_t)32 * p.K;
     const bf16* xr = (const bf16*)p.x + p.xs * grp + (size_t)min(r, p.M - 1) * p.ldx + kq;
@@ -874,42 +876,67 @@ __device__ __forceinline__ void dense_skinny_short_tile(const DenseParams& p, in
     if (GATED) red.at[wave][1][lane] = au;
     __syncthreads();
     if (wave != 0) return;
-    for (int w = 1; w < NW; ++w) {
+    for (int w = 1; w < WAVES; ++w) {
         ag += red.at[w][0][lane];
         if (GATED) au += red.at[w][1][lane];
     }
-    if (bx * 16 + r >= nout) return;
+    if constexpr (HALF) {                                                     // the other chains' sum of (output, row) lies at (output + 8, row + 8), 40 lanes on
+        if ((lane & 8) || lane >= 32) return;
+        for (int w = 0; w < WAVES; ++w) {
+            ag += red.at[w][0][lane + 40];
+            if (GATED) au += red.at[w][1][lane + 40];
+        }
+    }
+    if (bx * NO + r >= nout) return;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int row = (lane >> 4) * 4 + e;
         if (row >= p.M) continue;
         float g = ag[e], u = au[e];
         if (p.bias) { const bf16* Bi = (const bf16*)p.bias + (size_t)grp * p.N; g += dn_ld(Bi + n); if (GATED) u += dn_ld(Bi + n + 32); }
-        dn_store<bf16>(p, row, (int)(p.ys * grp) + bx * 16 + r, GATED ? dn_gated(g, u, p.act, p.act_param) : dn_act(g, p.act));
+        dn_store<bf16>(p, row, (int)(p.ys * grp) + bx * NO + r, GATED ? dn_gated(g, u, p.act, p.act_param) : dn_act(g, p.act));
     }
 }
-template <bool GATED, int NW>
-__global__ __launch_bounds__(64 * NW) void dense_skinny_short_kernel(DenseParams p) {
+template <bool GATED, int NW, int U, bool HALF>
+__global__ __launch_bounds__(64 * (HALF ? NW / 2 : NW)) void dense_skinny_short_kernel(DenseParams p) {
     __shared__ SkinnySums<NW> red;
-    dense_skinny_short_tile<GATED, NW>(p, blockIdx.x, blockIdx.y, red);
+    dense_skinny_short_tile<GATED, NW, U, HALF>(p, blockIdx.x, blockIdx.y, red);
 }
-template <bool GATED0, bool GATED1, int NW>
-__global__ __launch_bounds__(64 * NW) void dense_skinny_short_pair_kernel(DenseParams p0, DenseParams p1, int blocks0) {
+template <bool GATED0, bool GATED1, int NW, int U, bool HALF>
+__global__ __launch_bounds__(64 * (HALF ? NW / 2 : NW)) void dense_skinny_short_pair_kernel(DenseParams p0, DenseParams p1, int blocks0) {
     __shared__ SkinnySums<NW> red;
-    if ((int)blockIdx.x < blocks0) dense_skinny_short_tile<GATED0, NW>(p0, blockIdx.x, 0, red);
-    else                           dense_skinny_short_tile<GATED1, NW>(p1, blockIdx.x - blocks0, 0, red);
+    if ((int)blockIdx.x < blocks0) dense_skinny_short_tile<GATED0, NW, U, HALF>(p0, blockIdx.x, 0, red);
+    else                           dense_skinny_short_tile<GATED1, NW, U, HALF>(p1, blockIdx.x - blocks0, 0, red);
 }
-// Where that form is taken.  It has no stages to fill and half the blocks, but its wave loads are 16 rows by 64 bytes, which the weights' stream of long K pays for.  Random calls of 2 to 16 rows,
-// us of the DMA form / this one, weights from memory: 11 x 1024 x 47616 gated 29.1 / 24.5, 10 x 1024 x 22784 gated 16.4 / 13.1, 16 x 6720 gated x 872 7.2 / 6.4; read again and again from the
-// memory-side cache: 11 x 1352 x 34880 22.8 / 18.8, 7 x 1048 x 9344 8.3 / 6.9, 2 x 1176 x 4096 5.1 / 4.4; past the lines, from memory: 11 x 1728 x 10368 gated 13.0 / 14.0,
-// 12 x 1832 x 4224 8.3 / 9.5, 4 x 2048 x 30464 22.8 / 29.6, 5 x 2000 x 4160 7.4 / 8.3.
-bool skinny_short(int M, int K, long long weight_rows) {
-    return (K <= 1152 && weight_rows >= 6144) || (K <= (M > 4 ? 1792 : 1280) && weight_rows >= (M > 8 ? 12288 : 4096));
+// Which linears of M rows, K columns and so many weight rows are better off without LDS: they have no stages to fill, and a stage's columns past K cost what the others do, but their wave loads are 8
+// or 16 rows by 64 bytes, which the weights' stream of long K pays for.  Few rows, of which the stages hold copies, gain until K 2304; more rows to 1792; K below 512 leaves HALF's second
+// chains idle; many outputs fill the chip with 16 a block.  Time of the DMA form / HALF / 16 over that of the kernels before the DMA form, means over random calls, weights from memory:
+//   2 rows, K 512 to 1023, up to 512 weight rows 1.04 / 0.92 / 1.10; K 1500 to 2048 1.05 / 0.93 / 1.13; 3 rows, K 1024 to 1500, 512 to 1024 1.02 / 0.93 / 1.15; 4 rows, K 1500 to 2048, 512 to 1024 1.02 /
+//   0.93 / 1.15, K over 3000 0.76 / 0.95 / 1.20; 5 to 8 rows, K 1024 to 1500, 2048 to 4096 1.03 / 0.97 / 1.06, K 2048 to 3000, over 4096 0.79 / 0.98 / 0.99; K below 512, over 10000 1.45 / 1.03 / 0.97.
+//   9 to 16 rows, us: 11 x 1024 x 47616 gated 29.1 / - / 24.5, 10 x 1024 x 22784 gated 16.4 / - / 13.1; 12 x 1808 x 8128, just two blocks of 16 a compute unit, 11.8 / - / 10.6; past the lines
+//   11 x 1728 x 10368 gated 13.0 / - / 14.0, 16 x 1864 x 8256 gated 13.5 / - / 16.4, 12 x 1832 x 4224 8.3 / - / 9.5.
+// 1600 times of 800 random calls, from memory and from the memory-side cache: 1.018 of the fastest form's up to 8 rows (K of 1024 and more through LDS alone: 1.05) and 1.014 above; of 1700 others 30 are
+// more than 3 % behind the kernels before the DMA form, at worst 1.11, and most lie at 0.5 to 0.98.
+int skinny_short(int M, int K, long long weight_rows) {           // outputs a block; 0: through LDS
+    if (M > 8) return weight_rows >= 6144 && (K <= 1152 || (K <= 1856 && (weight_rows <= 8192 || weight_rows >= 12288))) ? 16 : 0;
+    if (K < 512) return M <= 3 || weight_rows > 512 ? 16 : 0;
+    if (K <= 1152 && weight_rows >= 6144) return 16;
+    return K <= (M <= 4 ? 2304 : 1792) && weight_rows <= 8192 ? 8 : 0;
+}
+int skinny_short_blocks(const DenseParams& p, int outputs) { return ((p.gated ? p.N / 2 : p.N) + outputs - 1) / outputs; }
+// launch(chains, steps in flight, half) with the instance for as many outputs a block
+template <class L>
+void skinny_short_form(int outputs, bool eight, L&& launch) {
+    const std::integral_constant<int, 4> four{};
+    const std::integral_constant<int, 8> eights{};
+    if (outputs == 16) { if (eight) launch(eights, four, std::false_type{}); else launch(four, four, std::false_type{}); }
+    else               { if (eight) launch(eights, eights, std::true_type{}); else launch(four, eights, std::true_type{}); }
 }
 
 // The partial sums that K is split into (part of a result's bits): eight, four of many outputs or short K.
 int skinny_chains(const DenseParams& p) { return (((p.gated ? p.N / 2 : p.N) + 15) / 16) * p.G >= 1024 || p.K < 1024 ? 4 : 8; }
 int skinny_blocks(const DenseParams& p) { return (p.N + SK_RB - 1) / SK_RB; }
+
 // A weight that the 256 MB memory-side cache does not hold from one step to the next is read past the caches where a launch reads 24 MB or more.  Only the caller knows: the same weight in a
 // small model, or under a draft's head, comes from that cache.  40 random weights of 24 to 130 MB, time with / without the hint: 0.97 (0.91 to 1.01) in a footprint of 1 GB, 0.96 in 400 MB,
 // 1.12 (0.99 to 1.37) in 256 MB, 1.10 in 128 MB.  17408 x 2048 from memory 15.5 / 14.4 us, 32000 x 2048 26.5 / 24.3; eight prompts and eight steps of a 16-layer model of width 2048 8920 / 8400 us.
@@ -921,9 +948,6 @@ bool skinny_nt(bool streamed, size_t weights) { return streamed && weights * 2 >
 //   512 (a stage's loads past K cost what the others do); and for 9 to 16 rows in more than 256 blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2);
 //   stages of 1024, half the barriers, in up to 192 blocks, where no compute unit has a second block to hide them (2 rows, 384 x 5960, six stages of 512 / three of 1024: 7.1 / 6.3) and the last
 //   stage is not mostly empty.
-// 400 random calls of 2 to 16 rows, weights from memory and from the memory-side cache, time over that of the fastest of the four forms: 1.010 with these lines and skinny_short's, 1.021 with
-// stages of 256 and 1024 for K < 1024 and up to 256 blocks alone.  34 of the 800 times are more than 3 % over those of 16 outputs a block throughout, 24 of them from the memory-side cache, the
-// worst 1.14; the others are 0.5 to 1.03.
 template <class L>
 void skinny_form(int M, int K, long long blocks, L&& launch) {
     auto rows = [&](auto kc, auto ns) {
@@ -957,10 +981,13 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         return;
     }
     const bool eight = skinny_chains(p) == 8;
-    if (skinny_short(p.M, p.K, (long long)p.N * p.G)) {
-        const dim3 grid(((p.gated ? p.N / 2 : p.N) + 15) / 16, p.G), block(eight ? 512 : 256);
-        if (eight) { if (p.gated) hipLaunchKernelGGL((dense_skinny_short_kernel<true, 8>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_short_kernel<false, 8>), grid, block, 0, st, p); }
-        else       { if (p.gated) hipLaunchKernelGGL((dense_skinny_short_kernel<true, 4>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_short_kernel<false, 4>), grid, block, 0, st, p); }
+    if (const int out = skinny_short(p.M, p.K, (long long)p.N * p.G)) {
+        skinny_short_form(out, eight, [&](auto nw, auto u, auto half) {
+            constexpr int NW = decltype(nw)::value, U = decltype(u)::value;
+            constexpr bool H = decltype(half)::value;
+            const dim3 grid(skinny_short_blocks(p, out), p.G), block(64 * (H ? NW / 2 : NW));
+            if (p.gated) hipLaunchKernelGGL((dense_skinny_short_kernel<true, NW, U, H>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_short_kernel<false, NW, U, H>), grid, block, 0, st, p);
+        });
         return;
     }
     const dim3 grid(skinny_blocks(p), p.G), block(256);
@@ -971,17 +998,19 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         else       { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, false>), grid, block, 0, st, p); }
     });
 }
-template <int NW>
-void launch_skinny_short_pair(const DenseParams (&p)[2], hipStream_t st) {
-    const int s0 = ((p[0].gated ? p[0].N / 2 : p[0].N) + 15) / 16, s1 = ((p[1].gated ? p[1].N / 2 : p[1].N) + 15) / 16;
-    const dim3 grid(s0 + s1), block(64 * NW);
-    if (p[0].gated) { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, true, NW>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, false, NW>), grid, block, 0, st, p[0], p[1], s0); }
-    else            { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, true, NW>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, false, NW>), grid, block, 0, st, p[0], p[1], s0); }
-}
 void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
     const int chains = skinny_chains(p[0]);
-    if (skinny_chains(p[1]) == chains && skinny_short(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N)) {
-        if (chains == 8) launch_skinny_short_pair<8>(p, st); else launch_skinny_short_pair<4>(p, st);
+    const int out = skinny_chains(p[1]) == chains ? skinny_short(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N) : 0;
+    if (out) {
+        const int s0 = skinny_short_blocks(p[0], out);
+        const dim3 grid(s0 + skinny_short_blocks(p[1], out));
+        skinny_short_form(out, chains == 8, [&](auto nw, auto u, auto half) {
+            constexpr int NW = decltype(nw)::value, U = decltype(u)::value;
+            constexpr bool H = decltype(half)::value;
+            const dim3 block(64 * (H ? NW / 2 : NW));
+            if (p[0].gated) { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, true, NW, U, H>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<true, false, NW, U, H>), grid, block, 0, st, p[0], p[1], s0); }
+            else            { if (p[1].gated) hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, true, NW, U, H>), grid, block, 0, st, p[0], p[1], s0); else hipLaunchKernelGGL((dense_skinny_short_pair_kernel<false, false, NW, U, H>), grid, block, 0, st, p[0], p[1], s0); }
+        });
         return;
     }
     const int b0 = skinny_blocks(p[0]), b1 = skinny_blocks(p[1]), c0 = skinny_chains(p[0]), c1 = skinny_chains(p[1]);

@@ -42,10 +42,11 @@ def test_few_rows_through_every_group():
 
 
 @pytest.mark.parametrize("N,K", [(2048, 1016), (2048, 1024), (2050, 1032), (4096, 1016), (4097, 1016), (8184, 1024), (8200, 1160), (6152, 2056), (6136, 2048), (64, 5640),
-                                 (6144, 1152), (6136, 1152), (6144, 1160), (4096, 1280), (4096, 1288), (4088, 1280), (4096, 1792), (4096, 1800), (12288, 1792), (12280, 1792), (16400, 1024), (16384, 1792),
-                                 (1536, 2048), (1544, 2048), (1536, 1032), (2048, 1056), (2056, 1056), (2056, 1288)])
+                                 (512, 504), (520, 504), (512, 512), (520, 512), (6144, 504), (6144, 1152), (6136, 1152), (6144, 1160), (8192, 1160), (8200, 1160), (8192, 1792), (8192, 1800),
+                                 (2048, 2304), (2048, 2312), (12288, 1856), (12280, 1856), (8192, 1856), (8192, 1864), (16400, 1024), (16384, 1792), (1536, 3072), (1544, 3072), (1536, 2320), (2048, 2568), (2056, 2568),
+                                 (2056, 2824)])
 def test_few_rows_forms(N, K):
-    """Either side of each rule that picks the form (K 1024, 1152, 1280, 1792; 4096, 6144, 12288 weight rows; four chains and eight), stages and columns of a stage (192 and 256 blocks, columns
+    """Either side of each rule that picks the form (3, 4 and 8 rows; K 512, 1152, 1792, 1856, 2304; 512, 6144, 8192, 12288 weight rows; four chains and eight), stages and columns of a stage (192 and 256 blocks, columns
     loaded for nothing, 24 MB), a last stage with one piece: against a 64-bit product, the same bits for any number of rows, alone and in a launch of two."""
     g = torch.Generator(device=DEV).manual_seed(N + K)
     x, w = torch.randn(16, K, device=DEV, generator=g).bfloat16(), (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
@@ -54,7 +55,7 @@ def test_few_rows_forms(N, K):
     ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
     assert float(((y.double() - ref).abs() / (2.0 ** -24 * 1.01 * ref.abs() + 2.0 ** -17 * mag)).max()) <= 1.0
     gated = hops.dense_linear(x2, w2, gated=True, act=hops.ACT_SILU)
-    for M in (2, 4, 5, 8, 9, 16):
+    for M in (2, 3, 4, 5, 8, 9, 16):
         a, b = hops.dense_pair(dict(x=x[:M], w=w, out_dtype=torch.float32), dict(x=x2[:M], w=w2, gated=True, act=hops.ACT_SILU))
         assert torch.equal(hops.dense_linear(x[:M], w, out_dtype=torch.float32), y[:M]) and torch.equal(a, y[:M]) and torch.equal(b, gated[:M]), M
     a, b = hops.dense_pair(dict(x=x2, w=w2, gated=True, act=hops.ACT_SILU), dict(x=x, w=w, out_dtype=torch.float32))
