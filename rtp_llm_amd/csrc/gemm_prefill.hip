@@ -46,11 +46,14 @@ __device__ __forceinline__ void store_bf16(const GemmParams& p, f32x4 v, int m, 
 // divides stay in rows: there an XCD has its columns to itself anyway, and their weights stay in its L2 from one row tile to the next (72 columns 1.6 % faster so, 32
 // columns 2 to 3 %).  us in rows / in bands: 8 bits 37888 x 3584 at 1055 rows 300 / 266, W4 at 4096 rows 1005 / 985, W16 11008 x 4096 at 2667 rows 418 / 315, 896 x 4864 at
 // 1753 rows 42 / 36; 110 random calls 0.97 of the time in rows; bands of 6, 8 and 12 alike, 24 1 % slower.  Tiles that stay in rows are the launch's own blocks: the divisions that
-// find a tile stand in front of a block's first load, 0.9 us of 15.  In bands only where a column tile's weights are 128 KB or x is 4 MB: a band's blocks of an XCD all wait for the same strip
-// of weights, and behind short strips the launch is over before that pays.  407 random calls of 65 to 4096 rows, band / rows: 201 inside these lines 0.935 (six above 1.03, at worst 1.06),
-// 206 outside 1.007 (0.84 to 1.13; W4 896 x 896 at 292 rows 5.2 / 5.9 us, 8 bits 5.2 / 5.6).
+// find a tile stand in front of a block's first load, 0.9 us of 15.  In bands except where K is short (up to 8 whole chunks of
+// 128) for more than 192 rows, a column tile's weights are below 128 KB and x below 4 MB: a band's blocks of an XCD all wait for the same strip of weights, and the launch is over before reading it
+// once pays.  565 random calls of 65 to 4096 rows, band / rows: 422 in bands 0.958 (39 above 1.03, at worst 1.11), 143 in rows 1.031
+// (0.96 to 1.13; W4 896 x 896 at 292 rows 5.2 / 5.9 us, 8 bits 5.2 / 5.6).
 constexpr int PF_XCD = 8, PF_BAND = 8;
-constexpr uint64_t PF_STRIP = 128 << 10, PF_ROWS = 4 << 20;
+bool prefill_short(const GemmParams& p, int wbits, int tile_cols) {
+    return p.K % 128 == 0 && p.K <= 1024 && p.M > 192 && (uint64_t)p.KC * 16 * tile_cols * wbits < 128 << 10 && (uint64_t)p.M * p.K * 2 < 4 << 20;
+}
 int prefill_band(int rows, int cols) {                        // 0: in rows; else the height of all bands but the last
     const int bands = (rows + PF_BAND - 1) / PF_BAND;
     return cols % PF_XCD == 0 ? 0 : (rows + bands - 1) / bands;
@@ -464,8 +467,7 @@ template <int WBITS, int GS, bool BF, int I>
 void launch_shape_t(const GemmParams& p, hipStream_t st) {
     constexpr PrefillShape s = kPrefillShapes[I];
     const dim3 grid(cdiv(p.NT, 8 / s.ks * s.tpw), cdiv(p.M, 16 * s.mb));
-    const bool worth = (uint64_t)p.KC * 128 * (8 / s.ks * s.tpw * 16) * WBITS / 8 >= PF_STRIP || (uint64_t)p.M * p.K * 2 >= PF_ROWS;
-    const int band = worth ? prefill_band(grid.y, grid.x) : 0;
+    const int band = prefill_short(p, WBITS, 8 / s.ks * s.tpw * 16) ? 0 : prefill_band(grid.y, grid.x);
     constexpr bool straight = !(I == 0 && (GS == 1 || GS == 2)) && !(I == 2 && GS == 1) && !(BF && WBITS == 4 && s.mb == 4) && !(WBITS == 4 && s.ks > 1);
     if constexpr (straight) {
         if ((uintptr_t)p.x % 16 == 0 && p.K % 128 == 0 && p.K < 1 << 23) {
