@@ -92,8 +92,15 @@ __device__ __forceinline__ void pace(int i0, int n) {         // the order of fr
         }
     }
 }
+// Waves a SIMD that the registers have to leave room for.  The general loop of 4-bit weights in groups of 64 and 128: 8 for 32 x 64 (64 registers, four blocks a CU; left alone the compiler takes
+// 62 to 67), 6 for bf16 in 64 x 128 (80, three blocks; it takes 77 and 90).  bf16 9728 x 896 in groups of 64 at 395 rows 22.6 -> 20.0 us, fp16 1408 x 256 at 362 rows 4.6 -> 3.9.
+constexpr int prefill_waves(int wbits, int gs, bool bf, int mb, int tpw, int ks, bool whole) {
+    if (wbits == 4 && gs != 1 && !whole && mb == 2 && ks == 2) return 8;
+    if (wbits == 4 && gs != 1 && !whole && bf && mb == 4 && tpw == 1 && ks == 1) return 6;
+    return tpw * mb <= 16 && wbits != 16 && !(bf && wbits == 4) ? 2 : 1;
+}
 template <int WBITS, int GS, bool BF, int MB, int TPW, int KS, bool WHOLE>
-__global__ __launch_bounds__(512, (TPW * MB <= 16 && WBITS != 16 && !(BF && WBITS == 4)) ? 2 : 1) void gemm_prefill_kernel(const GemmParams p, const int band) {
+__global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOLE)) void gemm_prefill_kernel(const GemmParams p, const int band) {
     constexpr int BM = 16 * MB, NWN = 8 / KS;                 // rows, waves side by side
     constexpr int LPC  = WBITS / 4;
     constexpr int NSUB = (GS > 0) ? 4 / GS : 1;
@@ -428,49 +435,78 @@ constexpr PrefillCost kPrefillCost[3][kPrefillShapeCount] = {
     {{1e9, 1e9},   {2.16, 2.45}, {1.52, 1.32}, {0.94, 0.708}, {0.98, 0.856}, {0.72, 0.507}, {0.69, 0.708}},      // bf16 under group scales: two sets of accumulators
     {{1e9, 1e9},   {1.41, 2.82}, {0.92, 1.84}, {0.49, 0.856}, {0.49, 0.779}, {0.45, 0.532}, {0.37, 0.742}},     // 16-bit weights
 };
-// The same for the shapes that do not slice K, in the loop without branches and with the tiles dealt in bands, per operand class: fp16 W4, fp16 and bf16 8 bits, 16-bit weights
-// (bf16 W4: as above).  One round of blocks takes `lat`, however few they are.  These shapes choose among each other only: whether K is sliced stays with the table above, so
-// that a call's sums keep their order.  Fitted to times and picks of 290 random calls of M = 65..4096: the pick takes 1.004 of the fastest shape's time on average, at worst 1.09,
-// where the table above took 1.024 and 1.2 (8 bits, 4608 x 3584 at 1055 rows: 52 -> 45 us).
+// Does shape I run the loop without branches (WHOLE) where x allows it?  gs: 4, 2, 1 for groups of 128, 64, 32.  Not 128 x 512 under groups of 32 or 64 (two or four scales a chunk and tile have
+// no registers left), 64 x 256 in groups of 32 and the 64-row forms of bf16 W4 (held in one piece the compiler takes more than 128 or 80 registers for them and a block less fits a CU:
+// 37888 x 3584 at 4096 rows 1293 -> 1485 us), bf16 W4 in groups of 32 (198 random calls 1.04 of the general loop's time), nor 4-bit weights under sliced K (8 or 16 products and 56 operand
+// instructions a wave and chunk: 2 % either way, 3584 x 18944 at 104 rows 59 -> 60 to 62 us).  The others take 0.85 to 1.00 of it, mean over about 200 calls each.
+constexpr bool prefill_straight(int I, int wbits, int gs, bool bf) {
+    if (wbits != 4) return true;
+    if (kPrefillShapes[I].ks > 1 || (bf && (kPrefillShapes[I].mb == 4 || gs == 1))) return false;
+    return I == 0 ? gs == 4 : I == 2 ? gs != 1 : true;
+}
+// The same for the shapes that do not slice K, fitted to the present loops, per operand class: where K or x leaves every shape the general loop (first row) and where each has the loop it can
+// have (second).  `base` us a launch beside its chunks: 12 for a block of 128 x 512, 5 for 64 x 128; one round of blocks takes `lat` a chunk, however few they are.  These shapes choose among each
+// other only: whether K is sliced stays with the table above, so that a call's sums keep their order.  Fitted to times and picks of 81 to 139 random calls of M = 65..4096 a row, weights from
+// memory: the pick takes 1.0003 to 1.0035 of the fastest shape's time on average; 412 other calls 1.004, at worst 1.13.  With 2.5 us for every shape and one row for both loops and all groups it
+// took 1.004 to 1.033, at worst 1.31 (16-bit weights, 37888 x 3584 at 1825 rows 590 us where 128 x 256 takes 462).
 constexpr int kWholeShapes = 4;
-constexpr PrefillCost kWholeCost[4][kWholeShapes] = {
-    {{3.12, 3.94}, {1.81, 2.08}, {1.10, 1.087}, {0.62, 0.635}},
-    {{3.16, 3.40}, {1.69, 1.81}, {1.01, 0.997}, {0.70, 0.583}},
-    {{1e9, 1e9},   {2.07, 2.28}, {1.27, 1.213}, {0.75, 0.668}},
-    {{1e9, 1e9},   {1.94, 2.65}, {0.89, 1.368}, {0.56, 0.737}},
+struct UnslicedCost { double base, lat, sat; };
+constexpr UnslicedCost kUnslicedCost[9][2][kWholeShapes] = {
+    {{{15.0, 2.40, 3.401}, {7.7, 1.60, 1.940}, {5.9, 1.09, 1.054}, {5.6, 0.50, 0.568}},
+     {{12.4, 2.20, 3.414}, {8.7, 1.30, 1.830}, {5.6, 1.02, 1.022}, {5.1, 0.49, 0.559}}},     // fp16 W4, groups of 128
+    {{{15.3, 2.59, 3.572}, {10.7, 1.43, 1.992}, {6.8, 1.08, 1.091}, {6.1, 0.49, 0.588}},
+     {{13.3, 2.65, 3.565}, {9.3, 1.24, 1.924}, {6.2, 0.97, 1.038}, {5.6, 0.42, 0.570}}},     // of 64
+    {{{12.4, 2.63, 3.678}, {8.2, 1.56, 2.079}, {6.3, 1.17, 1.132}, {5.3, 0.77, 0.623}},
+     {{12.7, 2.61, 3.630}, {8.5, 1.29, 2.047}, {8.0, 1.03, 1.108}, {4.6, 0.62, 0.602}}},     // of 32
+    {{{0, 1e9, 1e9}, {7.4, 2.00, 2.525}, {6.1, 1.48, 1.296}, {6.4, 0.30, 0.695}},
+     {{0, 1e9, 1e9}, {8.1, 1.65, 2.237}, {7.2, 1.45, 1.285}, {5.7, 0.34, 0.703}}},     // bf16 W4, groups of 128
+    {{{0, 1e9, 1e9}, {7.9, 2.30, 2.799}, {6.8, 1.72, 1.509}, {5.2, 1.05, 0.792}},
+     {{0, 1e9, 1e9}, {9.2, 2.17, 2.636}, {6.1, 1.78, 1.526}, {5.7, 1.57, 0.776}}},     // of 64
+    {{{0, 1e9, 1e9}, {7.9, 2.89, 3.573}, {5.7, 2.09, 2.402}, {7.1, 0.34, 0.981}},
+     {{0, 1e9, 1e9}, {7.6, 2.90, 3.575}, {5.5, 2.08, 2.410}, {7.0, 0.57, 0.980}}},     // of 32
+    {{{11.3, 2.70, 3.396}, {7.1, 1.55, 1.897}, {6.1, 1.01, 0.978}, {5.5, 0.62, 0.524}},
+     {{11.7, 2.35, 2.964}, {7.0, 1.33, 1.697}, {6.5, 0.91, 0.869}, {5.0, 0.57, 0.520}}},     // fp16 8 bits
+    {{{0, 1e9, 1e9}, {7.7, 1.75, 2.238}, {6.6, 1.23, 1.192}, {5.7, 0.79, 0.634}},
+     {{0, 1e9, 1e9}, {8.0, 1.48, 2.055}, {6.3, 1.16, 1.152}, {5.7, 0.49, 0.611}}},     // bf16 8 bits
+    {{{0, 1e9, 1e9}, {7.2, 1.54, 2.097}, {6.0, 1.17, 1.163}, {6.0, 0.45, 0.649}},
+     {{0, 1e9, 1e9}, {6.8, 1.39, 1.920}, {6.5, 0.79, 1.164}, {4.8, 0.47, 0.685}}},     // 16-bit weights
 };
-int pick_among(const PrefillCost* cost, int first, int count, bool round, int M, int NT, int KC, double* t_best) {
+// the share of a busy CU that a launch gives the fullest one, and how many rounds of blocks that is at least
+struct PrefillShare { double share; bool round; };
+PrefillShare prefill_share(const PrefillShape& s, int M, int NT) {
+    const double full = (double)cdiv(NT, 8 / s.ks * s.tpw) * cdiv(M, 16 * s.mb) / 256.0, whole = (double)(long)(full + 0.9999);
+    return {0.5 * (full + whole), whole <= 1.0};
+}
+int pick_shape(int M, int NT, int KC, bool bf, int wbits, int group_size, bool whole, double* t_best) {
+    const int first = (bf || wbits == 16) ? 1 : 0;
+    const PrefillCost* cost = kPrefillCost[wbits == 16 ? 2 : (bf && wbits == 4) ? 1 : 0];
     int best = 1;
     *t_best = 1e30;
-    for (int i = first; i < count; ++i) {
-        const PrefillShape s = kPrefillShapes[i];
-        const double full = (double)cdiv(NT, 8 / s.ks * s.tpw) * cdiv(M, 16 * s.mb) / 256.0;
-        const double whole = (double)(long)(full + 0.9999), share = round && whole <= 1.0 ? 0.0 : cost[i].sat * 0.5 * (full + whole);
-        const double t = cdiv(KC, s.ks) * (share > cost[i].lat ? share : cost[i].lat) + 2.5;
+    for (int i = first; i < kPrefillShapeCount; ++i) {
+        const double share = cost[i].sat * prefill_share(kPrefillShapes[i], M, NT).share;
+        const double t = cdiv(KC, kPrefillShapes[i].ks) * (share > cost[i].lat ? share : cost[i].lat) + 2.5;
         if (t < *t_best) { *t_best = t; best = i; }
+    }
+    if (best >= kWholeShapes) return best;
+    const UnslicedCost* own = kUnslicedCost[wbits == 16 ? 8 : wbits == 8 ? (bf ? 7 : 6) : (bf ? 3 : 0) + (group_size == 128 ? 0 : group_size == 64 ? 1 : 2)][whole];
+    double least = 1e30;
+    for (int i = first; i < kWholeShapes; ++i) {
+        const PrefillShare sh = prefill_share(kPrefillShapes[i], M, NT);
+        const double share = sh.round ? 0.0 : own[i].sat * sh.share, t = own[i].base + KC * (share > own[i].lat ? share : own[i].lat);
+        if (t < least) { least = t; best = i; }
     }
     return best;
 }
-int pick_shape(int M, int NT, int KC, bool bf, int wbits, double* t_best) {
-    const int first = (bf || wbits == 16) ? 1 : 0;
-    const int best = pick_among(kPrefillCost[wbits == 16 ? 2 : (bf && wbits == 4) ? 1 : 0], first, kPrefillShapeCount, false, M, NT, KC, t_best);
-    if (best >= kWholeShapes || (bf && wbits == 4)) return best;
-    double t;
-    return pick_among(kWholeCost[wbits == 16 ? 3 : wbits == 8 ? (bf ? 2 : 1) : 0], first, kWholeShapes, true, M, NT, KC, &t);
-}
+// K below 2^23: the 128 x 512 form's row offsets are formed past the last row, in 32 bits.
+bool prefill_whole(const void* x, int K) { return (uintptr_t)x % 16 == 0 && K % 128 == 0 && K < 1 << 23; }
 
-// The loop without branches where x allows it.  Not for 128 x 512 under groups of 32 or 64 (two or four scales a chunk and tile have no registers left), nor for 64 x 256
-// in groups of 32 and the 64-row forms of bf16 W4 (held in one piece the compiler takes more than 128 or 80 registers for them and a block less fits a CU: 37888 x 3584 at
-// 4096 rows 1293 -> 1485 us), nor for 4-bit weights under sliced K (8 or 16 products and 56 operand instructions a wave and chunk: 2 % either way, 3584 x 18944 at 104 rows
-// 59 -> 60 to 62 us).  K below 2^23: the 128 x 512 form's row offsets are formed past the last row, in 32 bits.
 template <int WBITS, int GS, bool BF, int I>
 void launch_shape_t(const GemmParams& p, hipStream_t st) {
     constexpr PrefillShape s = kPrefillShapes[I];
     const dim3 grid(cdiv(p.NT, 8 / s.ks * s.tpw), cdiv(p.M, 16 * s.mb));
     const int band = prefill_short(p, WBITS, 8 / s.ks * s.tpw * 16) ? 0 : prefill_band(grid.y, grid.x);
-    constexpr bool straight = !(I == 0 && (GS == 1 || GS == 2)) && !(I == 2 && GS == 1) && !(BF && WBITS == 4 && s.mb == 4) && !(WBITS == 4 && s.ks > 1);
-    if constexpr (straight) {
-        if ((uintptr_t)p.x % 16 == 0 && p.K % 128 == 0 && p.K < 1 << 23) {
+    if constexpr (prefill_straight(I, WBITS, GS, BF)) {
+        if (prefill_whole(p.x, p.K)) {
             hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, true>), grid, dim3(512), 0, st, p, band);
             return;
         }
@@ -502,10 +538,15 @@ extern "C" int64_t mi355_gemm_prefill_tile(int32_t id, int32_t rows, int32_t col
     return (int64_t)by << 32 | bx;
 }
 
-// The block shape of a call, by its place in kPrefillShapes: NT = N_pad / 16, KC = K_pad / 128.
+// The block shape of a call, by its place in kPrefillShapes: NT = N_pad / 16, KC = K_pad / 128.  4-bit weights in groups of 128, x on 16 bytes, K a multiple of 128.
 extern "C" int mi355_gemm_prefill_shape(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits) {
+    return mi355_gemm_prefill_form(M, NT, KC, bf16, wbits, 128, 1) & 15;
+}
+// The same for any call (whole: x on 16 bytes and K a multiple of 128), plus 16 where it runs the loop without branches.
+extern "C" int mi355_gemm_prefill_form(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits, int32_t group_size, int32_t whole) {
     double t;
-    return pick_shape(M, NT, KC, bf16 != 0, wbits, &t);
+    const int s = pick_shape(M, NT, KC, bf16 != 0, wbits, group_size, whole != 0, &t);
+    return s + (whole && prefill_straight(s, wbits, group_size / 32, bf16 != 0) ? 16 : 0);
 }
 
 // Direct-mode launch (fused epilogue in p.mode).  MI355_ERR_UNSUPPORTED: shape / format not covered, caller falls back.
@@ -517,7 +558,7 @@ extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, dou
     hipStream_t st = (hipStream_t)stream;
     const bool bf = g.bf16 != 0;
     double t;
-    const int s = pick_shape(g.M, g.NT, g.KC, bf, wbits, &t);
+    const int s = pick_shape(g.M, g.NT, g.KC, bf, wbits, group_size, prefill_whole(g.x, g.K), &t);
     if (t > t_limit) return MI355_ERR_UNSUPPORTED;
     if (wbits == 16) return bf ? launch_shape<16, 0, true>(s, g, st) : launch_shape<16, 0, false>(s, g, st);
     if (wbits == 8 && group_size == 0) return bf ? launch_shape<8, 0, true>(s, g, st) : launch_shape<8, 0, false>(s, g, st);

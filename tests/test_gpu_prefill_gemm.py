@@ -27,7 +27,8 @@ def _dense64(c):
 # holds the list to that
 SHAPES = [(65, 136, 24), (66, 4864, 64), (129, 1280, 200), (130, 896, 1152), (257, 640, 4096), (513, 384, 9728), (1100, 256, 8208),
           (131, 200, 37880), (201, 136, 37880), (300, 2048, 4104), (1537, 136, 4104), (2050, 136, 24), (517, 384, 37880),
-          (257, 136, 37880), (1537, 136, 8208), (257, 136, 8208), (777, 104, 8208)]
+          (257, 136, 37880), (1537, 136, 8208), (257, 136, 8208), (777, 104, 8208),
+          (417, 264, 8208), (326, 904, 16392), (263, 1160, 37880), (326, 904, 37880), (130, 520, 16392)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -53,7 +54,8 @@ def test_prefill_gemm_shapes(kind, group, dtype, M, K, N):
 
 # K a multiple of 128 (1 to 9 chunks, odd and even, fewer than the slices of K), every tile shape, the last row tile full, of one row, of some
 WHOLE = [(65, 128, 48), (100, 256, 1152), (130, 384, 896), (300, 512, 896), (577, 640, 1152), (129, 1152, 4600), (513, 384, 9728), (640, 1024, 4104), (1100, 256, 8208), (2049, 384, 4104),
-         (300, 896, 37880), (1537, 1152, 4104), (150, 384, 37880), (400, 896, 4104), (257, 128, 37880), (1537, 128, 8208), (257, 128, 8208)]
+         (300, 896, 37880), (1537, 1152, 4104), (150, 384, 37880), (400, 896, 4104), (257, 128, 37880), (1537, 128, 8208), (257, 128, 8208), (187, 128, 37880),
+         (325, 768, 37880)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -74,6 +76,33 @@ def test_prefill_gemm_straight_loop(kind, group, dtype):
         seen.add(_C.lib().mi355_gemm_prefill_shape(M, -(-N // 16), K // 128, int(dtype == torch.bfloat16), w.wbits))
     can = {0, 1, 2, 3, 4, 5, 6} - ({0} if kind == "fp16" or dtype == torch.bfloat16 else set())
     assert seen >= can, seen
+
+
+# the shapes of a class that have a loop without branches (any K, x on 16 bytes): the others run the general loop either way
+STRAIGHT = {("w4", 128, False): {0, 1, 2, 3}, ("w4", 64, False): {1, 2, 3}, ("w4", 32, False): {1, 3}, ("w4", 128, True): {1}, ("w4", 64, True): {1}, ("w4", 32, True): set(),
+            ("int8", 0, False): {0, 1, 2, 3, 4, 5, 6}, ("int8", 0, True): {1, 2, 3, 4, 5, 6}, ("fp16", 0, False): {1, 2, 3, 4, 5, 6}, ("fp16", 0, True): {1, 2, 3, 4, 5, 6}}
+
+
+@pytest.mark.parametrize("kind,group,bf16", STRAIGHT)
+def test_prefill_gemm_both_loops(kind, group, bf16):
+    """Calls that take the loop without branches with x on 16 bytes and the general one off them, in every shape that has both: the same bits."""
+    dtype, bits = (torch.bfloat16 if bf16 else torch.float16), {"w4": 4, "int8": 8, "fp16": 16}[kind]
+    form = lambda M, K, N, whole: _C.lib().mi355_gemm_prefill_form(M, -(-N // 16), K // 128, int(bf16), bits, group, int(whole))
+    left = set(STRAIGHT[kind, group, bf16])
+    for M, K, N in WHOLE + [(370, 896, 37880), (130, 640, 16392), (580, 384, 11016), (835, 640, 8208), (2000, 896, 4104)]:
+        whole, off = form(M, K, N, True), form(M, K, N, False)
+        assert off < 16 and (whole >= 16) == (whole & 15 in STRAIGHT[kind, group, bf16])
+        if whole & 15 not in left:
+            continue
+        left.discard(whole & 15)
+        c = model.synth_linear(K, N, kind, "cpu", _gen(K + N), group or 128)
+        if kind == "fp16":
+            c.w = c.w.to(dtype)
+        w, x = c.pack(dtype=dtype).to(DEV), (torch.randn(M, K, generator=_gen(M)) * 0.5).to(dtype).to(DEV)
+        moved = torch.zeros(M * K + 8, dtype=dtype, device=DEV)[4:4 + M * K].view(M, K).copy_(x)
+        assert x.data_ptr() % 16 == 0 and moved.data_ptr() % 16 == 8
+        assert torch.equal(ops.linear(x, w).view(torch.int16), ops.linear(moved, w).view(torch.int16)), (M, K, N, whole, off)
+    assert not left, left
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
