@@ -425,6 +425,7 @@ typedef struct {
     int32_t n_sequences, step;
     int32_t* token_ids;
 } mi355_sampler_host_t;
+int mi355_sampler_filters(const int32_t* top_k, const float* top_p, int32_t rows, int32_t V);   /* host: bit 0 every row greedy, bit 1 some row has a filter */
 size_t mi355_sampler_step_stage_bytes(int32_t rows, int32_t step);
 int mi355_sampler_step_takes(const mi355_sampler_host_t* host, int32_t rows, int32_t V);
 int mi355_sampler_step(float* logits, int32_t rows, int32_t V, int32_t ld, const mi355_sampler_host_t* host, void* pinned, void* device, int32_t* ids, void* workspace, mi355_stream_t stream);

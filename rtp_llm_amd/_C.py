@@ -131,6 +131,7 @@ SIGNATURES = {
     "mi355_sampling_probs": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp]),
     "mi355_sampling_draw_workspace_bytes": (sz, [i32, i32]),
     "mi355_sampling_draw": (i32, [vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp, vp, vp, vp, vp]),
+    "mi355_sampler_filters": (i32, [vp, vp, i32, i32]),
     "mi355_sampler_step_stage_bytes": (sz, [i32, i32]),
     "mi355_sampler_step_takes": (i32, [C.POINTER(SamplerHost), i32, i32]),
     "mi355_sampler_step": (i32, [vp, i32, i32, i32, C.POINTER(SamplerHost), vp, vp, vp, vp, vp]),

@@ -1391,20 +1391,34 @@ extern "C" int mi355_sampling_draw(float* logits, int32_t rows, int32_t V, int32
 
 // The host's part of a step in one place: of 184 us for 64 rows of 152064 values 110 were Python looking at the vectors and packing them, a copy from pageable memory and one back (108 us now).
 namespace {
+struct Filters { bool greedy, some; };
+Filters filters(const int32_t* top_k, const float* top_p, int rows, int V) {
+    bool greedy = true, some_k = false, some_p = false;
+    for (int r = 0; r < rows; ++r) {
+        greedy = greedy && top_k[r] == 1;
+        some_k = some_k || (top_k[r] > 0 && top_k[r] < V);
+        some_p = some_p || (top_p[r] != 1.f && !(fabsf(top_p[r]) < 1e-7f));
+    }
+    return {greedy, some_k || some_p};
+}
 struct HostLook { bool takes, scale, pen; };
 HostLook look(const mi355_sampler_host_t& h, int rows, int V) {
-    bool greedy = true, some_k = false, some_p = false, scale = false, pen = false;
+    const Filters f = filters(h.top_k, h.top_p, rows, V);
+    bool scale = false, pen = false;
     for (int r = 0; r < rows; ++r) {
-        greedy = greedy && h.top_k[r] == 1;
-        some_k = some_k || (h.top_k[r] > 0 && h.top_k[r] < V);
-        some_p = some_p || (h.top_p[r] != 1.f && !(fabsf(h.top_p[r]) < 1e-7f));
         scale = scale || h.temperature[r] != 1.f;
         if (h.repetition) pen = pen || h.repetition[r] != 1.f || h.presence[r] != 0.f || h.frequency[r] != 0.f;
     }
-    return {!greedy && (some_k || some_p) && h.step < kShortHistory && rows <= 65535, scale, pen};
+    return {!f.greedy && f.some && h.step < kShortHistory && rows <= 65535, scale, pen};
 }
 } // namespace
 
+// bit 0: every row greedy (top_k 1); bit 1: some row has a filter.  Of 110 us of Python for a step that this file does not take, looking at the vectors for it was 4 to 8.
+extern "C" int mi355_sampler_filters(const int32_t* top_k, const float* top_p, int32_t rows, int32_t V) {
+    if (!top_k || !top_p || rows <= 0) return 1;
+    const Filters f = filters(top_k, top_p, rows, V);
+    return f.greedy | f.some << 1;
+}
 extern "C" size_t mi355_sampler_step_stage_bytes(int32_t rows, int32_t step) { return rows > 0 && step >= 0 ? (size_t)rows * ((size_t)step + 10) * 4 : 0; }
 extern "C" int mi355_sampler_step_takes(const mi355_sampler_host_t* host, int32_t rows, int32_t V) {
     return host && host->temperature && host->top_k && host->top_p && rows > 0 && host->step >= 0 && !host->repetition == !host->presence && !host->repetition == !host->frequency &&

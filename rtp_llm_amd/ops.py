@@ -563,15 +563,27 @@ def sampling_draw(logits: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Op
     return ids
 
 
+def sampler_filters(top_k: torch.Tensor, top_p: torch.Tensor, V: int):
+    """(every row greedy, some row of a sampling step has a filter) of host vectors, or None where they are not contiguous host memory of int32 and float32 with as many rows."""
+    if top_k.dtype != torch.int32 or top_p.dtype != torch.float32 or not top_k.is_cpu or not top_p.is_cpu or top_k.numel() != top_p.numel() or not top_k.is_contiguous() or not top_p.is_contiguous():
+        return None
+    f = _C.lib().mi355_sampler_filters(top_k.data_ptr(), top_p.data_ptr(), top_k.numel(), V)
+    return bool(f & 1), bool(f & 2)
+
+
 def sampler_vectors(logits: torch.Tensor, token_ids: torch.Tensor, temperature: torch.Tensor, penalties, top_k: torch.Tensor, top_p: torch.Tensor, uniform: torch.Tensor,
-                    input_lengths: torch.Tensor, sequence_lengths: torch.Tensor):
+                    input_lengths: torch.Tensor, sequence_lengths: torch.Tensor, seen=None):
     """What sampling_draw takes as `host`: the vectors of a whole step, penalties (repetition, presence, frequency) or None, history token_ids [B, step + 1].  None where mi355_sampler_step
-    does not take the step, or a tensor is not contiguous host memory of its kernel's type with one value per row."""
+    does not take the step, or a tensor is not contiguous host memory of its kernel's type with one value per row.  seen: sampler_filters of the same top_k and top_p, where the caller has it."""
     f32, i32 = torch.float32, torch.int32
-    if logits.dim() != 2 or logits.dtype != f32 or not logits.is_contiguous() or token_ids.dim() != 2:
+    if logits.dim() != 2 or logits.dtype != f32 or not logits.is_contiguous() or token_ids.dim() != 2 or token_ids.shape[1] > 2048:
         return None
     B, V = logits.shape
-    vectors = [(temperature, f32), (top_p, f32), (uniform, f32), (top_k, i32)]
+    vectors = [(temperature, f32), (uniform, f32)]
+    if seen is None:
+        vectors += [(top_p, f32), (top_k, i32)]
+    elif top_k.numel() != B:
+        return None
     if penalties is not None:
         vectors += [(t, f32) for t in penalties] + [(input_lengths, i32)]
         if sequence_lengths.numel() > B or sequence_lengths.dtype != i32 or not sequence_lengths.is_cpu or not sequence_lengths.is_contiguous():
@@ -586,7 +598,8 @@ def sampler_vectors(logits: torch.Tensor, token_ids: torch.Tensor, temperature: 
     if penalties is not None:
         host.repetition, host.presence, host.frequency = (t.data_ptr() for t in penalties)
         host.input_lengths, host.sequence_lengths, host.n_sequences = input_lengths.data_ptr(), sequence_lengths.data_ptr(), sequence_lengths.numel()
-    return host if _C.lib().mi355_sampler_step_takes(host, B, V) else None
+    takes = _C.lib().mi355_sampler_step_takes(host, B, V) if seen is None else seen[1] and not seen[0] and B <= 65535
+    return host if takes else None
 
 
 def ban_repeat_ngram(logits: torch.Tensor, token_ids: torch.Tensor, sequence_last_index: torch.Tensor,

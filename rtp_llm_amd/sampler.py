@@ -76,12 +76,17 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
     step = int(params.step)
     if params.token_ids.shape != (B, step + 1):
         raise ValueError("sample_greedy: token_ids must be [batch_size, step + 1]")
-    # vectors and history on the host, nothing between the penalties and the draw: the whole step in one native call, where some row has a filter
+    # vectors and history on the host, nothing between the penalties and the draw: the whole step in one native call, where some row has a filter.  Where none has, what was seen serves below,
+    # and the step costs what it did without the question
     penalties = (params.repetition_penalty, params.presence_penalty, params.frequency_penalty)
+    seen = None
     if logits.is_cuda and params.uniform is not None and params.output_all_probs is None and (params.no_repeat_ngram_size is None or params.sequence_lengths.numel() == 0) and \
             (penalties[0] is None or (penalties[1] is not None and penalties[2] is not None)):
-        host = ops.sampler_vectors(logits, params.token_ids, params.temperature, None if penalties[0] is None else penalties, params.top_k, params.top_p, params.uniform,
-                                   params.input_lengths, params.sequence_lengths)
+        seen = ops.sampler_filters(params.top_k, params.top_p, V)
+        host = None
+        if seen is None or (seen[1] and not seen[0]):
+            host = ops.sampler_vectors(logits, params.token_ids, params.temperature, None if penalties[0] is None else penalties, params.top_k, params.top_p, params.uniform,
+                                       params.input_lengths, params.sequence_lengths, seen)
         if host is not None:
             return ops.sampling_draw(logits, None, None, params.uniform, host=host)
     temperature = _host(params.temperature, torch.float32)
@@ -93,7 +98,7 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
         rep, pres, freq = (_host(t, torch.float32) for t in (params.repetition_penalty, params.presence_penalty, params.frequency_penalty))
         penalise = _off(rep, 1.0) or _off(pres, 0.0) or _off(freq, 0.0)
     top_k = _host(params.top_k, torch.int32)
-    all_greedy = not _off(top_k, 1)
+    all_greedy = not _off(top_k, 1) if seen is None else seen[0]
     draw = not all_greedy
     if draw and params.uniform is None:
         raise ValueError("sample_greedy: sampling rows need params.uniform (one value in [0, 1) per row)")
@@ -122,7 +127,10 @@ def sample_greedy(params: GreedyParams) -> torch.Tensor:
         top_p = _host(params.top_p, torch.float32).clone()
         p = top_p.numpy()
         p[np.abs(p) < 1e-7] = 1.0
-        filtered = bool((p != 1.0).any()) or (_off(top_k, 0) and bool(((top_k.numpy() > 0) & (top_k.numpy() < V)).any()))
+        if seen is not None:
+            filtered = seen[1]
+        else:
+            filtered = bool((p != 1.0).any()) or (_off(top_k, 0) and bool(((top_k.numpy() > 0) & (top_k.numpy() < V)).any()))
         up.update(top_k=top_k, top_p=top_p)
         if params.uniform.device.type == "cpu":
             up["uniform"] = params.uniform.to(torch.float32)

@@ -132,3 +132,28 @@ def test_step_from_host_vectors(monkeypatch, B, V, n, pen, plain_t):
         got = run(True, change)
         assert got[0] == want[0] and torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
     assert [t is not None for t in taken] == [n < 2048, False, B == 1 and n < 2048]
+
+
+@pytest.mark.parametrize("n,top_k,pen", [(3, 0, False), (3, 1, True), (3, 0, True), (2048, 5, True), (2100, 0, False)])
+def test_steps_that_stay_general(monkeypatch, n, top_k, pen):
+    """Steps without a filter never have their vectors built for the native call, and those past its history are turned away before a vector is looked at: ids, probabilities and history as without
+    the question."""
+    B, V = 6, 500
+    x = torch.randn(B, V, device=DEV, generator=torch.Generator(device=DEV).manual_seed(n)) * 3
+    built, vectors, filters = [], ops.sampler_vectors, ops.sampler_filters
+
+    def run(native):
+        monkeypatch.setattr(ops, "sampler_vectors", (lambda *a: built.append(vectors(*a))) if native else (lambda *a: None))
+        monkeypatch.setattr(ops, "sampler_filters", filters if native else (lambda *a: None))
+        g = torch.Generator().manual_seed(n)
+        p = dict(top_k=torch.full((B,), top_k, dtype=torch.int32), top_p=torch.ones(B), temperature=torch.full((B,), 0.7), uniform=torch.rand(B, generator=g))
+        if pen:
+            p.update(repetition_penalty=torch.full((B,), 1.3), presence_penalty=torch.full((B,), 0.2), frequency_penalty=torch.zeros(B))
+        tokens, lens = torch.randint(0, V, (B, n + 1), generator=g, dtype=torch.int32), torch.full((B,), n, dtype=torch.int32)
+        logits = x.clone()
+        ids = sampler.sample_greedy(sampler.GreedyParams(logits=logits, input_lengths=lens, sequence_lengths=lens, token_ids=tokens, step=n, **p))
+        return ids.tolist(), logits, tokens
+
+    want, got = run(False), run(True)
+    assert got[0] == want[0] and torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    assert built == ([None] if top_k == 5 else [])

@@ -189,3 +189,24 @@ def test_sort_free_threshold_formulation_equals_sort_and_cumsum(V, levels):
     top_k = torch.tensor([0, 0, V // 3, 7, V + 5, 1], dtype=torch.int32)
     want = oracle.top_k_top_p_filter(probs, top_k, top_p)
     assert torch.equal(_threshold_model(probs, top_k, top_p), want)
+
+
+@pytest.mark.parametrize("V", [1, 5, 1000])
+def test_sampler_filters_of_host_vectors(V):
+    """What one native look at top_k and top_p says is what the step's flow finds with numpy: rows all greedy, some row filtered, top_p of next to nothing standing for 1."""
+    from rtp_llm_amd import ops
+    ks, ps = [-1, 0, 1, 4, V - 1, V, V + 1], [0.0, 1e-8, -1e-8, 1e-7, 2e-7, 0.5, 1.0, 1.5, float("nan")]
+    rng = np.random.default_rng(V)
+    for n in [1] * 200 + [2, 3, 64] * 40:
+        k, p = rng.choice(ks, n).astype(np.int32), rng.choice(ps, n).astype(np.float32)
+        if rng.random() < 0.5:
+            p[:] = rng.choice([0.0, 1.0], n)
+        if rng.random() < 0.3:
+            k[:] = rng.choice([0, 1, V], 1)
+        q = p.copy()
+        q[np.abs(q) < 1e-7] = 1.0
+        want = (not bool((k != 1).any()), bool((q != 1.0).any()) or bool(((k > 0) & (k < V)).any()))
+        assert ops.sampler_filters(torch.from_numpy(k), torch.from_numpy(p), V) == want, (k, p)
+    k, p = torch.ones(6, dtype=torch.int32), torch.ones(6)
+    assert ops.sampler_filters(k.long(), p, V) is None and ops.sampler_filters(k, p.double(), V) is None
+    assert ops.sampler_filters(k[::2], p[:3], V) is None and ops.sampler_filters(k, p[:3], V) is None
