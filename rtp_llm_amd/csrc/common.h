@@ -114,6 +114,26 @@ template <bool BF> __device__ __forceinline__ float act_round(float v) {   // th
     if constexpr (BF) return (float)(bf16)v;
     else              return (float)(f16)v;
 }
+// silu(gate) * up of two interleaved columns {g0, u0, g1, u1} of a linear, which are rounded to the activation type first, as one dword.  fp16: the first product is rounded once, the second to fp32
+// and from there to fp16.  The two differ in the last bit now and then; they are written out so that every kernel that one row of a step may go through (by the number of rows) has the same bits,
+// whatever the compiler would fold around a plain product.
+template <bool BF> __device__ __forceinline__ uint32_t silu_pair(f32x4 v) {
+    float sg[2], u[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const float g = act_round<BF>(v[2 * t]);
+        u[t] = act_round<BF>(v[2 * t + 1]);
+        sg[t] = g / (1.f + __expf(-g));
+    }
+    if constexpr (BF) return act_pack<BF>(sg[0] * u[0], sg[1] * u[1]);
+    else {
+        float second = sg[1] * u[1];
+        uint32_t first;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(first) : "v"(sg[0]), "v"(u[0]));
+        asm("" : "+v"(second));
+        return (first & 0xFFFFu) | (uint32_t)__builtin_bit_cast(uint16_t, (f16)second) << 16;
+    }
+}
 template <bool BF> __device__ __forceinline__ float act_dot_ones(uint32_t v, float acc) {   // acc + v[0] + v[1]
     if constexpr (BF) { const bf16x2 ones = {(bf16)1.f, (bf16)1.f}; return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, v), ones, acc, false); }
     else              { const f16x2 ones = {(f16)1.f, (f16)1.f};   return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, v), ones, acc, false); }

@@ -443,16 +443,11 @@ __global__ __launch_bounds__(64 * NWN * KG) void gemm_wq_kernel(const GemmParams
                         *reinterpret_cast<u32x2*>((f16*)p.y + (size_t)m * p.ldy + n0) = o;
                     }
                 } else { // MODE_SILU: (gate, up) interleaved; round GEMM output to the activation dtype first
-                    float sg[2];
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        const float g = act_round<BF>(v[2 * t]), u = act_round<BF>(v[2 * t + 1]);
-                        sg[t] = (g / (1.f + __expf(-g))) * u;
-                    }
+                    const uint32_t pair = silu_pair<BF>(v);
                     if (p.y_img)
-                        *reinterpret_cast<uint32_t*>((f16*)p.y + act_img_index(m, n0 >> 1, (p.M + 15) >> 4)) = act_pack<false>(img_val<BF>(act_round<BF>(sg[0])), img_val<BF>(act_round<BF>(sg[1])));
+                        *reinterpret_cast<uint32_t*>((f16*)p.y + act_img_index(m, n0 >> 1, (p.M + 15) >> 4)) = act_pack<false>(img_val<BF>(act_lo<BF>(pair)), img_val<BF>(act_hi<BF>(pair)));
                     else
-                        *reinterpret_cast<uint32_t*>((f16*)p.y + (size_t)m * p.ldy + (n0 >> 1)) = act_pack<BF>(sg[0], sg[1]);
+                        *reinterpret_cast<uint32_t*>((f16*)p.y + (size_t)m * p.ldy + (n0 >> 1)) = pair;
                 }
             }
         }
@@ -501,16 +496,11 @@ __global__ __launch_bounds__(256) void reduce_epilogue_kernel(const float* __res
             *reinterpret_cast<u32x2*>((f16*)y + (size_t)m * ldy + n0) = o;
         }
     } else {
-        float sg[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const float g = act_round<BF>(v[2 * t]), u = act_round<BF>(v[2 * t + 1]);
-            sg[t] = (g / (1.f + __expf(-g))) * u;
-        }
+        const uint32_t pair = silu_pair<BF>(v);
         if (y_img_mblk > 0)
-            *reinterpret_cast<uint32_t*>((f16*)y + act_img_index(m, n0 >> 1, y_img_mblk)) = act_pack<false>(img_val<BF>(act_round<BF>(sg[0])), img_val<BF>(act_round<BF>(sg[1])));
+            *reinterpret_cast<uint32_t*>((f16*)y + act_img_index(m, n0 >> 1, y_img_mblk)) = act_pack<false>(img_val<BF>(act_lo<BF>(pair)), img_val<BF>(act_hi<BF>(pair)));
         else
-            *reinterpret_cast<uint32_t*>((f16*)y + (size_t)m * ldy + (n0 >> 1)) = act_pack<BF>(sg[0], sg[1]);
+            *reinterpret_cast<uint32_t*>((f16*)y + (size_t)m * ldy + (n0 >> 1)) = pair;
     }
 }
 

@@ -238,24 +238,7 @@ __global__ __launch_bounds__(D <= 3 ? 1024 : 512) void gemm_rows16_kernel(const 
             for (int e = 0; e < 4; ++e) o[e] = act_round<BF>(v[e]) + r[e];
             *reinterpret_cast<u32x2*>(p.res_out + (size_t)jj * p.N + n0) = u32x2{act_pack<BF>(o[0], o[1]), act_pack<BF>(o[2], o[3])};
         } else {
-            const f32x4 v = acc;                                      // one slice (checked on the host), this wave's
-            float sg[2], u[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float g = act_round<BF>(v[2 * e]);
-                u[e] = act_round<BF>(v[2 * e + 1]);
-                sg[e] = g / (1.f + __expf(-g));
-            }
-            uint32_t out;
-            if constexpr (BF) out = act_pack<BF>(sg[0] * u[0], sg[1] * u[1]);
-            else {   // as the staged kernel's code has it: the first product rounded once, the second to fp32 first
-                float second = sg[1] * u[1];
-                uint32_t first;
-                asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(first) : "v"(sg[0]), "v"(u[0]));
-                asm("" : "+v"(second));
-                out = (first & 0xFFFFu) | (uint32_t)__builtin_bit_cast(uint16_t, (f16)second) << 16;
-            }
-            *reinterpret_cast<uint32_t*>(p.y + (size_t)jj * (p.N / 2) + (n0 >> 1)) = out;
+            *reinterpret_cast<uint32_t*>(p.y + (size_t)jj * (p.N / 2) + (n0 >> 1)) = silu_pair<BF>(acc);   // one slice (checked on the host), this wave's
         }
     }
 }
