@@ -17,7 +17,7 @@
 //   * up to 4 rows every GEMM is a full-K launch with its consumer fused (gemm_fullk.hip), 5 launches:
 //     [RMSNorm on load +] QKV + bias + RoPE + KV write -> attention -> O + residual (leaves the
 //     per-tile sums of squares) -> RMSNorm on load + gate_up + SiLU-gate -> down + residual;
-//   * up to 8 rows, 16-bit weights whose K slices are short (small models): five launches as well, gemm_rows16.hip (six with an INT8 cache);
+//   * up to 8 rows, 16-bit weights, hidden size up to 1024 (tp = 1): five launches as well, gemm_rows16.hip (six with an INT8 cache); the weight-prefetch mask does nothing on those steps;
 //   * other formats / TP (above 12 rows): QKV GEMM (split-K slabs) -> reduce+bias+RoPE+KV-write -> paged attention
 //     -> O GEMM (slabs) -> reduce+residual+RMSNorm -> gate_up GEMM with fused SiLU-gate -> down GEMM (slabs) ->
 //     reduce+residual+RMSNorm (already the next layer's input norm).  No standalone reduce / add / activation kernels.

@@ -1,7 +1,7 @@
-// Linears of up to 8 rows through 16-bit weights with the whole layer's elementwise work fused in, gfx950: a step of a small model is a chain of short launches.
+// Linears of up to 8 rows through 16-bit weights, hidden size at most 1024, with the whole layer's elementwise work fused in, gfx950: a step of a small model is a chain of short launches.
 //
 // A 0.5B model in fp16 reads 30 MB a layer, 6 us of memory, in launches of 2.5 to 7.5 us; two of eight were RMSNorms, one RoPE and the cache write, and three handed fp32 slabs of split K
-// to them.  Here a block owns one to four 16-column tiles and all of K, its waves are the tiles' K slices (slice s of a tile is what split s of the staged kernel of gemm.hip was: the same
+// to them.  Taken where gate_up is one slice of at most eight chunks of 128, so hidden sizes up to 1024, and the other linears' slices are at most three chunks.  Here a block owns one to three 16-column tiles and all of K, its waves are the tiles' K slices (slice s of a tile is what split s of the staged kernel of gemm.hip was: the same
 // chunks in the same order, each slice's sum by one wave, the slices added in order), and
 //   NORM   the input rows are normalised on load: every block rebuilds the rows' sums of squares, lane by lane as add_rmsnorm_kernel adds them, while its weights are on their way;
 //   ROPE   bias + rotation + Q + 16-bit cache write in the epilogue, the tile pair (d, d + hd / 2) of one head a block;     SLAB  fp32 sums, for the cache writer that quantises;
@@ -33,11 +33,12 @@ struct Rows16Params {
 // Every block normalises all rows, which costs more than the launches it saves from some 12 rows on: a step of the 0.5B model, the staged launches / these, us: 1 row 762 / 618, 4 (8-bit cache)
 // 867 / 778, 8 889 / 806; 12 825 / 817, 16 903 / 940, 16 (8-bit cache) 916 / 1009.
 constexpr int kRows16 = 8;
+constexpr int kHidden = 1024;                        // columns of the residual rows
 constexpr int kNormJobs = 2;                         // (row, 64 lanes of 8 columns) pairs a wave adds up at most
 
-// D: chunks a slice has at most; all of them are asked for at once.  What a block waits for is the number of its vector-memory instructions as much as their bytes (a wave load of 16 bytes a
+// D: chunks a slice has at most (SILU: 3 or 8; 3 in the others); all of them are asked for at once.  What a block waits for is the number of its vector-memory instructions as much as their bytes (a wave load of 16 bytes a
 // lane is 16 cycles of a compute unit's address path whatever its lanes ask for), so none is half empty:
-// PARTS 2: a block owns eight of its tiles' sixteen columns (block b: half b & 1); a wave load is two k-steps of them, lanes jj < 8 the even one, and the odd one is turned by eight lanes
+// PARTS 2 (RESID; ROPE and SLAB of up to 128 blocks): a block owns eight of its tiles' sixteen columns (block b: half b & 1); a wave load is two k-steps of them, lanes jj < 8 the even one, and the odd one is turned by eight lanes
 //   into the product's first rows.  Twice the blocks where whole tiles leave more than half of the chip without one (down_proj of the 0.5B model, 56 tiles: 6.4 us whole).
 // XL (RESID): activation loads a chunk.  1 (M <= 4): lane jj row jj % 4 of k-step jj / 4; 2 (M <= 8): row jj % 8, k-steps 2 l + jj / 8.
 template <bool BF, int EPI, int D, int PARTS, int XL = 1>
@@ -243,42 +244,35 @@ __global__ __launch_bounds__(D <= 3 ? 1024 : 512) void gemm_rows16_kernel(const 
     }
 }
 
-// The launch's shape, or false: M rows, the splits that the staged kernel would take (mi355_gemm_plan: shapes without k-groups), no slice of more than eight chunks, room for the
-// normalised rows and their sums.
+// The launch's shape, or false: M rows, the splits that the staged kernel would take (mi355_gemm_plan: shapes without k-groups), no slice of more chunks than a form has (gate_up's one slice
+// bounds the hidden size), few enough columns for the grid.
 bool rows16_shape(int M, const mi355_weight_t* w, int epi, int max_splits, Rows16Params& p, int& waves, size_t& lds) {
     if (!w || !w->qweight || w->wbits != 16 || M < 1 || M > kRows16 || w->K % 128 != 0 || w->K_pad != w->K || w->N % 16 != 0 || w->N_pad != w->N) return false;
+    if (epi == R16_RESID ? w->N > kHidden : w->K > kHidden) return false;
     int cfg = 0, cps = 0;
     const int slices = mi355_gemm_plan(M, w, max_splits, &cfg, &cps);
-    if (cfg != 5 || cps > 8 || (epi == R16_RESID && cps > 3) || (epi == R16_SILU && slices != 1)) return false;
+    if (cfg != 5 || cps > (epi == R16_SILU ? 8 : 3) || (epi == R16_SILU && slices != 1)) return false;
     p.M = M; p.K = w->K; p.N = w->N; p.N_pad = w->N_pad; p.NT = w->N_pad / 16; p.KC = w->K_pad / 128; p.qw = w->qweight;
     p.slices = slices; p.cps = cps; p.x_bytes = (uint32_t)((size_t)M * w->K * 2);
     // one round of blocks over the chip where a block has room for the tiles (RESID: K is deep, a tile a block); the cache writer's pair
-    p.tw = epi == R16_ROPE ? 2 : epi == R16_SILU ? (cdiv(p.NT, 256) < 4 ? cdiv(p.NT, 256) : 4) : 1;
+    p.tw = epi == R16_ROPE ? 2 : epi == R16_SILU ? cdiv(p.NT, 256) : 1;
     p.units = epi == R16_ROPE ? p.NT / 2 : cdiv(p.NT, p.tw);
-    const int kw = slices * p.tw, most = cps <= 3 ? 16 : 8;
-    waves = epi == R16_RESID ? kw : kw > 8 ? kw : 8;
+    const int kw = slices * p.tw;
+    waves = epi == R16_RESID || kw > 8 ? kw : 8;                      // under the norm at least 8: eight rows of 1024 are kNormJobs jobs a wave
     lds = epi == R16_SILU ? 0 : (size_t)kw * 1024;
-    if (epi != R16_RESID) {
-        const size_t rows = (size_t)M * w->K * 2;
-        if (w->K > 4096 || rows > 48 * 1024 || M * cdiv(w->K / 8, 64) > kNormJobs * waves) return false;
-        lds += rows + 512;
-    }
-    return kw <= most && waves <= most;
+    if (epi != R16_RESID) lds += (size_t)M * w->K * 2 + 512;
+    return waves <= (cps <= 3 ? 16 : 8);
 }
 
-template <bool BF, int EPI, int D, int PARTS>
+template <bool BF, int EPI, int D, int PARTS, int XL = 1>
 void launch_rows16_t(const Rows16Params& p, int waves, size_t lds, hipStream_t st) {
-    const dim3 grid(p.units * PARTS), block(64 * waves);
-    if constexpr (EPI == R16_RESID) {
-        if (p.M <= 4) hipLaunchKernelGGL((gemm_rows16_kernel<BF, EPI, D, PARTS, 1>), grid, block, lds, st, p);
-        else          hipLaunchKernelGGL((gemm_rows16_kernel<BF, EPI, D, PARTS, 2>), grid, block, lds, st, p);
-    } else hipLaunchKernelGGL((gemm_rows16_kernel<BF, EPI, D, PARTS>), grid, block, lds, st, p);
+    hipLaunchKernelGGL((gemm_rows16_kernel<BF, EPI, D, PARTS, XL>), dim3(p.units * PARTS), dim3(64 * waves), lds, st, p);
 }
 template <bool BF, int EPI>
 void launch_rows16_bf(const Rows16Params& p, int waves, size_t lds, hipStream_t st) {
-    const bool half = EPI != R16_SILU && p.units <= 128;
-    if (EPI == R16_RESID || p.cps <= 3) { if (half) launch_rows16_t<BF, EPI, 3, 2>(p, waves, lds, st); else launch_rows16_t<BF, EPI, 3, 1>(p, waves, lds, st); }
-    else if constexpr (EPI != R16_RESID) { if (half) launch_rows16_t<BF, EPI, 8, 2>(p, waves, lds, st); else launch_rows16_t<BF, EPI, 8, 1>(p, waves, lds, st); }
+    if constexpr (EPI == R16_RESID) { if (p.M <= 4) launch_rows16_t<BF, EPI, 3, 2, 1>(p, waves, lds, st); else launch_rows16_t<BF, EPI, 3, 2, 2>(p, waves, lds, st); }
+    else if constexpr (EPI == R16_SILU) { if (p.cps <= 3) launch_rows16_t<BF, EPI, 3, 1>(p, waves, lds, st); else launch_rows16_t<BF, EPI, 8, 1>(p, waves, lds, st); }
+    else { if (p.units <= 128) launch_rows16_t<BF, EPI, 3, 2>(p, waves, lds, st); else launch_rows16_t<BF, EPI, 3, 1>(p, waves, lds, st); }
 }
 template <int EPI>
 int launch_rows16(const Rows16Params& p, bool bf, int waves, size_t lds, hipStream_t st) {
