@@ -14,6 +14,50 @@ struct RopeEpi {
     void*          kv_base;
     f16*           q_out;
 };
+// What a lane of a linear with the rotation and the 16-bit cache write inside does with its columns: x0 = dims d0..d0+3 of head h of row m, x1 = the same of the head's upper half, with the bias and
+// rounded to the activation type; rot gives {cos, sin} of dims d0, d0+1 and d0+2, d0+3 (asked for where the head is rotated); pos_in and blk are the row's position and the block that its table has
+// at the clamped position.  round and pack: the activation type's.  Rows of a negative position are padding and write no cache; a position past the pages or the rotations and a block id outside the
+// cache are refused and counted once a row, by the lane of the first K head's first dims: never somebody else's page.
+template <class Rot, class Round, class Pack>
+__device__ __forceinline__ void rope_rows_out(const RopeEpi& R, int m, int h, int d0, float (&x0)[4], float (&x1)[4], int pos_in, int blk, Rot rot, Round round, Pack pack) {
+    const int half = R.hd >> 1, pos = min(max(pos_in, 0), min(R.max_pos, R.max_blocks * R.page) - 1);
+    const bool is_v = h >= R.nh + R.nkv;
+    if (!is_v) {
+        f32x4 cs01, cs23;
+        rot(cs01, cs23);
+        const float c[4] = {cs01[0], cs01[2], cs23[0], cs23[2]}, s[4] = {cs01[1], cs01[3], cs23[1], cs23[3]};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float r0 = c[e] * x0[e] - s[e] * x1[e];
+            const float r1 = c[e] * x1[e] + s[e] * x0[e];
+            x0[e] = round(r0); x1[e] = round(r1);
+        }
+    }
+    const u32x2 o0 = {pack(x0[0], x0[1]), pack(x0[2], x0[3])}, o1 = {pack(x1[0], x1[1]), pack(x1[2], x1[3])};
+    if (h < R.nh) {
+        f16* dst = R.q_out + ((size_t)m * R.nh + h) * R.hd + d0;
+        *reinterpret_cast<u32x2*>(dst) = o0;
+        *reinterpret_cast<u32x2*>(dst + half) = o1;
+        return;
+    }
+    if (pos_in < 0) return;
+    if (pos != pos_in || blk < 0 || blk >= R.num_blocks) {
+        if (h == R.nh && d0 == 0 && R.oob_count) atomicAdd(R.oob_count, 1);
+        return;
+    }
+    const int kh = is_v ? h - R.nh - R.nkv : h - R.nh, tok = pos % R.page;
+    uint16_t* dst = (uint16_t*)R.kv_base + (((size_t)blk * 2 + (is_v ? 1 : 0)) * R.nkv + kh) * ((size_t)R.page * R.hd);
+    if (!is_v) {
+        *reinterpret_cast<u32x2*>(dst + tok * R.hd + d0) = o0;
+        *reinterpret_cast<u32x2*>(dst + tok * R.hd + d0 + half) = o1;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            dst[(d0 + e) * R.page + tok]        = (uint16_t)(o0[e >> 1] >> (16 * (e & 1)));
+            dst[(d0 + e + half) * R.page + tok] = (uint16_t)(o1[e >> 1] >> (16 * (e & 1)));
+        }
+    }
+}
 struct FullKParams {
     GemmParams g;
     const f16* res_in;

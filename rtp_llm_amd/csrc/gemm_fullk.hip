@@ -435,7 +435,7 @@ __global__ __launch_bounds__(MB >= 3 ? (TPB >= 2 ? 512 : 768) : 1024) void gemm_
     } else {
         // tile pair of one head: this lane holds dims d0..d0+3 (v[0]) and d0+half..+3 (v[1]) of row m = token m
         const RopeEpi& R = fp.r;
-        const int half = R.hd >> 1, hh = R.hd >> 5;
+        const int hh = R.hd >> 5;
         const int h  = tile[0] / (2 * hh);
         const int d0 = (tile[0] % (2 * hh)) * 16 + q * 4;
         float x0[4], x1[4];
@@ -445,48 +445,9 @@ __global__ __launch_bounds__(MB >= 3 ? (TPB >= 2 ? 512 : 768) : 1024) void gemm_
             x0[r] = (float)(f16)(v[0][r] + (float)b0[r]);
             x1[r] = (float)(f16)(v[TPB - 1][r] + (float)b1[r]);
         }
-        const int pos_in  = pre_pos;
-        const int pos_lim = min(R.max_pos, R.max_blocks * R.page);
-        const int pos = min(max(pos_in, 0), pos_lim - 1);
-        const bool is_v = h >= R.nh + R.nkv;
-        if (!is_v) {
-            const f32x4 cs01 = pre_cs[0], cs23 = pre_cs[1];
-            const float c[4] = {cs01[0], cs01[2], cs23[0], cs23[2]}, s[4] = {cs01[1], cs01[3], cs23[1], cs23[3]};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float r0 = c[r] * x0[r] - s[r] * x1[r];
-                const float r1 = c[r] * x1[r] + s[r] * x0[r];
-                x0[r] = (float)(f16)r0; x1[r] = (float)(f16)r1;
-            }
-        }
-        f16x4 o0, o1;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) { o0[r] = (f16)x0[r]; o1[r] = (f16)x1[r]; }
         FK_STAMP(5);
-        if (h < R.nh) {
-            f16* dst = R.q_out + ((size_t)m * R.nh + h) * R.hd + d0;
-            *reinterpret_cast<f16x4*>(dst) = o0;
-            *reinterpret_cast<f16x4*>(dst + half) = o1;
-            return;
-        }
-        const int kh = is_v ? h - R.nh - R.nkv : h - R.nh;
-        if (pos_in < 0) return;                                  // padding row of a multi-row step
-        const int blk = pre_blk;
-        if (pos != pos_in || blk < 0 || blk >= R.num_blocks) {   // stale position / block id: never write somebody else's page
-            if (h == R.nh && d0 == 0 && R.oob_count) atomicAdd(R.oob_count, 1);
-            return;
-        }
-        const int tok = pos % R.page;
-        const size_t head_elems = (size_t)R.page * R.hd;
-        const size_t blk_base   = ((size_t)blk * 2 + (is_v ? 1 : 0)) * R.nkv + kh;
-        f16* dst = (f16*)R.kv_base + blk_base * head_elems;
-        if (!is_v) {
-            *reinterpret_cast<f16x4*>(dst + tok * R.hd + d0) = o0;
-            *reinterpret_cast<f16x4*>(dst + tok * R.hd + d0 + half) = o1;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { dst[(d0 + r) * R.page + tok] = o0[r]; dst[(d0 + r + half) * R.page + tok] = o1[r]; }
-        }
+        rope_rows_out(R, m, h, d0, x0, x1, pre_pos, pre_blk, [&](f32x4& lo, f32x4& hi) { lo = pre_cs[0]; hi = pre_cs[1]; }, [](float x) { return act_round<false>(x); },
+                      [](float x, float y) { return act_pack<false>(x, y); });
     }
 }
 

@@ -314,7 +314,7 @@ __global__ __launch_bounds__(1024) void gemm_fullk64_kernel(const FullKParams fp
     } else if constexpr (EPI == FK_ROPE) {
         // tile pair tg of the block: this lane holds dims d0..d0+3 (v[0]) and d0+half..+3 (v[1]) of row m = token m
         const RopeEpi& R = fp.r;
-        const int half = R.hd >> 1, hh = R.hd >> 5;
+        const int hh = R.hd >> 5;
         const int pair = unit * (TPB / 2) + tg, tlo = (pair / hh) * 2 * hh + pair % hh;   // the pair's lower tile
         const int h  = tlo / (2 * hh);
         const int d0 = (tlo % (2 * hh)) * 16 + q * 4;
@@ -326,50 +326,10 @@ __global__ __launch_bounds__(1024) void gemm_fullk64_kernel(const FullKParams fp
             x0[r] = rt_round(v[0][r] + rt_from_bits(b0[r], bf), bf);
             x1[r] = rt_round(v[1][r] + rt_from_bits(b1[r], bf), bf);
         }
-        const int pos_in  = sg.pos[m];
-        const int pos_lim = min(R.max_pos, R.max_blocks * R.page);
-        const int pos = min(max(pos_in, 0), pos_lim - 1);
-        const bool is_v = h >= R.nh + R.nkv;
-        if (!is_v) {
-            const f32x4 cs01 = *reinterpret_cast<const f32x4*>(&sg.cs[m][tg * 32 + q * 8]), cs23 = *reinterpret_cast<const f32x4*>(&sg.cs[m][tg * 32 + q * 8 + 4]);
-            const float cc[4] = {cs01[0], cs01[2], cs23[0], cs23[2]}, ss[4] = {cs01[1], cs01[3], cs23[1], cs23[3]};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float r0 = cc[r] * x0[r] - ss[r] * x1[r];
-                const float r1 = cc[r] * x1[r] + ss[r] * x0[r];
-                x0[r] = rt_round(r0, bf); x1[r] = rt_round(r1, bf);
-            }
-        }
-        f16x4 o0, o1;                                 // 16-bit patterns of the activation dtype (moved as f16-typed words)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            o0[r] = __builtin_bit_cast(f16, rt_to_bits(x0[r], bf)); o1[r] = __builtin_bit_cast(f16, rt_to_bits(x1[r], bf));
-        }
         FK_STAMP(5);
-        if (h < R.nh) {
-            f16* dst = R.q_out + ((size_t)m * R.nh + h) * R.hd + d0;
-            *reinterpret_cast<f16x4*>(dst) = o0;
-            *reinterpret_cast<f16x4*>(dst + half) = o1;
-            continue;
-        }
-        const int kh = is_v ? h - R.nh - R.nkv : h - R.nh;
-        if (pos_in < 0) continue;                                  // padding row of a multi-row step
-        const int blk = sg.blk[m];
-        if (pos != pos_in || blk < 0 || blk >= R.num_blocks) {   // stale position / block id: never write somebody else's page
-            if (h == R.nh && d0 == 0 && R.oob_count) atomicAdd(R.oob_count, 1);
-            continue;
-        }
-        const int tok = pos % R.page;
-        const size_t head_elems = (size_t)R.page * R.hd;
-        const size_t blk_base   = ((size_t)blk * 2 + (is_v ? 1 : 0)) * R.nkv + kh;
-        f16* dst = (f16*)R.kv_base + blk_base * head_elems;
-        if (!is_v) {
-            *reinterpret_cast<f16x4*>(dst + tok * R.hd + d0) = o0;
-            *reinterpret_cast<f16x4*>(dst + tok * R.hd + d0 + half) = o1;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { dst[(d0 + r) * R.page + tok] = o0[r]; dst[(d0 + r + half) * R.page + tok] = o1[r]; }
-        }
+        rope_rows_out(R, m, h, d0, x0, x1, sg.pos[m], sg.blk[m],
+                      [&](f32x4& lo, f32x4& hi) { lo = *reinterpret_cast<const f32x4*>(&sg.cs[m][tg * 32 + q * 8]); hi = *reinterpret_cast<const f32x4*>(&sg.cs[m][tg * 32 + q * 8 + 4]); },
+                      [&](float x) { return rt_round(x, bf); }, [&](float x, float y) { return bf ? act_pack<true>(x, y) : act_pack<false>(x, y); });
     }
     }   // epilogue jobs of this wave
     if constexpr (EPI == FK_PUB) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's published bytes have reached memory before it ends (the kernel boundary then orders them in front of the all-reduce launch's flags)

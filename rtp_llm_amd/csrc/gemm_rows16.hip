@@ -191,42 +191,14 @@ __global__ __launch_bounds__(D <= 3 ? 1024 : 512) void gemm_rows16_kernel(const 
     if constexpr (EPI == R16_ROPE) {
         const RopeEpi& R = p.r;
         const f32x4 v0 = sum(0), v1 = sum(1);
-        const int half = R.hd >> 1, h = n0 / R.hd, d0 = n0 - h * R.hd;
-        const bool is_v = h >= R.nh + R.nkv;
+        const int h = n0 / R.hd, d0 = n0 - h * R.hd;
         const float b0[4] = {act_lo<BF>(pre0[0]), act_hi<BF>(pre0[0]), act_lo<BF>(pre0[1]), act_hi<BF>(pre0[1])};
         const float b1[4] = {act_lo<BF>(pre1[0]), act_hi<BF>(pre1[0]), act_lo<BF>(pre1[1]), act_hi<BF>(pre1[1])};
-        const float c[4] = {cs01[0], cs01[2], cs23[0], cs23[2]}, s[4] = {cs01[1], cs01[3], cs23[1], cs23[3]};
         float x0[4], x1[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x0[e] = act_round<BF>(v0[e] + b0[e]); x1[e] = act_round<BF>(v1[e] + b1[e]);   // the linear's output is a 16-bit tensor
-            if (!is_v) {
-                const float r0 = c[e] * x0[e] - s[e] * x1[e], r1 = c[e] * x1[e] + s[e] * x0[e];
-                x0[e] = act_round<BF>(r0); x1[e] = act_round<BF>(r1);
-            }
-        }
-        const u32x2 o0 = {act_pack<BF>(x0[0], x0[1]), act_pack<BF>(x0[2], x0[3])}, o1 = {act_pack<BF>(x1[0], x1[1]), act_pack<BF>(x1[2], x1[3])};
-        if (h < R.nh) {
-            f16* dst = R.q_out + ((size_t)jj * R.nh + h) * R.hd + d0;
-            *reinterpret_cast<u32x2*>(dst) = o0;
-            *reinterpret_cast<u32x2*>(dst + half) = o1;
-            return;
-        }
-        if (pre_pos < 0) return;                                      // padding row of a multi-row step
-        const int pos = min(max(pre_pos, 0), min(R.max_pos, R.max_blocks * R.page) - 1);
-        if (pos != pre_pos || pre_blk < 0 || pre_blk >= R.num_blocks) {   // stale position / block id: never write somebody else's page
-            if (h == R.nh && d0 == 0 && R.oob_count) atomicAdd(R.oob_count, 1);
-            return;
-        }
-        const int kh = is_v ? h - R.nh - R.nkv : h - R.nh, tok = pos % R.page;
-        uint16_t* dst = (uint16_t*)R.kv_base + (((size_t)pre_blk * 2 + (is_v ? 1 : 0)) * R.nkv + kh) * ((size_t)R.page * R.hd);
-        if (!is_v) {
-            *reinterpret_cast<u32x2*>(dst + tok * R.hd + d0) = o0;
-            *reinterpret_cast<u32x2*>(dst + tok * R.hd + d0 + half) = o1;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { dst[(d0 + e) * R.page + tok] = act_to_bits<BF>(x0[e]); dst[(d0 + e + half) * R.page + tok] = act_to_bits<BF>(x1[e]); }
-        }
+        for (int e = 0; e < 4; ++e) { x0[e] = act_round<BF>(v0[e] + b0[e]); x1[e] = act_round<BF>(v1[e] + b1[e]); }   // the linear's output is a 16-bit tensor
+        rope_rows_out(R, jj, h, d0, x0, x1, pre_pos, pre_blk, [&](f32x4& lo, f32x4& hi) { lo = cs01; hi = cs23; }, [](float x) { return act_round<BF>(x); },
+                      [](float x, float y) { return act_pack<BF>(x, y); });
     } else {
         if (n0 >= p.N) return;
         if constexpr (EPI == R16_SLAB) {
