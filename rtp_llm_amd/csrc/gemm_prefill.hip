@@ -9,8 +9,9 @@
 //     104 dequant VALU, so the matrix pipe, not the VALU, sets the pace; the second wave of each SIMD dequantises while the first one multiplies;
 //   * the activation chunk (128 rows x 128 k = 32 KiB) goes to LDS by DMA while the chunk before it is multiplied, row by row with the 16-byte pieces of a row swizzled
 //     by the row (conflict-free ds_read_b128); two buffers, one barrier a chunk.  Through registers, as before, the chunk cost 16 of them, and with them the reach of the
-//     fragment reads: 3 fragments are now read ahead of their products.  37888 x 3584 in fp16 W4 at 4096 rows 1066 -> 1002 us, 3584 x 18944 493 -> 459 us (at the rate of
-//     a large dense product on the 224 of 256 CUs that have a block); 8 bits at 1055 rows 343 -> 315 and 159 -> 157 us; bf16 W16 9728 x 896 at 512 rows 20.3 -> 17.8 us;
+//     fragment reads: 3 fragments are now read ahead of their products.  Both sides in turn on one machine: fp16 W4 37888 x 3584 and 3584 x 18944 at 4096 rows 6 and 7 % faster (at the rate
+//     of a large dense product on the 224 of 256 CUs that have a block), the same in 8 bits at 1055 rows 8 and 1 %, bf16 W16 9728 x 896 at 512 rows 12 %.  Times move by 5 to 8 % between machines
+//     and with the operands' values (power); those of the present loops are at WHOLE below;
 //   * weights stream from HBM/L2 once per row tile (an XCD's blocks walk a column tile's row tiles together and meet in its L2: prefill_tile),
 //     through a 2-deep register ring (128 x 512: half a chunk at a time, see WHOLE), buffer range checks instead of tail branches.
 #include <type_traits>
@@ -425,8 +426,9 @@ constexpr PrefillShape kPrefillShapes[] = {{8, 4, 1}, {8, 2, 1}, {4, 2, 1}, {4, 
 constexpr int kPrefillShapeCount = sizeof(kPrefillShapes) / sizeof(kPrefillShapes[0]);
 
 // The shape of a call: a time model in us.  A round of a block (KS chunks of 128 k) takes `lat` alone on its CU -- loads, LDS, barrier -- and `sat` of a CU whose
-// share of the grid keeps it busy; the share counts half as the exact quotient and half as the whole blocks of the fullest CU.  Measured (random operands, one MI355X) per
-// operand class over M = 70..4096 at the Qwen2-0.5B and 7B projections: the pick is within 8 % of the fastest shape.  Examples, us at 128x512 / 128x256 / 64x256 /
+// share of the grid keeps it busy; the share counts half as the exact quotient and half as the whole blocks of the fullest CU.  Fitted (random operands, one MI355X) per
+// operand class over M = 70..4096 at the Qwen2-0.5B and 7B projections to the loop with branches and tiles in rows, whose pick was within 8 % of the fastest shape; it now decides whether K is
+// sliced and by how many, and what other paths are compared with (kUnslicedCost has the present loops).  Examples of that loop, us at 128x512 / 128x256 / 64x256 /
 // 64x128 / 64x64 / 32x64 / 32x32 tiles: fp16 W4 37888 x 3584 at M = 4096 1002 / 1057 / 1144 / 1244 / 1503 / 1806 / 2516, bf16 W4 3584 x 18944 at M = 128 - / 309 / 223 / 144 / 81 /
 // 64 / 50; W16 9728 x 896 at M = 512 - / 22 / 23 / 18 / 18 / 23 / 33; bf16 W4 37888 x 3584 at M = 512 - / 192 / 180 / 188 / 222 / 263 / 363.
 struct PrefillCost { double lat, sat; };
