@@ -38,7 +38,6 @@ struct DenseParams {
     const void* x; const void* w; const void* bias; void* y;
     int M, N, K, ldx, ldy;
     int gated;       // 0: N outputs; 1: rows of w are [32 gate | 32 up] groups, N / 2 outputs
-    int streamed;    // MI355_DENSE_STREAMED
     int act;         // DN_ACT_* applied to the gate
     float act_param; // DN_ACT_SWIGLU_CLAMP: the limit of the gate (from above) and of the up value (both sides)
     int out_f32;
@@ -56,6 +55,7 @@ struct DenseParams {
     const float* egate; int ldg, goff;
     // a weight that a later launch streams (its lines of 128 bytes): blocks past the list of tiles read one word of each
     const char* ahead = nullptr; uint32_t ahead_lines = 0;
+    int streamed = 0;    // MI355_DENSE_STREAMED (host only)
 };
 
 // The chip deals consecutive blocks to its eight XCDs in turn, each with an L2 of its own.  The (column tile, row tile) pair of a block is chosen such
@@ -735,7 +735,7 @@ void launch_rows(const DenseParams& p, hipStream_t st) {
 // lie side by side, and read as MFMA fragments (16 rows by 64 bytes a wave load) they came at 3.2 TB/s however the steps were ordered.  Here every wave load is one
 // row's run of 1 KB, by DMA into LDS, three stages of 512 columns; the rows of x beside them the same way, so that nothing but the fragments passes through registers.  8 weight rows a
 // block and 48 KB (M <= 8): three blocks a compute unit, 96 KB of loads in flight.  More rows a block and more waves are slower; which stages
-// pay is in skinny_form, which shapes are better off without LDS in skinny_short.
+// pay is in skinny_stage, which shapes are better off without LDS in skinny_short.
 // Weights from memory, M = 8, us before / now: 17408 x 2048 22.4 / 14.4, 32000 x 2048 35.1 / 24.3, 4096 x 2048 7.5 / 5.2, 2048 x 5632 13.6 / 6.5, 2048 x 2048 5.4 / 3.6.
 // Sums: k in steps of 32, step s into chain s mod skinny_chains (4 or 8), the chains added in order: bits that depend on N, K and G only.
 // 16-byte pieces are permuted by the row (applied to the source address), so that the 8 or 16 rows of a fragment read hit different banks.
@@ -908,20 +908,37 @@ __global__ __launch_bounds__(64 * (HALF ? NW / 2 : NW)) void dense_skinny_short_
     if ((int)blockIdx.x < blocks0) dense_skinny_short_tile<GATED0, NW, U, HALF>(p0, blockIdx.x, 0, red);
     else                           dense_skinny_short_tile<GATED1, NW, U, HALF>(p1, blockIdx.x - blocks0, 0, red);
 }
-// Which linears of M rows, K columns and so many weight rows are better off without LDS: they have no stages to fill, and a stage's columns past K cost what the others do, but their wave loads are 8
-// or 16 rows by 64 bytes, which the weights' stream of long K pays for.  Few rows, of which the stages hold copies, gain until K 2304; more rows to 1792; K below 512 leaves HALF's second
-// chains idle; many outputs fill the chip with 16 a block.  Time of the DMA form / HALF / 16 over that of the kernels before the DMA form, means over random calls, weights from memory:
-//   2 rows, K 512 to 1023, up to 512 weight rows 1.04 / 0.92 / 1.10; K 1500 to 2048 1.05 / 0.93 / 1.13; 3 rows, K 1024 to 1500, 512 to 1024 1.02 / 0.93 / 1.15; 4 rows, K 1500 to 2048, 512 to 1024 1.02 /
-//   0.93 / 1.15, K over 3000 0.76 / 0.95 / 1.20; 5 to 8 rows, K 1024 to 1500, 2048 to 4096 1.03 / 0.97 / 1.06, K 2048 to 3000, over 4096 0.79 / 0.98 / 0.99; K below 512, over 10000 1.45 / 1.03 / 0.97.
+// The columns of a stage of the DMA form for M rows of K columns (the shorter of two) in so many blocks.  512 of them, three stages, except:
+//   256, four stages, and so more blocks a compute unit, for short K, of which a stage of 512 would be mostly empty; where many blocks would load a tenth more columns than there are with 512 (a stage's
+//   loads past K cost what the others do); and for 9 to 16 rows in more than 256 blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2);
+//   1024, three stages, half the barriers, for up to 8 rows where no compute unit has a second block to hide them and the last stage is not mostly empty.  Time over that of 512, K that fills both: up
+//   to 192 blocks 0.93 to 0.95 (2 rows), 0.95 to 0.98 (3 and 4), 0.98 to 0.99 (5 to 8); 193 to 256 0.97 to 1.00; 257 to 320 1.04 to 1.23; 9 to 16 rows 1.00 to 1.03.
+int skinny_stage(int M, int K, long long blocks) {
+    auto padded = [&](int kc) { return ((long long)K + kc - 1) / kc * kc; };
+    if (K < 1024 || (blocks > 256 && (M > 8 || padded(512) * 10 > padded(256) * 11))) return 256;
+    return M <= 8 && blocks <= 256 && padded(1024) * 10 <= padded(512) * 12 ? 1024 : 512;
+}
+bool skinny_fills(int K, int stage) { return ((long long)K + stage - 1) / stage * stage * 20 < 21ll * K; }      // less than a twentieth loaded for nothing
+
+// Which linears of M rows, K columns and so many weight rows are better off without LDS: they have no stages to fill, but their wave loads are 8 or 16 rows by 64 bytes, which the weights' stream of
+// long K pays for, and of gated weights half as many blocks read twice as much each.  So up to 8 rows HALF serves K of 1024 and more that does not fill the DMA form's stages (fills), up to a length that
+// falls with the rows, and at 2 rows, of which the stages hold copies, any K so short; gated weights only from 2048 rows on (128 blocks); 16 outputs a block serve many outputs of short K.
+// Time without LDS / with, means over random calls, each behind a launch that writes its x, as a step has them: 5 to 8 rows, K 1024 to 1279 that fills / does not, 512 to 4096 weight rows 1.04 to 1.09 / 0.96 to
+// 1.03, gated below 2048 1.08 to 1.15 / 1.03 to 1.06, gated 2048 to 4096 1.02 to 1.04 / 0.93 to 0.99; K 2048 to 2303 1.06 to 1.24; 2 rows, K 1024 to 2047 0.87 to 1.00, gated of K over 1536 below 2048 rows 1.04 to
+// 1.17; K below 512, over 8192 rows 0.78 to 0.92.  (Timed back to back with x in the caches the form without LDS looked 5 to 15 % better: by lines from such times 1408 gated x 1024 took 5.6 us in a
+// step of 8 rows and 4880 x 1024 6.7, through LDS 4.7 and 5.7.)
+// K below 1024 through fewer outputs goes through LDS although HALF is 0.87 to 1.02 of it alone: in a step the stages' code is at hand from the launches around.  Eight layers of experts with such linears (704
+// and 64 columns), eight prompts and seven steps 6400 / 6300 us, two prompts 5520 / 5460.
 //   9 to 16 rows, us: 11 x 1024 x 47616 gated 29.1 / - / 24.5, 10 x 1024 x 22784 gated 16.4 / - / 13.1; 12 x 1808 x 8128, just two blocks of 16 a compute unit, 11.8 / - / 10.6; past the lines
 //   11 x 1728 x 10368 gated 13.0 / - / 14.0, 16 x 1864 x 8256 gated 13.5 / - / 16.4, 12 x 1832 x 4224 8.3 / - / 9.5.
-// 1600 times of 800 random calls, from memory and from the memory-side cache: 1.018 of the fastest form's up to 8 rows (K of 1024 and more through LDS alone: 1.05) and 1.014 above; of 1700 others 30 are
-// more than 3 % behind the kernels before the DMA form, at worst 1.11, and most lie at 0.5 to 0.98.
-int skinny_short(int M, int K, long long weight_rows) {           // outputs a block; 0: through LDS
+// 1986 times of 993 random calls of 2 to 8 rows that the lines were not fitted to, from memory and from the memory-side cache: 1.018 of the fastest form's, at worst 1.18; 0.958 of the time of the kernels
+// before the DMA form, 297 more than 3 % behind it, most of them of K below 1024.
+int skinny_short(int M, int K, long long weight_rows, bool gated, bool fills) {           // outputs a block; 0: through LDS
     if (M > 8) return weight_rows >= 6144 && (K <= 1152 || (K <= 1856 && (weight_rows <= 8192 || weight_rows >= 12288))) ? 16 : 0;
-    if (K < 512) return M <= 3 || weight_rows > 512 ? 16 : 0;
-    if (K <= 1152 && weight_rows >= 6144) return 16;
-    return K <= (M <= 4 ? 2304 : 1792) && weight_rows <= 8192 ? 8 : 0;
+    if (weight_rows < (K < 512 ? 8192 : K < 1024 ? 4096 : gated ? 2048 : 0)) return 0;
+    if (fills && M > 2 && weight_rows < (K < 1024 ? 8192 : 12288)) return 0;
+    if (K <= 1152 && weight_rows >= (K < 512 ? 8192 : K < 1024 ? 6144 : 12288)) return 16;
+    return K <= (M <= 2 ? 2304 : M <= 4 ? 2048 : 1792) && weight_rows < 12288 ? 8 : 0;
 }
 int skinny_short_blocks(const DenseParams& p, int outputs) { return ((p.gated ? p.N / 2 : p.N) + outputs - 1) / outputs; }
 // launch(chains, steps in flight, half) with the instance for as many outputs a block
@@ -940,26 +957,23 @@ int skinny_blocks(const DenseParams& p) { return (p.N + SK_RB - 1) / SK_RB; }
 // A weight that the 256 MB memory-side cache does not hold from one step to the next is read past the caches where a launch reads 24 MB or more.  Only the caller knows: the same weight in a
 // small model, or under a draft's head, comes from that cache.  40 random weights of 24 to 130 MB, time with / without the hint: 0.97 (0.91 to 1.01) in a footprint of 1 GB, 0.96 in 400 MB,
 // 1.12 (0.99 to 1.37) in 256 MB, 1.10 in 128 MB.  17408 x 2048 from memory 15.5 / 14.4 us, 32000 x 2048 26.5 / 24.3; eight prompts and eight steps of a 16-layer model of width 2048 8920 / 8400 us.
+// What a marked weight displaces counts too: a head of 64 MB read past the caches leaves them to the layers (eight layers, 247 MB a step, eight prompts and seven steps 2690 -> 2622 us, the head itself
+// 16.4 -> 17.7), so up to 8 rows such a launch goes through LDS, which has the hint.
 bool skinny_nt(bool streamed, size_t weights) { return streamed && weights * 2 >= (size_t)24 << 20; }
 
-// launch(form) with the form for M rows of K columns (the shorter of two) in `blocks` blocks.  As few rows of x staged as there are: they come from the L2, but pass through the same loads
-// as the weights (32000 x 2048 with 4 / 8 / 16: 21.2 / 24.3 / 28.6 us).  Stages of 512 columns, three of them, except:
-//   stages of 256, four of them, and so more blocks a compute unit, for short K, of which a stage of 512 would be mostly empty; where many blocks would load a tenth more columns than there are with
-//   512 (a stage's loads past K cost what the others do); and for 9 to 16 rows in more than 256 blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2);
-//   stages of 1024, half the barriers, in up to 192 blocks, where no compute unit has a second block to hide them (2 rows, 384 x 5960, six stages of 512 / three of 1024: 7.1 / 6.3) and the last
-//   stage is not mostly empty.
+// launch(form) with the form of skinny_stage columns.  As few rows of x staged as there are: they come from the L2, but pass through the same loads as the weights (32000 x 2048 with 4 / 8 / 16:
+// 21.2 / 24.3 / 28.6 us).
 template <class L>
-void skinny_form(int M, int K, long long blocks, L&& launch) {
+void skinny_form(int M, int stage, L&& launch) {
     auto rows = [&](auto kc, auto ns) {
         constexpr int KC = decltype(kc)::value, NS = decltype(ns)::value;
-        if (M > 8) launch(SkinnyForm<16, KC, NS>{});
+        if (M > 8) launch(SkinnyForm<16, KC < 1024 ? KC : 512, NS>{});                       // no stage of 1024 there
         else if (M > 4 || KC < 512) launch(SkinnyForm<8, KC, NS>{});
         else if constexpr (KC >= 512) launch(SkinnyForm<4, KC, NS>{});
     };
-    auto padded = [&](int kc) { return ((long long)K + kc - 1) / kc * kc; };
-    if (K < 1024 || (blocks > 256 && (M > 8 || padded(512) * 10 > padded(256) * 11))) rows(std::integral_constant<int, 256>{}, std::integral_constant<int, 4>{});
-    else if (blocks <= 192 && padded(1024) * 10 <= padded(512) * 12)                    rows(std::integral_constant<int, 1024>{}, std::integral_constant<int, 3>{});
-    else                                                                                rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 3>{});
+    if (stage == 256)       rows(std::integral_constant<int, 256>{}, std::integral_constant<int, 4>{});
+    else if (stage == 1024) rows(std::integral_constant<int, 1024>{}, std::integral_constant<int, 3>{});
+    else                    rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 3>{});
 }
 // The DMA form adds 32-bit byte offsets to the first row of x and of a block's weight rows.  Rows of x further apart than that reaches (15 steps of 143 million elements: the last tokens of eight
 // sequences of 131072 x 2048) go in launches of fewer rows, the same bits; a K that the 35 rows between a gate and the last up row of a block do not reach has no such form.
@@ -981,7 +995,9 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         return;
     }
     const bool eight = skinny_chains(p) == 8;
-    if (const int out = skinny_short(p.M, p.K, (long long)p.N * p.G)) {
+    const int stage = skinny_stage(p.M, p.K, (long long)skinny_blocks(p) * p.G);
+    const bool nt = skinny_nt(p.streamed, (size_t)p.N * p.K * p.G);
+    if (const int out = nt && p.M <= 8 ? 0 : skinny_short(p.M, p.K, (long long)p.N * p.G, p.gated, skinny_fills(p.K, stage))) {
         skinny_short_form(out, eight, [&](auto nw, auto u, auto half) {
             constexpr int NW = decltype(nw)::value, U = decltype(u)::value;
             constexpr bool H = decltype(half)::value;
@@ -991,16 +1007,19 @@ void launch_skinny(const DenseParams& p, hipStream_t st) {
         return;
     }
     const dim3 grid(skinny_blocks(p), p.G), block(256);
-    const bool nt = skinny_nt(p.streamed, (size_t)p.N * p.K * p.G);
-    skinny_form(p.M, p.K, (long long)grid.x * grid.y, [&](auto f) {
+    skinny_form(p.M, stage, [&](auto f) {
         using F = decltype(f);
         if (eight) { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 8, false>), grid, block, 0, st, p); }
         else       { if (nt) hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, true>), grid, block, 0, st, p); else hipLaunchKernelGGL((dense_skinny_bf16_kernel<F, 4, false>), grid, block, 0, st, p); }
     });
 }
 void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
-    const int chains = skinny_chains(p[0]);
-    const int out = skinny_chains(p[1]) == chains ? skinny_short(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N) : 0;
+    const int chains = skinny_chains(p[0]), M = p[0].M > p[1].M ? p[0].M : p[1].M, b0 = skinny_blocks(p[0]), b1 = skinny_blocks(p[1]);
+    const int stage = skinny_stage(M, p[0].K < p[1].K ? p[0].K : p[1].K, (long long)b0 + b1);
+    const bool nt = skinny_nt(p[0].streamed && p[1].streamed, (size_t)p[0].N * p[0].K + (size_t)p[1].N * p[1].K);
+    // two launches' weights keep the stages full: by the lines of 3 rows at least (2 rows, K 1024 through 832 to 960 blocks: 5.3 to 5.9 us through LDS, 6.8 to 7.1 without)
+    const int out = (nt && M <= 8) || skinny_chains(p[1]) != chains ? 0 : skinny_short(M < 3 ? 3 : M, p[0].K > p[1].K ? p[0].K : p[1].K, (long long)p[0].N + p[1].N, p[0].gated || p[1].gated,
+                                                                     skinny_fills(p[0].K, stage) && skinny_fills(p[1].K, stage));
     if (out) {
         const int s0 = skinny_short_blocks(p[0], out);
         const dim3 grid(s0 + skinny_short_blocks(p[1], out));
@@ -1013,9 +1032,8 @@ void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
         });
         return;
     }
-    const int b0 = skinny_blocks(p[0]), b1 = skinny_blocks(p[1]), c0 = skinny_chains(p[0]), c1 = skinny_chains(p[1]);
-    const bool nt = skinny_nt(p[0].streamed && p[1].streamed, (size_t)p[0].N * p[0].K + (size_t)p[1].N * p[1].K);
-    skinny_form(p[0].M > p[1].M ? p[0].M : p[1].M, p[0].K < p[1].K ? p[0].K : p[1].K, (long long)b0 + b1, [&](auto f) {
+    const int c0 = skinny_chains(p[0]), c1 = skinny_chains(p[1]);
+    skinny_form(M, stage, [&](auto f) {
         using F = decltype(f);
         if (nt) hipLaunchKernelGGL((dense_skinny_pair_kernel<F, true>), dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, c0, c1);
         else    hipLaunchKernelGGL((dense_skinny_pair_kernel<F, false>), dim3(b0 + b1), dim3(256), 0, st, p[0], p[1], b0, c0, c1);

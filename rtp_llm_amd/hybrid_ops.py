@@ -88,9 +88,10 @@ def dense_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
 _STREAMED = 1 << 30         # MI355_DENSE_STREAMED
 
 
-def mark_streamed(weights, nbytes: int, cached: int = 256 << 20) -> bool:
+def mark_streamed(weights, nbytes: int, cached: int = 192 << 20) -> bool:
     """A model's weights (tensors, or objects, lists and dicts that hold some) get the attribute `streamed` where the nbytes that a step reads are more than the memory-side cache keeps for the
-    next: the linears of a few rows then read the large ones past the caches.  -> whether they did."""
+    next: the linears of a few rows then read the large ones past the caches.  Of its 256 MB a quarter is left to the cache pages, states and activations of a step (of 247 MB of weights it did not
+    keep the layers': 2690 -> 2622 us for eight prompts and seven steps with the head marked).  -> whether they did."""
     seen = set()
 
     def walk(o):

@@ -44,10 +44,10 @@ def test_few_rows_through_every_group():
 @pytest.mark.parametrize("N,K", [(2048, 1016), (2048, 1024), (2050, 1032), (4096, 1016), (4097, 1016), (8184, 1024), (8200, 1160), (6152, 2056), (6136, 2048), (64, 5640),
                                  (512, 504), (520, 504), (512, 512), (520, 512), (6144, 504), (6144, 1152), (6136, 1152), (6144, 1160), (8192, 1160), (8200, 1160), (8192, 1792), (8192, 1800),
                                  (2048, 2304), (2048, 2312), (12288, 1856), (12280, 1856), (8192, 1856), (8192, 1864), (16400, 1024), (16384, 1792), (1536, 3072), (1544, 3072), (1536, 2320), (2048, 2568), (2056, 2568),
-                                 (2056, 2824)])
+                                 (2056, 2824), (1024, 968), (1024, 976), (8184, 976), (8192, 976), (4880, 1024), (12280, 1024), (12288, 1024), (4096, 1000), (4088, 1000), (8192, 488), (4096, 1960), (4096, 2056), (12280, 1048), (12288, 1160)])
 def test_few_rows_forms(N, K):
-    """Either side of each rule that picks the form (3, 4 and 8 rows; K 512, 1152, 1792, 1856, 2304; 512, 6144, 8192, 12288 weight rows; four chains and eight), stages and columns of a stage (192 and 256 blocks, columns
-    loaded for nothing, 24 MB), a last stage with one piece: against a 64-bit product, the same bits for any number of rows, alone and in a launch of two."""
+    """Either side of each rule that picks the form (2, 4 and 8 rows; K 512, 1024, 1152, 1792, 1856, 2048, 2304, K that fills the stages and K that leaves a twentieth empty; 512, 4096, 6144, 8192, 12288 weight rows; four chains
+    and eight), stages and columns of a stage (256 blocks, columns loaded for nothing, 24 MB), a last stage with one piece: against a 64-bit product, the same bits for any number of rows, alone and in a launch of two."""
     g = torch.Generator(device=DEV).manual_seed(N + K)
     x, w = torch.randn(16, K, device=DEV, generator=g).bfloat16(), (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
     x2, w2 = torch.randn(16, 72, device=DEV, generator=g).bfloat16(), torch.randn(64, 72, device=DEV, generator=g).bfloat16()
@@ -60,6 +60,21 @@ def test_few_rows_forms(N, K):
         assert torch.equal(hops.dense_linear(x[:M], w, out_dtype=torch.float32), y[:M]) and torch.equal(a, y[:M]) and torch.equal(b, gated[:M]), M
     a, b = hops.dense_pair(dict(x=x2, w=w2, gated=True, act=hops.ACT_SILU), dict(x=x, w=w, out_dtype=torch.float32))
     assert torch.equal(a, gated) and torch.equal(b, y)
+
+
+@pytest.mark.parametrize("N,K", [(448, 488), (1984, 504), (2048, 504), (1984, 1032), (1984, 1024), (4096, 968), (4032, 968), (2048, 1024), (2048, 1032), (4096, 1160), (8128, 1000), (8192, 976), (12224, 1024), (12288, 1024)])
+def test_few_rows_gated_forms(N, K):
+    """Gated weights either side of their rules (2048, 4096, 8192, 12288 weight rows; K 1024; K that fills the stages) against 64-bit products, the same bits for any number of rows.  silu(g) u: both sums are off by 2^-17 of
+    their magnitudes at most (as above), silu's slope is below 1.1, __expf and the division add a few 2^-24 of the gate."""
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x, w = torch.randn(16, K, device=DEV, generator=g).bfloat16(), (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
+    y = hops.dense_linear(x, w, gated=True, act=hops.ACT_SILU, out_dtype=torch.float32)
+    gate, up = (x.double() @ v.double().t() for v in (w.view(-1, 64, K)[:, :32].reshape(-1, K), w.view(-1, 64, K)[:, 32:].reshape(-1, K)))
+    mag_g, mag_u = (2.0 ** -17 * (x.double().abs() @ v.double().abs().t()) for v in (w.view(-1, 64, K)[:, :32].reshape(-1, K), w.view(-1, 64, K)[:, 32:].reshape(-1, K)))
+    ref = torch.nn.functional.silu(gate) * up
+    assert bool(((y.double() - ref).abs() <= 1.1 * mag_g * (up.abs() + mag_u) + torch.nn.functional.silu(gate).abs() * mag_u + 2.0 ** -20 * ref.abs() + 1e-30).all())
+    for M in (2, 3, 4, 5, 8, 9):
+        assert torch.equal(hops.dense_linear(x[:M], w, gated=True, act=hops.ACT_SILU, out_dtype=torch.float32), y[:M]), M
 
 
 @pytest.mark.parametrize("M,ldx", [(3, 1 << 30), (16, 143165608), (9, (1 << 29) + 8)])
