@@ -563,12 +563,19 @@ def sampling_draw(logits: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Op
     return ids
 
 
+def _host_vector(t: torch.Tensor, dtype: torch.dtype) -> bool:
+    return t.dtype is dtype and t.is_cpu and t.is_contiguous()
+
+
 def sampler_filters(top_k: torch.Tensor, top_p: torch.Tensor, V: int):
     """(every row greedy, some row of a sampling step has a filter) of host vectors, or None where they are not contiguous host memory of int32 and float32 with as many rows."""
-    if top_k.dtype != torch.int32 or top_p.dtype != torch.float32 or not top_k.is_cpu or not top_p.is_cpu or top_k.numel() != top_p.numel() or not top_k.is_contiguous() or not top_p.is_contiguous():
+    n = top_k.numel()
+    if top_p.numel() != n or not _host_vector(top_k, torch.int32) or not _host_vector(top_p, torch.float32):
         return None
-    f = _C.lib().mi355_sampler_filters(top_k.data_ptr(), top_p.data_ptr(), top_k.numel(), V)
-    return bool(f & 1), bool(f & 2)
+    return _FILTERS[_C.lib().mi355_sampler_filters(top_k.data_ptr(), top_p.data_ptr(), n, V)]
+
+
+_FILTERS = ((False, False), (True, False), (False, True), (True, True))
 
 
 def sampler_vectors(logits: torch.Tensor, token_ids: torch.Tensor, temperature: torch.Tensor, penalties, top_k: torch.Tensor, top_p: torch.Tensor, uniform: torch.Tensor,
@@ -576,28 +583,23 @@ def sampler_vectors(logits: torch.Tensor, token_ids: torch.Tensor, temperature: 
     """What sampling_draw takes as `host`: the vectors of a whole step, penalties (repetition, presence, frequency) or None, history token_ids [B, step + 1].  None where mi355_sampler_step
     does not take the step, or a tensor is not contiguous host memory of its kernel's type with one value per row.  seen: sampler_filters of the same top_k and top_p, where the caller has it."""
     f32, i32 = torch.float32, torch.int32
-    if logits.dim() != 2 or logits.dtype != f32 or not logits.is_contiguous() or token_ids.dim() != 2 or token_ids.shape[1] > 2048:
+    if logits.dim() != 2 or logits.dtype is not f32 or not logits.is_contiguous() or token_ids.dim() != 2:
         return None
-    B, V = logits.shape
-    vectors = [(temperature, f32), (uniform, f32)]
-    if seen is None:
-        vectors += [(top_p, f32), (top_k, i32)]
-    elif top_k.numel() != B:
+    (B, V), (rows, history) = logits.shape, token_ids.shape
+    if B == 0 or rows != B or not 0 < history <= 2048 or top_k.numel() != B or not _host_vector(token_ids, i32):
         return None
-    if penalties is not None:
-        vectors += [(t, f32) for t in penalties] + [(input_lengths, i32)]
-        if sequence_lengths.numel() > B or sequence_lengths.dtype != i32 or not sequence_lengths.is_cpu or not sequence_lengths.is_contiguous():
+    if seen is None and (top_p.numel() != B or not _host_vector(top_p, f32) or not _host_vector(top_k, i32)):
+        return None
+    for t in (temperature, uniform) if penalties is None else (temperature, uniform, *penalties):
+        if t.numel() != B or t.dtype is not f32 or not t.is_cpu or not t.is_contiguous():
             return None
-    for t, dt in vectors:
-        if t.dtype != dt or not t.is_cpu or t.numel() != B or not t.is_contiguous():
-            return None
-    if B == 0 or token_ids.dtype != i32 or not token_ids.is_cpu or not token_ids.is_contiguous() or token_ids.shape[0] != B or token_ids.shape[1] == 0:
-        return None
-    host = _C.SamplerHost(temperature=temperature.data_ptr(), top_k=top_k.data_ptr(), top_p=top_p.data_ptr(), uniform=uniform.data_ptr(), step=token_ids.shape[1] - 1,
-                          token_ids=token_ids.data_ptr())
+    pen, lengths = (None, None, None), (None, None, 0)
     if penalties is not None:
-        host.repetition, host.presence, host.frequency = (t.data_ptr() for t in penalties)
-        host.input_lengths, host.sequence_lengths, host.n_sequences = input_lengths.data_ptr(), sequence_lengths.data_ptr(), sequence_lengths.numel()
+        n = sequence_lengths.numel()
+        if n > B or input_lengths.numel() != B or not _host_vector(input_lengths, i32) or not _host_vector(sequence_lengths, i32):
+            return None
+        pen, lengths = [t.data_ptr() for t in penalties], (input_lengths.data_ptr(), sequence_lengths.data_ptr(), n)
+    host = _C.SamplerHost(temperature.data_ptr(), *pen, top_k.data_ptr(), top_p.data_ptr(), uniform.data_ptr(), *lengths, history - 1, token_ids.data_ptr())
     takes = _C.lib().mi355_sampler_step_takes(host, B, V) if seen is None else seen[1] and not seen[0] and B <= 65535
     return host if takes else None
 
