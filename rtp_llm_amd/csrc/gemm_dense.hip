@@ -910,12 +910,13 @@ __global__ __launch_bounds__(64 * (HALF ? NW / 2 : NW)) void dense_skinny_short_
 }
 // The columns of a stage of the DMA form for M rows of K columns (the shorter of two) in so many blocks.  512 of them, three stages, except:
 //   256, four stages, and so more blocks a compute unit, for short K, of which a stage of 512 would be mostly empty; where many blocks would load a tenth more columns than there are with 512 (a stage's
-//   loads past K cost what the others do); and for 9 to 16 rows in more than 256 blocks (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2);
+//   loads past K cost what the others do); and for 9 to 16 rows in more than 256 blocks of K below 2048, or 1024 of any (32000 x 2048 26.2 us; 2048 x 5632, 256 blocks, 7.8 against 7.2; steps of 9 and
+//   16 rows at width 2048 7535 and 8170 us with 256 from 257 blocks on, 7475 and 8080 with 512 there; of 12 rows at width 1024 6065 / 6120);
 //   1024, three stages, half the barriers, for up to 8 rows where no compute unit has a second block to hide them and the last stage is not mostly empty.  Time over that of 512, K that fills both: up
 //   to 192 blocks 0.93 to 0.95 (2 rows), 0.95 to 0.98 (3 and 4), 0.98 to 0.99 (5 to 8); 193 to 256 0.97 to 1.00; 257 to 320 1.04 to 1.23; 9 to 16 rows 1.00 to 1.03.
 int skinny_stage(int M, int K, long long blocks) {
     auto padded = [&](int kc) { return ((long long)K + kc - 1) / kc * kc; };
-    if (K < 1024 || (blocks > 256 && (M > 8 || padded(512) * 10 > padded(256) * 11))) return 256;
+    if (K < 1024 || (blocks > 256 && (padded(512) * 10 > padded(256) * 11 || (M > 8 && (K < 2048 || blocks >= 1024))))) return 256;
     return M <= 8 && blocks <= 256 && padded(1024) * 10 <= padded(512) * 12 ? 1024 : 512;
 }
 bool skinny_fills(int K, int stage) { return ((long long)K + stage - 1) / stage * stage * 20 < 21ll * K; }      // less than a twentieth loaded for nothing
