@@ -17,7 +17,7 @@ LAYOUTS = {"interleaved": 0, "halves": 1}
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _C.current_stream()
 
 
 def _p(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -484,7 +484,7 @@ class DecoderEngine:
         self.block_table[:bt.shape[0], : bt.shape[1]].copy_(bt)   # one row per token (decode) or per sequence (q_len > 1)
 
     def _st(self) -> int:
-        return torch.cuda.current_stream().cuda_stream
+        return _C.current_stream()
 
     def capacity(self, block_table=None) -> int:
         """Tokens one sequence may hold: bounded by the engine's max_seq_len, the rotation table and the block table."""

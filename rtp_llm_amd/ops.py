@@ -14,7 +14,7 @@ from .quant import PackedWeight
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _C.current_stream()
 
 
 def _p(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -8,9 +8,11 @@
     prompt and everything it may generate.  New tokens come from the framework's sampler (sampler.sample_greedy: greedy, or temperature /
     top-k / top-p with explicit uniforms).
 """
+from array import array
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from .kvcache import CacheManager
@@ -50,60 +52,68 @@ class ServingEngine:
     # ------------------------------------------------------------------ the step function
     def build_batch(self, entries: Sequence[Tuple[object, Sequence[int], Sequence[int]]]) -> StepBatch:
         """entries: (sequence id, its next tokens, indices among them whose logits are wanted).  Admits new sequences and takes pages."""
-        tokens, pos, seq, row_start, slot, first, want, tables, prev = [], [], [], [0], [], [], [], [], []
         seen, admitted = set(), []
         try:
-            return self._build(entries, tokens, pos, seq, row_start, slot, first, want, tables, seen, admitted, prev)
+            return self._build(entries, seen, admitted)
         except Exception:
             for sid in admitted:                      # a step that cannot run leaves no half-admitted sequence behind
                 self.cache.release(sid)
             raise
 
-    def _build(self, entries, tokens, pos, seq, row_start, slot, first, want, tables, seen, admitted, prev):
+    def _build(self, entries, seen, admitted):
+        tokens, lens, slot, first, last, want, tables = array("i"), [], [], [], [], [], []
         for sid, toks, wants in entries:
             if sid in seen:
                 raise ValueError(f"sequence {sid!r} appears twice in one step")
             seen.add(sid)
-            if not len(toks):
+            n, base = len(toks), len(tokens)
+            if not n:
                 raise ValueError(f"sequence {sid!r}: an entry without tokens")
             if sid not in self.cache.live:
                 self.cache.admit(sid)
                 admitted.append(sid)
-            sc = self.cache.grow(sid, len(toks))
-            s = len(slot)
-            base = len(tokens)
-            tokens += [int(t) for t in toks]
-            prev += [sc.last_token if sc.length else -1] + [int(t) for t in toks[:-1]]
-            pos += list(range(sc.length, sc.length + len(toks)))
-            seq += [s] * len(toks)
-            row_start.append(len(tokens))
+            sc = self.cache.grow(sid, n)
+            try:
+                tokens.extend(array("i", list(toks)))
+            except TypeError:                         # numbers of another kind
+                tokens.extend([int(t) for t in toks])
+            lens.append(n)
             slot.append(sc.slot)
             first.append(sc.length)
+            last.append(sc.last_token if sc.length else -1)
             for w in wants:
-                if not 0 <= int(w) < len(toks):
-                    raise ValueError(f"sequence {sid!r}: wanted row {w} of {len(toks)}")
+                if not 0 <= int(w) < n:
+                    raise ValueError(f"sequence {sid!r}: wanted row {w} of {n}")
                 want.append(base + int(w))
             tables.append(sc.pages)
+        nseq, T = len(tables), len(tokens)
         width = max(8, -(-max(len(t) for t in tables) // 8) * 8)
-        t0, tn = [], []
-        for a, b in zip(row_start[:-1], row_start[1:]):           # tiles of at most 16 consecutive rows of one sequence
-            t0 += list(range(a, b, 16))
-            tn += [min(16, b - r) for r in range(a, b, 16)]
-        bt = []
-        for t in tables:
-            bt += t + [0] * (width - len(t))
+        ln = np.array(lens)
+        row_start = np.zeros(nseq + 1, dtype=np.int64)
+        np.cumsum(ln, out=row_start[1:])
+        start, seq = row_start[:-1], np.repeat(np.arange(nseq), ln)
+        prev = np.empty(T, dtype=np.int32)
+        prev[1:] = tokens[:-1]
+        prev[start] = last
+        tiles = (ln + 15) // 16                                   # tiles of at most 16 consecutive rows of one sequence
+        tseq = np.repeat(np.arange(nseq), tiles)
+        t0 = start[tseq] + 16 * (np.arange(tseq.size) - (np.cumsum(tiles) - tiles)[tseq])
+        tn = np.minimum(16, row_start[1:][tseq] - t0)
+        bt = np.zeros((nseq, width), dtype=np.int32)
+        for row, t in zip(bt, tables):
+            row[:len(t)] = t
         # every index array of the step travels in ONE pinned int32 buffer and one copy; the fields are views into the device copy
-        parts = [tokens, pos, seq, row_start, slot, first, bt, want, t0, tn, prev]
+        parts = [tokens, np.arange(T) + (np.array(first) - start)[seq], seq, row_start, slot, first, bt.reshape(-1), want, t0, tn, prev]
         offs = [0]
         for part in parts:
             offs.append(offs[-1] + (len(part) + 3) // 4 * 4)      # 16-byte aligned fields
         host = torch.zeros(offs[-1], dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        view = host.numpy()
         for o, part in zip(offs, parts):
-            if part:
-                host[o:o + len(part)] = torch.tensor(part, dtype=torch.int32)
-        batch = self.batch_views(host.to(self.device, non_blocking=True), [len(part) for part in parts], len(tables), width)
+            view[o:o + len(part)] = part
+        batch = self.batch_views(host.to(self.device, non_blocking=True), [len(part) for part in parts], nseq, width)
         batch.host = host
-        batch.max_rows = max(b - a for a, b in zip(row_start[:-1], row_start[1:]))
+        batch.max_rows = max(lens)
         return batch
 
     @staticmethod
