@@ -111,6 +111,23 @@ int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, int32_t qo,
                         const float* z, int32_t ldz, const void* lower, const void* fbias, float tau, float qscale, int32_t H, int32_t dim, int32_t vdim, const int32_t* row_start,
                         const int32_t* slot, const int32_t* first_pos, int32_t nseq, float* state, const void* w, int32_t w_heads, float eps, void* out, int32_t act_dtype,
                         mi355_stream_t stream);
+/* The same of bf16 rows with a linear of 2 to 16 bf16 rows beside it in the launch (neither reads what the other writes): the results are those of the two calls, bit for bit.  The arguments of
+ * mi355_hy_recur_step by name.  MI355_ERR_UNSUPPORTED: forms that take two calls. */
+typedef struct {
+    const float* proj; int32_t ld, qo, ko, vo, go, ao, rank;
+    const void* w2; const void* b2;
+    const float* z; int32_t ldz;
+    const void* lower; const void* fbias;
+    float tau, qscale;
+    int32_t mode, H, dim, vdim;
+    const int32_t* row_start; const int32_t* slot; const int32_t* first_pos; int32_t nseq;
+    float* state;
+    const void* w; int32_t w_heads;
+    float eps;
+    void* out;
+} mi355_recur_args_t;
+int mi355_hy_recur_step_beside_fits(int32_t dim, int32_t vdim, int32_t M, int32_t N, int32_t K, int32_t gated);       /* host only: the sizes that it takes */
+int mi355_hy_recur_step_beside(const mi355_recur_args_t* recur, const mi355_dense_args_t* linear, mi355_stream_t stream);
 /* Further extended forms: an activation with a parameter (act 5: clamped gated form g' sigmoid(1.702 g') (u' + 1)), routers that score by sigmoids, rank
  * groups by their two best experts and scale the weights, a query / key norm over all heads at once, an embedding with a multiplier, and the end of a
  * sublayer whose output is normed before it joins the stream (layer norm or RMS norm), also as the last norm on gathered rows. */

@@ -78,6 +78,12 @@ class DenseArgs(C.Structure):  # mi355_dense_args_t
                 ("act_param", f32)]
 
 
+class RecurArgs(C.Structure):  # mi355_recur_args_t
+    _fields_ = [("proj", vp), ("ld", i32), ("qo", i32), ("ko", i32), ("vo", i32), ("go", i32), ("ao", i32), ("rank", i32), ("w2", vp), ("b2", vp), ("z", vp), ("ldz", i32),
+                ("lower", vp), ("fbias", vp), ("tau", f32), ("qscale", f32), ("mode", i32), ("H", i32), ("dim", i32), ("vdim", i32), ("row_start", vp), ("slot", vp), ("first_pos", vp),
+                ("nseq", i32), ("state", vp), ("w", vp), ("w_heads", i32), ("eps", f32), ("out", vp)]
+
+
 ALL_REDUCE_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
 ALL_GATHER_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
 
@@ -220,6 +226,8 @@ HYBRID_SIGNATURES = {
     "mi355_hy_attn_prep_ex": (i32, [vp, i32, i32, i32, ip, vp, vp, i32, f32, vp, vp, vp, i32, vp, vp, vp, vp, f32, f32, i32, i32, vp]),
     "mi355_hy_attn_rows_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, f32, vp, i32, i32, vp]),
     "mi355_dense_linear_pair": (i32, [C.POINTER(DenseArgs), vp]),
+    "mi355_hy_recur_step_beside_fits": (i32, [i32] * 6),
+    "mi355_hy_recur_step_beside": (i32, [C.POINTER(RecurArgs), C.POINTER(DenseArgs), vp]),
     "mi355_hy_recur_step_fits": (i32, [i32, i32]),
     "mi355_hy_recur_step": (i32, [i32, vp] + [i32] * 7 + [vp, vp, vp, i32, vp, vp, f32, f32, i32, i32, i32, vp, vp, vp, i32, vp, vp, i32, f32, vp, i32, vp]),
     "mi355_hy_attn_tiles_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, f32, vp, i32, i32, vp]),

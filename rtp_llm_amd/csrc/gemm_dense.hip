@@ -15,6 +15,7 @@
 // Output is fp32 or the activation type.  A result row depends only on its own input row: the k order of the accumulation is fixed by
 // the kernel, never by M or by the row's place in the batch.
 #include "common.h"
+#include "hybrid_recur.h"
 #include "../../include/mi355_hybrid.h"
 
 // The tile shape of a bf16 call of M x N x K through `groups` weights (64-row tiles of sorted rows in `row_tiles`, 0: all M rows through each): 0 64x64, 1 64x128 in three stages,
@@ -842,6 +843,20 @@ __global__ __launch_bounds__(256) void dense_skinny_pair_kernel(DenseParams p0, 
     }
 }
 
+// A linear and the recurrence of the same decode step, which need nothing of each other: the recurrence is 128 blocks (16 heads of 8 sequences) in a chain of four trips to memory, 8.5 us, and
+// the linear's blocks stream their weights meanwhile.  The recurrence's blocks come first, so that none of them waits for a unit.  A layer of width 2048 with 8 rows: both input linears 16.4 us and
+// the recurrence 8.5 before, now the mixer's own 8.2 and this launch 13.5 (11264 x 2048); a prompt pass and 12 steps of 2 / 4 / 8 / 16 sequences, us before / now: width 1024, 8 layers 3483 / 3274,
+// 3529 / 3335, 3691 / 3450, 4066 / 3727; width 2048, 16 layers 9389 / 8927, 9650 / 9175, 10456 / 9998, 12044 / 11845.
+template <class F, int RPT, bool NT>
+__global__ __launch_bounds__(256) void hy_recur_linear_kernel(RecurStep r, DenseParams p, int nseq, int chains) {
+    __shared__ __attribute__((aligned(1024))) char smem[F::BYTES];
+    static_assert(sizeof(RecurLds) <= F::BYTES, "the recurrence's arrays lie where the stages do");
+    const int heads = nseq * r.H, b = blockIdx.x;
+    if (b < heads) hy_recur_step<bf16, RPT>(r, b % nseq, b / nseq, *(RecurLds*)smem);
+    else if (chains == 8) dense_skinny_tile<F, 8, NT>(p, b - heads, 0, smem);
+    else                  dense_skinny_tile<F, 4, NT>(p, b - heads, 0, smem);
+}
+
 // Where that costs more than it gains (skinny_short): fragments straight from memory, the same sums.  16 outputs a block, a wave for each of the NW chains, U steps of it in flight.
 // HALF (M <= 8): 8 outputs a block and half the waves, each with two chains: rows 0 to 7 of the first operand are x in the steps of chain w, rows 8 to 15 x in those of chain w + NW / 2, the second
 // operand likewise; of the 16 x 16 sums the two 8 x 8 blocks on the diagonal are the two chains, the rest is not used.
@@ -1041,6 +1056,36 @@ void launch_skinny_pair(const DenseParams (&p)[2], hipStream_t st) {
     });
 }
 
+// The parameters of a linear of 2 to 16 bf16 rows from a caller's arguments; MI355_ERR_UNSUPPORTED where the kernels that share a launch do not take it.
+int few_rows_params(mi355_dense_args_t d, const char* who, DenseParams& q) {
+    const int streamed = (d.gated & MI355_DENSE_STREAMED) != 0; d.gated &= ~MI355_DENSE_STREAMED;
+    MI355_CHECK_ARG(d.x && d.w && d.y && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && (!d.gated || d.N % 64 == 0) && d.ldy >= (d.gated ? d.N / 2 : d.N) && d.act >= 0 &&
+                        d.act <= DN_ACT_RELU2 && (d.act != DN_ACT_SWIGLU_CLAMP || (d.gated && d.act_param > 0.f)),
+                    "%s: M=%d N=%d K=%d ldx=%d ldy=%d gated=%d act=%d", who, d.M, d.N, d.K, d.ldx, d.ldy, d.gated, d.act);
+    if (d.M < 2 || d.M > 16 || d.K % 8 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16 || !skinny_weight_reach(d.K) || d.M > skinny_rows_reach(d.ldx)) return MI355_ERR_UNSUPPORTED;
+    q.x = d.x; q.w = d.w; q.bias = d.bias; q.y = d.y; q.M = d.M; q.N = d.N; q.K = d.K; q.ldx = d.ldx; q.ldy = d.ldy;
+    q.gated = d.gated; q.streamed = streamed; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
+    q.yvec = (d.ldy % 4 == 0) && ((uintptr_t)d.y % (d.out_f32 ? 16 : 8) == 0);
+    q.G = 1; q.xs = q.ws = q.ys = 0; q.offs = nullptr; q.gather = nullptr; q.tiles = nullptr; q.egate = nullptr; q.ldg = q.goff = 0;
+    return MI355_OK;
+}
+
+// Where a recurrence takes a linear along: up to 8 key rows a thread (registers: three blocks a compute unit are left), and a linear that goes through LDS, by the lines of 3 rows at least as in a pair.
+bool recur_linear_fits(int dim, int vdim, int M, int N, int K, bool gated, bool streamed) {
+    const int blocks = (N + SK_RB - 1) / SK_RB;
+    return hy_recur_rows(dim, vdim) <= 8 && ((skinny_nt(streamed, (size_t)N * K) && M <= 8) || !skinny_short(M < 3 ? 3 : M, K, N, gated, skinny_fills(K, skinny_stage(M, K, blocks))));
+}
+void launch_recur_linear(const RecurStep& r, int nseq, const DenseParams& p, hipStream_t st) {
+    const dim3 grid(nseq * r.H + skinny_blocks(p));
+    const int chains = skinny_chains(p);
+    const bool nt = skinny_nt(p.streamed, (size_t)p.N * p.K);
+    skinny_form(p.M, skinny_stage(p.M, p.K, skinny_blocks(p)), [&](auto f) {
+        using F = decltype(f);
+        if (nt) hipLaunchKernelGGL((hy_recur_linear_kernel<F, 8, true>), grid, dim3(256), 0, st, r, p, nseq, chains);
+        else    hipLaunchKernelGGL((hy_recur_linear_kernel<F, 8, false>), grid, dim3(256), 0, st, r, p, nseq, chains);
+    });
+}
+
 } // namespace
 
 // x [M, K] (row stride ldx) and w [N, K] of act_dtype (MI355_ACT_BF16 or MI355_ACT_F32); bias [N] of act_dtype or null;
@@ -1101,22 +1146,31 @@ extern "C" int mi355_dense_linear_ex(const void* x, int32_t ldx, int32_t M, cons
 extern "C" int mi355_dense_linear_pair(const mi355_dense_args_t* a, mi355_stream_t stream) {
     MI355_CHECK_ARG(a, "dense_linear_pair: null arguments");
     DenseParams p[2];
-    for (int i = 0; i < 2; ++i) {
-        mi355_dense_args_t d = a[i];
-        const int streamed = (d.gated & MI355_DENSE_STREAMED) != 0; d.gated &= ~MI355_DENSE_STREAMED;
-        MI355_CHECK_ARG(d.x && d.w && d.y && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && (!d.gated || d.N % 64 == 0) && d.ldy >= (d.gated ? d.N / 2 : d.N) && d.act >= 0 &&
-                            d.act <= DN_ACT_RELU2 && (d.act != DN_ACT_SWIGLU_CLAMP || (d.gated && d.act_param > 0.f)),
-                        "dense_linear_pair: M=%d N=%d K=%d ldx=%d ldy=%d gated=%d act=%d", d.M, d.N, d.K, d.ldx, d.ldy, d.gated, d.act);
-        if (d.M < 2 || d.M > 16 || d.K % 8 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16 || !skinny_weight_reach(d.K) || d.M > skinny_rows_reach(d.ldx)) return MI355_ERR_UNSUPPORTED;
-        DenseParams& q = p[i];
-        q.x = d.x; q.w = d.w; q.bias = d.bias; q.y = d.y; q.M = d.M; q.N = d.N; q.K = d.K; q.ldx = d.ldx; q.ldy = d.ldy;
-        q.gated = d.gated; q.streamed = streamed; q.act = d.act; q.act_param = d.act_param; q.out_f32 = d.out_f32; q.softcap = 0.f; q.vec = 1;
-        q.yvec = (d.ldy % 4 == 0) && ((uintptr_t)d.y % (d.out_f32 ? 16 : 8) == 0);
-        q.G = 1; q.xs = q.ws = q.ys = 0; q.offs = nullptr; q.gather = nullptr; q.tiles = nullptr; q.egate = nullptr; q.ldg = q.goff = 0;
-    }
+    for (int i = 0; i < 2; ++i)
+        if (int e = few_rows_params(a[i], "dense_linear_pair", p[i])) return e;
     hipStream_t st = (hipStream_t)stream;
     launch_skinny_pair(p, st);
     MI355_CHECK_LAUNCH("dense_skinny_pair_kernel");
+    return MI355_OK;
+}
+
+// Whether mi355_hy_recur_step_beside takes aligned operands of these sizes.  Host only.
+extern "C" int mi355_hy_recur_step_beside_fits(int32_t dim, int32_t vdim, int32_t M, int32_t N, int32_t K, int32_t gated) {
+    return mi355_hy_recur_step_fits(dim, vdim) && M >= 2 && M <= 16 && N > 0 && K > 0 && K % 8 == 0 && skinny_weight_reach(K) &&
+           recur_linear_fits(dim, vdim, M, N, K, gated & ~MI355_DENSE_STREAMED, (gated & MI355_DENSE_STREAMED) != 0);
+}
+
+// mi355_hy_recur_step (bf16) and a linear that neither reads nor writes anything of it, in one launch: the same bits as the two calls.
+extern "C" int mi355_hy_recur_step_beside(const mi355_recur_args_t* a, const mi355_dense_args_t* lin, mi355_stream_t stream) {
+    MI355_CHECK_ARG(a && lin, "hy_recur_step_beside: null arguments");
+    const RecurStep r{a->proj, a->ld, a->qo, a->ko, a->vo, a->go, a->ao, a->rank, a->w2, a->b2, a->z, a->ldz, a->lower, a->fbias, a->tau, a->qscale, a->mode, a->H, a->dim, a->vdim, a->row_start,
+                      a->slot, a->first_pos, a->state, a->w, a->w_heads, a->eps, a->out};
+    if (int e = hy_recur_check(r, a->nseq)) return e;
+    DenseParams p;
+    if (int e = few_rows_params(*lin, "hy_recur_step_beside", p)) return e;
+    if (!recur_linear_fits(r.dim, r.vdim, p.M, p.N, p.K, p.gated, p.streamed)) return MI355_ERR_UNSUPPORTED;
+    launch_recur_linear(r, a->nseq, p, (hipStream_t)stream);
+    MI355_CHECK_LAUNCH("hy_recur_linear_kernel");
     return MI355_OK;
 }
 

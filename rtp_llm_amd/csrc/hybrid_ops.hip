@@ -16,17 +16,10 @@
 // here whatever the activation type T (bf16 or float): positions and angles, scores and softmax, norms, gates, decays, states, residual.
 #include <algorithm>
 #include "common.h"
+#include "hybrid_recur.h"
 #include "../../include/mi355_hybrid.h"
 
 namespace {
-
-template <typename T> __device__ __forceinline__ void hy_load8(const T* p, float (&o)[8]);
-template <> __device__ __forceinline__ void hy_load8<bf16>(const bf16* p, float (&o)[8]) { act_unpack8<true>(*(const u32x4*)p, o); }
-template <> __device__ __forceinline__ void hy_load8<float>(const float* p, float (&o)[8]) {
-    const f32x4 a = *(const f32x4*)p, b = *(const f32x4*)(p + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { o[i] = a[i]; o[4 + i] = b[i]; }
-}
 
 // eight consecutive cache elements as loaded (16 bytes of bf16, 32 of fp32), widened only where they are used: more loads fit in flight
 template <typename T> struct HyRaw8;
@@ -46,19 +39,11 @@ template <> struct HyRaw8<float> {
     }
 };
 
-__device__ __forceinline__ float hy_wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 __device__ __forceinline__ float hy_wave_max(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     return v;
 }
-__device__ __forceinline__ float hy_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
-__device__ __forceinline__ float hy_silu(float z) { return z / (1.f + expf(-z)); }
-
 // channel indices of rotation pair i under a layout: 0 = interleaved (2i, 2i+1), 1 = halves (i, i + n/2)
 __device__ __forceinline__ void hy_pair(int layout, int i, int n, int& c0, int& c1) {
     if (layout == 0) { c0 = 2 * i; c1 = 2 * i + 1; } else { c0 = i; c1 = i + n / 2; }
@@ -1254,7 +1239,6 @@ __global__ __launch_bounds__(256) void hy_chunk_prefix_kernel(const int32_t* cs,
 // at a time: all threads compute the gates of the staged tokens once into LDS, then every thread walks the tokens in order (its RD rows:
 // decay, rank-one update, partial q . S), and the DS partial outputs per token are summed from LDS.  Short RD keeps the dependent chain per
 // token short; the walk itself is the sequential part of the recurrence.
-enum { SCAN_HGRN2 = 0, SCAN_GLA = 1, SCAN_FIXED = 2, SCAN_FIXED_SILU = 3 };
 
 // Matrix memory under exponential gates (MEM instances of the scan kernel).  Per head log gates i (input) and f (forget) and a running maximum m that keeps
 // the exponentials in range:  m_t = max(f_t + m_(t-1), i_t),  keep_t = e^(f_t + m_(t-1) - m_t),  take_t = e^(i_t - m_t),
@@ -2259,113 +2243,10 @@ __global__ __launch_bounds__(256) void hy_head_norm4_kernel(const float* o, int 
 // first low-rank linear, now a part of the input linear) of 4 to 6 us each for a state of a few MB.  Here a block has a head of one sequence: thread (kg, cg) holds four value
 // columns of the key rows kg, kg + KG, .., loaded while the gates are formed.  16 heads of 64 x 128, 8 sequences: 8.3 us under a low-rank decay, with 6.1 + 2.8 of the scan and the
 // norm and 2.8 of that decay's second linear before; what is left is a chain of four trips to memory.
-struct RecurStep {
-    const float* proj; int ld, qo, ko, vo, go, ao, rank;
-    const void* w2; const void* b2;
-    const float* z; int ldz;
-    const void* lower; const void* fbias;
-    float tau, qscale;
-    int mode, H, dim, vdim;
-    const int32_t* row_start; const int32_t* slot; const int32_t* first_pos;
-    float* state;
-    const void* w; int w_heads;
-    float eps;
-    void* out;
-};
 template <typename T, int RPT>
 __global__ __launch_bounds__(256) void hy_recur_step_kernel(RecurStep p) {
-    __shared__ float q_s[256], k_s[256], a_s[256], red[8];
-    __shared__ __attribute__((aligned(16))) float part[1024];
-    const int sq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, CG = p.vdim >> 2, KG = 256 / CG, cg = tid % CG, kg = tid / CG;
-    const int r0 = p.row_start[sq], r1 = p.row_start[sq + 1];
-    const bool on = kg < KG;
-    float* st = p.state + ((size_t)p.slot[sq] * p.H + h) * p.dim * p.vdim + cg * 4;
-    f32x4 s[RPT];
-    const bool fresh = p.first_pos[sq] == 0;
-#pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int d = kg + j * KG;
-        s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (on && !fresh && d < p.dim) s[j] = *(const f32x4*)(st + (size_t)d * p.vdim);
-    }
-    const int hd = h * p.dim + min(tid, p.dim - 1), hv = h * p.vdim + min(tid, p.vdim - 1);
-    const float norm = p.w ? (float)((const T*)p.w)[p.w_heads ? hv : min(tid, p.vdim - 1)] : 1.f;
-    const bool low = p.mode == SCAN_GLA && p.ao >= 0;
-    for (int t = r0; t < r1; ++t) {
-        // everything the token needs is asked for at once: a later load is another trip to memory in a launch of a few microseconds
-        const float* row = p.proj + (size_t)t * p.ld;
-        float qv = row[p.qo + hd], kv = row[p.ko + hd], av = 0.f, zz = 0.f, lr = 0.f;
-        f32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = row[p.vo + h * p.vdim + cg * 4 + e];
-        const float gz = p.go >= 0 ? row[p.go + hv] : 0.f;
-        if (low) {
-            lr = (float)(T)row[p.ao + min(tid & 63, p.rank - 1)];
-            zz = p.b2 ? (float)((const T*)p.b2)[hd] : 0.f;
-            const T* w2 = (const T*)p.w2 + (size_t)hd * p.rank;
-            float dot = 0.f;
-            if (p.rank % 8 == 0 && (uintptr_t)p.w2 % 32 == 0)
-                for (int j = 0; j < p.rank; j += 8) {
-                    float w8[8];
-                    hy_load8<T>(w2 + j, w8);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(w8[e], __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lr), j + e)), dot);
-                }
-            else
-                for (int j = 0; j < p.rank; ++j)
-                    dot = __builtin_fmaf((float)w2[j], __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lr), j)), dot);
-            zz += dot;
-        } else if (p.mode == SCAN_GLA) zz = p.z[(size_t)t * p.ldz + hd];
-        if (p.mode == SCAN_HGRN2) {
-            const float lw = (float)((const T*)p.lower)[hd], f = lw + (1.f - lw) * hy_sigmoid(kv + (float)((const T*)p.fbias)[hd]);
-            qv = hy_silu(qv); av = f; kv = 1.f - f;
-        } else if (p.mode == SCAN_GLA) {
-            qv *= p.qscale;
-            av = expf((fminf(zz, 0.f) - log1pf(expf(-fabsf(zz)))) / p.tau);
-        } else {
-            if (p.mode == SCAN_FIXED_SILU) {
-                qv = hy_silu(qv); kv = hy_silu(kv);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = hy_silu(v[e]);
-            }
-            av = ((const float*)p.lower)[h];
-        }
-        if (tid < p.dim) { q_s[tid] = qv; k_s[tid] = kv; a_s[tid] = av; }
-        __syncthreads();
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-        if (on) {
-#pragma unroll
-            for (int j = 0; j < RPT; ++j) {
-                const int d = kg + j * KG;
-                if (d >= p.dim) continue;
-                const float a = a_s[d], k = k_s[d], q = q_s[d];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { s[j][e] = __builtin_fmaf(a, s[j][e], k * v[e]); o[e] = __builtin_fmaf(s[j][e], q, o[e]); }
-            }
-            *(f32x4*)(part + (kg * CG + cg) * 4) = o;
-        }
-        __syncthreads();
-        float y = 0.f;
-        if (tid < p.vdim)
-            for (int g = 0; g < KG; ++g) y += part[g * p.vdim + tid];
-        const float ss = hy_wave_sum(y * y);
-        if ((tid & 63) == 0) red[(t & 1) * 4 + (tid >> 6)] = ss;
-        __syncthreads();
-        if (tid < p.vdim) {
-            const float* rd = red + (t & 1) * 4;
-            y *= 1.f / sqrtf(((rd[0] + rd[1]) + (rd[2] + rd[3])) / (float)p.vdim + p.eps);
-            if (p.w) y *= norm;
-            if (p.go >= 0) y *= hy_silu(gz);
-            ((T*)p.out)[((size_t)t * p.H + h) * p.vdim + tid] = (T)y;
-        }
-    }
-    if (r0 < r1) {
-#pragma unroll
-        for (int j = 0; j < RPT; ++j) {
-            const int d = kg + j * KG;
-            if (on && d < p.dim) *(f32x4*)(st + (size_t)d * p.vdim) = s[j];
-        }
-    }
+    __shared__ RecurLds lds;
+    hy_recur_step<T, RPT>(p, blockIdx.x, blockIdx.y, lds);
 }
 
 // ------------------------------------------------------------------------------------------------ latent attention: normed latent + shared rotated key -> page; queries split
@@ -3052,16 +2933,9 @@ extern "C" int mi355_hy_recur_step(int32_t mode, const float* proj, int32_t ld, 
                                    const void* b2, const float* z, int32_t ldz, const void* lower, const void* fbias, float tau, float qscale, int32_t H, int32_t dim,
                                    int32_t vdim, const int32_t* row_start, const int32_t* slot, const int32_t* first_pos, int32_t nseq, float* state, const void* w,
                                    int32_t w_heads, float eps, void* out, int32_t act_dtype, mi355_stream_t stream) {
-    MI355_CHECK_ARG(proj && row_start && slot && first_pos && state && out && nseq > 0 && H > 0 && dim > 0 && vdim > 0, "hy_recur_step: bad argument");
-    MI355_CHECK_ARG(mode == SCAN_HGRN2 ? (lower && fbias) : (mode == SCAN_FIXED || mode == SCAN_FIXED_SILU) ? lower != nullptr
-                                                          : (mode == SCAN_GLA && tau > 0.f && (ao >= 0 ? (w2 && rank > 0 && rank <= 64) : z != nullptr)),
-                    "hy_recur_step: mode %d lacks its gate inputs", mode);
-    if (!mi355_hy_recur_step_fits(dim, vdim) || (uintptr_t)state % 16) {
-        mi355_set_error("hy_recur_step: heads of %d x %d", dim, vdim);
-        return MI355_ERR_UNSUPPORTED;
-    }
     const RecurStep p{proj, ld, qo, ko, vo, go, ao, rank, w2, b2, z, ldz, lower, fbias, tau, qscale, mode, H, dim, vdim, row_start, slot, first_pos, state, w, w_heads, eps, out};
-    const int KG = 256 / (vdim / 4), rows = (dim + KG - 1) / KG;
+    if (int e = hy_recur_check(p, nseq)) return e;
+    const int rows = hy_recur_rows(dim, vdim);
     const dim3 grid(nseq, H);
     hipStream_t st = (hipStream_t)stream;
     if (rows <= 4)       HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_recur_step_kernel<T, 4>), grid, dim3(256), 0, st, p));

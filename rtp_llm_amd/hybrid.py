@@ -599,12 +599,15 @@ class HybridModel:
                     g = hops.dense_linear(h1, gate_w[n_pad:], gate_b[n_pad:], out_dtype=torch.float32)
                 a = mixer.forward(h1, batch, *cache, proj=proj) if isinstance(cache, tuple) else mixer.forward(h1, batch, cache, proj=proj)
             elif gate_w is None and isinstance(mlp, GatedMLP) and hasattr(mixer, "few_rows") and mixer.few_rows(T, batch) is not None:
-                # few rows: the two branches read the same stream, so their input linears are one launch, and their output linears another
+                # few rows: the two branches read the same stream, so their output linears are one launch; their input linears another, or, in front of a recurrence, the feed-forward's runs beside it
                 g = None
                 w, bias = mixer.few_rows(T, batch)
-                proj, up = hops.dense_pair(dict(x=h1, w=w, bias=bias, out_dtype=torch.float32),
-                                           dict(x=h2, w=mlp.w_gate_up, gated=True, act=mlp.act, act_param=mlp.act_param))
-                o = mixer.forward(h1, batch, *(cache if isinstance(cache, tuple) else (cache,)), proj=proj, out_proj=False)
+                own, ff = dict(x=h1, w=w, bias=bias, out_dtype=torch.float32), dict(x=h2, w=mlp.w_gate_up, gated=True, act=mlp.act, act_param=mlp.act_param)
+                if isinstance(mixer, GatedLinearRecurrence) and hops.recur_step_takes(mixer.spec.dim, mixer.spec.vdim, T, mlp.w_gate_up, True):
+                    o, up = mixer.forward(h1, batch, cache, proj=hops.dense_linear(**own), out_proj=False, beside=ff)
+                else:
+                    proj, up = hops.dense_pair(own, ff)
+                    o = mixer.forward(h1, batch, *(cache if isinstance(cache, tuple) else (cache,)), proj=proj, out_proj=False)
                 a, b = hops.dense_pair(dict(x=o, w=mixer.w_o, bias=getattr(mixer, "b_o", None), out_dtype=torch.float32),
                                        dict(x=up, w=mlp.w_down, out_dtype=torch.float32))
                 continue

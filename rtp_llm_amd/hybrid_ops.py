@@ -121,28 +121,35 @@ def _gated(w: torch.Tensor, rows: int, gated: bool) -> int:
 FEW_ROWS = 16              # rows up to which the linears are bound by their weights' stream and every launch by its own cost
 
 
+def _few_rows_args(a: "_C.DenseArgs", x, w, bias=None, out_dtype=None, gated=False, act=ACT_NONE, act_param=0.0, name="dense_pair") -> Optional[torch.Tensor]:
+    """Fills the arguments of a linear that may share a launch -> its output, or None: not bf16 with 2 to FEW_ROWS rows."""
+    M, K = x.shape
+    if w.dtype != torch.bfloat16 or not 2 <= M <= FEW_ROWS:
+        return None
+    _dev(x, w.dtype, name + ".x"); _dev(w, w.dtype, name + ".w")
+    N, gated = w.shape[0], bool(gated)
+    if w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or (gated and N % 64) or (bias is not None and (bias.numel() != N or not bias.is_contiguous())):
+        raise _C.Mi355Error(f"{name}: x {tuple(x.shape)} against w {tuple(w.shape)}")
+    if bias is not None:
+        _dev(bias, w.dtype, name + ".bias")
+    od = out_dtype or w.dtype
+    if od not in (torch.float32, w.dtype):
+        raise _C.Mi355Error(f"{name}: output {od} from {w.dtype} operands")
+    n_out = N // 2 if gated else N
+    out = torch.empty(M, n_out, dtype=od, device=x.device)
+    a.x, a.ldx, a.M, a.w, a.N, a.K, a.bias, a.y, a.ldy = x.data_ptr(), _rows(x, name + ".x"), M, w.data_ptr(), N, K, _p(bias), out.data_ptr(), n_out
+    a.out_f32, a.gated, a.act, a.act_param = int(od == torch.float32), _gated(w, M, gated), int(act), float(act_param)
+    return out
+
+
 def dense_pair(first: dict, second: dict):
     """Two dense_linear calls (keywords x, w, bias, out_dtype, gated, act, act_param) as one launch where both are bf16 with 2 to FEW_ROWS rows, else as two; the same bits either way."""
     args, outs = (_C.DenseArgs * 2)(), []
     for a, d in zip(args, (first, second)):
-        x, w, bias = d["x"], d["w"], d.get("bias")
-        M, K = x.shape
-        if w.dtype != torch.bfloat16 or not 2 <= M <= FEW_ROWS:
+        out = _few_rows_args(a, **d)
+        if out is None:
             return dense_linear(**first), dense_linear(**second)
-        _dev(x, w.dtype, "dense_pair.x"); _dev(w, w.dtype, "dense_pair.w")
-        N, gated = w.shape[0], bool(d.get("gated"))
-        if w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or (gated and N % 64) or (bias is not None and (bias.numel() != N or not bias.is_contiguous())):
-            raise _C.Mi355Error(f"dense_pair: x {tuple(x.shape)} against w {tuple(w.shape)}")
-        if bias is not None:
-            _dev(bias, w.dtype, "dense_pair.bias")
-        od = d.get("out_dtype") or w.dtype
-        if od not in (torch.float32, w.dtype):
-            raise _C.Mi355Error(f"dense_pair: output {od} from {w.dtype} operands")
-        n_out = N // 2 if gated else N
-        out = torch.empty(M, n_out, dtype=od, device=x.device)
         outs.append(out)
-        a.x, a.ldx, a.M, a.w, a.N, a.K, a.bias, a.y, a.ldy = x.data_ptr(), _rows(x, "dense_pair.x"), M, w.data_ptr(), N, K, _p(bias), out.data_ptr(), n_out
-        a.out_f32, a.gated, a.act, a.act_param = int(od == torch.float32), _gated(w, M, gated), int(d.get("act", ACT_NONE)), float(d.get("act_param", 0.0))
     rc = _C.hybrid_lib().mi355_dense_linear_pair(args, _stream())
     if rc == _C.ERR_UNSUPPORTED:               # operands off 16 bytes, K % 8
         return dense_linear(**first), dense_linear(**second)
@@ -664,17 +671,28 @@ def recur_step_supported(dim: int, vdim: int) -> bool:
     return bool(_C.hybrid_lib().mi355_hy_recur_step_fits(dim, vdim))
 
 
+@functools.lru_cache(maxsize=256)
+def _recur_takes(dim: int, vdim: int, M: int, N: int, K: int, gated: int) -> bool:
+    return bool(_C.hybrid_lib().mi355_hy_recur_step_beside_fits(dim, vdim, M, N, K, gated))
+
+
+def recur_step_takes(dim: int, vdim: int, rows: int, w: torch.Tensor, gated: bool) -> bool:
+    """Whether recur_step runs a linear of so many rows through w in its own launch."""
+    return w.dtype == torch.bfloat16 and 2 <= rows <= FEW_ROWS and _recur_takes(dim, vdim, rows, w.shape[0], w.shape[1], _gated(w, rows, gated))
+
+
 def recur_step(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, go: Optional[int], low_rank, z: Optional[torch.Tensor], lower, fbias, tau: float, qscale: float, heads: int,
-               dim: int, vdim: int, row_start, slot, first_pos, state: torch.Tensor, w: Optional[torch.Tensor], eps: float, act: torch.dtype) -> torch.Tensor:
+               dim: int, vdim: int, row_start, slot, first_pos, state: torch.Tensor, w: Optional[torch.Tensor], eps: float, act: torch.dtype, beside: Optional[dict] = None):
     """scan and head_norm (weight w, gate through silu at column go) over few rows in one launch -> act type [T, heads * vdim].  low_rank: None, or (column of proj, w2
-    [heads * dim, rank], b2 or None) that SCAN_GLA forms its decay pre-activations from instead of z."""
+    [heads * dim, rank], b2 or None) that SCAN_GLA forms its decay pre-activations from instead of z.
+    beside: the keywords of a dense_linear call that reads nothing of this one -> (this result, that one), in one launch where both are bf16 of few rows; the same bits either way."""
     _dev(proj, torch.float32, "recur_step.proj"); _dev(state, torch.float32, "recur_step.state")
     if not state.is_contiguous() or state.shape[1:] != (heads, dim, vdim):
         raise _C.Mi355Error(f"recur_step: state {tuple(state.shape)} for {heads} heads of {dim} x {vdim}")
     T, nseq = proj.shape[0], slot.numel()
     out = torch.empty(T, heads * vdim, dtype=act, device=proj.device)
     if not (T and nseq):
-        return out
+        return out if beside is None else (out, dense_linear(**beside))
     ao, w2, b2 = low_rank if low_rank is not None else (-1, None, None)
     for t, n in ((w2, None), (b2, heads * dim), (w, None)):
         if t is not None:
@@ -683,12 +701,22 @@ def recur_step(mode: int, proj: torch.Tensor, qo: int, ko: int, vo: int, go: Opt
                 raise _C.Mi355Error(f"recur_step: weight {tuple(t.shape)}")
     if (w2 is not None and (w2.dim() != 2 or w2.shape[0] != heads * dim)) or (w is not None and w.numel() not in (vdim, heads * vdim)):
         raise _C.Mi355Error("recur_step: weights do not fit the heads")
-    _C.check_hybrid(_C.hybrid_lib().mi355_hy_recur_step(mode, proj.data_ptr(), _rows(proj, "recur_step.proj"), qo, ko, vo, -1 if go is None else go, ao,
-                                                        0 if w2 is None else w2.shape[1], _p(w2), _p(b2), _p(z), 0 if z is None else _rows(z, "recur_step.z"), _p(lower),
-                                                        _p(fbias), float(tau), float(qscale), heads, dim, vdim, row_start.data_ptr(), slot.data_ptr(), first_pos.data_ptr(),
-                                                        nseq, state.data_ptr(), _p(w), int(w is not None and w.numel() == heads * vdim and heads > 1), float(eps),
+    ld, ldz, w_heads = _rows(proj, "recur_step.proj"), 0 if z is None else _rows(z, "recur_step.z"), int(w is not None and w.numel() == heads * vdim and heads > 1)
+    go, rank = -1 if go is None else go, 0 if w2 is None else w2.shape[1]
+    if beside is not None and act == torch.bfloat16:
+        a = _C.DenseArgs()
+        y = _few_rows_args(a, **beside, name="recur_step.beside")
+        if y is not None:
+            r = _C.RecurArgs(proj.data_ptr(), ld, qo, ko, vo, go, ao, rank, _p(w2), _p(b2), _p(z), ldz, _p(lower), _p(fbias), float(tau), float(qscale), mode, heads, dim, vdim,
+                             row_start.data_ptr(), slot.data_ptr(), first_pos.data_ptr(), nseq, state.data_ptr(), _p(w), w_heads, float(eps), out.data_ptr())
+            rc = _C.hybrid_lib().mi355_hy_recur_step_beside(C.byref(r), C.byref(a), _stream())
+            if rc != _C.ERR_UNSUPPORTED:
+                _C.check_hybrid(rc, "hy_recur_step_beside")
+                return out, y
+    _C.check_hybrid(_C.hybrid_lib().mi355_hy_recur_step(mode, proj.data_ptr(), ld, qo, ko, vo, go, ao, rank, _p(w2), _p(b2), _p(z), ldz, _p(lower), _p(fbias), float(tau), float(qscale),
+                                                        heads, dim, vdim, row_start.data_ptr(), slot.data_ptr(), first_pos.data_ptr(), nseq, state.data_ptr(), _p(w), w_heads, float(eps),
                                                         out.data_ptr(), act_code(act), _stream()), "hy_recur_step")
-    return out
+    return out if beside is None else (out, dense_linear(**beside))
 
 
 def _chunk_plan(row_start, T: int, nseq: int, per_chunk_bytes: int, plans: Optional[dict], C: int = 0) -> ChunkPlan:

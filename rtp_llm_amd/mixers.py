@@ -347,8 +347,9 @@ class GatedLinearRecurrence:
             few = longest <= 1 and (s.vdim <= 128 or s.dim * s.vdim <= 16384)
         return (self.w_few, None) if few else None
 
-    def forward(self, h: torch.Tensor, batch: StepBatch, state: torch.Tensor, proj: Optional[torch.Tensor] = None, out_proj: bool = True) -> torch.Tensor:
-        """proj: h w^T for the weight that few_rows names, when the caller has computed it.  out_proj False: without the output projection."""
+    def forward(self, h: torch.Tensor, batch: StepBatch, state: torch.Tensor, proj: Optional[torch.Tensor] = None, out_proj: bool = True, beside: Optional[dict] = None):
+        """proj: h w^T for the weight that few_rows names, when the caller has computed it.  out_proj False: without the output projection.  beside (a step that few_rows takes): see
+        hybrid_ops.recur_step, -> (this result, that linear's)."""
         s = self.spec
         few = self.few_rows(h.shape[0], batch)
         if few is not None:
@@ -356,7 +357,9 @@ class GatedLinearRecurrence:
                 proj = hops.dense_linear(h, self.w_few, out_dtype=torch.float32)
             low_rank = (self.ao, self.w_a2, self.b_a2) if self.mode == hops.SCAN_GLA else None
             o = hops.recur_step(self.mode, proj, self.qo, self.ko, self.vo, self.go, low_rank, None, self.lower, self.fbias, s.tau, 1.0 / math.sqrt(s.dim), s.heads, s.dim,
-                                s.vdim, batch.row_start, batch.slot, batch.first_pos, state, self.norm, self.eps, self.act)
+                                s.vdim, batch.row_start, batch.slot, batch.first_pos, state, self.norm, self.eps, self.act, beside=beside)
+            if beside is not None:
+                return (hops.dense_linear(o[0], self.w_o, out_dtype=torch.float32) if out_proj else o[0]), o[1]
             return hops.dense_linear(o, self.w_o, out_dtype=torch.float32) if out_proj else o
         proj = hops.dense_linear(h, self.w_in, out_dtype=torch.float32)
         z = None
