@@ -2458,6 +2458,70 @@ __global__ __launch_bounds__(64) void hy_moe_route_kernel(const float* z, int ld
     hy_route_token(true, z + (size_t)t * ld, hy_rs, hy_rs + E, E, groups, keep, top, ids + (size_t)t * top, wts + (size_t)t * top, threadIdx.x, rm);
 }
 
+// Up to 64 experts: G lanes a token, each with one expert's score, 256 / G tokens a block, and no chain over the choices: a lane counts the experts in front of its own, which is the
+// place of its own among the chosen.  The order is that of hy_route_token (eligible first, then by score, ties to the lower index), the sums add in the same order.
+// Us a launch, before / now: 1537 tokens, 4 of 16 experts 8.6 / 3.5, 8192 of them 14.9 / 3.8, 2048 tokens, 6 of 64 in 8 groups 12.0 / 5.3, 400 tokens, 2 of 64 4.4 / 3.8.
+template <int G>
+__global__ __launch_bounds__(256) void hy_moe_route_lanes_kernel(const float* z, int ld, int T, int E, int groups, int keep, int top, int32_t* ids, float* wts, RouteMode rm) {
+    constexpr int TPB = 256 / G;
+    __shared__ __attribute__((aligned(16))) float s_s[256], k_s[256], g_s[256];
+    const int tid = threadIdx.x, l = tid % G, at = tid - l, t = blockIdx.x * TPB + tid / G;
+    const bool on = t < T && l < E;
+    const float zv = on ? z[(size_t)t * ld + l] : -INFINITY;
+    float sc;
+    if (rm.score == 1) sc = hy_sigmoid(zv);
+    else {
+        float m = zv;
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, G));
+        sc = on ? expf(zv - m) : 0.f;
+        float sum = sc;
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, G);
+        if (rm.score == 0) sc = sc / sum;
+    }
+    const float key = rm.score ? zv : sc;
+    s_s[tid] = sc;
+    __syncthreads();
+    bool kept = true;
+    if (groups > 1 && keep < groups) {
+        const int per = E / groups, g = min(l, E - 1) / per;
+        float b1 = -1.f, b2 = -1.f;                               // the group's two largest scores (scores are >= 0)
+        for (int j = 0; j < per; ++j) {
+            const float v = s_s[at + g * per + j];
+            if (v > b1) { b2 = b1; b1 = v; } else if (v > b2) b2 = v;
+        }
+        const float mine = (rm.group_top >= 2 && per >= 2) ? b1 + b2 : b1;
+        if (l < E && l % per == 0) g_s[at + g] = mine;
+        __syncthreads();
+        int front = 0;
+        for (int j = 0; j < groups; ++j) { const float v = g_s[at + j]; front += v > mine || (v == mine && j < g); }
+        kept = front < keep;
+    }
+    const bool ok = on && kept && sc >= 0.f;                      // a score that is no number is never in front of one that is
+    k_s[tid] = ok ? key : NAN;                                    // not in front of any
+    const unsigned long long okm = __builtin_amdgcn_ballot_w64(ok) >> ((tid & 63) - l) & (G == 64 ? ~0ull : (1ull << (G & 63)) - 1), before = (1ull << l) - 1;
+    __syncthreads();
+    int rank = 0;
+#pragma unroll
+    for (int j0 = 0; j0 < G; j0 += 4) {
+        const f32x4 v = *(const f32x4*)(k_s + at + j0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rank += (int)(v[e] > key) + ((int)(v[e] == key) & (int)(j0 + e < l));
+    }
+    if (!ok) rank = __popcll(okm) + __popcll(~okm & before);
+    const bool chosen = on && rank < top;
+    if (rm.score == 2) {                                          // normalised over the chosen, added in their order
+        __syncthreads();
+        if (chosen) s_s[at + rank] = sc;
+        __syncthreads();
+        float sum = 0.f;
+        for (int k = 0; k < top; ++k) sum += s_s[at + k];
+        if (chosen) wts[(size_t)t * top + rank] = sc * rm.wscale / sum;
+    } else if (chosen) wts[(size_t)t * top + rank] = sc * rm.wscale;
+    if (chosen) ids[(size_t)t * top + rank] = l;
+}
+
 // Counting sort of the n = tokens * top (token, choice) pairs by expert, one block: offs [E + 1], src_row[sorted place] = token,
 // place_of[pair] = sorted place, tiles = {count, (expert, first row) x count}: the 64-row tiles of the sorted list that hold rows.  The order
 // inside an expert is arbitrary (rows are independent of each other).
@@ -2484,25 +2548,83 @@ __device__ __forceinline__ void hy_align_pairs(const int32_t* ids, int n, int to
     }
 }
 
+// The same of up to 64 experts and 32768 pairs: a pair's place among its wave's of the same expert comes with the count, so that the pairs are counted once; the sums over waves and experts
+// and the list of tiles are one wave's, a lane for each expert.  Us a launch, before / now: 6148 pairs, 16 experts 8.1 / 4.8, 400
+// 3.3 / 2.5, 32768 31.3 / 23.5; 12288 pairs, 64 experts 18.2 / 11.6.
+constexpr int kSortPairs = 32, kSortExperts = 64;            // pairs a thread at most
+template <int PER>
+__device__ __forceinline__ void hy_align_few_experts(const int32_t* ids, int n, int top, int E, int (&cnt)[16][kSortExperts], int (&first)[kSortExperts], int32_t* offs, int32_t* src_row,
+                                                     int32_t* place_of, int32_t* tiles) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int id[PER], at[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) id[k] = k * 1024 + tid < n ? ids[k * 1024 + tid] : 0;
+    cnt[wave][lane] = 0;                                     // a wave's own counts
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) if (k * 1024 + tid < n) at[k] = atomicAdd(&cnt[wave][id[k]], 1);
+    __syncthreads();
+    if (wave == 0) {
+        int c[16], sum = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) c[w] = cnt[w][lane];
+#pragma unroll
+        for (int w = 0; w < 16; ++w) { cnt[w][lane] = sum; sum += c[w]; }
+        const int nt = (sum + 63) >> 6;
+        int o = sum, ot = nt;                                // sums over the experts up to this one
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int po = __shfl_up(o, d, 64), pt = __shfl_up(ot, d, 64);
+            if (lane >= d) { o += po; ot += pt; }
+        }
+        const int o0 = o - sum, t0 = ot - nt;
+        first[lane] = o0;
+        if (lane < E) {
+            offs[lane] = o0;
+            for (int m = 0; m < nt; ++m) { tiles[1 + 2 * (t0 + m)] = lane; tiles[2 + 2 * (t0 + m)] = o0 + m * 64; }
+        }
+        if (lane == 63) { offs[E] = o; tiles[0] = ot; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int i = k * 1024 + tid;
+        if (i < n) {
+            const int to = first[id[k]] + cnt[wave][id[k]] + at[k];
+            src_row[to] = i / top;
+            place_of[i] = to;
+        }
+    }
+}
+
 // The sort keeps one CU busy and the rest of the chip waiting, while the grouped linear behind it would start on weights that lie in HBM: spare blocks of the launch read them
-// (`lines` lines of 128 bytes) into the Infinity Cache.  1537 tokens, 4 of 16 experts of 704 at width 1024: the sort 9.2 -> 11.4 us with 46 MB read, the linear behind it 45 -> 38.
-// In the routing launch, one wave a token, the same reads cost 4 to 9 us: its 1537 blocks are dealt before them, or wait behind them.
+// (`lines` lines of 128 bytes) into the Infinity Cache.  1537 tokens, 4 of 16 experts of 704 at width 1024: the launch takes 11.4 us with 46 MB read, the linear behind it 45 -> 38.
+// Half of the same reads beside the routing instead gain nothing more (a prompt 1974 us against 1976).
 constexpr int kAlignLines = 2;
+// Block b of those that a launch has to spare: its share of a weight's lines of 128 bytes, a word of each, all of a thread asked for at once.
+__device__ __forceinline__ void hy_read_ahead(const char* ahead, uint32_t lines, uint32_t b) {
+    uint32_t v[kAlignLines];
+#pragma unroll
+    for (int k = 0; k < kAlignLines; ++k) {
+        const uint32_t i = (b * kAlignLines + k) * blockDim.x + threadIdx.x;
+        v[k] = i < lines ? *(const uint32_t*)(ahead + (size_t)i * 128) : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kAlignLines; ++k) asm volatile("" :: "v"(v[k]));
+}
 __global__ __launch_bounds__(1024) void hy_moe_align_kernel(const int32_t* ids, int n, int top, int E, int32_t* offs, int32_t* src_row, int32_t* place_of,
                                                             int32_t* tiles, const char* ahead, uint32_t lines) {
     extern __shared__ int hy_cnt[];             // counts [E], cursors [E]
-    if (blockIdx.x > 0) {                       // spare blocks: a word of each 128-byte line, all of a thread asked for at once
-        uint32_t v[kAlignLines];
-#pragma unroll
-        for (int k = 0; k < kAlignLines; ++k) {
-            const uint32_t i = ((blockIdx.x - 1) * kAlignLines + k) * 1024 + threadIdx.x;
-            v[k] = i < lines ? *(const uint32_t*)(ahead + (size_t)i * 128) : 0u;
-        }
-#pragma unroll
-        for (int k = 0; k < kAlignLines; ++k) asm volatile("" :: "v"(v[k]));
-        return;
-    }
+    if (blockIdx.x > 0) { hy_read_ahead(ahead, lines, blockIdx.x - 1); return; }
     hy_align_pairs(ids, n, top, E, hy_cnt, hy_cnt + E, offs, src_row, place_of, tiles);
+}
+
+template <int PER>
+__global__ __launch_bounds__(1024) void hy_moe_align_few_kernel(const int32_t* ids, int n, int top, int E, int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles,
+                                                                const char* ahead, uint32_t lines) {
+    __shared__ int cnt[16][kSortExperts], first[kSortExperts];
+    if (blockIdx.x > 0) { hy_read_ahead(ahead, lines, blockIdx.x - 1); return; }
+    hy_align_few_experts<PER>(ids, n, top, E, cnt, first, offs, src_row, place_of, tiles);
 }
 
 // Routing and sorting of a few tokens (a decode step) in ONE block: its sixteen waves route a token each per trip, then the block sorts the pairs.
@@ -3207,18 +3329,36 @@ extern "C" int mi355_hy_moe_route(const float* z, int32_t ld, int32_t tokens, in
 
 // The same with the router's form as arguments: score (0: softmax over all logits, 1: a sigmoid of each, 2: softmax over the chosen ones), group_top (1: a group
 // scores as its best expert; 2: as the sum of its two best), wscale (the chosen experts weigh score * wscale).
-extern "C" int mi355_hy_moe_route_ex(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
-                                     int32_t score, int32_t group_top, float wscale, mi355_stream_t stream) {
+static int moe_route_check(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, const int32_t* ids, const float* wts, int32_t score,
+                           int32_t group_top) {
     MI355_CHECK_ARG(score >= 0 && score <= 2, "hy_moe_route: score form %d", score);
     MI355_CHECK_ARG(group_top == 1 || group_top == 2, "hy_moe_route: a group scores by its best %d experts (1 or 2)", group_top);
-    const RouteMode rm{score, group_top, wscale};
     MI355_CHECK_ARG(z && ids && wts && tokens > 0 && E > 0 && ld >= E, "hy_moe_route: tokens=%d experts=%d", tokens, E);
     MI355_CHECK_ARG(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && top >= 1 && top <= (E / groups) * keep, "hy_moe_route: %d experts in %d groups, keep %d, top %d",
                     E, groups, keep, top);
     MI355_CHECK_ARG((size_t)(E + groups) * 4 <= 48 * 1024, "hy_moe_route: %d experts do not fit the block's scratch", E);
-    hipLaunchKernelGGL(hy_moe_route_kernel, dim3(tokens), dim3(64), (size_t)(E + groups) * 4, (hipStream_t)stream, z, ld, E, groups, keep, top, ids, wts, rm);
+    return MI355_OK;
+}
+
+static int moe_route(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts, int32_t score, int32_t group_top,
+                     float wscale, hipStream_t st) {
+    const RouteMode rm{score, group_top, wscale};
+    auto lanes = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        hipLaunchKernelGGL((hy_moe_route_lanes_kernel<G>), dim3((tokens + 256 / G - 1) / (256 / G)), dim3(256), 0, st, z, ld, tokens, E, groups, keep, top, ids, wts, rm);
+    };
+    if (E <= 16)      lanes(std::integral_constant<int, 16>{});
+    else if (E <= 32) lanes(std::integral_constant<int, 32>{});
+    else if (E <= 64) lanes(std::integral_constant<int, 64>{});
+    else hipLaunchKernelGGL(hy_moe_route_kernel, dim3(tokens), dim3(64), (size_t)(E + groups) * 4, st, z, ld, E, groups, keep, top, ids, wts, rm);
     MI355_CHECK_LAUNCH("hy_moe_route_kernel");
     return MI355_OK;
+}
+
+extern "C" int mi355_hy_moe_route_ex(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
+                                     int32_t score, int32_t group_top, float wscale, mi355_stream_t stream) {
+    if (int e = moe_route_check(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top)) return e;
+    return moe_route(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top, wscale, (hipStream_t)stream);
 }
 
 static int moe_align(const int32_t* ids, int32_t n, int32_t top, int32_t E, int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, const void* ahead, int64_t bytes,
@@ -3226,7 +3366,12 @@ static int moe_align(const int32_t* ids, int32_t n, int32_t top, int32_t E, int3
     MI355_CHECK_ARG(ids && offs && src_row && place_of && tiles && n > 0 && top > 0 && E > 0 && (size_t)E * 8 <= 48 * 1024, "hy_moe_align: n=%d experts=%d", n, E);
     const uint32_t lines = ahead && bytes > 0 ? (uint32_t)((bytes < (int64_t)48 << 20 ? bytes : (int64_t)48 << 20) / 128) : 0u;
     const int spare = (lines + 1024 * kAlignLines - 1) / (1024 * kAlignLines);
-    hipLaunchKernelGGL(hy_moe_align_kernel, dim3(1 + spare), dim3(1024), (size_t)E * 8, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
+    if (E <= kSortExperts && n <= 1024 * 8)
+        hipLaunchKernelGGL(hy_moe_align_few_kernel<8>, dim3(1 + spare), dim3(1024), 0, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
+    else if (E <= kSortExperts && n <= 1024 * kSortPairs)
+        hipLaunchKernelGGL(hy_moe_align_few_kernel<kSortPairs>, dim3(1 + spare), dim3(1024), 0, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
+    else
+        hipLaunchKernelGGL(hy_moe_align_kernel, dim3(1 + spare), dim3(1024), (size_t)E * 8, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
     MI355_CHECK_LAUNCH("hy_moe_align_kernel");
     return MI355_OK;
 }
@@ -3241,8 +3386,9 @@ extern "C" int mi355_hy_moe_align(const int32_t* ids, int32_t n, int32_t top, in
 extern "C" int mi355_hy_moe_route_sorted(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
                                          int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top, float wscale,
                                          const void* ahead, int64_t ahead_bytes, mi355_stream_t stream) {
-    const int e = mi355_hy_moe_route_ex(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top, wscale, stream);
-    return e != MI355_OK ? e : moe_align(ids, tokens * top, top, E, offs, src_row, place_of, tiles, ahead, ahead_bytes, (hipStream_t)stream);
+    if (int e = moe_route_check(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top)) return e;
+    if (int e = moe_route(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top, wscale, (hipStream_t)stream)) return e;
+    return moe_align(ids, tokens * top, top, E, offs, src_row, place_of, tiles, ahead, ahead_bytes, (hipStream_t)stream);
 }
 
 // Both in one launch for a few tokens (tokens <= 64 and the scratch of sixteen waves fits: MI355_ERR_UNSUPPORTED otherwise).
