@@ -146,6 +146,10 @@ int mi355_hy_moe_route_ex(const float* z, int32_t ld, int32_t tokens, int32_t E,
 int mi355_hy_moe_route_sorted(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
                               int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top, float wscale,
                               const void* ahead, int64_t ahead_bytes, mi355_stream_t stream);
+/* ... and one more expert, number E, that takes every token (shared != 0): its rows lie in token order behind the pairs', offs has E + 2 entries, src_row tokens * (top + 1), tiles room for tokens / 64 + 1 more. */
+int mi355_hy_moe_route_sorted_shared(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts, int32_t* offs,
+                                     int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top, float wscale, int32_t shared, const void* ahead,
+                                     int64_t ahead_bytes, mi355_stream_t stream);
 int mi355_hy_moe_route_align_ex(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
                                 int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top,
                                 float wscale, mi355_stream_t stream);

@@ -238,6 +238,7 @@ HYBRID_SIGNATURES = {
     "mi355_dense_grouped_ahead": (i32, [vp, i32, i32, vp, i32, i32, vp, vp, i32, i32, i32, i32, f32, i32, i32, C.c_int64, C.c_int64, vp, vp, vp, i32, vp, i32, i32, vp, C.c_int64, vp]),
     "mi355_hy_moe_route_ex": (i32, [vp, i32, i32, i32, i32, i32, i32, vp, vp, i32, i32, f32, vp]),
     "mi355_hy_moe_route_sorted": (i32, [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, i32, f32, vp, C.c_int64, vp]),
+    "mi355_hy_moe_route_sorted_shared": (i32, [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, i32, f32, i32, vp, C.c_int64, vp]),
     "mi355_hy_moe_route_align_ex": (i32, [vp, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, i32, f32, vp]),
     "mi355_hy_attn_prep_ex2": (i32, [vp, i32, i32, i32, ip, vp, vp, i32, f32, vp, vp, vp, i32, vp, vp, vp, vp, i32, f32, f32, i32, i32, vp]),
     "mi355_hy_embed_scaled": (i32, [vp, i32, vp, i32, i32, f32, vp, vp, i32, vp]),

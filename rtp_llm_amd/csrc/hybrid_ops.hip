@@ -2525,6 +2525,12 @@ __global__ __launch_bounds__(256) void hy_moe_route_lanes_kernel(const float* z,
 // Counting sort of the n = tokens * top (token, choice) pairs by expert, one block: offs [E + 1], src_row[sorted place] = token,
 // place_of[pair] = sorted place, tiles = {count, (expert, first row) x count}: the 64-row tiles of the sorted list that hold rows.  The order
 // inside an expert is arbitrary (rows are independent of each other).
+// shared > 0: one more expert, E, that so many tokens all take, in order, behind the pairs (offs [E + 2], their tiles behind the others).
+__device__ __forceinline__ void hy_align_shared(int shared, int n, int E, int nt, int32_t* offs, int32_t* src_row, int32_t* tiles) {
+    for (int t = threadIdx.x; t < shared; t += blockDim.x) src_row[n + t] = t;
+    for (int m = threadIdx.x; m * 64 < shared; m += blockDim.x) { tiles[1 + 2 * (nt + m)] = E; tiles[2 + 2 * (nt + m)] = n + m * 64; }
+    if (threadIdx.x == 0) { offs[E + 1] = n + shared; tiles[0] = nt + ((shared + 63) >> 6); }
+}
 __device__ __forceinline__ void hy_align_pairs(const int32_t* ids, int n, int top, int E, int* cnt, int* cur, int32_t* offs, int32_t* src_row,
                                                int32_t* place_of, int32_t* tiles) {
     for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
@@ -2553,7 +2559,7 @@ __device__ __forceinline__ void hy_align_pairs(const int32_t* ids, int n, int to
 // 3.3 / 2.5, 32768 31.3 / 23.5; 12288 pairs, 64 experts 18.2 / 11.6.
 constexpr int kSortPairs = 32, kSortExperts = 64;            // pairs a thread at most
 template <int PER>
-__device__ __forceinline__ void hy_align_few_experts(const int32_t* ids, int n, int top, int E, int (&cnt)[16][kSortExperts], int (&first)[kSortExperts], int32_t* offs, int32_t* src_row,
+__device__ __forceinline__ void hy_align_few_experts(const int32_t* ids, int n, int top, int E, int (&cnt)[16][kSortExperts], int (&first)[kSortExperts], int& all, int32_t* offs, int32_t* src_row,
                                                      int32_t* place_of, int32_t* tiles) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int id[PER], at[PER];
@@ -2583,7 +2589,7 @@ __device__ __forceinline__ void hy_align_few_experts(const int32_t* ids, int n, 
             offs[lane] = o0;
             for (int m = 0; m < nt; ++m) { tiles[1 + 2 * (t0 + m)] = lane; tiles[2 + 2 * (t0 + m)] = o0 + m * 64; }
         }
-        if (lane == 63) { offs[E] = o; tiles[0] = ot; }
+        if (lane == 63) { offs[E] = o; tiles[0] = all = ot; }
     }
     __syncthreads();
 #pragma unroll
@@ -2613,18 +2619,20 @@ __device__ __forceinline__ void hy_read_ahead(const char* ahead, uint32_t lines,
     for (int k = 0; k < kAlignLines; ++k) asm volatile("" :: "v"(v[k]));
 }
 __global__ __launch_bounds__(1024) void hy_moe_align_kernel(const int32_t* ids, int n, int top, int E, int32_t* offs, int32_t* src_row, int32_t* place_of,
-                                                            int32_t* tiles, const char* ahead, uint32_t lines) {
+                                                            int32_t* tiles, const char* ahead, uint32_t lines, int shared) {
     extern __shared__ int hy_cnt[];             // counts [E], cursors [E]
     if (blockIdx.x > 0) { hy_read_ahead(ahead, lines, blockIdx.x - 1); return; }
     hy_align_pairs(ids, n, top, E, hy_cnt, hy_cnt + E, offs, src_row, place_of, tiles);
+    if (shared > 0) { const int nt = tiles[0]; __syncthreads(); hy_align_shared(shared, n, E, nt, offs, src_row, tiles); }
 }
 
 template <int PER>
 __global__ __launch_bounds__(1024) void hy_moe_align_few_kernel(const int32_t* ids, int n, int top, int E, int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles,
-                                                                const char* ahead, uint32_t lines) {
-    __shared__ int cnt[16][kSortExperts], first[kSortExperts];
+                                                                const char* ahead, uint32_t lines, int shared) {
+    __shared__ int cnt[16][kSortExperts], first[kSortExperts], all;
     if (blockIdx.x > 0) { hy_read_ahead(ahead, lines, blockIdx.x - 1); return; }
-    hy_align_few_experts<PER>(ids, n, top, E, cnt, first, offs, src_row, place_of, tiles);
+    hy_align_few_experts<PER>(ids, n, top, E, cnt, first, all, offs, src_row, place_of, tiles);
+    if (shared > 0) hy_align_shared(shared, n, E, all, offs, src_row, tiles);
 }
 
 // Routing and sorting of a few tokens (a decode step) in ONE block: its sixteen waves route a token each per trip, then the block sorts the pairs.
@@ -3361,17 +3369,17 @@ extern "C" int mi355_hy_moe_route_ex(const float* z, int32_t ld, int32_t tokens,
     return moe_route(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top, wscale, (hipStream_t)stream);
 }
 
-static int moe_align(const int32_t* ids, int32_t n, int32_t top, int32_t E, int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, const void* ahead, int64_t bytes,
+static int moe_align(const int32_t* ids, int32_t n, int32_t top, int32_t E, int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, const void* ahead, int64_t bytes, int32_t shared,
                      hipStream_t st) {
     MI355_CHECK_ARG(ids && offs && src_row && place_of && tiles && n > 0 && top > 0 && E > 0 && (size_t)E * 8 <= 48 * 1024, "hy_moe_align: n=%d experts=%d", n, E);
     const uint32_t lines = ahead && bytes > 0 ? (uint32_t)((bytes < (int64_t)48 << 20 ? bytes : (int64_t)48 << 20) / 128) : 0u;
     const int spare = (lines + 1024 * kAlignLines - 1) / (1024 * kAlignLines);
     if (E <= kSortExperts && n <= 1024 * 8)
-        hipLaunchKernelGGL(hy_moe_align_few_kernel<8>, dim3(1 + spare), dim3(1024), 0, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
+        hipLaunchKernelGGL(hy_moe_align_few_kernel<8>, dim3(1 + spare), dim3(1024), 0, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines, shared);
     else if (E <= kSortExperts && n <= 1024 * kSortPairs)
-        hipLaunchKernelGGL(hy_moe_align_few_kernel<kSortPairs>, dim3(1 + spare), dim3(1024), 0, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
+        hipLaunchKernelGGL(hy_moe_align_few_kernel<kSortPairs>, dim3(1 + spare), dim3(1024), 0, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines, shared);
     else
-        hipLaunchKernelGGL(hy_moe_align_kernel, dim3(1 + spare), dim3(1024), (size_t)E * 8, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines);
+        hipLaunchKernelGGL(hy_moe_align_kernel, dim3(1 + spare), dim3(1024), (size_t)E * 8, st, ids, n, top, E, offs, src_row, place_of, tiles, (const char*)ahead, lines, shared);
     MI355_CHECK_LAUNCH("hy_moe_align_kernel");
     return MI355_OK;
 }
@@ -3379,16 +3387,23 @@ static int moe_align(const int32_t* ids, int32_t n, int32_t top, int32_t E, int3
 // tiles: int32 [1 + 2 * (n / 64 + E)] (at most n / 64 + E tiles hold rows)
 extern "C" int mi355_hy_moe_align(const int32_t* ids, int32_t n, int32_t top, int32_t E, int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles,
                                   mi355_stream_t stream) {
-    return moe_align(ids, n, top, E, offs, src_row, place_of, tiles, nullptr, 0, (hipStream_t)stream);
+    return moe_align(ids, n, top, E, offs, src_row, place_of, tiles, nullptr, 0, 0, (hipStream_t)stream);
 }
 
 // Both launches of many tokens; the second also reads the weight of the grouped linear behind it (ahead_bytes of ahead, at most 48 MB: about what HBM gives meanwhile).
 extern "C" int mi355_hy_moe_route_sorted(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
                                          int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top, float wscale,
                                          const void* ahead, int64_t ahead_bytes, mi355_stream_t stream) {
+    return mi355_hy_moe_route_sorted_shared(z, ld, tokens, E, groups, keep, top, ids, wts, offs, src_row, place_of, tiles, score, group_top, wscale, 0, ahead, ahead_bytes, stream);
+}
+
+// The same; shared: one more expert, number E, takes every token, behind the pairs: offs [E + 2], src_row [tokens * (top + 1)], tiles for tokens / 64 + 1 more.
+extern "C" int mi355_hy_moe_route_sorted_shared(const float* z, int32_t ld, int32_t tokens, int32_t E, int32_t groups, int32_t keep, int32_t top, int32_t* ids, float* wts,
+                                                int32_t* offs, int32_t* src_row, int32_t* place_of, int32_t* tiles, int32_t score, int32_t group_top, float wscale, int32_t shared,
+                                                const void* ahead, int64_t ahead_bytes, mi355_stream_t stream) {
     if (int e = moe_route_check(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top)) return e;
     if (int e = moe_route(z, ld, tokens, E, groups, keep, top, ids, wts, score, group_top, wscale, (hipStream_t)stream)) return e;
-    return moe_align(ids, tokens * top, top, E, offs, src_row, place_of, tiles, ahead, ahead_bytes, (hipStream_t)stream);
+    return moe_align(ids, tokens * top, top, E, offs, src_row, place_of, tiles, ahead, ahead_bytes, shared ? tokens : 0, (hipStream_t)stream);
 }
 
 // Both in one launch for a few tokens (tokens <= 64 and the scratch of sixteen waves fits: MI355_ERR_UNSUPPORTED otherwise).

@@ -1033,25 +1033,27 @@ def _ahead(t: Optional[torch.Tensor], name: str):
 
 
 def moe_route_sorted(z: torch.Tensor, experts: int, groups: int, keep: int, top: int, *, sigmoid: bool = False, chosen: bool = False, group_top: int = 1, scale: float = 1.0,
-                     ahead: Optional[torch.Tensor] = None):
+                     ahead: Optional[torch.Tensor] = None, shared: bool = False):
     """moe_route followed by moe_align -> (ids, wts, offs, src_row, place_of, tiles); a few tokens (a decode step) take one launch for both.  ahead: the
-    contiguous weight of the grouped linear behind, which the sort of many tokens reads into the caches on the way."""
+    contiguous weight of the grouped linear behind, which the sort of many tokens reads into the caches on the way.  shared: one more expert, number `experts`, takes every token: its rows lie
+    behind the pairs' in token order, src_row and tiles go on over them and offs has an entry more."""
     _dev(z, torch.float32, "moe_route_sorted.z")
     T = z.shape[0]
     if z.shape[1] != experts:
         raise _C.Mi355Error(f"moe_route_sorted: logits {tuple(z.shape)} for {experts} experts")
-    many = not 0 < T <= 64 or 16 * (experts + groups) * 4 + experts * 8 > 48 * 1024
+    more = 1 if shared else 0
+    many = shared or not 0 < T <= 64 or 16 * (experts + groups) * 4 + experts * 8 > 48 * 1024
     if T == 0:
         ids, wts = moe_route(z, groups, keep, top, sigmoid=sigmoid, chosen=chosen, group_top=group_top, scale=scale)
-        return (ids, wts) + moe_align(ids, experts)
+        return (ids, wts) + moe_align(ids, experts + more)
     dev = z.device
     ids, wts = torch.empty(T, top, dtype=torch.int32, device=dev), torch.empty(T, top, dtype=torch.float32, device=dev)
-    offs, src, place = torch.empty(experts + 1, dtype=torch.int32, device=dev), torch.empty(T * top, dtype=torch.int32, device=dev), torch.empty(T * top, dtype=torch.int32, device=dev)
-    tiles = torch.empty(1 + 2 * (T * top // 64 + experts), dtype=torch.int32, device=dev)
+    offs, src, place = torch.empty(experts + 1 + more, dtype=torch.int32, device=dev), torch.empty(T * (top + more), dtype=torch.int32, device=dev), torch.empty(T * top, dtype=torch.int32, device=dev)
+    tiles = torch.empty(1 + 2 * (T * top // 64 + experts + more * (T // 64 + 1)), dtype=torch.int32, device=dev)
     args = (z.data_ptr(), _rows(z, "moe_route_sorted.z"), T, experts, groups, keep, top, ids.data_ptr(), wts.data_ptr(), offs.data_ptr(), src.data_ptr(), place.data_ptr(),
             tiles.data_ptr(), 2 if chosen else 1 if sigmoid else 0, int(group_top), float(scale))
     if many:
-        _C.check_hybrid(_C.hybrid_lib().mi355_hy_moe_route_sorted(*args, *_ahead(ahead, "moe_route_sorted.ahead"), _stream()), "hy_moe_route_sorted")
+        _C.check_hybrid(_C.hybrid_lib().mi355_hy_moe_route_sorted_shared(*args, more, *_ahead(ahead, "moe_route_sorted.ahead"), _stream()), "hy_moe_route_sorted")
     else:
         _C.check_hybrid(_C.hybrid_lib().mi355_hy_moe_route_align_ex(*args, _stream()), "hy_moe_route_align")
     return ids, wts, offs, src, place, tiles
