@@ -439,6 +439,12 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
     const bf16* Bi = p.bias ? (const bf16*)p.bias + gr.bo : nullptr;
     char* mine = smem + wave * (PH * 4096);
     const int nc = n0 + wn * WN;                                            // the wave's first weight row
+    // What most calls ask for has code of its own: the choice among activations, caps, gates and output types a value took 1400 cycles a trip of the general loops (8192 x 11264 x 2048
+    // gated: 11 of a block's 67 us, 3.6 now; all of it 359 / 325 us, 1537 x 1408 x 1024 gated 14.2 / 11.8, 456 x 11264 x 2048 gated 41.3 / 39.1, 1537 x 2176 x 1024 15.3 / 14.5).
+    const bool lean = p.softcap <= 0.f && p.yvec && p.N % 4 == 0;
+    const bool lean_gated = lean && p.gated && !p.egate && !Bi && !p.out_f32 && (p.act == DN_ACT_RELU || p.act == DN_ACT_SILU) && p.ldy % 8 == 0 && (uintptr_t)p.y % 16 == 0 && gr.yo % 8 == 0;
+    const bool lean_plain = lean && !p.gated && !p.egate && p.out_f32 && p.act == DN_ACT_NONE && gr.yo % 4 == 0;
+    const bool lean_scaled = lean && !p.gated && p.egate && !Bi && !p.out_f32 && p.act == DN_ACT_NONE && gr.yo % 4 == 0 && p.ldg % 4 == 0 && p.goff % 4 == 0 && (uintptr_t)p.egate % 16 == 0;
     __syncthreads();
 #pragma unroll
     for (int i0 = 0; i0 < MI; i0 += PH) {
@@ -448,7 +454,70 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
             for (int j = 0; j < NJ; ++j) *(f32x4*)(mine + (i * 16 + fr) * 256 + (((j * 4 + q) ^ fr) << 4)) = acc[i0 + i][j];
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // the wave's own stores, read by its other lanes
         const int r0 = m0 + wm * WM + i0 * 16, rows = min(PH * 16, gr.rend - r0);
-        if (p.gated) {
+        if (lean_gated) {                                                   // 8 channels a lane, 4 lanes a row: 16 bytes a store
+            const int c8 = lane & 3, c = nc + c8 * 8;
+            bf16* y = (bf16*)p.y + (size_t)(r0 + (lane >> 2)) * p.ldy + (int)gr.yo + (nc >> 1) + c8 * 8;
+            auto out = [&](auto gate) {
+#pragma unroll
+                for (int k = 0; k < PH; ++k) {
+                    const int r = k * 16 + (lane >> 2);
+                    const char* at = mine + r * 256;
+                    f32x4 g[2], u[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        g[h] = *(const f32x4*)(at + (((2 * c8 + h) ^ (r & 15)) << 4));
+                        u[h] = *(const f32x4*)(at + (((2 * c8 + h + 8) ^ (r & 15)) << 4));
+                    }
+                    u32x4 o;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        float v[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = gate(g[h][e]) * u[h][e];
+                        o[2 * h] = act_pack<true>(v[0], v[1]); o[2 * h + 1] = act_pack<true>(v[2], v[3]);
+                    }
+                    if (r < rows && c < p.N) *(u32x4*)(y + (size_t)(k * 16) * p.ldy) = o;
+                }
+            };
+            if (p.act == DN_ACT_SILU) out([](float g) { return dn_act(g, DN_ACT_SILU); }); else out([](float g) { return dn_act(g, DN_ACT_RELU); });
+        } else if (lean_plain) {
+            const int c4 = lane & 15, n = nc + c4 * 4;
+            f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+            if (Bi && n < p.N) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bias[e] = dn_ld(Bi + n + e);
+            }
+            float* y = (float*)p.y + (size_t)(r0 + (lane >> 4)) * p.ldy + (int)gr.yo + n;
+#pragma unroll 4
+            for (int k = 0; k < PH * 4; ++k) {
+                const int r = k * 4 + (lane >> 4);
+                f32x4 v = *(const f32x4*)(mine + r * 256 + ((c4 ^ (r & 15)) << 4));
+                if (Bi) v += bias;
+                if (r < rows && n < p.N) *(f32x4*)(y + (size_t)(k * 4) * p.ldy) = v;
+            }
+        } else if (lean_scaled) {
+            const int c4 = lane & 15, n = nc + c4 * 4;
+            const size_t row = r0 + (lane >> 4);
+            const float* z = p.egate + row * p.ldg + p.goff + (int)gr.yo + n;
+            bf16* y = (bf16*)p.y + row * p.ldy + (int)gr.yo + n;
+            constexpr int U = 4;                                            // rows whose gates are asked for together
+#pragma unroll 1
+            for (int k0 = 0; k0 < PH * 4; k0 += U) {
+                f32x4 zv[U];
+#pragma unroll
+                for (int k = 0; k < U; ++k)
+                    if ((k0 + k) * 4 + (lane >> 4) < rows && n < p.N) zv[k] = *(const f32x4*)(z + (size_t)((k0 + k) * 4) * p.ldg);
+#pragma unroll
+                for (int k = 0; k < U; ++k) {
+                    const int r = (k0 + k) * 4 + (lane >> 4);
+                    f32x4 v = *(const f32x4*)(mine + r * 256 + ((c4 ^ (r & 15)) << 4));
+                    if (r >= rows || n >= p.N) continue;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] *= 1.f / (1.f + expf(-zv[k][e]));
+                    *(u32x2*)(y + (size_t)((k0 + k) * 4) * p.ldy) = u32x2{act_pack<true>(v[0], v[1]), act_pack<true>(v[2], v[3])};
+                }
+            }
+        } else if (p.gated) {
             const int c4 = lane & 7;                                        // channels 4 c4 .. of the wave's 32
             if (nc + c4 * 4 + 32 < p.N)
 #pragma unroll 1
