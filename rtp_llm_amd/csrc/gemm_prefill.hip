@@ -41,6 +41,63 @@ __device__ __forceinline__ void store_bf16(const GemmParams& p, f32x4 v, int m, 
     }
 }
 
+// The stores of tiles two or four weight tiles wide to rows on 16 bytes: the finished values pass through LDS, so that a store writes 16 bytes a lane and whole runs of a row (128 bytes of it where
+// a wave has 64 columns, 64 of gated ones).  From the accumulators a store was 16 rows by 32 bytes, of gated pairs 16 by 16, with a choice of mode, bias and image in front of each: us a block, before /
+// now: 128 x 512 gated 10.7 / 5.2 (divisions), plain 7.6 / 3.0, 128 x 256 4.4 / 1.9, 64 x 256 2.2 / 1.3.  us a call: fp16 W4 at 4096 rows 37888 x 3584 gated 925 / 888, 3584 x 3584 97 / 90, 8 bits
+// at 1055 rows 37888 x 3584 gated 270 / 256.
+__device__ __forceinline__ bool lean_store(const GemmParams& p) {
+    const bool silu = p.mode == MODE_SILU;
+    return !p.y_img && (silu || p.mode == MODE_F16) && p.ldy % 8 == 0 && (uintptr_t)p.y % 16 == 0 && p.N % (silu ? 16 : 8) == 0;
+}
+// acc of a wave: row m0 + 16 mb + (lane & 15), columns n0 + 16 t + 4 (lane >> 4) + r, times the column's scale.  mine: the wave's 1 KB of LDS per 16 rows.  The arithmetic of gemm_store and store_bf16.
+template <bool BF, int MB, int TPW, bool SILU>
+__device__ __forceinline__ void store_rows(const GemmParams& p, const f32x4 (&acc)[TPW][MB], const f32x4 (&sc)[TPW], char* mine, int m0, int n0, int lane) {
+    constexpr int RB = SILU ? TPW * 16 : TPW * 32, P = RB / 16;              // bytes and 16-byte pieces of a row of the wave's results
+    constexpr int PH = MB * 1024 / (RB * 16) < MB ? MB * 1024 / (RB * 16) : MB;   // 16-row blocks that fit the wave's LDS together
+    const int jj = lane & 15, q = lane >> 4;
+    auto place = [](int row, int piece) { return row * RB + ((piece ^ (P == 8 ? row & 7 : P == 4 ? (row >> 1) & 3 : (row >> 2) & 1)) << 4); };
+    f32x4 bias[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+        bias[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int n = n0 + t * 16 + q * 4;
+        if (p.bias && n < p.N) {
+            const u32x2 b = *reinterpret_cast<const u32x2*>(p.bias + n);
+            bias[t] = f32x4{act_lo<BF>(b[0]), act_hi<BF>(b[0]), act_lo<BF>(b[1]), act_hi<BF>(b[1])};
+        }
+    }
+#pragma unroll
+    for (int p0 = 0; p0 < MB; p0 += PH) {
+#pragma unroll
+        for (int mb = p0; mb < p0 + PH; ++mb)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) {
+                f32x4 v = acc[t][mb] * sc[t];
+                if (p.bias) v += bias[t];
+                const int row = (mb - p0) * 16 + jj;
+                if constexpr (SILU) {
+                    float o[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const float g = act_round<BF>(v[2 * e]), u = act_round<BF>(v[2 * e + 1]);
+                        o[e] = (g / (1.f + __expf(-g))) * u;
+                    }
+                    *(uint32_t*)(mine + place(row, t) + q * 4) = act_pack<BF>(o[0], o[1]);
+                } else *(u32x2*)(mine + place(row, t * 2 + (q >> 1)) + (q & 1) * 8) = u32x2{act_pack<BF>(v[0], v[1]), act_pack<BF>(v[2], v[3])};
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                  // the wave's own, read by its other lanes
+        const int r0 = lane / P, piece = lane % P, col = (SILU ? n0 >> 1 : n0) + piece * 8, m = m0 + p0 * 16 + r0;
+        f16* y = (f16*)p.y + (size_t)m * p.ldy + col;
+        const bool ok = col < (SILU ? p.N >> 1 : p.N);
+#pragma unroll
+        for (int k = 0; k < PH * 16 * P / 64; ++k) {
+            const u32x4 v = *(const u32x4*)(mine + place(k * (64 / P) + r0, piece));
+            if (ok && m + k * (64 / P) < p.M) *(u32x4*)(y + (size_t)(k * (64 / P)) * p.ldy) = v;
+        }
+        if (p0 + PH < MB) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+}
+
 // The chip deals consecutive blocks to its eight XCDs in turn, each with an L2 of its own.  Dealt row by row, the 32 blocks of an XCD read 32 column tiles of the weights
 // and hardly share one: at 128 x 512 tiles 2 MB of 8-bit codes per XCD and 128-k chunk from the Infinity Cache, 5.7 TB/s over the chip.  So an XCD takes a contiguous run
 // of tiles in an order of bands of up to PF_BAND row tiles, column by column: per chunk 4 column tiles and 8 row tiles, a quarter of the bytes.  Column counts that eight
@@ -397,19 +454,34 @@ __global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOL
                 for (int mb = 0; mb < MB; ++mb) acc[t][mb] += red[((((k - 1) * NWN + wn) * TPW + t) * MB + mb) * 64 + lane];
     }
 
+    f32x4 scales[TPW];                               // of 8 bits a column
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+        scales[t] = (f32x4){1.f, 1.f, 1.f, 1.f};
+        if (!GROUPED && WBITS != 16) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t m = __builtin_amdgcn_raw_buffer_load_b32(rm[t], (uint32_t)(q * 4 + r) * 4u, 0, 0);
+                scales[t][r] = (float)as_h2(m)[1];
+            }
+        }
+    }
+    if constexpr (KS == 1 && TPW >= 2 && !(TPW == 4 && GS == 1)) {           // 128 x 512 in groups of 32 has no registers left for it
+        if (lean_store(p)) {                         // the x buffers hold nothing any more: no DMA is left, and behind the barrier no reader
+            __syncthreads();
+            char* mine = (char*)&xs[0][0][0] + wave * (sizeof(xs) / 8);
+            if (p.mode == MODE_SILU) store_rows<BF, MB, TPW, true>(p, acc, scales, mine, m0, nt_base * 16, lane);
+            else                     store_rows<BF, MB, TPW, false>(p, acc, scales, mine, m0, nt_base * 16, lane);
+            return;
+        }
+    }
+
     // ---- epilogue: lane holds, for row m0 + mb*16 + jj, the 4 consecutive columns 16 nt + 4q + r
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
         if (!tile_ok[t]) continue;
         const int n0 = (nt_base + t) * 16 + q * 4;
-        f32x4 sc = {1.f, 1.f, 1.f, 1.f};
-        if (!GROUPED && WBITS != 16) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t m = __builtin_amdgcn_raw_buffer_load_b32(rm[t], (uint32_t)(q * 4 + r) * 4u, 0, 0);
-                sc[r] = (float)as_h2(m)[1];
-            }
-        }
+        const f32x4 sc = scales[t];
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
             const int m = m0 + mb * 16 + jj;
