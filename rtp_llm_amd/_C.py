@@ -102,6 +102,7 @@ SIGNATURES = {
     "mi355_linear_forward": (i32, [vp, i32, C.POINTER(Weight), vp, vp, i32, vp, sz, vp]),
     "mi355_gemm_prefill_shape": (i32, [i32] * 5),
     "mi355_gemm_prefill_form": (i32, [i32] * 7),
+    "mi355_gemm_prefill_rest": (i32, [i32] * 7),
     "mi355_gemm_prefill_tile": (C.c_int64, [i32] * 3),
     "mi355_linear_partial": (i32, [vp, i32, C.POINTER(Weight), vp, i32, vp]),
     "mi355_rmsnorm": (i32, [vp, vp, f32, i32, i32, vp, vp]),

@@ -157,9 +157,10 @@ constexpr int prefill_waves(int wbits, int gs, bool bf, int mb, int tpw, int ks,
     if (wbits == 4 && gs != 1 && !whole && bf && mb == 4 && tpw == 1 && ks == 1) return 6;
     return tpw * mb <= 16 && wbits != 16 && !(bf && wbits == 4) ? 2 : 1;
 }
+// xmem: the block's LDS, 8 MB KS KB; the block's tile: rows from m0 on, weight tiles from nt_block on
 template <int WBITS, int GS, bool BF, int MB, int TPW, int KS, bool WHOLE>
-__global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOLE)) void gemm_prefill_kernel(const GemmParams p, const int band) {
-    constexpr int BM = 16 * MB, NWN = 8 / KS;                 // rows, waves side by side
+__device__ __forceinline__ void prefill_block(const GemmParams& p, u32x4* xmem, const int m0, const int nt_block) {
+    constexpr int NWN = 8 / KS;                               // waves side by side
     constexpr int LPC  = WBITS / 4;
     constexpr int NSUB = (GS > 0) ? 4 / GS : 1;
     constexpr int SPG  = 4 / NSUB;
@@ -170,17 +171,14 @@ __global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOL
     constexpr bool HALVES = WHOLE && TPW == 4;                // the weights of half a chunk in registers, not of two chunks
     constexpr int WLD = TPW * ((HALVES ? 2 : LPC) + (GS > 0 ? NSUB : 0));     // weight loads per wave and chunk
     static_assert(!HALVES || (WBITS != 16 && !CSCALE && NSUB == 1 && KS == 1), "one scale a chunk");
-    __shared__ u32x4 xs[KS][2][XSLOTS];
+    u32x4 (*xs)[2][XSLOTS] = (u32x4(*)[2][XSLOTS])xmem;
     static_assert(KS == 1 || (size_t)(KS - 1) * NWN * TPW * MB * 1024 <= sizeof(u32x4) * 2 * KS * XSLOTS, "the slices' sums meet in the x buffers");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ks = wave / NWN;
     const int jj = lane & 15, q = lane >> 4;
-    int bx = blockIdx.x, by = blockIdx.y;
-    if (band) prefill_tile(by * (int)gridDim.x + bx, gridDim.y, gridDim.x, band, bx, by);
-    const int m0 = by * BM;
-    const int nt_base = (bx * NWN + wave % NWN) * TPW;
+    const int nt_base = nt_block + wave % NWN * TPW;
     const int KC = p.KC;
 
     constexpr uint32_t FLAGS = 0x00020000u;
@@ -469,7 +467,7 @@ __global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOL
     if constexpr (KS == 1 && TPW >= 2 && !(TPW == 4 && GS == 1)) {           // 128 x 512 in groups of 32 has no registers left for it
         if (lean_store(p)) {                         // the x buffers hold nothing any more: no DMA is left, and behind the barrier no reader
             __syncthreads();
-            char* mine = (char*)&xs[0][0][0] + wave * (sizeof(xs) / 8);
+            char* mine = (char*)&xs[0][0][0] + wave * (MB * 1024);
             if (p.mode == MODE_SILU) store_rows<BF, MB, TPW, true>(p, acc, scales, mine, m0, nt_base * 16, lane);
             else                     store_rows<BF, MB, TPW, false>(p, acc, scales, mine, m0, nt_base * 16, lane);
             return;
@@ -489,6 +487,34 @@ __global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOL
             if constexpr (BF) store_bf16(p, acc[t][mb] * sc, m, n0);
             else              gemm_store(p, acc[t][mb] * sc, m, n0, 0);
         }
+    }
+}
+
+template <int WBITS, int GS, bool BF, int MB, int TPW, int KS, bool WHOLE>
+__global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, KS, WHOLE)) void gemm_prefill_kernel(const GemmParams p, const int band) {
+    __shared__ u32x4 xs[KS * 512 * MB];
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (band) prefill_tile(by * (int)gridDim.x + bx, gridDim.y, gridDim.x, band, bx, by);
+    prefill_block<WBITS, GS, BF, MB, TPW, KS, WHOLE>(p, xs, by * 16 * MB, bx * (8 / KS * TPW));
+}
+// Two shapes in one launch (pick_rest): blocks of 16 MB rows for the first `cols` column tiles, whole rounds of them over the chip, and smaller ones for the columns behind.  Blocks start in order, so
+// the small ones run where the large ones are done first.  In a launch of their own they waited for the last of them: fp16 W4 at 4096 rows, us one shape / two launches / one, the same bits:
+// 37888 x 3584 gated 902 / 885 / 868, 4608 x 3584 138 / 126 / 114.
+template <int WBITS, int GS, bool BF, int MB, int TPW, int MB2, int TPW2>
+__global__ __launch_bounds__(512, prefill_waves(WBITS, GS, BF, MB, TPW, 1, true)) void gemm_prefill_rest_kernel(const GemmParams p, const int cols, const int band, const int band2) {
+    static_assert(MB2 <= MB && TPW2 <= TPW, "the rest's blocks are smaller");
+    __shared__ u32x4 xs[512 * MB];
+    const int rows = (p.M + 16 * MB - 1) / (16 * MB), n = rows * cols, id = blockIdx.x;
+    int bx, by;
+    if (id < n) {
+        bx = id % cols; by = id / cols;
+        if (band) prefill_tile(id, rows, cols, band, bx, by);
+        prefill_block<WBITS, GS, BF, MB, TPW, 1, true>(p, xs, by * 16 * MB, bx * 8 * TPW);
+    } else {
+        const int rows2 = (p.M + 16 * MB2 - 1) / (16 * MB2), cols2 = (p.NT - cols * 8 * TPW + 8 * TPW2 - 1) / (8 * TPW2);
+        bx = (id - n) % cols2; by = (id - n) / cols2;
+        if (band2) prefill_tile(id - n, rows2, cols2, band2, bx, by);
+        prefill_block<WBITS, GS, BF, MB2, TPW2, 1, true>(p, xs, by * 16 * MB2, (cols * TPW + bx * TPW2) * 8);
     }
 }
 
@@ -551,6 +577,14 @@ PrefillShare prefill_share(const PrefillShape& s, int M, int NT) {
     const double full = (double)cdiv(NT, 8 / s.ks * s.tpw) * cdiv(M, 16 * s.mb) / 256.0, whole = (double)(long)(full + 0.9999);
     return {0.5 * (full + whole), whole <= 1.0};
 }
+const UnslicedCost* unsliced_cost(bool bf, int wbits, int group_size, bool whole) {
+    return kUnslicedCost[wbits == 16 ? 8 : wbits == 8 ? (bf ? 7 : 6) : (bf ? 3 : 0) + (group_size == 128 ? 0 : group_size == 64 ? 1 : 2)][whole];
+}
+double unsliced_us(const UnslicedCost* own, int i, int M, int NT, int KC) {
+    const PrefillShare sh = prefill_share(kPrefillShapes[i], M, NT);
+    const double share = sh.round ? 0.0 : own[i].sat * sh.share;
+    return own[i].base + KC * (share > own[i].lat ? share : own[i].lat);
+}
 int pick_shape(int M, int NT, int KC, bool bf, int wbits, int group_size, bool whole, double* t_best) {
     const int first = (bf || wbits == 16) ? 1 : 0;
     const PrefillCost* cost = kPrefillCost[wbits == 16 ? 2 : (bf && wbits == 4) ? 1 : 0];
@@ -562,14 +596,39 @@ int pick_shape(int M, int NT, int KC, bool bf, int wbits, int group_size, bool w
         if (t < *t_best) { *t_best = t; best = i; }
     }
     if (best >= kWholeShapes) return best;
-    const UnslicedCost* own = kUnslicedCost[wbits == 16 ? 8 : wbits == 8 ? (bf ? 7 : 6) : (bf ? 3 : 0) + (group_size == 128 ? 0 : group_size == 64 ? 1 : 2)][whole];
+    const UnslicedCost* own = unsliced_cost(bf, wbits, group_size, whole);
     double least = 1e30;
     for (int i = first; i < kWholeShapes; ++i) {
-        const PrefillShare sh = prefill_share(kPrefillShapes[i], M, NT);
-        const double share = sh.round ? 0.0 : own[i].sat * sh.share, t = own[i].base + KC * (share > own[i].lat ? share : own[i].lat);
+        const double t = unsliced_us(own, i, M, NT, KC);
         if (t < least) { least = t; best = i; }
     }
     return best;
+}
+// Two shapes in one launch: a last round of blocks that is nearly empty costs most of a full one (37888 x 3584 at 4096 rows has 9.25 rounds of 128 x 512).  The first shape takes the columns that fill
+// whole rounds, a smaller one, a block to a CU like it, the rest, where the model expects 2.5 % of it.  Of codes (4 bits: groups of 128), where K is not sliced and runs the loop without branches.
+// 660 random calls (130 to 135 a class) that could: mean share of the time with one shape, over all of them, fp16 W4 0.971 (best choice of each 0.956), fp16 8 bits 0.972 (0.962), bf16 W4 0.982 (0.974), bf16 8
+// bits 0.973 (0.967); 11 above 1.02, at worst 1.05.  16-bit weights 0.996, at worst 1.17: one shape.  us one shape / two: fp16 W4 37888 x 3584 gated at 4096 rows 902 / 868 (128 x 512 and 64 x 256),
+// 2667 625 / 577 (and 64 x 128), 1825 442 / 415 (and 128 x 256), 4608 x 3584 at 4096 138 / 114; fp16 8 bits the same at 4096 845 / 822 and 123 / 105; bf16 W4 4608 x 3584 at 4096 161 / 137
+// (128 x 256 and 64 x 128), 37888 x 3584 at 1055 331 / 306.
+struct PrefillRest { int shape, rest, cols; };               // cols 0: one shape
+PrefillRest pick_rest(int best, int M, int NT, int KC, bool bf, int wbits, int group_size, bool whole) {
+    PrefillRest pick{best, 0, 0};
+    if (!whole || best >= kWholeShapes || wbits == 16 || (wbits == 4 && group_size != 128)) return pick;
+    const UnslicedCost* own = unsliced_cost(bf, wbits, group_size, true);
+    double least = 0.975 * unsliced_us(own, best, M, NT, KC);
+    for (int i = bf ? 1 : 0; i < 2; ++i) {
+        const int rows = cdiv(M, 128), tiles = 8 * kPrefillShapes[i].tpw, rounds = rows * cdiv(NT, tiles) / 256, cols = rounds * 256 / rows;
+        if (cols == 0 || cols * tiles >= NT) continue;
+        for (int r = i == 0 ? 1 : 3; r < kWholeShapes; ++r) {
+            const int blocks = cdiv(M, 16 * kPrefillShapes[r].mb) * cdiv(NT - cols * tiles, 8 * kPrefillShapes[r].tpw);
+            // a full round takes what the chip's throughput asks for, the last as much less as it is empty, at least 0.8 of a block alone
+            const int n = cdiv(blocks, 256);
+            const double full = own[r].lat > own[r].sat ? own[r].lat : own[r].sat, alone = 0.8 * own[r].lat;
+            const double t = own[i].base + KC * own[i].sat * rows * cols / 256.0 + n + KC * ((n - 1) * full + alone + (full - alone) * (blocks / 256.0 - (n - 1)));
+            if (t < least) { least = t; pick = {i, r, cols}; }
+        }
+    }
+    return pick;
 }
 // K below 2^23: the 128 x 512 form's row offsets are formed past the last row, in 32 bits.
 bool prefill_whole(const void* x, int K) { return (uintptr_t)x % 16 == 0 && K % 128 == 0 && K < 1 << 23; }
@@ -587,9 +646,29 @@ void launch_shape_t(const GemmParams& p, hipStream_t st) {
     }
     hipLaunchKernelGGL((gemm_prefill_kernel<WBITS, GS, BF, s.mb, s.tpw, s.ks, false>), grid, dim3(512), 0, st, p, band);
 }
+template <int WBITS, int GS, bool BF, int I, int J>
+void launch_rest_t(int cols, const GemmParams& p, hipStream_t st) {
+    constexpr PrefillShape s = kPrefillShapes[I], r = kPrefillShapes[J];
+    const int rows = cdiv(p.M, 16 * s.mb), rows2 = cdiv(p.M, 16 * r.mb), cols2 = cdiv(p.NT - cols * 8 * s.tpw, 8 * r.tpw);
+    hipLaunchKernelGGL((gemm_prefill_rest_kernel<WBITS, GS, BF, s.mb, s.tpw, r.mb, r.tpw>), dim3(rows * cols + rows2 * cols2), dim3(512), 0, st, p, cols,
+                       prefill_short(p, WBITS, s.tpw * 128) ? 0 : prefill_band(rows, cols), prefill_short(p, WBITS, r.tpw * 128) ? 0 : prefill_band(rows2, cols2));
+}
 template <int WBITS, int GS, bool BF>
-int launch_shape(int i, const GemmParams& p, hipStream_t st) {
-    switch (i) {
+int launch_shape(const PrefillRest& pick, const GemmParams& p, hipStream_t st) {
+    if constexpr (WBITS == 8 || (WBITS == 4 && GS == 4)) {
+        if (pick.cols) {
+            switch (pick.shape * 4 + pick.rest) {
+                case 1: if constexpr (!BF) { launch_rest_t<WBITS, GS, BF, 0, 1>(pick.cols, p, st); break; } return MI355_ERR_UNSUPPORTED;
+                case 2: if constexpr (!BF) { launch_rest_t<WBITS, GS, BF, 0, 2>(pick.cols, p, st); break; } return MI355_ERR_UNSUPPORTED;
+                case 3: if constexpr (!BF) { launch_rest_t<WBITS, GS, BF, 0, 3>(pick.cols, p, st); break; } return MI355_ERR_UNSUPPORTED;
+                case 7: launch_rest_t<WBITS, GS, BF, 1, 3>(pick.cols, p, st); break;
+                default: return MI355_ERR_UNSUPPORTED;
+            }
+            MI355_CHECK_LAUNCH("gemm_prefill_rest_kernel");
+            return MI355_OK;
+        }
+    }
+    switch (pick.shape) {
         case 0: if constexpr (!BF && WBITS != 16) { launch_shape_t<WBITS, GS, BF, 0>(p, st); break; } return MI355_ERR_UNSUPPORTED;
         case 1: launch_shape_t<WBITS, GS, BF, 1>(p, st); break;
         case 2: launch_shape_t<WBITS, GS, BF, 2>(p, st); break;
@@ -623,6 +702,14 @@ extern "C" int mi355_gemm_prefill_form(int32_t M, int32_t NT, int32_t KC, int32_
     return s + (whole && prefill_straight(s, wbits, group_size / 32, bf16 != 0) ? 16 : 0);
 }
 
+// Whether such a call runs two shapes in one launch: 0, or the first shape's place + 4 times the rest's + 16 times the first's column tiles.
+extern "C" int mi355_gemm_prefill_rest(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits, int32_t group_size, int32_t whole) {
+    double t;
+    const int s = pick_shape(M, NT, KC, bf16 != 0, wbits, group_size, whole != 0, &t);
+    const PrefillRest r = pick_rest(s, M, NT, KC, bf16 != 0, wbits, group_size, whole != 0);
+    return r.cols ? r.shape + 4 * r.rest + 16 * r.cols : 0;
+}
+
 // Direct-mode launch (fused epilogue in p.mode).  MI355_ERR_UNSUPPORTED: shape / format not covered, caller falls back.
 // t_limit: the caller's estimate (us) for its other path; a launch expected to take longer is not made (MI355_ERR_UNSUPPORTED).
 extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, double t_limit, mi355_stream_t stream) {
@@ -632,8 +719,10 @@ extern "C" int mi355_gemm_prefill(const void* gp, int wbits, int group_size, dou
     hipStream_t st = (hipStream_t)stream;
     const bool bf = g.bf16 != 0;
     double t;
-    const int s = pick_shape(g.M, g.NT, g.KC, bf, wbits, group_size, prefill_whole(g.x, g.K), &t);
+    const bool whole = prefill_whole(g.x, g.K);
+    const int one = pick_shape(g.M, g.NT, g.KC, bf, wbits, group_size, whole, &t);
     if (t > t_limit) return MI355_ERR_UNSUPPORTED;
+    const PrefillRest s = pick_rest(one, g.M, g.NT, g.KC, bf, wbits, group_size, whole);
     if (wbits == 16) return bf ? launch_shape<16, 0, true>(s, g, st) : launch_shape<16, 0, false>(s, g, st);
     if (wbits == 8 && group_size == 0) return bf ? launch_shape<8, 0, true>(s, g, st) : launch_shape<8, 0, false>(s, g, st);
     if (wbits == 4) {
