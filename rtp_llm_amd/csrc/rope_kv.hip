@@ -128,6 +128,86 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(const RopeParams p) 
     }
 }
 
+// The same for the rows of prompts (16-bit tensors and cache): a block takes 16 rows of 4 query or key heads, a thread 8 pairs of a row at a time in 16-byte loads and stores, or 16 rows of a value head,
+// whose columns lie token by token in a page: through LDS, so that a store's lanes are 16 tokens of a column.  By a wave per row and head a value went out as 64 lines of 2 bytes, and the lines of
+// consecutive rows from eight L2s.  us by waves / here: 28 over 4 heads of 128, 4096 rows 31.7 / 15.9
+// (4.7 TB/s), 1055 10.5 / 6.6, 265 4.5 / 4.2; 14 over 2 of 64, 4096 15.7 / 6.1, 512 4.1 / 3.2; 32 over 32 of 64, 1055 25.8 / 8.6, 64 3.8 / 3.0.
+constexpr int RP_ROWS = 16, RP_HEADS = 4;
+template <bool BF, int HD>
+__global__ __launch_bounds__(256) void rope_kv_prompt_kernel(const RopeParams p) {
+    constexpr int half = HD / 2, P = half / 8, LD = HD + 2;                  // 16-byte pieces of a half, a row of values in LDS
+    __shared__ uint32_t vs[RP_ROWS * LD / 2];
+    const int t0 = blockIdx.x * RP_ROWS, nrot = p.nh + p.nkv, chunks = (nrot + RP_HEADS - 1) / RP_HEADS;
+    const int pos_lim = min(p.max_pos, p.max_blocks * p.page);
+    const uint16_t* qkv = reinterpret_cast<const uint16_t*>(p.qkv);
+    const uint16_t* bias = reinterpret_cast<const uint16_t*>(p.bias);
+    auto load8 = [&](int t, int col, float (&x)[8]) {                        // a row's 8 columns with their bias, rounded
+        const u32x4 v = *reinterpret_cast<const u32x4*>(qkv + (size_t)t * p.ld + col);
+        u32x4 b = {0, 0, 0, 0};
+        if (bias) b = *reinterpret_cast<const u32x4*>(bias + col);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { x[2 * i] = act_round<BF>(act_lo<BF>(v[i]) + act_lo<BF>(b[i])); x[2 * i + 1] = act_round<BF>(act_hi<BF>(v[i]) + act_hi<BF>(b[i])); }
+    };
+    auto place = [&](int t, int pos_in, int pos, size_t heads, uint16_t*& dst, int& tok) -> int {     // the page of a row (heads: units of heads behind a block's first): 0 none, -1 out of range
+        if (pos_in < 0) return 0;
+        const int blk = p.block_table[(size_t)(p.row_seq ? p.row_seq[t] : t / p.q_len) * p.max_blocks + pos / p.page];
+        if (pos != pos_in || blk < 0 || blk >= p.num_blocks) return -1;
+        tok = pos % p.page;
+        dst = (uint16_t*)p.kv_base + ((size_t)blk * 2 * p.nkv + heads) * p.page * HD;
+        return 1;
+    };
+    if ((int)blockIdx.y < chunks) {
+#pragma unroll
+        for (int i = 0; i < RP_ROWS * RP_HEADS * P / 256; ++i) {
+            const int item = i * 256 + (int)threadIdx.x, c = item % P * 8, h = blockIdx.y * RP_HEADS + item / P % RP_HEADS, t = t0 + item / (P * RP_HEADS);
+            if (h >= nrot || t >= p.T) continue;
+            const int pos_in = p.positions[t], pos = min(max(pos_in, 0), pos_lim - 1);
+            float x0[8], x1[8];
+            load8(t, h * HD + c, x0); load8(t, h * HD + half + c, x1);
+            const float4* rot = reinterpret_cast<const float4*>(p.cos_sin + ((size_t)pos * half + c) * 2);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float4 cs = rot[k];
+                const float a0 = x0[2 * k], b0 = x1[2 * k], a1 = x0[2 * k + 1], b1 = x1[2 * k + 1];
+                x0[2 * k] = cs.x * a0 - cs.y * b0; x1[2 * k] = cs.x * b0 + cs.y * a0;
+                x0[2 * k + 1] = cs.z * a1 - cs.w * b1; x1[2 * k + 1] = cs.z * b1 + cs.w * a1;
+            }
+            u32x4 y0, y1;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { y0[k] = act_pack<BF>(x0[2 * k], x0[2 * k + 1]); y1[k] = act_pack<BF>(x1[2 * k], x1[2 * k + 1]); }
+            uint16_t* dst;
+            if (h < p.nh) dst = reinterpret_cast<uint16_t*>(p.q_out) + ((size_t)t * p.nh + h) * HD + c;
+            else {
+                int tok = 0;
+                const int at = place(t, pos_in, pos, h - p.nh, dst, tok);
+                if (at < 0 && h == p.nh && c == 0 && p.oob_count) atomicAdd(p.oob_count, 1);
+                if (at <= 0) continue;
+                dst += tok * HD + c;
+            }
+            *reinterpret_cast<u32x4*>(dst) = y0;
+            *reinterpret_cast<u32x4*>(dst + half) = y1;
+        }
+        return;
+    }
+    const int kh = (int)blockIdx.y - chunks;
+    for (int item = threadIdx.x; item < RP_ROWS * HD / 8; item += 256) {
+        const int r = item / (HD / 8), c = item % (HD / 8) * 8;
+        if (t0 + r >= p.T) continue;
+        float x[8];
+        load8(t0 + r, (nrot + kh) * HD + c, x);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) vs[(r * LD + c) / 2 + k] = act_pack<BF>(x[2 * k], x[2 * k + 1]);
+    }
+    __syncthreads();
+    const int r = threadIdx.x % RP_ROWS, t = t0 + r;
+    if (t >= p.T) return;
+    const int pos_in = p.positions[t];
+    uint16_t* dst;
+    int tok = 0;
+    if (place(t, pos_in, min(max(pos_in, 0), pos_lim - 1), p.nkv + kh, dst, tok) <= 0) return;
+    for (int d = threadIdx.x / RP_ROWS; d < HD; d += 256 / RP_ROWS) dst[(size_t)d * p.page + tok] = reinterpret_cast<const uint16_t*>(vs)[r * LD + d];
+}
+
 } // namespace
 
 extern "C" int mi355_rope_kv_write(const void* qkv_f16, const float* partials, int32_t nsplit, int32_t ld,
@@ -174,6 +254,19 @@ extern "C" int mi355_rope_kv_write_rows_ragged(const void* qkv_f16, const float*
     p.T = T; p.nh = nh; p.nkv = kv->nkv; p.hd = kv->hd; p.page = kv->page; p.kv_base = kv->kv_base;
     p.max_pos = max_pos; p.num_blocks = kv->num_blocks; p.oob_count = oob_count; p.q_len = q_len; p.row_seq = row_seq;
     p.scale_base = kv->scale_base; p.kv_int8 = kv->kv_dtype == MI355_KV_INT8; p.q_out = (f16*)q_out;
+    const uintptr_t at = (uintptr_t)qkv_f16 | (uintptr_t)qkv_bias | (uintptr_t)cos_sin | (uintptr_t)q_out | (uintptr_t)kv->kv_base;
+    // Few waves: a block's two trips of 16 bytes a thread take longer than one wave's single one.  28 over 4 heads of 128, us by waves / by blocks: 64 rows 3.2 / 3.9, 192 3.9 / 4.1, 265 4.5 / 4.2; 5 over 1, 512
+    // rows 3.4 / 4.4, 1055 4.4 / 4.3.  Heads of 64 (one trip): 64 rows 2.9 / 2.9, 192 3.2 / 3.2.
+    if (T >= 64 && (kv->hd == 64 || (long)T * nheads >= 7400) && qkv_f16 && !p.kv_int8 && at % 16 == 0 && ld % 8 == 0) {
+        const dim3 grid(cdiv(T, RP_ROWS), cdiv(nh + kv->nkv, RP_HEADS) + kv->nkv);
+        hipStream_t st = (hipStream_t)stream;
+        if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((rope_kv_prompt_kernel<true, 128>), grid, dim3(256), 0, st, p);
+                             else    hipLaunchKernelGGL((rope_kv_prompt_kernel<false, 128>), grid, dim3(256), 0, st, p); }
+        else               { if (bf) hipLaunchKernelGGL((rope_kv_prompt_kernel<true, 64>), grid, dim3(256), 0, st, p);
+                             else    hipLaunchKernelGGL((rope_kv_prompt_kernel<false, 64>), grid, dim3(256), 0, st, p); }
+        MI355_CHECK_LAUNCH("rope_kv_prompt_kernel");
+        return MI355_OK;
+    }
     if (bf)
         hipLaunchKernelGGL(rope_kv_write_kernel<true>, dim3(T, cdiv(nheads, 4)), dim3(256), 0, (hipStream_t)stream, p);
     else
