@@ -645,7 +645,9 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
 // step.  Products transposed as there (a lane owns one row: its maximum, sum and rescaling are its own; the weights are the second product's operand where they
 // are: the keys of a step are handed to the first product in an order that leaves every lane eight consecutive ones).  16-byte pieces of a key row are swizzled by the
 // key, a value row (one channel, 32 tokens) is 64 bytes and needs none.
-// 8 x 512 rows, 28 over 4 heads of 128: 169 -> 79 us; 3 of 389: 51 -> 30.
+// Blocks are dealt late rows first over all sequences and key/value heads: the longest start together, and as consecutive blocks go to the eight XCDs in turn, the row tiles of one sequence and head,
+// as many blocks apart as there are such pairs, meet in one L2 where eight divides that number.  Row tiles first (every XCD reads every pair's keys, the last pairs' long rows start late) / so, us: 28
+// over 4 heads of 128, 8 x 512 rows 77 / 50 (by 4 rows a block 169), 3 of 300 to 389 25.8 / 23.6, 1500 91 / 71, 2 x 2048 behind 2048 449 / 361; 32 over 8, 4096 rows 357 / 248.
 // What bounds it: a step of one wave, about 1.4 us of product, softmax and product in series whatever the depth of the staging (3 to 6 stages measured the same).
 constexpr int PR_STAGES = 3;
 template <int HD, bool BF>
@@ -657,10 +659,10 @@ __global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p,
     const int NW = HW * TW, JT = (LOADS + NW - 1) / NW, stage = JT * NW * 1024;
     int* klim_s = reinterpret_cast<int*>(pr_sm + NS * stage);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lq = lane >> 4;
-    const int b = blockIdx.z, h = blockIdx.y * HW + wave % HW, kh = (int)blockIdx.y * HW / p.G;
+    const int b = blockIdx.y, h = blockIdx.x * HW + wave % HW, kh = (int)blockIdx.x * HW / p.G;
     int base = b * p.q_len, len = p.q_len;
     if (p.row_start) { base = p.row_start[b]; len = p.row_start[b + 1] - base; }
-    const int t0r = ((int)gridDim.x - 1 - (int)blockIdx.x) * TW * 16;                // late (long) rows first
+    const int t0r = ((int)gridDim.z - 1 - (int)blockIdx.z) * TW * 16;                // late (long) rows first
     if (t0r >= len) return;
     const int r0 = t0r + wave / HW * 16, n = min(16, len - r0);                       // n <= 0: a wave without rows
     const int row = base + min(max(r0 + lr, 0), len - 1);
@@ -928,11 +930,11 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     while (p.G % HW) --HW;                                  // heads of a key/value head per block
     const int TW = 8 / HW, NW = HW * TW, JT = (kv->hd / 8 + NW - 1) / NW;
     // Prompt rows: where the rows fill the waves of about as many blocks as the chip has compute units (a third more where heads share no keys: a block then holds 128 rows of one
-    // head); with fewer the other kernel's smaller row tiles and split contexts win.  us there / here: 28 over 4 heads of 128, 8 x 512 rows 169 / 79, 3 x 352 72 / 52, 1 x 1500 108 /
+    // head); with fewer the other kernel's smaller row tiles and split contexts win.  us there / here (row tiles first): 28 over 4 heads of 128, 8 x 512 rows 169 / 79, 3 x 352 72 / 52, 1 x 1500 108 /
     // 92, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100, 37 x 20 behind 3477 188 / 250; 16 over 16 heads of 64, 16 x 34 behind 3628 75 / 117; 32 over 32 of 128, 38 x 23 behind
     // 3378 409 / 603.  Over 300 random calls the pick is 1.7 x faster than the other kernel, 3 of them slower (by up to a fifth, at contexts of thousands).
     if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)p.rows * nh >= 16L * NW * (HW == 1 ? 310 : 240) && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
-        const dim3 grid(cdiv(q_len, 16 * TW), nh / HW, B);
+        const dim3 grid(nh / HW, B, cdiv(q_len, 16 * TW));
         const size_t lds = (size_t)PR_STAGES * JT * NW * 1024 + 16;
         hipStream_t st = (hipStream_t)stream;
         if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW);
