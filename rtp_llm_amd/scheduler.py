@@ -107,8 +107,9 @@ class ServingEngine:
         offs = [0]
         for part in parts:
             offs.append(offs[-1] + (len(part) + 3) // 4 * 4)      # 16-byte aligned fields
-        host = torch.zeros(offs[-1], dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        host = torch.empty(offs[-1], dtype=torch.int32, pin_memory=self.device.type == "cuda")
         view = host.numpy()
+        view[:] = 0                                               # zeros() of 2^15 numbers wakes all threads of the host, milliseconds now and then
         for o, part in zip(offs, parts):
             view[o:o + len(part)] = part
         batch = self.batch_views(host.to(self.device, non_blocking=True), [len(part) for part in parts], nseq, width)
