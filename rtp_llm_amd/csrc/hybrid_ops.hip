@@ -885,7 +885,7 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
                                                                            int HW, int same, int vec, int KG, int heads_first) {
     extern __shared__ __attribute__((aligned(16))) char at_smem[];
     const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6 & 3), lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
-    const int TW = 4 / HW, set = heads_first ? blockIdx.x : blockIdx.y, h = set * HW + wave % HW, tw = wave / HW;
+    const int TW = 4 / HW, set = DK <= 4 && heads_first ? blockIdx.x : blockIdx.y, h = set * HW + wave % HW, tw = wave / HW;
     const int kvh = set * HW / (g.H / g.G);
     const int NCB = g.vdim / 16;
     // pieces of 16 bytes in a key row, of a value row; DMA loads per wave and step; swizzle: piece c of key k lies at c ^ (k & mask)
@@ -896,10 +896,10 @@ __global__ __launch_bounds__(256 * at_groups(DK, NCBM), DK <= 4 && NCBM <= 8 ? 3
     int32_t* bt_s = (int32_t*)(at_smem + KG * AT_STAGES * stage);
     char* at_sm = at_smem + group * AT_STAGES * stage;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)at_sm;
-    // Long (late) tiles of a prompt first.  Of several key/value heads the heads are dealt before the tiles: consecutive blocks go to the eight XCDs in turn, so a head's tiles share one or a few L2s, and
+    // Long (late) tiles of a prompt first.  Of several key/value heads of up to 128 channels (wider ones, mostly one latent row, keep their code: the choice alone took 2 % there) the heads are dealt before the tiles: consecutive blocks go to the eight XCDs in turn, so a head's tiles share one or a few L2s, and
     // the blocks at work at one time read one sequence.  us tiles first / heads first: 16 over 4 heads of 128, 4 x 2048 rows 234 / 182, 2048 100 / 87, 8192 645 / 579, 64 x 128 49.9 / 45.7, 2 x 4096 in
     // a window of 512 108 / 101; 32 over 8, 1000, 300 and 1700 rows 161 / 118; 16 over 16 of 128, 4 x 2048 306 / 188; of 64, 2 x 4096 362 / 228, 4 x 1024 63.6 / 65.2.
-    const int first_tile = (heads_first ? (int)gridDim.y - 1 - (int)blockIdx.y : (int)gridDim.x - 1 - (int)blockIdx.x) * TW, ntw = min(TW, ntiles - first_tile);
+    const int first_tile = (DK <= 4 && heads_first ? (int)gridDim.y - 1 - (int)blockIdx.y : (int)gridDim.x - 1 - (int)blockIdx.x) * TW, ntw = min(TW, ntiles - first_tile);
     bool has = tw < ntw;
     const int tile = first_tile + min(tw, ntw - 1), r0 = __builtin_amdgcn_readfirstlane(tile_row0[tile]), n = __builtin_amdgcn_readfirstlane(tile_n[tile]);
     const int p0 = __builtin_amdgcn_readfirstlane(pos[r0]), plast = p0 + n - 1;
@@ -2995,7 +2995,7 @@ extern "C" int mi355_hy_attn_tiles_ex3(const float* q, int32_t ldq, float scale,
     const int same = kcache == vcache && g.v_ld == g.dim && g.vdim <= g.dim;    // the value is a part of the staged key row
     const int vec = ((uintptr_t)q % 16 == 0 && ldq % 4 == 0 ? 1 : 0) | (((uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 ? 2 : 0) | ((uintptr_t)out % 8 == 0 ? 4 : 0);
     const int staged = AT_STAGES * 4096 * ((g.dim / 8 + 7) / 8 + (same ? 0 : (g.vdim / 8 + 7) / 8)), turned = vfreq ? 4 * 16 * (g.vdim + 4) * 4 : 0;
-    const int blocks = (tiles + 4 / HW - 1) / (4 / HW), heads_first = g.G > 1 && blocks <= 65535;
+    const int blocks = (tiles + 4 / HW - 1) / (4 / HW), heads_first = g.G > 1 && g.dim <= 128 && blocks <= 65535;
     const dim3 grid = heads_first ? dim3(g.H / HW, blocks) : dim3(blocks, g.H / HW);
     // Two groups of waves walk the keys of a block where the grid leaves them compute units: us with one / two, 8 heads over a latent row of 256 (192) 64 rows 10.3 / 11.9, 131 14.4 / 14.5,
     // 256 18.7 / 17.5, 512 30.2 / 24.8, 1024 52.4 / 39.4, 1537 76.5 / 55.3, 2048 (256 blocks) 99.5 / 71.2, 2 x 2048 (512) 127.2 / 127.5; 16 over 4 heads of 128 131 rows 12.5 / 11.5,
