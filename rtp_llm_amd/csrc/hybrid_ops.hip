@@ -2201,7 +2201,7 @@ __global__ __launch_bounds__(1024) void hy_head_norm_kernel(const float* o, int 
 
 
 // The same, with the same sums, for heads of up to 4 G channels: lane l of G has channels l + G e of one head, all loads at once: one trip to memory and several heads a block.
-// 8192 rows of 16 heads of 128 with gate: 77.3 -> 44.6 us (36.4 with four adjacent channels a lane, whose sums differ).
+// 8192 rows of 16 heads of 128 with gate: 77.3 -> 44.6 us.
 template <typename T, int G>
 __global__ __launch_bounds__(256) void hy_head_norm4_kernel(const float* o, int ldo, int H, int vdim, const T* w, float eps, const float* gate, int ldg, int goff, T* out,
                                                             int w_heads, int gate_sigmoid, const float* den, int heads) {
@@ -2238,6 +2238,47 @@ __global__ __launch_bounds__(256) void hy_head_norm4_kernel(const float* o, int 
         if (gate) y *= gate_sigmoid ? hy_sigmoid(gz[e]) : hy_silu(gz[e]);
         if (c < vdim) out[(size_t)i * vdim + c] = (T)y;
     }
+}
+
+// Heads of 128 channels: lane L of 32 has four adjacent ones, 16 bytes a load, and the sums of the kernel above all the same.  There lane l adds the squares of channels l, l + 32, l + 64 and l + 96,
+// which lie here in the lanes 8, 16 and 24 apart; each of those four takes one of the four l they share from there on, through the tree over l: bits 16, 8 and 4 of l are bits 4, 2 and 1 of L, and its
+// bits 2 and 1 the four lanes again.  us with gate, 4-byte / 16-byte pieces: 8192 rows of 16 heads 42.0 / 36.9 (4.5 TB/s), 456 rows 4.9 / 4.5, 1537 of 8 heads 6.0 / 5.4.
+template <typename T>
+__global__ __launch_bounds__(256) void hy_head_norm128_kernel(const float* o, int ldo, int H, const T* w, float eps, const float* gate, int ldg, int goff, T* out, int w_heads, int gate_sigmoid,
+                                                              const float* den, int heads) {
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const int i = blockIdx.x * 8 + threadIdx.x / 32, L = threadIdx.x % 32, c = L * 4;
+    if (i >= heads) return;                             // whole groups of 32 lanes
+    const int r = i / H, h = i - r * H;
+    f32x4 v = *(const f32x4*)(o + (size_t)r * ldo + (size_t)h * 128 + c), gz = {0.f, 0.f, 0.f, 0.f};
+    T4 wv = {(T)1.f, (T)1.f, (T)1.f, (T)1.f};
+    if (gate) gz = *(const f32x4*)(gate + (size_t)r * ldg + goff + h * 128 + c);
+    if (w) wv = *(const T4*)(w + (w_heads ? h * 128 + c : c));
+    if (den) v *= 1.f / den[i];
+    const bool low = L < 16, odd = L & 8;
+    float t[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const float own = low ? v[e] : v[2 + e], far = __shfl_xor(low ? v[2 + e] : v[e], 16, 32);      // the lane 16 apart has the other two values of the pair
+        const float first = low ? own : far, second = low ? far : own;
+        t[e] = __builtin_fmaf(second, second, first * first);
+    }
+    float ss = odd ? t[1] : t[0];
+    ss += __shfl_xor(odd ? t[0] : t[1], 8, 32);
+#pragma unroll
+    for (int m = 4; m; m >>= 1) ss += __shfl_xor(ss, m, 32);
+    ss += __shfl_xor(ss, 16, 32);
+    ss += __shfl_xor(ss, 8, 32);
+    const float inv = 1.f / sqrtf(ss / 128.f + eps);
+    T4 y4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float y = v[e] * inv;
+        if (w) y *= (float)wv[e];
+        if (gate) y *= gate_sigmoid ? hy_sigmoid(gz[e]) : hy_silu(gz[e]);
+        y4[e] = (T)y;
+    }
+    *(T4*)(out + (size_t)i * 128 + c) = y4;
 }
 
 // ------------------------------------------------------------------------------------------------ recurrences of a few rows: gates, update, output, norm and output gate in one launch
@@ -3271,7 +3312,15 @@ extern "C" int mi355_hy_head_norm_ex3(const float* o, int32_t ldo, int32_t rows,
     // Us of a wave each / several a block, with gate: 128 heads of 64 2.6 / 3.4, 2048 2.9 / 3.5, 4096 3.5 / 3.5, 8192 4.6 / 3.9; 128 heads of 128 3.1 / 3.6,
     // 2048 3.5 / 3.6, 4096 4.1 / 3.9, 32768 18.4 / 11.4; 16 heads of 192 3.6 / 3.0.
     if (vdim <= 256 && (int64_t)rows * H <= INT32_MAX - 256 && (vdim > 128 || rows * H >= 4096)) {
-        const int n = rows * H, G = vdim <= 32 ? 8 : vdim <= 64 ? 16 : vdim <= 128 ? 32 : 64;
+        const int n = rows * H;
+        const uintptr_t at = (uintptr_t)o | (uintptr_t)gate | (uintptr_t)w | (uintptr_t)out;
+        if (vdim == 128 && at % 16 == 0 && ldo % 4 == 0 && (!gate || (ldg % 4 == 0 && goff % 4 == 0))) {
+            HY_DISPATCH(act_dtype, hipLaunchKernelGGL(hy_head_norm128_kernel<T>, dim3((n + 7) / 8), dim3(256), 0, (hipStream_t)stream, o, ldo, H, (const T*)w, eps, gate, ldg, goff, (T*)out, w_heads,
+                                                      gate_sigmoid, den, n));
+            MI355_CHECK_LAUNCH("hy_head_norm128_kernel");
+            return MI355_OK;
+        }
+        const int G = vdim <= 32 ? 8 : vdim <= 64 ? 16 : vdim <= 128 ? 32 : 64;
 #define HY_HEAD_NORM4(G_) HY_DISPATCH(act_dtype, hipLaunchKernelGGL((hy_head_norm4_kernel<T, G_>), dim3((n + 256 / G_ - 1) / (256 / G_)), dim3(256), 0, (hipStream_t)stream, o, ldo, H, \
                                       vdim, (const T*)w, eps, gate, ldg, goff, (T*)out, w_heads, gate_sigmoid, den, n))
         if (G == 8) HY_HEAD_NORM4(8); else if (G == 16) HY_HEAD_NORM4(16); else if (G == 32) HY_HEAD_NORM4(32); else HY_HEAD_NORM4(64);
