@@ -651,7 +651,7 @@ __global__ __launch_bounds__(64 * NW) void paged_attn_kernel(const AttnParams p)
 // What bounds it: a step of one wave, about 1.4 us of product, softmax and product in series whatever the depth of the staging (3 to 6 stages measured the same).
 constexpr int PR_STAGES = 3;
 template <int HD, bool BF>
-__global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p, int HW, int TW) {
+__global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p, int HW, int TW, int tiles_last) {
     constexpr int NS = PR_STAGES;
     constexpr int NSTEP = HD / 32, NDB = HD / 16, KL = HD / 16, LOADS = 2 * KL;     // 1 KB loads of a key tile (32 rows), of a step
     constexpr int CK = HD / 8;
@@ -659,10 +659,10 @@ __global__ __launch_bounds__(512, 2) void prompt_attn_kernel(const AttnParams p,
     const int NW = HW * TW, JT = (LOADS + NW - 1) / NW, stage = JT * NW * 1024;
     int* klim_s = reinterpret_cast<int*>(pr_sm + NS * stage);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lq = lane >> 4;
-    const int b = blockIdx.y, h = blockIdx.x * HW + wave % HW, kh = (int)blockIdx.x * HW / p.G;
+    const int b = tiles_last ? blockIdx.y : blockIdx.z, set = tiles_last ? blockIdx.x : blockIdx.y, h = set * HW + wave % HW, kh = set * HW / p.G;
     int base = b * p.q_len, len = p.q_len;
     if (p.row_start) { base = p.row_start[b]; len = p.row_start[b + 1] - base; }
-    const int t0r = ((int)gridDim.z - 1 - (int)blockIdx.z) * TW * 16;                // late (long) rows first
+    const int t0r = (tiles_last ? (int)gridDim.z - 1 - (int)blockIdx.z : (int)gridDim.x - 1 - (int)blockIdx.x) * TW * 16;                // late (long) rows first
     if (t0r >= len) return;
     const int r0 = t0r + wave / HW * 16, n = min(16, len - r0);                       // n <= 0: a wave without rows
     const int row = base + min(max(r0 + lr, 0), len - 1);
@@ -934,13 +934,14 @@ int launch_attn(const void* q, const mi355_kv_layer_t* kv, const int32_t* block_
     // 92, 1 x 512 35 / 38, 64 rows behind 2048 tokens 32 / 100, 37 x 20 behind 3477 188 / 250; 16 over 16 heads of 64, 16 x 34 behind 3628 75 / 117; 32 over 32 of 128, 38 x 23 behind
     // 3378 409 / 603.  Over 300 random calls the pick is 1.7 x faster than the other kernel, 3 of them slower (by up to a fifth, at contexts of thousands).
     if (!int8 && img_mblk == 0 && q_len >= 16 && !done && (long)p.rows * nh >= 16L * NW * (HW == 1 ? 310 : 240) && ((uintptr_t)kv->kv_base | (uintptr_t)q) % 16 == 0) {
-        const dim3 grid(nh / HW, B, cdiv(q_len, 16 * TW));
+        const int tiles = cdiv(q_len, 16 * TW), tiles_last = tiles <= 65535;                     // a grid has no more along z
+        const dim3 grid = tiles_last ? dim3(nh / HW, B, tiles) : dim3(tiles, nh / HW, B);
         const size_t lds = (size_t)PR_STAGES * JT * NW * 1024 + 16;
         hipStream_t st = (hipStream_t)stream;
-        if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW);
-                             else          hipLaunchKernelGGL((prompt_attn_kernel<128, false>), grid, dim3(64 * NW), lds, st, p, HW, TW); }
-        else               { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<64, true>), grid, dim3(64 * NW), lds, st, p, HW, TW);
-                             else          hipLaunchKernelGGL((prompt_attn_kernel<64, false>), grid, dim3(64 * NW), lds, st, p, HW, TW); }
+        if (kv->hd == 128) { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<128, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, tiles_last);
+                             else          hipLaunchKernelGGL((prompt_attn_kernel<128, false>), grid, dim3(64 * NW), lds, st, p, HW, TW, tiles_last); }
+        else               { if (bf) hipLaunchKernelGGL((prompt_attn_kernel<64, true>), grid, dim3(64 * NW), lds, st, p, HW, TW, tiles_last);
+                             else          hipLaunchKernelGGL((prompt_attn_kernel<64, false>), grid, dim3(64 * NW), lds, st, p, HW, TW, tiles_last); }
         MI355_CHECK_LAUNCH("prompt_attn_kernel");
         return MI355_OK;
     }
