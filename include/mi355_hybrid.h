@@ -102,9 +102,6 @@ typedef struct {
     float       act_param;
 } mi355_dense_args_t;
 int mi355_dense_linear_pair(const mi355_dense_args_t* two, mi355_stream_t stream);
-/* x += mult * (the two linears' sum), x fp32 of row stride ldx, bf16 operands of the same M (more than 16) and N: one product over both K.  x, ldx, M, w, N and K of the arguments are read.
- * MI355_ERR_UNSUPPORTED: sizes that two launches are better for, K off 64, operands off 16 bytes. */
-int mi355_dense_joined(const mi355_dense_args_t* two, float* x, int32_t ldx, float mult, mi355_stream_t stream);
 /* mi355_hy_scan over a few rows and mi355_hy_head_norm_ex2 (weight, gate through silu) in one launch, a block per sequence and head.  mode, projections, state and gates as
  * there; with ao >= 0 the decay pre-activations of mode 1 are formed here: column hd is b2[hd] + sum over j < rank of w2[hd, j] (act type) times proj[:, ao + j] rounded to the
  * act type.  w null: unit RMS only; go < 0: no gate.  out [rows, H * vdim] of the act type.  MI355_ERR_UNSUPPORTED: a state off 16 bytes, and heads

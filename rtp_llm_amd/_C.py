@@ -227,7 +227,6 @@ HYBRID_SIGNATURES = {
     "mi355_hy_attn_prep_ex": (i32, [vp, i32, i32, i32, ip, vp, vp, i32, f32, vp, vp, vp, i32, vp, vp, vp, vp, f32, f32, i32, i32, vp]),
     "mi355_hy_attn_rows_ex": (i32, [vp, i32, f32, ip, i32, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, f32, vp, i32, i32, vp]),
     "mi355_dense_linear_pair": (i32, [C.POINTER(DenseArgs), vp]),
-    "mi355_dense_joined": (i32, [C.POINTER(DenseArgs), vp, i32, f32, vp]),
     "mi355_hy_recur_step_beside_fits": (i32, [i32] * 6),
     "mi355_hy_recur_step_beside": (i32, [C.POINTER(RecurArgs), C.POINTER(DenseArgs), vp]),
     "mi355_hy_recur_step_fits": (i32, [i32, i32]),

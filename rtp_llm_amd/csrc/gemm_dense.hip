@@ -57,10 +57,6 @@ struct DenseParams {
     // a weight that a later launch streams (its lines of 128 bytes): blocks past the list of tiles read one word of each
     const char* ahead = nullptr; uint32_t ahead_lines = 0;
     int streamed = 0;    // MI355_DENSE_STREAMED (host only)
-    // JOIN: a second pair of operands whose products go on the same sums, behind the first's K; y (fp32) += mult * the sums
-    const void* x2 = nullptr; const void* w2 = nullptr;
-    int K2 = 0, ldx2 = 0;
-    float mult = 0.f;
 };
 
 // The chip deals consecutive blocks to its eight XCDs in turn, each with an L2 of its own.  The (column tile, row tile) pair of a block is chosen such
@@ -279,10 +275,7 @@ __global__ __launch_bounds__(256) void dense_tile_bf16_kernel(DenseParams p) {
 //   M x N x K       8192x2048x2048 62 / 71 / 82 / 86 / 112, 118    6148x1408x1024 gated 33 / 31 / 29 / 32 / 37, 43     768x11264x2048 gated 50 / 52 / 49 / 53 / 61, 73
 //                   1537x2176x1024 30 / 15 / 14 / 13 /  17,  25    1537x1024x1024       29 / 15 / 13 / 11 / 10, 21     768x2048x5632       109 / 57 / 52 / 36 / 34, 77
 //                   1537x3072x1024 30 / 20 / 18 / 21 /  22,  30    1537x1024x2816       60 / 32 / 29 / 21 / 20, 45      70x2048x2048        42 / 23 / 20 / 16 / 12, 32
-//
-// JOIN: two linears of the same rows that are added to the fp32 stream, x += mult * (a A^T + b B^T), as one product over both K (whole tiles of each), and the sum in its epilogue.  The two results took
-// a launch, a write and a read each, the addition a read and a write of the stream in front of the norm: joined_shape has the times.
-template <int BM, int BN, int WM, int WN, int BK, int NS, bool JOIN = false>
+template <int BM, int BN, int WM, int WN, int BK, int NS>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_kernel(DenseParams p) {
     constexpr int NWM = BM / WM, NWN = BN / WN, NW = NWM * NWN, MI = WM / 16, NJ = WN / 16;
     constexpr bool AHEAD = BK == 32;                                          // fragments of tile t + 1 are read while tile t is multiplied
@@ -318,24 +311,11 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
             voff[u] = (uint32_t)min(r, p.N - 1 - n0) * (uint32_t)p.K * 2u + piece * 16u;
         }
     }
-    const int nk0 = p.K / BK, nk = JOIN ? nk0 + p.K2 / BK : nk0;
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem);
     auto issue1 = [&](int buf, int kt, int u) {
         dma16(lds0 + buf * STAGE + (u < ULA ? 0 : BM * RB) + ((u < ULA ? u : u - ULA) * NW + wave) * 1024, voff[u], u < ULA ? X + kt * BK : W + kt * BK);
     };
-    auto turn = [&](int kt) {                                               // in front of the loads of tile kt: the second operands' first one
-        if constexpr (JOIN)
-            if (kt == nk0) {
-                X = (const bf16*)p.x2 + (size_t)m0 * p.ldx2 - nk0 * BK; W = (const bf16*)p.w2 + (size_t)n0 * p.K2 - nk0 * BK;
-#pragma unroll
-                for (int u = 0; u < ULD; ++u) {
-                    const int r = ((u < ULA ? u : u - ULA) * NW + wave) * RPL + lr;
-                    voff[u] = (u < ULA ? (uint32_t)min(r, gr.rend - 1 - m0) * (uint32_t)p.ldx2 : (uint32_t)min(r, p.N - 1 - n0) * (uint32_t)p.K2) * 2u + piece * 16u;
-                }
-            }
-    };
     auto issue = [&](int buf, int kt) {
-        turn(kt);
 #pragma unroll
         for (int u = 0; u < ULD; ++u) issue1(buf, kt, u);
     };
@@ -361,6 +341,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
 #pragma unroll
             for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j], f.x[i], acc[i][j], 0, 0, 0);
     };
+    const int nk = p.K / BK;
     Frags fa, fb;
 #pragma unroll
     for (int t = 0; t < NS - 1; ++t) if (t < nk) issue(t, t);
@@ -398,7 +379,6 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
         constexpr int RP = (MI + NJ + ULD - 1) / ULD, MP = MI / ULD;
         static_assert(!AHEAD || MI % ULD == 0, "whole rows of products a part");
         auto tile = [&](const Frags& cur, Frags& nxt) {
-            turn(kt + NS - 1);
             wait_vm<decltype(steady)::value>();
             __builtin_amdgcn_s_barrier();
             const int foff = ((q ^ swizzle(fr)) << 4) + fr * RB;
@@ -440,7 +420,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
             if (kt + 1 < nk) fa = fb;
         }
     }
-    if (!JOIN && p.K % BK) {                                                // the last K % BK columns: through registers, zeros behind them
+    if (p.K % BK) {                                                         // the last K % BK columns: through registers, zeros behind them
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < ULD; ++u) {
@@ -459,32 +439,6 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2) void dense_dma_bf16_
     const bf16* Bi = p.bias ? (const bf16*)p.bias + gr.bo : nullptr;
     char* mine = smem + wave * (PH * 4096);
     const int nc = n0 + wn * WN;                                            // the wave's first weight row
-    if constexpr (JOIN) {                                                   // the general loop below with the stream's old values, asked for in front of the passage through LDS
-        const int c4 = lane & 15, n = nc + c4 * 4;
-        float* y = (float*)p.y + (size_t)(m0 + wm * WM + (lane >> 4)) * p.ldy + n;
-        __syncthreads();
-#pragma unroll
-        for (int i0 = 0; i0 < MI; i0 += PH) {
-            const int rows = gr.rend - (m0 + wm * WM + i0 * 16);
-            f32x4 old[PH * 4];
-#pragma unroll
-            for (int k = 0; k < PH * 4; ++k)
-                if (k * 4 + (lane >> 4) < rows && n < p.N) old[k] = *(const f32x4*)(y + (size_t)(i0 * 16 + k * 4) * p.ldy);
-#pragma unroll
-            for (int i = 0; i < PH; ++i)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) *(f32x4*)(mine + (i * 16 + fr) * 256 + (((j * 4 + q) ^ fr) << 4)) = acc[i0 + i][j];
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int k = 0; k < PH * 4; ++k) {
-                const int r = k * 4 + (lane >> 4);
-                const f32x4 v = *(const f32x4*)(mine + r * 256 + ((c4 ^ (r & 15)) << 4));
-                if (r < rows && n < p.N) *(f32x4*)(y + (size_t)(i0 * 16 + k * 4) * p.ldy) = old[k] + p.mult * v;
-            }
-            if (i0 + PH < MI) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        }
-        return;
-    }
     // What most calls ask for has code of its own: the choice among activations, caps, gates and output types a value took 1400 cycles a trip of the general loops (8192 x 11264 x 2048
     // gated: 11 of a block's 67 us, 3.6 now; all of it 359 / 325 us, 1537 x 1408 x 1024 gated 14.2 / 11.8, 456 x 11264 x 2048 gated 41.3 / 39.1, 1537 x 2176 x 1024 15.3 / 14.5).
     const bool lean = p.softcap <= 0.f && p.yvec && p.N % 4 == 0;
@@ -815,22 +769,6 @@ __global__ __launch_bounds__(256) void dense_rows_grouped_kernel(DenseParams p) 
         if (lane != 0 || o >= nout) continue;
         dn_store<T>(p, r, (int)(p.ys * g) + o, GATED ? dn_gated(gsum, u, p.act, p.act_param) : dn_act(gsum, p.act));
     }
-}
-
-// The tile shape of a joined product, -1: two launches are better.  us of both linears and the norm behind them, separate / joined (weights from memory): K 2048 + 5632 to 2048 columns, 456 rows 49 / 52,
-// 800 75 / 70, 1100 84 / 80, 2000 115 / 105, 3000 143 / 161 (64 x 128) or 170 (256 x 256), 4096 172 / 185 (256 x 256), 5000 237 / 182, 8192 296 / 252; K 1024 + 2816 to 1024 columns, 456 29.0 / 29.5,
-// 1100 37.5 / 34, 2000 42 / 36, 4096 65 / 56, 6000 87 / 91 (256 x 256), 8192 106 / 113 (128 x 128) or 95 (256 x 256).  128 x 128 tiles and two stages of 64 x 128 lose up to 40 %: with
-// one block fewer a compute unit.
-int joined_shape(int M, int N, int K) {
-    const int shape = mi355_dense_tile_shape(M, N, K, 1, 0);
-    if (shape == 4 || (shape >= 2 && ((M + 255) / 256) * ((N + 255) / 256) >= 144)) return 4;
-    return shape <= 1 && M >= 1024 ? shape : -1;
-}
-void launch_joined(const DenseParams& p, int shape, hipStream_t st) {
-    const int gy = (p.M + 63) / 64;
-    if (shape == 0)      hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 64, 16, 64, 64, 4, true>), dim3((p.N + 63) / 64, gy), dim3(256), 0, st, p);
-    else if (shape == 1) hipLaunchKernelGGL((dense_dma_bf16_kernel<64, 128, 32, 64, 64, 3, true>), dim3((p.N + 127) / 128, gy), dim3(256), 0, st, p);
-    else                 hipLaunchKernelGGL((dense_dma_bf16_kernel<256, 256, 128, 64, 32, 4, true>), dim3((p.N + 255) / 256, (p.M + 255) / 256), dim3(512), 0, st, p);
 }
 
 // The bf16 tile launch of p: gy64 row tiles of 64 rows (blockIdx.y) when the rows are grouped, groups in z.
@@ -1302,28 +1240,6 @@ extern "C" int mi355_hy_recur_step_beside(const mi355_recur_args_t* a, const mi3
     if (!recur_linear_fits(r.dim, r.vdim, p.M, p.N, p.K, p.gated, p.streamed)) return MI355_ERR_UNSUPPORTED;
     launch_recur_linear(r, a->nseq, p, (hipStream_t)stream);
     MI355_CHECK_LAUNCH("hy_recur_linear_kernel");
-    return MI355_OK;
-}
-
-// x[m, n] += mult * (sum over k of two[0].x[m, k] two[0].w[n, k] + the same of two[1]): bf16 operands of the same M of more than 16 rows and N, x fp32 of row stride ldx.  Of each argument x, ldx, M, w, N
-// and K are read.  MI355_ERR_UNSUPPORTED: sizes that two launches are better for (joined_shape), K that are no multiples of 64, operands or rows off 16 bytes, rows out of reach of 32-bit offsets.
-extern "C" int mi355_dense_joined(const mi355_dense_args_t* two, float* x, int32_t ldx, float mult, mi355_stream_t stream) {
-    MI355_CHECK_ARG(two && x, "dense_joined: null arguments");
-    for (int i = 0; i < 2; ++i) {
-        const mi355_dense_args_t& d = two[i];
-        MI355_CHECK_ARG(d.x && d.w && d.M > 0 && d.N > 0 && d.K > 0 && d.ldx >= d.K && d.M == two[0].M && d.N == two[0].N && ldx >= d.N, "dense_joined: M=%d N=%d K=%d ldx=%d ld=%d", d.M, d.N, d.K, d.ldx,
-                        ldx);
-        if (d.M <= 16 || d.K % 64 || d.ldx % 8 || (uintptr_t)d.x % 16 || (uintptr_t)d.w % 16 || (uint64_t)d.ldx * 512 >= 0xFFFFFFFFull || (uint64_t)d.K * 512 >= 0xFFFFFFFFull) return MI355_ERR_UNSUPPORTED;
-    }
-    const int shape = joined_shape(two[0].M, two[0].N, two[0].K + two[1].K);
-    if (shape < 0 || two[0].N % 4 || ldx % 4 || (uintptr_t)x % 16) return MI355_ERR_UNSUPPORTED;
-    DenseParams p;
-    p.x = two[0].x; p.w = two[0].w; p.bias = nullptr; p.y = x; p.M = two[0].M; p.N = two[0].N; p.K = two[0].K; p.ldx = two[0].ldx; p.ldy = ldx;
-    p.gated = 0; p.act = 0; p.act_param = 0.f; p.out_f32 = 1; p.softcap = 0.f; p.vec = 1; p.yvec = 1;
-    p.G = 1; p.xs = p.ws = p.ys = 0; p.offs = nullptr; p.gather = nullptr; p.tiles = nullptr; p.egate = nullptr; p.ldg = p.goff = 0;
-    p.x2 = two[1].x; p.w2 = two[1].w; p.K2 = two[1].K; p.ldx2 = two[1].ldx; p.mult = mult;
-    launch_joined(p, shape, (hipStream_t)stream);
-    MI355_CHECK_LAUNCH("dense_dma_bf16_kernel");
     return MI355_OK;
 }
 

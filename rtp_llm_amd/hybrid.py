@@ -571,14 +571,12 @@ class HybridModel:
         else:
             x = hops.embed(batch.tokens, self.embed)
         a = b = g = None
-        joined = False                                 # the last layer's branches are in the stream already
         shared = self.n_mix
         router_at = 2 * W if cfg.branch_gates else 0   # column of the router's logits behind the mixer's
         for run, (i, cache) in enumerate(zip(self.runs, caches)):
             L, mixer, mlp, n1, n2, gate_w, gate_b = self.layers[i]
             bg = g if cfg.branch_gates else None
             done = collect is not None and a is not None
-            joined = False
             if run in self.pass_at:                    # x <- A [x; x0] + s: the last layer's branches join the stream in the launch that rounds it
                 hops.residual_round(x, a, b, cfg.residual_mult, pair[:, :W], gate=bg)
                 if done:
@@ -613,17 +611,6 @@ class HybridModel:
                 a, b = hops.dense_pair(dict(x=o, w=mixer.w_o, bias=getattr(mixer, "b_o", None), out_dtype=torch.float32),
                                        dict(x=up, w=mlp.w_down, out_dtype=torch.float32))
                 continue
-            elif gate_w is None and isinstance(mlp, GatedMLP) and hasattr(mixer, "few_rows") and getattr(mixer, "b_o", None) is None:
-                # prompts: the two branches' output linears join the stream in one launch
-                o = mixer.forward(h1, batch, *(cache if isinstance(cache, tuple) else (cache,)), out_proj=False)
-                up = hops.dense_linear(h2, mlp.w_gate_up, gated=True, act=mlp.act, act_param=mlp.act_param)
-                g = a = b = None
-                joined = hops.dense_joined(x, cfg.residual_mult, o, mixer.w_o, up, mlp.w_down)
-                if not joined:
-                    a, b = hops.dense_linear(o, mixer.w_o, out_dtype=torch.float32), hops.dense_linear(up, mlp.w_down, out_dtype=torch.float32)
-                elif collect is not None:
-                    collect.append(x.clone())
-                continue
             else:
                 g = hops.dense_linear(h1, gate_w, gate_b, out_dtype=torch.float32) if gate_w is not None else None
                 a = mixer.forward(h1, batch, *cache) if isinstance(cache, tuple) else mixer.forward(h1, batch, cache)
@@ -634,7 +621,7 @@ class HybridModel:
             else:
                 b = mlp.forward(h2)
         bg = g if cfg.branch_gates else None
-        if collect is not None and not joined:
+        if collect is not None:
             hops.residual_norm(x, a, b, cfg.residual_mult, self.final_norm, None, cfg.eps, weight_offset=cfg.norm_offset, gate=bg)
             collect.append(x.clone())
             a = b = bg = None

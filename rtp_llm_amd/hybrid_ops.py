@@ -157,26 +157,6 @@ def dense_pair(first: dict, second: dict):
     return tuple(outs)
 
 
-def dense_joined(x: torch.Tensor, mult: float, a: torch.Tensor, w_a: torch.Tensor, b: torch.Tensor, w_b: torch.Tensor) -> bool:
-    """x (fp32 [T, N], in place) += mult * (a w_a^T + b w_b^T) as one product over both K; False, and x as it was, where that is not built or no gain: few rows, other types than bf16, K off 64, rows off
-    16 bytes."""
-    _dev(x, torch.float32, "dense_joined.x")
-    T, N = x.shape
-    args = (_C.DenseArgs * 2)()
-    for d, t, w in zip(args, (a, b), (w_a, w_b)):
-        if w.dtype != torch.bfloat16 or T <= FEW_ROWS:
-            return False
-        _dev(t, w.dtype, "dense_joined.a"); _dev(w, w.dtype, "dense_joined.w")
-        if t.dim() != 2 or t.shape[0] != T or w.shape != (N, t.shape[1]) or not w.is_contiguous():
-            raise _C.Mi355Error(f"dense_joined: {tuple(t.shape)} against {tuple(w.shape)} for x {tuple(x.shape)}")
-        d.x, d.ldx, d.M, d.w, d.N, d.K = t.data_ptr(), _rows(t, "dense_joined.a"), T, w.data_ptr(), N, w.shape[1]
-    rc = _C.hybrid_lib().mi355_dense_joined(args, x.data_ptr(), _rows(x, "dense_joined.x"), float(mult), _stream())
-    if rc == _C.ERR_UNSUPPORTED:
-        return False
-    _C.check_hybrid(rc, "dense_joined")
-    return True
-
-
 def group_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """[ff, K] gate and up weights -> the [2 ff, K] weight of a gated dense_linear: per 32 channels, 32 gate rows then 32 up rows
     (ff % 32 == 0)."""
