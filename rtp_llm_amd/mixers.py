@@ -761,6 +761,11 @@ def ahead_from(experts: int, nbytes: int) -> float:
 
 # tokens above which a shared expert of the experts' form runs in their grouped linears; up to 64 the routing and the sort are one launch, which does not give it rows
 JOINT_FROM = 64
+# tokens x width x channels up to which it does in bf16.  It saves two launches (9 to 20 us, a host's work beside), and costs the shared expert the larger tiles that its own launches would take (sorted
+# rows come in tiles of 64): a share of its products.  Joint / alone, 173 layers of 65 to 16384 tokens, 1024 to 7168 wide, 256 to 4096 channels, 4 to 128 experts, 1 to 8 chosen: 126 below the line 0.93
+# on average, at worst 1.05; 47 above 1.04, up to 1.20 (4096 x 4096, 8 experts, 2 of them, 8192 tokens 3475 / 3033 us; at 512 385 / 391); the pick is 0.1 % off the faster one.  fp32 rows have tiles of
+# 64 either way: 14 of 65 to 4096 tokens 0.54 to 1.005.
+JOINT_WORK = 12e9
 
 
 class RoutedExperts:
@@ -810,6 +815,11 @@ class RoutedExperts:
             shared.w_gate_up, shared.w_down = (w[r.experts] for w in self.w_all)
         self.ahead_from = [ahead_from(r.experts, w.numel() * w.element_size()) for w in (self.w_gate_up, self.w_down)]
 
+    def _joint(self, T: int) -> bool:
+        """Whether the shared expert's T rows run in the grouped linears."""
+        _, W, ff = self.w_down.shape
+        return self.joint and T > JOINT_FROM and (self.w_down.dtype != torch.bfloat16 or T * W * ff <= JOINT_WORK)
+
     def forward(self, h: torch.Tensor, logits: Optional[torch.Tensor] = None, defer: bool = False):
         """logits: the router's fp32 logits [T, experts] when the caller has computed them (in a linear shared with other projections of h).
         defer: return the parts of the weighted sum (hybrid_ops.MoeSum) for a residual kernel that forms it, instead of the summed tensor
@@ -822,7 +832,7 @@ class RoutedExperts:
                 logits, sgate = logits[:, :self.n_router], logits[:, self.n_router]
         pairs = logits.shape[0] * r.top
         T = logits.shape[0]
-        joint = self.joint and T > JOINT_FROM
+        joint = self._joint(T)
         w_gate_up, w_down = self.w_all if joint else (self.w_gate_up, self.w_down)
         ids, wts, offs, src, place, tiles = hops.moe_route_sorted(logits, r.experts, r.groups, r.keep, r.top, sigmoid=r.score == "sigmoid", chosen=r.score == "softmax_chosen",
                                                                   group_top=r.group_top, scale=r.scale, ahead=self.w_gate_up if pairs >= self.ahead_from[0] else None, shared=joint)

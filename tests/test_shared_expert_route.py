@@ -1,0 +1,36 @@
+"""Which steps run a mixture's shared expert in the grouped linears of the others: decided on the host."""
+import pytest
+import torch
+
+from rtp_llm_amd import mixers
+
+
+class _Asked(Exception):
+    pass
+
+
+def _mixture(W, ff, E, dtype=torch.bfloat16, seed=0, shared=None):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    shared = shared or mixers.GatedMLP(r(ff, W), r(ff, W), r(W, ff), act="silu")
+    return mixers.RoutedExperts(mixers.RouterSpec(E, 2), r(E, W), [r(ff, W) for _ in range(E)], [r(ff, W) for _ in range(E)], [r(W, ff) for _ in range(E)], shared, act="silu")
+
+
+def _asks(monkeypatch, m, T):
+    """Whether a forward pass over T rows asks the sort for the shared expert's rows."""
+    def sort(*a, shared=False, **k):
+        raise _Asked(bool(shared))
+    monkeypatch.setattr(mixers.hops, "moe_route_sorted", sort)
+    W, E = m.w_down.shape[1], m.router.experts
+    with pytest.raises(_Asked) as e:
+        m.forward(torch.zeros(1, W, dtype=m.w_down.dtype).expand(T, W), torch.zeros(1, E).expand(T, E))
+    return e.value.args[0]
+
+
+# 65 rows and more, up to 12e9 products of a linear: above them the shared expert's own launches have larger tiles (fp32 has one)
+@pytest.mark.parametrize("W,ff,last", [(1024, 704, 16645), (256, 96, 488281), (2048, 2048, 2861)])
+def test_many_rows_of_a_large_expert_run_alone(monkeypatch, W, ff, last):
+    m = _mixture(W, ff, 2)
+    assert [_asks(monkeypatch, m, T) for T in (1, 64, 65, last, last + 1, 4 * last)] == [False, False, True, True, False, False]
+    if W == 1024:
+        assert _asks(monkeypatch, _mixture(W, ff, 2, torch.float32), 4 * last)
