@@ -805,7 +805,7 @@ class RoutedExperts:
         # a shared expert of the same form lies behind the others: the prompts' grouped linears run it as one more, the same bits.  1537 tokens, 4 of 16 experts of 704 at width 1024: gate and up
         # 41.5 + 15.1 -> 46.2 us, down 24.5 + 10.4 -> 31.2
         self.shared, self.act, self.act_param = shared, hops.ACTIVATIONS[act], float(act_param)
-        self.joint = (shared is not None and self.gated and shared.act == self.act and shared.act_param == self.act_param and shared.w_gate_up.shape == gu[0].shape
+        self.joint = (type(shared) is GatedMLP and self.gated and shared.act == self.act and shared.act_param == self.act_param and shared.w_gate_up.shape == gu[0].shape
                       and shared.w_down.shape == dn[0].shape and shared.w_gate_up.dtype == gu[0].dtype)
         if self.joint:
             gu.append(shared.w_gate_up); dn.append(shared.w_down)

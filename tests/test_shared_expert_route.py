@@ -34,3 +34,24 @@ def test_many_rows_of_a_large_expert_run_alone(monkeypatch, W, ff, last):
     assert [_asks(monkeypatch, m, T) for T in (1, 64, 65, last, last + 1, 4 * last)] == [False, False, True, True, False, False]
     if W == 1024:
         assert _asks(monkeypatch, _mixture(W, ff, 2, torch.float32), 4 * last)
+
+
+class _Other:
+    """A shared expert of a kind of its own: nothing but forward."""
+
+    def forward(self, h):
+        return h.float()
+
+
+def test_a_shared_expert_of_another_kind_runs_alone(monkeypatch):
+    class Wrapped(mixers.GatedMLP):
+        def forward(self, h):
+            return super().forward(h) * 2
+
+    r = lambda *s: torch.randn(*s).bfloat16()
+    wrapped = Wrapped(r(96, 256), r(96, 256), r(256, 96), act="silu")
+    before = wrapped.w_gate_up, wrapped.w_down
+    poly = mixers.PolyNormMLP(r(96, 256), r(256, 96), torch.ones(4), 1e-6)
+    for shared in (_Other(), poly, wrapped):
+        assert not _asks(monkeypatch, _mixture(256, 96, 2, shared=shared), 100)
+    assert wrapped.w_gate_up is before[0] and wrapped.w_down is before[1]
