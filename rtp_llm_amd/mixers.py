@@ -803,13 +803,15 @@ class RoutedExperts:
                 d = torch.cat([d, torch.zeros(d.shape[0], pad, dtype=d.dtype, device=d.device)], 1)
             gu.append(hops.group_gate_up(g, u) if self.gated else u); dn.append(d)
         # a shared expert of the same form lies behind the others: the prompts' grouped linears run it as one more, the same bits.  1537 tokens, 4 of 16 experts of 704 at width 1024: gate and up
-        # 41.5 + 15.1 -> 46.2 us, down 24.5 + 10.4 -> 31.2
+        # 41.5 + 15.1 -> 46.2 us, down 24.5 + 10.4 -> 31.2.  The caller's module then holds views of the stack, so that its weights lie in memory once
         self.shared, self.act, self.act_param = shared, hops.ACTIVATIONS[act], float(act_param)
         self.joint = (type(shared) is GatedMLP and self.gated and shared.act == self.act and shared.act_param == self.act_param and shared.w_gate_up.shape == gu[0].shape
                       and shared.w_down.shape == dn[0].shape and shared.w_gate_up.dtype == gu[0].dtype)
         if self.joint:
             gu.append(shared.w_gate_up); dn.append(shared.w_down)
         self.w_all = torch.stack(gu).contiguous(), torch.stack(dn).contiguous()
+        self.behind = [r.experts * w.stride(0) * w.element_size() for w in self.w_all]           # where the shared expert lies in them
+        self.products = dn[0].numel() if dn[0].dtype == torch.bfloat16 else 0                    # of a linear and a row, for JOINT_WORK
         self.w_gate_up, self.w_down = (w[:r.experts] for w in self.w_all)
         if self.joint:
             shared.w_gate_up, shared.w_down = (w[r.experts] for w in self.w_all)
@@ -817,8 +819,13 @@ class RoutedExperts:
 
     def _joint(self, T: int) -> bool:
         """Whether the shared expert's T rows run in the grouped linears."""
-        _, W, ff = self.w_down.shape
-        return self.joint and T > JOINT_FROM and (self.w_down.dtype != torch.bfloat16 or T * W * ff <= JOINT_WORK)
+        if not self.joint or T <= JOINT_FROM or T * self.products > JOINT_WORK:
+            return False
+        # a caller may have given the experts or the shared one other weights since: the stack is read only where it is theirs
+        s, (gu, dn) = self.shared, self.w_all
+        return (type(s) is GatedMLP and s.act == self.act and s.act_param == self.act_param and s.w_gate_up.shape == gu.shape[1:] and s.w_down.shape == dn.shape[1:]
+                and self.w_gate_up.data_ptr() == gu.data_ptr() and s.w_gate_up.data_ptr() == gu.data_ptr() + self.behind[0]
+                and self.w_down.data_ptr() == dn.data_ptr() and s.w_down.data_ptr() == dn.data_ptr() + self.behind[1])
 
     def forward(self, h: torch.Tensor, logits: Optional[torch.Tensor] = None, defer: bool = False):
         """logits: the router's fp32 logits [T, experts] when the caller has computed them (in a linear shared with other projections of h).

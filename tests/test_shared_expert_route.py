@@ -55,3 +55,31 @@ def test_a_shared_expert_of_another_kind_runs_alone(monkeypatch):
     for shared in (_Other(), poly, wrapped):
         assert not _asks(monkeypatch, _mixture(256, 96, 2, shared=shared), 100)
     assert wrapped.w_gate_up is before[0] and wrapped.w_down is before[1]
+
+
+@pytest.mark.parametrize("what", ["shared gate and up", "shared down", "shared in place", "gate and up", "down", "activation", "parameter", "none", "another"])
+def test_weights_given_later_are_the_ones_that_run(monkeypatch, what):
+    """The stack of all weights stands for the attributes only while they are parts of it."""
+    m, other = _mixture(256, 96, 3), _mixture(256, 96, 3, seed=1)
+    assert _asks(monkeypatch, m, 100)
+    if what == "shared gate and up":
+        m.shared.w_gate_up = other.shared.w_gate_up.clone()
+    elif what == "shared down":
+        m.shared.w_down = other.shared.w_down.clone()
+    elif what == "shared in place":                                  # a copy into the view reaches the stack
+        m.shared.w_down.copy_(other.shared.w_down)
+        assert torch.equal(m.w_all[1][3], other.shared.w_down) and _asks(monkeypatch, m, 100)
+        return
+    elif what == "gate and up":
+        m.w_gate_up = other.w_gate_up.clone()
+    elif what == "down":
+        m.w_down = other.w_down.clone()
+    elif what == "activation":
+        m.shared.act = mixers.hops.ACT_RELU
+    elif what == "parameter":
+        m.shared.act_param = 1.0
+    elif what == "none":
+        m.shared = None
+    elif what == "another":
+        m.shared = other.shared
+    assert not _asks(monkeypatch, m, 100)
