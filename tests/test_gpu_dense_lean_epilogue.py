@@ -14,8 +14,11 @@ def _out(M, n, dtype, pad, off):
     return buf, buf[off:off + M * (n + pad)].view(M, n + pad)[:, :n]
 
 
-# every tile shape: 64x64 (few blocks), 64x128, 128x128, 256x256; rows and columns past the last whole tile
-@pytest.mark.parametrize("M,N,K", [(17, 64, 64), (130, 192, 96), (333, 1088, 1024), (1537, 2176, 136), (700, 11264, 256), (2049, 4160, 512)])
+# every tile shape: 64x64 (few blocks), 64x128 in three and in two stages, 128x128, 256x256 (test_tile_shapes.py holds the lists to that); rows and columns past the last whole tile
+SIZES = [(17, 64, 64), (130, 192, 96), (333, 1088, 1024), (1537, 2176, 136), (700, 11264, 256), (2049, 4160, 512), (3001, 11264, 136), (4099, 4160, 264), (8190, 2048, 2056), (4099, 11264, 2048)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
 @pytest.mark.parametrize("form", ["relu", "silu", "gelu_tanh", "plain", "bias", "odd columns"])
 def test_stores(M, N, K, form):
     g = torch.Generator(device=DEV).manual_seed(M + N)
@@ -45,7 +48,11 @@ def test_stores(M, N, K, form):
     assert bool(((got[0].double() - y).abs() <= (2.0 ** -7 if gated else 2.0 ** -16) * y.abs() + 2.0 ** -14).all())
 
 
-@pytest.mark.parametrize("M,H,R,dv", [(65, 3, 64, 64), (1537, 8, 192, 128), (200, 5, 96, 40)])
+# heads of one row block a wave, of two (two or four trips of the loop over rows), of eight in two phases: every tile shape too
+HEADS = [(65, 3, 64, 64), (1537, 8, 192, 128), (200, 5, 96, 40), (1537, 3, 96, 512), (2049, 8, 96, 256), (4099, 8, 256, 508), (8190, 2, 1024, 4092)]
+
+
+@pytest.mark.parametrize("M,H,R,dv", HEADS)
 def test_outputs_times_a_gate(M, H, R, dv):
     g = torch.Generator(device=DEV).manual_seed(M)
     x, w = torch.randn(M, H * R, device=DEV, generator=g).bfloat16(), (torch.randn(H, dv, R, device=DEV, generator=g) * R ** -0.5).bfloat16()

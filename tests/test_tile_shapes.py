@@ -1,5 +1,6 @@
 """The lists of the tile tests reach every tile shape that a call can take: the shape chosen for each listed call, against all shapes chosen over a grid of sizes."""
 import pytest
+import test_gpu_dense_lean_epilogue as lean
 import test_gpu_dense_tiles as dense
 import test_gpu_prefill_gemm as prefill
 
@@ -43,3 +44,9 @@ def test_dense_shapes():
     # the largest tile with an even and an odd count of K tiles of 32, both with a remainder
     assert {K // 32 % 2 for M, N, K in dense.SHAPES if pick(M, N, K, 1, 0) == 4 and K % 32} == {0, 1}
     assert {pick(M, N, K, 1, 64) for M, N, K in dense.SHAPES} <= {0, 1, 2}           # sorted rows: tiles of 64
+
+
+def test_dense_lean_store_shapes():
+    pick = _C.hybrid_lib().mi355_dense_tile_shape
+    assert {pick(M, N, K, 1, 0) for M, N, K in lean.SIZES} == {pick(M, N - 3, K, 1, 0) for M, N, K in lean.SIZES} == {0, 1, 2, 3, 4}
+    assert {pick(M, dv, R, H, 0) for M, H, R, dv in lean.HEADS} == {0, 1, 2, 3, 4}
