@@ -3,6 +3,7 @@ import pytest
 import test_gpu_dense_lean_epilogue as lean
 import test_gpu_dense_tiles as dense
 import test_gpu_prefill_gemm as prefill
+import test_gpu_prefill_stores as stores
 
 from rtp_llm_amd import _C
 
@@ -50,3 +51,18 @@ def test_dense_lean_store_shapes():
     pick = _C.hybrid_lib().mi355_dense_tile_shape
     assert {pick(M, N, K, 1, 0) for M, N, K in lean.SIZES} == {pick(M, N - 3, K, 1, 0) for M, N, K in lean.SIZES} == {0, 1, 2, 3, 4}
     assert {pick(M, dv, R, H, 0) for M, H, R, dv in lean.HEADS} == {0, 1, 2, 3, 4}
+
+
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("kind,group", stores.KINDS)
+def test_prefill_store_shapes(kind, group, bf16):
+    """Each tile whose results pass through LDS, by class: a launch of that shape alone, a last tile of some rows and one of some columns, gated rows of whole 16 bytes."""
+    bits = {"w4": 4, "int8": 8, "fp16": 16}[kind]
+    tile = {0: (128, 512), 1: (128, 256), 2: (64, 256)}
+    seen = set()
+    for M, K, N in stores.SHAPES:
+        args = (M, -(-N // 16), K // 128, bf16, bits, group, 1)
+        s = _C.lib().mi355_gemm_prefill_form(*args) & 15
+        if s in tile and not _C.lib().mi355_gemm_prefill_rest(*args) and M % tile[s][0] and N % tile[s][1] and N % 16 == 0:
+            seen.add(s)
+    assert seen >= {1, 2} | ({0} if not bf16 and kind != "fp16" and group != 32 else set())
