@@ -1,4 +1,7 @@
 """Prompt linears that run two tile shapes in one launch against the general loop in one shape, which x off 16 bytes takes: the same bits, and nothing beside them."""
+import math
+import random
+
 import pytest
 import torch
 
@@ -39,11 +42,27 @@ def test_same_bits_as_one_shape(kind, bf16, M, N, K, pick):
         assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
-def test_first_shape_fills_whole_rounds_and_leaves_some():
-    for kind, bf16, M, N, K, (first, second, cols) in CALLS:
-        tiles = -(-M // 128) * cols
-        width = 512 if first == 0 else 256
-        assert second > first and 0 < cols * width < N and (tiles % 256 == 0 or tiles % 256 + -(-M // 128) > 256)
+def _whole_rounds(M, N, first, second, cols):
+    """The first shape's tiles end on a round of the chip's 256 places, but for less than a column of them, and leave columns behind; the pair of shapes is one that the launch builds."""
+    rows, width = -(-M // 128), 512 if first == 0 else 256
+    assert 0 < cols * width < N and -(rows * cols) % 256 < rows and (first, second) in {(0, 1), (0, 2), (0, 3), (1, 3)}
+
+
+@pytest.mark.parametrize("kind,bf16", [("w4", False), ("w4", True), ("int8", False), ("int8", True)])
+def test_first_shape_fills_whole_rounds_and_leaves_some(kind, bf16):
+    g, pairs = random.Random(f"{kind} {bf16}"), set()
+    sizes = [(M, N, K) for k, b, M, N, K, _ in CALLS if (k, b) == (kind, bf16)]
+    sizes += [(int(math.exp(g.uniform(math.log(65), math.log(12000)))), 8 * g.randint(8, 4750), 128 * g.randint(1, 150)) for _ in range(3000)]
+    for M, N, K in sizes:
+        pick = rest(kind, bf16, M, N, K)
+        if pick:
+            _whole_rounds(M, N, *pick)
+            pairs.add(pick[:2])
+            assert rest(kind, bf16, M, N, K, whole=0) is None
+    assert pairs == ({(1, 3)} if bf16 else {(0, 1), (0, 2), (0, 3), (1, 3)})
+    for k, b, M, N, K, pick in CALLS:
+        if (k, b) == (kind, bf16):
+            assert rest(k, b, M, N, K) == pick
 
 
 def test_one_shape_where_two_are_not_built():
