@@ -132,9 +132,10 @@ int mi355_linear_forward(const void* x, int32_t M, const mi355_weight_t* w, cons
 /* The block shape of a linear over more than 64 rows (N_pad / 16 weight tiles, K_pad / 128 chunks): 0 128x512, 1 128x256, 2 64x256, 3 64x128, 4 64x64, 5 32x64,
  * 6 32x32.  Host only. */
 int mi355_gemm_prefill_shape(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits);   /* 4-bit weights in groups of 128; x on 16 bytes, K a multiple of 128 */
-/* the same for any group size and x (whole: x on 16 bytes and K a multiple of 128), plus 16 where the call runs the loop without branches */
+/* the same for any group size and x (whole: x on 16 bytes and K a multiple of 128), plus 16 where the call runs the loop without branches.  Both: the shape of a call that runs one; where
+ * mi355_gemm_prefill_rest is not 0 the call runs those two instead, both in that loop, and this is the one shape that they were compared with */
 int mi355_gemm_prefill_form(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits, int32_t group_size, int32_t whole);
-/* 0, or, where such a call runs two shapes in one launch, the first shape + 4 * the rest's + 16 * the first's column tiles. */
+/* 0, or, where such a call runs two shapes in one launch, the first shape + 4 * the rest's + 16 * the first's column tiles.  Host only. */
 int mi355_gemm_prefill_rest(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits, int32_t group_size, int32_t whole);
 /* the tile that block `id` of a call with rows x cols tiles takes where the tiles are not dealt in rows for another reason: column tile in the low 32 bits, row tile in the high ones */
 int64_t mi355_gemm_prefill_tile(int32_t id, int32_t rows, int32_t cols);

@@ -691,7 +691,7 @@ extern "C" int64_t mi355_gemm_prefill_tile(int32_t id, int32_t rows, int32_t col
     return (int64_t)by << 32 | bx;
 }
 
-// The block shape of a call, by its place in kPrefillShapes: NT = N_pad / 16, KC = K_pad / 128.  4-bit weights in groups of 128, x on 16 bytes, K a multiple of 128.
+// The block shape of a call that runs one (mi355_gemm_prefill_rest 0; else the one that the two were compared with), by its place in kPrefillShapes: NT = N_pad / 16, KC = K_pad / 128.  4-bit weights in groups of 128, x on 16 bytes, K a multiple of 128.
 extern "C" int mi355_gemm_prefill_shape(int32_t M, int32_t NT, int32_t KC, int32_t bf16, int32_t wbits) {
     return mi355_gemm_prefill_form(M, NT, KC, bf16, wbits, 128, 1) & 15;
 }

@@ -73,7 +73,8 @@ def test_prefill_gemm_straight_loop(kind, group, dtype):
         off = buf[4:4 + M * K].view(M, K).copy_(x)
         assert x.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 8
         assert torch.equal(ops.linear(x, w).view(torch.int16), ops.linear(off, w).view(torch.int16)), (M, K, N)
-        seen.add(_C.lib().mi355_gemm_prefill_shape(M, -(-N // 16), K // 128, int(dtype == torch.bfloat16), w.wbits))
+        if not _C.lib().mi355_gemm_prefill_rest(M, -(-N // 16), K // 128, int(dtype == torch.bfloat16), w.wbits, group, 1):           # two shapes in one launch: test_gpu_prefill_rest.py
+            seen.add(_C.lib().mi355_gemm_prefill_shape(M, -(-N // 16), K // 128, int(dtype == torch.bfloat16), w.wbits))
     can = {0, 1, 2, 3, 4, 5, 6} - ({0} if kind == "fp16" or dtype == torch.bfloat16 else set())
     assert seen >= can, seen
 
@@ -90,6 +91,8 @@ def test_prefill_gemm_both_loops(kind, group, bf16):
     form = lambda M, K, N, whole: _C.lib().mi355_gemm_prefill_form(M, -(-N // 16), K // 128, int(bf16), bits, group, int(whole))
     left = set(STRAIGHT[kind, group, bf16])
     for M, K, N in WHOLE + [(370, 896, 37880), (130, 640, 16392), (580, 384, 11016), (835, 640, 8208), (2000, 896, 4104)]:
+        if _C.lib().mi355_gemm_prefill_rest(M, -(-N // 16), K // 128, int(bf16), bits, group, 1):                                     # two shapes in one launch: test_gpu_prefill_rest.py
+            continue
         whole, off = form(M, K, N, True), form(M, K, N, False)
         assert off < 16 and (whole >= 16) == (whole & 15 in STRAIGHT[kind, group, bf16])
         if whole & 15 not in left:
