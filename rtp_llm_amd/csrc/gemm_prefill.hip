@@ -610,6 +610,9 @@ int pick_shape(int M, int NT, int KC, bool bf, int wbits, int group_size, bool w
 // bits 0.973 (0.967); 11 above 1.02, at worst 1.05.  16-bit weights 0.996, at worst 1.17: one shape.  us one shape / two: fp16 W4 37888 x 3584 gated at 4096 rows 902 / 868 (128 x 512 and 64 x 256),
 // 2667 625 / 577 (and 64 x 128), 1825 442 / 415 (and 128 x 256), 4608 x 3584 at 4096 138 / 114; fp16 8 bits the same at 4096 845 / 822 and 123 / 105; bf16 W4 4608 x 3584 at 4096 161 / 137
 // (128 x 256 and 64 x 128), 37888 x 3584 at 1055 331 / 306.
+// Under bf16 W4 the rest's 64 x 128 blocks run the loop without branches, which a call of that shape alone does not (prefill_straight), while the table's row for it is the general loop's.  It decides as
+// well as one of their own: 152 random calls that could take two, of 400 to 9000 rows, 0.977 of the time with one shape (best choice of each 0.971; 41 take two, none of them slower), with the row
+// fitted to their times (0.48 and 0.74) 0.979.
 struct PrefillRest { int shape, rest, cols; };               // cols 0: one shape
 PrefillRest pick_rest(int best, int M, int NT, int KC, bool bf, int wbits, int group_size, bool whole) {
     PrefillRest pick{best, 0, 0};
