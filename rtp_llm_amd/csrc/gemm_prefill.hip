@@ -126,16 +126,17 @@ __host__ __device__ __forceinline__ void prefill_tile(int id, int rows, int cols
 // LDS at the end).  TPW = weight tiles per wave, MB = 16-row blocks of the tile, so the tile is 16 MB rows x 16 TPW NWN columns.
 //   TPW = 4, MB = 8 (128 x 512, one block per CU): one B-fragment read from LDS feeds four MFMAs.  At TPW = 2 (128 x 256, two blocks per CU) the 8 waves of a
 //   block pull 256 KiB of fragments per 128-k chunk through the CU's LDS port for 512 MFMAs -- 2048 cycles of each, neither hidden behind the other.
-//   MB = 4 and the K-sliced forms are for grids that would leave most CUs without a block (narrow outputs, short prompts): see launch_prefill_t.
+//   MB = 4 and the K-sliced forms are for grids that would leave most CUs without a block (narrow outputs, short prompts): see pick_shape.
 // BF: bf16 activations.  16-bit weights are the MFMA operand as they are; a 4-bit code enters it as the exact integer u - z and the group's scale multiplies the
 // group's fp32 sums (a bf16 product s (u - z) would round the weight to 8 bits); an 8-bit code as the exact u - 128, its column scale on the finished sums.
 // WHOLE: K is a multiple of 128 and x lies on 16 bytes, so that every chunk comes by DMA and the loop has no branch.  With the branches of the general loop the
 // compiler's count of loads in flight, taken over all paths, made the products wait for the DMA of the chunk after (37 to 42 % of the waves' time at 128 x 512 went into
 // waits), and the first three fragment reads of a chunk waited one by one.  In front of the last chunk of a straight loop lies one DMA too many (K sliced: left out);
 // it reads a chunk again that is there, and is waited for.
-// us general / WHOLE, same bits: 8 bits 37888 x 3584 at 1055 rows 279 / 263 (128 x 512), 3584 x 18944 155 / 136 (64 x 256); fp16 W4 37888 x 3584 at 4096 rows 1060 / 1004
-// (power), 3584 x 3584 at 512 rows 36 / 32 (64 x 256), 26.6 / 22.7 (64 x 128); bf16 W4 37888 x 3584 at 4096 rows 1257 / 1091 (128 x 256); W16 896 x 4864 at 777 rows
-// 21.3 / 19.1 (64 x 64), 9728 x 896 39 / 34 (32 x 64).
+// us general / WHOLE, same bits, one shape, both with the stores from the accumulators: 8 bits 37888 x 3584 at 1055 rows 279 / 263 (128 x 512), 3584 x 18944 155 / 136
+// (64 x 256); fp16 W4 37888 x 3584 at 4096 rows 1060 / 1004 (power), 3584 x 3584 at 512 rows 36 / 32 (64 x 256), 26.6 / 22.7 (64 x 128); bf16 W4 37888 x 3584 at 4096 rows
+// 1257 / 1091 (128 x 256); W16 896 x 4864 at 777 rows 21.3 / 19.1 (64 x 64), 9728 x 896 39 / 34 (32 x 64).  Whole calls of the present code, plain, us: 8 bits 235 and 134,
+// fp16 W4 845 (two shapes) and 21.4, bf16 W4 1068, W16 16.5; fp16 W4 at 4096 rows 1305 TFLOP/s over the four linears of a 7B layer, 1639 on zeros.
 // The 128 x 512 form has 128 registers of sums and none for two chunks of weights: it holds one chunk's, each half loaded again as soon as its last operand is formed
 // (a little more than half a chunk, 1.4 us, ahead of its use; the other row tiles of the XCD's band have most of them in L2).  230 and 236 registers; a ring of two spills.
 template <int WBITS, int TPW, int MB, int AHEAD>
